@@ -420,53 +420,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_packed_kernel(const bf16_t* _
       }
     }
   } else if constexpr (MODE == PK_ROTARY) {
-    const int dim = rotary.dim;
-    const int half = dim / 2;
-    const int per_head = dim / 16;                                  // blocks of a head
-    const int rotated_blocks = (rotary.heads + rotary.kv_heads) * per_head;
-    const int b = blockIdx.x;
-    const bool turns = b < rotated_blocks;
-    const int head = b / per_head;                                  // among q, k, v heads in this order
-    const int sub = b % per_head;
-    // the first of this lane's four columns within its head
-    const int d0 = turns ? (g / 2) * half + 8 * sub + 4 * (g % 2) : 16 * sub + 4 * g;
-    float own[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) own[i] = acc[i] + (bias != nullptr ? bias[static_cast<int64_t>(head) * dim + d0 + i] : 0.f);
-    float other[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) other[i] = __shfl_xor(own[i], 32, 64);
-    if (r >= M) return;
-    float v[4];
-    if (turns) {
-      const float2* angles = rotary.table + static_cast<int64_t>(r) * half + 8 * sub + 4 * (g % 2);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float2 cs = angles[i];
-        // first half: x1 cos - x2 sin; second half: x2 cos + x1 sin
-        v[i] = g < 2 ? own[i] * cs.x - other[i] * cs.y : own[i] * cs.x + other[i] * cs.y;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = own[i];
-    }
-    const uint2 packed = pack_bf16x4(v);
-    *reinterpret_cast<uint2*>(y + static_cast<int64_t>(r) * N + static_cast<int64_t>(head) * dim + d0) = packed;
-    if (rotary.write && head >= rotary.heads) {
-      const int64_t slot = rotary.slots[r];
-      const int64_t page = slot / rotary.block_size;
-      const int offset = static_cast<int>(slot % rotary.block_size);
-      if (turns) {
-        const int kv_head = head - rotary.heads;
-        *reinterpret_cast<uint2*>(rotary.k_cache + ((page * rotary.kv_heads + kv_head) * rotary.block_size + offset) * dim + d0) =
-            packed;
-      } else {
-        const int kv_head = head - rotary.heads - rotary.kv_heads;
-        bf16_t* at = rotary.v_cache + ((page * rotary.kv_heads + kv_head) * dim + d0) * rotary.block_size + offset;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) at[static_cast<int64_t>(i) * rotary.block_size] = static_cast<bf16_t>(v[i]);
-      }
-    }
+    const float sums[4] = {acc[0], acc[1], acc[2], acc[3]};
+    store_rotary(sums, r, r < M, g, blockIdx.x, bias, y, N, rotary);
   } else {
     Y* out = y + static_cast<int64_t>(blockIdx.y) * m_all * N;
     const bool with_bias = bias != nullptr && blockIdx.y == 0;

@@ -46,3 +46,55 @@ static __device__ __forceinline__ uint2 pack_bf16x4(const float v[4]) {
   for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(uint16_t, static_cast<bf16_t>(v[i]));
   return uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
 }
+
+// The first of the four columns, in the weight's own order, that lane group g holds of block `block` of a ROTARY copy:
+// block (head, sub) of a q or k head holds the head's rows 8 sub .. + 7 and dim / 2 + 8 sub .. + 7, of a v head 16 in order.
+static __device__ __forceinline__ int rotary_column(int block, int g, int turned_heads, int dim) {
+  const int per_head = dim / 16, head = block / per_head, sub = block % per_head;
+  return head * dim + (head < turned_heads ? (g / 2) * (dim / 2) + 8 * sub + 4 * (g % 2) : 16 * sub + 4 * g);
+}
+
+// The end of a q/k/v product on a ROTARY copy: sums[i] is row 4 g + i of the block for token m. Adds the bias, turns the
+// pairs (partners are lanes 32 apart: every lane of the wave has to come here), writes y and the paged cache where
+// `inside` says that the token exists.
+static __device__ __forceinline__ void store_rotary(const float sums[4], int64_t m, bool inside, int g, int block,
+                                                    const float* bias, bf16_t* y, int N, const RotaryOut& rotary) {
+  const int dim = rotary.dim, half = dim / 2, per_head = dim / 16;
+  const int head = block / per_head, sub = block % per_head;          // among q, k, v heads in this order
+  const bool turns = head < rotary.heads + rotary.kv_heads;
+  const int column = rotary_column(block, g, rotary.heads + rotary.kv_heads, dim), d0 = column - head * dim;
+  float own[4], other[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) own[i] = sums[i] + (bias != nullptr ? bias[column + i] : 0.f);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) other[i] = __shfl_xor(own[i], 32, 64);
+  if (!inside) return;
+  float v[4];
+  if (turns) {
+    const float2* angles = rotary.table + m * half + 8 * sub + 4 * (g % 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float2 cs = angles[i];
+      // first half: x1 cos - x2 sin; second half: x2 cos + x1 sin
+      v[i] = g < 2 ? own[i] * cs.x - other[i] * cs.y : own[i] * cs.x + other[i] * cs.y;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = own[i];
+  }
+  const uint2 packed = pack_bf16x4(v);
+  *reinterpret_cast<uint2*>(y + m * N + column) = packed;
+  if (!rotary.write || head < rotary.heads) return;
+  const int slot = rotary.slots[m];                    // (divided in 32 bits: in 64 it is some hundred instructions a block)
+  const int64_t page = slot / rotary.block_size;
+  const int offset = slot % rotary.block_size;
+  if (turns) {
+    const int kv_head = head - rotary.heads;
+    *reinterpret_cast<uint2*>(rotary.k_cache + ((page * rotary.kv_heads + kv_head) * rotary.block_size + offset) * dim + d0) = packed;
+  } else {
+    const int kv_head = head - rotary.heads - rotary.kv_heads;
+    bf16_t* at = rotary.v_cache + ((page * rotary.kv_heads + kv_head) * dim + d0) * rotary.block_size + offset;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) at[static_cast<int64_t>(i) * rotary.block_size] = static_cast<bf16_t>(v[i]);
+  }
+}

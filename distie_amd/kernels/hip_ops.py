@@ -202,6 +202,32 @@ class HipOps(Ops):
     # (7B shape: decode step at batch 80 6.8 ms in one pass of 80 rows, 7.7 as 64 + 16; at batch 96 8.1 and 8.3;
     # a portion of 160 tokens 7.4 ms in two passes of 80 and 8.4 in three of 64, 64 and 32)
     WIDE_PASS_MAX_BLOCKS = 6
+    # From TILES_MIN_ROWS rows of x on, products on a packed copy whose K is a multiple of 64 run in tiles
+    # (`packed_tiles.hip`) where that is faster than the passes above and than the library, which is a matter of the
+    # product's size. Measured with every weight coming from memory (us, tiles / passes up to 96 rows, the library beyond):
+    #  * up to TILES_MAX_WORK multiplications: [64, 8960] x [1536, 8960] 9.1 / 12.0, [64, 1536] x [2048, 1536] 5.8 / 7.1,
+    #    [301, 2048] x [2048, 2048] 10.6 / 11.4, [512, 1024] x [1280, 1024] 7.2 / 10.9, [1200, 1536] x [2048, 1536] 16.3 / 17.7;
+    #    beyond, the library's larger tiles come level: [512, 3584] x [4608, 3584] 30.6 / 28.9;
+    #  * K at least twice as long as the weight has rows: cut along K, as many rows as there are, but for small weights
+    #    of many rows (TILES_LONG_ROWS): [301, 8960] x [1536, 8960] 18.1 / 26.3, [900, 8960] 38.1 / 41.6, [301, 18944] x
+    #    [3584, 18944] 67.7 / 100.5, [2025, 18944] 260 / 350; [1600, 8192] x [2048, 8192] 69.5 / 63.7;
+    #  * gated products, which save the activation's kernel: up to TILES_MAX_GATED_WORK; [64, 1536] x [17920, 1536] 19.8 /
+    #    21.9, [176, 1536] 27.7 / 30.2, [301, 1536] 33.5 / 34.7, [512, 1024] x [8192, 1024] 17.8 / 22.3, [400, 1536] x
+    #    [17920, 1536] 42.2 / 39.0; below 80 rows a weight of up to TILES_SMALL_GATED elements is faster in passes
+    #    ([64, 1024] x [8192, 1024] 9.1 / 8.2);
+    #  * q/k/v with rotation and cache write in the epilogue: from TILES_MIN_ROTARY_ROWS on, up to TILES_MAX_WORK.
+    TILES_MIN_ROWS = 33
+    TILES_MIN_ROTARY_ROWS = 80
+    TILES_MAX_WORK = 4.5e9
+    TILES_MAX_GATED_WORK = 8.5e9
+    TILES_LONG_ROWS = 1100
+    TILES_SMALL_GATED = 10 << 20
+    # (A weight that no role was named for stays with the passes: who reads its product is not known.)
+    # What a cut product costs beyond its slices where the reader of the result cannot add them itself (the readers of a
+    # layer's output projections can), and what rotation and cache write cost as a kernel of their own
+    ADDS_SLICES = ("attn_out", "down")
+    SUM_SLICES_US = 4.5
+    ROPE_KV_WRITE_US = 7.0
     # attention over a portion of a prompt: from so many visible keys on, the walk over the keys is cut into so
     # many parts that run side by side (measured at 12 heads of 128, 2,048 new tokens: 3 parts are best up to
     # 4,096 keys, 5 at 8,192, 8 from 16,384 on; the kernel takes up to 16)
@@ -254,6 +280,7 @@ class HipOps(Ops):
         self._tuning = False
         self.library_timed_rows = 0
         self._packed_left_out = 0
+        self._tile_plans: Dict[tuple, Optional[tuple]] = {}
         self._ops = ctypes.CDLL(str(build.ensure("ops")))
         self._declare()
         self._attn: Dict[int, ctypes.CDLL] = {}
@@ -308,6 +335,9 @@ class HipOps(Ops):
         o.distie_gemm_packed_wide_slices.argtypes = [_I, _I]
         o.distie_gemm_packed_wide_qkv_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_packed_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
+        o.distie_packed_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F, ctypes.POINTER(_I), ctypes.POINTER(_I)]
+        o.distie_packed_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
+        o.distie_packed_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_packed_each_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _P, _P]
         o.distie_decode_norm_fits.argtypes = [_I]
         o.distie_decode_product_residual.argtypes = [_P, _P, _P, _P, _I, _I, _I, _P]
@@ -586,6 +616,7 @@ class HipOps(Ops):
                                           row_map.numel() // 16, K, self._stream()), "pack_rows")
         torch.cuda.current_stream(self.device).synchronize()      # row_map is freed on return
         # the copy lives and dies with the weight
+        weight._distie_role = role
         setattr(weight, name, (packed, tuple(rotary)) if name == "_distie_rotary" else packed)
 
     def _norm_product(self, x: PendingNorm, packed, bias, out, mode, N, rotary=None):
@@ -640,7 +671,11 @@ class HipOps(Ops):
             out = torch.empty((x.shape[0], N // 2), dtype=torch.bfloat16, device=self.device)
             return self._norm_product(x, packed, None, out, gated, N)
         x = self.dense(x)
-        if packed is None or x.dtype != torch.bfloat16 or x.shape[0] > self._packed_rows(x.shape[0], *gate_up_weight.shape):
+        plan = None
+        if packed is not None and x.dtype == torch.bfloat16:
+            plan = self._tiles(x.shape[0], *gate_up_weight.shape, "gated")
+        if packed is None or x.dtype != torch.bfloat16 or \
+                (plan is None and x.shape[0] > self._packed_rows(x.shape[0], *gate_up_weight.shape)):
             return apart(self.linear(x, gate_up_weight))
         self._own(x)
         M, K = x.shape
@@ -649,6 +684,8 @@ class HipOps(Ops):
             raise KernelError(f"linear: x is [{M}, {K}], weight is {list(gate_up_weight.shape)}")
         if packed.numel() != self._packed_elements(N, K, True):
             raise KernelError("linear_silu_mul: the packed copy does not belong to this weight")
+        if plan is not None:
+            return self._run_tiles(plan, x, packed, None, x.dtype, M, N, K, gated, clamp=clamp)
         out = torch.empty((M, N // 2), dtype=x.dtype, device=self.device)
         if M <= self.ONE_WAVE_MAX_ROWS:
             _check(self._ops.distie_gemm_packed_bf16(x.data_ptr(), packed.data_ptr(), None, out.data_ptr(), _code(out),
@@ -684,9 +721,12 @@ class HipOps(Ops):
             return self._norm_product(x, packed, bias, out, 2, N, rotary=(
                 table, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, meta.block_size, 1 if write else 0))
         x = self.dense(x)
-        fused = held is not None and held[1] == (num_heads, num_kv_heads, head_dim) and \
-            x.dtype == torch.bfloat16 and x.shape[0] <= self._packed_rows(x.shape[0], *weight.shape) and \
+        plan = None
+        fused = held is not None and held[1] == (num_heads, num_kv_heads, head_dim) and x.dtype == torch.bfloat16 and \
             inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and k_cache.dtype == torch.bfloat16
+        if fused:
+            plan = self._tiles(x.shape[0], *weight.shape, "rotary", self.ROPE_KV_WRITE_US)
+            fused = plan is not None or x.shape[0] <= self._packed_rows(x.shape[0], *weight.shape)
         if not fused:
             return self.rope_kv_write(self.linear(x, weight, bias), meta, group, k_cache, v_cache, inv_freq,
                                       num_heads, num_kv_heads, head_dim, write)
@@ -704,7 +744,11 @@ class HipOps(Ops):
         self._check_cache(k_cache, v_cache, num_kv_heads, meta.block_size, head_dim)
         if M != meta.num_tokens or slots.shape[0] != M:
             raise KernelError("linear_rope_kv_write: rows do not match the batch")
-        if M >= self.WIDE_QKV_MIN_ROWS and N * K > self.ROW_GROUPS_MAX_ELEMENTS:
+        if plan is not None and plan[1] > 1:
+            product = self._run_tiles(plan, x, packed, bias, torch.bfloat16, M, N, K, heads=(num_heads, num_kv_heads, head_dim))
+            return self.rope_kv_write(product, meta, group, k_cache, v_cache, inv_freq, num_heads, num_kv_heads,
+                                      head_dim, write)
+        if plan is None and M >= self.WIDE_QKV_MIN_ROWS and N * K > self.ROW_GROUPS_MAX_ELEMENTS:
             # more than one group of 16 rows against a weight that fills the chip through the wide kernel: the
             # epilogue kernel would read the weight once per group, so the product runs wide (weights once, K in
             # slices) and the rotation with the cache write behind it adds the slices
@@ -721,6 +765,12 @@ class HipOps(Ops):
                                       head_dim, write)
         table = self._rope_table(meta, inv_freq)
         out = torch.empty((M, N), dtype=torch.bfloat16, device=self.device)
+        if plan is not None:
+            _check(self._ops.distie_packed_tiles_rotary_bf16(
+                x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads,
+                num_kv_heads, head_dim, meta.block_size, 1 if write else 0, plan[0], self._stream()), "packed_tiles_rotary_bf16")
+            return out
         _check(self._ops.distie_gemm_packed_rotary_bf16(
             x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
             table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads,
@@ -734,6 +784,48 @@ class HipOps(Ops):
                 return self.PACKED_MAX_ROWS_LARGE
             return self.PACKED_MAX_ROWS_LARGE_WIDE_TIMED if M <= self.library_timed_rows else self.PACKED_MAX_ROWS_LARGE_WIDE
         return self.PACKED_MAX_ROWS if self.captured else self.PACKED_MAX_ROWS_EAGER
+
+    TILE_PLANS = 4096                # products whose cut is remembered
+
+    def _tiles(self, M: int, N: int, K: int, kind: str, cut_us: Optional[float] = None):
+        """(shape, slices) of the tiled kernels for a product of M rows with an [N, K] weight, None if another kernel is
+        the better one. kind: "plain", "gated" or "rotary"; cut_us: what a cut of K costs the reader of the result beyond
+        reading the slices (None: it must not be cut)."""
+        if M < self.TILES_MIN_ROWS:
+            return None
+        key = (M, N, K, kind, cut_us, self.library_timed_rows)
+        try:
+            return self._tile_plans[key]
+        except KeyError:
+            pass
+        work, plan = M * N * K, None
+        if kind == "gated":
+            wanted = work <= self.TILES_MAX_GATED_WORK and (M >= 80 or N * K > self.TILES_SMALL_GATED)
+        elif kind == "rotary":
+            wanted = work <= self.TILES_MAX_WORK and M >= self.TILES_MIN_ROTARY_ROWS
+        else:
+            wanted = work <= self.TILES_MAX_WORK or \
+                (K >= 2 * N and cut_us is not None and (M <= self.TILES_LONG_ROWS or N * K > self.PACKED_LARGE_ELEMENTS))
+        if wanted:
+            shape, slices = ctypes.c_int(0), ctypes.c_int(0)
+            if self._ops.distie_packed_tiles_plan(M, N, K, kind == "gated", cut_us is not None, cut_us or 0.0,
+                                                  ctypes.byref(shape), ctypes.byref(slices)):
+                plan = (shape.value, slices.value)
+        if len(self._tile_plans) >= self.TILE_PLANS:
+            self._tile_plans.clear()
+        self._tile_plans[key] = plan
+        return plan
+
+    def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, heads=(0, 0, 0), clamp=(0.0, 1.0, 0.0)):
+        """The tiled product; float32 slices if the plan cuts K."""
+        shape, slices = plan
+        columns = N // 2 if gated else N
+        out = torch.empty((M, columns), dtype=out_dtype, device=self.device) if slices == 1 else \
+            torch.empty((slices, M, columns), dtype=torch.float32, device=self.device)
+        _check(self._ops.distie_packed_tiles_bf16(
+            x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), _code(out),
+            M, N, K, gated, shape, slices, *heads, *clamp, self._stream()), "packed_tiles_bf16")
+        return out if slices == 1 else PartialSums(out, out_dtype)
 
     def _library(self):
         """The vendor library's products, called directly; loaded at the first large product."""
@@ -858,6 +950,15 @@ class HipOps(Ops):
         packed = packed if both_bf16 else None
         if lazy and packed is not None and self._fused(M) and K % 8 == 0 and out_dtype == torch.bfloat16:
             return PendingProduct(x, weight, bias)
+        plan = None
+        if packed is not None and weight._distie_role is not None:
+            adds = partial_ok and weight._distie_role in self.ADDS_SLICES
+            plan = self._tiles(M, N, K, "plain", 0.0 if adds else self.SUM_SLICES_US)
+        if plan is not None:
+            if packed.numel() != self._packed_elements(N, K, False):
+                raise KernelError("linear: the packed copy does not belong to this weight")
+            out = self._run_tiles(plan, x, packed, bias, out_dtype, M, N, K)
+            return out if partial_ok else self.dense(out)
         if packed is not None and self.ONE_WAVE_MAX_ROWS < M <= self._packed_rows(M, N, K) and K % 8 == 0 and \
                 N * K > self.ROW_GROUPS_MAX_ELEMENTS:
             if packed.numel() != self._packed_elements(N, K, False):

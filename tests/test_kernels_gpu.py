@@ -262,6 +262,40 @@ def test_linear_silu_mul_fused(ops, M, I, K):
     close(ops.linear_silu_mul(big, w), want, torch.bfloat16, scale=2 * want.abs().max().item())
 
 
+@pytest.mark.parametrize("shape,rows", [(0, 64), (1, 64), (2, 96), (3, 128), (4, 128)])
+@pytest.mark.parametrize("N,K", [(16, 128), (250, 192), (1030, 1088), (520, 4096)])
+def test_packed_tiles(ops, shape, rows, N, K):
+    """Every tile of the products of many rows on packed copies: rows and columns that do not fill a tile, fewer stages
+    than are under way and more, odd and even, K whole and cut; plain with a bias in both types, and gated with both
+    kinds of activation. Sums are float32, rounded once: the bounds are those of the other products on packed copies."""
+    w, b = rand(N, K, dtype=torch.bfloat16, seed=2, scale=K ** -0.5), rand(N, seed=3)
+    gate_up = rand(N, K, dtype=torch.bfloat16, seed=4, scale=2.0 * K ** -0.5)
+    ops.prepare_linear(w, role="down")
+    ops.prepare_linear(gate_up, gated=True, role="gate_up")
+    for M in (1, rows - 1, rows, rows + 1, 2 * rows + 17):
+        x = rand(M, K, dtype=torch.bfloat16, seed=M)
+        want = x.double() @ w.double().T + b.double()
+        stages = K // 64
+        for slices in (1, 2, 3, 8):
+            if -(-stages // -(-stages // slices)) != slices:
+                continue
+            got = ops._run_tiles((shape, slices), x, w._distie_packed, b, torch.float32, M, N, K)
+            close(ops.dense(got), want, torch.float32, scale=5 * want.abs().max().item())
+            assert slices == 1 or got.slices == slices
+        got = ops._run_tiles((shape, 1), x, w._distie_packed, b, torch.bfloat16, M, N, K)
+        close(got, want, torch.bfloat16, scale=want.abs().max().item())
+        product = x.double() @ gate_up.double().T
+        gate, up = product[:, :N // 2], product[:, N // 2:]
+        got = ops._run_tiles((shape, 1), x, gate_up._distie_gated, None, torch.bfloat16, M, N, K, gated=1)
+        want = gate / (1 + torch.exp(-gate)) * up
+        close(got, want, torch.bfloat16, scale=want.abs().max().item())
+        got = ops._run_tiles((shape, 1), x, gate_up._distie_gated, None, torch.bfloat16, M, N, K,
+                             gated=1 | (ops.CLAMPED << 8), clamp=(0.7, 1.702, 1.0))
+        gate, up = gate.clamp(max=0.7), up.clamp(-0.7, 0.7)
+        want = gate / (1 + torch.exp(-1.702 * gate)) * (up + 1)
+        close(got, want, torch.bfloat16, scale=want.abs().max().item())
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 17, 45, 64, 70, 96, 129, 224])
 @pytest.mark.parametrize("heads,kv_heads,dim,K,P", [(3, 1, 32, 2048, 4), (12, 2, 128, 1536, 16), (4, 4, 16, 72, 16),
                                                     (5, 5, 48, 240, 8), (2, 1, 80, 520, 16), (7, 1, 256, 136, 32),
