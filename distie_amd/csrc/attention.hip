@@ -16,6 +16,7 @@
 //  * attn_decode + attn_reduce, attn_prefill: bfloat16 on the matrix cores (described further down).
 
 #include "common.h"
+#include <algorithm>
 
 #ifndef DISTIE_HEAD_DIM
 #error "compile with -DDISTIE_HEAD_DIM=<head size>"
@@ -232,7 +233,12 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_generic_kernel(
 // eighth of the key's row of K (a run of D / 8 floats, so a wave's load covers eight whole rows; with a lane
 // to a key every 16-byte load of a wave touched 64 lines) against its slices of the heads' queries, which it
 // keeps in registers; the sums of the eight lanes are added by three exchanges. With G > 1 every row of K
-// and every value of V^T is read once for G heads; the caller takes G as large as leaves enough workgroups.
+// and every value of V^T is read once for G heads.
+//
+// What bounds it is the chain of trips to memory that a wave makes for 64 keys (page, K, V), so the keys of a token go to
+// gridDim.z workgroups in runs of whole chunks (each token's own keys cut alike), which leave their sums for
+// attn_grouped_merge_kernel. 8 requests of 770 to 1,000 keys, 12 heads of 128 on 2: 24.5 us a call with one workgroup of
+// eight waves a (token, head), 96 in all; 12.7 and 4.7 with three heads to a workgroup of four waves and four runs.
 constexpr bool GQ_FITS = D % 32 == 0;
 constexpr int GQ_SLICE = GQ_FITS ? D / 8 : 4;
 
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_request,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ table_rows,
     float* __restrict__ out, int heads, int kv_heads, int parts, int block_size, float scale, int window,
-    const float* __restrict__ sinks) {
+    const float* __restrict__ sinks, float* __restrict__ part_o, float* __restrict__ part_ml) {
   __shared__ float p_s[WAVES][G][DISTIE_WAVE];
   __shared__ int64_t base_s[WAVES][DISTIE_WAVE];
   __shared__ float m_s[WAVES][G], l_s[WAVES][G];
@@ -282,7 +288,11 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
     for (int i = 0; i < DIMS_PER_LANE; ++i) acc[g][i] = 0.f;
   }
 
-  for (int c = first / DISTIE_WAVE * DISTIE_WAVE + wave * DISTIE_WAVE; c <= last; c += DISTIE_WAVE * WAVES) {
+  const int chunk0 = first / DISTIE_WAVE, chunks = last / DISTIE_WAVE - chunk0 + 1;
+  const int per_run = (chunks + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
+  const int run0 = static_cast<int>(blockIdx.z) * per_run;
+  const int run_end = min(chunks, run0 + per_run);          // (a run may hold no chunk)
+  for (int c = (chunk0 + run0 + wave) * DISTIE_WAVE; c < (chunk0 + run_end) * DISTIE_WAVE; c += DISTIE_WAVE * WAVES) {
     // Every load of a phase is issued before its results are used (a chunk costs a few trips to memory, not one
     // for every pass and page): lane j looks up the page of key c + j, the addresses go from lane to lane.
     const int key = c + lane;
@@ -406,8 +416,9 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
     }
   __syncthreads();
   // wave w writes heads w, w + WAVES, ... of the part
+  const bool whole = gridDim.z == 1;
   for (int g = wave; g < n; g += WAVES) {
-    const float sink = sinks != nullptr ? sinks[h0 + g] : -INFINITY;      // one more term of the denominator, no value
+    const float sink = whole && sinks != nullptr ? sinks[h0 + g] : -INFINITY;      // one more term of the denominator, no value
     float top = sink;
     for (int w = 0; w < WAVES; ++w) top = fmaxf(top, m_s[w][g]);
     float total = sink == -INFINITY ? 0.f : expf(sink - top);
@@ -416,8 +427,14 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
       weight[w] = m_s[w][g] == -INFINITY ? 0.f : expf(m_s[w][g] - top);    // a wave without keys counts nothing
       total += l_s[w][g] * weight[w];
     }
-    const float inv = 1.f / total;
-    float* o = out + (t * heads + h0 + g) * D;
+    const int64_t at = t * heads + h0 + g + (whole ? 0 : static_cast<int64_t>(blockIdx.z) * gridDim.x * heads);
+    const float inv = whole ? 1.f / total : 1.f;
+    float* o = (whole ? out : part_o) + at * D;
+    if (!whole && lane == 0) {
+      part_ml[2 * at] = top;
+      part_ml[2 * at + 1] = total;
+    }
+    if (!whole && total == 0.f) continue;                   // no key in this run: its sums are not read
 #pragma unroll
     for (int i = 0; i < DIMS_PER_LANE; ++i) {
       const int d = lane + i * DISTIE_WAVE;
@@ -429,40 +446,101 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
   }
 }
 
+// The runs of attn_grouped_f32_kernel put together in their order: a workgroup of one wave a (token, head).
+constexpr int GQ_MAX_RUNS = 16;
+
+__global__ __launch_bounds__(DISTIE_WAVE) void attn_grouped_merge_kernel(const float* __restrict__ part_o,
+                                                                         const float* __restrict__ part_ml,
+                                                                         float* __restrict__ out, int heads, int runs,
+                                                                         const float* __restrict__ sinks) {
+  const int64_t at = static_cast<int64_t>(blockIdx.x) * heads + blockIdx.y;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * heads;
+  float2 ml[GQ_MAX_RUNS];
+#pragma unroll
+  for (int s = 0; s < GQ_MAX_RUNS; ++s)
+    ml[s] = s < runs ? *reinterpret_cast<const float2*>(part_ml + 2 * (s * stride + at)) : float2{-INFINITY, 0.f};
+  const float sink = sinks != nullptr ? sinks[blockIdx.y] : -INFINITY;
+  float top = sink;
+#pragma unroll
+  for (int s = 0; s < GQ_MAX_RUNS; ++s) top = fmaxf(top, ml[s].x);
+  float total = sink == -INFINITY ? 0.f : expf(sink - top);
+  float weight[GQ_MAX_RUNS];
+#pragma unroll
+  for (int s = 0; s < GQ_MAX_RUNS; ++s) {
+    weight[s] = ml[s].y > 0.f ? expf(ml[s].x - top) : 0.f;
+    total += ml[s].y * weight[s];
+  }
+  const float inv = 1.f / total;
+  for (int d = 4 * threadIdx.x; d < D; d += 4 * DISTIE_WAVE) {
+    float4 o[GQ_MAX_RUNS];
+#pragma unroll
+    for (int s = 0; s < GQ_MAX_RUNS; ++s) {
+      o[s] = float4{0.f, 0.f, 0.f, 0.f};
+      if (s < runs && ml[s].y > 0.f) o[s] = *reinterpret_cast<const float4*>(part_o + (s * stride + at) * D + d);
+    }
+    float4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < GQ_MAX_RUNS; ++s) {
+      sum.x = fmaf(weight[s], o[s].x, sum.x);
+      sum.y = fmaf(weight[s], o[s].y, sum.y);
+      sum.z = fmaf(weight[s], o[s].z, sum.z);
+      sum.w = fmaf(weight[s], o[s].w, sum.w);
+    }
+    *reinterpret_cast<float4*>(out + at * D + d) = float4{sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv};
+  }
+}
+
+// Query heads of a kv head that a workgroup takes together, and the workgroups for all of them.
+static int grouped_parts(int group) { return (group + 3) / 4; }
+
+static bool grouped_fits(int64_t tokens, int heads) { return GQ_FITS && tokens * heads < 2048; }
+
 // qkv: [T, q_stride] with q of head h at columns h*D; out: [T, heads*D]. window: see the head of the file.
 // head_slopes (float32 [heads], may be null): score += slope[h] * (key - position); score_cap > 0: the scaled score
 // goes through cap * tanh(score / cap) first. Only this kernel takes the two. sinks (float32 [heads], may be null): the
 // softmax's denominator holds exp(sinks[h]) beside the keys' terms; every kernel of this file takes them.
+// Into how many runs distie_attention_generic is best asked to cut each token's keys (float32, plain scores; the runs that a
+// launch takes do not change what it computes): enough workgroups for every compute unit twice over, 256 keys each at
+// least. visible: the most keys that a token sees.
+extern "C" int distie_attention_f32_runs(int tokens, int heads, int kv_heads, int visible) {
+  if (tokens < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || !grouped_fits(tokens, heads)) return 1;
+  const int64_t units = static_cast<int64_t>(tokens) * kv_heads * grouped_parts(heads / kv_heads);
+  const int64_t wanted = (512 + units - 1) / units;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({wanted, (visible + 255) / 256, GQ_MAX_RUNS})));
+}
+
 extern "C" int distie_attention_generic(const void* qkv, int dtype, int64_t q_stride, const void* k_cache,
                                         const void* v_cache, int cache_dtype, const int32_t* positions,
                                         const int32_t* token_request, const int32_t* block_table,
                                         int table_width, const int32_t* table_rows, void* out, int tokens, int heads, int kv_heads,
                                         int block_size, float scale, int window, const float* head_slopes,
-                                        float score_cap, const float* sinks, hipStream_t stream) {
+                                        float score_cap, const float* sinks, float* part_o, float* part_ml, int runs,
+                                        hipStream_t stream) {
   if (tokens <= 0) return 0;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || block_size < 1 || table_width < 1 ||
-      score_cap < 0.f)
+      score_cap < 0.f || runs < 1 || runs > GQ_MAX_RUNS || (runs > 1 && (part_o == nullptr || part_ml == nullptr)))
     return DISTIE_BAD_ARGUMENT;
   const bool plain_scores = head_slopes == nullptr && score_cap == 0.f;
   if (heads > 65535) return DISTIE_BAD_ARGUMENT;
   dim3 grid(tokens, heads);
   const int group = heads / kv_heads;
-  if (plain_scores && GQ_FITS && dtype == DISTIE_F32 && cache_dtype == DISTIE_F32 && q_stride % 4 == 0 && block_size % 4 == 0 &&
-      DISTIE_WAVE % block_size == 0 && static_cast<int64_t>(tokens) * heads < 2048) {
-    // requests that decode, float32: as many heads of a kv head to a workgroup as leaves a workgroup a compute unit
-    int per = 1;
-    for (int g : {2, 4})
-      if (group >= g && static_cast<int64_t>(tokens) * kv_heads * ((group + g - 1) / g) >= 256) per = g;
-    const int parts = (group + per - 1) / per;
-    const dim3 grouped(tokens, kv_heads * parts);
-#define DISTIE_GROUPED(G, WAVES)                                                                                   \
-    attn_grouped_f32_kernel<G, WAVES><<<grouped, DISTIE_WAVE * WAVES, 0, stream>>>(                                  \
+  if (plain_scores && grouped_fits(tokens, heads) && dtype == DISTIE_F32 && cache_dtype == DISTIE_F32 && q_stride % 4 == 0 &&
+      block_size % 4 == 0 && DISTIE_WAVE % block_size == 0) {
+    // requests that decode, float32: up to four heads of a kv head to a workgroup of four waves, equally many in each
+    const int parts = grouped_parts(group), per = (group + parts - 1) / parts;
+    const dim3 grouped(tokens, kv_heads * parts, runs);
+#define DISTIE_GROUPED(G)                                                                                          \
+    attn_grouped_f32_kernel<G, 4><<<grouped, DISTIE_WAVE * 4, 0, stream>>>(                                         \
         static_cast<const float*>(qkv), q_stride, static_cast<const float*>(k_cache),                               \
         static_cast<const float*>(v_cache), positions, token_request, block_table, table_width, table_rows,         \
-        static_cast<float*>(out), heads, kv_heads, parts, block_size, scale, window, sinks)
-    if (per == 4) DISTIE_GROUPED(4, 8);
-    else if (per == 2) DISTIE_GROUPED(2, 8);
-    else DISTIE_GROUPED(1, 8);
+        static_cast<float*>(out), heads, kv_heads, parts, block_size, scale, window, sinks, part_o, part_ml)
+    if (per == 4) DISTIE_GROUPED(4);
+    else if (per == 3) DISTIE_GROUPED(3);
+    else if (per == 2) DISTIE_GROUPED(2);
+    else DISTIE_GROUPED(1);
+    if (runs > 1)
+      attn_grouped_merge_kernel<<<dim3(tokens, heads), DISTIE_WAVE, 0, stream>>>(part_o, part_ml, static_cast<float*>(out),
+                                                                                 heads, runs, sinks);
 #undef DISTIE_GROUPED
     return launch_status();
   }

@@ -15,7 +15,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 struct RotaryOut {
   const float2* table;        // [M, D / 2] cosine and sine of each token's angles
   const int32_t* slots;       // [M] place of each token in the cache
-  bf16_t* k_cache;            // [pages, kv_heads, block_size, D]
+  bf16_t* k_cache;            // [pages, kv_heads, block_size, D] (float32 behind these pointers where the result is)
   bf16_t* v_cache;            // [pages, kv_heads, D, block_size]
   int heads, kv_heads, dim, block_size, write;
   int act;                    // gated products only: the activation on the gate (see gate_activation)
@@ -47,6 +47,19 @@ static __device__ __forceinline__ uint2 pack_bf16x4(const float v[4]) {
   return uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
 }
 
+// four neighbouring values of a row, from column n0 on, of which those below `columns` exist
+template <typename Y>
+static __device__ __forceinline__ void store_four(Y* row, int n0, int columns, const float v[4]) {
+  if (n0 + 4 <= columns && columns % 4 == 0) {
+    if constexpr (sizeof(Y) == 2) *reinterpret_cast<uint2*>(row + n0) = pack_bf16x4(v);
+    else *reinterpret_cast<float4*>(row + n0) = float4{v[0], v[1], v[2], v[3]};
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n0 + i < columns) row[n0 + i] = from_float<Y>(v[i]);
+  }
+}
+
 // The first of the four columns, in the weight's own order, that lane group g holds of block `block` of a ROTARY copy:
 // block (head, sub) of a q or k head holds the head's rows 8 sub .. + 7 and dim / 2 + 8 sub .. + 7, of a v head 16 in order.
 static __device__ __forceinline__ int rotary_column(int block, int g, int turned_heads, int dim) {
@@ -57,8 +70,9 @@ static __device__ __forceinline__ int rotary_column(int block, int g, int turned
 // The end of a q/k/v product on a ROTARY copy: sums[i] is row 4 g + i of the block for token m. Adds the bias, turns the
 // pairs (partners are lanes 32 apart: every lane of the wave has to come here), writes y and the paged cache where
 // `inside` says that the token exists.
+template <typename Y>
 static __device__ __forceinline__ void store_rotary(const float sums[4], int64_t m, bool inside, int g, int block,
-                                                    const float* bias, bf16_t* y, int N, const RotaryOut& rotary) {
+                                                    const float* bias, Y* y, int N, const RotaryOut& rotary) {
   const int dim = rotary.dim, half = dim / 2, per_head = dim / 16;
   const int head = block / per_head, sub = block % per_head;          // among q, k, v heads in this order
   const bool turns = head < rotary.heads + rotary.kv_heads;
@@ -82,19 +96,19 @@ static __device__ __forceinline__ void store_rotary(const float sums[4], int64_t
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = own[i];
   }
-  const uint2 packed = pack_bf16x4(v);
-  *reinterpret_cast<uint2*>(y + m * N + column) = packed;
+  store_four(y + m * N, column, N, v);
   if (!rotary.write || head < rotary.heads) return;
   const int slot = rotary.slots[m];                    // (divided in 32 bits: in 64 it is some hundred instructions a block)
   const int64_t page = slot / rotary.block_size;
   const int offset = slot % rotary.block_size;
   if (turns) {
     const int kv_head = head - rotary.heads;
-    *reinterpret_cast<uint2*>(rotary.k_cache + ((page * rotary.kv_heads + kv_head) * rotary.block_size + offset) * dim + d0) = packed;
+    Y* at = reinterpret_cast<Y*>(rotary.k_cache) + ((page * rotary.kv_heads + kv_head) * rotary.block_size + offset) * dim;
+    store_four(at, d0, dim, v);
   } else {
     const int kv_head = head - rotary.heads - rotary.kv_heads;
-    bf16_t* at = rotary.v_cache + ((page * rotary.kv_heads + kv_head) * dim + d0) * rotary.block_size + offset;
+    Y* at = reinterpret_cast<Y*>(rotary.v_cache) + ((page * rotary.kv_heads + kv_head) * dim + d0) * rotary.block_size + offset;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) at[static_cast<int64_t>(i) * rotary.block_size] = static_cast<bf16_t>(v[i]);
+    for (int i = 0; i < 4; ++i) at[static_cast<int64_t>(i) * rotary.block_size] = from_float<Y>(v[i]);
   }
 }

@@ -44,19 +44,6 @@ struct TilesPlace {
   int stages;                   // of a slice
 };
 
-// four neighbouring values of a row, from column n0 on, of which those below `columns` exist
-template <typename Y>
-__device__ __forceinline__ void store_four(Y* row, int n0, int columns, const float v[4]) {
-  if (n0 + 4 <= columns && columns % 4 == 0) {
-    if constexpr (sizeof(Y) == 2) *reinterpret_cast<uint2*>(row + n0) = pack_bf16x4(v);
-    else *reinterpret_cast<float4*>(row + n0) = float4{v[0], v[1], v[2], v[3]};
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n0 + i < columns) row[n0 + i] = from_float<Y>(v[i]);
-  }
-}
-
 // MODE: PK_PLAIN (also on a ROTARY copy, rotary.heads > 0: every sum into the column that its row of W has), PK_GATED,
 // PK_ROTARY. K a multiple of PT_K.
 template <int MB, int NB, int DEPTH, int MODE, typename Y>

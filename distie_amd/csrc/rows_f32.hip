@@ -1,0 +1,229 @@
+// The true 32-bit path's products of few rows of x on the matrix cores: y[M, N] = x[M, K] W[N, K]^T, float32 operands,
+// products and sums (v_mfma_f32_16x16x4_f32: no mode of reduced precision), W in the checkpoint's layout.
+//
+// A wave owns 16 rows of W (the A operand) and streams its share of K; up to 32 rows of x are the B operand, 16 a block.
+// A lane's sixteen bytes of a row of W or x hold four k, which four products take one after the other: the summed index
+// runs in the lanes' order (lane 16 g + r: row r, k 4 g .. 4 g + 3 of every 16), the same for both. Which rows a wave
+// owns is free, as W is not packed: gate rows beside their up rows, or the partners of a rotation, so that activation,
+// rotation and cache write happen in the epilogue as in the bfloat16 products.
+//
+// What bounds it: W from memory, at 3.1 to 4.0 TB/s of the 4.7 that a copy reaches (a wave's loads touch 64 bytes of each
+// of 16 rows); the matrix cores need a third of that time. 1.5B shape, cold weights, us, this and the kernel on the vector
+// ALU (gemv_rows) with what stood behind it: gate+up with activation at 1, 8, 32 rows 25.2, 29.8, 47.6 / 32.0, 39.2, 84.6;
+// down in 8 slices at 1, 8, 32 rows 15.9, 17.7, 23.2 / 16.6, 22.6, 40.2; q/k/v with rotation and cache write at 8 rows 8.8 /
+// 14.5. With more than 32 rows the sums' chains no longer fit the registers at the precision of the vector ALU's kernel.
+
+#include "common.h"
+#include "packed.h"
+#include <algorithm>
+
+namespace {
+
+constexpr int RF_STEP = 64;           // k of a step: four loads of 16 bytes a lane and operand
+
+struct RowsShare {
+  const float* w;                     // the lane's row of W
+  const float* x[2];                  // and of x, a block of 16 rows each
+};
+
+// COUNT steps, every load issued before the first product. Their products go into CHAINS sums that start at zero, which
+// are added up in pairs and then to the total: one chain over the whole K rounds five times as far from the sum in 64
+// bits (5e-7 of it at K = 1,536; the vector ALU's kernel, whose lanes keep sums of their own, 1.1e-7).
+template <int MB, int COUNT>
+__device__ __forceinline__ void rows_steps(const RowsShare& at, int begin, int steps, int& step, floatx4 (&total)[MB]) {
+  constexpr int CHAINS = 16 / MB;
+  floatx4 a[COUNT][4], b[COUNT][MB][4];
+#pragma unroll
+  for (int u = 0; u < COUNT; ++u) {
+    const int k = RF_STEP * (begin + step);
+    step = step + 1 == steps ? 0 : step + 1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[u][j] = *reinterpret_cast<const floatx4*>(at.w + k + 16 * j);
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[u][m][j] = *reinterpret_cast<const floatx4*>(at.x[m] + k + 16 * j);
+  }
+  __builtin_amdgcn_sched_barrier(0);           // (left alone the compiler asks for each piece shortly before its use)
+  floatx4 acc[CHAINS][MB];
+#pragma unroll
+  for (int c = 0; c < CHAINS; ++c)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) acc[c][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < COUNT; ++u)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+          floatx4& c = acc[(4 * j + e) % CHAINS][m];
+          c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][j][e], b[u][m][j][e], c, 0, 0, 0);
+        }
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+#pragma unroll
+    for (int half = CHAINS / 2; half >= 1; half /= 2)
+#pragma unroll
+      for (int c = 0; c < half; ++c) acc[c][m] += acc[c + half][m];
+    total[m] += acc[0][m];
+  }
+}
+
+// blockIdx.x: block of 16 rows; blockIdx.y: slice of K (plain products only; slices side by side in y, bias on the
+// first). The waves of a workgroup share the slice's steps and add their sums through LDS; the first one writes.
+template <int MB, int MODE, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                              const float* __restrict__ bias, float* __restrict__ y, int M, int N,
+                                                              int K, int steps_per_slice, RotaryOut rotary) {
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, r = lane % 16, g = lane / 16;
+  const int block = blockIdx.x;
+  int64_t row;
+  if constexpr (MODE == PK_GATED) {
+    const int half = N / 2, j = min(8 * block + r % 8, half - 1);        // rows beyond the last: results dropped
+    row = r < 8 ? j : half + j;
+  } else if constexpr (MODE == PK_ROTARY) {
+    row = rotary_column(block, r / 4, rotary.heads + rotary.kv_heads, rotary.dim) + r % 4;
+  } else {
+    row = min(16 * block + r, N - 1);
+  }
+  RowsShare at;
+  at.w = w + row * K + 4 * g;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) at.x[m] = x + static_cast<int64_t>(min(16 * m + r, M - 1)) * K + 4 * g;
+  const int all = K / RF_STEP;
+  const int s_begin = blockIdx.y * steps_per_slice, s_end = min(all, s_begin + steps_per_slice);
+  const int share = (s_end - s_begin + WAVES - 1) / WAVES;
+  const int begin = min(s_end, s_begin + wave * share), steps = min(s_end, begin + share) - begin;
+  floatx4 acc[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // workgroups begin at different steps and wrap around, so that they do not pull on the same memory channels at once
+  int step = steps > 0 ? static_cast<int>((blockIdx.x + wave) % steps) : 0;
+  constexpr int UN = MB == 1 && WAVES == 1 ? 4 : 2;      // (gate+up at 8 rows, four waves: two 29.8 us, four 31.6)
+  int s = 0;
+  for (; s + UN <= steps; s += UN) rows_steps<MB, UN>(at, begin, steps, step, acc);
+  if constexpr (UN > 2) {
+    if (steps - s >= 2) {
+      rows_steps<MB, 2>(at, begin, steps, step, acc);
+      s += 2;
+    }
+  }
+  if (s < steps) rows_steps<MB, 1>(at, begin, steps, step, acc);
+
+  if constexpr (WAVES > 1) {
+    __shared__ float part[WAVES - 1][MB][4][64];
+    if (wave > 0) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[wave - 1][m][i][lane] = acc[m][i];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int v = 0; v < WAVES - 1; ++v)
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[m][i] += part[v][m][i][lane];
+  }
+  // acc[m][i]: row 4 g + i of the block, row 16 m + r of x
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const int at_row = 16 * m + r;
+    float v[4] = {acc[m][0], acc[m][1], acc[m][2], acc[m][3]};
+    if constexpr (MODE == PK_GATED) {
+      const int half = N / 2;
+      float up[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(v[i], 32, 64);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = gated_value(v[i], up[i], rotary.act, rotary.limit, rotary.slope, rotary.up_shift);
+      if (g < 2 && at_row < M) store_four(y + static_cast<int64_t>(at_row) * half, 8 * block + 4 * g, half, v);
+    } else if constexpr (MODE == PK_ROTARY) {
+      store_rotary(v, at_row, at_row < M, g, block, bias, y, N, rotary);
+    } else {
+      const int n0 = 16 * block + 4 * g;
+      if (bias != nullptr && blockIdx.y == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += n0 + i < N ? bias[n0 + i] : 0.f;
+      }
+      if (at_row < M) store_four(y + (static_cast<int64_t>(blockIdx.y) * M + at_row) * N, n0, N, v);
+    }
+  }
+}
+
+// Slices of K: workgroups for every compute unit several times over, each at least three steps long.
+void rows_plan(int row_blocks, int K, int* slices, int* steps) {
+  const int all = K / RF_STEP;
+  int want = 1;
+  while (want < 16 && row_blocks * want < 640 && all / (want * 2) >= 3) want *= 2;
+  *steps = (all + want - 1) / want;
+  *slices = (all + *steps - 1) / *steps;
+}
+
+template <int MODE, int WAVES>
+int launch_rows_f32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int row_blocks, int slices,
+                    int steps, const RotaryOut& rotary, hipStream_t stream) {
+  const dim3 grid(row_blocks, slices);
+#define ROWS(MB) rows_f32_kernel<MB, MODE, WAVES><<<grid, 64 * WAVES, 0, stream>>>(x, w, bias, y, M, N, K, steps, rotary)
+  if (M <= 16) ROWS(1);
+  else ROWS(2);
+#undef ROWS
+  return launch_status();
+}
+
+bool takes(int M, int N, int K) { return M <= 32 && N >= 1 && K >= RF_STEP && K % RF_STEP == 0; }
+
+}  // namespace
+
+// How many slices distie_rows_f32 writes for this weight (0: it does not take it). `whole`: not to be cut.
+extern "C" int distie_rows_f32_slices(int M, int N, int K, int whole) {
+  if (!takes(M, N, K)) return 0;
+  int slices = 1, steps;
+  if (!whole) rows_plan((N + 15) / 16, K, &slices, &steps);
+  return slices;
+}
+
+// mode 0: y [M, N], or [slices, M, N] if the plan cuts K; 1 | (activation << 8): gated, [M, N / 2] (limit, slope, up_shift:
+// of the clamped activation, 5); both as the products on packed copies. Up to 32 rows of x.
+extern "C" int distie_rows_f32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int mode,
+                               int slices, float limit, float slope, float up_shift, hipStream_t stream) {
+  if (M <= 0) return 0;
+  const int act = mode >> 8;
+  mode &= 0xff;
+  if (!takes(M, N, K) || mode > 1 || (mode == 1 && (N % 2 != 0 || bias != nullptr || slices != 1)) || act < 0 || act > 5 ||
+      (act == 5 && !(limit > 0.f)) || slices < 1)
+    return DISTIE_BAD_ARGUMENT;
+  RotaryOut none = {};
+  none.act = act, none.limit = limit, none.slope = slope, none.up_shift = up_shift;
+  const int all = K / RF_STEP, steps = (all + slices - 1) / slices;
+  if ((all + steps - 1) / steps != slices) return DISTIE_BAD_ARGUMENT;
+  if (mode == 1) {
+    const int blocks = (N / 2 + 7) / 8;
+    if (blocks < 2048) return launch_rows_f32<PK_GATED, 4>(x, w, nullptr, y, M, N, K, blocks, 1, all, none, stream);
+    return launch_rows_f32<PK_GATED, 1>(x, w, nullptr, y, M, N, K, blocks, 1, all, none, stream);
+  }
+  const int blocks = (N + 15) / 16;
+  if (slices == 1 && blocks < 1024) return launch_rows_f32<PK_PLAIN, 4>(x, w, bias, y, M, N, K, blocks, 1, all, none, stream);
+  return launch_rows_f32<PK_PLAIN, 1>(x, w, bias, y, M, N, K, blocks, slices, steps, none, stream);
+}
+
+// The stacked q/k/v product with bias, rotation and cache write: w [(heads + 2 kv_heads) * dim, K] as stored, table
+// [M, dim / 2] (cos, sin), y [M, N] and the caches in float32.
+extern "C" int distie_rows_f32_rotary(const float* x, const float* w, const float* bias, float* y, const void* table,
+                                      const int32_t* slots, void* k_cache, void* v_cache, int M, int K, int heads, int kv_heads,
+                                      int dim, int block_size, int write, hipStream_t stream) {
+  if (M <= 0) return 0;
+  const int N = (heads + 2 * kv_heads) * dim;
+  if (!takes(M, N, K) || heads < 1 || kv_heads < 1 || dim < 16 || dim % 16 != 0 || block_size < 1 || table == nullptr ||
+      (write && (slots == nullptr || k_cache == nullptr || v_cache == nullptr)))
+    return DISTIE_BAD_ARGUMENT;
+  const RotaryOut rotary = {static_cast<const float2*>(table), slots, static_cast<bf16_t*>(k_cache),
+                            static_cast<bf16_t*>(v_cache), heads, kv_heads, dim, block_size, write};
+  const int all = K / RF_STEP;
+  if (all >= 16) return launch_rows_f32<PK_ROTARY, 8>(x, w, bias, y, M, N, K, N / 16, 1, all, rotary, stream);
+  return launch_rows_f32<PK_ROTARY, 4>(x, w, bias, y, M, N, K, N / 16, 1, all, rotary, stream);
+}

@@ -152,6 +152,8 @@ class HipOps(Ops):
     # float32 products (and products against weights kept in float32) of up to ROWS_MAX_ROWS rows stream the weights
     # through `gemv_rows` (FMAs on the vector ALU); beyond that the tiled float32 kernel
     ROWS_MAX_ROWS = 64
+    ROWS_F32_FEW = 4
+    ROWS_F32_LARGE_ELEMENTS = 8 << 20
     # bfloat16 products by rows of x: up to SKINNY_MAX_ROWS the weights are streamed by one wave per block
     # of 16 weight rows, x straight from memory (above that, the library's tiles are faster);
     SKINNY_MAX_ROWS = 16
@@ -327,6 +329,9 @@ class HipOps(Ops):
         o.distie_gather_rows.argtypes = [_P, _P, _P, _I, _L, _I, _P]
         o.distie_gemm_generic.argtypes = [_P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _P]
         o.distie_gemv_rows.argtypes = [_P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _P]
+        o.distie_rows_f32_slices.argtypes = [_I, _I, _I, _I]
+        o.distie_rows_f32.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _F, _P]
+        o.distie_rows_f32_rotary.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_skinny_slices.argtypes = [_I, _I, _I]
         o.distie_gemm_skinny_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _P]
         o.distie_pack_rows.argtypes = [_P, _P, _P, _I, _I, _P]
@@ -420,7 +425,8 @@ class HipOps(Ops):
                 raise KernelError(f"attention kernels take even head sizes up to {self.LARGEST_HEAD}, not {head_dim}")
             lib = ctypes.CDLL(str(build.ensure(f"attn_d{head_dim}")))
             lib.distie_attention_generic.argtypes = [_P, _I, _L, _P, _P, _I, _P, _P, _P, _I, _P, _P,
-                                                     _I, _I, _I, _I, _F, _I, _P, _F, _P, _P]
+                                                     _I, _I, _I, _I, _F, _I, _P, _F, _P, _P, _P, _I, _P]
+            lib.distie_attention_f32_runs.argtypes = [_I, _I, _I, _I]
             lib.distie_attention_prefill_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I,
                                                           _F, _I, _I, _P, _P, _P, _I, _P, _P]
             lib.distie_attention_prefill_f32.argtypes = lib.distie_attention_prefill_bf16.argtypes
@@ -671,6 +677,15 @@ class HipOps(Ops):
             out = torch.empty((x.shape[0], N // 2), dtype=torch.bfloat16, device=self.device)
             return self._norm_product(x, packed, None, out, gated, N)
         x = self.dense(x)
+        M, K = x.shape
+        N = gate_up_weight.shape[0]
+        if x.dtype == torch.float32 and gate_up_weight.dtype == torch.float32 and gate_up_weight.shape[1] == K and N % 2 == 0 and \
+                self._ops.distie_rows_f32_slices(M, N, K, 1):
+            self._own(x, gate_up_weight)
+            out = torch.empty((M, N // 2), dtype=torch.float32, device=self.device)
+            _check(self._ops.distie_rows_f32(x.data_ptr(), gate_up_weight.data_ptr(), None, out.data_ptr(), M, N, K, gated, 1,
+                                             *clamp, self._stream()), "rows_f32")
+            return out
         plan = None
         if packed is not None and x.dtype == torch.bfloat16:
             plan = self._tiles(x.shape[0], *gate_up_weight.shape, "gated")
@@ -678,8 +693,6 @@ class HipOps(Ops):
                 (plan is None and x.shape[0] > self._packed_rows(x.shape[0], *gate_up_weight.shape)):
             return apart(self.linear(x, gate_up_weight))
         self._own(x)
-        M, K = x.shape
-        N = gate_up_weight.shape[0]
         if gate_up_weight.shape[1] != K:
             raise KernelError(f"linear: x is [{M}, {K}], weight is {list(gate_up_weight.shape)}")
         if packed.numel() != self._packed_elements(N, K, True):
@@ -721,6 +734,25 @@ class HipOps(Ops):
             return self._norm_product(x, packed, bias, out, 2, N, rotary=(
                 table, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, meta.block_size, 1 if write else 0))
         x = self.dense(x)
+        M, K = x.shape
+        N = weight.shape[0]
+        if x.dtype == torch.float32 and weight.dtype == torch.float32 and k_cache.dtype == torch.float32 and \
+                inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and head_dim % 16 == 0 and \
+                N == (num_heads + 2 * num_kv_heads) * head_dim and weight.shape[1] == K and \
+                (bias is None or (bias.dtype == torch.float32 and bias.shape[0] == N)) and \
+                self._ops.distie_rows_f32_slices(M, N, K, 1):
+            slots = meta.groups[group].slots
+            self._own(x, weight, bias, k_cache, v_cache, inv_freq, slots)
+            self._check_cache(k_cache, v_cache, num_kv_heads, meta.block_size, head_dim)
+            if M != meta.num_tokens or slots.shape[0] != M:
+                raise KernelError("linear_rope_kv_write: rows do not match the batch")
+            table = self._rope_table(meta, inv_freq)
+            out = torch.empty((M, N), dtype=torch.float32, device=self.device)
+            _check(self._ops.distie_rows_f32_rotary(
+                x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads, num_kv_heads,
+                head_dim, meta.block_size, 1 if write else 0, self._stream()), "rows_f32_rotary")
+            return out
         plan = None
         fused = held is not None and held[1] == (num_heads, num_kv_heads, head_dim) and x.dtype == torch.bfloat16 and \
             inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and k_cache.dtype == torch.bfloat16
@@ -1010,6 +1042,19 @@ class HipOps(Ops):
             out = self._library_linear(x, weight, bias, out_dtype)
             if out is not None:
                 return out
+        if both_f32 and partial_ok:
+            # few rows in the true 32-bit path, for a caller that takes slices (the head's product does not, and runs at 5
+            # TB/s as it is): the weights streamed through the matrix cores' float32 products. At up to ROWS_F32_FEW rows a
+            # small weight is faster on the vector ALU (one row against [1536, 1536] 4.4 us, 6.1 here)
+            slices = 0
+            if M > self.ROWS_F32_FEW or N * K >= self.ROWS_F32_LARGE_ELEMENTS:
+                slices = self._ops.distie_rows_f32_slices(M, N, K, 0)
+            if slices:
+                out = torch.empty((M, N) if slices == 1 else (slices, M, N), dtype=torch.float32, device=self.device)
+                _check(self._ops.distie_rows_f32(
+                    x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), M, N, K,
+                    0, slices, 0.0, 1.0, 0.0, self._stream()), "rows_f32")
+                return out if slices == 1 else PartialSums(out, out_dtype)
         out = torch.empty((M, N), dtype=out_dtype, device=self.device)
         if M <= self.ROWS_MAX_ROWS and K % 8 == 0:
             # few rows in float32 (or against a weight kept in float32): the weights are streamed, FMAs only
@@ -1168,11 +1213,26 @@ class HipOps(Ops):
                 plan["prefill_ml"].data_ptr() if parts > 1 else None, parts, sinks_ptr, self._stream()),
                 "attention_prefill_f32")
             return out
+        part_o = part_ml = None
+        runs = 1
+        if plain and f32:
+            # requests that decode in float32: the keys of a token are cut into runs of at least 256 that run side by
+            # side, so that few requests occupy the chip as well
+            runs = lib.distie_attention_f32_runs(T, num_heads, num_kv_heads, min(meta.max_kv, abs(reach) or meta.max_kv))
+            if runs > 1:
+                key = ("attention_f32_runs", runs, num_heads, head_dim)
+                held = meta.scratch.get(key)
+                if held is None:
+                    held = meta.scratch[key] = (
+                        torch.empty((runs, T, num_heads, head_dim), dtype=torch.float32, device=self.device),
+                        torch.empty((runs, T, num_heads, 2), dtype=torch.float32, device=self.device))
+                part_o, part_ml = held
         _check(lib.distie_attention_generic(
             qkv.data_ptr(), _code(qkv), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
             meta.positions.data_ptr(), meta.token_request.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr,
             out.data_ptr(), T, num_heads, num_kv_heads, meta.block_size, float(scale), reach,
-            slopes.data_ptr() if slopes is not None else None, cap, sinks_ptr, self._stream()), "attention_generic")
+            slopes.data_ptr() if slopes is not None else None, cap, sinks_ptr, part_o.data_ptr() if runs > 1 else None,
+            part_ml.data_ptr() if runs > 1 else None, runs, self._stream()), "attention_generic")
         return out
 
     def _mixed_attention(self, q, meta: BatchMeta, table, rows_ptr, k_cache, v_cache, out, num_heads, num_kv_heads, head_dim,

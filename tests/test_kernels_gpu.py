@@ -131,6 +131,52 @@ def test_products_of_few_rows_in_float32_stream_the_weights(ops, xd, wd, M, N, K
                                      65, N, K, None) == -1                     # more rows than it takes: refused
 
 
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 64), (102, 128), (250, 320), (1030, 1088), (96, 8960)])
+def test_float32_products_of_few_rows_on_the_matrix_cores(ops, M, N, K):
+    """Plain in every number of slices, gated, and q/k/v with rotation and cache write: rows that do not fill a block of 16,
+    fewer steps than are loaded together and more, odd and even. The sums are float32 and no further from those in 64 bits
+    than the vector ALU's kernel's (a quarter more is allowed for the difference of two samples)."""
+    x, w, b = rand(M, K, seed=1), rand(N, K, seed=2), rand(N, seed=3)
+    want = x.double() @ w.double().T
+    off = lambda y, z: ((y.double() - z).norm() / z.norm()).item()
+    plain = torch.empty(M, N, device="cuda")
+    assert ops._ops.distie_gemv_rows(x.data_ptr(), 0, w.data_ptr(), 0, None, plain.data_ptr(), 0, M, N, K, None) == 0
+    steps = K // 64
+    for slices in (1, 2, 3, 5, 16):
+        out = torch.empty(slices, M, N, device="cuda")
+        rc = ops._ops.distie_rows_f32(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, 0, slices,
+                                      0.0, 1.0, 0.0, None)
+        assert (rc == 0) == (-(-steps // -(-steps // slices)) == slices)
+        if rc == 0:
+            close(out.sum(0), want + b.double(), torch.float32, scale=5 * want.abs().max().item())
+            assert off(out.sum(0) - b, want) <= 1.25 * off(plain, want) + 1e-7
+    gate, up = want[:, :N // 2], want[:, N // 2:]
+    got = ops.linear_silu_mul(x, w)
+    assert got.dtype == torch.float32
+    wanted = gate / (1 + torch.exp(-gate)) * up
+    close(got, wanted, torch.float32, scale=5 * wanted.abs().max().item())
+    gate, up = gate.clamp(max=0.7), up.clamp(-0.7, 0.7)
+    wanted = gate / (1 + torch.exp(-1.702 * gate)) * (up + 1)
+    close(ops.linear_clamped_glu(x, w, 0.7, 1.702, 1.0), wanted, torch.float32, scale=5 * wanted.abs().max().item())
+    assert ops._ops.distie_rows_f32(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), 33, N, K, 0, 1, 0.0, 1.0, 0.0, None) == -1
+    heads, kv_heads, dim, P = 3, 1, 32, 4
+    w, b = rand((heads + 2 * kv_heads) * dim, K, seed=6, scale=K ** -0.5), rand((heads + 2 * kv_heads) * dim, seed=7)
+    slots = [(7 * i) % 61 for i in range(M)]
+    meta = make_meta([11 * i for i in range(M)], list(range(M)), list(range(M + 1)), [11 * i + 1 for i in range(M)],
+                     [[0] * 8] * M, slots, P)
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, dim, 2, dtype=torch.float32) / dim))).cuda()
+    k1, v1 = rand(16, kv_heads, P, dim, seed=8), rand(16, kv_heads, dim, P, seed=9)
+    k2, v2 = k1.clone(), v1.clone()
+    dense = (x.double() @ w.double().T + b.double()).float()
+    wanted = TorchOps("cuda").rope_kv_write(dense, meta, 0, k2, v2, inv_freq, heads, kv_heads, dim, True)
+    got = ops.linear_rope_kv_write(x, w, b, meta, 0, k1, v1, inv_freq, heads, kv_heads, dim, True)
+    scale = 5 * wanted.abs().max().item()
+    close(got, wanted, torch.float32, scale=scale)
+    close(k1, k2, torch.float32, scale=scale)
+    close(v1, v2, torch.float32, scale=scale)
+
+
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(48, 128), (100, 264), (1536, 1536), (333, 8960), (2050, 72)])
 def test_gemm_skinny_bf16(ops, M, N, K):
@@ -848,6 +894,28 @@ def test_paged_attention_decode_step(ops, dtype, heads, kv_heads, dim, P, window
         meta.max_kv = limit
         got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window)
         close(got, want, dtype, scale=want.abs().max().item())
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(12, 2, 128, 16, None), (8, 1, 256, 16, None), (7, 1, 32, 32, 300),
+                                                         (4, 4, 64, 8, None), (2, 1, 64, 4, 65)])
+@pytest.mark.parametrize("runs", [1, 2, 3, 16])
+def test_float32_decode_keys_in_runs(ops, heads, kv_heads, dim, P, window, runs, monkeypatch):
+    """The float32 kernel of requests that decode, its keys cut into runs: requests of one key, of a chunk of 64 and one
+    more, runs that hold no chunk, sinks that count once, and buffers that held NaN before."""
+    from distie_amd.kernels.interface import ScoreExtras
+
+    lens = [1, 64, 65, 130, 257, 700, 1100]
+    meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, [1] * len(lens), torch.float32, seed=21)
+    monkeypatch.setattr(ops.attention_library(dim), "distie_attention_f32_runs", lambda *sizes: runs)
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: empty(*a, **kw).fill_(float("nan"))
+                        if kw.get("dtype") == torch.float32 else empty(*a, **kw))
+    for sinks in (None, rand(heads, seed=22)):
+        extras = None if sinks is None else ScoreExtras(sinks=sinks)
+        want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, k.double(), v.double(), heads, kv_heads, dim,
+                                                dim ** -0.5, window, extras)
+        got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window, extras)
+        close(got, want, torch.float32, scale=want.abs().max().item())
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,P", [(12, 2, 128, 16), (4, 2, 64, 16), (3, 1, 48, 16), (2, 1, 256, 32)])
