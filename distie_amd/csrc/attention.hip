@@ -675,14 +675,15 @@ extern "C" int distie_attention_decode_run_len(const int32_t* kv_len, int num_re
 // instead of 1,024, and a batch whose runs are a few more than 1,024, or whose requests differ in length, no
 // longer waits for the last waves to get a place: 7B shape's heads at 2,100 keys, 96 requests 91 -> 83 us a layer,
 // 160 requests 165 -> 130; contexts of 1,050 to 3,150 keys, 96 requests 121 -> 96, 160 requests 222 -> 157.
-template <int MB>
-__global__ __launch_bounds__(DISTIE_WAVE, (MB == 1 && D <= 128 ? 2 : 1)) void attn_decode_kernel(
+template <int MB, int W>
+__global__ __launch_bounds__(DISTIE_WAVE * W, (MB == 1 && D <= 128 ? 2 : 1)) void attn_decode_kernel(
     const bf16_t* __restrict__ qkv, int64_t q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ kv_len, const int32_t* __restrict__ cu_q,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ table_rows, float* __restrict__ part_o,
     float* __restrict__ part_ml, int heads, int kv_heads, int block_size, float scale, int window, int split_hint,
     int max_splits, int dense_rows, const int32_t* __restrict__ shared_run_len) {
-  const int lane = threadIdx.x;
+  const int lane = W > 1 ? threadIdx.x % DISTIE_WAVE : threadIdx.x;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / DISTIE_WAVE) : 0;
   const int r = lane % 16;
   const int g = lane / 16;
   const int group = heads / kv_heads;
@@ -691,7 +692,8 @@ __global__ __launch_bounds__(DISTIE_WAVE, (MB == 1 && D <= 128 ? 2 : 1)) void at
   // waves leave at once, then come after all the others (in front of them they held the places on the SIMDs that
   // the working waves behind them were waiting for: 64 requests took 106 us instead of 54, at one wave a SIMD).
   const bool shared = shared_run_len != nullptr;
-  const int run = shared ? blockIdx.z : blockIdx.x;
+  const int share = shared ? blockIdx.z : blockIdx.x;        // the runs W share .. W share + W - 1, one a wave
+  const int run = W * share + wave;
   const int request = shared ? blockIdx.y : blockIdx.z;
   const int kh = shared ? blockIdx.x : blockIdx.y;
   const int32_t* table = block_table + static_cast<int64_t>(table_rows != nullptr ? table_rows[request] : request) * table_width;
@@ -709,10 +711,11 @@ __global__ __launch_bounds__(DISTIE_WAVE, (MB == 1 && D <= 128 ? 2 : 1)) void at
   if (!dense_rows && cu_q[request + 1] - token != 1) return;        // a portion of a prompt: the tiled kernel's
   const int q_pos = kv_len[request] - 1;              // the new token is the last one cached
   const KeyRuns runs = key_runs(q_pos, window, max_splits, run_len);
-  if (run >= runs.count) return;
+  if (W * share >= runs.count) return;
   const int run_begin = runs.origin + run * runs.length;
   const int key_begin = max(runs.first, run_begin);
-  const int key_end = min(q_pos, run_begin + runs.length - 1);
+  // (a wave past the last run has no key)
+  const int key_end = W == 1 || run < runs.count ? min(q_pos, run_begin + runs.length - 1) : -1;
 
   // ---- the query of this lane's column (head kh * G + 16 mb + r; columns past the group repeat the last)
   bf16x8 q_reg[MB][DK32 > 0 ? DK32 : 1];
@@ -867,6 +870,11 @@ __global__ __launch_bounds__(DISTIE_WAVE, (MB == 1 && D <= 128 ? 2 : 1)) void at
     l_run[mb] += __shfl_xor(l_run[mb], 16, DISTIE_WAVE);
     l_run[mb] += __shfl_xor(l_run[mb], 32, DISTIE_WAVE);
   }
+  const int places = (max_splits + W - 1) / W;                  // for partial results, per request and head
+  const int64_t head0 = static_cast<int64_t>(request) * heads + kh * group;
+  // W > 1: sums [W][group][D], then maxima and sums of weights [W][group][2]
+  extern __shared__ __attribute__((aligned(16))) float decode_lds[];
+  float* ml_lds = decode_lds + W * group * D;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -875,15 +883,44 @@ __global__ __launch_bounds__(DISTIE_WAVE, (MB == 1 && D <= 128 ? 2 : 1)) void at
       const float l_col = __shfl(l_run[mb], 4 * g + i, DISTIE_WAVE);
       const float m_col = __shfl(m_run[mb], 4 * g + i, DISTIE_WAVE);
       if (col >= group) continue;
-      const int64_t slot = (static_cast<int64_t>(request) * heads + kh * group + col) * max_splits + run;
-      float* po = part_o + slot * D;
+      const int64_t slot = W > 1 ? wave * group + col : (head0 + col) * max_splits + run;
+      float* po = (W > 1 ? decode_lds : part_o) + slot * D;
+      float* ml = (W > 1 ? ml_lds : part_ml) + 2 * slot;
 #pragma unroll
       for (int db = 0; db < DB16; ++db) po[16 * db + r] = o_acc[mb][db][i];
       if (r == 0) {
-        part_ml[2 * slot] = m_col;
-        part_ml[2 * slot + 1] = l_col;
+        ml[0] = m_col;
+        ml[1] = l_col;
       }
     }
+  if constexpr (W > 1) {
+    // the workgroup's runs in their order, four dims of a column a thread
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < group * (D / 4); idx += DISTIE_WAVE * W) {
+      const int col = idx / (D / 4), d = 4 * (idx % (D / 4));
+      float m = -INFINITY;
+#pragma unroll
+      for (int v = 0; v < W; ++v) m = fmaxf(m, ml_lds[2 * (v * group + col)]);      // finite: the first wave holds a key
+      float l = 0.f;
+      float4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int v = 0; v < W; ++v) {
+        const float weight = fast_exp2(ml_lds[2 * (v * group + col)] - m);        // 0 for a wave without a key, whose sums are 0
+        l = fmaf(weight, ml_lds[2 * (v * group + col) + 1], l);
+        const float4 o = *reinterpret_cast<const float4*>(decode_lds + (v * group + col) * D + d);
+        sum.x = fmaf(weight, o.x, sum.x);
+        sum.y = fmaf(weight, o.y, sum.y);
+        sum.z = fmaf(weight, o.z, sum.z);
+        sum.w = fmaf(weight, o.w, sum.w);
+      }
+      const int64_t slot = (head0 + col) * places + share;
+      *reinterpret_cast<float4*>(part_o + slot * D + d) = sum;
+      if (d == 0) {
+        part_ml[2 * slot] = m;
+        part_ml[2 * slot + 1] = l;
+      }
+    }
+  }
 }
 
 // Combines the partial results of the runs of keys of one (request, head): grid (heads, requests), four waves.
@@ -902,8 +939,9 @@ constexpr int RD_FAST_RUNS = RD_FAST_PER_WAVE * RD_WAVES;
 template <bool FAST>
 __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ kv_len,
-    const int32_t* __restrict__ cu_q, bf16_t* __restrict__ out, int heads, int window, int max_splits,
+    const int32_t* __restrict__ cu_q, bf16_t* __restrict__ out, int heads, int window, int all_splits, int together,
     int dense_rows, const int32_t* __restrict__ shared_run_len, const float* __restrict__ sinks) {
+  const int max_splits = (all_splits + together - 1) / together;      // places: the runs of a workgroup share one
   __shared__ float weight_s[FAST ? RD_FAST_RUNS : RD_MAX_RUNS];
   __shared__ float sum_s[RD_WAVES][D];
   __shared__ float scratch[32];
@@ -932,7 +970,8 @@ __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
   const int token = dense_rows ? request : cu_q[request];
   if (!dense_rows && cu_q[request + 1] - token != 1) return;
   const int q_pos = kv_len[request] - 1;
-  const int runs = key_runs(q_pos, window, max_splits, shared_run_len != nullptr ? *shared_run_len : 0).count;     // the first `runs` places hold results
+  const int all_runs = key_runs(q_pos, window, all_splits, shared_run_len != nullptr ? *shared_run_len : 0).count;
+  const int runs = (all_runs + together - 1) / together;     // the first `runs` places hold results
   const int64_t base = base0;
   bf16_t* o = out + (static_cast<int64_t>(token) * heads + head) * D;
   // a sink: one more maximum and one more term of the denominator, in the runs' units of log 2; it has no value
@@ -1016,6 +1055,20 @@ __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
   }
 }
 
+// How many consecutive runs a workgroup puts together, one a wave. 1 as a rule: waves of their own spread best over the
+// chip (8 of them in a workgroup read through one CU: 28 layers, 12 heads on 2, 1 request of 500 keys 1,442 -> 1,537 us,
+// 8 of 2,048 keys 1,577 -> 1,645, 64 of 2,048 keys 2,580 -> 2,640). More than RD_FAST_RUNS partial results, though, cost the
+// reduce 8.9 us a layer instead of 4.6, trip after trip to memory: put together by 8 they fit it (4 requests of 16,000
+// keys 1,861 -> 1,788 us; by 4, which is for heads whose sums would fill the LDS, some 18 us more).
+constexpr size_t DECODE_LDS = 64 * 1024;
+constexpr int DECODE_MOST_TOGETHER = D <= 128 ? 8 : 4;        // more than 256 registers a wave: one wave a SIMD
+extern "C" int distie_attention_decode_together(int max_splits, int group) {
+  if (max_splits <= RD_FAST_RUNS || group > 16) return 1;
+  for (int together = DECODE_MOST_TOGETHER; together >= 4; together /= 2)
+    if (static_cast<size_t>(together) * group * (D + 2) * sizeof(float) <= DECODE_LDS) return together;
+  return 1;
+}
+
 constexpr int DECODE_MAX_MB = (D <= 128) ? 4 : 2;   // registers: the output tile is 16 * MB x D floats a wave
 
 // most query heads per kv head the decode kernel takes
@@ -1032,7 +1085,8 @@ extern "C" int distie_attention_decode_bf16(const void* qkv, int64_t q_stride, c
                                             int table_width, const int32_t* table_rows, void* out, float* part_o, float* part_ml,
                                             int num_requests, int heads, int kv_heads, int block_size, float scale,
                                             int window, int split_hint, int max_splits, int dense_rows,
-                                            const int32_t* shared_run_len, const float* sinks, hipStream_t stream) {
+                                            const int32_t* shared_run_len, const float* sinks, int together,
+                                            hipStream_t stream) {
   if (num_requests <= 0) return 0;
   const int group = kv_heads > 0 ? heads / kv_heads : 0;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || block_size % 16 != 0 || table_width < 1 ||
@@ -1040,32 +1094,40 @@ extern "C" int distie_attention_decode_bf16(const void* qkv, int64_t q_stride, c
       group > 16 * DECODE_MAX_MB || kv_heads > 65535 || num_requests > 65535 || heads > 65535 ||
       (shared_run_len != nullptr && (window != 0 || !dense_rows)))
     return DISTIE_BAD_ARGUMENT;
-  const dim3 grid = shared_run_len != nullptr ? dim3(kv_heads, num_requests, max_splits) : dim3(max_splits, kv_heads, num_requests);
+  const size_t lds = together > 1 ? static_cast<size_t>(together) * group * (D + 2) * sizeof(float) : 0;
+  if ((together != 1 && together != 4 && together != DECODE_MOST_TOGETHER) || (together > 1 && group > 16) || lds > DECODE_LDS)
+    return DISTIE_BAD_ARGUMENT;
+  const int places = (max_splits + together - 1) / together;
+  const dim3 grid = shared_run_len != nullptr ? dim3(kv_heads, num_requests, places) : dim3(places, kv_heads, num_requests);
   const bf16_t* q = static_cast<const bf16_t*>(qkv);
   const bf16_t* kc = static_cast<const bf16_t*>(k_cache);
   const bf16_t* vc = static_cast<const bf16_t*>(v_cache);
-#define DECODE_LAUNCH(MB)                                                                                             \
-  attn_decode_kernel<MB><<<grid, DISTIE_WAVE, 0, stream>>>(q, q_stride, kc, vc, kv_len, cu_q, block_table, table_width, table_rows, \
-                                                           part_o, part_ml, heads, kv_heads, block_size, scale, window, \
-                                                           split_hint, max_splits, dense_rows, shared_run_len)
-  if (group <= 16) {
-    DECODE_LAUNCH(1);
+#define DECODE_LAUNCH(MB, W)                                                                                          \
+  attn_decode_kernel<MB, W><<<grid, DISTIE_WAVE * W, lds, stream>>>(                                                   \
+      q, q_stride, kc, vc, kv_len, cu_q, block_table, table_width, table_rows, part_o, part_ml, heads, kv_heads, block_size, \
+      scale, window, split_hint, max_splits, dense_rows, shared_run_len)
+  if (together == 4) {
+    DECODE_LAUNCH(1, 4);
+  } else if (together > 1) {
+    DECODE_LAUNCH(1, DECODE_MOST_TOGETHER);
+  } else if (group <= 16) {
+    DECODE_LAUNCH(1, 1);
   } else if (group <= 32) {
-    DECODE_LAUNCH(2);
+    DECODE_LAUNCH(2, 1);
   } else {
-    DECODE_LAUNCH(DECODE_MAX_MB);
+    DECODE_LAUNCH(DECODE_MAX_MB, 1);
   }
 #undef DECODE_LAUNCH
   int status = launch_status();
   if (status != 0) return status;
-  if (max_splits <= RD_FAST_RUNS) {
+  if (places <= RD_FAST_RUNS) {
     attn_reduce_kernel<true><<<dim3(heads, num_requests), RD_THREADS, 0, stream>>>(
-        part_o, part_ml, kv_len, cu_q, static_cast<bf16_t*>(out), heads, window, max_splits, dense_rows, shared_run_len,
-        sinks);
+        part_o, part_ml, kv_len, cu_q, static_cast<bf16_t*>(out), heads, window, max_splits, together, dense_rows,
+        shared_run_len, sinks);
   } else {
     attn_reduce_kernel<false><<<dim3(heads, num_requests), RD_THREADS, 0, stream>>>(
-        part_o, part_ml, kv_len, cu_q, static_cast<bf16_t*>(out), heads, window, max_splits, dense_rows, shared_run_len,
-        sinks);
+        part_o, part_ml, kv_len, cu_q, static_cast<bf16_t*>(out), heads, window, max_splits, together, dense_rows,
+        shared_run_len, sinks);
   }
   return launch_status();
 }
@@ -1805,9 +1867,11 @@ extern "C" int distie_attention_decode_columns() { return 0; }
 
 extern "C" int distie_attention_decode_bf16(const void*, int64_t, const void*, const void*, const int32_t*, const int32_t*,
                                             const int32_t*, int, const int32_t*, void*, void*, void*, int, int, int, int, float, int, int,
-                                            int, int, const int32_t*, const float*, hipStream_t) {
+                                            int, int, const int32_t*, const float*, int, hipStream_t) {
   return DISTIE_BAD_ARGUMENT;
 }
+
+extern "C" int distie_attention_decode_together(int, int) { return 1; }
 
 extern "C" int distie_attention_decode_run_len(const int32_t*, int, int, int, int32_t*, hipStream_t) { return DISTIE_BAD_ARGUMENT; }
 

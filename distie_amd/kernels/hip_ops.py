@@ -431,7 +431,8 @@ class HipOps(Ops):
                                                           _F, _I, _I, _P, _P, _P, _I, _P, _P]
             lib.distie_attention_prefill_f32.argtypes = lib.distie_attention_prefill_bf16.argtypes
             lib.distie_attention_decode_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I,
-                                                         _I, _F, _I, _I, _I, _I, _P, _P, _P]
+                                                         _I, _F, _I, _I, _I, _I, _P, _P, _I, _P]
+            lib.distie_attention_decode_together.argtypes = [_I, _I]
             lib.distie_attention_decode_run_len.argtypes = [_P, _I, _I, _I, _P, _P]
             if lib.distie_attention_head_dim() != head_dim:
                 raise KernelError("attention library was built for another head size")
@@ -1182,8 +1183,8 @@ class HipOps(Ops):
                     plan["decode_o"].data_ptr(), plan["decode_ml"].data_ptr(), meta.num_requests, num_heads,
                     num_kv_heads, meta.block_size, float(scale), reach, plan["split_len"],
                     plan["max_splits"], 1 if meta.all_decode else 0,
-                    plan["run_len"].data_ptr() if plan["run_len"] is not None else None, sinks_ptr, self._stream()),
-                    "attention_decode_bf16")
+                    plan["run_len"].data_ptr() if plan["run_len"] is not None else None, sinks_ptr, plan["together"],
+                    self._stream()), "attention_decode_bf16")
             if plan["prefill"]:
                 parts = plan["parts"]
                 _check(lib.distie_attention_prefill_bf16(
@@ -1334,9 +1335,12 @@ class HipOps(Ops):
                                                            plan["run_len"].data_ptr(), self._stream()),
                        "attention_decode_run_len")
             plan["max_splits"] = max_splits
-            plan["decode_o"] = torch.empty((meta.num_requests, num_heads, max_splits, head_dim), dtype=torch.float32,
+            # many runs: a workgroup puts consecutive ones together before it writes their result
+            plan["together"] = together = lib.distie_attention_decode_together(max_splits, group)
+            places = -(-max_splits // together)
+            plan["decode_o"] = torch.empty((meta.num_requests, num_heads, places, head_dim), dtype=torch.float32,
                                            device=self.device)
-            plan["decode_ml"] = torch.empty((meta.num_requests, num_heads, max_splits, 2), dtype=torch.float32,
+            plan["decode_ml"] = torch.empty((meta.num_requests, num_heads, places, 2), dtype=torch.float32,
                                             device=self.device)
         plan["prefill"] = singles < meta.num_requests or not plan["decode"] or \
             (meta.singles_bound is not None and not meta.all_decode)

@@ -896,6 +896,29 @@ def test_paged_attention_decode_step(ops, dtype, heads, kv_heads, dim, P, window
         close(got, want, dtype, scale=want.abs().max().item())
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
+                                                                  (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8)])
+def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, window, together):
+    """Past 64 runs a request and head, the consecutive runs of a workgroup are put together before their result is
+    written: a last workgroup with one, some and all of its runs, a request with one key, one that brings a portion (the
+    tiled kernel's), a head with a sink, and places sized for far longer requests. Against plain attention."""
+    from distie_amd.kernels.interface import ScoreExtras
+
+    for lens, q_lens in (([4161, 1, 4609, 5120], [1] * 4), ([4700, 70, 513], [1, 3, 1])):
+        meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.bfloat16, seed=7)
+        sinks = torch.randn(heads, device="cuda")
+        for extras in (None, ScoreExtras(sinks=sinks)):
+            want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, k.double(), v.double(), heads, kv_heads, dim,
+                                                    dim ** -0.5, window, extras)
+            for limit in (max(lens), 16384):
+                meta.max_kv = limit
+                meta.scratch.clear()
+                got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window, extras)
+                plans = [plan for plan in meta.scratch.values() if isinstance(plan, dict) and plan.get("decode")]
+                assert [plan["together"] for plan in plans] == [together] and plans[0]["max_splits"] > 64
+                close(got, want, torch.bfloat16, scale=want.abs().max().item())
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(12, 2, 128, 16, None), (8, 1, 256, 16, None), (7, 1, 32, 32, 300),
                                                          (4, 4, 64, 8, None), (2, 1, 64, 4, 65)])
 @pytest.mark.parametrize("runs", [1, 2, 3, 16])
