@@ -896,6 +896,26 @@ def test_paged_attention_decode_step(ops, dtype, heads, kv_heads, dim, P, window
         close(got, want, dtype, scale=want.abs().max().item())
 
 
+@pytest.mark.parametrize("T", [17, 64, 205, 700])
+@pytest.mark.parametrize("H,N,K,lx,lo", [(8, 192, 128, 192, 256), (8, 128, 192, 256, 128), (3, 17, 36, 40, 20), (1, 1, 4, 4, 1),
+                                         (16, 100, 60, 64, 100), (2, 33, 30, 31, 33)])
+def test_float32_products_for_every_head(ops, T, H, N, K, lx, lo):
+    """A product for every head in float32 (the matrix-core kernel in its three tiles, ends of tiles in rows, columns and k;
+    the last size and an input off 16 bytes keep the tiled kernel) against 64 bits: sums in four chains of at most K / 16
+    steps of four products, then two additions, so within (K / 16 + 6) roundings of 2^-24 of the sum of the products'
+    sizes; the plain kernel's one chain has K."""
+    x = torch.randn(T, H * lx, device="cuda")
+    w = torch.randn(H, N, K, device="cuda")
+    xk = x.view(T, H, lx)[:, :, :K].cpu()
+    want = torch.einsum("thk,hnk->thn", xk.double(), w.cpu().double())
+    size = torch.einsum("thk,hnk->thn", xk.double().abs(), w.cpu().double().abs())
+    shifted = torch.empty(x.numel() + 1, device="cuda")[1:].view_as(x).copy_(x)
+    for given, steps in ((x, K // 16 + 6 if K % 4 == 0 else K), (shifted, K)):
+        got = ops.heads_linear(given, w, lx, lo).cpu().view(T, H, lo)
+        assert ((got[:, :, :N].double() - want).abs() <= 4 * steps * 2.0 ** -24 * size).all()
+        assert (got[:, :, N:] == 0).all()
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
                                                                   (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8)])
 def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, window, together):
