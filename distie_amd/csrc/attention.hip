@@ -241,6 +241,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_generic_kernel(
 // eight waves a (token, head), 96 in all; 12.7 and 4.7 with three heads to a workgroup of four waves and four runs.
 constexpr bool GQ_FITS = D % 32 == 0;
 constexpr int GQ_SLICE = GQ_FITS ? D / 8 : 4;
+static bool grouped_fits(int64_t tokens, int heads) { return GQ_FITS && tokens * heads < 2048; }
 
 template <int G, int WAVES>
 __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
@@ -490,10 +491,268 @@ __global__ __launch_bounds__(DISTIE_WAVE) void attn_grouped_merge_kernel(const f
   }
 }
 
+// The same attention on the float32 matrix instruction (v_mfma_f32_16x16x4_f32), for any step: the 16 columns of a
+// product are the query heads of one kv head (at most 16 of them) for as many consecutive tokens of a request as fit, so a
+// row of K and of V^T is read once for all of them. A workgroup of four waves a (tile of tokens, kv head, run of keys): the
+// waves take chunks of CF_KEYS keys in turn, straight from the cache to registers (a lane's 16 bytes are its operand of four
+// products: of K's row `lane % 16`, of V^T's row of a dim `lane % 16`), K and V of a chunk asked for together. Scores are
+// summed over the head's dimensions in sixteen chains, values
+// in one for every 16 keys: no further from 64 bits than the vector kernels. The waves' results are put together in LDS, the runs' by
+// attn_grouped_merge_kernel.
+constexpr bool CF_FITS = D % 32 == 0 && D <= 256;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float cf_floatx4;
+constexpr int CF_WAVES = 4;
+constexpr int CF_BLOCKS = D <= 128 ? 4 : 2;               // of 16 keys a chunk: what the registers of one wave a SIMD hold
+constexpr int CF_KEYS = 16 * CF_BLOCKS;
+
+__global__ __launch_bounds__(DISTIE_WAVE * CF_WAVES, 1) void attn_columns_f32_kernel(
+    const float* __restrict__ qkv, int64_t q_stride, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ block_table,
+    int table_width, const int32_t* __restrict__ table_rows, float* __restrict__ out, int tokens, int num_requests, int heads,
+    int kv_heads, int block_size, float scale, int window, const float* __restrict__ sinks, float* __restrict__ part_o,
+    float* __restrict__ part_ml) {
+  if constexpr (CF_FITS) {
+  constexpr int DJ = D / 16;
+  __shared__ __attribute__((aligned(16))) float acc_s[CF_WAVES][16][D];
+  __shared__ float m_s[CF_WAVES][16], l_s[CF_WAVES][16];
+  const int lane = threadIdx.x % DISTIE_WAVE;
+  const int wave = threadIdx.x / DISTIE_WAVE;
+  const int r = lane % 16, g = lane / 16;
+  const int kh = blockIdx.y;
+  const int group = heads / kv_heads;
+  const int most = 16 / group;                              // tokens of a tile
+  // ---- which request's tile this is: 64 requests at a time
+  int request = -1, tile = blockIdx.x;
+  for (int i0 = 0; i0 < num_requests && request < 0; i0 += DISTIE_WAVE) {
+    const int i = i0 + lane;
+    const int own = i < num_requests ? (cu_q[i + 1] - cu_q[i] + most - 1) / most : 0;
+    int upto = own;
+#pragma unroll
+    for (int o = 1; o < DISTIE_WAVE; o *= 2) {
+      const int before = __shfl_up(upto, o, DISTIE_WAVE);
+      if (lane >= o) upto += before;
+    }
+    const uint64_t holds = __ballot(upto > tile);
+    if (holds != 0) {
+      const int at = __ffsll(static_cast<unsigned long long>(holds)) - 1;
+      request = i0 + at;
+      tile -= __shfl(upto - own, at, DISTIE_WAVE);
+    } else {
+      tile -= __shfl(upto, DISTIE_WAVE - 1, DISTIE_WAVE);
+    }
+  }
+  if (request < 0) return;                                  // (the grid is an upper bound)
+  const int token0 = cu_q[request] + tile * most;
+  const int count = min(most, cu_q[request + 1] - token0);
+  const int pos0 = positions[token0];
+  const int first = first_visible(pos0, window);
+  const int last = pos0 + count - 1;                        // inclusive, of the tile's last token
+  const int32_t* table = block_table + static_cast<int64_t>(table_rows != nullptr ? table_rows[request] : request) * table_width;
+
+  // ---- the lane's column: head kh * group + r % group of token token0 + r / group (columns past the end repeat the last)
+  const int col = min(r, count * group - 1);
+  const int col_last = pos0 + col / group;
+  const int col_first = first_visible(col_last, window);
+  cf_floatx4 q_reg[DJ];
+  {
+    const float* q = qkv + (token0 + col / group) * q_stride + static_cast<int64_t>(kh * group + col % group) * D + 4 * g;
+#pragma unroll
+    for (int j = 0; j < DJ; ++j) q_reg[j] = *reinterpret_cast<const cf_floatx4*>(q + 16 * j);
+  }
+  cf_floatx4 o_acc[DJ];
+#pragma unroll
+  for (int j = 0; j < DJ; ++j) o_acc[j] = cf_floatx4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;                     // (each lane of a column keeps a part of the sum)
+
+  const int chunk0 = first / CF_KEYS, chunks = last / CF_KEYS - chunk0 + 1;
+  const int per_run = (chunks + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
+  const int run0 = static_cast<int>(blockIdx.z) * per_run;
+  const int run_end = min(chunks, run0 + per_run);          // (a run may hold no chunk)
+  for (int c = (chunk0 + run0 + wave) * CF_KEYS; c < (chunk0 + run_end) * CF_KEYS; c += CF_KEYS * CF_WAVES) {
+    // lane j looks up the page of key c + j; keys that do not count read the start of the cache
+    const int lo = max(first - c, 0), hi = min(CF_KEYS - 1, last - c);      // keys lo .. hi of the chunk count
+    int64_t base = 0;
+    if (lane >= lo && lane <= hi)
+      base = (static_cast<int64_t>(table[(c + lane) / block_size]) * kv_heads + kh) * block_size * D;
+    cf_floatx4 k_reg[CF_BLOCKS][DJ], v_reg[CF_BLOCKS][DJ];
+#pragma unroll
+    for (int b = 0; b < CF_BLOCKS; ++b) {
+      const int key = 16 * b + r;
+      const bool counts = key >= lo && key <= hi;
+      const int64_t page = __shfl(base, key, DISTIE_WAVE);
+      const float* k = k_cache + page + (counts ? (c + key) % block_size : 0) * D + 4 * g;
+#pragma unroll
+      for (int j = 0; j < DJ; ++j) k_reg[b][j] = *reinterpret_cast<const cf_floatx4*>(k + 16 * j);
+    }
+#pragma unroll
+    for (int b = 0; b < CF_BLOCKS; ++b) {
+      // four keys of a dim lie in one page; the page is that of one of them that counts
+      const int key = 16 * b + 4 * g;
+      const int64_t page = __shfl(base, min(max(key, lo), hi), DISTIE_WAVE);
+      const float* v = v_cache + page + static_cast<int64_t>(r) * block_size + (c + key) % block_size;
+#pragma unroll
+      for (int j = 0; j < DJ; ++j) v_reg[b][j] = *reinterpret_cast<const cf_floatx4*>(v + static_cast<int64_t>(16 * j) * block_size);
+    }
+    __builtin_amdgcn_sched_barrier(0);                      // all of these loads are under way before the first is used
+    // ---- scores: the lane holds keys 16 b + 4 g + i of its column
+    cf_floatx4 s[CF_BLOCKS];
+    float best = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < CF_BLOCKS; ++b) {
+      cf_floatx4 chain[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) chain[e] = cf_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < DJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          chain[4 * (j % 4) + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_reg[b][j][e], q_reg[j][e], chain[4 * (j % 4) + e], 0, 0, 0);
+#pragma unroll
+      for (int half = 8; half > 1; half /= 2)
+#pragma unroll
+        for (int e = 0; e < half; ++e) chain[e] += chain[e + half];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = c + 16 * b + 4 * g + i;
+        const float v = (chain[0][i] + chain[1][i]) * scale;
+        s[b][i] = key >= col_first && key <= col_last ? v : -INFINITY;
+        best = fmaxf(best, s[b][i]);
+      }
+    }
+    best = fmaxf(best, __shfl_xor(best, 16, DISTIE_WAVE));
+    best = fmaxf(best, __shfl_xor(best, 32, DISTIE_WAVE));
+    const float m_new = fmaxf(m_run, best);
+    const float alpha = m_new == -INFINITY ? 0.f : expf(m_run - m_new);      // 0 on the first chunk with a key (m = -inf)
+    float sum = 0.f;
+#pragma unroll
+    for (int b = 0; b < CF_BLOCKS; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = c + 16 * b + 4 * g + i;
+        s[b][i] = key >= col_first && key <= col_last ? expf(s[b][i] - m_new) : 0.f;
+        sum += s[b][i];
+      }
+    l_run = l_run * alpha + sum;
+    m_run = m_new;
+    float a4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a4[i] = __shfl(alpha, 4 * g + i, DISTIE_WAVE);
+    // ---- O += P . V: the lane ends with columns 4 g + i of dim 16 j + r; a sum of its own for every 16 keys, added in pairs
+#pragma unroll
+    for (int j = 0; j < DJ; ++j) {
+      cf_floatx4 part[CF_BLOCKS];
+#pragma unroll
+      for (int b = 0; b < CF_BLOCKS; ++b) {
+        part[b] = cf_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = 16 * b + 4 * g + i;
+          // never a value of a key that does not count (a weight of zero times what lies there could be NaN)
+          const float v = key >= lo && key <= hi ? v_reg[b][j][i] : 0.f;
+          part[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[b][i], v, part[b], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float sum4 = part[0][i] + part[1][i];
+        if constexpr (CF_BLOCKS == 4) sum4 += part[2][i] + part[3][i];
+        o_acc[j][i] = fmaf(o_acc[j][i], a4[i], sum4);
+      }
+    }
+  }
+  l_run += __shfl_xor(l_run, 16, DISTIE_WAVE);
+  l_run += __shfl_xor(l_run, 32, DISTIE_WAVE);
+  if (g == 0) {
+    m_s[wave][r] = m_run;
+    l_s[wave][r] = l_run;
+  }
+#pragma unroll
+  for (int j = 0; j < DJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc_s[wave][4 * g + i][16 * j + r] = o_acc[j][i];
+  __syncthreads();
+  // ---- the waves' parts, in wave order; four dims of a column a thread
+  const bool whole = gridDim.z == 1;
+  for (int idx = threadIdx.x; idx < count * group * (D / 4); idx += DISTIE_WAVE * CF_WAVES) {
+    const int cl = idx / (D / 4), d = 4 * (idx % (D / 4));
+    const int head = kh * group + cl % group;
+    const float sink = whole && sinks != nullptr ? sinks[head] : -INFINITY;      // one more term of the denominator, no value
+    float top = sink;
+#pragma unroll
+    for (int w = 0; w < CF_WAVES; ++w) top = fmaxf(top, m_s[w][cl]);
+    float total = sink == -INFINITY ? 0.f : expf(sink - top);
+    float4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < CF_WAVES; ++w) {
+      const float weight = m_s[w][cl] == -INFINITY ? 0.f : expf(m_s[w][cl] - top);      // a wave without keys counts nothing
+      const float4 o = *reinterpret_cast<const float4*>(&acc_s[w][cl][d]);
+      total += l_s[w][cl] * weight;
+      sum.x = fmaf(weight, o.x, sum.x);
+      sum.y = fmaf(weight, o.y, sum.y);
+      sum.z = fmaf(weight, o.z, sum.z);
+      sum.w = fmaf(weight, o.w, sum.w);
+    }
+    const int64_t at = static_cast<int64_t>(token0 + cl / group) * heads + head +
+                       (whole ? 0 : static_cast<int64_t>(blockIdx.z) * tokens * heads);
+    const float inv = whole ? 1.f / total : 1.f;
+    if (!whole && d == 0) {
+      part_ml[2 * at] = top;
+      part_ml[2 * at + 1] = total;
+    }
+    *reinterpret_cast<float4*>((whole ? out : part_o) + at * D + d) = float4{sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv};
+  }
+  }
+}
+
+// Into how many runs distie_attention_columns_f32 is to cut each tile's keys: enough workgroups for every compute unit twice
+// over, a round of the four waves each at least; 0 where the step is not for it. Against the kernels below, us a call:
+//  - more than 2,048 (token, head) pairs, where a wave a pair walked its keys alone: 300 requests of 600 keys, 8 heads of 128
+//    on 2 273 -> 127, on 4 322 -> 212, 8 of 64 on 2 125 -> 48, 5 single tokens and 12 portions of 24, 8 of 128 on 2 125 -> 26;
+//    a single token and a head of its own each fill one column of sixteen and stay (8 on 8: 389, would be 397);
+//  - heads beyond 128, whose rows leave attn_grouped_f32_kernel one wave a SIMD: 8 heads of 256 on 1, 8 requests of 1,000 keys
+//    30.4 -> 19.7, 5 single tokens and a prompt of 200 90 -> 34, a prompt of 500 378 -> 69, of 1,500 2,736 -> 273; not for single
+//    tokens with few heads to share a row (8 on 4, 8 requests: 22.8, would be 24.0);
+//  - up to 128 that kernel stays for few pairs: its chain is shorter (8 requests of 1,000, 12 of 128 on 2: 14.3, would be 19.2).
+extern "C" int distie_attention_columns_f32_runs(int tokens, int num_requests, int heads, int kv_heads, int block_size,
+                                                 int64_t q_stride, int visible) {
+  if (!CF_FITS || tokens < 1 || num_requests < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || kv_heads > 65535 ||
+      heads / kv_heads > 16 || block_size < 4 || block_size % 4 != 0 || q_stride % 4 != 0)
+    return 0;
+  const int group = heads / kv_heads;
+  const bool fills = grouped_fits(tokens, heads) ? D > 128 && (group >= 4 || tokens / 2 >= num_requests)
+                                                 : group >= 2 || tokens > num_requests;
+  if (!fills) return 0;
+  const int64_t tiles = tokens == num_requests ? tokens : tokens / (16 / group) + num_requests;
+  const int64_t wanted = (512 + tiles * kv_heads - 1) / (tiles * kv_heads);
+  constexpr int ROUND = CF_WAVES * CF_KEYS;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({wanted, (visible + ROUND - 1) / ROUND, GQ_MAX_RUNS})));
+}
+
+// Attention of a float32 step whose requests' tokens are rows cu_q[i] .. cu_q[i + 1] at consecutive positions (plain scores,
+// a float32 cache). runs > 1: part_o (float32 [runs, tokens, heads, D]) and part_ml (float32 [runs, tokens, heads, 2]).
+extern "C" int distie_attention_columns_f32(const void* qkv, int64_t q_stride, const void* k_cache, const void* v_cache,
+                                            const int32_t* positions, const int32_t* cu_q, const int32_t* block_table,
+                                            int table_width, const int32_t* table_rows, void* out, int tokens, int num_requests,
+                                            int heads, int kv_heads, int block_size, float scale, int window, const float* sinks,
+                                            float* part_o, float* part_ml, int runs, hipStream_t stream) {
+  if (tokens <= 0) return 0;
+  if (distie_attention_columns_f32_runs(tokens, num_requests, heads, kv_heads, block_size, q_stride, 1) < 1 || table_width < 1 ||
+      heads > 65535 || runs < 1 || runs > GQ_MAX_RUNS || (runs > 1 && (part_o == nullptr || part_ml == nullptr)))
+    return DISTIE_BAD_ARGUMENT;
+  const int most = 16 / (heads / kv_heads);
+  const int tiles = tokens == num_requests ? tokens : tokens / most + num_requests;      // an upper bound; spare blocks leave at once
+  attn_columns_f32_kernel<<<dim3(tiles, kv_heads, runs), DISTIE_WAVE * CF_WAVES, 0, stream>>>(
+      static_cast<const float*>(qkv), q_stride, static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), positions,
+      cu_q, block_table, table_width, table_rows, static_cast<float*>(out), tokens, num_requests, heads, kv_heads, block_size,
+      scale, window, sinks, part_o, part_ml);
+  if (runs > 1)
+    attn_grouped_merge_kernel<<<dim3(tokens, heads), DISTIE_WAVE, 0, stream>>>(part_o, part_ml, static_cast<float*>(out), heads,
+                                                                               runs, sinks);
+  return launch_status();
+}
+
 // Query heads of a kv head that a workgroup takes together, and the workgroups for all of them.
 static int grouped_parts(int group) { return (group + 3) / 4; }
-
-static bool grouped_fits(int64_t tokens, int heads) { return GQ_FITS && tokens * heads < 2048; }
 
 // qkv: [T, q_stride] with q of head h at columns h*D; out: [T, heads*D]. window: see the head of the file.
 // head_slopes (float32 [heads], may be null): score += slope[h] * (key - position); score_cap > 0: the scaled score

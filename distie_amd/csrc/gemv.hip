@@ -1,6 +1,6 @@
 // Weight-streaming products on the vector ALU for few rows of x: y[M, N] = x[M, K] * W[N, K]^T (+ bias), any mix
-// of float32 and bfloat16 for x, W and y, products and sums in float32 FMAs. This is the decode product of
-// the true 32-bit path (no matrix-core mode) and of weights that a file keeps in 32-bit; gemm_generic's
+// of float32 and bfloat16 for x, W and y, products and sums in float32 FMAs. These are the products of
+// few rows that rows_f32 does not take (mixed types, ends of K, callers that want no slices); gemm_generic's
 // 64 x 64 tiles spend 7/8 of their work on padding at 8 rows and leave most of the chip idle.
 //
 // A workgroup of four waves owns four rows of W (several such groups, one after the other, when the rows are

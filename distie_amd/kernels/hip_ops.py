@@ -426,6 +426,9 @@ class HipOps(Ops):
             lib = ctypes.CDLL(str(build.ensure(f"attn_d{head_dim}")))
             lib.distie_attention_generic.argtypes = [_P, _I, _L, _P, _P, _I, _P, _P, _P, _I, _P, _P,
                                                      _I, _I, _I, _I, _F, _I, _P, _F, _P, _P, _P, _I, _P]
+            lib.distie_attention_columns_f32_runs.argtypes = [_I, _I, _I, _I, _I, _L, _I]
+            lib.distie_attention_columns_f32.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I,
+                                                         _P, _P, _P, _I, _P]
             lib.distie_attention_f32_runs.argtypes = [_I, _I, _I, _I]
             lib.distie_attention_prefill_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I,
                                                           _F, _I, _I, _P, _P, _P, _I, _P, _P]
@@ -1214,20 +1217,27 @@ class HipOps(Ops):
                 plan["prefill_ml"].data_ptr() if parts > 1 else None, parts, sinks_ptr, self._stream()),
                 "attention_prefill_f32")
             return out
+        runs = 0
+        if plain and f32 and (qkv.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0:
+            runs = lib.distie_attention_columns_f32_runs(T, meta.num_requests, num_heads, num_kv_heads, meta.block_size,
+                                                         qkv.shape[1], min(meta.max_kv, abs(reach) or meta.max_kv))
+        if runs > 0:
+            # wide heads, or many tokens: a tile of tokens and a kv head's query heads are the columns of matrix products
+            part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
+            _check(lib.distie_attention_columns_f32(
+                qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
+                meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
+                num_heads, num_kv_heads, meta.block_size, float(scale), reach, sinks_ptr,
+                part_o.data_ptr() if runs > 1 else None, part_ml.data_ptr() if runs > 1 else None, runs, self._stream()),
+                "attention_columns_f32")
+            return out
         part_o = part_ml = None
         runs = 1
         if plain and f32:
             # requests that decode in float32: the keys of a token are cut into runs of at least 256 that run side by
             # side, so that few requests occupy the chip as well
             runs = lib.distie_attention_f32_runs(T, num_heads, num_kv_heads, min(meta.max_kv, abs(reach) or meta.max_kv))
-            if runs > 1:
-                key = ("attention_f32_runs", runs, num_heads, head_dim)
-                held = meta.scratch.get(key)
-                if held is None:
-                    held = meta.scratch[key] = (
-                        torch.empty((runs, T, num_heads, head_dim), dtype=torch.float32, device=self.device),
-                        torch.empty((runs, T, num_heads, 2), dtype=torch.float32, device=self.device))
-                part_o, part_ml = held
+            part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
         _check(lib.distie_attention_generic(
             qkv.data_ptr(), _code(qkv), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
             meta.positions.data_ptr(), meta.token_request.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr,
@@ -1302,6 +1312,18 @@ class HipOps(Ops):
             plan["partial_o"] = torch.empty((*shape, head_dim), dtype=torch.float32, device=self.device)
             plan["partial_ml"] = torch.empty((*shape, 2), dtype=torch.float32, device=self.device)
         return plan
+
+    def _run_parts(self, meta: BatchMeta, runs, T, num_heads, head_dim):
+        """The buffers for the sums of `runs` runs of keys, kept for the step's layers."""
+        if runs == 1:
+            return None, None
+        key = ("attention_f32_runs", runs, num_heads, head_dim)
+        held = meta.scratch.get(key)
+        if held is None:
+            held = meta.scratch[key] = (
+                torch.empty((runs, T, num_heads, head_dim), dtype=torch.float32, device=self.device),
+                torch.empty((runs, T, num_heads, 2), dtype=torch.float32, device=self.device))
+        return held
 
     def _attention_plan(self, lib, meta: BatchMeta, T, num_heads, num_kv_heads, head_dim, window) -> dict:
         group = num_heads // num_kv_heads

@@ -916,6 +916,31 @@ def test_float32_products_for_every_head(ops, T, H, N, K, lx, lo):
         assert (got[:, :, N:] == 0).all()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(8, 1, 256, 16, None), (16, 1, 256, 4, 130), (3, 1, 192, 12, None),
+                                                         (4, 4, 256, 32, 65), (10, 2, 256, 64, None), (64, 4, 128, 16, 100),
+                                                         (96, 16, 64, 8, None), (64, 64, 32, 16, None)])
+def test_float32_attention_in_columns(ops, heads, kv_heads, dim, P, window):
+    """The float32 kernel whose columns are the heads of a kv head for several tokens: wide heads, or more pairs of token and
+    head than the kernels for few take. Single tokens among portions that end inside, at and past a tile of tokens, more
+    requests than a wave looks through at once, contexts of 1 to 1,100 keys, one run of keys or several, sinks. Against plain
+    attention, and no further from 64 bits than rounding allows: sums over `dim` and over the keys in 32 bits."""
+    from distie_amd.kernels.interface import ScoreExtras
+
+    for lens, q_lens in (([1100, 17, 64, 300, 1, 65], [1, 17, 16, 24, 1, 3]), ([31 + 7 * i for i in range(70)], [2 + i % 3 for i in range(70)])):
+        meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.float32, seed=11)
+        runs = ops.attention_library(dim).distie_attention_columns_f32_runs(qkv.shape[0], len(lens), heads, kv_heads, P,
+                                                                              qkv.shape[1], max(lens))
+        assert runs >= 1
+        for extras in (None, ScoreExtras(sinks=torch.randn(heads, device="cuda"))):
+            want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, k.double(), v.double(), heads, kv_heads, dim,
+                                                    dim ** -0.5, window, extras)
+            got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window, extras)
+            # a score's rounding is at most about dim / 4 + 2 steps of 2^-24 of |q| |k| * scale ~ a few units, and moves a
+            # weight by as much; the weighted sum over keys adds at most keys / 4 + 2 more
+            bound = (dim / 4 + max(lens) / 4 + 16) * 2.0 ** -24 * 8
+            assert (got.double() - want).abs().max().item() <= bound * v.double().abs().max().item()
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
                                                                   (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8)])
 def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, window, together):
