@@ -152,6 +152,8 @@ class HipOps(Ops):
     # float32 products (and products against weights kept in float32) of up to ROWS_MAX_ROWS rows stream the weights
     # through `gemv_rows` (FMAs on the vector ALU); beyond that the tiled float32 kernel
     ROWS_MAX_ROWS = 64
+    # float32 weights below ROWS_F32_MIN_ELEMENTS stay on the vector ALU: such a product is one launch's latency on either unit
+    ROWS_F32_MIN_ELEMENTS = 64 << 10
     ROWS_F32_FEW = 4
     ROWS_F32_LARGE_ELEMENTS = 8 << 20
     # bfloat16 products by rows of x: up to SKINNY_MAX_ROWS the weights are streamed by one wave per block
@@ -684,7 +686,7 @@ class HipOps(Ops):
         M, K = x.shape
         N = gate_up_weight.shape[0]
         if x.dtype == torch.float32 and gate_up_weight.dtype == torch.float32 and gate_up_weight.shape[1] == K and N % 2 == 0 and \
-                self._ops.distie_rows_f32_slices(M, N, K, 1):
+                N * K >= self.ROWS_F32_MIN_ELEMENTS and self._ops.distie_rows_f32_slices(M, N, K, 1):
             self._own(x, gate_up_weight)
             out = torch.empty((M, N // 2), dtype=torch.float32, device=self.device)
             _check(self._ops.distie_rows_f32(x.data_ptr(), gate_up_weight.data_ptr(), None, out.data_ptr(), M, N, K, gated, 1,
@@ -744,7 +746,7 @@ class HipOps(Ops):
                 inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and head_dim % 16 == 0 and \
                 N == (num_heads + 2 * num_kv_heads) * head_dim and weight.shape[1] == K and \
                 (bias is None or (bias.dtype == torch.float32 and bias.shape[0] == N)) and \
-                self._ops.distie_rows_f32_slices(M, N, K, 1):
+                N * K >= self.ROWS_F32_MIN_ELEMENTS and self._ops.distie_rows_f32_slices(M, N, K, 1):
             slots = meta.groups[group].slots
             self._own(x, weight, bias, k_cache, v_cache, inv_freq, slots)
             self._check_cache(k_cache, v_cache, num_kv_heads, meta.block_size, head_dim)
@@ -1051,7 +1053,7 @@ class HipOps(Ops):
             # TB/s as it is): the weights streamed through the matrix cores' float32 products. At up to ROWS_F32_FEW rows a
             # small weight is faster on the vector ALU (one row against [1536, 1536] 4.4 us, 6.1 here)
             slices = 0
-            if M > self.ROWS_F32_FEW or N * K >= self.ROWS_F32_LARGE_ELEMENTS:
+            if N * K >= self.ROWS_F32_MIN_ELEMENTS and (M > self.ROWS_F32_FEW or N * K >= self.ROWS_F32_LARGE_ELEMENTS):
                 slices = self._ops.distie_rows_f32_slices(M, N, K, 0)
             if slices:
                 out = torch.empty((M, N) if slices == 1 else (slices, M, N), dtype=torch.float32, device=self.device)
