@@ -941,6 +941,36 @@ def test_float32_attention_in_columns(ops, heads, kv_heads, dim, P, window):
             assert (got.double() - want).abs().max().item() <= bound * v.double().abs().max().item()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(8, 1, 256, 16, None), (8, 1, 256, 16, 40), (3, 1, 192, 12, 9),
+                                                         (64, 8, 128, 16, None), (64, 16, 64, 8, 33)])
+def test_float32_columns_keep_values_from_tokens_that_do_not_see_them(ops, heads, kv_heads, dim, P, window):
+    """Tokens of a tile share the products with V: a value that is not finite, of a key that a later token of the tile brings
+    or that has left the window of some of its tokens, reaches the tokens that see the key and no other. Those keep their
+    results bit for bit: left out, the key adds nothing, and finite it adds a weight of zero times its value."""
+    lens, q_lens = [37, 90, 64, 130, 300, 71], [5, 16, 3, 30, 2, 24]
+    meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.float32, seed=13)
+    assert ops.attention_library(dim).distie_attention_columns_f32_runs(qkv.shape[0], len(lens), heads, kv_heads, P,
+                                                                          qkv.shape[1], max(lens)) >= 1
+    clean = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window)
+    table, sees = meta.groups[0].block_table.tolist(), []
+    for b, (n, q) in enumerate(zip(lens, q_lens)):
+        # one key among the new tokens', and one that is at the edge of the window where there is one
+        keys = [(n - q + q // 2, math.nan)]
+        edge = n - q + q // 4 - (window or n)
+        if edge >= 0:
+            keys.append((edge, math.inf))
+        for t in range(q):
+            pos = n - q + t
+            sees.append(any(key <= pos and (window is None or key > pos - window) for key, _ in keys))
+        for key, value in keys:
+            v[table[b][key // P], :, :, key % P] = value
+    got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window)
+    sees = torch.tensor(sees, device="cuda")
+    assert sees.any() and not sees.all()
+    assert torch.equal(got[~sees], clean[~sees])
+    assert not torch.isfinite(got[sees]).any()
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
                                                                   (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8)])
 def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, window, together):
