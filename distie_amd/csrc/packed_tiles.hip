@@ -28,7 +28,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 // waits for all of them before any read of LDS. The s_nop is the wait state between writing m0 and the load.
 __device__ __forceinline__ void load_to_lds(const bf16_t* from, bf16_t* to) {
   const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)to)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from) : "memory", "m0");
 }
 
 // What this wave asked for has arrived and what it read from LDS is in its registers; then the same for all waves.
