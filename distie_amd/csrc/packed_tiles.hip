@@ -44,8 +44,7 @@ struct TilesPlace {
   int stages;                   // of a slice
 };
 
-// MODE: PK_PLAIN (also on a ROTARY copy, rotary.heads > 0: every sum into the column that its row of W has), PK_GATED,
-// PK_ROTARY. K a multiple of PT_K.
+// MODE: PK_PLAIN, PK_GATED, PK_ROTARY. K a multiple of PT_K.
 template <int MB, int NB, int DEPTH, int MODE, typename Y>
 __global__ __launch_bounds__(256, 2) void packed_tiles_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                               const float* __restrict__ bias, Y* __restrict__ y, int M, int N,
@@ -173,8 +172,7 @@ __global__ __launch_bounds__(256, 2) void packed_tiles_kernel(const bf16_t* __re
       } else if constexpr (MODE == PK_ROTARY) {
         store_rotary(v, m, m < M, g, block, bias, y, N, rotary);
       } else {
-        int n0 = 16 * block + 4 * g;
-        if (rotary.heads > 0) n0 = rotary_column(block, g, rotary.heads + rotary.kv_heads, rotary.dim);
+        const int n0 = 16 * block + 4 * g;
         if (bias != nullptr && slice == 0) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[i] += n0 + i < N ? bias[n0 + i] : 0.f;
@@ -266,29 +264,32 @@ int row_blocks_of(int N, bool gated) { return gated ? (N / 2 + 7) / 8 : (N + 15)
 }  // namespace
 
 // How the kernels of this file cut a product; 0 if they do not take it. gated: the copy's rows are gate and up in turn;
-// may_cut: the caller takes float32 slices, at cut_us more. *shape and *slices go to the launch as they are.
-extern "C" int distie_packed_tiles_plan(int M, int N, int K, int gated, int may_cut, float cut_us, int* shape, int* slices) {
+// may_cut: the caller takes float32 slices, at cut_us more. *shape and *slices go to the launch as they are; *workgroups: how
+// many it will have.
+extern "C" int distie_packed_tiles_plan(int M, int N, int K, int gated, int may_cut, float cut_us, int* shape, int* slices,
+                                        int* workgroups) {
   if (M < 1 || N < 1 || K < 2 * PT_K || K % PT_K != 0 || (gated && N % 2 != 0)) return 0;
   const TilesPlan plan = plan_tiles(M, N, K, row_blocks_of(N, gated != 0), gated != 0, may_cut != 0 && !gated, cut_us);
-  *shape = plan.shape, *slices = plan.slices;
+  const TileShape& s = SHAPES[plan.shape];
+  const int64_t blocks = row_blocks_of(N, gated != 0);
+  const int64_t all = (static_cast<int64_t>(M) + 16 * s.mb - 1) / (16 * s.mb) * ((blocks + 4 * s.nb - 1) / (4 * s.nb)) * plan.slices;
+  *shape = plan.shape, *slices = plan.slices, *workgroups = static_cast<int>(std::min<int64_t>(all, 1 << 30));
   return 1;
 }
 
 // y: [M, N] of y_dtype (gated: [M, N / 2] in bfloat16), or with slices > 1 float32 [slices, M, N], to be added in order by
-// whoever reads it, the bias in the first. heads > 0: w_packed is the ROTARY copy of a q/k/v weight.
+// whoever reads it, the bias in the first.
 extern "C" int distie_packed_tiles_bf16(const void* x, const void* w_packed, const float* bias, void* y, int y_dtype, int M,
-                                        int N, int K, int gated, int shape, int slices, int heads, int kv_heads, int dim,
-                                        float limit, float slope, float up_shift, hipStream_t stream) {
+                                        int N, int K, int gated, int shape, int slices, float limit, float slope, float up_shift,
+                                        hipStream_t stream) {
   if (M <= 0) return 0;
   const int act = gated >> 8;           // the activation on the gate, above the low eight bits
   gated &= 0xff;
   if (N < 1 || K < 2 * PT_K || K % PT_K != 0 || shape < 0 || shape >= SHAPE_COUNT ||
       slices < 1 || gated > 1 || (gated && (N % 2 != 0 || slices != 1 || y_dtype != DISTIE_BF16 || bias != nullptr)) || act < 0 ||
-      act > 5 || (act == 5 && !(limit > 0.f)) || (slices > 1 && y_dtype != DISTIE_F32) ||
-      (heads > 0 && (gated || kv_heads < 1 || dim < 16 || dim % 16 != 0 || N != (heads + 2 * kv_heads) * dim)))
+      act > 5 || (act == 5 && !(limit > 0.f)) || (slices > 1 && y_dtype != DISTIE_F32))
     return DISTIE_BAD_ARGUMENT;
   RotaryOut out = {};
-  out.heads = heads, out.kv_heads = kv_heads, out.dim = dim;
   out.act = act, out.limit = limit, out.slope = slope, out.up_shift = up_shift;
   const bf16_t* xb = static_cast<const bf16_t*>(x);
   const bf16_t* wb = static_cast<const bf16_t*>(w_packed);

@@ -153,12 +153,13 @@ class LLM:
         most = min(tokens, self.TIMED_ROWS_MOST, max(self.TIMED_ROWS, -(-self.engine_config.max_seqs // 32) * 32))
         graphs, self.runner.graphs = self.runner.graphs, None        # (timing a kernel cannot be recorded into a graph)
         self.ops.tune_library_products(True)
+        # from here on products go where they will go once the library's kernels for them are timed
+        self.ops.library_timed_rows, self.ops.library_timed_portion = most, tokens
         done = False
         try:
             self.step([StepEntry("__tune__", ids, [tokens - 1])])
             self.finish("__tune__")
-            # from here on the products of these row counts go where they will go once their kernels are timed
-            self.ops.captured, self.ops.library_timed_rows = True, most
+            self.ops.captured = True
             for rows in range(96, most + 1, 32):
                 # every row wanted: the head's product has as many rows as a decode step of that batch
                 self.step([StepEntry("__tune__", ids[:rows], list(range(rows)))])
@@ -168,7 +169,7 @@ class LLM:
         finally:
             self.ops.captured = False
             if not done:
-                self.ops.library_timed_rows = 0
+                self.ops.library_timed_rows = self.ops.library_timed_portion = 0
             self.finish("__tune__")
             self.ops.tune_library_products(False)
             self.runner.graphs = graphs

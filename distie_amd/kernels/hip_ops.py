@@ -207,31 +207,64 @@ class HipOps(Ops):
     # a portion of 160 tokens 7.4 ms in two passes of 80 and 8.4 in three of 64, 64 and 32)
     WIDE_PASS_MAX_BLOCKS = 6
     # From TILES_MIN_ROWS rows of x on, products on a packed copy whose K is a multiple of 64 run in tiles
-    # (`packed_tiles.hip`) where that is faster than the passes above and than the library, which is a matter of the
-    # product's size. Measured with every weight coming from memory (us, tiles / passes up to 96 rows, the library beyond):
-    #  * up to TILES_MAX_WORK multiplications: [64, 8960] x [1536, 8960] 9.1 / 12.0, [64, 1536] x [2048, 1536] 5.8 / 7.1,
-    #    [301, 2048] x [2048, 2048] 10.6 / 11.4, [512, 1024] x [1280, 1024] 7.2 / 10.9, [1200, 1536] x [2048, 1536] 16.3 / 17.7;
-    #    beyond, the library's larger tiles come level: [512, 3584] x [4608, 3584] 30.6 / 28.9;
-    #  * K at least twice as long as the weight has rows: cut along K, as many rows as there are, but for small weights
-    #    of many rows (TILES_LONG_ROWS): [301, 8960] x [1536, 8960] 18.1 / 26.3, [900, 8960] 38.1 / 41.6, [301, 18944] x
-    #    [3584, 18944] 67.7 / 100.5, [2025, 18944] 260 / 350; [1600, 8192] x [2048, 8192] 69.5 / 63.7;
-    #  * gated products, which save the activation's kernel: up to TILES_MAX_GATED_WORK; [64, 1536] x [17920, 1536] 19.8 /
-    #    21.9, [176, 1536] 27.7 / 30.2, [301, 1536] 33.5 / 34.7, [512, 1024] x [8192, 1024] 17.8 / 22.3, [400, 1536] x
-    #    [17920, 1536] 42.2 / 39.0; below 80 rows a weight of up to TILES_SMALL_GATED elements is faster in passes
-    #    ([64, 1024] x [8192, 1024] 9.1 / 8.2);
-    #  * q/k/v with rotation and cache write in the epilogue: from TILES_MIN_ROTARY_ROWS on, up to TILES_MAX_WORK.
+    # (`packed_tiles.hip`) where that is faster than the passes above and than the library, or level with them
+    # (`_tiles_take`). Measured on 46 weights of 0.6 to 141 million elements, 33 to 2,048 rows, every weight from memory, the
+    # kernel that reads the result included (us, tiles / what there was: passes up to 96 rows, beyond them the library's
+    # first choice and its best by timing):
+    #  * whole K: while every workgroup has a compute unit to itself and the tile is one of the two small ones. Past that the
+    #    library's tiles are level or ahead: [512, 1536] x [1536, 1536] 12 / 13, 13; [1200, 1536] 17 / 19, 19; [1400, 1536] 21
+    #    / 21, 20; [900, 8192] x [3072, 8192] on 96 x 128 68 / 64, 66. 96 x 128 pays where the weight has more rows than K
+    #    and the library was not timed: [576, 1024] x [4352, 1024] 12.7 / 15.0, 12.4;
+    #  * K cut, for readers that add the slices (TILES_CUT_ROWS): K at least twice as long as the weight has rows up to
+    #    TILES_LONG_ROWS: [97, 8960] x [1536, 8960] 15 / 26, 26; [320, 8960] 24 / 33, 34; [1024, 8960] 47 / 53, 55; other
+    #    weights up to TILES_CUT_MAX_ROWS: [256, 3584] x [3584, 3584] 21 / 24, 22; [384, 1536] x [1536, 1536] 13 / 12, 12. Up to 64
+    #    rows the passes are level or ahead but for weights of few rows: [64, 8960] x [1536, 8960] 15 / 16; [64, 18944] x
+    #    [3584, 18944] 41 / 36; [64, 5120] x [5120, 5120] 25 / 22. From 65 to 80 rows a pass over a weight of more than 64 MB holds them
+    #    all: [80, 18944] x [3584, 18944] 42 / 41, in one round of small tiles [80, 11008] x [4096, 11008] 30 / 42. Small
+    #    weights (TILES_SMALL_ELEMENTS) only against the library's first choice: [97, 1024] x [1024, 1024] 8 / 11, 8;
+    #  * K cut beyond TILES_LONG_ROWS, for the large weights of a portion of a prompt (TILES_PORTION_ELEMENTS) as far as they were
+    #    measured, against the library's first choice: [2048, 18944] x [3584, 18944] 296 / 382, 268; [1600, 27648] x
+    #    [5120, 27648] 571 / 681, 416; not [1800, 27648] 560 / 455, 470 nor [1400, 11008] x [4096, 11008] 160 / 149, 148. An engine
+    #    that timed the library's kernels for a portion of these rows stays with them;
+    #  * gated products, which save the activation's kernel: [64, 1536] x [17920, 1536] 20 / 22; [192, 1536] 28 / 30, 29; [301,
+    #    1536] 34 / 34, 35; [193, 2048] x [16384, 2048] 32 / 31, 32: up to TILES_MAX_GATED_WORK, and where the host bounds the step,
+    #    or one pass of 96 rows is what there is, as far as they are level, TILES_LEVEL_GATED_WORK. Weights of up to
+    #    TILES_SMALL_GATED elements from 81 rows on where one round of tiles holds them ([88, 1024] x [8192, 1024] 9 / 10;
+    #    [88, 896] x [9728, 896] 12 / 11), or beyond the passes' rows; up to TILES_MAX_SMALL_GATED_WORK ([512, 1024] x [8192,
+    #    1024] 21 / 22, 23; [832, 1024] 28 / 26, 27);
+    #  * q/k/v with rotation and cache write in the epilogue: one round of 64 x 64 tiles: [80, 3584] x [4608, 3584] 20 / 22;
+    #    [512, 1536] x [2048, 1536] 11 / 14, 13; in tiles of 64 x 128 the epilogue costs what it saves ([640, 1536] 18 / 17, 17)
+    #    but for large weights beside an untimed library ([224, 3584] x [4608, 3584] 30 / 37, 27). Weights of up to
+    #    ROW_GROUPS_MAX_ELEMENTS have kernels of 16 rows, up to 96 rows of a captured step and 192 of another ([96, 1024] x [1536,
+    #    1024] 9.1 / 6.7): from there on.
     TILES_MIN_ROWS = 33
     TILES_MIN_ROTARY_ROWS = 80
     TILES_MAX_WORK = 4.5e9
-    TILES_MAX_GATED_WORK = 8.5e9
-    TILES_LONG_ROWS = 1100
+    TILES_MAX_GATED_WORK = 6.45e9
+    TILES_LEVEL_GATED_WORK = 8.5e9
+    TILES_MAX_SMALL_GATED_WORK = 4.8e9
     TILES_SMALL_GATED = 10 << 20
+    TILES_SMALL_ELEMENTS = 2 << 20
+    TILES_CUT_ROWS = 65
+    TILES_FEW_WEIGHT_ROWS = 2048
+    TILES_CUT_MAX_ROWS = 320
+    TILES_LONG_ROWS = 1024
+    TILES_PORTION_ELEMENTS = 56 << 20
+    TILES_PORTION_ROWS = 2048
+    TILES_PORTION_WORK = 2.3e11
+    TILES_LARGE_ROTARY = 12 << 20
+    # In a step that is launched kernel by kernel a product of the library's costs the host 10 us more than one of these, the
+    # kernel behind it for activation or rotation its own launch, and the passes' rules take longer to walk through. Where
+    # weights are small (TILES_SMALL_GATED) the host bounds such a step up to about TILES_HOST_ROWS, whatever its kernels take:
+    # tiles then go up to TILES_MAX_WORK (a layer of the Mepapel decoder of width 1024, 899 rows: gate+up in tiles 29 us instead
+    # of 28, the step 20 us a layer shorter; a prompt of 100 tokens, 1.5B shape, q/k/v in tiles 10 us instead of 9, the step
+    # 2,245 us instead of 2,302).
+    TILES_HOST_ROWS = 2048
     # (A weight that no role was named for stays with the passes: who reads its product is not known.)
     # What a cut product costs beyond its slices where the reader of the result cannot add them itself (the readers of a
-    # layer's output projections can), and what rotation and cache write cost as a kernel of their own
+    # layer's output projections can)
     ADDS_SLICES = ("attn_out", "down")
     SUM_SLICES_US = 4.5
-    ROPE_KV_WRITE_US = 7.0
     # attention over a portion of a prompt: from so many visible keys on, the walk over the keys is cut into so
     # many parts that run side by side (measured at 12 heads of 128, 2,048 new tokens: 3 parts are best up to
     # 4,096 keys, 5 at 8,192, 8 from 16,384 on; the kernel takes up to 16)
@@ -282,7 +315,7 @@ class HipOps(Ops):
         self._compute_units = torch.cuda.get_device_properties(self.device).multi_processor_count
         self._lib = None
         self._tuning = False
-        self.library_timed_rows = 0
+        self.library_timed_rows = self.library_timed_portion = 0
         self._packed_left_out = 0
         self._tile_plans: Dict[tuple, Optional[tuple]] = {}
         self._ops = ctypes.CDLL(str(build.ensure("ops")))
@@ -342,8 +375,8 @@ class HipOps(Ops):
         o.distie_gemm_packed_wide_slices.argtypes = [_I, _I]
         o.distie_gemm_packed_wide_qkv_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_packed_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
-        o.distie_packed_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F, ctypes.POINTER(_I), ctypes.POINTER(_I)]
-        o.distie_packed_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
+        o.distie_packed_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F] + 3 * [ctypes.POINTER(_I)]
+        o.distie_packed_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
         o.distie_packed_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_packed_each_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _P, _P]
         o.distie_decode_norm_fits.argtypes = [_I]
@@ -763,7 +796,7 @@ class HipOps(Ops):
         fused = held is not None and held[1] == (num_heads, num_kv_heads, head_dim) and x.dtype == torch.bfloat16 and \
             inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and k_cache.dtype == torch.bfloat16
         if fused:
-            plan = self._tiles(x.shape[0], *weight.shape, "rotary", self.ROPE_KV_WRITE_US)
+            plan = self._tiles(x.shape[0], *weight.shape, "rotary")
             fused = plan is not None or x.shape[0] <= self._packed_rows(x.shape[0], *weight.shape)
         if not fused:
             return self.rope_kv_write(self.linear(x, weight, bias), meta, group, k_cache, v_cache, inv_freq,
@@ -782,10 +815,6 @@ class HipOps(Ops):
         self._check_cache(k_cache, v_cache, num_kv_heads, meta.block_size, head_dim)
         if M != meta.num_tokens or slots.shape[0] != M:
             raise KernelError("linear_rope_kv_write: rows do not match the batch")
-        if plan is not None and plan[1] > 1:
-            product = self._run_tiles(plan, x, packed, bias, torch.bfloat16, M, N, K, heads=(num_heads, num_kv_heads, head_dim))
-            return self.rope_kv_write(product, meta, group, k_cache, v_cache, inv_freq, num_heads, num_kv_heads,
-                                      head_dim, write)
         if plan is None and M >= self.WIDE_QKV_MIN_ROWS and N * K > self.ROW_GROUPS_MAX_ELEMENTS:
             # more than one group of 16 rows against a weight that fills the chip through the wide kernel: the
             # epilogue kernel would read the weight once per group, so the product runs wide (weights once, K in
@@ -831,30 +860,62 @@ class HipOps(Ops):
         reading the slices (None: it must not be cut)."""
         if M < self.TILES_MIN_ROWS:
             return None
-        key = (M, N, K, kind, cut_us, self.library_timed_rows)
+        key = (M, N, K, kind, cut_us, self.captured, self.library_timed_rows, self.library_timed_portion)
         try:
             return self._tile_plans[key]
         except KeyError:
             pass
-        work, plan = M * N * K, None
-        if kind == "gated":
-            wanted = work <= self.TILES_MAX_GATED_WORK and (M >= 80 or N * K > self.TILES_SMALL_GATED)
-        elif kind == "rotary":
-            wanted = work <= self.TILES_MAX_WORK and M >= self.TILES_MIN_ROTARY_ROWS
-        else:
-            wanted = work <= self.TILES_MAX_WORK or \
-                (K >= 2 * N and cut_us is not None and (M <= self.TILES_LONG_ROWS or N * K > self.PACKED_LARGE_ELEMENTS))
-        if wanted:
-            shape, slices = ctypes.c_int(0), ctypes.c_int(0)
-            if self._ops.distie_packed_tiles_plan(M, N, K, kind == "gated", cut_us is not None, cut_us or 0.0,
-                                                  ctypes.byref(shape), ctypes.byref(slices)):
-                plan = (shape.value, slices.value)
+        plan = None
+        shape, slices, workgroups = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+        if self._ops.distie_packed_tiles_plan(M, N, K, kind == "gated", cut_us is not None, cut_us or 0.0, ctypes.byref(shape),
+                                              ctypes.byref(slices), ctypes.byref(workgroups)) and \
+                self._tiles_take(M, N, K, kind, shape.value, slices.value, workgroups.value):
+            plan = (shape.value, slices.value)
         if len(self._tile_plans) >= self.TILE_PLANS:
             self._tile_plans.clear()
         self._tile_plans[key] = plan
         return plan
 
-    def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, heads=(0, 0, 0), clamp=(0.0, 1.0, 0.0)):
+    def _tiles_take(self, M, N, K, kind, shape, slices, workgroups) -> bool:
+        """Whether a product of the plan (shape, slices) and so many workgroups is to run in tiles: see the constants."""
+        elements, work = N * K, M * N * K
+        # whether the library's kernels for these rows were chosen by timing (it goes by classes of 32 rows)
+        timed = M <= self.library_timed_rows or -(-M // 32) == -(-self.library_timed_portion // 32)
+        passes = self._packed_rows(M, N, K)               # rows of x up to which the passes over a packed copy go
+        one_round = workgroups <= self._compute_units
+        small = elements <= self.ROW_GROUPS_MAX_ELEMENTS
+        if not self.captured and M <= self.TILES_HOST_ROWS and elements <= self.TILES_SMALL_GATED and \
+                (M >= self.TILES_MIN_ROTARY_ROWS or kind == "plain") and \
+                work <= (self.TILES_LEVEL_GATED_WORK if kind == "gated" else self.TILES_MAX_WORK):
+            return True
+        if kind == "rotary":
+            return M >= self.TILES_MIN_ROTARY_ROWS and (M > passes or not small) and one_round and work <= self.TILES_MAX_WORK and \
+                (shape == 0 or (shape == 1 and elements > self.TILES_LARGE_ROTARY and not timed))
+        if kind == "gated":
+            if small:
+                return M > passes and work <= self.TILES_MAX_SMALL_GATED_WORK
+            if elements <= self.TILES_SMALL_GATED:
+                return (M > passes or (M > 80 and one_round)) and work <= self.TILES_MAX_SMALL_GATED_WORK
+            level = M <= self.PACKED_MAX_ROWS or not self.captured
+            return work <= (self.TILES_LEVEL_GATED_WORK if level else self.TILES_MAX_GATED_WORK)
+        long = K >= 2 * N
+        if not long and work > self.TILES_MAX_WORK:
+            return False
+        if slices == 1:
+            return one_round and not (long and M > self.TILES_LONG_ROWS) and \
+                (shape <= 1 or (shape == 2 and N > K and not small and not timed))
+        if elements <= self.TILES_SMALL_ELEMENTS:
+            return self.PACKED_MAX_ROWS < M <= self.TILES_LONG_ROWS and not timed
+        if M < self.TILES_CUT_ROWS:
+            return elements <= self.PACKED_LARGE_ELEMENTS // 2 and N <= self.TILES_FEW_WEIGHT_ROWS
+        if M <= 80 and elements > self.PACKED_LARGE_ELEMENTS:
+            return one_round and shape == 0
+        if long and M > self.TILES_LONG_ROWS:
+            return not timed and elements > self.TILES_PORTION_ELEMENTS and M <= self.TILES_PORTION_ROWS and \
+                work <= self.TILES_PORTION_WORK
+        return long or M <= self.TILES_CUT_MAX_ROWS
+
+    def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, clamp=(0.0, 1.0, 0.0)):
         """The tiled product; float32 slices if the plan cuts K."""
         shape, slices = plan
         columns = N // 2 if gated else N
@@ -862,7 +923,7 @@ class HipOps(Ops):
             torch.empty((slices, M, columns), dtype=torch.float32, device=self.device)
         _check(self._ops.distie_packed_tiles_bf16(
             x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), _code(out),
-            M, N, K, gated, shape, slices, *heads, *clamp, self._stream()), "packed_tiles_bf16")
+            M, N, K, gated, shape, slices, *clamp, self._stream()), "packed_tiles_bf16")
         return out if slices == 1 else PartialSums(out, out_dtype)
 
     def _library(self):
