@@ -235,10 +235,9 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_generic_kernel(
 // keeps in registers; the sums of the eight lanes are added by three exchanges. With G > 1 every row of K
 // and every value of V^T is read once for G heads.
 //
-// What bounds it is the chain of trips to memory that a wave makes for 64 keys (page, K, V), so the keys of a token go to
+// What bounds it is the chain of trips to memory that a wave makes for 64 keys (page, K, V), so the keys of a token can go to
 // gridDim.z workgroups in runs of whole chunks (each token's own keys cut alike), which leave their sums for
-// attn_grouped_merge_kernel. 8 requests of 770 to 1,000 keys, 12 heads of 128 on 2: 24.5 us a call with one workgroup of
-// eight waves a (token, head), 96 in all; 12.7 and 4.7 with three heads to a workgroup of four waves and four runs.
+// attn_grouped_merge_kernel. `grouped_plan` chooses heads, waves and runs.
 constexpr bool GQ_FITS = D % 32 == 0;
 constexpr int GQ_SLICE = GQ_FITS ? D / 8 : 4;
 static bool grouped_fits(int64_t tokens, int heads) { return GQ_FITS && tokens * heads < 2048; }
@@ -249,7 +248,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_request,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ table_rows,
     float* __restrict__ out, int heads, int kv_heads, int parts, int block_size, float scale, int window,
-    const float* __restrict__ sinks, float* __restrict__ part_o, float* __restrict__ part_ml) {
+    const float* __restrict__ sinks, float* __restrict__ part_o, float* __restrict__ part_ml, int runs) {
   __shared__ float p_s[WAVES][G][DISTIE_WAVE];
   __shared__ int64_t base_s[WAVES][DISTIE_WAVE];
   __shared__ float m_s[WAVES][G], l_s[WAVES][G];
@@ -290,7 +289,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
   }
 
   const int chunk0 = first / DISTIE_WAVE, chunks = last / DISTIE_WAVE - chunk0 + 1;
-  const int per_run = (chunks + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
+  const int per_run = runs == 1 ? chunks : (chunks + runs - 1) / runs;
   const int run0 = static_cast<int>(blockIdx.z) * per_run;
   const int run_end = min(chunks, run0 + per_run);          // (a run may hold no chunk)
   for (int c = (chunk0 + run0 + wave) * DISTIE_WAVE; c < (chunk0 + run_end) * DISTIE_WAVE; c += DISTIE_WAVE * WAVES) {
@@ -417,7 +416,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
     }
   __syncthreads();
   // wave w writes heads w, w + WAVES, ... of the part
-  const bool whole = gridDim.z == 1;
+  const bool whole = runs == 1;
   for (int g = wave; g < n; g += WAVES) {
     const float sink = whole && sinks != nullptr ? sinks[h0 + g] : -INFINITY;      // one more term of the denominator, no value
     float top = sink;
@@ -769,30 +768,81 @@ extern "C" int distie_attention_columns_f32(const void* qkv, int64_t q_stride, c
   return launch_status();
 }
 
-// Query heads of a kv head that a workgroup takes together, and the workgroups for all of them.
-static int grouped_parts(int group) { return (group + 3) / 4; }
+// How attn_grouped_f32_kernel takes a step: query heads to a workgroup, its waves, and the runs of keys.
+struct GroupedPlan {
+  int per, waves, runs;
+};
+
+// visible: the most keys that a token sees. From 650 steps (1 to 128 requests of 30 to 16,000 keys, portions of up to 31
+// tokens, heads of 64 to 256, groups of 1 to 8; K and V from memory), each with every number of heads, 4 and 8 waves, 1 to 16
+// runs; what this takes is 2 % from the best of them on average. us, one run of eight waves a workgroup / this:
+//  * runs cost a merge and its launch, some 4.5 us, so keys are cut only where one run has eight waves take two chunks each:
+//    1 request, 12 heads of 128 on 2: 200 keys 8.6 / 8.4, 400 keys 11.9 / 11.9 (two runs: 14.2), 700 keys 16.0 / 11.8, 1,000 keys
+//    24.9 / 13.9, 4,000 keys 82 / 15.2. Runs of one chunk a wave, or of as many as the chip has room for: 512 workgroups of
+//    four waves, fewer where contexts are short for heads of 64 or the registers hold one wave a SIMD, more for long ones;
+//  * heads share a workgroup, and a row of K its load, as far as the chip is full without it: 64 requests of 128 keys, 12 heads
+//    of 128 on 2 14.9 / 11.8; a head to itself otherwise (8 requests of 128 keys 8.8 / 8.6, in threes 11.2);
+//  * without runs four waves for up to four chunks, then eight, but for more workgroups than compute units, which run two at a
+//    time (64 requests of 700 keys, 28 heads of 128 on 4: 57 / 47), and where eight waves do not fit the registers: beyond 128
+//    (runs from five chunks on there: 8 heads of 256 on 4, 1 request of 400 keys 38 / 21), and at 96, where the compiler then
+//    spills, with more than one head (156 requests of 500 keys, 8 of 96 on 2: 112 / 48).
+constexpr int GQ_EIGHT_HEADS = D > 128 ? 0 : D <= 64 || D == 128 ? 4 : 1;      // heads with which eight waves fit
+static GroupedPlan grouped_plan(int64_t tokens, int heads, int kv_heads, int visible) {
+  const int group = heads / kv_heads, most = std::min(4, group), chunks = (visible + DISTIE_WAVE - 1) / DISTIE_WAVE;
+  const int64_t pairs = tokens * kv_heads;
+  const auto parts = [&](int per) { return (group + per - 1) / per; };
+  const auto even = [&](int per) { return (group + parts(per) - 1) / parts(per); };      // as many heads in each part
+  const auto fewest = [&](int64_t limit, int runs) {          // heads a workgroup with which there are at most `limit`; 0: none
+    for (int per = 1; per <= most; ++per)
+      if (pairs * parts(per) * runs <= limit) return per;
+    return 0;
+  };
+  constexpr bool WIDE = D > 128, NARROW = D <= 64;
+  if (chunks > (WIDE ? 4 : most == 1 ? 6 : 8)) {
+    const bool lasting = chunks > 18;
+    const int64_t apart = NARROW && lasting ? 512 : 256;              // workgroups up to which heads are kept apart
+    const int64_t room = NARROW ? (!lasting ? 256 : most == 4 ? 1024 : 512) : D > 192 && !lasting ? 320 : 512;
+    for (int trips = 1;; ++trips) {                             // chunks that a wave takes one after the other
+      const int runs = std::min(GQ_MAX_RUNS, (chunks + 4 * trips - 1) / (4 * trips));
+      // two runs of four waves are one run of eight, where those fit; side by side they spread better for heads of their own
+      const bool two = WIDE || (most == 1 && trips == 1);
+      if (runs < (two ? 2 : 3)) break;
+      const int per = fewest(apart, runs);
+      if (per > 0) return {even(per), 4, runs};
+      if (pairs * parts(most) * runs <= room && (WIDE || runs > 2)) return {even(most), 4, runs};
+    }
+  }
+  const bool four = WIDE || chunks <= 4;
+  int per = fewest(NARROW && four ? 512 : 256, 1);
+  // more workgroups than compute units: those of eight waves run one at a time at heads of 128, two at 64
+  const bool crowded = per == 0 && !(NARROW && pairs * parts(most) <= 512) && most > 1;
+  if (per == 0) per = most;
+  return {even(per), four || crowded || even(per) > GQ_EIGHT_HEADS ? 4 : 8, 1};
+}
+
+// The plan for a step of distie_attention_generic (float32, plain scores): -> runs, which the caller has buffers for; what a plan
+// changes in the results is their rounding. 1 and no heads where another kernel takes the step.
+extern "C" int distie_attention_f32_plan(int tokens, int heads, int kv_heads, int visible, int* per, int* waves) {
+  *per = *waves = 0;
+  if (tokens < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || visible < 1 || !grouped_fits(tokens, heads)) return 1;
+  const GroupedPlan plan = grouped_plan(tokens, heads, kv_heads, visible);
+  *per = plan.per, *waves = plan.waves;
+  return plan.runs;
+}
 
 // qkv: [T, q_stride] with q of head h at columns h*D; out: [T, heads*D]. window: see the head of the file.
 // head_slopes (float32 [heads], may be null): score += slope[h] * (key - position); score_cap > 0: the scaled score
 // goes through cap * tanh(score / cap) first. Only this kernel takes the two. sinks (float32 [heads], may be null): the
 // softmax's denominator holds exp(sinks[h]) beside the keys' terms; every kernel of this file takes them.
-// Into how many runs distie_attention_generic is best asked to cut each token's keys (float32, plain scores; the runs that a
-// launch takes do not change what it computes): enough workgroups for every compute unit twice over, 256 keys each at
-// least. visible: the most keys that a token sees.
-extern "C" int distie_attention_f32_runs(int tokens, int heads, int kv_heads, int visible) {
-  if (tokens < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || !grouped_fits(tokens, heads)) return 1;
-  const int64_t units = static_cast<int64_t>(tokens) * kv_heads * grouped_parts(heads / kv_heads);
-  const int64_t wanted = (512 + units - 1) / units;
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({wanted, (visible + 255) / 256, GQ_MAX_RUNS})));
-}
-
+// runs, per, waves: of distie_attention_f32_plan (1, 0, 0: none); runs > 1: part_o (float32 [runs, T, heads, D]) and part_ml
+// (float32 [runs, T, heads, 2]).
 extern "C" int distie_attention_generic(const void* qkv, int dtype, int64_t q_stride, const void* k_cache,
                                         const void* v_cache, int cache_dtype, const int32_t* positions,
                                         const int32_t* token_request, const int32_t* block_table,
                                         int table_width, const int32_t* table_rows, void* out, int tokens, int heads, int kv_heads,
                                         int block_size, float scale, int window, const float* head_slopes,
-                                        float score_cap, const float* sinks, float* part_o, float* part_ml, int runs,
-                                        hipStream_t stream) {
+                                        float score_cap, const float* sinks, float* part_o, float* part_ml, int runs, int per,
+                                        int waves, hipStream_t stream) {
   if (tokens <= 0) return 0;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || block_size < 1 || table_width < 1 ||
       score_cap < 0.f || runs < 1 || runs > GQ_MAX_RUNS || (runs > 1 && (part_o == nullptr || part_ml == nullptr)))
@@ -802,23 +852,33 @@ extern "C" int distie_attention_generic(const void* qkv, int dtype, int64_t q_st
   dim3 grid(tokens, heads);
   const int group = heads / kv_heads;
   if (plain_scores && grouped_fits(tokens, heads) && dtype == DISTIE_F32 && cache_dtype == DISTIE_F32 && q_stride % 4 == 0 &&
-      block_size % 4 == 0 && DISTIE_WAVE % block_size == 0) {
-    // requests that decode, float32: up to four heads of a kv head to a workgroup of four waves, equally many in each
-    const int parts = grouped_parts(group), per = (group + parts - 1) / parts;
+      block_size % 4 == 0 && DISTIE_WAVE % block_size == 0 && per != 0) {
+    // few pairs of token and head, as when requests decode, float32
+    if (per < 1 || per > std::min(4, group) || (waves != 4 && (waves != 8 || per > GQ_EIGHT_HEADS))) return DISTIE_BAD_ARGUMENT;
+    const int parts = (group + per - 1) / per;
     const dim3 grouped(tokens, kv_heads * parts, runs);
-#define DISTIE_GROUPED(G)                                                                                          \
-    attn_grouped_f32_kernel<G, 4><<<grouped, DISTIE_WAVE * 4, 0, stream>>>(                                         \
+#define DISTIE_GROUPED(G, WAVES)                                                                                   \
+    attn_grouped_f32_kernel<G, WAVES><<<grouped, DISTIE_WAVE * WAVES, 0, stream>>>(                                 \
         static_cast<const float*>(qkv), q_stride, static_cast<const float*>(k_cache),                               \
         static_cast<const float*>(v_cache), positions, token_request, block_table, table_width, table_rows,         \
-        static_cast<float*>(out), heads, kv_heads, parts, block_size, scale, window, sinks, part_o, part_ml)
-    if (per == 4) DISTIE_GROUPED(4);
-    else if (per == 3) DISTIE_GROUPED(3);
-    else if (per == 2) DISTIE_GROUPED(2);
-    else DISTIE_GROUPED(1);
+        static_cast<float*>(out), heads, kv_heads, parts, block_size, scale, window, sinks, part_o, part_ml, runs)
+#define DISTIE_GROUPED_OF(WAVES, MOST)                                                                             \
+    if (per == 1) DISTIE_GROUPED(1, WAVES);                                                                         \
+    if constexpr (MOST > 1) {                                                                                      \
+      if (per == 2) DISTIE_GROUPED(2, WAVES);                                                                       \
+      if (per == 3) DISTIE_GROUPED(3, WAVES);                                                                       \
+      if (per == 4) DISTIE_GROUPED(4, WAVES);                                                                       \
+    }
+    if (waves == 4) {
+      DISTIE_GROUPED_OF(4, 4);
+    } else if constexpr (GQ_EIGHT_HEADS > 0) {
+      DISTIE_GROUPED_OF(8, GQ_EIGHT_HEADS);
+    }
+#undef DISTIE_GROUPED_OF
+#undef DISTIE_GROUPED
     if (runs > 1)
       attn_grouped_merge_kernel<<<dim3(tokens, heads), DISTIE_WAVE, 0, stream>>>(part_o, part_ml, static_cast<float*>(out),
                                                                                  heads, runs, sinks);
-#undef DISTIE_GROUPED
     return launch_status();
   }
   // few (token, head) pairs, as when requests decode: eight waves share each pair's keys

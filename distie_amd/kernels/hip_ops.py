@@ -460,11 +460,11 @@ class HipOps(Ops):
                 raise KernelError(f"attention kernels take even head sizes up to {self.LARGEST_HEAD}, not {head_dim}")
             lib = ctypes.CDLL(str(build.ensure(f"attn_d{head_dim}")))
             lib.distie_attention_generic.argtypes = [_P, _I, _L, _P, _P, _I, _P, _P, _P, _I, _P, _P,
-                                                     _I, _I, _I, _I, _F, _I, _P, _F, _P, _P, _P, _I, _P]
+                                                     _I, _I, _I, _I, _F, _I, _P, _F, _P, _P, _P, _I, _I, _I, _P]
             lib.distie_attention_columns_f32_runs.argtypes = [_I, _I, _I, _I, _I, _L, _I]
             lib.distie_attention_columns_f32.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I,
                                                          _P, _P, _P, _I, _P]
-            lib.distie_attention_f32_runs.argtypes = [_I, _I, _I, _I]
+            lib.distie_attention_f32_plan.argtypes = [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]
             lib.distie_attention_prefill_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I,
                                                           _F, _I, _I, _P, _P, _P, _I, _P, _P]
             lib.distie_attention_prefill_f32.argtypes = lib.distie_attention_prefill_bf16.argtypes
@@ -1295,18 +1295,18 @@ class HipOps(Ops):
                 "attention_columns_f32")
             return out
         part_o = part_ml = None
-        runs = 1
+        runs, per, waves = 1, 0, 0
         if plain and f32:
-            # requests that decode in float32: the keys of a token are cut into runs of at least 256 that run side by
-            # side, so that few requests occupy the chip as well
-            runs = lib.distie_attention_f32_runs(T, num_heads, num_kv_heads, min(meta.max_kv, abs(reach) or meta.max_kv))
+            # requests that decode in float32: the keys of a token can be cut into runs that run side by side, so that few
+            # requests occupy the chip as well
+            runs, per, waves = self._grouped_plan(lib, T, num_heads, num_kv_heads, min(meta.max_kv, abs(reach) or meta.max_kv))
             part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
         _check(lib.distie_attention_generic(
             qkv.data_ptr(), _code(qkv), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
             meta.positions.data_ptr(), meta.token_request.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr,
             out.data_ptr(), T, num_heads, num_kv_heads, meta.block_size, float(scale), reach,
             slopes.data_ptr() if slopes is not None else None, cap, sinks_ptr, part_o.data_ptr() if runs > 1 else None,
-            part_ml.data_ptr() if runs > 1 else None, runs, self._stream()), "attention_generic")
+            part_ml.data_ptr() if runs > 1 else None, runs, per, waves, self._stream()), "attention_generic")
         return out
 
     def _mixed_attention(self, q, meta: BatchMeta, table, rows_ptr, k_cache, v_cache, out, num_heads, num_kv_heads, head_dim,
@@ -1375,6 +1375,13 @@ class HipOps(Ops):
             plan["partial_o"] = torch.empty((*shape, head_dim), dtype=torch.float32, device=self.device)
             plan["partial_ml"] = torch.empty((*shape, 2), dtype=torch.float32, device=self.device)
         return plan
+
+    @staticmethod
+    def _grouped_plan(lib, T, num_heads, num_kv_heads, visible):
+        """(runs, heads a workgroup, waves) of the float32 kernel for few pairs of token and head."""
+        per, waves = ctypes.c_int(0), ctypes.c_int(0)
+        runs = lib.distie_attention_f32_plan(T, num_heads, num_kv_heads, visible, ctypes.byref(per), ctypes.byref(waves))
+        return runs, per.value, waves.value
 
     def _run_parts(self, meta: BatchMeta, runs, T, num_heads, head_dim):
         """The buffers for the sums of `runs` runs of keys, kept for the step's layers."""

@@ -995,16 +995,20 @@ def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, w
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(12, 2, 128, 16, None), (8, 1, 256, 16, None), (7, 1, 32, 32, 300),
-                                                         (4, 4, 64, 8, None), (2, 1, 64, 4, 65)])
+                                                         (4, 4, 64, 8, None), (2, 1, 64, 4, 65), (3, 1, 192, 16, 200), (6, 2, 96, 8, None)])
 @pytest.mark.parametrize("runs", [1, 2, 3, 16])
 def test_float32_decode_keys_in_runs(ops, heads, kv_heads, dim, P, window, runs, monkeypatch):
-    """The float32 kernel of requests that decode, its keys cut into runs: requests of one key, of a chunk of 64 and one
-    more, runs that hold no chunk, sinks that count once, and buffers that held NaN before."""
+    """The float32 kernel of requests that decode, its keys cut into runs, for every number of heads and waves that a workgroup
+    may have: requests of one key, of a chunk of 64 and one more, runs that hold no chunk, sinks that count once, and buffers
+    that held NaN before."""
     from distie_amd.kernels.interface import ScoreExtras
 
     lens = [1, 64, 65, 130, 257, 700, 1100]
     meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, [1] * len(lens), torch.float32, seed=21)
-    monkeypatch.setattr(ops.attention_library(dim), "distie_attention_f32_runs", lambda *sizes: runs)
+    lib = ops.attention_library(dim)
+    monkeypatch.setattr(lib, "distie_attention_columns_f32_runs", lambda *sizes: 0)
+    # (eight waves do not fit the registers of every size)
+    asked, eight_heads = [], 4 if dim in (32, 64, 128) else 1 if dim < 128 else 0
     empty = torch.empty
     monkeypatch.setattr(torch, "empty", lambda *a, **kw: empty(*a, **kw).fill_(float("nan"))
                         if kw.get("dtype") == torch.float32 else empty(*a, **kw))
@@ -1012,8 +1016,13 @@ def test_float32_decode_keys_in_runs(ops, heads, kv_heads, dim, P, window, runs,
         extras = None if sinks is None else ScoreExtras(sinks=sinks)
         want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, k.double(), v.double(), heads, kv_heads, dim,
                                                 dim ** -0.5, window, extras)
-        got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window, extras)
-        close(got, want, torch.float32, scale=want.abs().max().item())
+        for per in range(1, min(4, heads // kv_heads) + 1):
+            for waves in (4, 8) if per <= eight_heads else (4,):
+                monkeypatch.setattr(ops, "_grouped_plan", lambda *sizes: asked.append(sizes) or (runs, per, waves))
+                meta.scratch.clear()
+                got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window, extras)
+                close(got, want, torch.float32, scale=want.abs().max().item())
+    assert len(asked) >= 2 * min(4, heads // kv_heads)
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,P", [(12, 2, 128, 16), (4, 2, 64, 16), (3, 1, 48, 16), (2, 1, 256, 32)])

@@ -1,5 +1,5 @@
-"""Which kernel a product goes to, by its rows, its weight and what reads its result: the rule alone, without a GPU. Each line
-names a product on one side of a boundary where the kernels of both sides were measured."""
+"""Which kernel a product or a step's attention goes to: the rules alone, without a GPU. Each line names a call on one side of a
+boundary where the kernels of both sides were measured."""
 
 import ctypes
 
@@ -77,3 +77,44 @@ def test_plans_are_kept_apart_by_what_the_rule_reads(rules):
     rules.library_timed_portion = 2040               # classes of 32 rows
     assert [rules._tiles(rows, 3584, 18944, "plain", 0.0) is None for rows in (1400, 2016, 2017, 2048)] == [False, False, True, True]
     rules.library_timed_portion = 0
+
+
+def grouped(dim, *sizes):
+    return HipOps._grouped_plan(attention(dim), *sizes)
+
+
+def attention(dim):
+    lib = ctypes.CDLL(str(build.ensure(f"attn_d{dim}")))
+    lib.distie_attention_f32_plan.argtypes = [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int)] * 2
+    return lib
+
+
+@pytest.mark.parametrize("dim,requests,heads,kv_heads,visible,plan", [
+    # (runs, heads a workgroup, waves): short contexts in one run, a head to itself while workgroups are few
+    (128, 1, 12, 2, 30, (1, 1, 4)), (128, 1, 12, 2, 256, (1, 1, 4)), (128, 1, 12, 2, 257, (1, 1, 8)), (128, 1, 12, 2, 512, (1, 1, 8)),
+    (128, 1, 12, 2, 513, (3, 1, 4)), (128, 3, 40, 8, 1136, (5, 3, 4)), (128, 1, 12, 2, 4000, (16, 1, 4)),
+    (64, 8, 8, 2, 500, (1, 1, 8)), (64, 8, 8, 2, 1000, (4, 1, 4)), (64, 37, 14, 2, 2702, (6, 4, 4)), (64, 64, 8, 2, 1000, (1, 2, 8)),
+    (64, 12, 16, 16, 1427, (1, 1, 8)), (64, 2, 16, 16, 1427, (6, 1, 4)), (128, 4, 8, 8, 449, (2, 1, 4)), (128, 32, 8, 8, 449, (1, 1, 8)),
+    (64, 146, 8, 2, 288, (1, 4, 8)), (128, 16, 28, 4, 2058, (3, 4, 4)), (192, 140, 3, 1, 714, (3, 3, 4)), (256, 4, 8, 4, 256, (1, 1, 4)), (256, 4, 8, 4, 400, (2, 1, 4)),
+    (96, 156, 8, 2, 503, (1, 4, 4)), (96, 1, 8, 2, 466, (1, 1, 8)),
+    # heads share a workgroup where their workgroups fill the chip, and four waves where they are more than compute units
+    (128, 64, 12, 2, 128, (1, 3, 4)), (128, 16, 12, 2, 4000, (8, 3, 4)), (128, 64, 12, 2, 1000, (1, 3, 8)),
+    (128, 29, 12, 2, 389, (1, 2, 8)), (128, 32, 8, 8, 1000, (1, 1, 8)), (128, 64, 28, 4, 700, (1, 4, 4)), (64, 127, 16, 4, 128, (1, 4, 4)),
+    # more pairs of token and head than it is for, and a step without keys
+    (128, 128, 16, 4, 700, (1, 0, 0)), (128, 1, 12, 2, 0, (1, 0, 0)),
+])
+def test_float32_attention_of_few_pairs(dim, requests, heads, kv_heads, visible, plan):
+    assert grouped(dim, requests, heads, kv_heads, visible) == plan
+
+
+@pytest.mark.parametrize("dim", [32, 64, 96, 128, 192, 256])
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (7, 1), (12, 2), (8, 8), (28, 4), (40, 8), (5, 1)])
+def test_float32_attention_plans_are_in_bounds(dim, heads, kv_heads):
+    for requests in (1, 2, 3, 7, 16, 33, 64, 100, 200, 2047):
+        for visible in (1, 63, 64, 65, 300, 449, 1153, 5000, 32768):
+            runs, per, waves = grouped(dim, requests, heads, kv_heads, visible)
+            if requests * heads >= 2048:
+                assert (runs, per, waves) == (1, 0, 0)
+                continue
+            assert 1 <= runs <= 16 and 1 <= per <= min(4, heads // kv_heads) and (waves == 4 or (waves == 8 and (dim in (32, 64, 128) or dim == 96 and per == 1)))
+            assert runs * 64 <= max(64, visible)                    # no more runs than chunks of keys
