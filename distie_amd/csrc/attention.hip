@@ -1395,13 +1395,18 @@ __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
 // How many consecutive runs a workgroup puts together, one a wave. 1 as a rule: waves of their own spread best over the
 // chip (8 of them in a workgroup read through one CU: 28 layers, 12 heads on 2, 1 request of 500 keys 1,442 -> 1,537 us,
 // 8 of 2,048 keys 1,577 -> 1,645, 64 of 2,048 keys 2,580 -> 2,640). More than RD_FAST_RUNS partial results, though, cost the
-// reduce 8.9 us a layer instead of 4.6, trip after trip to memory: put together by 8 they fit it (4 requests of 16,000
-// keys 1,861 -> 1,788 us; by 4, which is for heads whose sums would fill the LDS, some 18 us more).
+// reduce 8.9 us a layer instead of 4.6, trip after trip to memory: put together they fit it. By 4 while those workgroups
+// have a compute unit each, by 8 beyond; us a layer apart, by 4, by 8 (both kernels): 12 heads of 128 on 2, 1 request of
+// 16,500 keys 15.0, 13.5, 18.7, of 65,000 28.6, 21.9, 30.1; 4 of 8,000 keys 16.4, 11.2, 13.9; 3 of 16,000 keys (378 workgroups
+// by 4) 24.7, 15.2, 14.5; 28 on 4, 2 of 8,000 keys (256 workgroups) 16.6, 11.2, 13.9, 2 of 20,000 24.7, 20.7, 19.8.
+// Of 240 steps (1 to 4 requests of 4,500 to 65,000 keys, heads of 32 to 256) this is at most 7 % from the best of the three and 2 % from runs apart.
+// By 4 also for heads whose sums would fill the LDS. pairs: (request, kv head) pairs.
 constexpr size_t DECODE_LDS = 64 * 1024;
 constexpr int DECODE_MOST_TOGETHER = D <= 128 ? 8 : 4;        // more than 256 registers a wave: one wave a SIMD
-extern "C" int distie_attention_decode_together(int max_splits, int group) {
+extern "C" int distie_attention_decode_together(int max_splits, int group, int pairs) {
   if (max_splits <= RD_FAST_RUNS || group > 16) return 1;
-  for (int together = DECODE_MOST_TOGETHER; together >= 4; together /= 2)
+  const bool by_four = (max_splits + 3) / 4 <= RD_FAST_RUNS && static_cast<int64_t>((max_splits + 3) / 4) * pairs <= 256;
+  for (int together = by_four ? 4 : DECODE_MOST_TOGETHER; together >= 4; together /= 2)
     if (static_cast<size_t>(together) * group * (D + 2) * sizeof(float) <= DECODE_LDS) return together;
   return 1;
 }
@@ -2208,7 +2213,7 @@ extern "C" int distie_attention_decode_bf16(const void*, int64_t, const void*, c
   return DISTIE_BAD_ARGUMENT;
 }
 
-extern "C" int distie_attention_decode_together(int, int) { return 1; }
+extern "C" int distie_attention_decode_together(int, int, int) { return 1; }
 
 extern "C" int distie_attention_decode_run_len(const int32_t*, int, int, int, int32_t*, hipStream_t) { return DISTIE_BAD_ARGUMENT; }
 

@@ -470,7 +470,7 @@ class HipOps(Ops):
             lib.distie_attention_prefill_f32.argtypes = lib.distie_attention_prefill_bf16.argtypes
             lib.distie_attention_decode_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I,
                                                          _I, _F, _I, _I, _I, _I, _P, _P, _I, _P]
-            lib.distie_attention_decode_together.argtypes = [_I, _I]
+            lib.distie_attention_decode_together.argtypes = [_I, _I, _I]
             lib.distie_attention_decode_run_len.argtypes = [_P, _I, _I, _I, _P, _P]
             if lib.distie_attention_head_dim() != head_dim:
                 raise KernelError("attention library was built for another head size")
@@ -1428,7 +1428,7 @@ class HipOps(Ops):
                        "attention_decode_run_len")
             plan["max_splits"] = max_splits
             # many runs: a workgroup puts consecutive ones together before it writes their result
-            plan["together"] = together = lib.distie_attention_decode_together(max_splits, group)
+            plan["together"] = together = lib.distie_attention_decode_together(max_splits, group, pairs)
             places = -(-max_splits // together)
             plan["decode_o"] = torch.empty((meta.num_requests, num_heads, places, head_dim), dtype=torch.float32,
                                            device=self.device)

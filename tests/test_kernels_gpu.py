@@ -972,13 +972,15 @@ def test_float32_columns_keep_values_from_tokens_that_do_not_see_them(ops, heads
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
-                                                                  (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8)])
-def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, window, together):
+                                                                  (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8),
+                                                                  (12, 2, 128, 16, None, 4), (8, 2, 64, 16, 4500, 4)])
+def test_decode_runs_put_together_in_a_workgroup(ops, heads, kv_heads, dim, P, window, together, monkeypatch):
     """Past 64 runs a request and head, the consecutive runs of a workgroup are put together before their result is
     written: a last workgroup with one, some and all of its runs, a request with one key, one that brings a portion (the
     tiled kernel's), a head with a sink, and places sized for far longer requests. Against plain attention."""
     from distie_amd.kernels.interface import ScoreExtras
 
+    monkeypatch.setattr(ops.attention_library(dim), "distie_attention_decode_together", lambda *sizes: together)
     for lens, q_lens in (([4161, 1, 4609, 5120], [1] * 4), ([4700, 70, 513], [1, 3, 1])):
         meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.bfloat16, seed=7)
         sinks = torch.randn(heads, device="cuda")

@@ -118,3 +118,13 @@ def test_float32_attention_plans_are_in_bounds(dim, heads, kv_heads):
                 continue
             assert 1 <= runs <= 16 and 1 <= per <= min(4, heads // kv_heads) and (waves == 4 or (waves == 8 and (dim in (32, 64, 128) or dim == 96 and per == 1)))
             assert runs * 64 <= max(64, visible)                    # no more runs than chunks of keys
+
+
+@pytest.mark.parametrize("dim,splits,group,pairs,together", [
+    # four while those workgroups have a compute unit each, eight beyond
+    (128, 64, 6, 2, 1), (128, 65, 6, 2, 4), (128, 256, 6, 2, 4), (128, 256, 6, 4, 4), (128, 250, 6, 6, 8), (128, 192, 6, 8, 8),
+    (128, 125, 7, 8, 4), (128, 129, 7, 8, 8), (64, 256, 8, 1, 4), (64, 192, 4, 8, 8),
+    # heads whose sums fill the LDS, and groups that the kernel does not put together
+    (128, 192, 16, 8, 4), (256, 192, 8, 8, 4), (128, 256, 17, 2, 1)])
+def test_runs_of_keys_put_together(dim, splits, group, pairs, together):
+    assert attention(dim).distie_attention_decode_together(splits, group, pairs) == together
