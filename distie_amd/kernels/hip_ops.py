@@ -152,10 +152,20 @@ class HipOps(Ops):
     # float32 products (and products against weights kept in float32) of up to ROWS_MAX_ROWS rows stream the weights
     # through `gemv_rows` (FMAs on the vector ALU); beyond that the tiled float32 kernel
     ROWS_MAX_ROWS = 64
-    # float32 weights below ROWS_F32_MIN_ELEMENTS stay on the vector ALU: such a product is one launch's latency on either unit
+    # float32 products of up to 32 rows on the matrix cores (`rows_f32`), timed beside `gemv_rows` on 42 weights of 0.1 to 105
+    # million elements, each from memory, with the kernel that reads the result (us, `rows_f32` / `gemv_rows`):
+    #  * gated and q/k/v products, with activation, or rotation and cache write, in the epilogue: always (1 row: gate+up [128, 64]
+    #    2.9 / 4.6, [9728, 896] 11.4 / 12.1, [17920, 1536] 23.7 / 26.6, q/k/v [2048, 1536] 7.7 / 11.2; 32 rows 3.8 / 6.1, 20 / 46, 45 /
+    #    82, 13 / 24), but for weights below ROWS_F32_MIN_ELEMENTS, which keep the rounding of the kernel on the vector ALU;
+    #  * plain ones, whose slices of K the reader has to add (`_rows_f32_take`): at up to 4 rows only long weights (1 row: [1536,
+    #    1536] 8.7 / 6.9, [3584, 3584] 19.5 / 14.1, [1536, 8960] 18.7 / 17.2, [5120, 20480] 97 / 89, but [2560, 10240] 29.8 / 32.0,
+    #    [4096, 16384] 54 / 60; 2 to 4 rows: [4096, 10240] 37 / 38 to 43, [2048, 8192] 20 / 19 to 22); at 5 to 8 rows, where the vector
+    #    ALU takes another group of rows, weights past ROWS_F32_EIGHT_ELEMENTS ([2048, 2048] 9.7 / 9.3, [1536, 8960] 18.9 / 23.7);
+    #    beyond, weights of enough rows to fill the chip ([512, 2048] 6.9 / 6.4 at 12 rows, 8.5 / 7.2 at 24; [640, 1600] 7.0 / 7.5 and
+    #    8.8 / 7.8; [768, 768] 7.5 / 7.5 and 8.2 / 9.8; [1536, 1536] 9.4 / 11.4 and 10.7 / 14.4).
     ROWS_F32_MIN_ELEMENTS = 64 << 10
-    ROWS_F32_FEW = 4
-    ROWS_F32_LARGE_ELEMENTS = 8 << 20
+    ROWS_F32_FEW_ELEMENTS = 20 << 20
+    ROWS_F32_EIGHT_ELEMENTS = 4 << 20
     # bfloat16 products by rows of x: up to SKINNY_MAX_ROWS the weights are streamed by one wave per block
     # of 16 weight rows, x straight from memory (above that, the library's tiles are faster);
     SKINNY_MAX_ROWS = 16
@@ -1111,11 +1121,8 @@ class HipOps(Ops):
                 return out
         if both_f32 and partial_ok:
             # few rows in the true 32-bit path, for a caller that takes slices (the head's product does not, and runs at 5
-            # TB/s as it is): the weights streamed through the matrix cores' float32 products. At up to ROWS_F32_FEW rows a
-            # small weight is faster on the vector ALU (one row against [1536, 1536] 4.4 us, 6.1 here)
-            slices = 0
-            if N * K >= self.ROWS_F32_MIN_ELEMENTS and (M > self.ROWS_F32_FEW or N * K >= self.ROWS_F32_LARGE_ELEMENTS):
-                slices = self._ops.distie_rows_f32_slices(M, N, K, 0)
+            # TB/s as it is): the weights streamed through the matrix cores' float32 products
+            slices = self._ops.distie_rows_f32_slices(M, N, K, 0) if self._rows_f32_take(M, N, K) else 0
             if slices:
                 out = torch.empty((M, N) if slices == 1 else (slices, M, N), dtype=torch.float32, device=self.device)
                 _check(self._ops.distie_rows_f32(
@@ -1133,6 +1140,16 @@ class HipOps(Ops):
             x.data_ptr(), _code(x), weight.data_ptr(), _code(weight), bias.data_ptr() if bias is not None else None,
             out.data_ptr(), _CODES[out_dtype], M, N, K, self._stream()), "gemm_generic")
         return out
+
+    def _rows_f32_take(self, M, N, K) -> bool:
+        """Whether a plain float32 product of few rows is the faster one on the matrix cores: see the constants."""
+        if N * K < self.ROWS_F32_MIN_ELEMENTS:
+            return False
+        if M <= 4:
+            return N * K >= self.ROWS_F32_FEW_ELEMENTS and (K >= 4 * N and N <= 4096 if M == 1 else K >= 2 * N)
+        if M <= 8:
+            return N * K > self.ROWS_F32_EIGHT_ELEMENTS
+        return N >= (640 if M <= 16 else 768)
 
     def linear(self, x, weight, bias=None):
         """May return `PartialSums` (see there)."""
