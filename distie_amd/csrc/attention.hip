@@ -722,14 +722,11 @@ __global__ __launch_bounds__(DISTIE_WAVE * CF_WAVES, 1) void attn_columns_f32_ke
 }
 
 // Into how many runs distie_attention_columns_f32 is to cut each tile's keys: enough workgroups for every compute unit twice
-// over, a round of the four waves each at least; 0 where the step is not for it. Against the kernels below, us a call:
-//  - more than 2,048 (token, head) pairs, where a wave a pair walked its keys alone: 300 requests of 600 keys, 8 heads of 128
-//    on 2 273 -> 127, on 4 322 -> 212, 8 of 64 on 2 125 -> 48, 5 single tokens and 12 portions of 24, 8 of 128 on 2 125 -> 26;
-//    a single token and a head of its own each fill one column of sixteen and stay (8 on 8: 389, would be 397);
-//  - heads beyond 128, whose rows leave attn_grouped_f32_kernel one wave a SIMD: 8 heads of 256 on 1, 8 requests of 1,000 keys
-//    30.4 -> 19.7, 5 single tokens and a prompt of 200 90 -> 34, a prompt of 500 378 -> 69, of 1,500 2,736 -> 273; not for single
-//    tokens with few heads to share a row (8 on 4, 8 requests: 22.8, would be 24.0);
-//  - up to 128 that kernel stays for few pairs: its chain is shorter (8 requests of 1,000, 12 of 128 on 2: 14.3, would be 19.2).
+// over, a round of the four waves each at least; 0 where the step is not for it: few pairs of token and head up to heads of
+// 128 (the chain of attn_grouped_f32_kernel is shorter: 8 requests of 1,000 keys, 12 of 128 on 2 14.3 us, would be 19.2), beyond
+// 128 single tokens with few heads to share a row (8 on 4, 8 requests: 22.8, would be 24.0), more pairs where a single token
+// and a head of its own each fill one column of sixteen (300 requests of 600 keys, 8 on 8: 389, would be 397). Where it may
+// be taken, distie_attention_columns_f32_pays says whether it is.
 extern "C" int distie_attention_columns_f32_runs(int tokens, int num_requests, int heads, int kv_heads, int block_size,
                                                  int64_t q_stride, int visible) {
   if (!CF_FITS || tokens < 1 || num_requests < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || kv_heads > 65535 ||
@@ -818,6 +815,53 @@ static GroupedPlan grouped_plan(int64_t tokens, int heads, int kv_heads, int vis
   const bool crowded = per == 0 && !(NARROW && pairs * parts(most) <= 512) && most > 1;
   if (per == 0) per = most;
   return {even(per), four || crowded || even(per) > GQ_EIGHT_HEADS ? 4 : 8, 1};
+}
+
+// Whether distie_attention_columns_f32 in so many runs is faster than the kernels that take the step otherwise, by what each
+// is reckoned to take: whole rounds of workgroups on the compute units (the last one counted half empty), each as long as its
+// waves' trips to memory for a chunk of keys, and the merge of runs. A least-squares fit to 700 steps timed both ways (1 to 400
+// requests of 8 to 2,500 keys, portions of up to 30 tokens, heads of 32 to 256, groups of 1 to 16), off by 11 to 20 %; with a
+// tenth of doubt against the columns what it chooses takes 1 % more than the faster of the two on average. us, columns / otherwise:
+//  * short contexts, where a chunk of columns is mostly empty, stay: 8 heads of 256 on 1, 1 request of 24 keys 12.0 / 9.9; 24 on 2
+//    of 192, 6 of 139 15.9 / 8.8; 16 on 8 of 64, 259 requests of 13 keys 74 / 10; 28 on 4 of 128, 82 of 21 24 / 12;
+//  * many tokens with longer ones, and wide heads, go: 28 on 4 of 64, 151 requests of 1,000 keys 87 / 340; 8 on 1 of 256, 79 of
+//    2,000 92 / 136; 12 on 2 of 256, portions of up to 44 tokens behind 300 keys 91 / 432.
+// visible: the most keys that a token sees, or, behind a window, that its chunks hold.
+extern "C" int distie_attention_columns_f32_pays(int tokens, int num_requests, int heads, int kv_heads, int block_size, int visible,
+                                                 int runs) {
+  if (tokens < 1 || num_requests < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || heads / kv_heads > 16 || visible < 1 ||
+      runs < 1)
+    return 0;
+  const bool few = grouped_fits(tokens, heads);
+  if (few && (block_size < 1 || DISTIE_WAVE % block_size != 0)) return 1;       // (attn_grouped_f32_kernel does not take it)
+  const int group = heads / kv_heads;
+  const int64_t pairs = static_cast<int64_t>(tokens) * heads;
+  const auto rounds = [](int64_t workgroups) {
+    const float x = static_cast<float>(workgroups) / 256;
+    return std::max(1.f, 0.5f * (x + static_cast<float>((workgroups + 255) / 256)));
+  };
+  const auto trips = [&](int chunk, int cut, int waves) {
+    const int chunks = (visible + chunk - 1) / chunk, of_run = (chunks + cut - 1) / cut;
+    return static_cast<float>((of_run + waves - 1) / waves);
+  };
+  const auto merge = [&](float start, float each, int cut) { return cut > 1 ? start + each * pairs * cut * D * 1e-6f : 0.f; };
+  constexpr float WIDTH = D / 256.f;
+  const int64_t tiles = tokens == num_requests ? tokens : tokens / (16 / group) + num_requests;
+  float columns, otherwise;
+  if (few) {
+    const GroupedPlan plan = grouped_plan(tokens, heads, kv_heads, visible);
+    const int64_t workgroups = static_cast<int64_t>(tokens) * kv_heads * ((group + plan.per - 1) / plan.per) * plan.runs;
+    otherwise = -2.3f + rounds(workgroups) * (4.05f + trips(DISTIE_WAVE, plan.runs, plan.waves) * (5.75f + 3.75f * plan.per)) * WIDTH +
+                merge(5.6f, 11.5f, plan.runs);
+    columns = 3.3f + rounds(tiles * kv_heads * runs) * 10.5f * trips(CF_KEYS, runs, CF_WAVES) * WIDTH;
+  } else {
+    // a wave a pair, sixteen of them on a compute unit, key after key
+    const float start = D <= 64 ? 2.35f : D <= 128 ? 1.35f : 2.5f, key0 = D <= 128 ? 6.65f : 8.35f;
+    otherwise = start + std::max(1.f, static_cast<float>(pairs) / 4096) * (key0 + 1.05f * visible) * WIDTH;
+    columns = (D <= 64 ? 3.9f : D <= 128 ? 6.1f : 8.9f) + rounds(tiles * kv_heads * runs) *
+              (D <= 64 ? 27.7f : D <= 128 ? 22.f : 10.1f) * trips(CF_KEYS, runs, CF_WAVES) * WIDTH;
+  }
+  return columns + merge(5.f, 7.3f, runs) < 0.92f * otherwise;
 }
 
 // The plan for a step of distie_attention_generic (float32, plain scores): -> runs, which the caller has buffers for; what a plan

@@ -472,6 +472,7 @@ class HipOps(Ops):
             lib.distie_attention_generic.argtypes = [_P, _I, _L, _P, _P, _I, _P, _P, _P, _I, _P, _P,
                                                      _I, _I, _I, _I, _F, _I, _P, _F, _P, _P, _P, _I, _I, _I, _P]
             lib.distie_attention_columns_f32_runs.argtypes = [_I, _I, _I, _I, _I, _L, _I]
+            lib.distie_attention_columns_f32_pays.argtypes = [_I, _I, _I, _I, _I, _I, _I]
             lib.distie_attention_columns_f32.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I,
                                                          _P, _P, _P, _I, _P]
             lib.distie_attention_f32_plan.argtypes = [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]
@@ -1299,8 +1300,8 @@ class HipOps(Ops):
             return out
         runs = 0
         if plain and f32 and (qkv.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0:
-            runs = lib.distie_attention_columns_f32_runs(T, meta.num_requests, num_heads, num_kv_heads, meta.block_size,
-                                                         qkv.shape[1], min(meta.max_kv, abs(reach) or meta.max_kv))
+            runs = self._columns_runs(lib, T, meta.num_requests, num_heads, num_kv_heads, meta.block_size, qkv.shape[1], meta.max_kv,
+                                      abs(reach))
         if runs > 0:
             # wide heads, or many tokens: a tile of tokens and a kv head's query heads are the columns of matrix products
             part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
@@ -1392,6 +1393,19 @@ class HipOps(Ops):
             plan["partial_o"] = torch.empty((*shape, head_dim), dtype=torch.float32, device=self.device)
             plan["partial_ml"] = torch.empty((*shape, 2), dtype=torch.float32, device=self.device)
         return plan
+
+    COLUMNS_KEYS = 32                # a window's keys begin anywhere in a chunk of so many
+
+    @classmethod
+    def _columns_runs(cls, lib, T, requests, num_heads, num_kv_heads, block_size, stride, max_kv, reach):
+        """The runs of the float32 kernel in columns, 0 where it does not take the step or another kernel is faster."""
+        runs = lib.distie_attention_columns_f32_runs(T, requests, num_heads, num_kv_heads, block_size, stride,
+                                                     min(max_kv, reach or max_kv))
+        if runs > 0:
+            spans = min(max_kv, reach + cls.COLUMNS_KEYS - 1) if reach else max_kv
+            if not lib.distie_attention_columns_f32_pays(T, requests, num_heads, num_kv_heads, block_size, spans, runs):
+                return 0
+        return runs
 
     @staticmethod
     def _grouped_plan(lib, T, num_heads, num_kv_heads, visible):

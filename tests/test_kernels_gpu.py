@@ -919,13 +919,14 @@ def test_float32_products_for_every_head(ops, T, H, N, K, lx, lo):
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(8, 1, 256, 16, None), (16, 1, 256, 4, 130), (3, 1, 192, 12, None),
                                                          (4, 4, 256, 32, 65), (10, 2, 256, 64, None), (64, 4, 128, 16, 100),
                                                          (96, 16, 64, 8, None), (64, 64, 32, 16, None)])
-def test_float32_attention_in_columns(ops, heads, kv_heads, dim, P, window):
+def test_float32_attention_in_columns(ops, heads, kv_heads, dim, P, window, monkeypatch):
     """The float32 kernel whose columns are the heads of a kv head for several tokens: wide heads, or more pairs of token and
     head than the kernels for few take. Single tokens among portions that end inside, at and past a tile of tokens, more
     requests than a wave looks through at once, contexts of 1 to 1,100 keys, one run of keys or several, sinks. Against plain
     attention, and no further from 64 bits than rounding allows: sums over `dim` and over the keys in 32 bits."""
     from distie_amd.kernels.interface import ScoreExtras
 
+    monkeypatch.setattr(ops.attention_library(dim), "distie_attention_columns_f32_pays", lambda *sizes: 1)
     for lens, q_lens in (([1100, 17, 64, 300, 1, 65], [1, 17, 16, 24, 1, 3]), ([31 + 7 * i for i in range(70)], [2 + i % 3 for i in range(70)])):
         meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.float32, seed=11)
         runs = ops.attention_library(dim).distie_attention_columns_f32_runs(qkv.shape[0], len(lens), heads, kv_heads, P,
@@ -943,10 +944,11 @@ def test_float32_attention_in_columns(ops, heads, kv_heads, dim, P, window):
 
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window", [(8, 1, 256, 16, None), (8, 1, 256, 16, 40), (3, 1, 192, 12, 9),
                                                          (64, 8, 128, 16, None), (64, 16, 64, 8, 33)])
-def test_float32_columns_keep_values_from_tokens_that_do_not_see_them(ops, heads, kv_heads, dim, P, window):
+def test_float32_columns_keep_values_from_tokens_that_do_not_see_them(ops, heads, kv_heads, dim, P, window, monkeypatch):
     """Tokens of a tile share the products with V: a value that is not finite, of a key that a later token of the tile brings
     or that has left the window of some of its tokens, reaches the tokens that see the key and no other. Those keep their
     results bit for bit: left out, the key adds nothing, and finite it adds a weight of zero times its value."""
+    monkeypatch.setattr(ops.attention_library(dim), "distie_attention_columns_f32_pays", lambda *sizes: 1)
     lens, q_lens = [37, 90, 64, 130, 300, 71], [5, 16, 3, 30, 2, 24]
     meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.float32, seed=13)
     assert ops.attention_library(dim).distie_attention_columns_f32_runs(qkv.shape[0], len(lens), heads, kv_heads, P,

@@ -140,3 +140,28 @@ def test_float32_attention_plans_are_in_bounds(dim, heads, kv_heads):
     (128, 192, 16, 8, 4), (256, 192, 8, 8, 4), (128, 256, 17, 2, 1)])
 def test_runs_of_keys_put_together(dim, splits, group, pairs, together):
     assert attention(dim).distie_attention_decode_together(splits, group, pairs) == together
+
+
+@pytest.mark.parametrize("dim,tokens,requests,heads,kv_heads,max_kv,window,columns", [
+    # wide heads, few pairs: short contexts and windows stay with the vector kernel
+    (256, 1, 1, 8, 1, 24, 0, False), (256, 8, 8, 8, 1, 1000, 0, False), (192, 6, 6, 24, 2, 139, 0, False), (192, 25, 3, 4, 4, 413, 128, False),
+    (256, 120, 120, 24, 2, 36, 0, True), (256, 79, 79, 8, 1, 2011, 0, True), (256, 23, 23, 7, 1, 1232, 0, True),
+    (192, 56, 8, 28, 4, 63, 0, True),
+    # more pairs, where a wave takes a pair alone otherwise
+    (64, 259, 259, 16, 8, 13, 0, False), (128, 82, 82, 28, 4, 21, 0, False), (64, 332, 332, 9, 3, 24, 0, False),
+    (192, 240, 240, 10, 2, 13, 0, False), (64, 151, 151, 28, 4, 1002, 0, True), (128, 372, 372, 24, 4, 579, 0, True),
+    (256, 430, 119, 12, 2, 306, 0, True), (64, 463, 174, 14, 2, 10000, 128, True), (192, 256, 256, 16, 1, 13, 0, True),
+    # up to 128 the vector kernel keeps few pairs whatever their contexts
+    (128, 8, 8, 12, 2, 4000, 0, False)])
+def test_float32_attention_in_columns_where_it_pays(dim, tokens, requests, heads, kv_heads, max_kv, window, columns):
+    lib = attention(dim)
+    lib.distie_attention_columns_f32_runs.argtypes = [ctypes.c_int] * 5 + [ctypes.c_int64, ctypes.c_int]
+    runs = HipOps._columns_runs(lib, tokens, requests, heads, kv_heads, 16, (heads + 2 * kv_heads) * dim, max_kv, window)
+    assert (runs > 0) == columns
+
+
+def test_wide_heads_on_pages_that_only_columns_take():
+    lib = attention(256)
+    lib.distie_attention_columns_f32_runs.argtypes = [ctypes.c_int] * 5 + [ctypes.c_int64, ctypes.c_int]
+    assert HipOps._columns_runs(lib, 1, 1, 8, 1, 16, 2560, 24, 0) == 0
+    assert HipOps._columns_runs(lib, 1, 1, 8, 1, 12, 2560, 24, 0) == 1
