@@ -161,8 +161,9 @@ class HipOps(Ops):
     #    1536] 8.7 / 6.9, [3584, 3584] 19.5 / 14.1, [1536, 8960] 18.7 / 17.2, [5120, 20480] 97 / 89, but [2560, 10240] 29.8 / 32.0,
     #    [4096, 16384] 54 / 60; 2 to 4 rows: [4096, 10240] 37 / 38 to 43, [2048, 8192] 20 / 19 to 22); at 5 to 8 rows, where the vector
     #    ALU takes another group of rows, weights past ROWS_F32_EIGHT_ELEMENTS ([2048, 2048] 9.7 / 9.3, [1536, 8960] 18.9 / 23.7);
-    #    beyond, weights of enough rows to fill the chip ([512, 2048] 6.9 / 6.4 at 12 rows, 8.5 / 7.2 at 24; [640, 1600] 7.0 / 7.5 and
-    #    8.8 / 7.8; [768, 768] 7.5 / 7.5 and 8.2 / 9.8; [1536, 1536] 9.4 / 11.4 and 10.7 / 14.4).
+    #    beyond, weights of enough rows to fill the chip ([512, 2048] 6.9 / 6.4 at 12 rows, 8.5 / 7.2 at 24; [640, 1600] 7.0 / 7.5 at
+    #    12, 8.8 / 7.8 at 24, where the vector ALU takes three groups of eight rows, and 8.9 / 10.3 at 32, four; [768, 768] 7.5 / 7.5
+    #    and 8.2 / 9.8; [1536, 1536] 9.4 / 11.4 and 10.7 / 14.4).
     ROWS_F32_MIN_ELEMENTS = 64 << 10
     ROWS_F32_FEW_ELEMENTS = 20 << 20
     ROWS_F32_EIGHT_ELEMENTS = 4 << 20
@@ -1150,7 +1151,7 @@ class HipOps(Ops):
             return N * K >= self.ROWS_F32_FEW_ELEMENTS and (K >= 4 * N and N <= 4096 if M == 1 else K >= 2 * N)
         if M <= 8:
             return N * K > self.ROWS_F32_EIGHT_ELEMENTS
-        return N >= (640 if M <= 16 else 768)
+        return N >= (768 if 16 < M <= 24 else 640)
 
     def linear(self, x, weight, bias=None):
         """May return `PartialSums` (see there)."""

@@ -85,7 +85,8 @@ def test_plans_are_kept_apart_by_what_the_rule_reads(rules):
     (1, (3072, 7680), False), (4, (3072, 7680), True), (1, (5120, 20480), False), (2, (5120, 20480), True), (4, (5120, 5120), False),
     (3, (2048, 8192), False),
     (5, (2048, 2048), False), (8, (1024, 4096), False), (5, (1536, 3840), True), (8, (1536, 8960), True), (4, (1536, 3840), False),
-    (9, (1536, 1536), True), (9, (512, 2048), False), (16, (640, 1600), True), (17, (640, 1600), False), (32, (768, 768), True),
+    (9, (1536, 1536), True), (9, (512, 2048), False), (16, (640, 1600), True), (17, (640, 1600), False),
+    (24, (640, 1024), False), (25, (640, 1024), True), (32, (512, 1280), False), (17, (768, 768), True), (32, (768, 768), True),
     (24, (512, 2048), False), (12, (640, 64), False)])
 def test_plain_float32_products_of_few_rows(rules, rows, weight, takes):
     assert rules._rows_f32_take(rows, *weight) == takes
