@@ -1299,13 +1299,18 @@ class HipOps(Ops):
                 plan["prefill_ml"].data_ptr() if parts > 1 else None, parts, sinks_ptr, self._stream()),
                 "attention_prefill_f32")
             return out
-        runs = 0
-        if plain and f32 and (qkv.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0:
-            runs = self._columns_runs(lib, T, meta.num_requests, num_heads, num_kv_heads, meta.block_size, qkv.shape[1], meta.max_kv,
-                                      abs(reach))
-        if runs > 0:
+        columns, runs, per, waves = 0, 1, 0, 0
+        if plain and f32:
+            # which kernel takes the step and how it is cut: the same for every layer with these sizes
+            aligned = (qkv.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
+            key = ("attention_f32_plan", reach, num_heads, num_kv_heads, head_dim, qkv.shape[1], meta.max_kv, aligned)
+            plan = meta.scratch.get(key)
+            if plan is None:
+                plan = meta.scratch[key] = self._plan_f32(lib, meta, T, num_heads, num_kv_heads, qkv.shape[1], abs(reach), aligned)
+            columns, runs, per, waves = plan
+        part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
+        if columns:
             # wide heads, or many tokens: a tile of tokens and a kv head's query heads are the columns of matrix products
-            part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
             _check(lib.distie_attention_columns_f32(
                 qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
                 meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
@@ -1313,13 +1318,6 @@ class HipOps(Ops):
                 part_o.data_ptr() if runs > 1 else None, part_ml.data_ptr() if runs > 1 else None, runs, self._stream()),
                 "attention_columns_f32")
             return out
-        part_o = part_ml = None
-        runs, per, waves = 1, 0, 0
-        if plain and f32:
-            # requests that decode in float32: the keys of a token can be cut into runs that run side by side, so that few
-            # requests occupy the chip as well
-            runs, per, waves = self._grouped_plan(lib, T, num_heads, num_kv_heads, min(meta.max_kv, abs(reach) or meta.max_kv))
-            part_o, part_ml = self._run_parts(meta, runs, T, num_heads, head_dim)
         _check(lib.distie_attention_generic(
             qkv.data_ptr(), _code(qkv), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
             meta.positions.data_ptr(), meta.token_request.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr,
@@ -1407,6 +1405,15 @@ class HipOps(Ops):
             if not lib.distie_attention_columns_f32_pays(T, requests, num_heads, num_kv_heads, block_size, spans, runs):
                 return 0
         return runs
+
+    def _plan_f32(self, lib, meta: BatchMeta, T, num_heads, num_kv_heads, stride, reach, aligned):
+        """(in columns, runs of keys, heads a workgroup, waves) of a float32 step with plain scores. The keys of a token can be
+        cut into runs that run side by side, so that few requests occupy the chip as well."""
+        runs = self._columns_runs(lib, T, meta.num_requests, num_heads, num_kv_heads, meta.block_size, stride, meta.max_kv,
+                                  reach) if aligned else 0
+        if runs > 0:
+            return True, runs, 0, 0
+        return (False, *self._grouped_plan(lib, T, num_heads, num_kv_heads, min(meta.max_kv, reach or meta.max_kv)))
 
     @staticmethod
     def _grouped_plan(lib, T, num_heads, num_kv_heads, visible):
