@@ -9,9 +9,10 @@
 // stages of x and W are under way in registers (waited for by count), x goes from there into LDS (down of the 1.5B shape,
 // [301, 8960] x [1536, 8960]: 20.2 -> 18.1 us; [64, 8960]: 11.5 -> 9.1). Large tiles (DEPTH 2): the matrix cores, which
 // the whole chip's power holds at two thirds of their nominal rate, and the L2 (12 to 17 TB/s reach the compute units):
-// one stage ahead, x without a stop in registers, which the sums need. [2025, 3584] x [37888, 3584] runs at 1,050
-// TFLOP/s, the same loop without any loads at 1,460. Three parts of LDS there, 32 x 32 products, or touching the lines of
-// later stages for the L2 changed nothing or lost up to a fifth.
+// one stage ahead, x without a stop in registers, which the sums need. [2025, 3584] x [37888, 3584] runs at 1,063 TFLOP/s
+// (517 us; gated 957, 573 us in either large tile, where the library and the activation's kernel take 567), the same loop
+// without any loads at 1,460. Three parts of LDS there, 32 x 32 products, or touching the lines of later stages for the L2
+// changed nothing or lost up to a fifth.
 
 #include "common.h"
 #include "packed.h"

@@ -7,11 +7,13 @@
 // owns is free, as W is not packed: gate rows beside their up rows, or the partners of a rotation, so that activation,
 // rotation and cache write happen in the epilogue as in the bfloat16 products.
 //
-// What bounds it: W from memory, at 3.1 to 4.0 TB/s of the 4.7 that a copy reaches (a wave's loads touch 64 bytes of each
-// of 16 rows); the matrix cores need a third of that time. 1.5B shape, cold weights, us, this and the kernel on the vector
-// ALU (gemv_rows) with what stood behind it: gate+up with activation at 1, 8, 32 rows 25.2, 29.8, 47.6 / 32.0, 39.2, 84.6;
-// down in 8 slices at 1, 8, 32 rows 15.9, 17.7, 23.2 / 16.6, 22.6, 40.2; q/k/v with rotation and cache write at 8 rows 8.8 /
-// 14.5. With more than 32 rows the sums' chains no longer fit the registers at the precision of the vector ALU's kernel.
+// What bounds it. Few rows: W from memory, large weights at 3.3 to 4.5 TB/s (a read of weights alone reaches 6.4: a wave's loads
+// touch 64 bytes of each of 16 rows); 32 rows: the matrix instructions and the loads of x beside them, at 2.4 TB/s of W; q/k/v,
+// whose weights are small: its launch and one wave's chain of trips to memory. 1.5B shape, every weight from memory, us and TB/s of
+// W at 1, 8, 32 rows, behind the slash us of the kernel on the vector ALU (gemv_rows) with what stands behind it: gate+up with
+// activation 24.7 (4.5), 27.9 (4.0), 45.5 (2.4) / 27.4, 37.6, 82.2; down in 8 slices 16.1 (3.4), 16.8 (3.3), 22.5 (2.5) / 15.7, 21.7,
+// 37.8; q/k/v with rotation and cache write 7.7 (1.6), 8.8 (1.4), 13.1 (1.0) / 11.2, 13.8, 23.6. With more than 32 rows the
+// sums' chains no longer fit the registers at the precision of the vector ALU's kernel.
 
 #include "common.h"
 #include "packed.h"
