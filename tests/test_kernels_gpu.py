@@ -1091,6 +1091,19 @@ def test_float32_decode_keys_in_runs(ops, heads, kv_heads, dim, P, window, runs,
     assert len(asked) >= 2 * min(4, heads // kv_heads)
 
 
+def test_float32_attention_is_planned_once_a_step(ops, monkeypatch):
+    """The layers of a step share how it is cut; another window, or another longest context, is cut on its own."""
+    meta, qkv, k, v = paged_case(12, 2, 128, 16, [900, 40, 300], [1, 1, 1], torch.float32, seed=5)
+    asked, plan = [], ops._plan_f32
+    monkeypatch.setattr(ops, "_plan_f32", lambda *given: asked.append(given) or plan(*given))
+    for window, limit, plans in ((None, 900, 1), (None, 900, 1), (64, 900, 2), (64, 900, 2), (None, 4096, 3), (None, 900, 3)):
+        meta.max_kv = limit
+        want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, k.double(), v.double(), 12, 2, 128, 128 ** -0.5, window)
+        got = ops.paged_attention(qkv, meta, 0, k, v, 12, 2, 128, 128 ** -0.5, window)
+        close(got, want, torch.float32, scale=want.abs().max().item())
+        assert len(asked) == plans
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P", [(12, 2, 128, 16), (4, 2, 64, 16), (3, 1, 48, 16), (2, 1, 256, 32)])
 @pytest.mark.parametrize("per_key", [0.1, 1.0, -0.1, 0.02])
 @pytest.mark.parametrize("dtype", DTYPES)
