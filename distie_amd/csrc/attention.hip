@@ -777,6 +777,10 @@ struct GroupedPlan {
 //    1 request, 12 heads of 128 on 2: 200 keys 8.6 / 8.4, 400 keys 11.9 / 11.9 (two runs: 14.2), 700 keys 16.0 / 11.8, 1,000 keys
 //    24.9 / 13.9, 4,000 keys 82 / 15.2. Runs of one chunk a wave, or of as many as the chip has room for: 512 workgroups of
 //    four waves, fewer where contexts are short for heads of 64 or the registers hold one wave a SIMD, more for long ones;
+//    Heads of 96 and 128 then take as many runs as there is room for: a captured step is made for longer contexts than it
+//    holds, and of 100 steps of 300 to 5,400 keys (half of them under twice the bound) none was more than 1 % slower, the
+//    rest by up to 28 % faster (24 requests of 1,050 keys planned for 2,048, 16 heads on 4: 29 -> 22 us). Heads of 64 do not:
+//    up to 16 % slower where the bound is the context (17 requests of 4,600 keys, 16 on 4: 33, would be 38);
 //  * heads share a workgroup, and a row of K its load, as far as the chip is full without it: 64 requests of 128 keys, 12 heads
 //    of 128 on 2 14.9 / 11.8; a head to itself otherwise (8 requests of 128 keys 8.8 / 8.6, in threes 11.2);
 //  * without runs four waves for up to four chunks, then eight, but for more workgroups than compute units, which run two at a
@@ -799,14 +803,18 @@ static GroupedPlan grouped_plan(int64_t tokens, int heads, int kv_heads, int vis
     const bool lasting = chunks > 18;
     const int64_t apart = NARROW && lasting ? 512 : 256;              // workgroups up to which heads are kept apart
     const int64_t room = NARROW ? (!lasting ? 256 : most == 4 ? 1024 : 512) : D > 192 && !lasting ? 320 : 512;
+    const auto filled = [&](int per, int64_t limit, int runs) {          // as many as there is room for, a chunk a wave or more
+      if (NARROW || WIDE) return runs;
+      return std::max(runs, static_cast<int>(std::min<int64_t>({GQ_MAX_RUNS, limit / (pairs * parts(per)), chunks / 4})));
+    };
     for (int trips = 1;; ++trips) {                             // chunks that a wave takes one after the other
       const int runs = std::min(GQ_MAX_RUNS, (chunks + 4 * trips - 1) / (4 * trips));
       // two runs of four waves are one run of eight, where those fit; side by side they spread better for heads of their own
       const bool two = WIDE || (most == 1 && trips == 1);
       if (runs < (two ? 2 : 3)) break;
       const int per = fewest(apart, runs);
-      if (per > 0) return {even(per), 4, runs};
-      if (pairs * parts(most) * runs <= room && (WIDE || runs > 2)) return {even(most), 4, runs};
+      if (per > 0) return {even(per), 4, filled(per, parts(per) == parts(most) ? room : apart, runs)};
+      if (pairs * parts(most) * runs <= room && (WIDE || runs > 2)) return {even(most), 4, filled(most, room, runs)};
     }
   }
   const bool four = WIDE || chunks <= 4;

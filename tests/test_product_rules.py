@@ -108,7 +108,7 @@ def attention(dim):
     (128, 1, 12, 2, 513, (3, 1, 4)), (128, 3, 40, 8, 1136, (5, 3, 4)), (128, 1, 12, 2, 4000, (16, 1, 4)),
     (64, 8, 8, 2, 500, (1, 1, 8)), (64, 8, 8, 2, 1000, (4, 1, 4)), (64, 37, 14, 2, 2702, (6, 4, 4)), (64, 64, 8, 2, 1000, (1, 2, 8)),
     (64, 12, 16, 16, 1427, (1, 1, 8)), (64, 2, 16, 16, 1427, (6, 1, 4)), (128, 4, 8, 8, 449, (2, 1, 4)), (128, 32, 8, 8, 449, (1, 1, 8)),
-    (64, 146, 8, 2, 288, (1, 4, 8)), (128, 16, 28, 4, 2058, (3, 4, 4)), (192, 140, 3, 1, 714, (3, 3, 4)), (256, 4, 8, 4, 256, (1, 1, 4)), (256, 4, 8, 4, 400, (2, 1, 4)),
+    (64, 146, 8, 2, 288, (1, 4, 8)), (128, 16, 28, 4, 2058, (4, 4, 4)), (128, 32, 12, 2, 1400, (4, 3, 4)), (128, 23, 16, 4, 2048, (5, 4, 4)), (64, 23, 16, 4, 2048, (8, 4, 4)), (192, 140, 3, 1, 714, (3, 3, 4)), (256, 4, 8, 4, 256, (1, 1, 4)), (256, 4, 8, 4, 400, (2, 1, 4)),
     (96, 156, 8, 2, 503, (1, 4, 4)), (96, 1, 8, 2, 466, (1, 1, 8)),
     # heads share a workgroup where their workgroups fill the chip, and four waves where they are more than compute units
     (128, 64, 12, 2, 128, (1, 3, 4)), (128, 16, 12, 2, 4000, (8, 3, 4)), (128, 64, 12, 2, 1000, (1, 3, 8)),
