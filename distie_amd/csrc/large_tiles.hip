@@ -1,0 +1,445 @@
+// Products of many rows (portions of prompts, prompts of a few hundred tokens) on packed weight copies: y[M, N] = x[M, K]
+// W[N, K]^T for bfloat16 x and the copies of packed.h, with the activation, or rotation and cache write, in the epilogue.
+//
+// A workgroup of 2 x 2 waves owns a tile of 64 TM rows of x and 64 TN rows of W and one slice of K; a wave owns 32 TM x 32 TN of
+// it as TM x TN products of 32 x 32 x 16, whose sums stay in the accumulation registers. x and W both go straight from memory
+// into LDS: x in stages of 64 k, three of them (whole lines of 128 bytes: halves cost the L2 twice the requests), W, whose copy
+// lies in lane order, in halves of a stage, four of them. The waits count loads, so that one to two stages are under way all the
+// time; reads of LDS and loads stand between the matrix instructions of the 16 k before.
+//
+// What bounds it. [4096, 4096] x [4096, 4096] takes 110 us (1,244 TFLOP/s; the library 98): the matrix cores are 90 % busy and the
+// chip's power holds the clock at 1.45 GHz, whatever the loop does (eight waves of 128 x 64, which read half as much again from
+// LDS, take 2,570 to 2,940 cycles a stage instead of 2,270 and the same 124 us at 1.58 to 1.81 GHz). That is why a wave owns as
+// much as it can hold. Smaller tiles run into the L2, which gives the chip's LDS 15 to 17 TB/s: 128 x 128 need 32 KB for 512
+// cycles of products (fragments of a whole stage read ahead changed nothing). With few rows it is the weight from memory.
+// 1.5B shape, 2,048 rows, isolated and with the kernel that the library needs behind its own: gate+up with its activation 104 us
+// (129), down in four slices 54 (80; the norm reads 12 us more). 7B shape, 2,025 rows: 460 (567) and 220 (359; packed_tiles
+// 261). 301 rows: gate+up of the 1.5B shape 25 us, 36 in packed_tiles.
+
+#include "common.h"
+#include "packed.h"
+#include <algorithm>
+
+namespace {
+
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+typedef __attribute__((__vector_size__(4 * sizeof(int)))) int intx4;
+typedef __attribute__((address_space(3))) void lds_void;
+
+constexpr int LT_K = 64;              // k of a stage of x; W comes in halves of it
+constexpr int LT_X_STAGES = 3, LT_W_PARTS = 4;
+
+// A buffer of `bytes` from `base` on (both the same in all lanes): reads beyond it give zeros.
+__device__ __forceinline__ intx4 buffer_of(const void* base, uint32_t bytes) {
+  const uint64_t at = reinterpret_cast<uint64_t>(base);
+  intx4 d;
+  d[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(at));
+  d[1] = __builtin_amdgcn_readfirstlane(static_cast<int>(at >> 32) & 0xffff);
+  d[2] = __builtin_amdgcn_readfirstlane(static_cast<int>(bytes));
+  d[3] = 0x00020000;
+  return d;
+}
+
+// Sixteen bytes a lane from `from` + lane_at + wave_at into LDS, the lanes' pieces one behind the other from `to` on. The wait
+// is the caller's. The s_nop is the wait state between writing m0 and the load.
+__device__ __forceinline__ void buffer_to_lds(const intx4& from, int lane_at, int wave_at, uint32_t to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(lane_at), "s"(from),
+               "s"(wave_at)
+               : "m0");
+}
+
+// All but the newest LEFT loads into LDS of this wave have arrived and what it read from LDS is in its registers; then the
+// same for all waves.
+template <int LEFT>
+__device__ __forceinline__ void arrived() {
+  static_assert(LEFT < 64, "the counter's range");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The workgroups of a launch: workgroup i runs on die i % 8 and every die gets a run of neighbouring tiles, the rows of x
+// fastest, so that the tiles at work on a die share W and x through its L2.
+struct LargePlace {
+  int row_blocks;               // blocks of 16 rows of the packed copy
+  int m_tiles, n_tiles, slices;
+  int stages;                   // of a slice
+};
+
+// MODE: PK_PLAIN, PK_GATED, PK_ROTARY. K a multiple of LT_K; columns of y a multiple of 16 bytes.
+template <int TM, int TN, int MODE, typename Y>
+__global__ __launch_bounds__(256, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias, Y* __restrict__ y, int M, int N,
+    int K, LargePlace at, RotaryOut rotary) {
+  constexpr int BM = 64 * TM, BN = 64 * TN;            // of the workgroup: 2 x 2 waves
+  constexpr int X_BYTES = BM * LT_K * 2, W_BYTES = BN * LT_K;
+  constexpr int W_AT = LT_X_STAGES * X_BYTES;
+  constexpr int LDS_BYTES = W_AT + LT_W_PARTS * W_BYTES;
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS of a compute unit");
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int r = lane % 32, h = lane / 32;
+  const int wm = wave % 2, wn = wave / 2;
+  const int tiles = at.m_tiles * at.n_tiles;
+  const int place = static_cast<int>(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  if (place >= tiles * at.slices) return;
+  const int slice = place / tiles, n_tile = place % tiles / at.m_tiles, m_tile = place % at.m_tiles;
+  const int m0 = m_tile * BM, b0 = n_tile * (BN / 16);
+  const int s_begin = slice * at.stages;
+  const int stages = min(K / LT_K - s_begin, at.stages);
+  const int k_tiles = K / 32;
+
+  const int rows = min(M - m0, BM), blocks = min(at.row_blocks - b0, BN / 16);
+  const intx4 x_buffer = buffer_of(x + static_cast<int64_t>(m0) * K, static_cast<uint32_t>(rows) * K * 2u);
+  const intx4 w_buffer =
+      buffer_of(w + static_cast<int64_t>(b0) * k_tiles * PK_TILE, static_cast<uint32_t>(blocks) * k_tiles * 1024u);
+  // A row of x's stage is eight pieces of 16 bytes; eight neighbouring lanes bring a row, piece p to place p ^ (row / 2 % 8), so
+  // that the rows a product reads at once spread over all banks. Rows and blocks beyond the last are read from it and dropped.
+  int x_lane[2 * TM], w_lane[TN];
+#pragma unroll
+  for (int p = 0; p < 2 * TM; ++p) {
+    const int row = 8 * (wave * 2 * TM + p) + lane / 8;
+    x_lane[p] = min(row, rows - 1) * K * 2 + 16 * ((lane % 8) ^ ((row >> 1) & 7));
+  }
+#pragma unroll
+  for (int p = 0; p < TN; ++p) w_lane[p] = min(wave * TN + p, blocks - 1) * k_tiles * 1024 + lane * 16;
+  const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds)));
+  auto bring_x = [&](int stage, int slot, int p) {
+    buffer_to_lds(x_buffer, x_lane[p], (s_begin + min(stage, stages - 1)) * (LT_K * 2),
+                  base + slot * X_BYTES + (wave * 2 * TM + p) * 1024);
+  };
+  auto bring_w = [&](int part, int p) {
+    buffer_to_lds(w_buffer, w_lane[p], (2 * s_begin + min(part, 2 * stages - 1)) * 1024,
+                  base + W_AT + part % LT_W_PARTS * W_BYTES + (wave * TN + p) * 1024);
+  };
+
+  // acc[a][b][4 q + i]: row 8 (q % 2) + 4 h + i of block first_block + 2 b + q / 2, row 32 a + r of the wave's part of x
+  floatx16 acc[TM][TN];
+  const int first_block = b0 + wn * TN * 2;
+#pragma unroll
+  for (int b = 0; b < TN; ++b) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float4 start = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (MODE != PK_GATED) {
+        const int block = first_block + 2 * b + q / 2;
+        const int column = MODE == PK_ROTARY ? rotary_column(block, 2 * (q % 2) + h, rotary.heads + rotary.kv_heads, rotary.dim)
+                                             : 16 * block + 8 * (q % 2) + 4 * h;
+        if (bias != nullptr && slice == 0 && block < at.row_blocks && column < N)
+          start = *reinterpret_cast<const float4*>(bias + column);
+      }
+#pragma unroll
+      for (int a = 0; a < TM; ++a) {
+        acc[a][b][4 * q] = start.x, acc[a][b][4 * q + 1] = start.y;
+        acc[a][b][4 * q + 2] = start.z, acc[a][b][4 * q + 3] = start.w;
+      }
+    }
+  }
+
+  const int x_row = (wm * TM * 32 + r) * (LT_K * 2), x_turn = (r >> 1) & 7;
+  bf16x8 fx[2][TM], fw[2][TN];
+  const int w_at = W_AT + (wn * TN * 2 + r / 16) * 1024 + (h * 16 + r % 16) * 16;
+  auto read = [&](int t, int x_slot, int w_slot, int set, int i) {
+    if (i < TN)
+      fw[set][i] = *reinterpret_cast<const bf16x8*>(lds + w_slot * W_BYTES + w_at + 2 * i * 1024 + t % 2 * 512);
+    else
+      fx[set][i - TN] = *reinterpret_cast<const bf16x8*>(lds + x_slot * X_BYTES + x_row + 16 * ((2 * t + h) ^ x_turn) +
+                                                         (i - TN) * 32 * LT_K * 2);
+  };
+  // The products of set `set`; between them the reads of the next 16 k, and `loads` loads into LDS.
+  auto multiply = [&](int set, int t, int x_slot, int w_slot, int loads, auto&& load) {
+    constexpr int ALL = TM * TN, READS = TM + TN;
+#pragma unroll
+    for (int i = 0; i < ALL; ++i) {
+      const int b = i / TM, a = i % TM;
+      acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[set][b], fx[set][a], acc[a][b], 0, 0, 0);
+#pragma unroll
+      for (int q = i * READS / ALL; q < (i + 1) * READS / ALL; ++q) read(t, x_slot, w_slot, 1 - set, q);
+#pragma unroll
+      for (int q = i * loads / ALL; q < (i + 1) * loads / ALL; ++q) load(q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // Past the last stage the loads bring it once more, so that their number, which the waits count, stays what it is.
+#pragma unroll
+  for (int p = 0; p < 2 * TM; ++p) bring_x(0, 0, p);
+#pragma unroll
+  for (int p = 0; p < TN; ++p) bring_w(0, p);
+#pragma unroll
+  for (int p = 0; p < TN; ++p) bring_w(1, p);
+#pragma unroll
+  for (int p = 0; p < TM; ++p) bring_x(1, 1, p);
+#pragma unroll
+  for (int p = 0; p < TN; ++p) bring_w(2, p);
+#pragma unroll
+  for (int p = TM; p < 2 * TM; ++p) bring_x(1, 1, p);
+#pragma unroll
+  for (int p = 0; p < TN; ++p) bring_w(3, p);
+  arrived<3 * TN + 2 * TM>();
+#pragma unroll
+  for (int i = 0; i < TM + TN; ++i) read(0, 0, 0, 0, i);
+  // Iteration s holds x(s) and W's parts 2 s and 2 s + 1. Before the first wait W(2 s + 1) has to be there, and behind it in order
+  // stand x(s + 1) and halves of it, W(2 s + 2), W(2 s + 3) and half of x(s + 2); before the second x(s + 1) and W(2 s + 2). A
+  // wait also says that all waves have read what the loads behind it write over.
+  int slot = 0;
+  for (int s = 0; s < stages; ++s) {
+    const int next = slot == LT_X_STAGES - 1 ? 0 : slot + 1, free = slot == 0 ? LT_X_STAGES - 1 : slot - 1;
+    const int w_slot = 2 * (s % 2);
+    multiply(0, 1, slot, w_slot, TM, [&](int q) { bring_x(s + 2, free, q); });
+    arrived<3 * TM + 2 * TN>();
+    multiply(1, 2, slot, w_slot + 1, TN, [&](int q) { bring_w(2 * s + 4, q); });
+    multiply(0, 3, slot, w_slot + 1, TM, [&](int q) { bring_x(s + 2, free, TM + q); });
+    arrived<2 * TM + 2 * TN>();
+    multiply(1, 0, next, 2 - w_slot, TN, [&](int q) { bring_w(2 * s + 5, q); });
+    slot = next;
+  }
+  arrived<0>();
+
+  // The results of 32 rows of x and up to 128 bytes of columns at a time go through LDS, so that rows leave in whole lines.
+  constexpr int EACH = MODE == PK_GATED ? 16 : 32;                                  // columns of y that 32 rows of W give
+  constexpr int GROUP = 128 / (EACH * static_cast<int>(sizeof(Y)));                 // so many blocks of 32 at a time
+  constexpr int STRIDE = 128 + 16, PIECE = 16 / static_cast<int>(sizeof(Y));        // bytes of a row there; values of a store
+  char* own = lds + wave * (32 * STRIDE);
+  const int columns = MODE == PK_GATED ? N / 2 : N;
+  const int column0 = first_block * (MODE == PK_GATED ? 8 : 16);
+  Y* out = y + static_cast<int64_t>(slice) * M * N;
+  const int half = rotary.dim / 2, per_head = rotary.dim / 16, turned = rotary.heads + rotary.kv_heads;      // (PK_ROTARY)
+  // first and second: four values each of the two halves of a block, of token m; turns the pairs of q and k, and puts the values
+  // into their cache, where neighbouring tokens lie side by side
+  auto turn = [&](float* first, float* second, int m, int block) {
+    const int head = block / per_head, sub = block % per_head;
+    if (head < turned) {
+      const float4* angles =
+          reinterpret_cast<const float4*>(rotary.table + static_cast<int64_t>(min(m, M - 1)) * half + 8 * sub + 4 * h);
+      const float4 low = angles[0], high = angles[1];
+      const float c[4] = {low.x, low.z, high.x, high.z}, s[4] = {low.y, low.w, high.y, high.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float one = first[i], two = second[i];
+        first[i] = one * c[i] - two * s[i];
+        second[i] = two * c[i] + one * s[i];
+      }
+    } else if (rotary.write && m < M && block < at.row_blocks) {
+      const int slot = rotary.slots[m];
+      const int64_t page = slot / rotary.block_size, row = 16 * sub + 4 * h;
+      Y* value = reinterpret_cast<Y*>(rotary.v_cache) +
+                 ((page * rotary.kv_heads + head - turned) * rotary.dim + row) * rotary.block_size + slot % rotary.block_size;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        value[static_cast<int64_t>(i) * rotary.block_size] = from_float<Y>(first[i]);
+        value[static_cast<int64_t>(8 + i) * rotary.block_size] = from_float<Y>(second[i]);
+      }
+    }
+  };
+  auto finish = [&](auto&& gated) {
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+      const int row0 = m0 + (wm * TM + a) * 32;
+#pragma unroll
+      for (int g = 0; g < TN; g += GROUP) {
+        const int count = TN - g < GROUP ? TN - g : GROUP;
+#pragma unroll
+        for (int b = g; b < g + count; ++b) {
+          char* to = own + r * STRIDE + ((b - g) * EACH + 4 * h) * sizeof(Y);
+#pragma unroll
+          for (int q = 0; q < 4; q += MODE == PK_PLAIN ? 1 : 2) {
+            float v[4], v2[4];
+            if constexpr (MODE == PK_GATED) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v[i] = gated(acc[a][b][4 * q + i], acc[a][b][4 * q + 4 + i]);
+              *reinterpret_cast<uint2*>(to + q / 2 * 8 * sizeof(Y)) = pack_bf16x4(v);
+            } else if constexpr (MODE == PK_ROTARY) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v[i] = acc[a][b][4 * q + i], v2[i] = acc[a][b][4 * q + 4 + i];
+              turn(v, v2, row0 + r, first_block + 2 * b + q / 2);
+              *reinterpret_cast<uint2*>(to + q * 8 * sizeof(Y)) = pack_bf16x4(v);
+              *reinterpret_cast<uint2*>(to + (q + 1) * 8 * sizeof(Y)) = pack_bf16x4(v2);
+            } else {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v[i] = acc[a][b][4 * q + i];
+              if constexpr (sizeof(Y) == 2) *reinterpret_cast<uint2*>(to + q * 8 * sizeof(Y)) = pack_bf16x4(v);
+              else *reinterpret_cast<float4*>(to + q * 8 * sizeof(Y)) = float4{v[0], v[1], v[2], v[3]};
+            }
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const int pieces = count * EACH / PIECE;           // of a row
+#pragma unroll
+        for (int i = 0; i < 32 * pieces / 64; ++i) {
+          const int e = 64 * i + lane, row = e / pieces, piece = e % pieces;
+          const uint4 v = *reinterpret_cast<const uint4*>(own + row * STRIDE + 16 * piece);
+          if constexpr (MODE == PK_ROTARY) {
+            // a piece is half a block: eight neighbouring columns of a head
+            const int block = first_block + 2 * g + piece / 2;
+            if (row0 + row < M && block < at.row_blocks) {
+              const int column = rotary_column(block, 2 * (piece % 2), turned, rotary.dim);
+              *reinterpret_cast<uint4*>(out + static_cast<int64_t>(row0 + row) * N + column) = v;
+              const int head = block / per_head;
+              if (rotary.write && head >= rotary.heads && head < turned) {
+                const int slot = rotary.slots[row0 + row];
+                const int64_t page = slot / rotary.block_size;
+                Y* key = reinterpret_cast<Y*>(rotary.k_cache) +
+                         ((page * rotary.kv_heads + head - rotary.heads) * rotary.block_size + slot % rotary.block_size) * rotary.dim;
+                *reinterpret_cast<uint4*>(key + column - head * rotary.dim) = v;
+              }
+            }
+          } else {
+            const int column = column0 + g * EACH + piece * PIECE;
+            if (row0 + row < M && column < columns)
+              *reinterpret_cast<uint4*>(out + static_cast<int64_t>(row0 + row) * columns + column) = v;
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+    }
+  };
+  // silu on the units' own exp2 and reciprocal (each within one place of float32; the result is rounded to 8 bits): the library's
+  // expf and a true division, four times the instructions, took 9 us a tile of 256 x 256, a quarter of its products at K = 1,536.
+  if (MODE == PK_GATED && rotary.act == 0) {
+    finish([](float gate, float up) {
+      return gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.442695040889f * gate)) * up;
+    });
+  } else {
+    finish([&](float gate, float up) { return gated_value(gate, up, rotary.act, rotary.limit, rotary.slope, rotary.up_shift); });
+  }
+}
+
+// The tiles there are, and what a workgroup of one takes: for every stage few_us with hardly any compute unit at work, more_us
+// on top of it with all of them (the L2; and power: the clock falls from 2.4 to 1.45 GHz) and pair_us where two share them, and
+// turn_us to begin and end.
+struct LargeShape {
+  int tm, tn;
+  float few_us, more_us, pair_us, turn_us;
+};
+constexpr LargeShape LARGE_SHAPES[] = {{4, 4, 0.893f, 0.515f, 0.f, 6.7f},  {4, 3, 0.684f, 0.451f, 0.f, 5.3f},
+                                       {3, 4, 0.692f, 0.446f, 0.f, 5.7f},  {3, 3, 0.558f, 0.371f, 0.f, 4.3f},
+                                       {2, 4, 0.528f, 0.373f, 0.f, 3.4f},  {3, 2, 0.386f, 0.317f, 0.f, 2.7f},
+                                       {2, 3, 0.407f, 0.327f, 0.f, 2.55f}, {2, 2, 0.280f, 0.336f, 0.497f, 1.8f}};
+constexpr int LARGE_SHAPE_COUNT = static_cast<int>(sizeof(LARGE_SHAPES) / sizeof(LARGE_SHAPES[0]));
+constexpr float LARGE_GATED_TURN = 0.81f, LARGE_ROTARY_TURN = 3.4f;     // (half the stores; angles and the caches' stores)
+
+struct LargePlan {
+  int shape, slices;
+  float us;
+};
+
+// How a product is cut, as plan_tiles: whole rounds of workgroups on the compute units, the last of them with as many as are
+// left, no faster than memory brings W, and what the reader of the result moves. The numbers are a least-squares fit to 16,000
+// timings (25 weights of 0.9 to 136 million elements, 65 to 2,048 rows, in a captured graph; the fit is off by 6 %). What the
+// count chooses takes 2.8 % more than the best of them on average.
+LargePlan plan_large(int M, int N, int K, int row_blocks, int mode, bool may_cut, float cut_us) {
+  LargePlan best = {-1, 0, 0.f};
+  const int all = K / LT_K;
+  const float memory_us = static_cast<float>(row_blocks) * K * 32.f / 3.8e6f, values = static_cast<float>(M) * N;
+  for (int i = 0; i < LARGE_SHAPE_COUNT; ++i) {
+    const LargeShape& s = LARGE_SHAPES[i];
+    if (mode == PK_ROTARY && s.tm * s.tn > 12) continue;         // (its sums and angles do not fit the registers)
+    const int64_t tiles = static_cast<int64_t>((M + 64 * s.tm - 1) / (64 * s.tm)) * ((row_blocks + 4 * s.tn - 1) / (4 * s.tn));
+    const float turn = s.turn_us * (mode == PK_GATED ? LARGE_GATED_TURN : mode == PK_ROTARY ? LARGE_ROTARY_TURN : 1.f);
+    for (int cut = 1; cut <= 8; ++cut) {
+      if (cut > 1 && (!may_cut || all / cut < 6)) break;
+      const int stages = (all + cut - 1) / cut;
+      if ((all + stages - 1) / stages != cut) continue;
+      const int64_t units = s.pair_us > 0.f ? 512 : 256, work = tiles * cut, full = work / units, rest = work % units;
+      const float busy = rest / 256.f;
+      float us = full * (stages * (s.few_us + s.more_us + s.pair_us) + turn);
+      if (rest > 0) us += stages * (s.few_us + s.more_us * std::min(busy, 1.f) + s.pair_us * std::max(busy - 1.f, 0.f)) + turn;
+      us = 2.2f + std::max(us, memory_us);
+      if (cut > 1) us += 4.f * cut * values / 8.0e6f;
+      if (mode == PK_PLAIN && may_cut) {
+        if (cut_us == 0.f) us += std::max(3.7f, 3.8f + (4.f * cut + 10.f) * values / 8.6e6f);      // the norm that adds the slices
+        else if (cut > 1) us += cut_us + (4.f * cut + 2.f) * values / 8.6e6f;
+      }
+      if (best.shape < 0 || us < best.us) best = {i, cut, us};
+    }
+  }
+  return best;
+}
+
+template <int MODE, typename Y>
+int launch_large(const bf16_t* x, const bf16_t* w, const float* bias, Y* y, int M, int N, int K, int row_blocks, int shape,
+                 int slices, const RotaryOut& rotary, hipStream_t stream) {
+  const int bm = 64 * LARGE_SHAPES[shape].tm, blocks = 4 * LARGE_SHAPES[shape].tn;
+  const int all = K / LT_K;
+  const LargePlace at = {row_blocks, (M + bm - 1) / bm, (row_blocks + blocks - 1) / blocks, slices, (all + slices - 1) / slices};
+  if ((all + at.stages - 1) / at.stages != slices) return DISTIE_BAD_ARGUMENT;
+  const int64_t work = static_cast<int64_t>(at.m_tiles) * at.n_tiles * slices;
+  if (work > (1 << 30)) return DISTIE_BAD_ARGUMENT;
+  const unsigned grid = static_cast<unsigned>((work + 7) / 8 * 8);
+#define LARGE(TM, TN)                                                                                                     \
+  large_tiles_kernel<TM, TN, MODE, Y><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, at, rotary);                      \
+  break
+  switch (shape) {
+    case 0:
+      if constexpr (MODE == PK_ROTARY) return DISTIE_BAD_ARGUMENT;
+      else {
+        LARGE(4, 4);
+      }
+    case 1: LARGE(4, 3);
+    case 2: LARGE(3, 4);
+    case 3: LARGE(3, 3);
+    case 4: LARGE(2, 4);
+    case 5: LARGE(3, 2);
+    case 6: LARGE(2, 3);
+    default: LARGE(2, 2);
+  }
+#undef LARGE
+  return launch_status();
+}
+
+bool aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+// How the kernels of this file cut a product, 0 if they do not take it, as distie_packed_tiles_plan. mode: 0 plain, 1 gated, 2
+// with rotation and cache write; *us: what the count comes to.
+extern "C" int distie_large_tiles_plan(int M, int N, int K, int mode, int may_cut, float cut_us, int* shape, int* slices,
+                                       float* us) {
+  if (M < 1 || N < 16 || K < 4 * LT_K || K % LT_K != 0 || mode < 0 || mode > 2 || N % (mode == PK_GATED ? 16 : 8) != 0 ||
+      (mode == PK_ROTARY && N % 16 != 0) || K > (1 << 20))
+    return 0;
+  const LargePlan plan = plan_large(M, N, K, (N + 15) / 16, mode, may_cut != 0 && mode == PK_PLAIN, cut_us);
+  *shape = plan.shape, *slices = plan.slices, *us = plan.us;
+  return 1;
+}
+
+// y: [M, N] of y_dtype (gated: [M, N / 2] in bfloat16), or with slices > 1 float32 [slices, M, N], to be added in order by
+// whoever reads it, the bias in the first. All pointers at multiples of 16 bytes.
+extern "C" int distie_large_tiles_bf16(const void* x, const void* w_packed, const float* bias, void* y, int y_dtype, int M,
+                                       int N, int K, int gated, int shape, int slices, float limit, float slope, float up_shift,
+                                       hipStream_t stream) {
+  if (M <= 0) return 0;
+  const int act = gated >> 8;           // the activation on the gate, above the low eight bits
+  gated &= 0xff;
+  if (N < 16 || K < 4 * LT_K || K % LT_K != 0 || K > (1 << 20) || shape < 0 || shape >= LARGE_SHAPE_COUNT || slices < 1 ||
+      gated > 1 || N % (gated ? 16 : 8) != 0 || (gated && (slices != 1 || y_dtype != DISTIE_BF16 || bias != nullptr)) ||
+      act < 0 || act > 5 || (act == 5 && !(limit > 0.f)) || (slices > 1 && y_dtype != DISTIE_F32) || !aligned(x) ||
+      !aligned(w_packed) || !aligned(bias) || !aligned(y))
+    return DISTIE_BAD_ARGUMENT;
+  RotaryOut out = {};
+  out.act = act, out.limit = limit, out.slope = slope, out.up_shift = up_shift;
+  const bf16_t* xb = static_cast<const bf16_t*>(x);
+  const bf16_t* wb = static_cast<const bf16_t*>(w_packed);
+  const int blocks = (N + 15) / 16;
+  if (gated) return launch_large<PK_GATED, bf16_t>(xb, wb, nullptr, static_cast<bf16_t*>(y), M, N, K, blocks, shape, 1, out, stream);
+  DISTIE_DISPATCH(y_dtype, Y, return (launch_large<PK_PLAIN, Y>(xb, wb, bias, static_cast<Y*>(y), M, N, K, blocks, shape, slices,
+                                                                out, stream)));
+  return DISTIE_BAD_ARGUMENT;
+}
+
+// The stacked q/k/v product with rotation and cache write in its epilogue, as distie_gemm_packed_rotary_bf16.
+extern "C" int distie_large_tiles_rotary_bf16(const void* x, const void* w_packed, const float* bias, void* y, const void* table,
+                                              const int32_t* slots, void* k_cache, void* v_cache, int M, int K, int heads,
+                                              int kv_heads, int dim, int block_size, int write, int shape, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (K < 4 * LT_K || K % LT_K != 0 || K > (1 << 20) || heads < 1 || kv_heads < 1 || dim < 16 || dim % 16 != 0 || block_size < 1 ||
+      shape < 0 || shape >= LARGE_SHAPE_COUNT || LARGE_SHAPES[shape].tm * LARGE_SHAPES[shape].tn > 12 || table == nullptr ||
+      (write && (slots == nullptr || k_cache == nullptr || v_cache == nullptr)) || !aligned(x) || !aligned(w_packed) ||
+      !aligned(bias) || !aligned(y) || !aligned(table) || !aligned(k_cache))
+    return DISTIE_BAD_ARGUMENT;
+  const int N = (heads + 2 * kv_heads) * dim;
+  const RotaryOut rotary = {static_cast<const float2*>(table), slots, static_cast<bf16_t*>(k_cache),
+                            static_cast<bf16_t*>(v_cache), heads, kv_heads, dim, block_size, write};
+  return launch_large<PK_ROTARY, bf16_t>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w_packed), bias,
+                                         static_cast<bf16_t*>(y), M, N, K, N / 16, shape, 1, rotary, stream);
+}

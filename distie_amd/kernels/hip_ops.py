@@ -272,6 +272,36 @@ class HipOps(Ops):
     # 2,245 us instead of 2,302).
     TILES_HOST_ROWS = 2048
     # (A weight that no role was named for stays with the passes: who reads its product is not known.)
+    # From LARGE_MIN_ROWS rows on, products on a packed copy run in the tiles of `large_tiles.hip` where those are the faster ones
+    # (`_large_take`). Which is told by the rate, in TFLOP/s, that the count behind their plan comes to; measured on 25 weights of
+    # 0.9 to 136 million elements and 27 row counts, in a captured graph, with the kernels that read the result (us, these tiles /
+    # what there was, `packed_tiles` or the library's first choice with the kernels behind it):
+    #  * gated: from LARGE_GATED_RATE on ([65, 1536] x [17920, 1536] 17 / 22, [301, 1536] 25 / 36, [2048, 1536] 104 / 129; [2048,
+    #    3584] x [37888, 3584] 447 / 570, [65, 3584] 52 / 72; [128, 1024] x [8192, 1024] 9.5 / 9.2, [160, 1024] 10 / 12);
+    #  * with rotation and cache write in the epilogue: beyond one round of the 64 x 64 tiles of `packed_tiles` ([512, 1536] x
+    #    [2048, 1536] 17 / 12, [576, 1536] 17 / 18, [1152, 1536] 19 / 26, [2048, 1536] 26 / 24), for large weights, whose 64 x 128
+    #    tiles are two thirds as long as these, LARGE_ROTARY_ROWS ([352, 3584] x [4608, 3584] 34 / 30, [450, 3584] 33 / 36, [2048, 3584] 78
+    #    / 73, [1920, 3584] 66 / 69);
+    #  * plain, for readers that add the slices of K: K at least twice as long as the weight has rows from LARGE_LONG_RATE on
+    #    ([512, 8960] x [1536, 8960] 34 / 31, [576, 8960] 30 / 33, [2048, 8960] 66 / 83; [193, 18944] x [3584, 18944] 48 / 58, [2048,
+    #    18944] 271 / 300), and past TILES_LONG_ROWS, where `packed_tiles` ends, LARGE_LONG_RATE_BEYOND ([1024, 4096] x [1024,
+    #    4096] 22 / 21, [1280, 4096] 23 / 27); others from LARGE_SHORT_RATE on ([256, 3584] x [3584, 3584] 19.5 / 19, [301, 3584] 23 /
+    #    26; [1408, 1536] x [1536, 1536] 24 / 23, [1536, 1536] 21 / 23), weights of 2,048 rows and up to
+    #    ROW_GROUPS_MAX_ELEMENTS from LARGE_SHORT_RATE_SMALL on ([1536, 2048] x [2048, 2048] 30 / 28, [1667, 2048] 27 / 30);
+    #  * other plain ones from LARGE_PLAIN_RATE on ([1024, 2048] x [2048, 2048] 17 / 15, [1152, 2048] 17 / 20), weights of four times as
+    #    many rows as K from LARGE_WIDE_RATE on ([400, 1024] x [4352, 1024] 11 / 10, [450, 1024] 10 / 12), up to LARGE_DENSE_WORK
+    #    products, from where the library is the faster one ([900, 2048] x [8448, 2048] 36 / 40, [1024, 2048] 42 / 39, [2048, 2048] 76 / 66).
+    LARGE_MIN_ROWS = 65
+    LARGE_GATED_RATE = 240.0
+    LARGE_ROTARY_RATE = 150.0
+    LARGE_ROTARY_ROWS = 416
+    LARGE_LONG_RATE = 515.0
+    LARGE_LONG_RATE_BEYOND = 380.0
+    LARGE_SHORT_RATE = 316.0
+    LARGE_SHORT_RATE_SMALL = 440.0
+    LARGE_PLAIN_RATE = 480.0
+    LARGE_WIDE_RATE = 350.0
+    LARGE_DENSE_WORK = 1.65e10
     # What a cut product costs beyond its slices where the reader of the result cannot add them itself (the readers of a
     # layer's output projections can)
     ADDS_SLICES = ("attn_out", "down")
@@ -329,6 +359,7 @@ class HipOps(Ops):
         self.library_timed_rows = self.library_timed_portion = 0
         self._packed_left_out = 0
         self._tile_plans: Dict[tuple, Optional[tuple]] = {}
+        self._large_plans: Dict[tuple, Optional[tuple]] = {}
         self._ops = ctypes.CDLL(str(build.ensure("ops")))
         self._declare()
         self._attn: Dict[int, ctypes.CDLL] = {}
@@ -389,6 +420,9 @@ class HipOps(Ops):
         o.distie_packed_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F] + 3 * [ctypes.POINTER(_I)]
         o.distie_packed_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
         o.distie_packed_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
+        o.distie_large_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F] + 2 * [ctypes.POINTER(_I)] + [ctypes.POINTER(_F)]
+        o.distie_large_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
+        o.distie_large_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_packed_each_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _P, _P]
         o.distie_decode_norm_fits.argtypes = [_I]
         o.distie_decode_product_residual.argtypes = [_P, _P, _P, _P, _I, _I, _I, _P]
@@ -737,9 +771,10 @@ class HipOps(Ops):
             _check(self._ops.distie_rows_f32(x.data_ptr(), gate_up_weight.data_ptr(), None, out.data_ptr(), M, N, K, gated, 1,
                                              *clamp, self._stream()), "rows_f32")
             return out
-        plan = None
+        plan = large = None
         if packed is not None and x.dtype == torch.bfloat16:
-            plan = self._tiles(x.shape[0], *gate_up_weight.shape, "gated")
+            large = self._large(x.shape[0], *gate_up_weight.shape, "gated", (x,))
+            plan = large or self._tiles(x.shape[0], *gate_up_weight.shape, "gated")
         if packed is None or x.dtype != torch.bfloat16 or \
                 (plan is None and x.shape[0] > self._packed_rows(x.shape[0], *gate_up_weight.shape)):
             return apart(self.linear(x, gate_up_weight))
@@ -749,7 +784,7 @@ class HipOps(Ops):
         if packed.numel() != self._packed_elements(N, K, True):
             raise KernelError("linear_silu_mul: the packed copy does not belong to this weight")
         if plan is not None:
-            return self._run_tiles(plan, x, packed, None, x.dtype, M, N, K, gated, clamp=clamp)
+            return self._run_tiles(plan, x, packed, None, x.dtype, M, N, K, gated, clamp=clamp, large=large is not None)
         out = torch.empty((M, N // 2), dtype=x.dtype, device=self.device)
         if M <= self.ONE_WAVE_MAX_ROWS:
             _check(self._ops.distie_gemm_packed_bf16(x.data_ptr(), packed.data_ptr(), None, out.data_ptr(), _code(out),
@@ -804,11 +839,12 @@ class HipOps(Ops):
                 table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads, num_kv_heads,
                 head_dim, meta.block_size, 1 if write else 0, self._stream()), "rows_f32_rotary")
             return out
-        plan = None
+        plan = large = None
         fused = held is not None and held[1] == (num_heads, num_kv_heads, head_dim) and x.dtype == torch.bfloat16 and \
             inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and k_cache.dtype == torch.bfloat16
         if fused:
-            plan = self._tiles(x.shape[0], *weight.shape, "rotary")
+            large = self._large(x.shape[0], *weight.shape, "rotary", (x, bias, k_cache))
+            plan = large or self._tiles(x.shape[0], *weight.shape, "rotary")
             fused = plan is not None or x.shape[0] <= self._packed_rows(x.shape[0], *weight.shape)
         if not fused:
             return self.rope_kv_write(self.linear(x, weight, bias), meta, group, k_cache, v_cache, inv_freq,
@@ -845,10 +881,12 @@ class HipOps(Ops):
         table = self._rope_table(meta, inv_freq)
         out = torch.empty((M, N), dtype=torch.bfloat16, device=self.device)
         if plan is not None:
-            _check(self._ops.distie_packed_tiles_rotary_bf16(
+            kernel, name = (self._ops.distie_large_tiles_rotary_bf16, "large_tiles_rotary_bf16") if large is not None else \
+                (self._ops.distie_packed_tiles_rotary_bf16, "packed_tiles_rotary_bf16")
+            _check(kernel(
                 x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
                 table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads,
-                num_kv_heads, head_dim, meta.block_size, 1 if write else 0, plan[0], self._stream()), "packed_tiles_rotary_bf16")
+                num_kv_heads, head_dim, meta.block_size, 1 if write else 0, plan[0], self._stream()), name)
             return out
         _check(self._ops.distie_gemm_packed_rotary_bf16(
             x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
@@ -927,15 +965,58 @@ class HipOps(Ops):
                 work <= self.TILES_PORTION_WORK
         return long or M <= self.TILES_CUT_MAX_ROWS
 
-    def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, clamp=(0.0, 1.0, 0.0)):
+    LARGE_KINDS = {"plain": 0, "gated": 1, "rotary": 2}
+
+    def _large(self, M: int, N: int, K: int, kind: str, tensors, cut_us: Optional[float] = None):
+        """(shape, slices) of the kernels for many rows for a product as in `_tiles`, None if another kernel is the better one or
+        one of the caller's `tensors`, which they take 16 bytes at a time, begins at no multiple of that."""
+        if M < self.LARGE_MIN_ROWS:
+            return None
+        key = (M, N, K, kind, cut_us)
+        try:
+            plan = self._large_plans[key]
+        except KeyError:
+            plan = None
+            shape, slices, us = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0)
+            if self._ops.distie_large_tiles_plan(M, N, K, self.LARGE_KINDS[kind], cut_us is not None, cut_us or 0.0,
+                                                 ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)) and \
+                    self._large_take(M, N, K, kind, cut_us, us.value):
+                plan = (shape.value, slices.value)
+            if len(self._large_plans) >= self.TILE_PLANS:
+                self._large_plans.clear()
+            self._large_plans[key] = plan
+        if plan is not None:
+            for t in tensors:
+                if t is not None and t.data_ptr() % 16:
+                    return None
+        return plan
+
+    def _large_take(self, M, N, K, kind, cut_us, us) -> bool:
+        """Whether a product that comes to `us` there, with the reader that adds its slices, is to run so: see the constants."""
+        rate, elements = 2e-6 * M * N * K / us, N * K
+        if kind == "gated":
+            return rate >= self.LARGE_GATED_RATE
+        if kind == "rotary":
+            return -(-M // 64) * -(-N // 64) > self._compute_units and rate >= self.LARGE_ROTARY_RATE and \
+                (M >= self.LARGE_ROTARY_ROWS or elements <= self.TILES_LARGE_ROTARY)
+        if cut_us != 0.0:
+            return rate >= (self.LARGE_WIDE_RATE if N >= 4 * K else self.LARGE_PLAIN_RATE) and M * elements <= self.LARGE_DENSE_WORK
+        if K >= 2 * N:
+            return rate >= (self.LARGE_LONG_RATE if M <= self.TILES_LONG_ROWS else self.LARGE_LONG_RATE_BEYOND)
+        return rate >= (self.LARGE_SHORT_RATE if elements > self.ROW_GROUPS_MAX_ELEMENTS or N < self.TILES_FEW_WEIGHT_ROWS else
+                        self.LARGE_SHORT_RATE_SMALL)
+
+    def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, clamp=(0.0, 1.0, 0.0), large=False):
         """The tiled product; float32 slices if the plan cuts K."""
         shape, slices = plan
         columns = N // 2 if gated else N
         out = torch.empty((M, columns), dtype=out_dtype, device=self.device) if slices == 1 else \
             torch.empty((slices, M, columns), dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_packed_tiles_bf16(
+        kernel, name = (self._ops.distie_large_tiles_bf16, "large_tiles_bf16") if large else \
+            (self._ops.distie_packed_tiles_bf16, "packed_tiles_bf16")
+        _check(kernel(
             x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), _code(out),
-            M, N, K, gated, shape, slices, *clamp, self._stream()), "packed_tiles_bf16")
+            M, N, K, gated, shape, slices, *clamp, self._stream()), name)
         return out if slices == 1 else PartialSums(out, out_dtype)
 
     def _library(self):
@@ -1061,14 +1142,15 @@ class HipOps(Ops):
         packed = packed if both_bf16 else None
         if lazy and packed is not None and self._fused(M) and K % 8 == 0 and out_dtype == torch.bfloat16:
             return PendingProduct(x, weight, bias)
-        plan = None
+        plan = large = None
         if packed is not None and weight._distie_role is not None:
             adds = partial_ok and weight._distie_role in self.ADDS_SLICES
-            plan = self._tiles(M, N, K, "plain", 0.0 if adds else self.SUM_SLICES_US)
+            large = self._large(M, N, K, "plain", (x, bias), 0.0 if adds else self.SUM_SLICES_US)
+            plan = large or self._tiles(M, N, K, "plain", 0.0 if adds else self.SUM_SLICES_US)
         if plan is not None:
             if packed.numel() != self._packed_elements(N, K, False):
                 raise KernelError("linear: the packed copy does not belong to this weight")
-            out = self._run_tiles(plan, x, packed, bias, out_dtype, M, N, K)
+            out = self._run_tiles(plan, x, packed, bias, out_dtype, M, N, K, large=large is not None)
             return out if partial_ok else self.dense(out)
         if packed is not None and self.ONE_WAVE_MAX_ROWS < M <= self._packed_rows(M, N, K) and K % 8 == 0 and \
                 N * K > self.ROW_GROUPS_MAX_ELEMENTS:

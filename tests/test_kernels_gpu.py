@@ -399,6 +399,102 @@ def test_packed_tiles_with_rotation(ops, shape, rows, heads, kv_heads, dim, K, P
         assert torch.equal(v1.permute(0, 3, 1, 2)[keep], v2.permute(0, 3, 1, 2)[keep])
 
 
+LARGE_SHAPES = [(0, 256), (1, 256), (2, 192), (3, 192), (4, 128), (5, 192), (6, 128), (7, 128)]
+
+
+@pytest.mark.parametrize("shape,rows", LARGE_SHAPES)
+@pytest.mark.parametrize("N,K", [(16, 256), (40, 320), (1040, 1088), (528, 4096)])
+def test_large_tiles(ops, shape, rows, N, K):
+    """Every tile of the products of many rows: rows and columns that do not fill a tile, as few stages as there can be, odd and
+    even, K whole and cut; plain with and without a bias in both types, and gated with three activations. Sums are float32,
+    rounded once: the bounds are those of `packed_tiles`."""
+    w, b = rand(N, K, dtype=torch.bfloat16, seed=2, scale=K ** -0.5), rand(N, seed=3)
+    gate_up = rand(N, K, dtype=torch.bfloat16, seed=4, scale=2.0 * K ** -0.5)
+    ops.prepare_linear(w, role="down")
+    ops.prepare_linear(gate_up, gated=True, role="gate_up")
+    for M in (1, rows - 1, rows, rows + 1, 2 * rows + 17):
+        x = rand(M, K, dtype=torch.bfloat16, seed=M)
+        want = x.double() @ w.double().T + b.double()
+        stages = K // 64
+        for slices in (1, 2, 3, 8):
+            if -(-stages // -(-stages // slices)) != slices:
+                continue
+            got = ops._run_tiles((shape, slices), x, w._distie_packed, b, torch.float32, M, N, K, large=True)
+            close(ops.dense(got), want, torch.float32, scale=5 * want.abs().max().item())
+            assert slices == 1 or got.slices == slices
+        for bias in (b, None):
+            got = ops._run_tiles((shape, 1), x, w._distie_packed, bias, torch.bfloat16, M, N, K, large=True)
+            close(got, want if bias is not None else want - b.double(), torch.bfloat16, scale=want.abs().max().item())
+        if N % 16:
+            continue
+        product = x.double() @ gate_up.double().T
+        gate, up = product[:, :N // 2], product[:, N // 2:]
+        for gated, clamp, want in (
+                (1, (0.0, 1.0, 0.0), gate / (1 + torch.exp(-gate)) * up),
+                (1 | (2 << 8), (0.0, 1.0, 0.0), None), (1 | (4 << 8), (0.0, 1.0, 0.0), gate.clamp(min=0) * up),
+                (1 | (ops.CLAMPED << 8), (0.7, 1.702, 1.0),
+                 gate.clamp(max=0.7) / (1 + torch.exp(-1.702 * gate.clamp(max=0.7))) * (up.clamp(-0.7, 0.7) + 1))):
+            got = ops._run_tiles((shape, 1), x, gate_up._distie_gated, None, torch.bfloat16, M, N, K, gated=gated, clamp=clamp,
+                                 large=True)
+            if want is None:                  # (2 is silu by its other name)
+                want = gate / (1 + torch.exp(-gate)) * up
+            close(got, want, torch.bfloat16, scale=want.abs().max().item())
+
+
+def test_large_tiles_gate_at_its_limits(ops):
+    """Gates far out on either side: the activation is the gate or zero there, and values that are not finite stay so."""
+    K, I, M = 256, 64, 130
+    w = torch.zeros(2 * I, K, dtype=torch.bfloat16, device="cuda")
+    w[:, 0] = 1
+    ops.prepare_linear(w, gated=True, role="gate_up")
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda")
+    values = torch.tensor([0.0, 1e-30, 80.0, -80.0, 100.0, -100.0, 1e4, -1e4, float("inf"), float("-inf"), float("nan")])
+    x[:len(values), 0] = values.to(torch.bfloat16).cuda()
+    got = ops._run_tiles((7, 1), x, w._distie_gated, None, torch.bfloat16, M, 2 * I, K, gated=1, large=True).double()
+    v = x[:, 0].double()
+    want = v / (1 + torch.exp(-v)) * v
+    want[9] = float("nan")                        # -inf / inf
+    torch.testing.assert_close(got, want[:, None].expand(M, I), rtol=2 ** -8, atol=1e-30, equal_nan=True)
+
+
+@pytest.mark.parametrize("shape,rows", LARGE_SHAPES[1:])
+@pytest.mark.parametrize("heads,kv_heads,dim,K,P", [(3, 1, 16, 256, 4), (2, 2, 80, 320, 16), (12, 2, 128, 1088, 16)])
+def test_large_tiles_with_rotation(ops, shape, rows, heads, kv_heads, dim, K, P):
+    """As test_packed_tiles_with_rotation, every place of the result and of both caches."""
+    N = (heads + 2 * kv_heads) * dim
+    w, b = rand(N, K, dtype=torch.bfloat16, seed=6, scale=K ** -0.5), rand(N, seed=7)
+    ops.prepare_linear(w, rotary=(heads, kv_heads, dim))
+    packed = w._distie_rotary[0]
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, dim, 2, dtype=torch.float32) / dim))).cuda()
+    for M, bias, write in ((1, b, 1), (rows - 1, b, 1), (rows, None, 1), (rows + 1, b, 0), (2 * rows + 17, b, 1)):
+        x = rand(M, K, dtype=torch.bfloat16, seed=M)
+        pages = 2 * M + 2
+        g = torch.Generator().manual_seed(M)
+        slots = torch.randperm(pages * P, generator=g)[:M].tolist()
+        positions = torch.randint(0, 5000, (M,), generator=g).tolist()
+        meta = make_meta(positions, list(range(M)), list(range(M + 1)), [p + 1 for p in positions], [[0] * 8] * M, slots, P)
+        k1 = rand(pages, kv_heads, P, dim, dtype=torch.bfloat16, seed=8)
+        v1 = rand(pages, kv_heads, dim, P, dtype=torch.bfloat16, seed=9)
+        k2, v2 = k1.clone(), v1.clone()
+        dense = (x.double() @ w.double().T + (0.0 if bias is None else b.double())).float()
+        want = TorchOps("cuda").rope_kv_write(dense, meta, 0, k2, v2, inv_freq, heads, kv_heads, dim, bool(write))
+        got = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert ops._ops.distie_large_tiles_rotary_bf16(
+            x.data_ptr(), packed.data_ptr(), None if bias is None else bias.data_ptr(), got.data_ptr(),
+            ops._rope_table(meta, inv_freq).data_ptr(), meta.groups[0].slots.data_ptr(), k1.data_ptr(), v1.data_ptr(), M, K,
+            heads, kv_heads, dim, P, write, shape, ops._stream()) == 0
+        scale = want.abs().max().item()
+        close(got, want, torch.bfloat16, scale=scale)
+        close(k1, k2, torch.bfloat16, scale=scale)
+        close(v1, v2, torch.bfloat16, scale=scale)
+        untouched = torch.ones(pages * P, dtype=torch.bool)
+        if write:
+            untouched[slots] = False
+        keep = untouched.view(pages, P).cuda()
+        assert torch.equal(k1.permute(0, 2, 1, 3)[keep], k2.permute(0, 2, 1, 3)[keep])
+        assert torch.equal(v1.permute(0, 3, 1, 2)[keep], v2.permute(0, 3, 1, 2)[keep])
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 17, 45, 64, 70, 96, 129, 224])
 @pytest.mark.parametrize("heads,kv_heads,dim,K,P", [(3, 1, 32, 2048, 4), (12, 2, 128, 1536, 16), (4, 4, 16, 72, 16),
                                                     (5, 5, 48, 240, 8), (2, 1, 80, 520, 16), (7, 1, 256, 136, 32),

@@ -4,6 +4,7 @@ boundary where the kernels of both sides were measured."""
 import ctypes
 
 import pytest
+import torch
 
 from distie_amd.csrc import build
 from distie_amd.kernels.hip_ops import HipOps
@@ -14,7 +15,7 @@ def rules():
     ops = HipOps.__new__(HipOps)                   # the rules alone: nothing of this touches a device
     ops._ops = ctypes.CDLL(str(build.ensure("ops")))
     ops._declare()
-    ops._tile_plans, ops._compute_units, ops.library_timed_portion = {}, 256, 0
+    ops._tile_plans, ops._large_plans, ops._compute_units, ops.library_timed_portion = {}, {}, 256, 0
     return ops
 
 
@@ -77,6 +78,50 @@ def test_plans_are_kept_apart_by_what_the_rule_reads(rules):
     rules.library_timed_portion = 2040               # classes of 32 rows
     assert [rules._tiles(rows, 3584, 18944, "plain", 0.0) is None for rows in (1400, 2016, 2017, 2048)] == [False, False, True, True]
     rules.library_timed_portion = 0
+
+
+@pytest.mark.parametrize("kind,rows,weight,takes", [
+    # gated: nearly always; small weights from where they fill a few compute units
+    ("gated", 64, (37888, 3584), False), ("gated", 80, (37888, 3584), True), ("gated", 80, (17920, 1536), True),
+    ("gated", 65, (8192, 1024), False), ("gated", 193, (8192, 1024), True), ("gated", 2048, (17920, 1536), True),
+    ("gated", 301, (17920, 1536), True), ("gated", 97, (4096, 512), False), ("gated", 2048, (17912, 1536), False),
+    ("gated", 2048, (17920, 1544), False),
+    # rotation: beyond one round of the smaller tiles
+    ("rotary", 512, (2048, 1536), False), ("rotary", 576, (2048, 1536), True), ("rotary", 301, (3072, 2048), False),
+    ("rotary", 352, (3072, 2048), True), ("rotary", 640, (1536, 1024), False), ("rotary", 704, (1536, 1024), True),
+    ("rotary", 256, (4608, 3584), False), ("rotary", 2048, (4608, 3584), True),
+    # plain: where the count comes to a rate that neither the smaller tiles nor the library reach
+    ("down", 301, (1536, 8960), False), ("down", 2048, (1536, 8960), True), ("down", 128, (3584, 18944), False),
+    ("down", 301, (3584, 18944), True), ("down", 2048, (1024, 2048), False), ("attn_out", 1024, (1536, 1536), False),
+    ("attn_out", 2048, (1536, 1536), True), ("qkv", 1024, (1024, 1024), False), ("qkv", 640, (8448, 2048), True),
+    ("qkv", 2048, (8448, 2048), False)])
+def test_products_in_large_tiles(rules, kind, rows, weight, takes):
+    rules.captured, rules.library_timed_rows = False, 0
+    cut_us = None if kind in ("rotary", "gated") else 0.0 if kind in rules.ADDS_SLICES else rules.SUM_SLICES_US
+    plan = rules._large(rows, *weight, kind if cut_us is None else "plain", (), cut_us)
+    assert (plan is not None) == takes
+
+
+@pytest.mark.parametrize("N,K", [(16, 256), (40, 320), (1536, 8960), (152064, 3584), (4608, 18944)])
+def test_large_tiles_plans_are_launches_that_the_kernel_takes(rules, N, K):
+    for rows in (1, 65, 128, 129, 777, 2048, 16384):
+        for mode in (0, 1, 2):
+            for cut_us in (None, 0.0, 4.5):
+                shape, slices, us = ctypes.c_int(-1), ctypes.c_int(-1), ctypes.c_float(-1)
+                taken = rules._ops.distie_large_tiles_plan(rows, N, K, mode, cut_us is not None, cut_us or 0.0, ctypes.byref(shape),
+                                                           ctypes.byref(slices), ctypes.byref(us))
+                assert taken == (N % (16 if mode else 8) == 0)
+                if taken:
+                    stages = K // 64
+                    assert (1 if mode == 2 else 0) <= shape.value <= 7 and us.value > 0
+                    assert -(-stages // -(-stages // slices.value)) == slices.value and (slices.value == 1 or (mode == 0 and cut_us is not None))
+
+
+def test_large_tiles_leave_what_begins_off_16_bytes(rules):
+    rules.captured, rules.library_timed_rows = False, 0
+    data = torch.empty(64, dtype=torch.bfloat16)
+    assert rules._large(2048, 17920, 1536, "gated", (data, None)) is not None
+    assert rules._large(2048, 17920, 1536, "gated", (data[1:], None)) is None
 
 
 @pytest.mark.parametrize("rows,weight,takes", [
