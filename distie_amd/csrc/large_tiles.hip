@@ -1,17 +1,18 @@
 // Products of many rows (portions of prompts, prompts of a few hundred tokens) on packed weight copies: y[M, N] = x[M, K]
 // W[N, K]^T for bfloat16 x and the copies of packed.h, with the activation, or rotation and cache write, in the epilogue.
 //
-// A workgroup of 2 x 2 waves owns a tile of 64 TM rows of x and 64 TN rows of W and one slice of K; a wave owns 32 TM x 32 TN of
-// it as TM x TN products of 32 x 32 x 16, whose sums stay in the accumulation registers. x and W both go straight from memory
-// into LDS: x in stages of 64 k, three of them (whole lines of 128 bytes: halves cost the L2 twice the requests), W, whose copy
-// lies in lane order, in halves of a stage, four of them. The waits count loads, so that one to two stages are under way all the
-// time; reads of LDS and loads stand between the matrix instructions of the 16 k before.
+// A workgroup of four or two waves owns a tile of rows of x and rows of W and one slice of K; a wave owns 32 TM x 32 TN of it as
+// TM x TN products of 32 x 32 x 16, whose sums stay in the accumulation registers. x and W both go straight from memory into LDS:
+// x in stages of 64 k (whole lines of 128 bytes: halves cost the L2 twice the requests), W, whose copy lies in lane order, in halves
+// of a stage. The waits count loads, so that D stages (2, and up to 6 where tiles are small) are under way all the time; reads of
+// LDS and loads stand between the matrix instructions of the 16 k before.
 //
 // What bounds it. [4096, 4096] x [4096, 4096] takes 110 us (1,244 TFLOP/s; the library 98): the matrix cores are 90 % busy and the
 // chip's power holds the clock at 1.45 GHz, whatever the loop does (eight waves of 128 x 64, which read half as much again from
 // LDS, take 2,570 to 2,940 cycles a stage instead of 2,270 and the same 124 us at 1.58 to 1.81 GHz). That is why a wave owns as
 // much as it can hold. Smaller tiles run into the L2, which gives the chip's LDS 15 to 17 TB/s: 128 x 128 need 32 KB for 512
-// cycles of products (fragments of a whole stage read ahead changed nothing). With few rows it is the weight from memory.
+// cycles of products (fragments of a whole stage read ahead changed nothing). With few rows it is the weight from memory: 64 rows
+// of the 1.5B shape's gate+up 15.1 us (3.6 TB/s; 20.2 in packed_tiles), of the 7B shape's 52 (5.2 TB/s; 66 in passes).
 // 1.5B shape, 2,048 rows, isolated and with the kernel that the library needs behind its own: gate+up with its activation 104 us
 // (129), down in four slices 54 (80; the norm reads 12 us more). 7B shape, 2,025 rows: 460 (567) and 220 (359; packed_tiles
 // 261). 301 rows: gate+up of the 1.5B shape 25 us, 36 in packed_tiles.
@@ -27,7 +28,6 @@ typedef __attribute__((__vector_size__(4 * sizeof(int)))) int intx4;
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int LT_K = 64;              // k of a stage of x; W comes in halves of it
-constexpr int LT_X_STAGES = 3, LT_W_PARTS = 4;
 
 // A buffer of `bytes` from `base` on (both the same in all lanes): reads beyond it give zeros.
 __device__ __forceinline__ intx4 buffer_of(const void* base, uint32_t bytes) {
@@ -66,20 +66,23 @@ struct LargePlace {
   int stages;                   // of a slice
 };
 
-// MODE: PK_PLAIN, PK_GATED, PK_ROTARY. K a multiple of LT_K; columns of y a multiple of 16 bytes.
-template <int TM, int TN, int MODE, typename Y>
-__global__ __launch_bounds__(256, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
+// A workgroup: WM x WAVES / WM waves of TM x TN products of 32 x 32; D stages ahead. MODE: PK_PLAIN, PK_GATED, PK_ROTARY.
+// K a multiple of LT_K; columns of y a multiple of 16 bytes.
+template <int WAVES, int WM, int TM, int TN, int D, int MODE, typename Y>
+__global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias, Y* __restrict__ y, int M, int N,
     int K, LargePlace at, RotaryOut rotary) {
-  constexpr int BM = 64 * TM, BN = 64 * TN;            // of the workgroup: 2 x 2 waves
+  constexpr int BM = 32 * WM * TM, BN = 32 * (WAVES / WM) * TN;
+  constexpr int X_LOADS = BM / (8 * WAVES), W_LOADS = BN / (16 * WAVES);     // of a wave: of a stage of x, of half a stage of W
+  constexpr int XA = (X_LOADS + 1) / 2, XB = X_LOADS - XA;
   constexpr int X_BYTES = BM * LT_K * 2, W_BYTES = BN * LT_K;
-  constexpr int W_AT = LT_X_STAGES * X_BYTES;
-  constexpr int LDS_BYTES = W_AT + LT_W_PARTS * W_BYTES;
+  constexpr int W_AT = (D + 1) * X_BYTES;
+  constexpr int LDS_BYTES = W_AT + 2 * D * W_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of a compute unit");
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r = lane % 32, h = lane / 32;
-  const int wm = wave % 2, wn = wave / 2;
+  const int wm = wave % WM, wn = wave / WM;
   const int tiles = at.m_tiles * at.n_tiles;
   const int place = static_cast<int>(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
   if (place >= tiles * at.slices) return;
@@ -95,22 +98,22 @@ __global__ __launch_bounds__(256, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
       buffer_of(w + static_cast<int64_t>(b0) * k_tiles * PK_TILE, static_cast<uint32_t>(blocks) * k_tiles * 1024u);
   // A row of x's stage is eight pieces of 16 bytes; eight neighbouring lanes bring a row, piece p to place p ^ (row / 2 % 8), so
   // that the rows a product reads at once spread over all banks. Rows and blocks beyond the last are read from it and dropped.
-  int x_lane[2 * TM], w_lane[TN];
+  int x_lane[X_LOADS], w_lane[W_LOADS];
 #pragma unroll
-  for (int p = 0; p < 2 * TM; ++p) {
-    const int row = 8 * (wave * 2 * TM + p) + lane / 8;
+  for (int p = 0; p < X_LOADS; ++p) {
+    const int row = 8 * (wave * X_LOADS + p) + lane / 8;
     x_lane[p] = min(row, rows - 1) * K * 2 + 16 * ((lane % 8) ^ ((row >> 1) & 7));
   }
 #pragma unroll
-  for (int p = 0; p < TN; ++p) w_lane[p] = min(wave * TN + p, blocks - 1) * k_tiles * 1024 + lane * 16;
+  for (int p = 0; p < W_LOADS; ++p) w_lane[p] = min(wave * W_LOADS + p, blocks - 1) * k_tiles * 1024 + lane * 16;
   const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds)));
   auto bring_x = [&](int stage, int slot, int p) {
     buffer_to_lds(x_buffer, x_lane[p], (s_begin + min(stage, stages - 1)) * (LT_K * 2),
-                  base + slot * X_BYTES + (wave * 2 * TM + p) * 1024);
+                  base + slot * X_BYTES + (wave * X_LOADS + p) * 1024);
   };
-  auto bring_w = [&](int part, int p) {
+  auto bring_w = [&](int part, int slot, int p) {
     buffer_to_lds(w_buffer, w_lane[p], (2 * s_begin + min(part, 2 * stages - 1)) * 1024,
-                  base + W_AT + part % LT_W_PARTS * W_BYTES + (wave * TN + p) * 1024);
+                  base + W_AT + slot * W_BYTES + (wave * W_LOADS + p) * 1024);
   };
 
   // acc[a][b][4 q + i]: row 8 (q % 2) + 4 h + i of block first_block + 2 b + q / 2, row 32 a + r of the wave's part of x
@@ -162,36 +165,32 @@ __global__ __launch_bounds__(256, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
   };
   // Past the last stage the loads bring it once more, so that their number, which the waits count, stays what it is.
 #pragma unroll
-  for (int p = 0; p < 2 * TM; ++p) bring_x(0, 0, p);
+  for (int p = 0; p < X_LOADS; ++p) bring_x(0, 0, p);
 #pragma unroll
-  for (int p = 0; p < TN; ++p) bring_w(0, p);
+  for (int part = 0; part < 2 * D; ++part) {
 #pragma unroll
-  for (int p = 0; p < TN; ++p) bring_w(1, p);
+    for (int p = 0; p < W_LOADS; ++p) bring_w(part, part, p);
 #pragma unroll
-  for (int p = 0; p < TM; ++p) bring_x(1, 1, p);
-#pragma unroll
-  for (int p = 0; p < TN; ++p) bring_w(2, p);
-#pragma unroll
-  for (int p = TM; p < 2 * TM; ++p) bring_x(1, 1, p);
-#pragma unroll
-  for (int p = 0; p < TN; ++p) bring_w(3, p);
-  arrived<3 * TN + 2 * TM>();
+    for (int p = 0; p < X_LOADS; ++p)
+      if (part > 0 && part < 2 * D - 1 && (part % 2 == 1) == (p < XA)) bring_x((part + 1) / 2, (part + 1) / 2, p);
+  }
+  constexpr int STAGE = 2 * W_LOADS + X_LOADS;
+  arrived<(D - 1) * STAGE + W_LOADS>();
 #pragma unroll
   for (int i = 0; i < TM + TN; ++i) read(0, 0, 0, 0, i);
-  // Iteration s holds x(s) and W's parts 2 s and 2 s + 1. Before the first wait W(2 s + 1) has to be there, and behind it in order
-  // stand x(s + 1) and halves of it, W(2 s + 2), W(2 s + 3) and half of x(s + 2); before the second x(s + 1) and W(2 s + 2). A
-  // wait also says that all waves have read what the loads behind it write over.
-  int slot = 0;
+  // Iteration s holds x(s) and W's parts 2 s and 2 s + 1. The loads in order: x(0), W(0); then, for every stage, W(2 s - 1), the
+  // first half of x(s), W(2 s), the rest of x(s). Before the first wait W(2 s + 1) has to be there, before the second x(s + 1) and
+  // W(2 s + 2); D stages have been asked for. A wait also says that all waves have read what the loads behind it write over.
+  int slot = 0, w_slot = 0;
   for (int s = 0; s < stages; ++s) {
-    const int next = slot == LT_X_STAGES - 1 ? 0 : slot + 1, free = slot == 0 ? LT_X_STAGES - 1 : slot - 1;
-    const int w_slot = 2 * (s % 2);
-    multiply(0, 1, slot, w_slot, TM, [&](int q) { bring_x(s + 2, free, q); });
-    arrived<3 * TM + 2 * TN>();
-    multiply(1, 2, slot, w_slot + 1, TN, [&](int q) { bring_w(2 * s + 4, q); });
-    multiply(0, 3, slot, w_slot + 1, TM, [&](int q) { bring_x(s + 2, free, TM + q); });
-    arrived<2 * TM + 2 * TN>();
-    multiply(1, 0, next, 2 - w_slot, TN, [&](int q) { bring_w(2 * s + 5, q); });
-    slot = next;
+    const int next = slot == D ? 0 : slot + 1, free = slot == 0 ? D : slot - 1, w_next = w_slot == 2 * D - 2 ? 0 : w_slot + 2;
+    multiply(0, 1, slot, w_slot, XA, [&](int q) { bring_x(s + D, free, q); });
+    arrived<(D - 1) * STAGE + XA>();
+    multiply(1, 2, slot, w_slot + 1, W_LOADS, [&](int q) { bring_w(2 * (s + D), w_slot, q); });
+    multiply(0, 3, slot, w_slot + 1, XB, [&](int q) { bring_x(s + D, free, XA + q); });
+    arrived<(D - 1) * STAGE>();
+    multiply(1, 0, next, w_next, W_LOADS, [&](int q) { bring_w(2 * (s + D) + 1, w_slot + 1, q); });
+    slot = next, w_slot = w_next;
   }
   arrived<0>();
 
@@ -304,17 +303,24 @@ __global__ __launch_bounds__(256, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
   }
 }
 
-// The tiles there are, and what a workgroup of one takes: for every stage few_us with hardly any compute unit at work, more_us
-// on top of it with all of them (the L2; and power: the clock falls from 2.4 to 1.45 GHz) and pair_us where two share them, and
-// turn_us to begin and end.
+// The tiles there are, and what a workgroup of one of the first takes: for every stage few_us with hardly any compute unit at
+// work, more_us on top of it with all of them (the L2; and power: the clock falls from 2.4 to 1.45 GHz) and pair_us where two
+// share them, and turn_us to begin and end. The others are for few rows (`plan_few`).
 struct LargeShape {
-  int tm, tn;
+  int waves, wm, tm, tn;
   float few_us, more_us, pair_us, turn_us;
+
+  constexpr int rows() const { return 32 * wm * tm; }
+  constexpr int blocks() const { return 2 * (waves / wm) * tn; }
 };
-constexpr LargeShape LARGE_SHAPES[] = {{4, 4, 0.893f, 0.515f, 0.f, 6.7f},  {4, 3, 0.684f, 0.451f, 0.f, 5.3f},
-                                       {3, 4, 0.692f, 0.446f, 0.f, 5.7f},  {3, 3, 0.558f, 0.371f, 0.f, 4.3f},
-                                       {2, 4, 0.528f, 0.373f, 0.f, 3.4f},  {3, 2, 0.386f, 0.317f, 0.f, 2.7f},
-                                       {2, 3, 0.407f, 0.327f, 0.f, 2.55f}, {2, 2, 0.280f, 0.336f, 0.497f, 1.8f}};
+constexpr LargeShape LARGE_SHAPES[] = {
+    {4, 2, 4, 4, 0.893f, 0.515f, 0.f, 6.7f},  {4, 2, 4, 3, 0.684f, 0.451f, 0.f, 5.3f},
+    {4, 2, 3, 4, 0.692f, 0.446f, 0.f, 5.7f},  {4, 2, 3, 3, 0.558f, 0.371f, 0.f, 4.3f},
+    {4, 2, 2, 4, 0.528f, 0.373f, 0.f, 3.4f},  {4, 2, 3, 2, 0.386f, 0.317f, 0.f, 2.7f},
+    {4, 2, 2, 3, 0.407f, 0.327f, 0.f, 2.55f}, {4, 2, 2, 2, 0.280f, 0.336f, 0.497f, 1.8f},
+    {4, 1, 1, 1}, {4, 1, 1, 2}, {4, 1, 2, 1}, {4, 2, 1, 1}, {2, 1, 1, 1}, {2, 1, 2, 1}};
+constexpr int LARGE_COUNTED = 8, FEW_32_128 = 8, FEW_32_256 = 9, FEW_64_128 = 10, FEW_64_64 = 11, FEW_32_64 = 12, FEW_64_64_CUT = 13;
+constexpr int LARGE_ROTARY_FROM = 1, LARGE_ROTARY_TO = LARGE_COUNTED;          // (the sums and angles of the first do not fit the registers)
 constexpr int LARGE_SHAPE_COUNT = static_cast<int>(sizeof(LARGE_SHAPES) / sizeof(LARGE_SHAPES[0]));
 constexpr float LARGE_GATED_TURN = 0.81f, LARGE_ROTARY_TURN = 3.4f;     // (half the stores; angles and the caches' stores)
 
@@ -331,10 +337,10 @@ LargePlan plan_large(int M, int N, int K, int row_blocks, int mode, bool may_cut
   LargePlan best = {-1, 0, 0.f};
   const int all = K / LT_K;
   const float memory_us = static_cast<float>(row_blocks) * K * 32.f / 3.8e6f, values = static_cast<float>(M) * N;
-  for (int i = 0; i < LARGE_SHAPE_COUNT; ++i) {
+  for (int i = 0; i < LARGE_COUNTED; ++i) {
     const LargeShape& s = LARGE_SHAPES[i];
-    if (mode == PK_ROTARY && s.tm * s.tn > 12) continue;         // (its sums and angles do not fit the registers)
-    const int64_t tiles = static_cast<int64_t>((M + 64 * s.tm - 1) / (64 * s.tm)) * ((row_blocks + 4 * s.tn - 1) / (4 * s.tn));
+    if (mode == PK_ROTARY && (i < LARGE_ROTARY_FROM || i >= LARGE_ROTARY_TO)) continue;
+    const int64_t tiles = static_cast<int64_t>((M + s.rows() - 1) / s.rows()) * ((row_blocks + s.blocks() - 1) / s.blocks());
     const float turn = s.turn_us * (mode == PK_GATED ? LARGE_GATED_TURN : mode == PK_ROTARY ? LARGE_ROTARY_TURN : 1.f);
     for (int cut = 1; cut <= 8; ++cut) {
       if (cut > 1 && (!may_cut || all / cut < 6)) break;
@@ -356,32 +362,68 @@ LargePlan plan_large(int M, int N, int K, int row_blocks, int mode, bool may_cut
   return best;
 }
 
+// Few rows: the weight comes from memory once, and what counts is that every compute unit has one workgroup that asks for it and
+// no unit two, which would take twice as long: the smallest tile whose workgroups are no more than the units; K cut until they
+// are about as many. (us: gate+up of the 1.5B shape, 16 rows: 140 workgroups of 32 x 128 12.8, 280 of 32 x 64 15.5; [16384, 2048],
+// 256 of 32 x 64 14.5, 128 of 32 x 128 18.3; [37888, 3584], 32 rows, 148 of 32 x 256 53, 296 of 32 x 128 64; 64 rows, 198 of 128 x 192
+// 51.6, 592 of 64 x 64 62. [4096, 11008] in four, 64 rows: 256 of 64 x 64 25.) Beyond that many workgroups small tiles do best.
+constexpr int FEW_ROWS = 64;
+
+LargePlan plan_few(int M, int N, int K, int row_blocks, int mode, bool may_cut, float cut_us) {
+  const int all = K / LT_K;
+  const auto workgroups = [&](int shape) { return (row_blocks + LARGE_SHAPES[shape].blocks() - 1) / LARGE_SHAPES[shape].blocks(); };
+  if (mode == PK_PLAIN && may_cut && cut_us == 0.f) {
+    int shape = M <= 32 ? FEW_32_64 : FEW_64_64_CUT;
+    const auto cut_for = [&](int i) { return std::max(1, std::min(256 / workgroups(i), all / 4)); };
+    if (shape == FEW_64_64_CUT && all > 64 * cut_for(shape)) shape = FEW_64_128;       // long walks: wider tiles, twice as many cuts
+    const int stages = (all + cut_for(shape) - 1) / cut_for(shape);
+    return {shape, (all + stages - 1) / stages, 0.f};
+  }
+  if (M <= 32) {
+    for (int shape : {FEW_32_64, FEW_32_128, FEW_32_256})
+      if (workgroups(shape) <= 256) return {shape, 1, 0.f};
+    return {FEW_32_64, 1, 0.f};
+  }
+  for (int shape : {FEW_64_64, FEW_64_128, 6, 4})             // (128 x 192 and 128 x 256)
+    if (workgroups(shape) <= 256) return {shape, 1, 0.f};
+  return {FEW_64_128, 1, 0.f};
+}
+
 template <int MODE, typename Y>
 int launch_large(const bf16_t* x, const bf16_t* w, const float* bias, Y* y, int M, int N, int K, int row_blocks, int shape,
                  int slices, const RotaryOut& rotary, hipStream_t stream) {
-  const int bm = 64 * LARGE_SHAPES[shape].tm, blocks = 4 * LARGE_SHAPES[shape].tn;
+  const int bm = LARGE_SHAPES[shape].rows(), blocks = LARGE_SHAPES[shape].blocks();
   const int all = K / LT_K;
   const LargePlace at = {row_blocks, (M + bm - 1) / bm, (row_blocks + blocks - 1) / blocks, slices, (all + slices - 1) / slices};
   if ((all + at.stages - 1) / at.stages != slices) return DISTIE_BAD_ARGUMENT;
   const int64_t work = static_cast<int64_t>(at.m_tiles) * at.n_tiles * slices;
   if (work > (1 << 30)) return DISTIE_BAD_ARGUMENT;
   const unsigned grid = static_cast<unsigned>((work + 7) / 8 * 8);
-#define LARGE(TM, TN)                                                                                                     \
-  large_tiles_kernel<TM, TN, MODE, Y><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, at, rotary);                      \
-  break
+#define LARGE(I, WAVES, WM, TM, TN, D)                                                                                    \
+  case I:                                                                                                                 \
+    if constexpr (MODE != PK_ROTARY || (I >= LARGE_ROTARY_FROM && I < LARGE_ROTARY_TO)) {                                 \
+      static_assert(LARGE_SHAPES[I].waves == WAVES && LARGE_SHAPES[I].rows() == 32 * WM * TM &&                           \
+                        LARGE_SHAPES[I].blocks() == 2 * (WAVES / WM) * TN, "the table's tile");                           \
+      large_tiles_kernel<WAVES, WM, TM, TN, D, MODE, Y><<<grid, 64 * WAVES, 0, stream>>>(x, w, bias, y, M, N, K, at, rotary); \
+      break;                                                                                                              \
+    }                                                                                                                     \
+    return DISTIE_BAD_ARGUMENT
   switch (shape) {
-    case 0:
-      if constexpr (MODE == PK_ROTARY) return DISTIE_BAD_ARGUMENT;
-      else {
-        LARGE(4, 4);
-      }
-    case 1: LARGE(4, 3);
-    case 2: LARGE(3, 4);
-    case 3: LARGE(3, 3);
-    case 4: LARGE(2, 4);
-    case 5: LARGE(3, 2);
-    case 6: LARGE(2, 3);
-    default: LARGE(2, 2);
+    LARGE(0, 4, 2, 4, 4, 2);
+    LARGE(1, 4, 2, 4, 3, 2);
+    LARGE(2, 4, 2, 3, 4, 2);
+    LARGE(3, 4, 2, 3, 3, 2);
+    LARGE(4, 4, 2, 2, 4, 2);
+    LARGE(5, 4, 2, 3, 2, 2);
+    LARGE(6, 4, 2, 2, 3, 2);
+    LARGE(7, 4, 2, 2, 2, 2);
+    LARGE(8, 4, 1, 1, 1, 3);
+    LARGE(9, 4, 1, 1, 2, 3);
+    LARGE(10, 4, 1, 2, 1, 3);
+    LARGE(11, 4, 2, 1, 1, 3);
+    LARGE(12, 2, 1, 1, 1, 6);
+    LARGE(13, 2, 1, 2, 1, 3);
+    default: return DISTIE_BAD_ARGUMENT;
   }
 #undef LARGE
   return launch_status();
@@ -392,13 +434,15 @@ bool aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 }  // namespace
 
 // How the kernels of this file cut a product, 0 if they do not take it, as distie_packed_tiles_plan. mode: 0 plain, 1 gated, 2
-// with rotation and cache write; *us: what the count comes to.
+// with rotation and cache write; *us: what the count comes to (few rows: 0, not counted).
 extern "C" int distie_large_tiles_plan(int M, int N, int K, int mode, int may_cut, float cut_us, int* shape, int* slices,
                                        float* us) {
   if (M < 1 || N < 16 || K < 4 * LT_K || K % LT_K != 0 || mode < 0 || mode > 2 || N % (mode == PK_GATED ? 16 : 8) != 0 ||
       (mode == PK_ROTARY && N % 16 != 0) || K > (1 << 20))
     return 0;
-  const LargePlan plan = plan_large(M, N, K, (N + 15) / 16, mode, may_cut != 0 && mode == PK_PLAIN, cut_us);
+  const bool cut = may_cut != 0 && mode == PK_PLAIN;
+  const LargePlan plan = M <= FEW_ROWS && mode != PK_ROTARY ? plan_few(M, N, K, (N + 15) / 16, mode, cut, cut_us)
+                                                            : plan_large(M, N, K, (N + 15) / 16, mode, cut, cut_us);
   *shape = plan.shape, *slices = plan.slices, *us = plan.us;
   return 1;
 }
@@ -433,7 +477,7 @@ extern "C" int distie_large_tiles_rotary_bf16(const void* x, const void* w_packe
                                               int kv_heads, int dim, int block_size, int write, int shape, hipStream_t stream) {
   if (M <= 0) return 0;
   if (K < 4 * LT_K || K % LT_K != 0 || K > (1 << 20) || heads < 1 || kv_heads < 1 || dim < 16 || dim % 16 != 0 || block_size < 1 ||
-      shape < 0 || shape >= LARGE_SHAPE_COUNT || LARGE_SHAPES[shape].tm * LARGE_SHAPES[shape].tn > 12 || table == nullptr ||
+      shape < LARGE_ROTARY_FROM || shape >= LARGE_ROTARY_TO || table == nullptr ||
       (write && (slots == nullptr || k_cache == nullptr || v_cache == nullptr)) || !aligned(x) || !aligned(w_packed) ||
       !aligned(bias) || !aligned(y) || !aligned(table) || !aligned(k_cache))
     return DISTIE_BAD_ARGUMENT;

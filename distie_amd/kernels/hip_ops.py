@@ -272,7 +272,7 @@ class HipOps(Ops):
     # 2,245 us instead of 2,302).
     TILES_HOST_ROWS = 2048
     # (A weight that no role was named for stays with the passes: who reads its product is not known.)
-    # From LARGE_MIN_ROWS rows on, products on a packed copy run in the tiles of `large_tiles.hip` where those are the faster ones
+    # From LARGE_FEW_ROWS + 1 rows on, products on a packed copy run in the tiles of `large_tiles.hip` where those are the faster ones
     # (`_large_take`). Which is told by the rate, in TFLOP/s, that the count behind their plan comes to; measured on 25 weights of
     # 0.9 to 136 million elements and 27 row counts, in a captured graph, with the kernels that read the result (us, these tiles /
     # what there was, `packed_tiles` or the library's first choice with the kernels behind it):
@@ -291,7 +291,25 @@ class HipOps(Ops):
     #  * other plain ones from LARGE_PLAIN_RATE on ([1024, 2048] x [2048, 2048] 17 / 15, [1152, 2048] 17 / 20), weights of four times as
     #    many rows as K from LARGE_WIDE_RATE on ([400, 1024] x [4352, 1024] 11 / 10, [450, 1024] 10 / 12), up to LARGE_DENSE_WORK
     #    products, from where the library is the faster one ([900, 2048] x [8448, 2048] 36 / 40, [1024, 2048] 42 / 39, [2048, 2048] 76 / 66).
-    LARGE_MIN_ROWS = 65
+    # Up to LARGE_FEW_ROWS rows the kernel takes smaller tiles, and no count stands behind their plan (28 weights, 1 to 64 rows; what
+    # there was are the passes over the packed copy and `packed_tiles`):
+    #  * gated: from LARGE_FEW_GATED_ROWS rows on, weights of less than LARGE_FEW_GATED_ELEMENTS from LARGE_FEW_CUT_ROWS on ([8, 1536]
+    #    x [17920, 1536] 12.5 / 13.0, [9, 1536] 12.4 / 14.2, [32, 1536] 13.5 / 16.0, [64, 1536] 15.1 / 20.2; [16, 2048] x [16384, 2048]
+    #    14.3 / 15.3; [64, 3584] x [37888, 3584] 52 / 66; [9, 512] x [4096, 512] 4.6 / 4.4, [20, 512] 4.6 / 5.3);
+    #  * plain, for readers that add slices: LARGE_FEW_CUT_ROWS rows of large weights ([16, 3584] x [3584, 3584] 12.5 / 12.3, [20,
+    #    3584] 12.7 / 13.2, [64, 3584] 14.4 / 16.1; [32, 8192] x [2048, 8192] 13.0 / 15.2; [64, 11008] x [4096, 11008] 25 / 37; [24,
+    #    8960] x [1536, 8960] 13.0 / 13.0; [64, 2048] x [2048, 2048] 9.6 / 9.3);
+    #  * the heads of large vocabularies, LARGE_FEW_HEAD_ELEMENTS, from LARGE_FEW_CUT_ROWS rows on ([16, 1536] x [151936, 1536] 88 /
+    #    89, [20, 1536] 86 / 91, [64, 1536] 101 / 118; [32, 3584] x [152064, 3584] 201 / 217; [32, 2048] x [32768, 2048] 26.5 / 27.5 and
+    #    [64, 2048] 27.5 / 27.4).
+    LARGE_FEW_ROWS = 64
+    LARGE_FEW_GATED_ROWS = 9
+    LARGE_FEW_GATED_ELEMENTS = 8 << 20
+    LARGE_FEW_CUT_ROWS = 17
+    LARGE_FEW_LONG_ELEMENTS = 16 << 20
+    LARGE_FEW_SHORT_ELEMENTS = 12 << 20
+    LARGE_FEW_HEAD_ELEMENTS = 128 << 20
+    LARGE_MIN_ROWS = 9
     LARGE_GATED_RATE = 240.0
     LARGE_ROTARY_RATE = 150.0
     LARGE_ROTARY_ROWS = 416
@@ -993,7 +1011,15 @@ class HipOps(Ops):
 
     def _large_take(self, M, N, K, kind, cut_us, us) -> bool:
         """Whether a product that comes to `us` there, with the reader that adds its slices, is to run so: see the constants."""
-        rate, elements = 2e-6 * M * N * K / us, N * K
+        elements = N * K
+        if M <= self.LARGE_FEW_ROWS:
+            if kind == "gated":
+                return M >= (self.LARGE_FEW_GATED_ROWS if elements >= self.LARGE_FEW_GATED_ELEMENTS else self.LARGE_FEW_CUT_ROWS)
+            if kind == "plain" and cut_us == 0.0:
+                return M >= self.LARGE_FEW_CUT_ROWS and elements >= (self.LARGE_FEW_LONG_ELEMENTS if K >= 2 * N else
+                                                                     self.LARGE_FEW_SHORT_ELEMENTS)
+            return kind == "plain" and M >= self.LARGE_FEW_CUT_ROWS and elements >= self.LARGE_FEW_HEAD_ELEMENTS
+        rate = 2e-6 * M * elements / us
         if kind == "gated":
             return rate >= self.LARGE_GATED_RATE
         if kind == "rotary":

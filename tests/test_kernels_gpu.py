@@ -400,9 +400,10 @@ def test_packed_tiles_with_rotation(ops, shape, rows, heads, kv_heads, dim, K, P
 
 
 LARGE_SHAPES = [(0, 256), (1, 256), (2, 192), (3, 192), (4, 128), (5, 192), (6, 128), (7, 128)]
+FEW_ROWS_SHAPES = [(8, 32), (9, 32), (10, 64), (11, 64), (12, 32), (13, 64)]
 
 
-@pytest.mark.parametrize("shape,rows", LARGE_SHAPES)
+@pytest.mark.parametrize("shape,rows", LARGE_SHAPES + FEW_ROWS_SHAPES)
 @pytest.mark.parametrize("N,K", [(16, 256), (40, 320), (1040, 1088), (528, 4096)])
 def test_large_tiles(ops, shape, rows, N, K):
     """Every tile of the products of many rows: rows and columns that do not fill a tile, as few stages as there can be, odd and

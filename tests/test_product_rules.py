@@ -82,7 +82,7 @@ def test_plans_are_kept_apart_by_what_the_rule_reads(rules):
 
 @pytest.mark.parametrize("kind,rows,weight,takes", [
     # gated: nearly always; small weights from where they fill a few compute units
-    ("gated", 64, (37888, 3584), False), ("gated", 80, (37888, 3584), True), ("gated", 80, (17920, 1536), True),
+    ("gated", 64, (37888, 3584), True), ("gated", 80, (37888, 3584), True), ("gated", 80, (17920, 1536), True),
     ("gated", 65, (8192, 1024), False), ("gated", 193, (8192, 1024), True), ("gated", 2048, (17920, 1536), True),
     ("gated", 301, (17920, 1536), True), ("gated", 97, (4096, 512), False), ("gated", 2048, (17912, 1536), False),
     ("gated", 2048, (17920, 1544), False),
@@ -94,7 +94,13 @@ def test_plans_are_kept_apart_by_what_the_rule_reads(rules):
     ("down", 301, (1536, 8960), False), ("down", 2048, (1536, 8960), True), ("down", 128, (3584, 18944), False),
     ("down", 301, (3584, 18944), True), ("down", 2048, (1024, 2048), False), ("attn_out", 1024, (1536, 1536), False),
     ("attn_out", 2048, (1536, 1536), True), ("qkv", 1024, (1024, 1024), False), ("qkv", 640, (8448, 2048), True),
-    ("qkv", 2048, (8448, 2048), False)])
+    ("qkv", 2048, (8448, 2048), False),
+    # few rows
+    ("gated", 8, (17920, 1536), False), ("gated", 9, (17920, 1536), True), ("gated", 16, (4096, 512), False),
+    ("gated", 17, (4096, 512), True), ("down", 16, (2048, 8192), False), ("down", 17, (2048, 8192), True),
+    ("down", 64, (1536, 8960), False), ("attn_out", 64, (2048, 2048), False), ("attn_out", 17, (3584, 3584), True),
+    ("head", 16, (151936, 1536), False), ("head", 17, (151936, 1536), True), ("head", 64, (32768, 2048), False),
+    ("rotary", 64, (37888, 3584), False), ("qkv", 64, (8448, 2048), False)])
 def test_products_in_large_tiles(rules, kind, rows, weight, takes):
     rules.captured, rules.library_timed_rows = False, 0
     cut_us = None if kind in ("rotary", "gated") else 0.0 if kind in rules.ADDS_SLICES else rules.SUM_SLICES_US
@@ -104,7 +110,7 @@ def test_products_in_large_tiles(rules, kind, rows, weight, takes):
 
 @pytest.mark.parametrize("N,K", [(16, 256), (40, 320), (1536, 8960), (152064, 3584), (4608, 18944)])
 def test_large_tiles_plans_are_launches_that_the_kernel_takes(rules, N, K):
-    for rows in (1, 65, 128, 129, 777, 2048, 16384):
+    for rows in (1, 32, 33, 64, 65, 128, 129, 777, 2048, 16384):
         for mode in (0, 1, 2):
             for cut_us in (None, 0.0, 4.5):
                 shape, slices, us = ctypes.c_int(-1), ctypes.c_int(-1), ctypes.c_float(-1)
@@ -113,7 +119,8 @@ def test_large_tiles_plans_are_launches_that_the_kernel_takes(rules, N, K):
                 assert taken == (N % (16 if mode else 8) == 0)
                 if taken:
                     stages = K // 64
-                    assert (1 if mode == 2 else 0) <= shape.value <= 7 and us.value > 0
+                    few = rows <= 64 and mode != 2
+                    assert (1 if mode == 2 else 0) <= shape.value <= (13 if few else 7) and (us.value > 0) == (not few)
                     assert -(-stages // -(-stages // slices.value)) == slices.value and (slices.value == 1 or (mode == 0 and cut_us is not None))
 
 
