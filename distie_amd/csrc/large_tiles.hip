@@ -28,6 +28,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(int)))) int intx4;
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int LT_K = 64;              // k of a stage of x; W comes in halves of it
+constexpr int LT_EACH = 3;            // a mode beside PK_PLAIN, PK_GATED and PK_ROTARY
+constexpr int LT_EACH_MAX = 8;
 
 // A buffer of `bytes` from `base` on (both the same in all lanes): reads beyond it give zeros.
 __device__ __forceinline__ intx4 buffer_of(const void* base, uint32_t bytes) {
@@ -64,10 +66,12 @@ struct LargePlace {
   int row_blocks;               // blocks of 16 rows of the packed copy
   int m_tiles, n_tiles, slices;
   int stages;                   // of a slice
+  // LT_EACH: several weights one behind the other in one copy, each with an x of its own; what lies before the end of each
+  int tile_end[LT_EACH_MAX], block_end[LT_EACH_MAX];
 };
 
-// A workgroup: WM x WAVES / WM waves of TM x TN products of 32 x 32; D stages ahead. MODE: PK_PLAIN, PK_GATED, PK_ROTARY.
-// K a multiple of LT_K; columns of y a multiple of 16 bytes.
+// A workgroup: WM x WAVES / WM waves of TM x TN products of 32 x 32; D stages ahead. MODE: PK_PLAIN, PK_GATED, PK_ROTARY,
+// LT_EACH (plain, no bias). K a multiple of LT_K; columns of y a multiple of 16 bytes.
 template <int WAVES, int WM, int TM, int TN, int D, int MODE, typename Y>
 __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias, Y* __restrict__ y, int M, int N,
@@ -87,12 +91,19 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
   const int place = static_cast<int>(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
   if (place >= tiles * at.slices) return;
   const int slice = place / tiles, n_tile = place % tiles / at.m_tiles, m_tile = place % at.m_tiles;
-  const int m0 = m_tile * BM, b0 = n_tile * (BN / 16);
+  const int m0 = m_tile * BM;
+  int b0 = n_tile * (BN / 16), block_end = at.row_blocks;
+  if constexpr (MODE == LT_EACH) {
+    int e = 0, tile = 0, block = 0;
+    for (; n_tile >= at.tile_end[e]; ++e) tile = at.tile_end[e], block = at.block_end[e];
+    b0 = block + (n_tile - tile) * (BN / 16), block_end = at.block_end[e];
+    x += static_cast<int64_t>(e) * M * K;
+  }
   const int s_begin = slice * at.stages;
   const int stages = min(K / LT_K - s_begin, at.stages);
   const int k_tiles = K / 32;
 
-  const int rows = min(M - m0, BM), blocks = min(at.row_blocks - b0, BN / 16);
+  const int rows = min(M - m0, BM), blocks = min(block_end - b0, BN / 16);
   const intx4 x_buffer = buffer_of(x + static_cast<int64_t>(m0) * K, static_cast<uint32_t>(rows) * K * 2u);
   const intx4 w_buffer =
       buffer_of(w + static_cast<int64_t>(b0) * k_tiles * PK_TILE, static_cast<uint32_t>(blocks) * k_tiles * 1024u);
@@ -124,7 +135,7 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       float4 start = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (MODE != PK_GATED) {
+      if constexpr (MODE == PK_PLAIN || MODE == PK_ROTARY) {
         const int block = first_block + 2 * b + q / 2;
         const int column = MODE == PK_ROTARY ? rotary_column(block, 2 * (q % 2) + h, rotary.heads + rotary.kv_heads, rotary.dim)
                                              : 16 * block + 8 * (q % 2) + 4 * h;
@@ -199,7 +210,7 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
   constexpr int GROUP = 128 / (EACH * static_cast<int>(sizeof(Y)));                 // so many blocks of 32 at a time
   constexpr int STRIDE = 128 + 16, PIECE = 16 / static_cast<int>(sizeof(Y));        // bytes of a row there; values of a store
   char* own = lds + wave * (32 * STRIDE);
-  const int columns = MODE == PK_GATED ? N / 2 : N;
+  const int columns = MODE == PK_GATED ? N / 2 : N, column_end = MODE == LT_EACH ? 16 * block_end : columns;
   const int column0 = first_block * (MODE == PK_GATED ? 8 : 16);
   Y* out = y + static_cast<int64_t>(slice) * M * N;
   const int half = rotary.dim / 2, per_head = rotary.dim / 16, turned = rotary.heads + rotary.kv_heads;      // (PK_ROTARY)
@@ -241,7 +252,7 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
         for (int b = g; b < g + count; ++b) {
           char* to = own + r * STRIDE + ((b - g) * EACH + 4 * h) * sizeof(Y);
 #pragma unroll
-          for (int q = 0; q < 4; q += MODE == PK_PLAIN ? 1 : 2) {
+          for (int q = 0; q < 4; q += MODE == PK_GATED || MODE == PK_ROTARY ? 2 : 1) {
             float v[4], v2[4];
             if constexpr (MODE == PK_GATED) {
 #pragma unroll
@@ -284,7 +295,7 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
             }
           } else {
             const int column = column0 + g * EACH + piece * PIECE;
-            if (row0 + row < M && column < columns)
+            if (row0 + row < M && column < column_end)
               *reinterpret_cast<uint4*>(out + static_cast<int64_t>(row0 + row) * columns + column) = v;
           }
         }
@@ -391,10 +402,17 @@ LargePlan plan_few(int M, int N, int K, int row_blocks, int mode, bool may_cut, 
 
 template <int MODE, typename Y>
 int launch_large(const bf16_t* x, const bf16_t* w, const float* bias, Y* y, int M, int N, int K, int row_blocks, int shape,
-                 int slices, const RotaryOut& rotary, hipStream_t stream) {
+                 int slices, const RotaryOut& rotary, hipStream_t stream, int count = 0, const int32_t* ends = nullptr) {
   const int bm = LARGE_SHAPES[shape].rows(), blocks = LARGE_SHAPES[shape].blocks();
   const int all = K / LT_K;
-  const LargePlace at = {row_blocks, (M + bm - 1) / bm, (row_blocks + blocks - 1) / blocks, slices, (all + slices - 1) / slices};
+  LargePlace at = {row_blocks, (M + bm - 1) / bm, (row_blocks + blocks - 1) / blocks, slices, (all + slices - 1) / slices};
+  if (MODE == LT_EACH) {
+    at.n_tiles = 0;
+    for (int e = 0, begin = 0; e < count; begin = ends[e++]) {
+      at.n_tiles += (ends[e] - begin + blocks - 1) / blocks;
+      at.tile_end[e] = at.n_tiles, at.block_end[e] = ends[e];
+    }
+  }
   if ((all + at.stages - 1) / at.stages != slices) return DISTIE_BAD_ARGUMENT;
   const int64_t work = static_cast<int64_t>(at.m_tiles) * at.n_tiles * slices;
   if (work > (1 << 30)) return DISTIE_BAD_ARGUMENT;
@@ -486,4 +504,19 @@ extern "C" int distie_large_tiles_rotary_bf16(const void* x, const void* w_packe
                             static_cast<bf16_t*>(v_cache), heads, kv_heads, dim, block_size, write};
   return launch_large<PK_ROTARY, bf16_t>(static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w_packed), bias,
                                          static_cast<bf16_t*>(y), M, N, K, N / 16, shape, 1, rotary, stream);
+}
+
+// xs [count, M, K], each with its own rows of the copy, which end at block ends[e] (the last at `blocks`): y [M, 16 blocks] in
+// bfloat16, weight e in the columns that its blocks have. shape: as distie_large_tiles_plan gives it for 16 blocks columns.
+extern "C" int distie_large_tiles_each_bf16(const void* xs, const void* w_packed, void* y, int M, int K, int count,
+                                            const int32_t* ends, int shape, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (K < 4 * LT_K || K % LT_K != 0 || K > (1 << 20) || count < 1 || count > LT_EACH_MAX || ends == nullptr || shape < 0 ||
+      shape >= LARGE_SHAPE_COUNT || !aligned(xs) || !aligned(w_packed) || !aligned(y))
+    return DISTIE_BAD_ARGUMENT;
+  for (int e = 0; e < count; ++e)
+    if (ends[e] <= (e > 0 ? ends[e - 1] : 0) || ends[e] > (1 << 24)) return DISTIE_BAD_ARGUMENT;
+  return launch_large<LT_EACH, bf16_t>(static_cast<const bf16_t*>(xs), static_cast<const bf16_t*>(w_packed), nullptr,
+                                       static_cast<bf16_t*>(y), M, 16 * ends[count - 1], K, ends[count - 1], shape, 1, RotaryOut{},
+                                       stream, count, ends);
 }

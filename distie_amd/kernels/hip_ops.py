@@ -309,6 +309,10 @@ class HipOps(Ops):
     LARGE_FEW_LONG_ELEMENTS = 16 << 20
     LARGE_FEW_SHORT_ELEMENTS = 12 << 20
     LARGE_FEW_HEAD_ELEMENTS = 128 << 20
+    # Several products with inputs of their own share a launch of these tiles, as far as that was measured (four of [C, C] and a
+    # narrow unrounded one, which stays with the library at 12 us, us together / one by one in the library: C = 512, 300 rows 10 /
+    # 29; 1,024, 450 rows 18 / 42; 2,048, 33 rows 20 / 48, 1,802 rows 67 / 103; 3,072, 2,048 rows 147 / 185).
+    LARGE_EACH_WORK = 8e10
     LARGE_MIN_ROWS = 9
     LARGE_GATED_RATE = 240.0
     LARGE_ROTARY_RATE = 150.0
@@ -440,6 +444,7 @@ class HipOps(Ops):
         o.distie_packed_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_large_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F] + 2 * [ctypes.POINTER(_I)] + [ctypes.POINTER(_F)]
         o.distie_large_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
+        o.distie_large_tiles_each_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _P, _I, _P]
         o.distie_large_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_packed_each_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _P, _P]
         o.distie_decode_norm_fits.argtypes = [_I]
@@ -1031,6 +1036,15 @@ class HipOps(Ops):
             return rate >= (self.LARGE_LONG_RATE if M <= self.TILES_LONG_ROWS else self.LARGE_LONG_RATE_BEYOND)
         return rate >= (self.LARGE_SHORT_RATE if elements > self.ROW_GROUPS_MAX_ELEMENTS or N < self.TILES_FEW_WEIGHT_ROWS else
                         self.LARGE_SHORT_RATE_SMALL)
+
+    def _large_each(self, M, N, K, xs):
+        """The tile of the kernels for many rows for several products that share a launch, N columns in all, or None."""
+        if M * N * K > self.LARGE_EACH_WORK or not xs.is_contiguous() or xs.data_ptr() % 16:
+            return None
+        shape, slices, us = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0)
+        if not self._ops.distie_large_tiles_plan(M, N, K, 0, 0, 0.0, ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)):
+            return None
+        return shape.value
 
     def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, clamp=(0.0, 1.0, 0.0), large=False):
         """The tiled product; float32 slices if the plan cuts K."""
@@ -2081,19 +2095,33 @@ class HipOps(Ops):
 
     def linear_each(self, xs, weights, unrounded=()):
         held = getattr(weights[0], "_distie_each", None)
-        if held is None or xs.dtype != torch.bfloat16 or xs.shape[1] > self.EACH_MAX_ROWS:
+        if held is None or xs.dtype != torch.bfloat16:
             return super().linear_each(xs, weights, unrounded)
-        self._own(xs)
         packed, ends = held
         count, M, K = xs.shape
+        plan = None
+        if M > self.EACH_MAX_ROWS:
+            # the rounded ones in one launch, if they are the first; the others one by one
+            rounded = count - len(unrounded)
+            if rounded > 1 and all(k >= rounded for k in unrounded):
+                plan = self._large_each(M, 16 * int(ends[rounded - 1]), K, xs)
+            if plan is None:
+                return super().linear_each(xs, weights, unrounded)
+        self._own(xs)
         if count != len(weights) or any(w.shape[1] != K for w in weights) or \
                 [int(e) for e in np.diff(ends, prepend=0)] != [-(-w.shape[0] // 16) for w in weights] or \
                 packed.numel() != int(ends[-1]) * -(-K // 32) * 512:
             raise KernelError("linear_each: an input [rows, K] for every weight [N, K], the weights it was prepared for")
+        starts = [0] + [16 * int(e) for e in ends[:-1]]
+        if plan is not None:
+            out = torch.empty((M, 16 * int(ends[rounded - 1])), dtype=torch.bfloat16, device=self.device)
+            _check(self._ops.distie_large_tiles_each_bf16(xs.data_ptr(), packed.data_ptr(), out.data_ptr(), M, K, rounded,
+                                                          ends.ctypes.data, plan, self._stream()), "large_tiles_each_bf16")
+            return [out[:, at:at + w.shape[0]] for at, w in zip(starts, weights[:rounded])] + \
+                [self.linear_f32out(xs[k], weights[k]) for k in range(rounded, count)]
         out = torch.empty((M, 16 * int(ends[-1])), dtype=torch.float32, device=self.device)
         _check(self._ops.distie_gemm_packed_each_bf16(xs.data_ptr(), packed.data_ptr(), out.data_ptr(), M, K, count,
                                                       ends.ctypes.data, self._stream()), "gemm_packed_each_bf16")
-        starts = [0] + [16 * int(e) for e in ends[:-1]]
         return [out[:, at:at + w.shape[0]] for at, w in zip(starts, weights)]
 
     def wkv_decay_logits(self, low, up, up_bias):

@@ -182,6 +182,8 @@ def test_sixteen_queries_a_workgroup():
     """The wide form of the prefill kernel (steps of many tokens take it by themselves)."""
     from distie_amd.kernels.hip_ops import HipOps
 
+    from distie_amd.kernels.hip_ops import HipOps
+
     ops = HipOps("cuda:0")
     ops.MIXED_WIDE_TOKENS = 1
     for sizes in (dict(heads=6, kv_heads=3, dim=48, size=40, keep_first=18), dict(heads=16, kv_heads=4, dim=128, size=None)):
@@ -334,6 +336,30 @@ def test_products_of_each_mix(ops):
                 assert got[-1].dtype == torch.float32 and len({t.stride(0) for t in got[:-1] if t.shape == got[0].shape}) == 1
                 for k, w in enumerate(weights):
                     close(got[k].float(), xs[k].to(F) @ w.to(F).T, dtype, f"{rows} rows, product {k}", 0.6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [33, 64, 65, 129, 300])
+@pytest.mark.parametrize("widths,K", [((64, 64, 5), 256), ((40, 300, 512, 16, 7), 320), ((272,) * 4 + (16,), 576)])
+def test_products_of_each_mix_in_one_launch(rows, widths, K):
+    """`linear_each` beyond 32 rows: tiles that end inside a weight and at its end, blocks that are not whole, an x each."""
+    from distie_amd.kernels.hip_ops import HipOps
+
+    ops = HipOps("cuda:0")
+    xs = rnd(len(widths), rows, K, seed=rows).to(torch.bfloat16)
+    weights = [(rnd(n, K, seed=20 + i) / math.sqrt(K)).to(torch.bfloat16) for i, n in enumerate(widths)]
+    held = tuple(w.cuda() for w in weights)
+    ops.prepare_linear_each(held)
+    ends = held[0]._distie_each[1]
+    assert ops._large_each(rows, 16 * int(ends[-2]), K, xs.cuda()) is not None
+    strided = torch.empty(len(widths), 2, rows, K, dtype=torch.bfloat16, device="cuda")
+    strided[:, 0] = xs.cuda()
+    for given in (xs.cuda(), strided[:, 0]):                  # (the second takes the products one by one)
+        got = ops.linear_each(given, held, unrounded=(len(widths) - 1,))
+        assert got[-1].dtype == torch.float32
+        for k, w in enumerate(weights):
+            assert got[k].shape == (rows, widths[k])
+            close(got[k].float(), xs[k].to(F) @ w.to(F).T, torch.bfloat16, f"{rows} rows, product {k}", 0.6)
 
 
 def test_attention_refuses_what_it_does_not_take():
