@@ -131,6 +131,42 @@ def test_products_of_few_rows_in_float32_stream_the_weights(ops, xd, wd, M, N, K
                                      65, N, K, None) == -1                     # more rows than it takes: refused
 
 
+@pytest.mark.parametrize("M", [1, 7, 8, 16, 17, 32])
+@pytest.mark.parametrize("N,K,gated", [(3600, 3584, False), (1530, 8960, False), (3584, 18944, False), (17910, 1536, True),
+                                       (16000, 1600, True), (8210, 4096, True), (26000, 1536, True), (39990, 2560, True)])
+def test_float32_products_of_few_rows_through_lds(ops, M, N, K, gated):
+    """Large float32 weights, whole lines of them through LDS: every number of waves, rows of W and x that do not fill a
+    workgroup, K whole and cut, with a bias. A weight that begins off 16 bytes stays with the kernel on registers. Both are no
+    further from 64 bits than the vector ALU's kernel, by an eighth at most (which says that it is the rounding alone)."""
+    x, w, b = rand(M, K, seed=1), rand(N, K, seed=2), rand(N, seed=3)
+    off = lambda y, z: ((y.double() - z).norm() / z.norm()).item()
+    want = x.double() @ w.double().T
+    plain = torch.empty(M, N, device="cuda")
+    assert ops._ops.distie_gemv_rows(x.data_ptr(), 0, w.data_ptr(), 0, None, plain.data_ptr(), 0, M, N, K, None) == 0
+    slices = 1 if gated else ops._ops.distie_rows_f32_slices(M, N, K, 0)
+    if not gated and M >= 8:
+        groups = -(-N // 64)
+        cut = min((256 if M <= 16 else 512) // groups, K // 256)
+        assert slices == -(-(K // 64) // -(-(K // 64) // cut))
+    if gated:
+        gate, up = want[:, :N // 2], want[:, N // 2:]
+        want = gate / (1 + torch.exp(-gate)) * up
+        plain = plain[:, :N // 2] / (1 + torch.exp(-plain[:, :N // 2])) * plain[:, N // 2:]
+    shifted = torch.empty(N * K + 4, device="cuda")[1:N * K + 1].view(N, K)
+    shifted.copy_(w)
+    for weight in (w, shifted):
+        shape = (M, N // 2) if gated else (slices, M, N)
+        out = torch.full(shape, float("nan"), device="cuda")
+        assert ops._ops.distie_rows_f32(x.data_ptr(), weight.data_ptr(), None, out.data_ptr(), M, N, K, 1 if gated else 0, slices,
+                                        0.0, 1.0, 0.0, None) == 0
+        got = out if gated else out.sum(0)
+        assert off(got, want) <= 1.125 * off(plain, want)
+        if not gated:
+            assert ops._ops.distie_rows_f32(x.data_ptr(), weight.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, 0, slices,
+                                            0.0, 1.0, 0.0, None) == 0
+            close(out.sum(0), want + b.double(), torch.float32, scale=5 * want.abs().max().item())
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(16, 64), (102, 128), (250, 320), (1030, 1088), (96, 8960)])
 def test_float32_products_of_few_rows_on_the_matrix_cores(ops, M, N, K, monkeypatch):
