@@ -13,7 +13,8 @@
 //    their definitions.
 //
 // The reference leaves these products to a library (worker/src/inference/qwen2/model.py:149-152,
-// 231-233, 301); bfloat16 products of many rows (prefill) are left to the library here as well.
+// 231-233, 301); bfloat16 products of many rows (prefill) are in packed_tiles.hip and large_tiles.hip, those that neither is the
+// faster one for, or that have no packed copy, are left to the library here as well.
 
 #include "common.h"
 #include "packed.h"
