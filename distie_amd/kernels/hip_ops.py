@@ -280,14 +280,22 @@ class HipOps(Ops):
     #    3584] x [37888, 3584] 447 / 570, [65, 3584] 52 / 72; [128, 1024] x [8192, 1024] 9.5 / 9.2, [160, 1024] 10 / 12);
     #  * with rotation and cache write in the epilogue: beyond one round of the 64 x 64 tiles of `packed_tiles` ([512, 1536] x
     #    [2048, 1536] 17 / 12, [576, 1536] 17 / 18, [1152, 1536] 19 / 26, [2048, 1536] 26 / 24), for large weights, whose 64 x 128
-    #    tiles are two thirds as long as these, LARGE_ROTARY_ROWS ([352, 3584] x [4608, 3584] 34 / 30, [450, 3584] 33 / 36, [2048, 3584] 78
-    #    / 73, [1920, 3584] 66 / 69);
+    #    tiles are two thirds as long as these, LARGE_ROTARY_ROWS ([352, 3584] x [4608, 3584] 34 / 30, [450, 3584] 33 / 36, [1664,
+    #    3584] 60 / 61), up to LARGE_ROTARY_WORK products (alone [2048, 3584] takes 76 / 70, but a serving step of 2,025 tokens of the
+    #    7B shape 24.07 ms / 24.15: the library's kernel and the one behind it, 72 + 18 us there, suffer more from the clock that
+    #    the products around them leave; [1024, 4096] x [6144, 4096] 58 / 61, [2304, 4096] 136 / 106; [672, 5120] x [7168, 5120] 60 /
+    #    69, [2048, 5120] 166 / 143);
     #  * plain, for readers that add the slices of K: K at least twice as long as the weight has rows from LARGE_LONG_RATE on
     #    ([512, 8960] x [1536, 8960] 34 / 31, [576, 8960] 30 / 33, [2048, 8960] 66 / 83; [193, 18944] x [3584, 18944] 48 / 58, [2048,
     #    18944] 271 / 300), and past TILES_LONG_ROWS, where `packed_tiles` ends, LARGE_LONG_RATE_BEYOND ([1024, 4096] x [1024,
     #    4096] 22 / 21, [1280, 4096] 23 / 27); others from LARGE_SHORT_RATE on ([256, 3584] x [3584, 3584] 19.5 / 19, [301, 3584] 23 /
     #    26; [1408, 1536] x [1536, 1536] 24 / 23, [1536, 1536] 21 / 23), weights of 2,048 rows and up to
     #    ROW_GROUPS_MAX_ELEMENTS from LARGE_SHORT_RATE_SMALL on ([1536, 2048] x [2048, 2048] 30 / 28, [1667, 2048] 27 / 30);
+    #  * rotating ones and those of readers that add slices up to LARGE_ROWS rows; up to LARGE_MAX_ROWS where K is five times as long
+    #    as the weight has rows, and up to LARGE_MANY_ROWS_WORK products ([2304, 8192] x [2048, 8192] 88 / 96, [4096, 8192] 141 / 132,
+    #    [8192, 8192] 246 / 216; [3072, 8960] x [1536, 8960] 93 / 109, [4096, 8960] 116 / 119, [8192, 8960] 207 / 195; [8192, 1536] x
+    #    [2048, 1536] with rotation 79 / 58). Steps, us, with this line / without: 1.5B shape, 8,000 tokens 28,040 / 28,690; 7B shape,
+    #    4,096 tokens 49,220 / 50,600. The gated ones win at 8,192 rows, too ([8192, 1536] x [17920, 1536] 386 / 446);
     #  * other plain ones from LARGE_PLAIN_RATE on ([1024, 2048] x [2048, 2048] 17 / 15, [1152, 2048] 17 / 20), weights of four times as
     #    many rows as K from LARGE_WIDE_RATE on ([400, 1024] x [4352, 1024] 11 / 10, [450, 1024] 10 / 12), up to LARGE_DENSE_WORK
     #    products, from where the library is the faster one ([900, 2048] x [8448, 2048] 36 / 40, [1024, 2048] 42 / 39, [2048, 2048] 76 / 66).
@@ -317,6 +325,10 @@ class HipOps(Ops):
     LARGE_GATED_RATE = 240.0
     LARGE_ROTARY_RATE = 150.0
     LARGE_ROTARY_ROWS = 416
+    LARGE_ROTARY_WORK = 4e10
+    LARGE_ROWS = 2304
+    LARGE_MAX_ROWS = 4096
+    LARGE_MANY_ROWS_WORK = 1.3e10
     LARGE_LONG_RATE = 515.0
     LARGE_LONG_RATE_BEYOND = 380.0
     LARGE_SHORT_RATE = 316.0
@@ -1025,13 +1037,17 @@ class HipOps(Ops):
                                                                      self.LARGE_FEW_SHORT_ELEMENTS)
             return kind == "plain" and M >= self.LARGE_FEW_CUT_ROWS and elements >= self.LARGE_FEW_HEAD_ELEMENTS
         rate = 2e-6 * M * elements / us
+        many = M > self.LARGE_ROWS and (M > self.LARGE_MAX_ROWS or (M * elements > self.LARGE_MANY_ROWS_WORK and K < 5 * N))
         if kind == "gated":
             return rate >= self.LARGE_GATED_RATE
         if kind == "rotary":
             return -(-M // 64) * -(-N // 64) > self._compute_units and rate >= self.LARGE_ROTARY_RATE and \
+                not many and M * elements <= self.LARGE_ROTARY_WORK and \
                 (M >= self.LARGE_ROTARY_ROWS or elements <= self.TILES_LARGE_ROTARY)
         if cut_us != 0.0:
             return rate >= (self.LARGE_WIDE_RATE if N >= 4 * K else self.LARGE_PLAIN_RATE) and M * elements <= self.LARGE_DENSE_WORK
+        if many:
+            return False
         if K >= 2 * N:
             return rate >= (self.LARGE_LONG_RATE if M <= self.TILES_LONG_ROWS else self.LARGE_LONG_RATE_BEYOND)
         return rate >= (self.LARGE_SHORT_RATE if elements > self.ROW_GROUPS_MAX_ELEMENTS or N < self.TILES_FEW_WEIGHT_ROWS else

@@ -89,12 +89,16 @@ def test_plans_are_kept_apart_by_what_the_rule_reads(rules):
     # rotation: beyond one round of the smaller tiles
     ("rotary", 512, (2048, 1536), False), ("rotary", 576, (2048, 1536), True), ("rotary", 301, (3072, 2048), False),
     ("rotary", 352, (3072, 2048), True), ("rotary", 640, (1536, 1024), False), ("rotary", 704, (1536, 1024), True),
-    ("rotary", 256, (4608, 3584), False), ("rotary", 2048, (4608, 3584), True),
+    ("rotary", 256, (4608, 3584), False), ("rotary", 1792, (4608, 3584), True), ("rotary", 2048, (4608, 3584), True),
+    ("rotary", 2048, (7168, 5120), False), ("rotary", 4096, (2048, 1536), True), ("rotary", 4097, (2048, 1536), False),
+    ("rotary", 2304, (4608, 3072), True), ("rotary", 2305, (4608, 3072), False),
     # plain: where the count comes to a rate that neither the smaller tiles nor the library reach
     ("down", 301, (1536, 8960), False), ("down", 2048, (1536, 8960), True), ("down", 128, (3584, 18944), False),
     ("down", 301, (3584, 18944), True), ("down", 2048, (1024, 2048), False), ("attn_out", 1024, (1536, 1536), False),
     ("attn_out", 2048, (1536, 1536), True), ("qkv", 1024, (1024, 1024), False), ("qkv", 640, (8448, 2048), True),
-    ("qkv", 2048, (8448, 2048), False),
+    ("qkv", 2048, (8448, 2048), False), ("attn_out", 4096, (1536, 1536), True), ("attn_out", 4097, (1536, 1536), False),
+    ("down", 2304, (2048, 8192), True), ("down", 2305, (2048, 8192), False), ("down", 4096, (1536, 8960), True), ("down", 4097, (1536, 8960), False),
+    ("gated", 8192, (17920, 1536), True),
     # few rows
     ("gated", 8, (17920, 1536), False), ("gated", 9, (17920, 1536), True), ("gated", 16, (4096, 512), False),
     ("gated", 17, (4096, 512), True), ("down", 16, (2048, 8192), False), ("down", 17, (2048, 8192), True),
