@@ -494,6 +494,31 @@ def test_large_tiles_gate_at_its_limits(ops):
     torch.testing.assert_close(got, want[:, None].expand(M, I), rtol=2 ** -8, atol=1e-30, equal_nan=True)
 
 
+@pytest.mark.parametrize("shape", [0, 7, 10])
+@pytest.mark.parametrize("clamped", [False, True])
+def test_large_tiles_gate_keeps_32_bits(ops, shape, clamped):
+    """Gates down to where the exponential ends, exact sums, a large factor: the activation is off by a few units of 2^-24, so that
+    its rounding to 8 bits is another than that of the exact value only where that lies so near the middle of two of them. With
+    four units: a window of 2 x 4 x 2^-24 x 2 (the largest mantissa) in every 2^-7, a share of 2^-13."""
+    K, I, M = 256, 1024, 256
+    g = torch.Generator().manual_seed(3)
+    a = -(0.5 + 8.9 * torch.rand(M, generator=g)).to(torch.bfloat16)
+    b = (0.5 + 8.9 * torch.rand(I, generator=g)).to(torch.bfloat16)
+    a[:8], b[:8] = -9.375, 9.4375
+    x, w = torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(2 * I, K, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1], w[:I, 0], w[I:, 1] = a, 2.0 ** 60, b, 1.0
+    x, w = x.cuda(), w.cuda()
+    ops.prepare_linear(w, gated=True, role="gate_up")
+    act, clamp = (ops.CLAMPED, (120.0, 1.0, 1.0)) if clamped else (0, (0.0, 1.0, 0.0))
+    got = ops._run_tiles((shape, 1), x, w._distie_gated, None, torch.bfloat16, M, 2 * I, K, gated=1 | (act << 8), clamp=clamp,
+                         large=True).cpu()
+    v = a.double()[:, None] * b.double()[None, :]
+    want = v / (1 + torch.exp(-v)) * (121.0 if clamped else 2.0 ** 60)
+    assert v.min() < -88 and want.abs().min() > 1e-37
+    assert ((got.double() - want) / want).abs().max() <= 2 ** -8 * (1 + 2 ** -10)
+    assert (got != want.to(torch.bfloat16)).double().mean() <= 2 ** -13
+
+
 @pytest.mark.parametrize("shape,rows", LARGE_SHAPES[1:])
 @pytest.mark.parametrize("heads,kv_heads,dim,K,P", [(3, 1, 16, 256, 4), (2, 2, 80, 320, 16), (12, 2, 128, 1088, 16)])
 def test_large_tiles_with_rotation(ops, shape, rows, heads, kv_heads, dim, K, P):
