@@ -519,6 +519,34 @@ def test_large_tiles_gate_keeps_32_bits(ops, shape, clamped):
     assert (got != want.to(torch.bfloat16)).double().mean() <= 2 ** -13
 
 
+@pytest.mark.parametrize("shape,rows", LARGE_SHAPES + FEW_ROWS_SHAPES)
+def test_large_tiles_with_gelu_and_squares(ops, shape, rows):
+    """The two activations that `test_large_tiles` leaves out. Sums as there; then exact sums, where nothing but the activation
+    rounds: the argument of gelu's exponential, up to 36 here, is off by five roundings, 90 units of 2^-24, the result by another
+    half of 2^-7 in 8 bits."""
+    N, K = 1040, 320
+    w = rand(N, K, dtype=torch.bfloat16, seed=4, scale=2.0 * K ** -0.5)
+    ops.prepare_linear(w, gated=True, role="gate_up")
+    gelu = lambda z: z / (1 + torch.exp(-1.5957691216057308 * (z + 0.044715 * z ** 3)))
+    kinds = ((ops.ACTIVATIONS["gelu_tanh"], gelu), (ops.ACTIVATIONS["relu2"], lambda z: z.clamp(min=0) ** 2))
+    for M in (1, rows + 1):
+        x = rand(M, K, dtype=torch.bfloat16, seed=M)
+        product = x.double() @ w.double().T
+        for kind, act in kinds:
+            want = act(product[:, :N // 2]) * product[:, N // 2:]
+            got = ops._run_tiles((shape, 1), x, w._distie_gated, None, torch.bfloat16, M, N, K, gated=1 | ((kind + 1) << 8), large=True)
+            close(got, want, torch.bfloat16, scale=want.abs().max().item())
+    x, w = torch.zeros(rows, K, dtype=torch.bfloat16), torch.zeros(N, K, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = torch.linspace(-2.6, 2.6, rows).to(torch.bfloat16), 1.0
+    w[:N // 2, 0], w[N // 2:, 1] = torch.linspace(0.1, 2.6, N // 2).to(torch.bfloat16), 3.0
+    v = x[:, :1].double() * w[:N // 2, 0].double()
+    x, w = x.cuda(), w.cuda()
+    ops.prepare_linear(w, gated=True, role="gate_up")
+    for kind, act in kinds:
+        got = ops._run_tiles((shape, 1), x, w._distie_gated, None, torch.bfloat16, rows, N, K, gated=1 | ((kind + 1) << 8), large=True)
+        torch.testing.assert_close(got.double().cpu(), 3.0 * act(v), rtol=2 ** -8 * (1 + 2 ** -9), atol=0.0)
+
+
 @pytest.mark.parametrize("shape,rows", LARGE_SHAPES[1:])
 @pytest.mark.parametrize("heads,kv_heads,dim,K,P", [(3, 1, 16, 256, 4), (2, 2, 80, 320, 16), (12, 2, 128, 1088, 16)])
 def test_large_tiles_with_rotation(ops, shape, rows, heads, kv_heads, dim, K, P):
