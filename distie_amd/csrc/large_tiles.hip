@@ -379,7 +379,9 @@ LargePlan plan_large(int M, int N, int K, int row_blocks, int mode, bool may_cut
       const int64_t units = s.pair_us > 0.f ? 512 : 256, work = tiles * cut, full = work / units, rest = work % units;
       const float busy = rest / 256.f;
       float us = full * (stages * (s.few_us + s.more_us + s.pair_us) + turn);
-      if (rest > 0) us += stages * (s.few_us + s.more_us * std::min(busy, 1.f) + s.pair_us * std::max(busy - 1.f, 0.f)) + turn;
+      // (a unit with two takes its time however few such units there are, by how loaded the chip is: half of pair_us and up)
+      const float pair = busy > 1.f ? s.pair_us * (0.45f + 0.5f * (busy - 1.f)) : 0.f;
+      if (rest > 0) us += stages * (s.few_us + s.more_us * std::min(busy, 1.f) + pair) + turn;
       us = 2.2f + std::max(us, memory_us);
       if (cut > 1) us += 4.f * cut * values / 8.0e6f;
       if (mode == PK_PLAIN && may_cut) {

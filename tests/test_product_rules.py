@@ -222,3 +222,20 @@ def test_wide_heads_on_pages_that_only_columns_take():
     lib.distie_attention_columns_f32_runs.argtypes = [ctypes.c_int] * 5 + [ctypes.c_int64, ctypes.c_int]
     assert HipOps._columns_runs(lib, 1, 1, 8, 1, 16, 2560, 24, 0) == 0
     assert HipOps._columns_runs(lib, 1, 1, 8, 1, 12, 2560, 24, 0) == 1
+
+
+def large_plan(rules, rows, N, K, kind, cut_us=None):
+    shape, slices, us = ctypes.c_int(-1), ctypes.c_int(-1), ctypes.c_float(-1)
+    assert rules._ops.distie_large_tiles_plan(rows, N, K, rules.LARGE_KINDS[kind], cut_us is not None, cut_us or 0.0,
+                                              ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us))
+    return shape.value, slices.value, us.value
+
+
+@pytest.mark.parametrize("kind,rows,weight,cut_us,measured", [
+    # a few more tiles of 128 x 128 (shape 7) than compute units: us of those and of the tile that is taken instead
+    ("gated", 224, (17920, 1536), None, (30.7, 21.5)), ("gated", 400, (9728, 896), None, (17.1, 12.1)),
+    ("gated", 301, (11008, 2048), None, (27.0, 22.4)), ("rotary", 1024, (4608, 3584), None, (58.8, 46.8)),
+    ("rotary", 1408, (3072, 2048), None, (33.0, 28.3)), ("plain", 900, (4352, 1024), 4.5, (15.8, 14.1))])
+def test_units_with_two_workgroups_are_counted_in_full(rules, kind, rows, weight, cut_us, measured):
+    shape, slices, us = large_plan(rules, rows, *weight, kind, cut_us)
+    assert shape in (4, 5, 6) and slices == 1 and abs(us / measured[1] - 1) < 0.15
