@@ -366,7 +366,7 @@ struct LargePlan {
 LargePlan plan_large(int M, int N, int K, int row_blocks, int mode, bool may_cut, float cut_us) {
   LargePlan best = {-1, 0, 0.f};
   const int all = K / LT_K;
-  const float memory_us = static_cast<float>(row_blocks) * K * 32.f / 3.8e6f, values = static_cast<float>(M) * N;
+  const float memory_us = static_cast<float>(row_blocks) * K * 32.f / 5.2e6f, values = static_cast<float>(M) * N;
   for (int i = 0; i < LARGE_COUNTED; ++i) {
     const LargeShape& s = LARGE_SHAPES[i];
     if (mode == PK_ROTARY && (i < LARGE_ROTARY_FROM || i >= LARGE_ROTARY_TO)) continue;

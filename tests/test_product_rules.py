@@ -239,3 +239,20 @@ def large_plan(rules, rows, N, K, kind, cut_us=None):
 def test_units_with_two_workgroups_are_counted_in_full(rules, kind, rows, weight, cut_us, measured):
     shape, slices, us = large_plan(rules, rows, *weight, kind, cut_us)
     assert shape in (4, 5, 6) and slices == 1 and abs(us / measured[1] - 1) < 0.15
+
+
+@pytest.mark.parametrize("kind,rows,weight,cut_us,shapes,slices,measured", [
+    # few rows of large weights: us of the tile taken (a slower floor made all tiles equal and the first was taken: 72, 74.9, 37.1, 52.0)
+    ("gated", 65, (37888, 3584), None, (3, 6), 1, 53.7), ("gated", 128, (37888, 3584), None, (3, 6), 1, 60.5),
+    ("plain", 128, (4096, 11008), 0.0, (7,), 6, 30.7), ("plain", 160, (3584, 18944), 0.0, (5,), 8, 42.6)])
+def test_plans_of_few_rows_go_by_the_rate_that_memory_reaches(rules, kind, rows, weight, cut_us, shapes, slices, measured):
+    shape, cut, us = large_plan(rules, rows, *weight, kind, cut_us)
+    assert shape in shapes and cut == slices and abs(us / measured - 1) < 0.15
+
+
+@pytest.mark.parametrize("rows", [9, 64, 65, 66, 72, 73, 80])
+@pytest.mark.parametrize("weight", [(17920, 1536), (16384, 2048), (37888, 3584)])
+def test_gated_products_in_large_tiles_leave_no_rows_out(rules, rows, weight):
+    """Both sides of the row count where the smaller tiles end: us in these tiles / what there was, 65 rows 17 / 22, 21.5 / 22 and 52 / 72."""
+    rules.captured, rules.library_timed_rows = False, 0
+    assert rules._large(rows, *weight, "gated", ()) is not None
