@@ -393,7 +393,7 @@ class HipOps(Ops):
         self.library_timed_rows = self.library_timed_portion = 0
         self._packed_left_out = 0
         self._tile_plans: Dict[tuple, Optional[tuple]] = {}
-        self._large_plans: Dict[tuple, Optional[tuple]] = {}
+        self._large_plans: Dict[tuple, object] = {}       # of `_tiled` and `_large_each`
         self._ops = ctypes.CDLL(str(build.ensure("ops")))
         self._declare()
         self._attn: Dict[int, ctypes.CDLL] = {}
@@ -806,10 +806,9 @@ class HipOps(Ops):
             _check(self._ops.distie_rows_f32(x.data_ptr(), gate_up_weight.data_ptr(), None, out.data_ptr(), M, N, K, gated, 1,
                                              *clamp, self._stream()), "rows_f32")
             return out
-        plan = large = None
+        plan, large = None, False
         if packed is not None and x.dtype == torch.bfloat16:
-            large = self._large(x.shape[0], *gate_up_weight.shape, "gated", (x,))
-            plan = large or self._tiles(x.shape[0], *gate_up_weight.shape, "gated")
+            plan, large = self._tiled(x.shape[0], *gate_up_weight.shape, "gated", (x,))
         if packed is None or x.dtype != torch.bfloat16 or \
                 (plan is None and x.shape[0] > self._packed_rows(x.shape[0], *gate_up_weight.shape)):
             return apart(self.linear(x, gate_up_weight))
@@ -819,7 +818,7 @@ class HipOps(Ops):
         if packed.numel() != self._packed_elements(N, K, True):
             raise KernelError("linear_silu_mul: the packed copy does not belong to this weight")
         if plan is not None:
-            return self._run_tiles(plan, x, packed, None, x.dtype, M, N, K, gated, clamp=clamp, large=large is not None)
+            return self._run_tiles(plan, x, packed, None, x.dtype, M, N, K, gated, clamp=clamp, large=large)
         out = torch.empty((M, N // 2), dtype=x.dtype, device=self.device)
         if M <= self.ONE_WAVE_MAX_ROWS:
             _check(self._ops.distie_gemm_packed_bf16(x.data_ptr(), packed.data_ptr(), None, out.data_ptr(), _code(out),
@@ -874,12 +873,11 @@ class HipOps(Ops):
                 table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads, num_kv_heads,
                 head_dim, meta.block_size, 1 if write else 0, self._stream()), "rows_f32_rotary")
             return out
-        plan = large = None
+        plan, large = None, False
         fused = held is not None and held[1] == (num_heads, num_kv_heads, head_dim) and x.dtype == torch.bfloat16 and \
             inv_freq is not None and 2 * inv_freq.shape[0] == head_dim and k_cache.dtype == torch.bfloat16
         if fused:
-            large = self._large(x.shape[0], *weight.shape, "rotary", (x, bias, k_cache))
-            plan = large or self._tiles(x.shape[0], *weight.shape, "rotary")
+            plan, large = self._tiled(x.shape[0], *weight.shape, "rotary", (x, bias, k_cache))
             fused = plan is not None or x.shape[0] <= self._packed_rows(x.shape[0], *weight.shape)
         if not fused:
             return self.rope_kv_write(self.linear(x, weight, bias), meta, group, k_cache, v_cache, inv_freq,
@@ -916,7 +914,7 @@ class HipOps(Ops):
         table = self._rope_table(meta, inv_freq)
         out = torch.empty((M, N), dtype=torch.bfloat16, device=self.device)
         if plan is not None:
-            kernel, name = (self._ops.distie_large_tiles_rotary_bf16, "large_tiles_rotary_bf16") if large is not None else \
+            kernel, name = (self._ops.distie_large_tiles_rotary_bf16, "large_tiles_rotary_bf16") if large else \
                 (self._ops.distie_packed_tiles_rotary_bf16, "packed_tiles_rotary_bf16")
             _check(kernel(
                 x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
@@ -1002,29 +1000,38 @@ class HipOps(Ops):
 
     LARGE_KINDS = {"plain": 0, "gated": 1, "rotary": 2}
 
+    def _tiled(self, M: int, N: int, K: int, kind: str, tensors, cut_us: Optional[float] = None):
+        """((shape, slices), whether in the kernels for many rows) of a product as in `_tiles`, (None, False) if it runs in no
+        tiles; `tensors` as in `_large`. One look into what was found before: a step that is launched kernel by kernel comes
+        here for every product of every layer."""
+        if M < self.LARGE_MIN_ROWS:
+            return None, False
+        key = (M, N, K, kind, cut_us, self.captured, self.library_timed_rows, self.library_timed_portion)
+        try:
+            large, tiles = self._large_plans[key]
+        except KeyError:
+            large, tiles = self._large(M, N, K, kind, (), cut_us), self._tiles(M, N, K, kind, cut_us)
+            if len(self._large_plans) >= self.TILE_PLANS:
+                self._large_plans.clear()
+            self._large_plans[key] = large, tiles
+        if large is None:
+            return tiles, False
+        for t in tensors:
+            if t is not None and t.data_ptr() % 16:
+                return tiles, False
+        return large, True
+
     def _large(self, M: int, N: int, K: int, kind: str, tensors, cut_us: Optional[float] = None):
         """(shape, slices) of the kernels for many rows for a product as in `_tiles`, None if another kernel is the better one or
         one of the caller's `tensors`, which they take 16 bytes at a time, begins at no multiple of that."""
-        if M < self.LARGE_MIN_ROWS:
+        if M < self.LARGE_MIN_ROWS or any(t is not None and t.data_ptr() % 16 for t in tensors):
             return None
-        key = (M, N, K, kind, cut_us)
-        try:
-            plan = self._large_plans[key]
-        except KeyError:
-            plan = None
-            shape, slices, us = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0)
-            if self._ops.distie_large_tiles_plan(M, N, K, self.LARGE_KINDS[kind], cut_us is not None, cut_us or 0.0,
-                                                 ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)) and \
-                    self._large_take(M, N, K, kind, cut_us, us.value):
-                plan = (shape.value, slices.value)
-            if len(self._large_plans) >= self.TILE_PLANS:
-                self._large_plans.clear()
-            self._large_plans[key] = plan
-        if plan is not None:
-            for t in tensors:
-                if t is not None and t.data_ptr() % 16:
-                    return None
-        return plan
+        shape, slices, us = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0)
+        if self._ops.distie_large_tiles_plan(M, N, K, self.LARGE_KINDS[kind], cut_us is not None, cut_us or 0.0,
+                                             ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)) and \
+                self._large_take(M, N, K, kind, cut_us, us.value):
+            return shape.value, slices.value
+        return None
 
     def _large_take(self, M, N, K, kind, cut_us, us) -> bool:
         """Whether a product that comes to `us` there, with the reader that adds its slices, is to run so: see the constants."""
@@ -1057,10 +1064,19 @@ class HipOps(Ops):
         """The tile of the kernels for many rows for several products that share a launch, N columns in all, or None."""
         if M * N * K > self.LARGE_EACH_WORK or not xs.is_contiguous() or xs.data_ptr() % 16:
             return None
+        key = (M, N, K)
+        try:
+            return self._large_plans[key]
+        except KeyError:
+            pass
         shape, slices, us = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0)
-        if not self._ops.distie_large_tiles_plan(M, N, K, 0, 0, 0.0, ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)):
-            return None
-        return shape.value
+        plan = None
+        if self._ops.distie_large_tiles_plan(M, N, K, 0, 0, 0.0, ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)):
+            plan = shape.value
+        if len(self._large_plans) >= self.TILE_PLANS:
+            self._large_plans.clear()
+        self._large_plans[key] = plan
+        return plan
 
     def _run_tiles(self, plan, x, packed, bias, out_dtype, M, N, K, gated=0, clamp=(0.0, 1.0, 0.0), large=False):
         """The tiled product; float32 slices if the plan cuts K."""
@@ -1198,15 +1214,14 @@ class HipOps(Ops):
         packed = packed if both_bf16 else None
         if lazy and packed is not None and self._fused(M) and K % 8 == 0 and out_dtype == torch.bfloat16:
             return PendingProduct(x, weight, bias)
-        plan = large = None
+        plan, large = None, False
         if packed is not None and weight._distie_role is not None:
             adds = partial_ok and weight._distie_role in self.ADDS_SLICES
-            large = self._large(M, N, K, "plain", (x, bias), 0.0 if adds else self.SUM_SLICES_US)
-            plan = large or self._tiles(M, N, K, "plain", 0.0 if adds else self.SUM_SLICES_US)
+            plan, large = self._tiled(M, N, K, "plain", (x, bias), 0.0 if adds else self.SUM_SLICES_US)
         if plan is not None:
             if packed.numel() != self._packed_elements(N, K, False):
                 raise KernelError("linear: the packed copy does not belong to this weight")
-            out = self._run_tiles(plan, x, packed, bias, out_dtype, M, N, K, large=large is not None)
+            out = self._run_tiles(plan, x, packed, bias, out_dtype, M, N, K, large=large)
             return out if partial_ok else self.dense(out)
         if packed is not None and self.ONE_WAVE_MAX_ROWS < M <= self._packed_rows(M, N, K) and K % 8 == 0 and \
                 N * K > self.ROW_GROUPS_MAX_ELEMENTS:

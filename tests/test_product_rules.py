@@ -256,3 +256,24 @@ def test_gated_products_in_large_tiles_leave_no_rows_out(rules, rows, weight):
     """Both sides of the row count where the smaller tiles end: us in these tiles / what there was, 65 rows 17 / 22, 21.5 / 22 and 52 / 72."""
     rules.captured, rules.library_timed_rows = False, 0
     assert rules._large(rows, *weight, "gated", ()) is not None
+
+
+def test_products_met_before_take_one_look(rules):
+    """A step that is launched kernel by kernel asks for every product of every layer: what was found is kept, by what the rules
+    read, and an input off 16 bytes has the other kernels each time."""
+    rules.captured, rules.library_timed_rows = False, 0
+    data, xs = torch.empty(64, dtype=torch.bfloat16), torch.empty(2, 8, 64, dtype=torch.bfloat16)
+    asked = [(M, N, K, kind, cut_us) for M in (9, 32, 64, 301, 2048) for N, K in ((17920, 1536), (1536, 8960), (2048, 1536))
+             for kind, cut_us in (("gated", None), ("rotary", None), ("plain", 0.0), ("plain", rules.SUM_SLICES_US))]
+    first = [rules._tiled(*a[:4], (data, None), a[4]) for a in asked]
+    each = [rules._large_each(rows, 4096, 1024, xs) for rows in (33, 300)]
+    for (plan, large), (M, N, K, kind, cut_us) in zip(first, asked):
+        assert plan == (rules._large(M, N, K, kind, (), cut_us) or rules._tiles(M, N, K, kind, cut_us))
+        assert large == (rules._large(M, N, K, kind, (), cut_us) is not None)
+    off = [rules._tiled(*a[:4], (data[1:], None), a[4]) for a in asked]
+    assert off == [(rules._tiles(*a), False) for a in asked]
+    assert rules._tiled(8, 17920, 1536, "gated", (data,)) == (None, False)
+    rules._ops = None                                        # no rule is walked through again
+    assert [rules._tiled(*a[:4], (data, None), a[4]) for a in asked] == first
+    assert [rules._large_each(rows, 4096, 1024, xs) for rows in (33, 300)] == each
+    assert len(rules._large_plans) <= rules.TILE_PLANS
