@@ -486,6 +486,14 @@ extern "C" int distie_large_tiles_plan(int M, int N, int K, int mode, int may_cu
   return 1;
 }
 
+// How many tiles of that shape lie one below the other for M rows, and side by side for N columns.
+extern "C" int distie_large_tiles_grid(int M, int N, int shape, int* row_tiles, int* column_tiles) {
+  if (M < 1 || N < 1 || shape < 0 || shape >= LARGE_SHAPE_COUNT) return DISTIE_BAD_ARGUMENT;
+  const LargeShape& s = LARGE_SHAPES[shape];
+  *row_tiles = (M + s.rows() - 1) / s.rows(), *column_tiles = ((N + 15) / 16 + s.blocks() - 1) / s.blocks();
+  return 0;
+}
+
 // y: [M, N] of y_dtype (gated: [M, N / 2] in bfloat16), or with slices > 1 float32 [slices, M, N], to be added in order by
 // whoever reads it, the bias in the first. All pointers at multiples of 16 bytes.
 extern "C" int distie_large_tiles_bf16(const void* x, const void* w_packed, const float* bias, void* y, int y_dtype, int M,

@@ -299,6 +299,13 @@ class HipOps(Ops):
     #  * other plain ones from LARGE_PLAIN_RATE on ([1024, 2048] x [2048, 2048] 17 / 15, [1152, 2048] 17 / 20), weights of four times as
     #    many rows as K from LARGE_WIDE_RATE on ([400, 1024] x [4352, 1024] 11 / 10, [450, 1024] 10 / 12), up to LARGE_DENSE_WORK
     #    products, from where the library is the faster one ([900, 2048] x [8448, 2048] 36 / 40, [1024, 2048] 42 / 39, [2048, 2048] 76 / 66).
+    # A single row of tiles (65 to 192 rows), half of the compute units or fewer with one: such a tile takes 0.5 us and more for every
+    # 64 k, however idle the rest is, and the smaller tiles and passes of before, which spread over more units, are ahead where K is
+    # long: beyond LARGE_IDLE_K ([88, 2560] x [13824, 2560] 27 / 25, [160, 3072] x [16384, 3072] 39 / 35; plain [128, 3072] x [13056,
+    # 3072] 33 / 29, [192, 3584] x [15232, 3584] 45 / 35; with K = 2,048 level: [88, 2048] x [16384, 2048] 24.3 / 23.6, [128, 2048]
+    # 24.5 / 25.6), a quarter of them at any K ([128, 1536] x [8192, 1536] 18.0 / 13.2). Not where all that is left are passes over the
+    # weight, which are much slower than tiles there ([160, 2560] x [10880, 2560] in those of packed_tiles 22, [176, 2560] in passes 39).
+    LARGE_IDLE_K = 2048
     # Up to LARGE_FEW_ROWS rows the kernel takes smaller tiles, and no count stands behind their plan (28 weights, 1 to 64 rows; what
     # there was are the passes over the packed copy and `packed_tiles`):
     #  * gated: from LARGE_FEW_GATED_ROWS rows on, weights of less than LARGE_FEW_GATED_ELEMENTS from LARGE_FEW_CUT_ROWS on ([8, 1536]
@@ -455,6 +462,7 @@ class HipOps(Ops):
         o.distie_packed_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
         o.distie_packed_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_large_tiles_plan.argtypes = [_I, _I, _I, _I, _I, _F] + 2 * [ctypes.POINTER(_I)] + [ctypes.POINTER(_F)]
+        o.distie_large_tiles_grid.argtypes = [_I, _I, _I] + 2 * [ctypes.POINTER(_I)]
         o.distie_large_tiles_bf16.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P]
         o.distie_large_tiles_each_bf16.argtypes = [_P, _P, _P, _I, _I, _I, _P, _I, _P]
         o.distie_large_tiles_rotary_bf16.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]
@@ -1029,7 +1037,8 @@ class HipOps(Ops):
         shape, slices, us = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0)
         if self._ops.distie_large_tiles_plan(M, N, K, self.LARGE_KINDS[kind], cut_us is not None, cut_us or 0.0,
                                              ctypes.byref(shape), ctypes.byref(slices), ctypes.byref(us)) and \
-                self._large_take(M, N, K, kind, cut_us, us.value):
+                self._large_take(M, N, K, kind, cut_us, us.value) and \
+                not self._large_idle(M, N, K, kind, cut_us, shape.value, slices.value):
             return shape.value, slices.value
         return None
 
@@ -1059,6 +1068,16 @@ class HipOps(Ops):
             return rate >= (self.LARGE_LONG_RATE if M <= self.TILES_LONG_ROWS else self.LARGE_LONG_RATE_BEYOND)
         return rate >= (self.LARGE_SHORT_RATE if elements > self.ROW_GROUPS_MAX_ELEMENTS or N < self.TILES_FEW_WEIGHT_ROWS else
                         self.LARGE_SHORT_RATE_SMALL)
+
+    def _large_idle(self, M, N, K, kind, cut_us, shape, slices) -> bool:
+        """Whether these tiles leave half of the compute units or more without one where other kernels do not: see LARGE_IDLE_K."""
+        if kind == "rotary" or M <= self.LARGE_FEW_ROWS:
+            return False
+        rows, columns = ctypes.c_int(0), ctypes.c_int(0)
+        _check(self._ops.distie_large_tiles_grid(M, N, shape, ctypes.byref(rows), ctypes.byref(columns)), "large_tiles_grid")
+        busy = columns.value * slices
+        return rows.value == 1 and (4 * busy <= self._compute_units or (2 * busy <= self._compute_units and K > self.LARGE_IDLE_K)) and \
+            (M > self._packed_rows(M, N, K) or self._tiles(M, N, K, kind, cut_us) is not None)
 
     def _large_each(self, M, N, K, xs):
         """The tile of the kernels for many rows for several products that share a launch, N columns in all, or None."""

@@ -258,7 +258,7 @@ def test_gated_products_in_large_tiles_leave_no_rows_out(rules, rows, weight):
     assert rules._large(rows, *weight, "gated", ()) is not None
 
 
-def test_products_met_before_take_one_look(rules):
+def test_products_met_before_take_one_look(rules, monkeypatch):
     """A step that is launched kernel by kernel asks for every product of every layer: what was found is kept, by what the rules
     read, and an input off 16 bytes has the other kernels each time."""
     rules.captured, rules.library_timed_rows = False, 0
@@ -273,7 +273,26 @@ def test_products_met_before_take_one_look(rules):
     off = [rules._tiled(*a[:4], (data[1:], None), a[4]) for a in asked]
     assert off == [(rules._tiles(*a), False) for a in asked]
     assert rules._tiled(8, 17920, 1536, "gated", (data,)) == (None, False)
-    rules._ops = None                                        # no rule is walked through again
+    monkeypatch.setattr(rules, "_ops", None)                 # no rule is walked through again
     assert [rules._tiled(*a[:4], (data, None), a[4]) for a in asked] == first
     assert [rules._large_each(rows, 4096, 1024, xs) for rows in (33, 300)] == each
     assert len(rules._large_plans) <= rules.TILE_PLANS
+
+
+@pytest.mark.parametrize("kind,rows,weight,takes", [
+    # one row of tiles on half of the compute units or fewer, K long: us in these tiles / what there was
+    ("gated", 88, (13824, 2560), False),           # 27.2 / 24.7
+    ("gated", 128, (16384, 3072), False),          # 33.7 / 32.2
+    ("gated", 192, (16384, 3072), False),          # 40.8 / 35.1
+    ("gated", 200, (16384, 3072), True),           # 32.5 / 42.6: two rows of them
+    ("gated", 88, (20480, 2560), True),            # 29.5 / 34.6: 160 of them
+    ("gated", 128, (8192, 1536), False),           # 18.0 / 13.2: 64 of them
+    ("gated", 144, (12288, 1536), True),           # 16.7 / 22.0: K short
+    ("qkv", 128, (13056, 3072), False),            # 33.0 / 29.0
+    ("qkv", 192, (15232, 3584), False),            # 45.4 / 34.9
+    ("qkv", 256, (15232, 3584), True),             # 40.0 / 48.5
+    ("down", 128, (5120, 20480), True)])           # K cut: 74 / 76
+def test_large_tiles_that_would_leave_units_idle(rules, kind, rows, weight, takes):
+    rules.captured, rules.library_timed_rows = False, 0
+    cut_us = None if kind == "gated" else 0.0 if kind in rules.ADDS_SLICES else rules.SUM_SLICES_US
+    assert (rules._large(rows, *weight, "gated" if kind == "gated" else "plain", (), cut_us) is not None) == takes
