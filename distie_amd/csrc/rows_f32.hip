@@ -306,12 +306,17 @@ void rows_plan(int row_blocks, int K, int* slices, int* steps) {
 // has one workgroup that asks for W and no unit two: as many waves as that takes where K stays whole, or K cut until the workgroups
 // are about as many as the units (twice as many from 17 rows on, where a stage takes longer). Timed with the reader of the slices
 // (us, this way / the other; every weight from memory):
-//  * gated, weights of 24 million elements and more: [8, 1536] x [17920, 1536] 27.1 / 28.6, [4, 1536] 27.0 / 26.1, [32, 1536] 34 / 47;
-//    [8, 2048] x [16384, 2048] 32.8 / 33.5, [32, 2048] 38 / 49; from 96 million on always: [1, 3584] x [37888, 3584] 100 / 119, [8, 3584]
-//    99 / 141, [32, 3584] 113 / 224. Smaller ones are not: [16, 1024] x [8192, 1024] 15.0 / 12.2;
-//  * plain, weights of 12 million elements and more, from eight rows on: [8, 3584] x [3584, 3584] 18.4 / 21.6, [32, 3584] 21.5 / 27.8,
-//    [4, 3584] 18.0 / 18.5; with K at least four times as long always: [1, 18944] x [3584, 18944] 55 / 62, [32, 18944] 66 / 110; [8,
-//    8960] x [1536, 8960] 18.8 / 21.6. Smaller ones are level: [16, 4096] x [1024, 4096] 11.1 / 11.6, [8, 1536] x [1536, 1536] 9.0 / 8.6.
+//  * gated, weights of 24 million elements and more whose blocks of 16 rows make workgroups of four waves on every unit, from 12
+//    rows on, from eight with K of 1,536 and more: [8, 1536] x [17920, 1536] 27.7 / 28.6, [4, 1536] 26.3 / 25.8, [32, 1536] 35 / 46; [16,
+//    2048] x [16384, 2048] 32.9 / 35.0, [8, 2048] 33.0 / 31.3; [16, 1024] x [24576, 1024] 27.0 / 28.2, [8, 1024] 27.3 / 25.4. From 96 million on
+//    always: [1, 3584] x [37888, 3584] 100 / 124, [8, 3584] 99 / 139, [32, 3584] 114 / 223. With fewer blocks units are idle, or three
+//    waves have too little under way: [8, 4096] x [8192, 4096] 48 / 30, [8, 8192] x [4096, 8192] 87 / 33, [8, 3072] x [12288, 3072] 41 / 34.
+//    Smaller weights are not: [16, 1024] x [8192, 1024] 15.0 / 12.2;
+//  * plain, weights of 12 million elements and more, from eight rows on: [8, 3584] x [3584, 3584] 18.8 / 21.7, [32, 3584] 21.8 / 27.7,
+//    [4, 3584] 20.9 / 20.8; up to 15 rows not where every unit would have one: some then get two, others none ([8, 4096] x [4096, 4096]
+//    24.0 / 22.3, [8, 2048] x [8192, 2048] 25.4 / 23.8, [8, 11008] x [4096, 11008] 50 / 45; [8, 5120] x [5120, 5120], 240 workgroups, 28 / 34).
+//    With K at least four times as long always: [1, 8960] x [1536, 8960] 18.6 / 20.3, [8, 18944] x [3584, 18944] 58 / 68, [32, 18944] 63 /
+//    109. Smaller ones are level: [16, 4096] x [1024, 4096] 11.1 / 11.6, [8, 1536] x [1536, 1536] 9.0 / 8.6.
 struct RowsTiles {
   int waves, slices;
 };
@@ -319,15 +324,20 @@ RowsTiles rows_tiles(int M, int N, int K, bool gated) {
   const int64_t elements = static_cast<int64_t>(N) * K;
   const int blocks = gated ? (N / 2 + 7) / 8 : (N + 15) / 16, all = K / RF_STEP;
   if (gated) {
-    if (elements < (M < 8 ? int64_t{96} << 20 : int64_t{24} << 20) || blocks > 256 * 10) return {0, 1};
     const int waves = (blocks + 255) / 256;
-    return {waves <= 3 ? 3 : waves <= 5 ? waves : waves <= 7 ? 7 : 10, 1};
+    if (waves < 4 || waves > 10) return {0, 1};
+    if (elements < (int64_t{96} << 20) &&
+        (elements < (int64_t{24} << 20) || M < 8 || (M < 12 && (blocks <= 1024 || K < 1536))))
+      return {0, 1};
+    return {waves <= 5 ? waves : waves <= 7 ? 7 : 10, 1};
   }
   if (elements < (int64_t{12} << 20) || (M < 8 && K < 4 * N)) return {0, 1};
   const int groups = (blocks + 3) / 4;
   const int want = std::max(1, std::min((M <= 16 ? 256 : 512) / groups, all / 4));
   const int steps = (all + want - 1) / want;
-  return {4, (all + steps - 1) / steps};
+  const int slices = (all + steps - 1) / steps;
+  if (M < 16 && K < 4 * N && groups * slices > 240) return {0, 1};
+  return {4, slices};
 }
 
 template <int MODE>
@@ -351,7 +361,6 @@ int launch_rows_tiles(const float* x, const float* w, const float* bias, float* 
     }
   } else {
     switch (tiles.waves) {
-      TILES(3, 4, 4);
       TILES(4, 3, 2);
       TILES(5, 3, 3);
       TILES(7, 3, 2);
@@ -388,6 +397,11 @@ extern "C" int distie_rows_f32_slices(int M, int N, int K, int whole) {
     rows_plan((N + 15) / 16, K, &slices, &steps);
   }
   return slices;
+}
+
+// The waves of a workgroup where such a product goes through LDS, 0 where it does not.
+extern "C" int distie_rows_f32_waves(int M, int N, int K, int gated) {
+  return takes(M, N, K) ? rows_tiles(M, N, K, gated != 0).waves : 0;
 }
 
 // mode 0: y [M, N], or [slices, M, N] if the plan cuts K; 1 | (activation << 8): gated, [M, N / 2] (limit, slope, up_shift:

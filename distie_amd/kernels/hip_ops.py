@@ -448,6 +448,7 @@ class HipOps(Ops):
         o.distie_gemm_generic.argtypes = [_P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _P]
         o.distie_gemv_rows.argtypes = [_P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _P]
         o.distie_rows_f32_slices.argtypes = [_I, _I, _I, _I]
+        o.distie_rows_f32_waves.argtypes = [_I, _I, _I, _I]
         o.distie_rows_f32.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _F, _P]
         o.distie_rows_f32_rotary.argtypes = [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]
         o.distie_gemm_skinny_slices.argtypes = [_I, _I, _I]

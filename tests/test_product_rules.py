@@ -296,3 +296,20 @@ def test_large_tiles_that_would_leave_units_idle(rules, kind, rows, weight, take
     rules.captured, rules.library_timed_rows = False, 0
     cut_us = None if kind == "gated" else 0.0 if kind in rules.ADDS_SLICES else rules.SUM_SLICES_US
     assert (rules._large(rows, *weight, "gated" if kind == "gated" else "plain", (), cut_us) is not None) == takes
+
+
+@pytest.mark.parametrize("gated,rows,weight,through_lds", [
+    # gated: us through LDS / on registers
+    (True, 8, (8192, 4096), False), (True, 32, (8192, 4096), False),          # 48 / 30, 63 / 49: 171 workgroups of three waves
+    (True, 8, (4096, 8192), False), (True, 16, (12288, 3072), False),         # 87 / 33, 41 / 40
+    (True, 8, (16384, 2048), False), (True, 12, (16384, 2048), True),         # 33.0 / 31.3, 33.0 / 34.3
+    (True, 8, (17920, 1536), True), (True, 7, (17920, 1536), False),          # 27.7 / 28.6
+    (True, 8, (24576, 1024), False), (True, 16, (24576, 1024), True),         # 27.3 / 25.4, 27.0 / 28.2
+    (True, 1, (37888, 3584), True), (True, 8, (65536, 1536), False),          # 100 / 124
+    # plain
+    (False, 8, (4096, 4096), False), (False, 16, (4096, 4096), True),         # 24.0 / 22.3, 23.6 / 23.9
+    (False, 8, (4096, 11008), False), (False, 17, (4096, 11008), True),       # 50 / 45, 47 / 54
+    (False, 8, (3584, 3584), True), (False, 8, (5120, 5120), True),           # 18.8 / 21.7, 28 / 34
+    (False, 1, (1536, 8960), True), (False, 33, (1536, 8960), False)])
+def test_float32_products_through_lds(rules, gated, rows, weight, through_lds):
+    assert (rules._ops.distie_rows_f32_waves(rows, *weight, int(gated)) > 0) == through_lds
