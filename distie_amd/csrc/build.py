@@ -44,7 +44,7 @@ MIXED_ATTN_SOURCES = ["mixed_attention_mc.hip"]
 LIBRARY_SOURCES = ["library_products.hip"]
 LINK_LIBS = {"library": ["-lhipblaslt"]}
 HEADERS = ["common.h"]
-OPS_HEADERS = ["no_alloc.h", "packed.h", "vector_values.h"]
+OPS_HEADERS = ["lds_load.h", "no_alloc.h", "packed.h", "vector_values.h"]
 
 
 class BuildError(RuntimeError):

@@ -18,47 +18,17 @@
 // 261). 301 rows: gate+up of the 1.5B shape 25 us, 36 in packed_tiles.
 
 #include "common.h"
+#include "lds_load.h"
 #include "packed.h"
 #include <algorithm>
 
 namespace {
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
-typedef __attribute__((__vector_size__(4 * sizeof(int)))) int intx4;
-typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int LT_K = 64;              // k of a stage of x; W comes in halves of it
 constexpr int LT_EACH = 3;            // a mode beside PK_PLAIN, PK_GATED and PK_ROTARY
 constexpr int LT_EACH_MAX = 8;
-
-// A buffer of `bytes` from `base` on (both the same in all lanes): reads beyond it give zeros.
-__device__ __forceinline__ intx4 buffer_of(const void* base, uint32_t bytes) {
-  const uint64_t at = reinterpret_cast<uint64_t>(base);
-  intx4 d;
-  d[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(at));
-  d[1] = __builtin_amdgcn_readfirstlane(static_cast<int>(at >> 32) & 0xffff);
-  d[2] = __builtin_amdgcn_readfirstlane(static_cast<int>(bytes));
-  d[3] = 0x00020000;
-  return d;
-}
-
-// Sixteen bytes a lane from `from` + lane_at + wave_at into LDS, the lanes' pieces one behind the other from `to` on. The wait
-// is the caller's. The s_nop is the wait state between writing m0 and the load.
-__device__ __forceinline__ void buffer_to_lds(const intx4& from, int lane_at, int wave_at, uint32_t to) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(lane_at), "s"(from),
-               "s"(wave_at)
-               : "m0");
-}
-
-// All but the newest LEFT loads into LDS of this wave have arrived and what it read from LDS is in its registers; then the
-// same for all waves.
-template <int LEFT>
-__device__ __forceinline__ void arrived() {
-  static_assert(LEFT < 64, "the counter's range");
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT) : "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // g sigmoid(z), as g / (1 + expf(-z)) and to the same error: 0.67 units of 2^-24 in the mean and 3 at most, over |z| up to 88. The
 // quotient is the unit's reciprocal and one correction, a quarter of 1 + expf(-z) because the unit flushes a reciprocal below
@@ -126,7 +96,7 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
   }
 #pragma unroll
   for (int p = 0; p < W_LOADS; ++p) w_lane[p] = min(wave * W_LOADS + p, blocks - 1) * k_tiles * 1024 + lane * 16;
-  const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds)));
+  const uint32_t base = lds_place(lds);
   auto bring_x = [&](int stage, int slot, int p) {
     buffer_to_lds(x_buffer, x_lane[p], (s_begin + min(stage, stages - 1)) * (LT_K * 2),
                   base + slot * X_BYTES + (wave * X_LOADS + p) * 1024);
@@ -195,7 +165,7 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
       if (part > 0 && part < 2 * D - 1 && (part % 2 == 1) == (p < XA)) bring_x((part + 1) / 2, (part + 1) / 2, p);
   }
   constexpr int STAGE = 2 * W_LOADS + X_LOADS;
-  arrived<(D - 1) * STAGE + W_LOADS>();
+  lds_arrived<(D - 1) * STAGE + W_LOADS>();
 #pragma unroll
   for (int i = 0; i < TM + TN; ++i) read(0, 0, 0, 0, i);
   // Iteration s holds x(s) and W's parts 2 s and 2 s + 1. The loads in order: x(0), W(0); then, for every stage, W(2 s - 1), the
@@ -205,14 +175,14 @@ __global__ __launch_bounds__(64 * WAVES, TM * TN > 8 ? 1 : 2) void large_tiles_k
   for (int s = 0; s < stages; ++s) {
     const int next = slot == D ? 0 : slot + 1, free = slot == 0 ? D : slot - 1, w_next = w_slot == 2 * D - 2 ? 0 : w_slot + 2;
     multiply(0, 1, slot, w_slot, XA, [&](int q) { bring_x(s + D, free, q); });
-    arrived<(D - 1) * STAGE + XA>();
+    lds_arrived<(D - 1) * STAGE + XA>();
     multiply(1, 2, slot, w_slot + 1, W_LOADS, [&](int q) { bring_w(2 * (s + D), w_slot, q); });
     multiply(0, 3, slot, w_slot + 1, XB, [&](int q) { bring_x(s + D, free, XA + q); });
-    arrived<(D - 1) * STAGE>();
+    lds_arrived<(D - 1) * STAGE>();
     multiply(1, 0, next, w_next, W_LOADS, [&](int q) { bring_w(2 * (s + D) + 1, w_slot + 1, q); });
     slot = next, w_slot = w_next;
   }
-  arrived<0>();
+  lds_arrived<0>();
 
   // The results of 32 rows of x and up to 128 bytes of columns at a time go through LDS, so that rows leave in whole lines.
   constexpr int EACH = MODE == PK_GATED ? 16 : 32;                                  // columns of y that 32 rows of W give

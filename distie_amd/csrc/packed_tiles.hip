@@ -15,6 +15,7 @@
 // changed nothing or lost up to a fifth.
 
 #include "common.h"
+#include "lds_load.h"
 #include "packed.h"
 #include <algorithm>
 
@@ -22,20 +23,10 @@ namespace {
 
 constexpr int PT_K = 64;              // k of a stage
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-// Sixteen bytes a lane from memory into LDS, the lanes' pieces one behind the other from `to` on (the same in all lanes).
-// The wait is the caller's: `stage_ready`. An instruction of its own because the compiler, which knows of such a load,
-// waits for all of them before any read of LDS. The s_nop is the wait state between writing m0 and the load.
-__device__ __forceinline__ void load_to_lds(const bf16_t* from, bf16_t* to) {
-  const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)to)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from) : "memory", "m0");
-}
-
-// What this wave asked for has arrived and what it read from LDS is in its registers; then the same for all waves.
-__device__ __forceinline__ void stage_ready() {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
+// As `load_to_lds`, in its place among the reads and writes of memory around it (they stand in the order written).
+__device__ __forceinline__ void stage_to_lds(const bf16_t* from, bf16_t* to) {
+  asm volatile("" ::: "memory");
+  load_to_lds(from, lds_place(to));
   asm volatile("" ::: "memory");
 }
 
@@ -104,21 +95,21 @@ __global__ __launch_bounds__(256, 2) void packed_tiles_kernel(const bf16_t* __re
   if constexpr (DEPTH == 2) {
     auto fetch = [&](int stage, int half) {
 #pragma unroll
-      for (int p = 0; p < PARTS; ++p) load_to_lds(xp[p] + PT_K * stage, &xs[half][(32 * p + 8 * wave) * PT_K]);
+      for (int p = 0; p < PARTS; ++p) stage_to_lds(xp[p] + PT_K * stage, &xs[half][(32 * p + 8 * wave) * PT_K]);
       fetch_w(stage, half);
       __builtin_amdgcn_sched_barrier(0);         // (else the compiler asks late for what the next stage needs)
     };
     fetch(0, 0);
     int s = 0;
     for (; s + 2 <= stages; s += 2) {
-      stage_ready();
+      lds_arrived<0>();
       fetch(s + 1, 1);
       multiply(0, 0);
-      stage_ready();
+      lds_arrived<0>();
       fetch(min(s + 2, stages - 1), 0);          // (past the last stage: the last once more, not used)
       multiply(1, 1);
     }
-    stage_ready();                               // nothing is under way when the workgroup ends
+    lds_arrived<0>();                               // nothing is under way when the workgroup ends
     if (s < stages) multiply(0, 0);
   } else {
     bf16x8 xr[DEPTH][PARTS];

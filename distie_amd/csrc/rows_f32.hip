@@ -18,6 +18,7 @@
 // sums' chains no longer fit the registers at the precision of the vector ALU's kernel.
 
 #include "common.h"
+#include "lds_load.h"
 #include "packed.h"
 #include <algorithm>
 
@@ -169,24 +170,6 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_kernel(const float* __res
 
 // ---- the same through LDS
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-// Sixteen bytes a lane from memory into LDS, the lanes' pieces one behind the other from `to` on. The wait is the caller's. The
-// s_nop is the wait state between writing m0 and the load.
-__device__ __forceinline__ void row_to_lds(const float* from, uint32_t to) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "m0");
-}
-
-// All but the newest LEFT loads into LDS of this wave have arrived and what it read from LDS is in its registers; then the
-// same for all waves.
-template <int LEFT>
-__device__ __forceinline__ void arrived() {
-  static_assert(LEFT < 64, "the counter's range");
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT) : "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // A workgroup owns 16 WAVES rows of W (16 a wave), 16 MB rows of x and a slice of K. Stages of 64 k, whole lines
 // of W and x, go straight from memory into LDS, DEPTH of them under way. The products of a stage start 16 / MB sums each, which
 // are added in pairs; four totals take the stages in turn, so that the result is no further from 64 bits than the other kernel's
@@ -223,14 +206,14 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_tiles_kernel(const float*
     }
     w_lane[p] = w + of * K + 4 * ((lane % 16) ^ i);
   }
-  const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds)));
+  const uint32_t base = lds_place(lds);
   auto bring = [&](int step, int slot) {                       // (past the last step: it once more, so that the count stays)
     const int k = RF_STEP * (s_begin + min(step, steps - 1));
     const uint32_t to = base + slot * SLOT;
 #pragma unroll
-    for (int p = 0; p < X_LOADS; ++p) row_to_lds(x_lane[p] + k, to + (wave * X_LOADS + p) % (4 * MB) * 1024);
+    for (int p = 0; p < X_LOADS; ++p) load_to_lds(x_lane[p] + k, to + (wave * X_LOADS + p) % (4 * MB) * 1024);
 #pragma unroll
-    for (int p = 0; p < 4; ++p) row_to_lds(w_lane[p] + k, to + X_BYTES + (wave * 4 + p) * 1024);
+    for (int p = 0; p < 4; ++p) load_to_lds(w_lane[p] + k, to + X_BYTES + (wave * 4 + p) * 1024);
   };
   floatx4 total[4][MB];
 #pragma unroll
@@ -241,7 +224,7 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_tiles_kernel(const float*
   for (int s = 0; s < DEPTH; ++s) bring(s, s);
   int slot = 0, s = 0;
   auto step = [&](int turn) {
-    arrived<(DEPTH - 1) * LOADS>();
+    lds_arrived<(DEPTH - 1) * LOADS>();
     bring(s + DEPTH, slot == 0 ? DEPTH : slot - 1);
     const char* from = lds + slot * SLOT;
     floatx4 b[MB][4];
@@ -285,7 +268,7 @@ __global__ __launch_bounds__(64 * WAVES) void rows_f32_tiles_kernel(const float*
   if (s < steps) step(0);
   if (s < steps) step(1);
   if (s < steps) step(2);
-  arrived<0>();                                                // nothing is under way when the workgroup ends
+  lds_arrived<0>();                                                // nothing is under way when the workgroup ends
 #pragma unroll
   for (int m = 0; m < MB; ++m) {
     const floatx4 acc = (total[0][m] + total[1][m]) + (total[2][m] + total[3][m]);
