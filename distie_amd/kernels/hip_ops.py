@@ -297,8 +297,10 @@ class HipOps(Ops):
     #    [2048, 1536] with rotation 79 / 58). Steps, us, with this line / without: 1.5B shape, 8,000 tokens 28,040 / 28,690; 7B shape,
     #    4,096 tokens 49,220 / 50,600. The gated ones win at 8,192 rows, too ([8192, 1536] x [17920, 1536] 386 / 446);
     #  * other plain ones from LARGE_PLAIN_RATE on ([1024, 2048] x [2048, 2048] 17 / 15, [1152, 2048] 17 / 20), weights of four times as
-    #    many rows as K from LARGE_WIDE_RATE on ([400, 1024] x [4352, 1024] 11 / 10, [450, 1024] 10 / 12), up to LARGE_DENSE_WORK
-    #    products, from where the library is the faster one ([900, 2048] x [8448, 2048] 36 / 40, [1024, 2048] 42 / 39, [2048, 2048] 76 / 66).
+    #    many rows as K from LARGE_WIDE_RATE on ([352, 1280] x [5440, 1280] 15.5 / 14.2, [416, 1280] 14.3 / 14.8; [256, 1536] x [6528, 1536]
+    #    17.5 / 13.6, [416, 1536] 16.3 / 16.7; [160, 2560] x [10880, 2560] 25 / 23, [176, 2560] 24 / 39), with K of up to LARGE_WIDE_SHORT_K
+    #    from LARGE_WIDE_SHORT_RATE on ([400, 1024] x [4352, 1024] 11 / 10, [480, 1024] 11 / 12; [720, 768] x [3264, 768] 9.1 / 10.7), up to
+    #    LARGE_DENSE_WORK products, from where the library is the faster one ([900, 2048] x [8448, 2048] 36 / 40, [1024, 2048] 42 / 39, [2048, 2048] 76 / 66).
     # A single row of tiles (65 to 192 rows), half of the compute units or fewer with one: such a tile takes 0.5 us and more for every
     # 64 k, however idle the rest is, and the smaller tiles and passes of before, which spread over more units, are ahead where K is
     # long: beyond LARGE_IDLE_K ([88, 2560] x [13824, 2560] 27 / 25, [160, 3072] x [16384, 3072] 39 / 35; plain [128, 3072] x [13056,
@@ -341,7 +343,9 @@ class HipOps(Ops):
     LARGE_SHORT_RATE = 316.0
     LARGE_SHORT_RATE_SMALL = 440.0
     LARGE_PLAIN_RATE = 480.0
-    LARGE_WIDE_RATE = 350.0
+    LARGE_WIDE_RATE = 390.0
+    LARGE_WIDE_SHORT_RATE = 350.0
+    LARGE_WIDE_SHORT_K = 1024
     LARGE_DENSE_WORK = 1.65e10
     # What a cut product costs beyond its slices where the reader of the result cannot add them itself (the readers of a
     # layer's output projections can)
@@ -1062,7 +1066,9 @@ class HipOps(Ops):
                 not many and M * elements <= self.LARGE_ROTARY_WORK and \
                 (M >= self.LARGE_ROTARY_ROWS or elements <= self.TILES_LARGE_ROTARY)
         if cut_us != 0.0:
-            return rate >= (self.LARGE_WIDE_RATE if N >= 4 * K else self.LARGE_PLAIN_RATE) and M * elements <= self.LARGE_DENSE_WORK
+            least = self.LARGE_PLAIN_RATE if N < 4 * K else \
+                self.LARGE_WIDE_SHORT_RATE if K <= self.LARGE_WIDE_SHORT_K else self.LARGE_WIDE_RATE
+            return rate >= least and M * elements <= self.LARGE_DENSE_WORK
         if many:
             return False
         if K >= 2 * N:

@@ -313,3 +313,15 @@ def test_large_tiles_that_would_leave_units_idle(rules, kind, rows, weight, take
     (False, 1, (1536, 8960), True), (False, 33, (1536, 8960), False)])
 def test_float32_products_through_lds(rules, gated, rows, weight, through_lds):
     assert (rules._ops.distie_rows_f32_waves(rows, *weight, int(gated)) > 0) == through_lds
+
+
+@pytest.mark.parametrize("rows,weight,takes", [
+    # us in large tiles / what there was
+    (256, (6528, 1536), False), (301, (6528, 1536), False), (416, (6528, 1536), True),           # 17.5 / 13.6, 15.8 / 13.4, 16.3 / 16.7
+    (192, (8704, 2048), False), (256, (8704, 2048), True),                                       # 20.4 / 17.6, 21.8 / 26.8
+    (352, (5440, 1280), False), (416, (5440, 1280), True),                                       # 15.5 / 14.2, 14.3 / 14.8
+    (160, (10880, 2560), False), (176, (10880, 2560), True),                                     # 25.3 / 22.9, 24.4 / 38.6
+    (480, (4352, 1024), True), (720, (3264, 768), True)])                                        # 11.0 / 12.1, 9.1 / 10.7
+def test_wide_weights_in_large_tiles(rules, rows, weight, takes):
+    rules.captured, rules.library_timed_rows = False, 0
+    assert (rules._large(rows, *weight, "plain", (), rules.SUM_SLICES_US) is not None) == takes
