@@ -279,12 +279,14 @@ class HipOps(Ops):
     #  * gated: from LARGE_GATED_RATE on ([65, 1536] x [17920, 1536] 17 / 22, [301, 1536] 25 / 36, [2048, 1536] 104 / 129; [2048,
     #    3584] x [37888, 3584] 447 / 570, [65, 3584] 52 / 72; [128, 1024] x [8192, 1024] 9.5 / 9.2, [160, 1024] 10 / 12);
     #  * with rotation and cache write in the epilogue: beyond one round of the 64 x 64 tiles of `packed_tiles` ([512, 1536] x
-    #    [2048, 1536] 17 / 12, [576, 1536] 17 / 18, [1152, 1536] 19 / 26, [2048, 1536] 26 / 24), for large weights, whose 64 x 128
-    #    tiles are two thirds as long as these, LARGE_ROTARY_ROWS ([352, 3584] x [4608, 3584] 34 / 30, [450, 3584] 33 / 36, [1664,
-    #    3584] 60 / 61), up to LARGE_ROTARY_WORK products (alone [2048, 3584] takes 76 / 70, but a serving step of 2,025 tokens of the
-    #    7B shape 24.07 ms / 24.15: the library's kernel and the one behind it, 72 + 18 us there, suffer more from the clock that
-    #    the products around them leave; [1024, 4096] x [6144, 4096] 58 / 61, [2304, 4096] 136 / 106; [672, 5120] x [7168, 5120] 60 /
-    #    69, [2048, 5120] 166 / 143);
+    #    [2048, 1536] 17 / 12, [576, 1536] 17 / 18, [1152, 1536] 19 / 25, [2048, 1536] 24 / 26; [416, 2048] x [3072, 2048] 20 / 20, [512,
+    #    2048] x [2560, 2048] 23 / 21), with K beyond LARGE_ROTARY_SHORT_K one of their 64 x 128 tiles ([352, 3072] x [4096, 3072] 32 / 25,
+    #    [512, 3072] 33 / 29, [576, 3072] 31 / 33; [512, 2560] x [3328, 2560] 30 / 27, [640, 2560] 30 / 31), for large weights
+    #    LARGE_ROTARY_ROWS ([480, 3584] x [4608, 3584] 37 / 36, [800, 3584] 38 / 45, [1280, 3584] 50 / 54), up to LARGE_ROTARY_WORK
+    #    products: alone [1802, 3584] takes 66 / 70 and [2048, 3584] 78 / 71, but in a serving step of 2,025 tokens of the 7B shape the
+    #    kernel here takes 78 us a layer and the library's with the one behind it 68 + 17: they suffer more from the clock that the
+    #    products around them leave (the whole step 24.07 ms / 24.15, runs differ by as much); [1024, 4096] x [6144, 4096] 58 / 61,
+    #    [2304, 4096] 136 / 106; [672, 5120] x [7168, 5120] 60 / 69, [2048, 5120] 166 / 143. [4096, 1536] x [2048, 1536] 40 / 40;
     #  * plain, for readers that add the slices of K: K at least twice as long as the weight has rows from LARGE_LONG_RATE on
     #    ([512, 8960] x [1536, 8960] 34 / 31, [576, 8960] 30 / 33, [2048, 8960] 66 / 83; [193, 18944] x [3584, 18944] 48 / 58, [2048,
     #    18944] 271 / 300), and past TILES_LONG_ROWS, where `packed_tiles` ends, LARGE_LONG_RATE_BEYOND ([1024, 4096] x [1024,
@@ -334,6 +336,7 @@ class HipOps(Ops):
     LARGE_GATED_RATE = 240.0
     LARGE_ROTARY_RATE = 150.0
     LARGE_ROTARY_ROWS = 416
+    LARGE_ROTARY_SHORT_K = 2048
     LARGE_ROTARY_WORK = 4e10
     LARGE_ROWS = 2304
     LARGE_MAX_ROWS = 4096
@@ -1063,6 +1066,7 @@ class HipOps(Ops):
             return rate >= self.LARGE_GATED_RATE
         if kind == "rotary":
             return -(-M // 64) * -(-N // 64) > self._compute_units and rate >= self.LARGE_ROTARY_RATE and \
+                (K <= self.LARGE_ROTARY_SHORT_K or -(-M // 64) * -(-N // 128) > self._compute_units) and \
                 not many and M * elements <= self.LARGE_ROTARY_WORK and \
                 (M >= self.LARGE_ROTARY_ROWS or elements <= self.TILES_LARGE_ROTARY)
         if cut_us != 0.0:

@@ -325,3 +325,14 @@ def test_float32_products_through_lds(rules, gated, rows, weight, through_lds):
 def test_wide_weights_in_large_tiles(rules, rows, weight, takes):
     rules.captured, rules.library_timed_rows = False, 0
     assert (rules._large(rows, *weight, "plain", (), rules.SUM_SLICES_US) is not None) == takes
+
+
+@pytest.mark.parametrize("rows,weight,takes", [
+    # us in large tiles / what there was
+    (352, (4096, 3072), False), (512, (4096, 3072), False), (576, (4096, 3072), True),           # 31.9 / 24.8, 33.3 / 28.9, 31.2 / 33.3
+    (512, (3328, 2560), False), (640, (3328, 2560), True),                                       # 30.4 / 26.6, 30.3 / 31.2
+    (416, (4608, 3584), False), (800, (4608, 3584), True),                                       # 35.0 / 31.7, 37.8 / 44.5
+    (576, (2048, 1536), True), (416, (3072, 2048), True)])                                       # 17.0 / 17.8, 20 / 20
+def test_long_rotating_products_in_large_tiles(rules, rows, weight, takes):
+    rules.captured, rules.library_timed_rows = False, 0
+    assert (rules._large(rows, *weight, "rotary", ()) is not None) == takes
