@@ -1,5 +1,5 @@
-// Products of many rows (portions of prompts, prompts of a few hundred tokens) on packed weight copies: y[M, N] = x[M, K]
-// W[N, K]^T for bfloat16 x and the copies of packed.h, with the activation, or rotation and cache write, in the epilogue.
+// Products of 9 rows and more (batches of decoding requests, prompts and portions of them) on packed weight copies: y[M, N] =
+// x[M, K] W[N, K]^T for bfloat16 x and the copies of packed.h, with the activation, or rotation and cache write, in the epilogue.
 //
 // A workgroup of four or two waves owns a tile of rows of x and rows of W and one slice of K; a wave owns 32 TM x 32 TN of it as
 // TM x TN products of 32 x 32 x 16, whose sums stay in the accumulation registers. x and W both go straight from memory into LDS:
@@ -8,14 +8,14 @@
 // LDS and loads stand between the matrix instructions of the 16 k before.
 //
 // What bounds it. [4096, 4096] x [4096, 4096] takes 110 us (1,244 TFLOP/s; the library 98): the matrix cores are 90 % busy and the
-// chip's power holds the clock at 1.45 GHz, whatever the loop does (eight waves of 128 x 64, which read half as much again from
-// LDS, take 2,570 to 2,940 cycles a stage instead of 2,270 and the same 124 us at 1.58 to 1.81 GHz). That is why a wave owns as
-// much as it can hold. Smaller tiles run into the L2, which gives the chip's LDS 15 to 17 TB/s: 128 x 128 need 32 KB for 512
+// chip's power holds the clock at 1.45 GHz, 2,270 cycles a stage, 100 us for the loop. Eight waves of 128 x 64, which read half as
+// much again from LDS, needed 2,530 to 2,940 cycles at 1.58 to 1.81 GHz, 102 to 104 us whatever the cycles. That is why a wave
+// owns as much as it can hold. Smaller tiles run into the L2, which gives the chip's LDS 15 to 17 TB/s: 128 x 128 need 32 KB for 512
 // cycles of products (fragments of a whole stage read ahead changed nothing). With few rows it is the weight from memory: 64 rows
-// of the 1.5B shape's gate+up 15.1 us (3.6 TB/s; 20.2 in packed_tiles), of the 7B shape's 52 (5.2 TB/s; 66 in passes).
-// 1.5B shape, 2,048 rows, isolated and with the kernel that the library needs behind its own: gate+up with its activation 104 us
-// (129), down in four slices 54 (80; the norm reads 12 us more). 7B shape, 2,025 rows: 460 (567) and 220 (359; packed_tiles
-// 261). 301 rows: gate+up of the 1.5B shape 25 us, 36 in packed_tiles.
+// of the 1.5B shape's gate+up 15.5 us (3.6 TB/s; 20.5 in packed_tiles), of the 7B shape's 53 (5.1 TB/s; 66 in passes).
+// 1.5B shape, 2,048 rows, isolated and with the kernel that the library needs behind its own: gate+up with its activation 111 us
+// (129), down in four slices 54 (80; the norm reads 12 us more). 7B shape, 2,048 rows: 451 (570) and 220 (359; packed_tiles
+// 261). 301 rows: gate+up of the 1.5B shape 27 us, 35 in packed_tiles.
 
 #include "common.h"
 #include "lds_load.h"
@@ -331,8 +331,9 @@ struct LargePlan {
 
 // How a product is cut, as plan_tiles: whole rounds of workgroups on the compute units, the last of them with as many as are
 // left, no faster than memory brings W, and what the reader of the result moves. The numbers are a least-squares fit to 16,000
-// timings (25 weights of 0.9 to 136 million elements, 65 to 2,048 rows, in a captured graph; the fit is off by 6 %). What the
-// count chooses takes 2.8 % more than the best of them on average.
+// timings (25 weights of 0.9 to 136 million elements, 65 to 2,048 rows, in a captured graph; it is off by 6 %), but for two that
+// it could not tell: what a second workgroup costs a unit, and the rate of W from memory where rows are few, 5.2 TB/s. What the
+// count chooses takes 1.6 % more than the best of them on average, a tenth and more in 24 cases of 655.
 LargePlan plan_large(int M, int N, int K, int row_blocks, int mode, bool may_cut, float cut_us) {
   LargePlan best = {-1, 0, 0.f};
   const int all = K / LT_K;

@@ -236,7 +236,8 @@ class HipOps(Ops):
     #  * K cut beyond TILES_LONG_ROWS, for the large weights of a portion of a prompt (TILES_PORTION_ELEMENTS) as far as they were
     #    measured, against the library's first choice: [2048, 18944] x [3584, 18944] 296 / 382, 268; [1600, 27648] x
     #    [5120, 27648] 571 / 681, 416; not [1800, 27648] 560 / 455, 470 nor [1400, 11008] x [4096, 11008] 160 / 149, 148. An engine
-    #    that timed the library's kernels for a portion of these rows stays with them;
+    #    that timed the library's kernels for a portion of these rows stays with them. (`large_tiles` has taken over what begins at
+    #    multiples of 16 bytes; this is for the rest;)
     #  * gated products, which save the activation's kernel: [64, 1536] x [17920, 1536] 20 / 22; [192, 1536] 28 / 30, 29; [301,
     #    1536] 34 / 34, 35; [193, 2048] x [16384, 2048] 32 / 31, 32: up to TILES_MAX_GATED_WORK, and where the host bounds the step,
     #    or one pass of 96 rows is what there is, as far as they are level, TILES_LEVEL_GATED_WORK. Weights of up to
@@ -276,8 +277,9 @@ class HipOps(Ops):
     # (`_large_take`). Which is told by the rate, in TFLOP/s, that the count behind their plan comes to; measured on 25 weights of
     # 0.9 to 136 million elements and 27 row counts, in a captured graph, with the kernels that read the result (us, these tiles /
     # what there was, `packed_tiles` or the library's first choice with the kernels behind it):
-    #  * gated: from LARGE_GATED_RATE on ([65, 1536] x [17920, 1536] 17 / 22, [301, 1536] 25 / 36, [2048, 1536] 104 / 129; [2048,
-    #    3584] x [37888, 3584] 447 / 570, [65, 3584] 52 / 72; [128, 1024] x [8192, 1024] 9.5 / 9.2, [160, 1024] 10 / 12);
+    #  * gated: from LARGE_GATED_RATE on ([65, 1536] x [17920, 1536] 19 / 22, [301, 1536] 27 / 35, [2048, 1536] 111 / 128; [2048,
+    #    3584] x [37888, 3584] 451 / 570, [72, 3584] 56 / 74; [160, 1024] x [8192, 1024] 12 / 13, [2048, 1024] 37 / 44), with gelu, squares
+    #    or max(z, 0) on the gate as well (gelu [2048, 1024] x [8192, 1024] 39 / 46, [1802, 2048] x [16384, 2048] 122 / 124);
     #  * with rotation and cache write in the epilogue: beyond one round of the 64 x 64 tiles of `packed_tiles` ([512, 1536] x
     #    [2048, 1536] 17 / 12, [576, 1536] 17 / 18, [1152, 1536] 19 / 25, [2048, 1536] 24 / 26; [416, 2048] x [3072, 2048] 20 / 20, [512,
     #    2048] x [2560, 2048] 23 / 21), with K beyond LARGE_ROTARY_SHORT_K one of their 64 x 128 tiles ([352, 3072] x [4096, 3072] 32 / 25,
@@ -313,14 +315,15 @@ class HipOps(Ops):
     # Up to LARGE_FEW_ROWS rows the kernel takes smaller tiles, and no count stands behind their plan (28 weights, 1 to 64 rows; what
     # there was are the passes over the packed copy and `packed_tiles`):
     #  * gated: from LARGE_FEW_GATED_ROWS rows on, weights of less than LARGE_FEW_GATED_ELEMENTS from LARGE_FEW_CUT_ROWS on ([8, 1536]
-    #    x [17920, 1536] 12.5 / 13.0, [9, 1536] 12.4 / 14.2, [32, 1536] 13.5 / 16.0, [64, 1536] 15.1 / 20.2; [16, 2048] x [16384, 2048]
-    #    14.3 / 15.3; [64, 3584] x [37888, 3584] 52 / 66; [9, 512] x [4096, 512] 4.6 / 4.4, [20, 512] 4.6 / 5.3);
+    #    x [17920, 1536] 12.5 / 13.0, [9, 1536] 13.4 / 14.7, [32, 1536] 13.6 / 16.0, [64, 1536] 15.5 / 20.5; [16, 2048] x [16384, 2048]
+    #    15.1 / 16.0; [64, 3584] x [37888, 3584] 53 / 66; [16, 1024] x [8192, 1024] 7.0 / 6.9, [17, 1024] 7.1 / 7.5; [9, 512] x [4096, 512]
+    #    4.6 / 4.4, [20, 512] 4.6 / 5.3);
     #  * plain, for readers that add slices: LARGE_FEW_CUT_ROWS rows of large weights ([16, 3584] x [3584, 3584] 12.5 / 12.3, [20,
     #    3584] 12.7 / 13.2, [64, 3584] 14.4 / 16.1; [32, 8192] x [2048, 8192] 13.0 / 15.2; [64, 11008] x [4096, 11008] 25 / 37; [24,
     #    8960] x [1536, 8960] 13.0 / 13.0; [64, 2048] x [2048, 2048] 9.6 / 9.3);
     #  * the heads of large vocabularies, LARGE_FEW_HEAD_ELEMENTS, from LARGE_FEW_CUT_ROWS rows on ([16, 1536] x [151936, 1536] 88 /
-    #    89, [20, 1536] 86 / 91, [64, 1536] 101 / 118; [32, 3584] x [152064, 3584] 201 / 217; [32, 2048] x [32768, 2048] 26.5 / 27.5 and
-    #    [64, 2048] 27.5 / 27.4).
+    #    89, [20, 1536] 92 / 93, [64, 1536] 99 / 116; [24, 3584] x [151936, 3584] 197 / 206; of [152064, 3584] in a decoding step 199 / 212,
+    #    behind 2,025 rows of prompts 206 / 216; [32, 2048] x [32768, 2048] 26.5 / 27.5 and [64, 2048] 27.5 / 27.4).
     LARGE_FEW_ROWS = 64
     LARGE_FEW_GATED_ROWS = 9
     LARGE_FEW_GATED_ELEMENTS = 8 << 20
@@ -384,9 +387,9 @@ class HipOps(Ops):
     def __init__(self, device="cuda:0", packed_weights=True) -> None:
         """`packed_weights` (True, False, or the roles that get one, as the parts name them in
         `prepare_linear`: "qkv", "attn_out", "gate_up", "down", "head"): keep a second copy of every bfloat16 weight in the order in which the
-        matrix cores take it, for products with at most `PACKED_MAX_ROWS_EAGER` rows (decode, short portions). It doubles
-        the memory of the weights and makes those products 15-25 % faster, and it is what the fused
-        epilogues (activation, rotation and cache write) work on; without it products of up to
+        matrix cores take it, for the products that run in passes over the weight or in tiles: decode, portions of prompts, and
+        whole ones of thousands of tokens. It doubles the memory of the weights and makes those products 10-25 % faster, and it
+        is what the fused epilogues (activation, rotation and cache write) work on; without it products of up to
         `SKINNY_MAX_ROWS` rows stream the weights as they are stored and larger ones go to the library."""
         self.device = torch.device(device)
         if isinstance(packed_weights, (bool, int)) or packed_weights is None:
@@ -2125,11 +2128,12 @@ class HipOps(Ops):
         _mark_written(state)
         return out
 
-    EACH_MAX_ROWS = 32        # up to so many rows several products with inputs of their own run as one launch
+    EACH_MAX_ROWS = 32        # up to so many rows several products with inputs of their own run in the kernel for few rows
 
     def prepare_linear_each(self, weights):
         """One packed copy for all, kept on the first weight: the weights one behind the other, each rounded up to whole
-        row blocks (the projections of few rows); beside it nothing, as more rows go to the library."""
+        row blocks. Up to EACH_MAX_ROWS rows all products share a launch of the kernel for few rows; of more rows the rounded ones
+        share one of the large tiles, and the library takes the unrounded one and what is beyond LARGE_EACH_WORK."""
         first = weights[0]
         if (self.packed_roles is not None and "qkv" not in self.packed_roles) or not self.packed_weights or \
                 any(w.dtype != torch.bfloat16 or w.dim() != 2 or w.shape[1] != first.shape[1] for w in weights) or \

@@ -182,8 +182,6 @@ def test_sixteen_queries_a_workgroup():
     """The wide form of the prefill kernel (steps of many tokens take it by themselves)."""
     from distie_amd.kernels.hip_ops import HipOps
 
-    from distie_amd.kernels.hip_ops import HipOps
-
     ops = HipOps("cuda:0")
     ops.MIXED_WIDE_TOKENS = 1
     for sizes in (dict(heads=6, kv_heads=3, dim=48, size=40, keep_first=18), dict(heads=16, kv_heads=4, dim=128, size=None)):
