@@ -316,8 +316,8 @@ class HipOps(Ops):
     # there was are the passes over the packed copy and `packed_tiles`):
     #  * gated: from LARGE_FEW_GATED_ROWS rows on, weights of less than LARGE_FEW_GATED_ELEMENTS from LARGE_FEW_CUT_ROWS on ([8, 1536]
     #    x [17920, 1536] 12.5 / 13.0, [9, 1536] 13.4 / 14.7, [32, 1536] 13.6 / 16.0, [64, 1536] 15.5 / 20.5; [16, 2048] x [16384, 2048]
-    #    15.1 / 16.0; [64, 3584] x [37888, 3584] 53 / 66; [16, 1024] x [8192, 1024] 7.0 / 6.9, [17, 1024] 7.1 / 7.5; [9, 512] x [4096, 512]
-    #    4.6 / 4.4, [20, 512] 4.6 / 5.3);
+    #    15.1 / 16.0; [64, 3584] x [37888, 3584] 53 / 66; [12, 1536] x [8192, 1536] 8.4 / 8.6, [12, 1280] x [7168, 1280] 7.6 / 7.2; [16, 1024] x
+    #    [8192, 1024] 7.0 / 6.8, [17, 1024] 7.1 / 7.5; [9, 512] x [4096, 512] 4.6 / 4.4, [20, 512] 4.6 / 5.3);
     #  * plain, for readers that add slices: LARGE_FEW_CUT_ROWS rows of large weights ([16, 3584] x [3584, 3584] 12.5 / 12.3, [20,
     #    3584] 12.7 / 13.2, [64, 3584] 14.4 / 16.1; [32, 8192] x [2048, 8192] 13.0 / 15.2; [64, 11008] x [4096, 11008] 25 / 37; [24,
     #    8960] x [1536, 8960] 13.0 / 13.0; [64, 2048] x [2048, 2048] 9.6 / 9.3);
@@ -326,7 +326,7 @@ class HipOps(Ops):
     #    behind 2,025 rows of prompts 206 / 216; [32, 2048] x [32768, 2048] 26.5 / 27.5 and [64, 2048] 27.5 / 27.4).
     LARGE_FEW_ROWS = 64
     LARGE_FEW_GATED_ROWS = 9
-    LARGE_FEW_GATED_ELEMENTS = 8 << 20
+    LARGE_FEW_GATED_ELEMENTS = 10 << 20
     LARGE_FEW_CUT_ROWS = 17
     LARGE_FEW_LONG_ELEMENTS = 16 << 20
     LARGE_FEW_SHORT_ELEMENTS = 12 << 20

@@ -336,3 +336,13 @@ def test_wide_weights_in_large_tiles(rules, rows, weight, takes):
 def test_long_rotating_products_in_large_tiles(rules, rows, weight, takes):
     rules.captured, rules.library_timed_rows = False, 0
     assert (rules._large(rows, *weight, "rotary", ()) is not None) == takes
+
+
+@pytest.mark.parametrize("rows,weight,takes", [
+    # us in large tiles / what there was
+    (9, (7168, 1280), False), (16, (7168, 1280), False), (17, (7168, 1280), True),               # 7.6 / 7.2, 7.7 / 7.5, 7.8 / 8.2
+    (12, (8192, 1024), False), (17, (8192, 1024), True),                                         # 7.2 / 6.9, 7.1 / 7.5
+    (9, (8192, 1536), True), (9, (10240, 1280), True)])                                          # 8.4 / 8.6, 8.3 / 9.7
+def test_small_gated_weights_in_large_tiles(rules, rows, weight, takes):
+    rules.captured, rules.library_timed_rows = True, 0
+    assert (rules._large(rows, *weight, "gated", ()) is not None) == takes
