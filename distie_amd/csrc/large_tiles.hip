@@ -30,12 +30,24 @@ constexpr int LT_K = 64;              // k of a stage of x; W comes in halves of
 constexpr int LT_EACH = 3;            // a mode beside PK_PLAIN, PK_GATED and PK_ROTARY
 constexpr int LT_EACH_MAX = 8;
 
-// g sigmoid(z), as g / (1 + expf(-z)) and to the same error: 0.67 units of 2^-24 in the mean and 3 at most, over |z| up to 88. The
-// quotient is the unit's reciprocal and one correction, a quarter of 1 + expf(-z) because the unit flushes a reciprocal below
-// 2^-126 to zero; the last instruction has the quotient of infinities and of what is no number. A true division takes longer
-// ([2048, 1536] x [17920, 1536]: 154 us, 111 this way; without the correction and with exp2(-1.4427 z) 104, but off by 65 units).
+// exp(-z) by 2^n 2^f, n whole: log2(e) in two parts, so that f, at most a half, keeps what a rounded product loses (with the
+// contractions that the compiler would make it is off by tens of units at |z| of 30). The bounds on z keep infinities out of the
+// differences and lie beyond those of the result. The same bits as expf, whose own ends of the range take four instructions more.
+__device__ __forceinline__ float minus_exp(float z) {
+#pragma clang fp contract(off)
+  const float s = __builtin_amdgcn_fmed3f(z, -160.f, 160.f), high = -1.44269502162933349609375f * s, n = __builtin_rintf(high);
+  const float low = fmaf(-1.925962991e-8f, s, fmaf(-1.44269502162933349609375f, s, -high));
+  const float whole = high - n, f = whole + low;
+  return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
+}
+
+// g sigmoid(z), as g / (1 + exp(-z)) and to the same error: 0.67 units of 2^-24 in the mean and 3 at most, over |z| up to 88. The
+// quotient is the unit's reciprocal and one correction, a quarter of 1 + exp(-z) because the unit flushes a reciprocal below
+// 2^-126 to zero; the last instruction has the quotient of infinities and of what is no number. expf and a true division take
+// longer ([2048, 1536] x [17920, 1536]: 154 us, with this quotient 113, this way 111; without the correction and with exp2(-1.4427 z)
+// 104, but off by 65 units).
 __device__ __forceinline__ float times_sigmoid(float g, float z) {
-  const float d = fmaf(0.25f, expf(-z), 0.25f), n = 0.25f * g, r = __builtin_amdgcn_rcpf(d), q = n * r;
+  const float d = fmaf(0.25f, minus_exp(z), 0.25f), n = 0.25f * g, r = __builtin_amdgcn_rcpf(d), q = n * r;
   return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);
 }
 
