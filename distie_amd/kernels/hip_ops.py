@@ -288,7 +288,8 @@ class HipOps(Ops):
     #    products: alone [1802, 3584] takes 66 / 70 and [2048, 3584] 78 / 71, but in a serving step of 2,025 tokens of the 7B shape the
     #    kernel here takes 78 us a layer and the library's with the one behind it 68 + 17: they suffer more from the clock that the
     #    products around them leave (the whole step 24.07 ms / 24.15, runs differ by as much); [1024, 4096] x [6144, 4096] 58 / 61,
-    #    [2304, 4096] 136 / 106; [672, 5120] x [7168, 5120] 60 / 69, [2048, 5120] 166 / 143. [4096, 1536] x [2048, 1536] 40 / 40;
+    #    [2304, 4096] 136 / 106; [672, 5120] x [7168, 5120] 60 / 69, [2048, 5120] 166 / 143. Many rows of [2048,
+    #    1536]: 2,304 29 / 31, 3,072 32 / 32, 4,096 40 / 40;
     #  * plain, for readers that add the slices of K: K at least twice as long as the weight has rows from LARGE_LONG_RATE on
     #    ([512, 8960] x [1536, 8960] 34 / 31, [576, 8960] 30 / 33, [2048, 8960] 66 / 83; [193, 18944] x [3584, 18944] 48 / 58, [2048,
     #    18944] 271 / 300), and past TILES_LONG_ROWS, where `packed_tiles` ends, LARGE_LONG_RATE_BEYOND ([1024, 4096] x [1024,
