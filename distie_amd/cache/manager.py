@@ -120,6 +120,7 @@ class CacheManager:
         self.groups: List[CacheGroup] = []
         self._layers: List[LayerCache] = []
         self._state_slabs: List[torch.Tensor] = []
+        self._clear_rows = None               # `clear_rows_with`
         by_need: Dict[PagedTensors, CacheGroup] = {}
         borrowers: List[tuple] = []
         for layer, needs in enumerate(requirements):
@@ -244,6 +245,17 @@ class CacheManager:
         slabs = [t for group in self.groups for t in group.tensors.values()] + self._state_slabs
         return sum(t.numel() * t.element_size() for t in slabs)
 
+    def clear_rows_with(self, ops) -> None:
+        """From now on a slot's state rows are set to zeros by `ops`, all of them together."""
+        self._clear_rows = ops.row_clearer(self._state_slabs) if self._state_slabs else None
+
+    def _clear(self, slot: int) -> None:
+        if self._clear_rows is not None:
+            self._clear_rows(slot)
+            return
+        for slab in self._state_slabs:
+            slab[slot].zero_()
+
     # ------------------------------------------------------------- requests
     def __contains__(self, request_id) -> bool:
         return request_id in self._requests
@@ -262,8 +274,7 @@ class CacheManager:
             (slot,) = self.slots.allocate(1)
         except OutOfBlocks as exc:
             raise OutOfBlocks(f"no free state slot (all {self.num_slots} in use)") from exc
-        for slab in self._state_slabs:
-            slab[slot].zero_()
+        self._clear(slot)
         entry = RequestCache(slot=slot, tables=[[] for _ in self.groups], passed=[0 for _ in self.groups])
         self._requests[request_id] = entry
         return entry
@@ -363,8 +374,7 @@ class CacheManager:
         """Preemption by recompute: every page back, nothing cached, the slot's state zeroed."""
         entry = self._requests[request_id]
         self._give_back_pages(entry)
-        for slab in self._state_slabs:
-            slab[entry.slot].zero_()
+        self._clear(entry.slot)
 
     def release(self, request_id) -> None:
         """The request is over: pages and slot back."""

@@ -559,3 +559,30 @@ extern "C" int distie_scatter_i32(int32_t* table, const int32_t* index, const in
   scatter_i32_kernel<<<(count + 255) / 256, 256, 0, stream>>>(table, index, value, count, size);
   return launch_status();
 }
+
+// ---------------------------------------------------------------- rows of states
+// Row `row` of several tensors becomes zeros, in one launch: a new request's state rows in every layer. A block clears up to
+// CLEAR_BYTES bytes of one tensor's row; `pieces` holds {first byte of the tensor, bytes of a row, first byte of the piece in its
+// row, bytes of the piece}, multiples of four. Bound by its launch: a step with two new requests of a decoder with 16 such tensors
+// (9 MB) made 32 fills of 2.6 us on the device and 3.5 us on the host, and makes two of these.
+constexpr int CLEAR_BYTES = 16 * 1024;
+
+__global__ __launch_bounds__(256) void clear_rows_kernel(const longlong4* __restrict__ pieces, int row) {
+  const longlong4 piece = pieces[blockIdx.x];
+  char* to = reinterpret_cast<char*>(piece.x) + row * piece.y + piece.z;
+  const int bytes = static_cast<int>(piece.w);
+  if ((reinterpret_cast<uintptr_t>(to) | bytes) % 16 == 0) {
+    for (int i = threadIdx.x * 16; i < bytes; i += 256 * 16) *reinterpret_cast<uint4*>(to + i) = uint4{0u, 0u, 0u, 0u};
+  } else {
+    for (int i = threadIdx.x * 4; i < bytes; i += 256 * 4) *reinterpret_cast<uint32_t*>(to + i) = 0u;
+  }
+}
+
+extern "C" int distie_clear_rows_bytes() { return CLEAR_BYTES; }
+
+extern "C" int distie_clear_rows(const void* pieces, int count, int row, hipStream_t stream) {
+  if (count <= 0) return 0;
+  if (pieces == nullptr || row < 0) return DISTIE_BAD_ARGUMENT;
+  clear_rows_kernel<<<count, 256, 0, stream>>>(static_cast<const longlong4*>(pieces), row);
+  return launch_status();
+}

@@ -30,6 +30,7 @@ class ModelRunner:
         self.builder = BatchBuilder(cache, self.max_model_len, ops.device, model.spec.vocab_size, ops)
         self.graphs = None          # set by the engine when captured decode steps are on
         model.prepare(ops)
+        cache.clear_rows_with(ops)
 
     def step(self, entries: Sequence[StepEntry], reserve: bool = True,
              feed: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:

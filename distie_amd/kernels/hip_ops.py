@@ -449,6 +449,7 @@ class HipOps(Ops):
     def _declare(self) -> None:
         o = self._ops
         o.distie_scatter_i32.argtypes = [_P, _P, _P, _I, _L, _P]
+        o.distie_clear_rows.argtypes = [_P, _I, _I, _P]
         o.distie_embed.argtypes = [_P, _P, _I, _P, _I, _I, _I, _F, _P]
         o.distie_rmsnorm.argtypes = [_P, _P, _I, _I, _P, _I, _P, _I, _I, _I, _F, _P]
         o.distie_rope_kv_write.argtypes = [_P, _I, _I, _P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P]
@@ -615,6 +616,27 @@ class HipOps(Ops):
         _check(self._ops.distie_scatter_i32(table.data_ptr(), index.data_ptr(), value.data_ptr(), index.numel(),
                                             table.numel(), self._stream()), "scatter_i32")
         _mark_written(table)
+
+    def row_clearer(self, tensors):
+        pieces, others, most = [], [], self._ops.distie_clear_rows_bytes()
+        for t in tensors:
+            self._own(t)
+            size = t[0].numel() * t.element_size() if t.shape[0] else 0
+            if size % 4 or t.data_ptr() % 4:
+                others.append(t)
+                continue
+            pieces += [(t.data_ptr(), size, at, min(most, size - at)) for at in range(0, size, most)]
+        held, rows = list(tensors), min((t.shape[0] for t in tensors), default=0)      # (kept while the table names them)
+        table = torch.tensor(pieces, dtype=torch.int64).to(self.device) if pieces else None
+
+        def clear(row: int) -> None:
+            if held and not 0 <= row < rows:
+                raise KernelError(f"there is no row {row} to clear")
+            if table is not None:
+                _check(self._ops.distie_clear_rows(table.data_ptr(), len(pieces), row, self._stream()), "clear_rows")
+            for t in others:
+                t[row].zero_()
+        return clear
 
     def embed(self, ids, table, scale=1.0):
         self._own(ids, table)

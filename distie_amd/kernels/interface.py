@@ -141,6 +141,16 @@ class Ops(abc.ABC):
         changed entries of a step."""
         table.view(-1)[index.long()] = value
 
+    def row_clearer(self, tensors):
+        """-> a function that sets row `r` of every tensor of `tensors` (each [rows, ...]) to zeros: a new request's state rows.
+        The tensors stay where they are for as long as the function is used."""
+        tensors = list(tensors)
+
+        def clear(row: int) -> None:
+            for t in tensors:
+                t[row].zero_()
+        return clear
+
     @abc.abstractmethod
     def embed(self, ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
         """ids int32 [T], table [V, C] -> float32 [T, C], the rows times `scale` (in float32)."""

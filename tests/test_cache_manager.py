@@ -113,6 +113,30 @@ def test_page_bytes_counts_every_layer_and_tensor():
     assert CacheManager.page_bytes([None, FixedState.of((3,))], 4) == 0
 
 
+def test_a_slot_begins_with_zeros_however_rows_are_cleared():
+    class Clearer:
+        def row_clearer(self, tensors):
+            def clear(row):
+                self.rows.append(row)
+                for t in tensors:
+                    t[row].zero_()
+            self.rows = []
+            return clear
+
+    m = CacheManager([FixedState.of((3,)), PagedKV(1, 4), FixedState.of((2, 2))], 4, 12, 2)
+    clearer = Clearer()
+    m.clear_rows_with(clearer)
+    slabs = [next(iter(m.layer(i)["mixer"].tensors.values())) for i in (0, 2)]
+    for t in slabs:
+        t.fill_(1)
+    slot = m.add("a").slot
+    assert clearer.rows == [slot] and all(not t[slot].any() and t[1 - slot].all() and t[2].all() for t in slabs)
+    for t in slabs:
+        t.fill_(1)
+    m.reset("a")
+    assert clearer.rows == [slot, slot] and all(not t[slot].any() and t[1 - slot].all() for t in slabs)
+
+
 def test_reserve_commit_release_and_window():
     m = manager(block=4, pages=12, window=6)
     m.add("a")

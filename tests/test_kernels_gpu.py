@@ -42,6 +42,22 @@ def test_embed(ops, dtype):
     assert torch.equal(got, table[ids.long()].float())
 
 
+@pytest.mark.parametrize("shapes", [[(3, 5)], [(4096,), (4097,), (2, 4095), (1,)], [(8, 128, 128), (3, 1001), (4, 64)]])
+@pytest.mark.parametrize("row", [0, 2, 4])
+def test_state_rows_cleared_together(ops, shapes, row):
+    """One piece of 16 KB a block, its remainder, rows that begin at no multiple of 16 bytes, and 16-bit rows of odd length."""
+    slabs = [rand(5, *shape, seed=i) for i, shape in enumerate(shapes)] + [rand(5, 7, dtype=torch.bfloat16)]
+    want = [t.clone() for t in slabs]
+    for t in want:
+        t[row] = 0
+    clear = ops.row_clearer(slabs)
+    clear(row)
+    assert all(torch.equal(a, b) for a, b in zip(slabs, want))
+    with pytest.raises(RuntimeError):
+        clear(5)
+    assert all(torch.equal(a, b) for a, b in zip(slabs, want))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width", [(7, 40), (7, 1000), (7, 1002), (7, 3000), (7, 5000), (7, 8200),
                                         (2100, 1536), (5000, 332), (9000, 64)])     # many rows: two groups a thread
