@@ -37,7 +37,7 @@ HIP_FLAGS = ["-O3", f"--offload-arch={ARCH}", "-fPIC", "-std=c++17",
              "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option"]
 CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-pthread"]
 
-OPS_SOURCES = ["elementwise.hip", "gemm.hip", "packed_tiles.hip", "large_tiles.hip", "gemv.hip", "rows_f32.hip", "decode_products.hip", "sampling.hip", "sequence.hip", "recurrent.hip", "latent.hip", "ssm.hip",
+OPS_SOURCES = ["elementwise.hip", "gemm.hip", "packed_tiles.hip", "large_tiles.hip", "gemv.hip", "rows_f32.hip", "decode_products.hip", "layer_chain.hip", "sampling.hip", "sequence.hip", "recurrent.hip", "latent.hip", "ssm.hip",
                "depth.hip", "time_mixing.hip", "mixed_attention.hip", "delta.hip"]
 ATTN_SOURCES = ["attention.hip"]
 MIXED_ATTN_SOURCES = ["mixed_attention_mc.hip"]

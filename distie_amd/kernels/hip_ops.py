@@ -139,6 +139,41 @@ class NormedSum(_NotATensorYet):
         self.device = terms[0].device
 
 
+class LayerTail:
+    """What is left of a layer behind attention (`HipOps.layer_tail`), done in one launch (`distie_layer_chain`) once it is known whether
+    another layer's q/k/v product follows."""
+
+    def __init__(self, ops, residual, mixed, out_weight, norm_weight, eps, gate_up_weight, down_weight, scratch) -> None:
+        self.ops, self.residual, self.mixed, self.scratch = ops, residual, mixed, scratch
+        self.weights = (out_weight, gate_up_weight, down_weight)
+        self.norm = (norm_weight, float(eps))
+
+    def finish(self):
+        return self.ops._layer_chain(self, None)[0]
+
+    def finish_into(self, norm_weight, eps, weight, bias, meta, group, k_cache, v_cache, inv_freq, num_heads, num_kv_heads, head_dim,
+                    write):
+        held = getattr(weight, "_distie_rotary", None)
+        if held is None or held[1] != (num_heads, num_kv_heads, head_dim) or inv_freq is None or \
+                2 * inv_freq.shape[0] != head_dim or k_cache.dtype != torch.bfloat16 or self.mixed.dtype != torch.bfloat16:
+            return None
+        M, C = self.residual.shape
+        N, ops = weight.shape[0], self.ops
+        if weight.shape[1] != C or N != (num_heads + 2 * num_kv_heads) * head_dim or norm_weight.dtype not in _CODES or \
+                tuple(norm_weight.shape) != (C,) or M != meta.num_tokens or meta.groups[group].slots.shape[0] != M or \
+                (bias is not None and (bias.dtype != torch.float32 or bias.shape[0] != N)) or \
+                held[0].numel() != ops._packed_elements(N, C, False) or not ops._chain_fits(M, C, *self._inner(), N):
+            return None
+        ops._own(norm_weight, bias, k_cache, v_cache, inv_freq, meta.groups[group].slots)
+        ops._check_cache(k_cache, v_cache, num_kv_heads, meta.block_size, head_dim)
+        return ops._layer_chain(self, (norm_weight, float(eps), held[0], bias, ops._rope_table(meta, inv_freq),
+                                       meta.groups[group].slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim,
+                                       meta.block_size, 1 if write else 0))
+
+    def _inner(self):
+        return self.mixed.shape[1], self.weights[2].shape[1]
+
+
 class HipOps(Ops):
     # Steps of up to FUSED_MAX_ROWS rows can run their products with the norm in front and the residual sum behind
     # folded in (six launches a layer instead of eight, no partial sums handed on). On the device that is no
@@ -380,6 +415,19 @@ class HipOps(Ops):
     # attention with mixed heads: from so many tokens a step on a workgroup takes 16 queries instead of 8 (fewer would
     # leave compute units without one)
     MIXED_WIDE_TOKENS = 6144
+    # What a captured decode step of up to CHAIN_MAX_ROWS rows does between two layers' attention runs in one launch (`layer_chain.hip`),
+    # for the widths that the kernel is built for and as far as K of the sums fits its registers. Measured in a captured graph, every
+    # layer's weights from memory (us a layer, this / the six kernels, 1 and 8 rows): width 1,536, 8,960 hidden values 26.1 / 36.9 and
+    # 33.1 / 39.8, 4,096 21.3 / 29.0 and 25.9 / 30.4; width 2,048, 11,008 35.3 / 46.2 and 42.0 / 49.5, 5,632 27.5 / 35.0 and 31.0 /
+    # 37.3; width 1,024, 2,816 18.3 / 27.1 and 23.0 / 28.3, 8,192 20.4 / 30.6 and 26.7 / 32.0. Steps of the 1.5B shape: one request
+    # 1,437 -> 1,145, 4 requests of 16,000 keys 1,791 -> 1,568, 8 of 2,048 1,572 -> 1,404. Steps that are launched kernel by kernel
+    # keep their kernels. Values on their way between workgroups lie in memory that one fill prepares for CHAIN_CALLS layers.
+    CHAIN_MAX_ROWS = 8
+    CHAIN_WIDTHS = (1024, 1536, 2048)
+    CHAIN_CALLS = 32
+    CHAIN_WORKGROUPS = None          # workgroups of a launch (None: the compute units)
+    CHAIN_PATIENCE = 256             # looks for values, about 1 us each, before a workgroup does what nobody has taken
+    CHAIN_LIMIT = 1 << 14
     # the matrix-core attention kernels take heads up to 256; wider ones (a latent that all heads share) run on the
     # wave-per-token kernel, in either precision
     LARGEST_MATRIX_CORE_HEAD = 256
@@ -484,6 +532,10 @@ class HipOps(Ops):
         o.distie_decode_product_residual.argtypes = [_P, _P, _P, _P, _I, _I, _I, _P]
         o.distie_decode_norm_product.argtypes = [_P, _P, _F, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P,
                                                  _I, _I, _I, _I, _I, _P]
+        o.distie_layer_chain_fits.argtypes = [_I, _I, _I, _I, _I, _I]
+        o.distie_layer_chain_claims.argtypes = [_I]
+        o.distie_layer_chain.argtypes = [_P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P] + 9 * [_I] + \
+            [_P, _I, _I, _I, _I, _P]
         o.distie_hyper_step.argtypes = [_P, _I, _P, _P, _I, _I, _P, _I, _L, _I, _P, _P, _P, _P, _I, _I, _F, _P, _I, _I, _I, _P]
         o.distie_causal_conv.argtypes = [_P, _I, _L, _P, _I, _I, _P, _P, _I, _L, _I, _P, _P, _P, _P, _I, _I, _P]
         o.distie_conv_state.argtypes = [_P, _I, _L, _I, _P, _P, _P, _I, _I, _I, _P]
@@ -702,6 +754,66 @@ class HipOps(Ops):
             x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, residual.data_ptr(),
             M, N, K, self._stream()), "decode_product_residual")
         _mark_written(residual)
+
+    # ---- a layer's end and the next one's beginning in one launch
+    def _chain_fits(self, M, C, KO, inter, N) -> bool:
+        return bool(self._ops.distie_layer_chain_fits(M, C, KO, inter, N, self._compute_units))
+
+    def layer_tail(self, meta, residual, mixed, out_weight, norm_weight, eps, gate_up_weight, down_weight):
+        if not self.captured or residual.dim() != 2 or residual.shape[0] > self.CHAIN_MAX_ROWS or \
+                residual.shape[1] not in self.CHAIN_WIDTHS or mixed.dtype != torch.bfloat16 or residual.dtype != torch.float32:
+            return None
+        out_packed, gated, down_packed = (getattr(out_weight, "_distie_packed", None), getattr(gate_up_weight, "_distie_gated", None),
+                                          getattr(down_weight, "_distie_packed", None))
+        if out_packed is None or gated is None or down_packed is None:
+            return None
+        M, C = residual.shape
+        KO, inter = mixed.shape[1], down_weight.shape[1]
+        if mixed.shape[0] != M or tuple(out_weight.shape) != (C, KO) or tuple(gate_up_weight.shape) != (2 * inter, C) or \
+                down_weight.shape[0] != C or norm_weight.dtype not in _CODES or tuple(norm_weight.shape) != (C,) or \
+                out_packed.numel() != self._packed_elements(C, KO, False) or \
+                gated.numel() != self._packed_elements(2 * inter, C, True) or \
+                down_packed.numel() != self._packed_elements(C, inter, False) or not self._chain_fits(M, C, KO, inter, 0) or \
+                residual.data_ptr() % 16 or mixed.data_ptr() % 16:
+            return None
+        self._own(residual, mixed, norm_weight)
+        return LayerTail(self, residual, mixed, out_weight, norm_weight, eps, gate_up_weight, down_weight,
+                         self._chain_buffers(meta, M, C, inter))
+
+    def _chain_buffers(self, meta, M, C, inter):
+        """int32 words of one launch, every byte 0xff: `mid`, `out` [M, C], `hidden` [M, inter] / 2, the claims. The launches of a
+        step share a fill (each has words of its own)."""
+        words = 2 * M * C + -(-M * inter // 8) * 4 + self._ops.distie_layer_chain_claims(self._compute_units)
+        key = ("layer_chain", words)
+        left = meta.scratch.get(key)
+        if left is None or not left.shape[0]:
+            left = torch.full((self.CHAIN_CALLS, -(-words // 64) * 64), -1, dtype=torch.int32, device=self.device)
+        meta.scratch[key] = left[1:]
+        return left[0]
+
+    def _layer_chain(self, tail, following):
+        """-> (new residual, q/k/v of the layer behind or None)"""
+        M, C = tail.residual.shape
+        KO, inter = tail._inner()
+        out_weight, gate_up_weight, down_weight = tail.weights
+        words = tail.scratch
+        mid, out, hidden = words[:M * C], words[M * C:2 * M * C], words[2 * M * C:]
+        claims = words[words.shape[0] - self._ops.distie_layer_chain_claims(self._compute_units):]
+        norm_weight, eps = tail.norm
+        qkv, rest, next_norm, next_eps, packed, bias = None, (None, None, None, None, 0, 0, 0, 0, 0), None, 0.0, None, None
+        if following is not None:
+            next_norm, next_eps, packed, bias, table, slots, k_cache, v_cache, heads, kv_heads, dim, block_size, write = following
+            next_norm = self._f32(next_norm)
+            qkv = torch.empty((M, (heads + 2 * kv_heads) * dim), dtype=torch.bfloat16, device=self.device)
+            rest = (table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), heads, kv_heads, dim, block_size, write)
+        ptr = lambda t: t.data_ptr() if t is not None else None
+        _check(self._ops.distie_layer_chain(
+            tail.mixed.data_ptr(), out_weight._distie_packed.data_ptr(), tail.residual.data_ptr(), mid.data_ptr(),
+            self._f32(norm_weight).data_ptr(), eps, gate_up_weight._distie_gated.data_ptr(), hidden.data_ptr(),
+            down_weight._distie_packed.data_ptr(), out.data_ptr(), ptr(next_norm), next_eps, ptr(packed), ptr(bias), ptr(qkv), *rest,
+            M, C, KO, inter, claims.data_ptr(), self._compute_units, self.CHAIN_WORKGROUPS or self._compute_units,
+            self.CHAIN_PATIENCE, self.CHAIN_LIMIT, self._stream()), "layer_chain")
+        return out.view(torch.float32).view(M, C), qkv
 
     def dense(self, x):
         """The finished tensor of a value that an operation here returned in a form of its own (partial sums,

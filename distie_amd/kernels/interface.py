@@ -194,6 +194,14 @@ class Ops(abc.ABC):
         one stacked product); an implementation may choose another kernel than for a product that one operation reads."""
         return self.dense(self.linear(x, weight, bias))
 
+    def layer_tail(self, meta, residual, mixed, out_weight, norm_weight, eps, gate_up_weight, down_weight):
+        """What is left of a pre-norm layer behind attention's result `mixed`, if an implementation wants to do it in one piece (None:
+        it does not): h = residual + mixed out_weight^T, then h + down(silu(gate x) * up x) for x = rmsnorm(h) * norm_weight. The
+        answer has `finish()` -> the new residual (float32; `residual` stays as it is), and `finish_into(...)`, whose arguments are
+        the next layer's norm (weight, eps) and those of `linear_rope_kv_write` behind x -> (new residual, q/k/v), or None if it
+        cannot do these together (`finish` then still can). One of them is called, once."""
+        return None
+
     def prepare_linear(self, weight: torch.Tensor, gated: bool = False, rotary=None, role: Optional[str] = None) -> None:
         """Called once for every weight of a `linear` after it is loaded (`gated`: the weight of a
         `linear_silu_mul`; `rotary = (num_heads, num_kv_heads, head_dim)`: the stacked q/k/v weight

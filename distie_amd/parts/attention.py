@@ -115,14 +115,37 @@ class Attention(Mixer):
         classes = context_classes(limit, self.FIRST_CONTEXT)
         return classes[min(bisect.bisect_left(classes, longest), len(classes) - 1)]
 
-    def forward(self, ops, x, ctx, cache, writes_cache: bool):
-        k_cache, v_cache = cache["k"], cache["v"]
-        qkv = ops.linear_rope_kv_write(x, self.qkv_weight, self.qkv_bias_t, ctx.meta, cache.group, k_cache, v_cache,
-                                       self.position.rotary(), self.num_heads, self.num_kv_heads, self.head_dim,
+    @property
+    def staged(self) -> bool:
+        """An arrangement may run the stages of `forward` one by one."""
+        return type(self).forward is Attention.forward
+
+    def project(self, ops, x, ctx, cache, writes_cache: bool):
+        return ops.linear_rope_kv_write(x, self.qkv_weight, self.qkv_bias_t, ctx.meta, cache.group, cache["k"], cache["v"],
+                                        self.position.rotary(), self.num_heads, self.num_kv_heads, self.head_dim,
+                                        writes_cache)
+
+    def project_behind(self, ops, stream, norm, ctx, cache, writes_cache: bool):
+        """`project` of the normed stream together with what is left of the layer before; None if these are not one launch."""
+        if getattr(norm, "fused_kind", None) != "rms":
+            return None
+        done = stream.tail.finish_into(norm.weight, norm.eps, self.qkv_weight, self.qkv_bias_t, ctx.meta, cache.group, cache["k"],
+                                       cache["v"], self.position.rotary(), self.num_heads, self.num_kv_heads, self.head_dim,
                                        writes_cache)
-        mixed = ops.paged_attention(qkv, ctx.meta, cache.group, k_cache, v_cache, self.num_heads,
-                                    self.num_kv_heads, self.head_dim, self.scale, self.window, self.extras)
+        if done is None:
+            return None
+        stream.hidden, qkv = done
+        return qkv
+
+    def attend(self, ops, qkv, ctx, cache):
+        return ops.paged_attention(qkv, ctx.meta, cache.group, cache["k"], cache["v"], self.num_heads,
+                                   self.num_kv_heads, self.head_dim, self.scale, self.window, self.extras)
+
+    def finish(self, ops, mixed):
         return ops.linear(mixed, self.out_weight, self.out_bias_t)
+
+    def forward(self, ops, x, ctx, cache, writes_cache: bool):
+        return self.finish(ops, self.attend(ops, self.project(ops, x, ctx, cache, writes_cache), ctx, cache))
 
 
 register_part("mixer", "attention", Attention)

@@ -120,12 +120,27 @@ class ResidualStream:
     adds it while it reads the stream, which saves one pass over the activations."""
 
     def __init__(self, hidden: torch.Tensor) -> None:
-        self.hidden = hidden
+        self._hidden = hidden
         self.pending: Optional[torch.Tensor] = None
+        # What is left to do of a layer (`Ops.layer_tail`): the next layer may do it together with the beginning of its own, anyone
+        # else who asks for `hidden` has it done then.
+        self.tail = None
         # An arrangement that keeps the residual in a form of its own (several streams) hangs it here, with a
         # function that turns it back into `hidden` [T, C] and `pending` once the last block has run.
         self.lanes = None
         self.settle: Optional[Callable] = None
+
+    @property
+    def hidden(self) -> torch.Tensor:
+        if self.tail is not None:
+            tail, self.tail = self.tail, None
+            self._hidden = tail.finish()
+        return self._hidden
+
+    @hidden.setter
+    def hidden(self, value: torch.Tensor) -> None:
+        self.tail = None
+        self._hidden = value
 
     def close(self, ops) -> None:
         """After the last block: `hidden` (and `pending`) are the plain residual sum again."""

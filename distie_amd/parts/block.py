@@ -13,8 +13,27 @@ class PreNormResidual(Block):
     CHILDREN = {"mixer_norm": "norm", "mixer": "mixer", "feed_forward_norm": "norm", "feed_forward": "feed_forward"}
 
     def forward(self, ops, stream: ResidualStream, ctx: StepContext, cache, writes_cache: bool) -> None:
-        normed = self.mixer_norm.of_stream(ops, stream, ctx.act_dtype)
-        stream.pending = self.mixer.forward(ops, normed, ctx, cache["mixer"], writes_cache)
+        staged = getattr(self.mixer, "staged", False)
+        qkv = None
+        if staged and stream.tail is not None:
+            # the layer before is not finished: its end and this one's q/k/v product may be one launch
+            qkv = self.mixer.project_behind(ops, stream, self.mixer_norm, ctx, cache["mixer"], writes_cache)
+        if qkv is None:
+            normed = self.mixer_norm.of_stream(ops, stream, ctx.act_dtype)
+            if not staged:
+                stream.pending = self.mixer.forward(ops, normed, ctx, cache["mixer"], writes_cache)
+                normed = self.feed_forward_norm.of_stream(ops, stream, ctx.act_dtype)
+                stream.pending = self.feed_forward.forward(ops, normed, ctx)
+                return
+            qkv = self.mixer.project(ops, normed, ctx, cache["mixer"], writes_cache)
+        mixed = self.mixer.attend(ops, qkv, ctx, cache["mixer"])
+        weights = getattr(self.feed_forward, "silu_weights", None)
+        if weights is not None and self.mixer.out_bias_t is None and getattr(self.feed_forward_norm, "fused_kind", None) == "rms":
+            stream.tail = ops.layer_tail(ctx.meta, stream.hidden, mixed, self.mixer.out_weight, self.feed_forward_norm.weight,
+                                         self.feed_forward_norm.eps, *weights)
+            if stream.tail is not None:
+                return
+        stream.pending = self.mixer.finish(ops, mixed)
         normed = self.feed_forward_norm.of_stream(ops, stream, ctx.act_dtype)
         stream.pending = self.feed_forward.forward(ops, normed, ctx)
 

@@ -51,6 +51,12 @@ class SwiGLU(FeedForward):
         ops.prepare_linear(self.gate_up_weight, gated=True, role="gate_up")
         ops.prepare_linear(self.down_weight, role="down")
 
+    @property
+    def silu_weights(self):
+        """(gate and up, down) where `forward` is down(silu(gate x) * up x), else None."""
+        plain = self.activation == "silu" and type(self).forward is SwiGLU.forward
+        return (self.gate_up_weight, self.down_weight) if plain else None
+
     def forward(self, ops, x, ctx):
         if self.activation == "silu":
             return ops.linear(ops.linear_silu_mul(x, self.gate_up_weight), self.down_weight)

@@ -41,6 +41,48 @@ def test_cuttings(setup, cuts):
     runner.cache.check()
 
 
+class TailOps(TorchOps):
+    """Takes what is left of every layer in one piece, and the next layer's q/k/v with it every other time."""
+
+    def __init__(self):
+        super().__init__()
+        self.ended = [0, 0]
+
+    def layer_tail(self, meta, residual, mixed, out_weight, norm_weight, eps, gate_up_weight, down_weight):
+        ops = self
+
+        class Tail:
+            def finish(self):
+                ops.ended[0] += 1
+                h = residual + ops.linear(mixed, out_weight).float()
+                x = ops.rmsnorm(h, norm_weight, eps, mixed.dtype)
+                return h + ops.linear(ops.linear_silu_mul(x, gate_up_weight), down_weight).float()
+
+            def finish_into(self, weight, eps, qkv_weight, bias, *rest):
+                if sum(ops.ended) % 2:
+                    return None
+                h = self.finish()
+                ops.ended[0] -= 1
+                ops.ended[1] += 1
+                return h, ops.linear_rope_kv_write(ops.rmsnorm(h, weight, eps, mixed.dtype), qkv_weight, bias, *rest)
+
+        return Tail()
+
+
+@pytest.mark.parametrize("cuts", [[13], [1, 1, 1, 30]])
+def test_layers_whose_end_is_left_to_the_next_one(setup, cuts):
+    cfg, block, folder, weights = setup
+    ops = TailOps()
+    runner = build_runner(folder, ops, block_size=block)
+    ids = random_ids(cfg, 50, 2)
+    got = replay_cut(runner, "a", ids, cuts)
+    assert (got - oracle(weights, cfg, ids)).abs().max() < FP32_TOL
+    assert min(ops.ended) > 0
+    steps = len(cuts) + len(ids) - sum(cuts)
+    assert sum(ops.ended) == steps * cfg["num_hidden_layers"]
+    runner.cache.check()
+
+
 def test_mixed_batches_with_page_reuse(setup):
     cfg, block, folder, weights = setup
     lengths = [37, 50, 21, 44, 30, 26]

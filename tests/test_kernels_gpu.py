@@ -666,6 +666,84 @@ def test_linear_rope_kv_write_fused(ops, M, heads, kv_heads, dim, K, P, with_bia
     close(unfused, want, torch.bfloat16, scale=2 * scale)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
+@pytest.mark.parametrize("C,I,heads,kv_heads,dim,with_bias,write", [
+    (1536, 8960, 12, 2, 128, True, True), (1536, 9216, 4, 4, 48, False, True), (1536, 32, 12, 12, 128, True, False),
+    (1024, 2816, 16, 2, 64, True, True), (1024, 8192, 1, 1, 32, False, True), (2048, 11008, 16, 2, 128, True, True),
+    (2048, 1056, 8, 1, 16, True, True)])
+def test_a_layers_end_and_the_next_ones_beginning_in_one_launch(ops, M, C, I, heads, kv_heads, dim, with_bias, write):
+    """`layer_tail` against the same operations in float64 with the same roundings: sizes with K that fills no whole group of tiles,
+    fewer units than compute units and more, the longest K of each width; with another layer behind it and without. The same bits
+    come from workgroups that do the work of others who never start, in every phase that someone waits for (the last is theirs)."""
+    P, eps, KO, N = 8, 1e-5, heads * dim, (heads + 2 * kv_heads) * dim
+    bf = torch.bfloat16
+    mixed, residual = rand(M, KO, dtype=bf, seed=1), rand(M, C, seed=2)
+    w_o, w_gu = rand(C, KO, dtype=bf, seed=3, scale=KO ** -0.5), rand(2 * I, C, dtype=bf, seed=4, scale=C ** -0.5)
+    w_d, w_qkv = rand(C, I, dtype=bf, seed=5, scale=I ** -0.5), rand(N, C, dtype=bf, seed=6, scale=C ** -0.5)
+    norm, next_norm = rand(C, seed=7) * 0.2 + 1, (rand(C, seed=8) * 0.2 + 1).to(bf)
+    bias = rand(N, seed=9) if with_bias else None
+    ops.prepare_linear(w_o, role="attn_out")
+    ops.prepare_linear(w_gu, gated=True, role="gate_up")
+    ops.prepare_linear(w_d, role="down")
+    ops.prepare_linear(w_qkv, rotary=(heads, kv_heads, dim), role="qkv")
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, dim, 2, dtype=torch.float32) / dim))).cuda()
+    slots = [(5 * i + 3) % (4 * M) for i in range(M)]
+    new_meta = lambda: make_meta([17 * i for i in range(M)], list(range(M)), list(range(M + 1)), [17 * i + 1 for i in range(M)],
+                                 [[0] * 8] * M, slots, P)
+    k0, v0 = rand(M, kv_heads, P, dim, dtype=bf, seed=10), rand(M, kv_heads, dim, P, dtype=bf, seed=11)
+
+    def normed(h, weight):
+        return (h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + eps) * weight.double()).to(bf).double()
+
+    mid = residual.double() + mixed.double() @ w_o.double().T
+    gate_up = normed(mid, norm) @ w_gu.double().T
+    added = (torch.nn.functional.silu(gate_up[:, :I]) * gate_up[:, I:]).to(bf).double() @ w_d.double().T
+    want = mid + added
+    product = normed(want, next_norm) @ w_qkv.double().T + (bias.double() if with_bias else 0.0)
+    k_want, v_want = k0.clone(), v0.clone()
+    qkv_want = TorchOps("cuda").rope_kv_write(product.float().clone(), new_meta(), 0, k_want, v_want, inv_freq, heads, kv_heads, dim, write)
+    before = residual.clone()
+
+    def run(last=False):
+        meta, k, v = new_meta(), k0.clone(), v0.clone()
+        tail = ops.layer_tail(meta, residual, mixed, w_o, norm, eps, w_gu, w_d)
+        assert tail is not None
+        if last:
+            return (tail.finish(),)
+        hidden, qkv = tail.finish_into(next_norm, eps, w_qkv, bias, meta, 0, k, v, inv_freq, heads, kv_heads, dim, write)
+        torch.cuda.synchronize()
+        return hidden, qkv, k, v
+
+    ops.captured = True
+    try:
+        hidden, qkv, k, v = got = run()
+        assert hidden.dtype == torch.float32 and qkv.dtype == bf and torch.equal(residual, before)
+        # every hidden value may have been rounded the other way: half a unit of 2^-8 each, in the product
+        assert (hidden.double() - want).norm() <= 2.0 ** -9 * added.norm() + 1e-6 * want.norm()
+        scale = qkv_want.abs().max().item()
+        close(qkv, qkv_want, bf, scale=scale)
+        close(k, k_want, bf, scale=scale)
+        close(v, v_want, bf, scale=scale)
+        assert torch.equal(run(last=True)[0], hidden)
+        ops.CHAIN_WORKGROUPS, ops.CHAIN_PATIENCE = 40, 2
+        assert torch.equal(run()[0], hidden)
+        ops.CHAIN_WORKGROUPS = 1
+        assert torch.equal(run()[0], hidden)
+        del ops.CHAIN_WORKGROUPS, ops.CHAIN_PATIENCE
+        assert all(torch.equal(a, b) for a, b in zip(run(), got))
+        # values that are no numbers stay with their row and are not waited for
+        if M > 1:
+            residual[0, 5], residual[1, 7] = float("nan"), float("inf")
+            odd = run()[0]
+            assert not torch.isfinite(odd[:2]).all(dim=1).any() and torch.equal(odd[2:], hidden[2:])
+            residual.copy_(before)
+    finally:
+        ops.captured = False
+        for name in ("CHAIN_WORKGROUPS", "CHAIN_PATIENCE"):
+            ops.__dict__.pop(name, None)
+    assert ops.layer_tail(new_meta(), residual, mixed, w_o, norm, eps, w_gu, w_d) is None       # launched kernel by kernel
+
+
 @pytest.mark.parametrize("M", [1, 5, 8, 9, 16])
 @pytest.mark.parametrize("C,I,heads,kv_heads,dim", [(1536, 4484, 12, 2, 128), (72, 13, 3, 1, 16), (3584, 300, 4, 4, 48),
                                                     (4096, 88, 2, 1, 80), (264, 172, 5, 5, 32)])
