@@ -16,6 +16,7 @@
 //  * attn_decode + attn_reduce, attn_prefill: bfloat16 on the matrix cores (described further down).
 
 #include "common.h"
+#include "lds_load.h"
 #include <algorithm>
 
 #ifndef DISTIE_HEAD_DIM
@@ -1964,6 +1965,339 @@ extern "C" int distie_attention_prefill_bf16(const void* qkv, int64_t q_stride, 
 }
 
 // ===================================================================================================
+//  * attn_prefill_keys: the same products, cut the other way: the W waves of a workgroup share its 32 query columns (tokens of one
+//    head) and each walks every W-th tile of 32 keys on its own. A wave's K and V^T tiles come from memory straight into a piece of
+//    LDS of its own, the next ones while it multiplies the present ones, so the loop has no barrier; behind it the W sums
+//    meet in LDS. A prompt of a few hundred tokens is one trip for q, K and V, one to three tiles a wave and that end, where
+//    attn_prefill is a walk over all its keys by a fifth of the chip, and parts that a second launch merges.
+//    K rows lie in LDS with their 16-byte pieces turned by the row's number (piece j of row r at j ^ r), which the loads
+//    do and which keeps the reads of 32 rows free of bank conflicts; a row of V^T of 16 keys is two pieces, read in order. The
+//    rows of a product are taken in an order in which a lane's scores are eight keys in a row, and those it reads of V^T.
+//    12 heads of 128 and 2 kv heads, us, attn_prefill with its merge / this: 40 tokens 6.4 / 6.0, 301 13.8 / 7.8, 512 18.1 / 9.0, 1,024
+//    27.9 / 14.2, 2,048 39.3 / 27.3. What bounds it: of the 6, 2 are the launch and the rest a chain of trips (requests, positions
+//    and pages, keys, the sums); a tile costs a wave about 1 us alone on its SIMD and 1.3 beside another, a quarter of it products: reads
+//    of LDS, the softmax and the next loads' addresses, one behind the other. Two waves a SIMD need the small tile: 64 keys at one wave
+//    a SIMD 51 us for 2,048 tokens, 64 keys and 64 columns 42 (then 41 at 32 keys). The columns' maximum went through LDS at first, the
+//    queries were waited for together with the first keys, and loads beyond the last tile were issued: 40 (W = 8), 32 (W = 4).
+// ===================================================================================================
+#if DISTIE_HEAD_DIM == 64 || DISTIE_HEAD_DIM == 128
+constexpr int KEYS_BM = 32;                             // tokens of a workgroup
+constexpr int KEYS_BN = 32;                             // keys of a wave's tile
+constexpr int KEYS_PIECES = D / 8;                      // 16-byte pieces of a row of K
+constexpr int KEYS_LOADS = D / 32;                      // loads (of 1 KB) of 16 keys of K, and of V^T
+constexpr int KEYS_O_STRIDE = D + 4;                    // floats: rows of an odd number of 16-byte pieces
+
+// LDS: the waves' tiles and, in their place, their sums; behind that their references and the columns' factors
+template <int W>
+constexpr int prefill_keys_tiles() {
+  const int tiles = W * KEYS_BN * D * 4, sums = W * KEYS_BM * KEYS_O_STRIDE * 4;
+  return tiles > sums ? tiles : sums;
+}
+template <int W>
+constexpr int prefill_keys_lds() { return prefill_keys_tiles<W>() + (W + 1) * KEYS_BM * 8; }
+
+// The larger of a column's two values, in lanes c and c + 32.
+__device__ __forceinline__ float column_max(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  const uint32_t low = both[0], high = both[1];
+  return fmaxf(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
+}
+
+template <int W>
+__global__ __launch_bounds__(DISTIE_WAVE * W) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_keys_kernel(
+    const bf16_t* __restrict__ qkv, int64_t q_stride, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ positions, const int32_t* __restrict__ cu_q,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ table_rows, bf16_t* __restrict__ out,
+    int num_requests, int heads, int kv_heads, int block_size, float scale, int window, int min_q_len,
+    const float* __restrict__ sinks) {
+  constexpr int BLOCKS = KEYS_BN / 16;
+  constexpr int LOADS = BLOCKS * KEYS_LOADS;            // of a tile of K, and of V^T
+  constexpr int STEP = W * KEYS_BN;
+  extern __shared__ __attribute__((aligned(16))) char keys_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / DISTIE_WAVE);
+  const int lane = threadIdx.x % DISTIE_WAVE;
+  const int c = lane % 32;
+  const int h = lane / 32;
+  const float scale_log2 = scale * 1.4426950408889634f;
+
+  // ---- which tokens: as attn_prefill, the late ones first
+  int tile = gridDim.y - 1 - blockIdx.y;
+  int request = 0, begin = 0, end = 0;
+  for (; request < num_requests; ++request) {
+    begin = cu_q[request];
+    end = cu_q[request + 1];
+    if (end - begin < min_q_len) continue;
+    const int tiles = (end - begin + KEYS_BM - 1) / KEYS_BM;
+    if (tile < tiles) break;
+    tile -= tiles;
+  }
+  if (request >= num_requests) return;
+  const int head = blockIdx.x;
+  const int kh = head / (heads / kv_heads);
+  const int token0 = begin + tile * KEYS_BM;
+  const int columns = min(KEYS_BM, end - token0);
+  const int pos0 = positions[token0];                   // the tokens of a portion have consecutive positions
+  const int32_t* table = block_table + static_cast<int64_t>(table_rows != nullptr ? table_rows[request] : request) * table_width;
+  const int block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
+
+  // ---- the queries, on their way before anything says which keys they see
+  const int col = min(c, columns - 1);                  // columns past the end repeat the last; dropped later
+  bf16x8 q_reg[PF_DK];
+  {
+    const bf16_t* q = qkv + (token0 + col) * q_stride + static_cast<int64_t>(head) * D;
+#pragma unroll
+    for (int dk = 0; dk < PF_DK; ++dk) q_reg[dk] = *reinterpret_cast<const bf16x8*>(q + 16 * dk + 8 * h);
+  }
+
+  // ---- tiles into LDS
+  char* const k_tile = keys_lds + wave * (KEYS_BN * D * 4);
+  char* const v_tile = k_tile + KEYS_BN * D * 2;
+  const uint32_t k_at = lds_place(k_tile), v_at = lds_place(v_tile);
+  int k_lane[KEYS_LOADS], v_lane[KEYS_LOADS];
+#pragma unroll
+  for (int j = 0; j < KEYS_LOADS; ++j) {
+    const int row = (DISTIE_WAVE / KEYS_PIECES) * j + lane / KEYS_PIECES;
+    k_lane[j] = row * (2 * D) + ((lane % KEYS_PIECES) ^ (row % KEYS_PIECES)) * 16;
+    const int piece = DISTIE_WAVE * j + lane;
+    v_lane[j] = (piece / 2) * (2 * block_size) + (piece % 2) * 16;
+  }
+  struct Pages { int of[BLOCKS]; };
+  auto lookup = [&](int k0) __attribute__((always_inline)) {
+    Pages pages;
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) {
+      const int key = k0 + 16 * b;
+      const int slot = block_shift >= 0 ? key >> block_shift : key / block_size;
+      pages.of[b] = table[min(slot, table_width - 1)];
+    }
+    return pages;
+  };
+  // A block of 16 keys outside the workgroup's keys belongs to no page that is known here: its loads read beyond the end of
+  // an empty buffer, which gives zeros.
+  int key_begin = 0, key_end = 0;
+  const uint32_t page_bytes = 2u * static_cast<uint32_t>(kv_heads) * block_size * D;
+  const char* const k_head = reinterpret_cast<const char*>(k_cache) + 2 * static_cast<int64_t>(kh) * block_size * D;
+  const char* const v_head = reinterpret_cast<const char*>(v_cache) + 2 * static_cast<int64_t>(kh) * block_size * D;
+  auto ask = [&](int k0, const Pages& pages, bool values) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) {
+      const int key = k0 + 16 * b;
+      const bool live = key <= key_end && key + 15 >= key_begin;
+      const int offset = block_shift >= 0 ? key & (block_size - 1) : key % block_size;
+      const uint64_t page = static_cast<uint64_t>(static_cast<uint32_t>(pages.of[b])) * page_bytes;
+      if (values) {
+        const intx4 from = buffer_of(v_head + page + 2 * offset, live ? 2 * ((D - 1) * block_size + 16) : 0);
+#pragma unroll
+        for (int j = 0; j < KEYS_LOADS; ++j) buffer_to_lds(from, v_lane[j], 0, v_at + (b * KEYS_LOADS + j) * 1024);
+      } else {
+        const intx4 from = buffer_of(k_head + page + 2 * D * offset, live ? 32 * D : 0);
+#pragma unroll
+        for (int j = 0; j < KEYS_LOADS; ++j) buffer_to_lds(from, k_lane[j], 0, k_at + (b * KEYS_LOADS + j) * 1024);
+      }
+    }
+  };
+  // (without a window the first pages do not wait for the position)
+  int k0 = wave * KEYS_BN;
+  if (window != 0) k0 += first_visible(pos0, window) / KEYS_BN * KEYS_BN;
+  Pages pages = lookup(k0);
+  key_begin = first_visible(pos0, window);
+  key_end = pos0 + columns - 1;
+  const int col_last = pos0 + col, col_first = first_visible(col_last, window);       // what the lane's column sees
+  const int open_from = first_visible(key_end, window); // from here on every column sees (up to its own position)
+  // (the queries are waited for here: a wait for them inside the loop would wait for its tiles as well)
+#pragma unroll
+  for (int dk = 0; dk < PF_DK; ++dk) asm volatile("" : "+v"(q_reg[dk]));
+  if (k0 <= key_end) {
+    ask(k0, pages, false);
+    ask(k0, pages, true);
+    if (k0 + STEP <= key_end) pages = lookup(k0 + STEP);
+  }
+
+  floatx16 o_acc[PF_DB];
+#pragma unroll
+  for (int db = 0; db < PF_DB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o_acc[db][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  // the row of K behind row c of a product, and where its pieces are
+  const int row = 16 * (c / 16) + 8 * ((c / 4) % 2) + 4 * ((c / 8) % 2) + c % 4;
+  int piece_at[PF_DK];
+#pragma unroll
+  for (int dk = 0; dk < PF_DK; ++dk) piece_at[dk] = row * (2 * D) + ((2 * dk + h) ^ (row % KEYS_PIECES)) * 16;
+
+  for (; k0 <= key_end; k0 += STEP) {
+    const bool more = k0 + STEP <= key_end;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");       // K is there; V^T is under way
+    floatx16 s;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll
+    for (int dk = 0; dk < PF_DK; ++dk) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(k_tile + piece_at[dk]);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, q_reg[dk], s, 0, 0, 0);
+    }
+    // (all reads before the first product: left to itself the compiler keeps two under way)
+    __builtin_amdgcn_sched_group_barrier(0x100, PF_DK, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, PF_DK, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // K has been read: its place is free
+    if (more) ask(k0 + STEP, pages, false);
+
+    if (k0 + KEYS_BN - 1 > pos0 || k0 < open_from) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = k0 + 16 * (e / 8) + 8 * h + e % 8;
+        if (key < col_first || key > col_last) s[e] = -INFINITY;
+      }
+    }
+    // the running reference follows the largest score as in attn_prefill
+    float top = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) top = fmaxf(top, s[e]);
+    const float best = column_max(top) * scale_log2;
+    if (__any(best > m_run + PF_GROW)) {
+      const float m_new = fmaxf(m_run, best);
+      const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
+      l_run *= alpha;
+      m_run = m_new;
+#pragma unroll
+      for (int db = 0; db < PF_DB; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o_acc[db][e] *= alpha;
+    }
+    const float from = m_run == -INFINITY ? 0.f : -m_run;
+    bf16x8 p_reg[BLOCKS];                               // step t: keys 16 t + 8 h .. + 7 of the tile
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float p = fast_exp2(fmaf(s[e], scale_log2, from));
+      sum += p;
+      p_reg[e / 8][e % 8] = static_cast<bf16_t>(p);
+    }
+    l_run += sum;
+    if (more)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");     // V^T is there; the next K is under way
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (k0 + KEYS_BN - 1 > key_end && key_end % 16 != 15) {
+      // Slots after the last key were not written by this request (a weight of zero times NaN would still be NaN).
+      const int b = (key_end - k0) / 16, left = key_end % 16 + 1;       // the block of the last key, and its keys
+#pragma unroll
+      for (int j = 0; j < KEYS_LOADS; ++j) {
+        const int piece = DISTIE_WAVE * j + lane;
+        const int written = left - 8 * (piece % 2);
+        uint4* const at = reinterpret_cast<uint4*>(v_tile + b * (32 * D) + piece * 16);
+        const uint4 v = *at;
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        uint32_t m[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = written >= 2 * e + 2 ? w[e] : (written == 2 * e + 1 ? (w[e] & 0x0000ffffu) : 0u);
+        *at = uint4{m[0], m[1], m[2], m[3]};
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+#pragma unroll
+    for (int t = 0; t < BLOCKS; ++t)
+#pragma unroll
+      for (int db = 0; db < PF_DB; ++db) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(v_tile + t * (32 * D) + db * 1024 + (2 * c + h) * 16);
+        o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, p_reg[t], o_acc[db], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_group_barrier(0x100, BLOCKS * PF_DB, 1);
+    __builtin_amdgcn_sched_group_barrier(0x008, BLOCKS * PF_DB, 1);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // V^T has been read
+    if (more) {
+      ask(k0 + STEP, pages, true);
+      if (k0 + 2 * STEP <= key_end) pages = lookup(k0 + 2 * STEP);
+    }
+  }
+
+  // ---- the waves' sums, put together: each scaled to the largest reference (a sink is one more), then added in order
+  lds_arrived<0>();                                     // nothing under way, and every wave is done with its tiles
+  float* const sums = reinterpret_cast<float*>(keys_lds);
+  float2* const refs = reinterpret_cast<float2*>(keys_lds + prefill_keys_tiles<W>());     // [wave][column]
+  float* const inverse = reinterpret_cast<float*>(refs + W * KEYS_BM);                    // [column]
+  l_run += __shfl_xor(l_run, 32, DISTIE_WAVE);
+  if (h == 0) refs[wave * KEYS_BM + c] = float2{m_run, l_run};
+  __syncthreads();
+  {
+    const float sink = sinks != nullptr ? sinks[head] * 1.4426950408889634f : -INFINITY;
+    float2 ml[W];
+    float m = sink;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      ml[w] = refs[w * KEYS_BM + c];
+      m = fmaxf(m, ml[w].x);
+    }
+    float l = sink == -INFINITY ? 0.f : fast_exp2(sink - m);
+#pragma unroll
+    for (int w = 0; w < W; ++w) l += ml[w].x == -INFINITY ? 0.f : fast_exp2(ml[w].x - m) * ml[w].y;
+    if (wave == 0 && h == 0) inverse[c] = 1.f / l;
+    const float alpha = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m);
+    float* const to = sums + (wave * KEYS_BM + c) * KEYS_O_STRIDE + 4 * h;
+#pragma unroll
+    for (int db = 0; db < PF_DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(to + 32 * db + 8 * i) = float4{o_acc[db][4 * i] * alpha, o_acc[db][4 * i + 1] * alpha,
+                                                                 o_acc[db][4 * i + 2] * alpha, o_acc[db][4 * i + 3] * alpha};
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < columns * (D / 4); i += DISTIE_WAVE * W) {
+    const int to = i / (D / 4), d = 4 * (i % (D / 4));
+    float4 sum = *reinterpret_cast<const float4*>(sums + to * KEYS_O_STRIDE + d);
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+      const float4 part = *reinterpret_cast<const float4*>(sums + (w * KEYS_BM + to) * KEYS_O_STRIDE + d);
+      sum.x += part.x;
+      sum.y += part.y;
+      sum.z += part.z;
+      sum.w += part.w;
+    }
+    const float inv = inverse[to];
+    const float o[4] = {sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv};
+    uint32_t half[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) half[e] = __builtin_bit_cast(uint16_t, static_cast<bf16_t>(o[e]));
+    *reinterpret_cast<uint2*>(out + (static_cast<int64_t>(token0 + to) * heads + head) * D + d) =
+        uint2{half[0] | (half[1] << 16), half[2] | (half[3] << 16)};
+  }
+}
+
+extern "C" int distie_attention_prefill_keys_fits() { return 1; }
+
+// As distie_attention_prefill_bf16, with nothing between its parts. waves (of a workgroup): 2, 4 or 8.
+extern "C" int distie_attention_prefill_keys(const void* qkv, int64_t q_stride, const void* k_cache, const void* v_cache,
+                                             const int32_t* positions, const int32_t* cu_q, const int32_t* block_table,
+                                             int table_width, const int32_t* table_rows, void* out, int tokens, int num_requests,
+                                             int heads, int kv_heads, int block_size, float scale, int window, int min_q_len,
+                                             const float* sinks, int waves, hipStream_t stream) {
+  if (tokens <= 0) return 0;
+  if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || block_size < 16 || block_size % 16 != 0 || block_size > 65536 ||
+      table_width < 1 || num_requests < 1 || min_q_len < 1 || (waves != 2 && waves != 4 && waves != 8) || !(scale > 0.f))
+    return DISTIE_BAD_ARGUMENT;
+  const int64_t tiles = (static_cast<int64_t>(tokens) + KEYS_BM - 1) / KEYS_BM + num_requests;     // an upper bound; spare blocks leave at once
+  if (tiles > 65535) return DISTIE_BAD_ARGUMENT;
+  auto run = [&](auto kernel, int bytes) {
+    kernel<<<dim3(heads, static_cast<unsigned>(tiles)), DISTIE_WAVE * waves, bytes, stream>>>(
+        static_cast<const bf16_t*>(qkv), q_stride, static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache),
+        positions, cu_q, block_table, table_width, table_rows, static_cast<bf16_t*>(out), num_requests, heads, kv_heads,
+        block_size, scale, window, min_q_len, sinks);
+    return launch_status();
+  };
+  return waves == 8 ? run(attn_prefill_keys_kernel<8>, prefill_keys_lds<8>())
+                    : waves == 4 ? run(attn_prefill_keys_kernel<4>, prefill_keys_lds<4>())
+                                 : run(attn_prefill_keys_kernel<2>, prefill_keys_lds<2>());
+}
+#else
+extern "C" int distie_attention_prefill_keys_fits() { return 0; }
+extern "C" int distie_attention_prefill_keys(const void*, int64_t, const void*, const void*, const int32_t*, const int32_t*,
+                                             const int32_t*, int, const int32_t*, void*, int, int, int, int, int, float, int, int,
+                                             const float*, int, hipStream_t) {
+  return DISTIE_BAD_ARGUMENT;
+}
+#endif
+
+// ===================================================================================================
 //  * attn_prefill_f32: the tiled kernel in float32, for head sizes that are multiples of 32 up to 128. The same
 //    walk as attn_prefill (a workgroup of four waves owns 128 new tokens of one head, 32 query columns a wave,
 //    K and V^T tiles of 64 keys through LDS, the keys cut into parts that are merged) on the float32 products
@@ -2272,6 +2606,14 @@ extern "C" int distie_attention_decode_run_len(const int32_t*, int, int, int, in
 extern "C" int distie_attention_prefill_bf16(const void*, int64_t, const void*, const void*, const int32_t*, const int32_t*,
                                              const int32_t*, int, const int32_t*, void*, int, int, int, int, int, float, int, int,
                                              const int32_t*, void*, void*, int, const float*, hipStream_t) {
+  return DISTIE_BAD_ARGUMENT;
+}
+
+extern "C" int distie_attention_prefill_keys_fits() { return 0; }
+
+extern "C" int distie_attention_prefill_keys(const void*, int64_t, const void*, const void*, const int32_t*, const int32_t*,
+                                             const int32_t*, int, const int32_t*, void*, int, int, int, int, int, float, int, int,
+                                             const float*, int, hipStream_t) {
   return DISTIE_BAD_ARGUMENT;
 }
 

@@ -398,6 +398,27 @@ class HipOps(Ops):
     # 4,096 keys, 5 at 8,192, 8 from 16,384 on; the kernel takes up to 16)
     PREFILL_PARTS = ((1024, 3), (8192, 5), (16384, 8))
     PREFILL_WORKGROUPS = 512         # as many workgroups a short portion's attention should have, if its keys allow
+    # Heads of 64 and 128 in bfloat16 up to so many times the keys from which the tiled kernel's walk is cut (4,608 keys with up to 256
+    # workgroups of 32 tokens, 3,584 with more): the kernel whose waves share the columns and split the keys. Tiled with its merge /
+    # that one, us, 12 heads of 128: prompts of 40 tokens 6.4 / 5.7, 301 13.8 / 7.8, 1,024 27.9 / 14.2, 2,048 39.3 / 27.3, 3,500 78 /
+    # 64, 300 behind 4,000 36.0 / 27.8, 600 41 / 32; beyond, 28 heads, 600 behind 4,000 76 / 81, 1,500 147 / 156 (64 heads, 600: 129 /
+    # 149; heads of 64, 28 of them, 4,500 tokens 126 / 139); 12 heads, 128 behind 16,000 55 / 83
+    PREFILL_WAVES_REACH = ((256, 4.5), (None, 3.5))
+    # few tokens far behind are too few workgroups for either; the tiled kernel's parts are more: 64 behind 4,000 (16 heads) 23.2 /
+    # 26.0, 32 behind 3,000 (8 heads) 17.4 / 19.8, 32 behind 1,500 (12 heads) 18.4 / 13.1, 100 behind 3,000 30 / 20
+    PREFILL_WAVES_FEW = (96, 2560)
+    # many workgroups that all walk far (keys / tokens of a portion): the tiled kernel reads them for 128 tokens at once. 40 heads, 400 behind
+    # 3,100, 520 workgroups 55 / 66; 28 heads, 364 workgroups 46 / 44; 64 heads of 64, 1,000 behind 2,000, 2,048 75 / 81
+    PREFILL_WAVES_BEHIND = (480, 2560, 3)
+    # many workgroups and few keys: the tiled kernel reads a tile of keys once for 128 tokens and merges nothing (32 heads, 3 prompts
+    # of 667, 2,016 workgroups: 27.5 / 30.8; 28 heads, 4 of 512, 1,792 24.4 / 26.5; 64 heads, 2 of 1,000 55.9 / 67.4; 40 heads of 64, 6 of
+    # 130, 1,120 9.4 / 10.1)
+    PREFILL_WAVES_MANY = ((1700, 1024), (1024, 256))                     # from so many workgroups on, with fewer keys
+    # Waves of a workgroup, 8 / 4 / 2 (1, 2 or 4 workgroups a compute unit), us: 84 workgroups, 1,200 keys 12.5 / 14.4 / 22; 120 of 301
+    # keys 8.5 / 7.8 / 9.4; 240 of 640 9.8 / 10.0 / 13.9; 512 of 40 14.6 / 8.8 / 7.5; 560 of 640 20.5 / 13.3 / 15.4; 640 of 301 (64 heads)
+    # 19.4 / 14.2 / 10.7; 840 of 450 26 / 16.3 / 14.5; 812 of 901 29 / 20.5 / 20.5; 1,148 of 1,300 43 / 31.6 / 28.2; 1,792 of 2,048 76 /
+    # 58 / 50
+    PREFILL_WAVES = ((8, 256, 640), (4, 528, 65), (4, 576, 512), (4, 1024, 896), (4, 1400, 2560))    # waves, up to so many workgroups, from so many keys on
     PACKED_KEEPS_FREE = 0.3          # share of the device's memory that packed weight copies leave free
     PREFILL_F32_MIN_TOKENS = 32      # float32 steps with a portion of at least this many tokens go to the tiled float32 kernel
     # decode attention cuts the keys into runs so that about DECODE_WAVES waves are at work, with at most
@@ -622,6 +643,8 @@ class HipOps(Ops):
             lib.distie_attention_prefill_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I,
                                                           _F, _I, _I, _P, _P, _P, _I, _P, _P]
             lib.distie_attention_prefill_f32.argtypes = lib.distie_attention_prefill_bf16.argtypes
+            lib.distie_attention_prefill_keys.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I,
+                                                          _P, _I, _P]
             lib.distie_attention_decode_bf16.argtypes = [_P, _L, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I,
                                                          _I, _F, _I, _I, _I, _I, _P, _P, _I, _P]
             lib.distie_attention_decode_together.argtypes = [_I, _I, _I]
@@ -1577,8 +1600,8 @@ class HipOps(Ops):
             # with these sizes: worked out once per step (the layers run one after the other, so they can
             # share the buffers)
             key = ("attention", reach, num_heads, num_kv_heads, head_dim, meta.max_kv, meta.all_decode,
-                   meta.singles_bound, self.PREFILL_PARTS, self.PREFILL_WORKGROUPS, self.DECODE_WAVES, self.DECODE_MAX_RUNS,
-                   self.DECODE_SHARED_BELOW)
+                   meta.singles_bound, self.PREFILL_PARTS, self.PREFILL_WAVES_REACH, self.PREFILL_WORKGROUPS, self.DECODE_WAVES,
+                   self.DECODE_MAX_RUNS,                   self.DECODE_SHARED_BELOW)
             plan = meta.scratch.get(key)
             if plan is None or plan["cu_q"] is not meta.host_cu_q:
                 plan = meta.scratch[key] = self._attention_plan(lib, meta, T, num_heads, num_kv_heads, head_dim, abs(reach))
@@ -1591,7 +1614,13 @@ class HipOps(Ops):
                     plan["max_splits"], 1 if meta.all_decode else 0,
                     plan["run_len"].data_ptr() if plan["run_len"] is not None else None, sinks_ptr, plan["together"],
                     self._stream()), "attention_decode_bf16")
-            if plan["prefill"]:
+            if plan["prefill"] and plan["waves"]:
+                _check(lib.distie_attention_prefill_keys(
+                    qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
+                    meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
+                    num_heads, num_kv_heads, meta.block_size, float(scale), reach, 2 if plan["decode"] else 1, sinks_ptr,
+                    plan["waves"], self._stream()), "attention_prefill_keys")
+            elif plan["prefill"]:
                 parts = plan["parts"]
                 _check(lib.distie_attention_prefill_bf16(
                     qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
@@ -1797,8 +1826,31 @@ class HipOps(Ops):
         plan["prefill"] = singles < meta.num_requests or not plan["decode"] or \
             (meta.singles_bound is not None and not meta.all_decode)
         if plan["prefill"]:
-            plan.update(self._prefill_parts(meta, T, num_heads, head_dim, window))
+            plan["waves"] = self._prefill_waves(lib, meta, T, singles if plan["decode"] else 0, num_heads, window)
+            if not plan["waves"]:
+                plan.update(self._prefill_parts(meta, T, num_heads, head_dim, window))
         return plan
+
+    def _prefill_waves(self, lib, meta: BatchMeta, T, singles, num_heads, window) -> int:
+        """How many waves of a workgroup share a tile of 32 tokens of the portions of prompts and split its keys; 0: the tiled
+        kernel, whose waves share the keys."""
+        if not self.PREFILL_PARTS or not lib.distie_attention_prefill_keys_fits() or meta.block_size > 65536 or \
+                -(-T // 32) + meta.num_requests > 65535:
+            return 0
+        visible = min(meta.max_kv, int(window) + 32) if window else meta.max_kv
+        tokens, portions = max(1, T - singles), max(1, meta.num_requests - singles)
+        workgroups = num_heads * (-(-tokens // 32) + portions // 2)
+        many, far, times = self.PREFILL_WAVES_BEHIND
+        reach = next(reach for most, reach in self.PREFILL_WAVES_REACH if most is None or workgroups <= most)
+        if visible > reach * self.PREFILL_PARTS[0][0] or \
+                (tokens < self.PREFILL_WAVES_FEW[0] and visible > self.PREFILL_WAVES_FEW[1]) or \
+                (workgroups > many and visible > far and visible * portions >= times * tokens) or \
+                any(workgroups > least and visible < keys for least, keys in self.PREFILL_WAVES_MANY):
+            return 0
+        for waves, most, keys in self.PREFILL_WAVES:
+            if workgroups <= most and visible >= keys:
+                return waves
+        return 2
 
     def _prefill_parts(self, meta: BatchMeta, T, num_heads, head_dim, window) -> dict:
         """Into how many parts the tiled kernel cuts its walk over the keys, and the buffers between it and the

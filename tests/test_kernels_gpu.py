@@ -1315,6 +1315,46 @@ def test_float32_columns_keep_values_from_tokens_that_do_not_see_them(ops, heads
     assert not torch.isfinite(got[sees]).any()
 
 
+@pytest.mark.parametrize("waves", [2, 4, 8])
+@pytest.mark.parametrize("heads,kv_heads,dim,P,reach", [(6, 2, 128, 16, 0), (3, 3, 64, 48, 0), (4, 1, 128, 64, 37), (2, 2, 64, 16, -48),
+                                                        (3, 1, 128, 32, 300)])
+def test_portions_whose_keys_the_waves_of_a_workgroup_share(ops, heads, kv_heads, dim, P, reach, waves, monkeypatch):
+    """Tiles of 32 tokens and of 32 keys a wave: portions that end one before, at and one past a tile, of one and two tokens, with
+    keys for no, one, some and all waves, windows and chunks that begin inside a tile, sinks, tables in another order, and what the
+    keys behind the last one are (not a number) reaches nobody. Against plain attention, as the tiled kernel, which takes the same
+    step; that one and this differ by no more than twice that."""
+    from distie_amd.kernels.interface import ScoreExtras
+
+    lens = [31, 32, 33, 1, 64, 300, 257, 520, 66, 129]
+    q_lens = [31, 32, 33, 1, 2, 300, 64, 65, 1, 95]
+    meta, qkv, k, v = paged_case(heads, kv_heads, dim, P, lens, q_lens, torch.bfloat16, seed=17)
+    table = meta.groups[0].block_table
+    for b, n in enumerate(lens):
+        if n % P:
+            k[table[b, n // P], :, n % P:] = math.nan
+            v[table[b, n // P], :, :, n % P:] = math.nan
+    finite_k, finite_v = k.double().nan_to_num(), v.double().nan_to_num()
+    order = torch.randperm(len(lens), generator=torch.Generator().manual_seed(1))
+    window, chunk = (reach or None, 0) if reach >= 0 else (None, -reach)
+    for sinks, cu_q in ((None, meta.host_cu_q), (torch.randn(heads, device="cuda"), None)):       # None: single tokens as well
+        extras = ScoreExtras(sinks=sinks, chunk=chunk) if sinks is not None or chunk else None
+        want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, finite_k, finite_v, heads, kv_heads, dim, dim ** -0.5, window,
+                                                extras)
+        meta.host_cu_q = cu_q
+        meta.groups[0].block_table, meta.table_rows = table[order].contiguous(), order.argsort().int().cuda()
+        results = []
+        for form in (((waves, 1 << 30, 0),), ()):
+            monkeypatch.setattr(type(ops), "PREFILL_WAVES", form)
+            monkeypatch.setattr(type(ops), "PREFILL_WAVES_REACH", ((None, 4.5 if form else 0.0),))
+            meta.scratch.clear()
+            results.append(ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, dim, dim ** -0.5, window, extras))
+            plan, = (p for p in meta.scratch.values() if isinstance(p, dict) and "waves" in p)
+            assert plan["waves"] == (waves if form else 0)
+            close(results[-1], want, torch.bfloat16, scale=want.abs().max().item())
+        close(results[0], results[1], torch.bfloat16, scale=2 * want.abs().max().item())
+        meta.groups[0].block_table, meta.table_rows = table, None
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
                                                                   (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8),
                                                                   (12, 2, 128, 16, None, 4), (8, 2, 64, 16, 4500, 4)])
