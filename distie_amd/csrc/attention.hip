@@ -13,7 +13,7 @@
 // Formula: worker/src/inference/qwen2/model.py:154-161; softmax and all sums in float32.
 //
 //  * attn_generic: one wave per (token, head); any types; the true 32-bit path and the fallback.
-//  * attn_decode + attn_reduce, attn_prefill: bfloat16 on the matrix cores (described further down).
+//  * attn_decode + attn_reduce, attn_prefill, attn_prefill_keys: bfloat16 on the matrix cores (described further down).
 
 #include "common.h"
 #include "lds_load.h"

@@ -392,6 +392,7 @@ void layer_chain_kernel(const Chain given) {
       for (int i = 0; i < ROWS / HELP; ++i) {
         const int m = helper + HELP * i;
         if (m < M) {
+          // (vectors are cast whole: the cast of an element gave element 0 for each of them)
           float ss = 0.f;
 #pragma unroll
           for (int e = 0; e < T; ++e) {
