@@ -9,8 +9,8 @@ Five kinds of shared library, all built from the sources beside this file:
   kernels for multiples of 16 up to 256, the wave-per-token kernel for every even size up to 1024);
 * `mixattn_d<D>` - the matrix-core kernels of attention with mixed heads for head size D (a multiple of 32 up to 256).
 
-A library's file name carries a hash of its sources and flags, so a stale build is never
-loaded. Libraries live in `distie_amd/_lib/` (in-tree); if that folder cannot be written,
+A library's file name carries a hash of its sources, of the headers beside them that these include, and of the
+flags, so a stale build is never loaded. Libraries live in `distie_amd/_lib/` (in-tree); if that folder cannot be written,
 in a per-user folder under the temporary directory. `ensure(name)` returns the path and
 compiles first if the file is not there, printing a line when it starts and every few
 seconds while it waits, so a first call in a fresh checkout shows progress.
@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -43,8 +44,6 @@ ATTN_SOURCES = ["attention.hip"]
 MIXED_ATTN_SOURCES = ["mixed_attention_mc.hip"]
 LIBRARY_SOURCES = ["library_products.hip"]
 LINK_LIBS = {"library": ["-lhipblaslt"]}
-HEADERS = ["common.h"]
-OPS_HEADERS = ["lds_load.h", "no_alloc.h", "packed.h", "vector_values.h"]
 
 
 class BuildError(RuntimeError):
@@ -55,14 +54,21 @@ def _say(text: str) -> None:
     print(f"[distie_amd] {text}", file=sys.stderr, flush=True)
 
 
+def _with_headers(files: List[str]) -> List[str]:
+    """`files` and every file of this folder that they include, directly or through one another."""
+    found = list(files)
+    for name in found:                              # (grows while it is walked)
+        for include in re.findall(r'^[ \t]*#[ \t]*include[ \t]*"([^"]+)"', (SRC / name).read_text(), re.MULTILINE):
+            if include not in found and (SRC / include).is_file():
+                found.append(include)
+    return found
+
+
 def _hash(files: List[str], flags: List[str]) -> str:
     h = hashlib.sha256()
-    headers = HEADERS + (OPS_HEADERS if files == OPS_SOURCES else [])
-    for name in files + headers:
-        path = SRC / name
-        if path.is_file():
-            h.update(name.encode())
-            h.update(path.read_bytes())
+    for name in _with_headers(files):
+        h.update(name.encode())
+        h.update((SRC / name).read_bytes())
     h.update(" ".join(flags).encode())
     return h.hexdigest()[:10]
 
