@@ -343,19 +343,20 @@ __device__ __forceinline__ void run_scores(const float r[DP / 4], const float k[
   }
 }
 
-// Heads of up to 64: the state in front of the chunk waits in registers and takes the place of Kt in LDS when that has been
-// read, 35 KB instead of 51, and with 128 registers a lane four workgroups fit a compute unit instead of three: 960 of them (2 prompts
-// of 901, 32 heads) 50.4 -> 45.9 us, the same bits (with 130 registers and three of them 50.9).
-template <int DP>
-constexpr bool WK_LATE = DP <= 64;
-template <int DP>
+// LATE (heads of up to 64, more than WK_EARLY_WORKGROUPS workgroups): the state in front of the chunk waits in registers and takes
+// the place of Kt in LDS when that has been read, 35 KB instead of 51, and with 128 registers a lane four workgroups fit a compute unit
+// instead of three: 960 of them (2 prompts of 901, 32 heads) 50.4 -> 45.9 us, the same bits (with 130 registers and three of them 50.9).
+// Workgroups that all fit as they are gain nothing from it and wait for the state at the end instead: 16 of 20 rows 15.3 -> 16.7 us.
+// (The whole operation, early / late: 32 heads, 768 workgroups of 30 rows 85.1 / 86.0 us, 832 of them 94.8 / 92.3.)
+constexpr int WK_EARLY_WORKGROUPS = 3 * 256;
+template <int DP, bool LATE>
 constexpr int wk_shared() {
   const int k = WK_ROWS * DP, s = DP * DP;
-  return WK_LATE<DP> ? (k > s ? k : s) : k + s;
+  return LATE ? (k > s ? k : s) : k + s;
 }
 
-template <int DP, typename X, typename O>
-__global__ void __launch_bounds__(256, WK_LATE<DP> ? 4 : 2)
+template <int DP, bool LATE, typename X, typename O>
+__global__ void __launch_bounds__(256, LATE ? 4 : 2)
 wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in, const X* __restrict__ v_in,
                          const X* __restrict__ gates, int64_t ld, const float* __restrict__ z, const float* __restrict__ bonus,
                          const float* __restrict__ scratch, const float* __restrict__ norm_weight, float eps,
@@ -364,8 +365,8 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float* Vs = lds;                                  // [64][DP + 4]
   float* Kt = Vs + WK_ROWS * STRIDE;                // [4 runs][DL / 4][64 lanes][4]: k_j exp(the run's decay behind j)
-  float* Ss = WK_LATE<DP> ? Kt : Kt + WK_ROWS * DP; // [DP][DP], the columns of row d turned by 16 (d / DL) places
-  float* factor = Kt + wk_shared<DP>();             // [4][DP]: the runs' total factors
+  float* Ss = LATE ? Kt : Kt + WK_ROWS * DP;        // [DP][DP], the columns of row d turned by 16 (d / DL) places
+  float* factor = Kt + wk_shared<DP, LATE>();       // [4][DP]: the runs' total factors
   const int head = blockIdx.y;
   const int4 chunk = chunks[blockIdx.x];
   const int64_t row0 = chunk.y;
@@ -379,7 +380,7 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
   stage_rows<DP>(v_in + row0 * ld + head * D, ld, len, D, whole, Vs);
   const float* src = scratch + (static_cast<int64_t>(blockIdx.x) * H + head) * D * D;
   constexpr int PIECES = (DP * DP / 4 + 255) / 256; // of S, a thread's
-  float held[WK_LATE<DP> ? PIECES : 1][4];
+  float held[LATE ? PIECES : 1][4];
   auto load_state = [&](int idx, float v[4]) __attribute__((always_inline)) {
     const int d = idx / (DP / 4), e = idx % (DP / 4) * 4;
 #pragma unroll
@@ -396,7 +397,7 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
     const int d = idx / (DP / 4), e = idx % (DP / 4) * 4;
     if (DP * DP / 4 % 256 == 0 || d < DP) store_values<4>(Ss + d * DP + (e + 16 * (d / DL)) % DP, v);
   };
-  if constexpr (WK_LATE<DP>) {
+  if constexpr (LATE) {
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) load_state(threadIdx.x + 256 * p, held[p]);
   } else {
@@ -457,7 +458,7 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
 #pragma unroll
     for (int s = 0; s < DL; ++s) r[s] *= factor[before * DP + DL * g + s];
   }
-  if constexpr (WK_LATE<DP>) {
+  if constexpr (LATE) {
     __syncthreads();                                // every run has read Kt
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) stage_state(threadIdx.x + 256 * p, held[p]);
@@ -571,11 +572,13 @@ extern "C" int distie_wkv_scan_chunked(const void* r, const void* k, const void*
   int status = 0;
 #define DISTIE_WKV_CHUNKS(DP)                                                                                            \
   DISTIE_DISPATCH(dtype, X, DISTIE_DISPATCH(out_dtype, O, {                                                              \
-    constexpr int LDS = (WK_ROWS * (DP + 4) + wk_shared<DP>() + 4 * DP) * static_cast<int>(sizeof(float));               \
+    const bool late = DP <= 64 && static_cast<int64_t>(num_chunks) * H > WK_EARLY_WORKGROUPS;                            \
+    const auto outputs = late ? wkv_chunk_outputs_kernel<DP, DP <= 64, X, O> : wkv_chunk_outputs_kernel<DP, false, X, O>;\
+    const int shared = late ? wk_shared<DP, true>() : wk_shared<DP, false>();                                            \
+    const int bytes = (WK_ROWS * (DP + 4) + shared + 4 * DP) * static_cast<int>(sizeof(float));                          \
     const int whole = vectors && D == DP ? 1 : 0;                                                                        \
-    if (LDS > 48 * 1024 &&                                                                                               \
-        hipFuncSetAttribute(reinterpret_cast<const void*>(wkv_chunk_outputs_kernel<DP, X, O>),                           \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)                              \
+    if (bytes > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(outputs),                                 \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)       \
       return DISTIE_BAD_ARGUMENT;                                                                                        \
     wkv_chunk_sums_kernel<DP, X><<<grid, 256, 0, stream>>>(static_cast<const X*>(k), static_cast<const X*>(v), ld, z,    \
                                                            scratch, totals, table, H, D, whole);                         \
@@ -583,7 +586,7 @@ extern "C" int distie_wkv_scan_chunked(const void* r, const void* k, const void*
     wkv_chunk_states_kernel<<<dim3(B, H, (D * D + 255) / 256), 256, 0, stream>>>(scratch, totals, state, request_chunks, \
                                                                                 state_slots, H, D);                      \
     if ((status = launch_status()) != 0) return status;                                                                  \
-    wkv_chunk_outputs_kernel<DP, X, O><<<grid, 256, LDS, stream>>>(                                                      \
+    outputs<<<grid, 256, bytes, stream>>>(                                                                               \
         static_cast<const X*>(r), static_cast<const X*>(k), static_cast<const X*>(v), static_cast<const X*>(gates), ld,  \
         z, bonus, scratch, norm_weight, eps, static_cast<O*>(out), table, H, D, whole);                                  \
   }))

@@ -1355,6 +1355,35 @@ def test_portions_whose_keys_the_waves_of_a_workgroup_share(ops, heads, kv_heads
         meta.groups[0].block_table, meta.table_rows = table, None
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim", [8, 33, 48, 64])
+def test_time_mixing_in_chunks_does_not_hang_on_how_many_there_are(ops, dim, dtype):
+    """Up to three workgroups a compute unit the state in front of a chunk has a place of its own in LDS, beyond it takes that of the
+    keys: 160 and 768 workgroups of the one form and 800 of the other. The same requests, over and over: the same bits."""
+    heads, rank, lens = 40, 5, [70, 20, 64]
+    N, copies = heads * dim, 5
+    r, k, v, gates = (rand(sum(lens), N, dtype=dtype, seed=i) for i in range(4))
+    low, up, bias = rand(sum(lens), rank, seed=5), rand(N, rank, seed=6, scale=0.3), rand(N, seed=7, scale=0.3)
+    bonus, weight, first = rand(N, seed=8), rand(N, seed=9) * 0.2 + 1, rand(len(lens), heads, dim, dim, seed=10)
+
+    def run(times, h=heads):
+        q = lens * times
+        cu_q = np.concatenate([[0], np.cumsum(q)]).tolist()
+        meta = make_meta([0] * cu_q[-1], [0] * cu_q[-1], cu_q, q, [[0]] * len(q), [0] * cu_q[-1], 16)
+        meta.state_slots = torch.arange(len(q), dtype=torch.int32, device="cuda")
+        state, n = first[:, :h].repeat(times, 1, 1, 1).contiguous(), h * dim
+        rows = [t[:, :n].repeat(times, 1).contiguous() for t in (r, k, v, gates)]
+        out = ops.wkv_mix(*rows, low.repeat(times, 1), up[:n].contiguous(), bias[:n].contiguous(), bonus[:n].contiguous(), state, meta,
+                          h, dim, weight[:n].contiguous(), 1e-5, torch.float32)
+        return out.view(times, sum(lens), n), state.view(times, len(lens), h, dim, dim)
+
+    for times, h in ((6, 32), (copies, heads)):          # 4 chunks a copy: 768 workgroups, 800
+        want, moved = run(1, h)
+        assert torch.isfinite(want).all() and not torch.equal(moved[0], first[:, :h])
+        out, states = run(times, h)
+        assert all(torch.equal(o, want[0]) and torch.equal(s, moved[0]) for o, s in zip(out, states))
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,P,window,together", [(12, 2, 128, 16, None, 8), (16, 1, 128, 32, 4300, 4),
                                                                   (3, 3, 256, 16, None, 4), (7, 1, 48, 16, 5000, 8),
                                                                   (12, 2, 128, 16, None, 4), (8, 2, 64, 16, 4500, 4)])
