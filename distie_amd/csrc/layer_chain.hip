@@ -97,6 +97,9 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t uintx4;
 extern "C" __device__ uintx4 chain_buffer_load(intx4 from, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.load.v4i32");
 constexpr int DEVICE_SCOPE = 16;          // sc1
 __device__ __forceinline__ uintx4 load_shared(const intx4& from, int at) { return chain_buffer_load(from, at, 0, DEVICE_SCOPE); }
+// In front of every look for what may not be there yet. The load is declared to read memory and do nothing else: a loop that does not
+// say that memory changes could be given the first look's answer for ever.
+__device__ __forceinline__ void look_again() { asm volatile("" ::: "memory"); }
 __device__ __forceinline__ bool unwritten(const uintx4& v) {
   return v[0] == UNWRITTEN || v[1] == UNWRITTEN || v[2] == UNWRITTEN || v[3] == UNWRITTEN;
 }
@@ -241,6 +244,7 @@ void layer_chain_kernel(const Chain given) {
         uintx4 x[B][G];
         int tries = args->patience;
         for (;;) {
+          look_again();
           bool missing = false;
 #pragma unroll
           for (int b = 0; b < B; ++b) {
@@ -375,6 +379,7 @@ void layer_chain_kernel(const Chain given) {
       int tries = args->patience;
       bool missing;
       do {
+        look_again();
 #pragma unroll
         for (int i = 0; i < ROWS / HELP; ++i) {
           const int m = helper + HELP * i, at = (m < M ? m * C * 4 : OUTSIDE) + 16 * lane;
@@ -452,16 +457,21 @@ void layer_chain_kernel(const Chain given) {
       }
       continue;
     }
-    // What a sum is added to, asked for while the product is under way. (It was complete before x was, since whoever wrote x had
-    // read all of it: the look is for the letter.)
+    // What a sum is added to, asked for while the product is under way. It was complete before x was, since whoever wrote x had
+    // read all of it: the first look finds it. (A word that `limit` looks did not find is added as the NaN that it holds.)
     void* const to = args->phase[q].to;
+    auto added_to = [&](int at) __attribute__((always_inline)) {
+      uintx4 v;
+      int tries = args->limit;
+      do {
+        look_again();
+        v = load_shared(from, at);
+      } while (q > 0 && unwritten(v) && --tries > 0);
+      return v;
+    };
     uintx4 old = {};
     int k = helper * 4 + lane / 16;
-    if (kind == KIND_SUM && k < n && r < M) {
-      do {
-        old = load_shared(from, (r * C + 8 * (u0 + k) + 4 * g) * 4);
-      } while (q > 0 && unwritten(old));
-    }
+    if (kind == KIND_SUM && k < n && r < M) old = added_to((r * C + 8 * (u0 + k) + 4 * g) * 4);
     lds_barrier();                                               // (5): the parts of the sums are in LDS
     for (; k < n; k += HELP * 4) {
       const int u = u0 + k;
@@ -484,10 +494,7 @@ void layer_chain_kernel(const Chain given) {
         }
         if (kind == KIND_SUM) {
           const int at = r * C + 8 * u + 4 * g;
-          while (k >= HELP * 4) {
-            old = load_shared(from, at * 4);
-            if (q == 0 || !unwritten(old)) break;
-          }
+          if (k >= HELP * 4) old = added_to(at * 4);
           const float4 sum = __builtin_bit_cast(float4, old);
           store_shared(static_cast<float*>(to) + at, __builtin_bit_cast(uint32_t, sum.x + (near[0] + far[0])),
                        __builtin_bit_cast(uint32_t, sum.y + (near[1] + far[1])));

@@ -2,6 +2,7 @@
 does not name, m0 and the condition codes among them."""
 
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -61,3 +62,20 @@ def test_the_check_sees_an_undeclared_register():
     text = 'asm volatile("s_mov_b32 m0, %0\\n\\ts_nop 0\\n\\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(p) : "memory"MORE);'
     assert [target for _, target in undeclared(text.replace("MORE", ""))] == ["m0"]
     assert undeclared(text.replace("MORE", ', "m0"')) == []
+
+
+def test_what_other_workgroups_write_is_looked_for_in_memory_each_time(tmp_path):
+    """In the compiler's own terms: wherever the kernel asks for such words, the same stretch of code says that memory may have
+    changed, so that no look stands for the next one."""
+    from distie_amd.csrc import build
+
+    out = tmp_path / "layer_chain.ll"
+    subprocess.run([build._hipcc(), *build.HIP_FLAGS, "-x", "hip", "--offload-device-only", "-emit-llvm", "-S",
+                    str(CSRC / "layer_chain.hip"), "-o", str(out)], check=True, capture_output=True)
+    kernels = [body[:body.index("\n}")] for body in re.split(r"^define ", out.read_text(), flags=re.MULTILINE)[1:]
+               if "layer_chain_kernel" in body.split("\n", 1)[0]]
+    assert len(kernels) == 6
+    for body in kernels:
+        blocks = [b for b in re.split(r"^\d+:.*\n", body, flags=re.MULTILINE) if "call" in b and "llvm.amdgcn.raw.buffer.load" in b]
+        assert len(blocks) >= 4                        # x of a sum, x of a norm, and twice what a sum is added to
+        assert all('asm sideeffect "", "~{memory}"' in b[:b.index("llvm.amdgcn.raw.buffer.load")] for b in blocks)
