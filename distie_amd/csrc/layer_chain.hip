@@ -27,7 +27,8 @@
 // incomplete for `patience` looks takes, of the earliest phase that has any, a slot that nobody has claimed, works on it as on its own,
 // and then goes on. The earliest phase that is not complete consists of slots claimed by running workgroups, whose x is complete, and of
 // unclaimed ones, which the first to lose its patience takes: some workgroup always gets on, whatever else runs on the device.
-// (`limit` rounds of that without an end are never reached; a workgroup that reached them would write NaN and leave.)
+// (`limit` rounds of that without an end are never reached; a workgroup that reached them would write NaN, say so in `gave_up`, which
+// the host reads with the step's result, and leave.)
 #include "lds_load.h"
 #include "packed.h"
 #include <algorithm>
@@ -62,6 +63,7 @@ struct Chain {
   const float* bias;
   RotaryOut rotary;
   int32_t* claims;                        // [phase][slot], UNWRITTEN: nobody's
+  int32_t* gave_up;                       // in host memory: 1 once a wait came to its end without what it was for
   int M, I, NQ, phases, slots, patience, limit;
 };
 
@@ -108,6 +110,8 @@ __device__ __forceinline__ void store_shared(void* p, uint32_t a, uint32_t b) {
   __hip_atomic_store(static_cast<uint64_t*>(p), static_cast<uint64_t>(written(a)) | (static_cast<uint64_t>(written(b)) << 32),
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+__device__ __forceinline__ void give_up(int32_t* flag) { __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 
 // T: tiles of C a wave; G: tiles of a group, which are asked for together; R: groups of a wave's ring; B: groups of x a wave keeps (sums)
 template <int T, int G, int R, int B>
@@ -450,6 +454,7 @@ void layer_chain_kernel(const Chain given) {
       lds_barrier();                                             // (4): job[2]: deeper, the same again, or given up
       depth = __builtin_amdgcn_readfirstlane(job[2]);
       if (depth < 0) {
+        if (helper == 0 && lane == 0) give_up(args->gave_up);
         if (helper == 0)
           for (int i = lane; i < M * 8; i += 64)
             if (8 * own < C) static_cast<float*>(args->phase[2].to)[(i / 8) * C + 8 * own + i % 8] = __builtin_nanf("");
@@ -467,6 +472,7 @@ void layer_chain_kernel(const Chain given) {
         look_again();
         v = load_shared(from, at);
       } while (q > 0 && unwritten(v) && --tries > 0);
+      if (tries == 0) give_up(args->gave_up);
       return v;
     };
     uintx4 old = {};
@@ -598,15 +604,17 @@ extern "C" int distie_layer_chain_claims(int slots) { return MAX_PHASES * slots;
 
 // mid, out: float32 [M, C], hidden: bfloat16 [M, I], claims: all of them UNWRITTEN (bytes of 0xff) when the launch begins, each at a
 // multiple of 16 bytes. qkv_w null: no layer follows. grid: workgroups (`slots`. With fewer, to try what they do for others, the
-// last phase keeps its holes: nobody waits for it, it is left to those who start late).
+// last phase keeps its holes: nobody waits for it, it is left to those who start late). gave_up: host memory that the device writes.
 extern "C" int distie_layer_chain(const void* mixed, const void* o_w, const float* residual, float* mid, const float* norm, float eps,
                                   const void* gate_up_w, void* hidden, const void* down_w, float* out, const float* next_norm,
                                   float next_eps, const void* qkv_w, const float* bias, void* qkv, const void* table,
                                   const int32_t* cache_slots, void* k_cache, void* v_cache, int heads, int kv_heads, int dim,
-                                  int block_size, int write, int M, int C, int KO, int I, int32_t* claims, int slots, int grid,
-                                  int patience, int limit, hipStream_t stream) {
+                                  int block_size, int write, int M, int C, int KO, int I, int32_t* claims, int32_t* gave_up, int slots,
+                                  int grid, int patience, int limit, hipStream_t stream) {
   const int NQ = qkv_w != nullptr ? (heads + 2 * kv_heads) * dim : 0;
-  if (!distie_layer_chain_fits(M, C, KO, I, NQ, slots) || grid < 1 || grid > slots || patience < 1 || limit < 1) return DISTIE_BAD_ARGUMENT;
+  if (!distie_layer_chain_fits(M, C, KO, I, NQ, slots) || grid < 1 || grid > slots || patience < 1 || limit < 1 ||
+      gave_up == nullptr)
+    return DISTIE_BAD_ARGUMENT;
   if (qkv_w != nullptr && (heads < 1 || kv_heads < 1 || dim < 16 || dim % 16 || block_size < 1)) return DISTIE_BAD_ARGUMENT;
   Chain a = {};
   a.phases = qkv_w != nullptr ? 4 : 3;
@@ -635,6 +643,7 @@ extern "C" int distie_layer_chain(const void* mixed, const void* o_w, const floa
   a.rotary = RotaryOut{static_cast<const float2*>(table), cache_slots, static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache),
                        heads, kv_heads, dim, block_size, write, 0, 0.f, 1.f, 0.f};
   a.claims = claims;
+  a.gave_up = gave_up;
   a.M = M;
   a.I = I;
   a.NQ = NQ;

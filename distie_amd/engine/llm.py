@@ -179,7 +179,9 @@ class LLM:
     # ------------------------------------------------------------ the step function
     def step(self, entries: Seq[StepEntry]) -> Optional[torch.Tensor]:
         """Run the given tokens of the given requests as one batch; float32 logits at the wanted
-        places. Requests are created at their first step; `finish` gives back what they hold."""
+        places. Requests are created at their first step; `finish` gives back what they hold. Raises if a step before this
+        one turns out not to have finished its work."""
+        self.ops.raise_failures()
         return self.runner.step(entries)
 
     def finish(self, request_id) -> None:
@@ -267,6 +269,7 @@ class LLM:
                 if self.engine_config.lookahead:
                     self._launch_ahead(plan, chosen)
                 tokens = iter(fetch())
+                self.ops.raise_failures()
                 drawn = [next(tokens) if p.samples else None for p in plan.portions]
         except Exception as exc:  # noqa: BLE001 - every request of the step learns of it
             _log.exception("step failed; its %d requests end with the error", len(plan.portions))
@@ -425,6 +428,7 @@ class LLM:
             while len(chosen) < max_new_tokens:
                 row = self.runner.step([StepEntry(name, feed, [len(feed) - 1])])
                 greedy = int(self.ops.argmax(row)[0])
+                self.ops.raise_failures()
                 kept[len(chosen)].copy_(row[0])
                 chosen.append(greedy)
                 if forced is None and greedy in self.eos_ids:

@@ -488,6 +488,9 @@ class HipOps(Ops):
         # pinned staging buffers for `upload`, used in turn: [host tensor, its numpy view, event of the last copy]
         self._uploads = [[None, None, None] for _ in range(self.UPLOAD_BUFFERS)]
         self._next_upload = 0
+        # what a kernel whose workgroups wait for one another writes if a wait came to its end (`raise_failures`)
+        self._gave_up = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._gave_up_np = self._gave_up.numpy()
 
     # ------------------------------------------------------------ plumbing
     UPLOAD_BUFFERS = 8
@@ -556,7 +559,7 @@ class HipOps(Ops):
         o.distie_layer_chain_fits.argtypes = [_I, _I, _I, _I, _I, _I]
         o.distie_layer_chain_claims.argtypes = [_I]
         o.distie_layer_chain.argtypes = [_P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P] + 9 * [_I] + \
-            [_P, _I, _I, _I, _I, _P]
+            [_P, _P, _I, _I, _I, _I, _P]
         o.distie_hyper_step.argtypes = [_P, _I, _P, _P, _I, _I, _P, _I, _L, _I, _P, _P, _P, _P, _I, _I, _F, _P, _I, _I, _I, _P]
         o.distie_causal_conv.argtypes = [_P, _I, _L, _P, _I, _I, _P, _P, _I, _L, _I, _P, _P, _P, _P, _I, _I, _P]
         o.distie_conv_state.argtypes = [_P, _I, _L, _I, _P, _P, _P, _I, _I, _I, _P]
@@ -778,6 +781,12 @@ class HipOps(Ops):
             M, N, K, self._stream()), "decode_product_residual")
         _mark_written(residual)
 
+    def raise_failures(self):
+        if self._gave_up_np[0]:
+            self._gave_up_np[0] = 0
+            raise KernelError("layer_chain: a workgroup waited in vain for another one's values; what the steps since the last "
+                              "look computed is void")
+
     # ---- a layer's end and the next one's beginning in one launch
     def _chain_fits(self, M, C, KO, inter, N) -> bool:
         return bool(self._ops.distie_layer_chain_fits(M, C, KO, inter, N, self._compute_units))
@@ -834,7 +843,7 @@ class HipOps(Ops):
             tail.mixed.data_ptr(), out_weight._distie_packed.data_ptr(), tail.residual.data_ptr(), mid.data_ptr(),
             self._f32(norm_weight).data_ptr(), eps, gate_up_weight._distie_gated.data_ptr(), hidden.data_ptr(),
             down_weight._distie_packed.data_ptr(), out.data_ptr(), ptr(next_norm), next_eps, ptr(packed), ptr(bias), ptr(qkv), *rest,
-            M, C, KO, inter, claims.data_ptr(), self._compute_units, self.CHAIN_WORKGROUPS or self._compute_units,
+            M, C, KO, inter, claims.data_ptr(), self._gave_up.data_ptr(), self._compute_units, self.CHAIN_WORKGROUPS or self._compute_units,
             self.CHAIN_PATIENCE, self.CHAIN_LIMIT, self._stream()), "layer_chain")
         return out.view(torch.float32).view(M, C), qkv
 

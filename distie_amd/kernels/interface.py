@@ -136,6 +136,10 @@ class Ops(abc.ABC):
         shape. An implementation makes this a copy that does not wait for the work queued before it."""
         return torch.from_numpy(np.ascontiguousarray(values)).to(self.device)
 
+    def raise_failures(self) -> None:
+        """Raise, once, if a kernel reported since the last call that it could not finish its work. The report of what the host has
+        waited for has arrived; of work that is still queued it may arrive later."""
+
     def scatter_int32(self, table: torch.Tensor, index: torch.Tensor, value: torch.Tensor) -> None:
         """table.view(-1)[index] = value for int32 tensors on the device (distinct indexes): the block tables'
         changed entries of a step."""

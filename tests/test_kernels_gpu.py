@@ -744,6 +744,46 @@ def test_a_layers_end_and_the_next_ones_beginning_in_one_launch(ops, M, C, I, he
     assert ops.layer_tail(new_meta(), residual, mixed, w_o, norm, eps, w_gu, w_d) is None       # launched kernel by kernel
 
 
+@pytest.mark.parametrize("M,C", [(1, 1024), (8, 1536), (2, 2048)])
+@pytest.mark.parametrize("workgroups", [1, 40, None])
+def test_a_chain_that_gives_up_says_so(ops, M, C, workgroups):
+    """One round of one look: a workgroup whose values are not there at once gives up, as no launch does that may wait longer. Every
+    workgroup leaves, and the host learns of it, once."""
+    heads, dim, inter, bf = C // 128, 128, 2816, torch.bfloat16
+    mixed, residual, norm = rand(M, C, dtype=bf, seed=1), rand(M, C, seed=2), rand(C, seed=7)
+    w_o, w_gu, w_d = (rand(n, k, dtype=bf, seed=n, scale=k ** -0.5) for n, k in ((C, C), (2 * inter, C), (C, inter)))
+    w_qkv = rand((heads + 2) * dim, C, dtype=bf, seed=6, scale=C ** -0.5)
+    for weight, kinds in ((w_o, {}), (w_gu, {"gated": True}), (w_d, {}), (w_qkv, {"rotary": (heads, 1, dim)})):
+        ops.prepare_linear(weight, **kinds)
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, dim, 2, dtype=torch.float32) / dim))).cuda()
+    k, v = (torch.zeros(M, 1, *shape, dtype=bf, device="cuda") for shape in ((8, dim), (dim, 8)))
+
+    def run():
+        meta = make_meta([0] * M, list(range(M)), list(range(M + 1)), [1] * M, [[0]] * M, [8 * i for i in range(M)], 8)
+        tail = ops.layer_tail(meta, residual, mixed, w_o, norm, 1e-5, w_gu, w_d)
+        hidden, qkv = tail.finish_into(norm, 1e-5, w_qkv, None, meta, 0, k, v, inv_freq, heads, 1, dim, True)
+        torch.cuda.synchronize()
+        return hidden
+
+    ops.captured = True
+    try:
+        want = run()
+        ops.raise_failures()
+        ops.CHAIN_WORKGROUPS, ops.CHAIN_PATIENCE, ops.CHAIN_LIMIT = workgroups, 1, 1
+        hidden = run()
+        with pytest.raises(RuntimeError, match="in vain"):
+            ops.raise_failures()
+        ops.raise_failures()
+        assert hidden.isnan().any(dim=1).all()
+        del ops.CHAIN_WORKGROUPS, ops.CHAIN_PATIENCE, ops.CHAIN_LIMIT
+        assert torch.equal(run(), want)
+        ops.raise_failures()
+    finally:
+        ops.captured = False
+        for name in ("CHAIN_WORKGROUPS", "CHAIN_PATIENCE", "CHAIN_LIMIT"):
+            ops.__dict__.pop(name, None)
+
+
 @pytest.mark.parametrize("M", [1, 5, 8, 9, 16])
 @pytest.mark.parametrize("C,I,heads,kv_heads,dim", [(1536, 4484, 12, 2, 128), (72, 13, 3, 1, 16), (3584, 300, 4, 4, 48),
                                                     (4096, 88, 2, 1, 80), (264, 172, 5, 5, 32)])

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import plain_qwen2 as plain
-from distie_amd import LLM, SamplingParams
+from distie_amd import LLM, SamplingParams, StepEntry
 from engine_util import check_generation, make_model_dir, oracle, plain_uniform, random_ids
 from torch_ops import TorchOps
 
@@ -102,6 +102,36 @@ def test_request_larger_than_the_pool(tiny):
     llm = engine(folder, num_blocks=2)
     with pytest.raises(RuntimeError, match="out of KV blocks"):
         llm.generate([random_ids(cfg, 30, 6)], SamplingParams(max_new_tokens=4))
+
+
+def test_work_that_a_kernel_reports_as_not_done_is_not_taken_for_done(tiny):
+    """`raise_failures` raises after the tokens have been fetched: no token of that step is handed out, its requests end with the
+    error, and the engine goes on. The bare step function and a trace raise."""
+    cfg, folder, weights = tiny
+
+    class Reporting(TorchOps):
+        left = 3
+
+        def raise_failures(self):
+            self.left -= 1
+            if self.left == 0:
+                raise RuntimeError("a kernel gave up")
+
+    prompt = random_ids(cfg, 9, 1)
+    llm = LLM(folder, dtype="fp32", ops=Reporting(), block_size=8, num_blocks=64, lookahead=False)
+    out = llm.generate([prompt], SamplingParams(max_new_tokens=8))[0]
+    assert out.finish_reason == "error" and "gave up" in out.error
+    assert out.token_ids == plain_greedy(weights, cfg, prompt, 8)[:2]
+    assert llm.generate([prompt], SamplingParams(max_new_tokens=8))[0].token_ids == plain_greedy(weights, cfg, prompt, 8)
+    llm.ops.left = 1
+    with pytest.raises(RuntimeError, match="gave up"):
+        llm.step([StepEntry("a", prompt, [8])])
+    assert "a" not in llm.cache
+    llm.ops.left = 2
+    with pytest.raises(RuntimeError, match="gave up"):
+        llm.trace(prompt, 4)
+    llm.cache.check()
+    assert llm.cache.free_pages() == [64, 64]
 
 
 def test_a_failing_step_reaches_its_requests_and_frees(tiny):
