@@ -1648,7 +1648,7 @@ class HipOps(Ops):
                    self.PREFILL_WORKGROUPS)
             plan = meta.scratch.get(key)
             if plan is None:
-                plan = meta.scratch[key] = self._prefill_parts(meta, T, num_heads, head_dim, abs(reach))
+                plan = meta.scratch[key] = self._prefill_parts(meta, T, meta.max_kv, num_heads, head_dim, abs(reach))
             parts = plan["parts"]
             _check(lib.distie_attention_prefill_f32(
                 qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
@@ -1835,18 +1835,31 @@ class HipOps(Ops):
         plan["prefill"] = singles < meta.num_requests or not plan["decode"] or \
             (meta.singles_bound is not None and not meta.all_decode)
         if plan["prefill"]:
-            plan["waves"] = self._prefill_waves(lib, meta, T, singles if plan["decode"] else 0, num_heads, window)
+            keys = self._portions_keys(meta) if plan["decode"] else meta.max_kv
+            plan["waves"] = self._prefill_waves(lib, meta, T, singles if plan["decode"] else 0, keys, num_heads, window)
             if not plan["waves"]:
-                plan.update(self._prefill_parts(meta, T, num_heads, head_dim, window))
+                plan.update(self._prefill_parts(meta, T, keys, num_heads, head_dim, window))
         return plan
 
-    def _prefill_waves(self, lib, meta: BatchMeta, T, singles, num_heads, window) -> int:
+    @staticmethod
+    def _portions_keys(meta: BatchMeta) -> int:
+        """The most keys that a request with more than one token has: what a request decodes behind is nothing to the portions
+        beside it. Where the host does not know the requests (captured steps) the longest that any may have. By the longest context
+        of all before, us of both kernels: 12 heads, 300 tokens beside one request of 5,000 keys 30.7 -> 18.2, beside 24 of 900 22.0 ->
+        19.5; 28 heads, 3 prompts of 667 beside one of 5,000 66 -> 39, beside 4 of 16,000 114 -> 56, beside 24 of 1,500 (two waves ->
+        tiled) 51 -> 53 with the prompts in front, 55 either way behind the others, where the engine puts them."""
+        if meta.host_cu_q is None or meta.host_past is None:
+            return meta.max_kv
+        tokens = np.diff(np.asarray(meta.host_cu_q))
+        return int((np.asarray(meta.host_past) + tokens)[tokens > 1].max(initial=1))
+
+    def _prefill_waves(self, lib, meta: BatchMeta, T, singles, keys, num_heads, window) -> int:
         """How many waves of a workgroup share a tile of 32 tokens of the portions of prompts and split its keys; 0: the tiled
         kernel, whose waves share the keys."""
         if not self.PREFILL_PARTS or not lib.distie_attention_prefill_keys_fits() or meta.block_size > 65536 or \
                 -(-T // 32) + meta.num_requests > 65535:
             return 0
-        visible = min(meta.max_kv, int(window) + 32) if window else meta.max_kv
+        visible = min(keys, int(window) + 32) if window else keys
         tokens, portions = max(1, T - singles), max(1, meta.num_requests - singles)
         workgroups = num_heads * (-(-tokens // 32) + portions // 2)
         many, far, times = self.PREFILL_WAVES_BEHIND
@@ -1854,21 +1867,21 @@ class HipOps(Ops):
         if visible > reach * self.PREFILL_PARTS[0][0] or \
                 (tokens < self.PREFILL_WAVES_FEW[0] and visible > self.PREFILL_WAVES_FEW[1]) or \
                 (workgroups > many and visible > far and visible * portions >= times * tokens) or \
-                any(workgroups > least and visible < keys for least, keys in self.PREFILL_WAVES_MANY):
+                any(workgroups > least and visible < most for least, most in self.PREFILL_WAVES_MANY):
             return 0
-        for waves, most, keys in self.PREFILL_WAVES:
-            if workgroups <= most and visible >= keys:
+        for waves, most, least in self.PREFILL_WAVES:
+            if workgroups <= most and visible >= least:
                 return waves
         return 2
 
-    def _prefill_parts(self, meta: BatchMeta, T, num_heads, head_dim, window) -> dict:
-        """Into how many parts the tiled kernel cuts its walk over the keys, and the buffers between it and the
+    def _prefill_parts(self, meta: BatchMeta, T, keys, num_heads, head_dim, window) -> dict:
+        """Into how many parts the tiled kernel cuts its walk over up to `keys` keys, and the buffers between it and the
         merge. Portions of prompts (and single tokens too, if no other kernel took them): long walks over the
         keys are cut into parts that run side by side."""
-        visible = min(meta.max_kv, int(window) + 128) if window else meta.max_kv
+        visible = min(keys, int(window) + 128) if window else keys
         parts = 1
-        for keys, cut in self.PREFILL_PARTS:
-            if visible >= keys:
+        for least, cut in self.PREFILL_PARTS:
+            if visible >= least:
                 parts = cut
         # few new tokens make few workgroups (one per 128 tokens of a request and head), each walking all
         # the keys alone: more parts then, down to 128 keys a part

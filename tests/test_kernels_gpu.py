@@ -1395,6 +1395,21 @@ def test_portions_whose_keys_the_waves_of_a_workgroup_share(ops, heads, kv_heads
         meta.groups[0].block_table, meta.table_rows = table, None
 
 
+@pytest.mark.parametrize("heads,kv_heads,lens,q_lens,window,form", [
+    (12, 2, [300, 5000, 40, 1200], [300, 1, 40, 1], None, (4, None)), (12, 2, [2300, 700, 9000], [90, 2, 1], None, (8, None)),
+    (28, 4, [3000, 667, 667, 667, 40], [1, 667, 667, 667, 1], None, (0, 1)), (12, 2, [5200, 33, 7000], [400, 33, 1], None, (0, 7)),
+    (12, 2, [4000, 257, 6000], [64, 257, 1], 300, (4, None))])
+def test_portions_beside_requests_that_decode_further_behind(ops, heads, kv_heads, lens, q_lens, window, form):
+    """The portions' kernel and its parts go by the portions' own keys, fewer than the longest request's."""
+    meta, qkv, k, v = paged_case(heads, kv_heads, 128, 16, lens, q_lens, torch.bfloat16, seed=23)
+    meta.host_past = np.array(lens) - np.array(q_lens)
+    want = TorchOps("cuda").paged_attention(qkv.double(), meta, 0, k.double(), v.double(), heads, kv_heads, 128, 128 ** -0.5, window)
+    got = ops.paged_attention(qkv, meta, 0, k, v, heads, kv_heads, 128, 128 ** -0.5, window)
+    plan, = (p for p in meta.scratch.values() if isinstance(p, dict) and "waves" in p)
+    assert (plan["waves"], plan.get("parts")) == form and plan["decode"]
+    close(got, want, torch.bfloat16, scale=want.abs().max().item())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("dim", [8, 33, 48, 64])
 def test_time_mixing_in_chunks_does_not_hang_on_how_many_there_are(ops, dim, dtype):

@@ -3,11 +3,13 @@ boundary where the kernels of both sides were measured."""
 
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
 from distie_amd.csrc import build
 from distie_amd.kernels.hip_ops import HipOps
+from distie_amd.kernels.interface import BatchMeta
 
 
 @pytest.fixture(scope="module")
@@ -346,3 +348,33 @@ def test_long_rotating_products_in_large_tiles(rules, rows, weight, takes):
 def test_small_gated_weights_in_large_tiles(rules, rows, weight, takes):
     rules.captured, rules.library_timed_rows = True, 0
     assert (rules._large(rows, *weight, "gated", ()) is not None) == takes
+
+
+def prompts_plan(heads, portions, single_keys, window=0, known=True):
+    """How a step's portions (tokens, keys behind them) go beside requests that decode behind `single_keys` keys: 28 heads on 4 kv
+    heads, 12 on 2."""
+    ops = HipOps.__new__(HipOps)
+    ops.device = torch.device("cpu")
+    tokens = [n for n, _ in portions] + [1] * len(single_keys)
+    past = [behind for _, behind in portions] + [keys - 1 for keys in single_keys]
+    cu_q = np.concatenate([[0], np.cumsum(tokens)]).astype(np.int32)
+    meta = BatchMeta(num_tokens=sum(tokens), num_requests=len(tokens), positions=None, token_request=None, cu_q=None, kv_len=None,
+                     state_slots=None, max_q=max(tokens), max_kv=max(n + p for n, p in zip(tokens, past)), block_size=16,
+                     host_cu_q=cu_q if known else None, host_past=np.array(past) if known else None,
+                     singles_bound=None if known else len(tokens))
+    plan = ops._attention_plan(attention(128), meta, sum(tokens), heads, heads // 6 if heads == 12 else 4, 128, window)
+    return plan["waves"], plan.get("parts")
+
+
+@pytest.mark.parametrize("heads,portions,window,waves", [
+    (12, [(300, 0)], 0, 4), (12, [(300, 900)], 0, 8), (12, [(40, 0), (7, 30)], 0, 2), (12, [(600, 3500)], 0, 8),
+    (12, [(600, 5000)], 0, 0), (12, [(300, 2000)], 512, 4), (28, [(667, 0)] * 3, 0, 0), (28, [(667, 0), (667, 0), (600, 1400)], 0, 2),
+    (28, [(120, 0)], 0, 4)])
+def test_what_requests_decode_behind_is_nothing_to_the_portions_beside_them(heads, portions, window, waves):
+    plans = {prompts_plan(heads, portions, [keys, 100], window) for keys in (10, 500, 1100, 2000, 5000, 20000, 100000)}
+    assert len(plans) == 1 and plans.pop()[0] == waves
+
+
+def test_portions_of_a_captured_step_may_have_as_many_keys_as_any_request():
+    assert prompts_plan(12, [(300, 0)], [1000], known=False)[0] > 0
+    assert prompts_plan(12, [(300, 0)], [20000], known=False)[0] == 0
