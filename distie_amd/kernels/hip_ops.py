@@ -433,6 +433,9 @@ class HipOps(Ops):
     # length are cut as before). Everywhere else it is level or behind (32 requests: 30 -> 33 us).
     DECODE_SHARED_BELOW = 0.8
     DECODE_MAX_RUNS = 256
+    # what a step's plan of attention is made by, beside its sizes
+    ATTENTION_PLAN_RULES = ("PREFILL_PARTS", "PREFILL_WORKGROUPS", "PREFILL_WAVES_REACH", "PREFILL_WAVES_FEW", "PREFILL_WAVES_BEHIND",
+                            "PREFILL_WAVES_MANY", "PREFILL_WAVES", "DECODE_WAVES", "DECODE_MAX_RUNS", "DECODE_SHARED_BELOW")
     # attention with mixed heads: from so many tokens a step on a workgroup takes 16 queries instead of 8 (fewer would
     # leave compute units without one)
     MIXED_WIDE_TOKENS = 6144
@@ -1609,8 +1612,7 @@ class HipOps(Ops):
             # with these sizes: worked out once per step (the layers run one after the other, so they can
             # share the buffers)
             key = ("attention", reach, num_heads, num_kv_heads, head_dim, meta.max_kv, meta.all_decode,
-                   meta.singles_bound, self.PREFILL_PARTS, self.PREFILL_WAVES_REACH, self.PREFILL_WORKGROUPS, self.DECODE_WAVES,
-                   self.DECODE_MAX_RUNS,                   self.DECODE_SHARED_BELOW)
+                   meta.singles_bound, *(getattr(self, name) for name in self.ATTENTION_PLAN_RULES))
             plan = meta.scratch.get(key)
             if plan is None or plan["cu_q"] is not meta.host_cu_q:
                 plan = meta.scratch[key] = self._attention_plan(lib, meta, T, num_heads, num_kv_heads, head_dim, abs(reach))

@@ -350,10 +350,10 @@ def test_small_gated_weights_in_large_tiles(rules, rows, weight, takes):
     assert (rules._large(rows, *weight, "gated", ()) is not None) == takes
 
 
-def prompts_plan(heads, portions, single_keys, window=0, known=True):
+def prompts_plan(heads, portions, single_keys, window=0, known=True, cls=HipOps):
     """How a step's portions (tokens, keys behind them) go beside requests that decode behind `single_keys` keys: 28 heads on 4 kv
     heads, 12 on 2."""
-    ops = HipOps.__new__(HipOps)
+    ops = cls.__new__(cls)
     ops.device = torch.device("cpu")
     tokens = [n for n, _ in portions] + [1] * len(single_keys)
     past = [behind for _, behind in portions] + [keys - 1 for keys in single_keys]
@@ -378,3 +378,19 @@ def test_what_requests_decode_behind_is_nothing_to_the_portions_beside_them(head
 def test_portions_of_a_captured_step_may_have_as_many_keys_as_any_request():
     assert prompts_plan(12, [(300, 0)], [1000], known=False)[0] > 0
     assert prompts_plan(12, [(300, 0)], [20000], known=False)[0] == 0
+
+
+def test_a_steps_plan_of_attention_is_kept_by_every_rule_that_it_is_made_by():
+    read = set()
+
+    class Watched(HipOps):
+        def __getattribute__(self, name):
+            if name.isupper():
+                read.add(name)
+            return super().__getattribute__(name)
+
+    for heads in (12, 28):
+        for portions in ([(300, 0)], [(64, 4000)], [(667, 0)] * 3, [(600, 5000)], [(1500, 1400)]):
+            for known in (True, False):
+                prompts_plan(heads, portions, [700], known=known, cls=Watched)
+    assert len(read) > 6 and read <= set(HipOps.ATTENTION_PLAN_RULES)
