@@ -333,3 +333,46 @@ def test_decode_batches_beyond_the_packed_kernels_rows(tmp_path, monkeypatch, mo
             llm.finish(rid)
     llm.cache.check()
     llm.close()
+
+
+@pytest.mark.parametrize("width,layers,ff,std", [(1024, 34, 544, 0.03), (2048, 3, 1056, 0.03)])
+def test_captured_steps_whose_layers_end_in_one_launch(tmp_path, monkeypatch, width, layers, ff, std):
+    """Steps of 1 to 8 rows, replayed, at the widths of `layer_chain` that no benchmark has: more layers than one fill of the words
+    between workgroups is for, hidden values that fill no whole group of tiles. Judged by the plain model, beside the same engine
+    kernel by kernel: both round at the same places, so their errors are samples of one distribution, of some thousand logits each
+    row and 24 rows a request; the chain's may be a tenth larger."""
+    from distie_amd.kernels.hip_ops import HipOps
+
+    sizes = dict(SIZES_1_5B, num_hidden_layers=layers, hidden_size=width, num_attention_heads=width // 128, intermediate_size=ff,
+                 vocab_size=2048)
+    folder, weights = make_model_dir(tmp_path, sizes, seed=31, std=std, dtype=torch.bfloat16)
+    weights = {k: v.to("cuda", torch.float64) for k, v in weights.items()}
+    chained, chain = [], HipOps._layer_chain
+    monkeypatch.setattr(HipOps, "_layer_chain", lambda ops, tail, following: chained.append((tail.residual.shape[0], following is None))
+                        or chain(ops, tail, following))
+    new, errors = 24, {}
+    for rows in (HipOps.CHAIN_MAX_ROWS, 0):
+        monkeypatch.setattr(HipOps, "CHAIN_MAX_ROWS", rows)
+        llm = LLM(folder, dtype="bf16", block_size=16, num_blocks=8 * 16, max_seqs=8, max_model_len=256, use_graphs=True, lookahead=True)
+        for batch in (1, 2, 4, 8):
+            replays = llm.runner.graphs.replays
+            prompts = [random_ids(sizes, 40 + 9 * i, 10 * batch + i) for i in range(batch)]
+            outs, kept = run_and_keep_logits(llm, prompts, [SamplingParams(max_new_tokens=new, ignore_eos=True)] * batch)
+            torch.cuda.synchronize()
+            assert llm.runner.graphs.failures == 0 and llm.runner.graphs.replays > replays + new - 4
+            # in the order of capture: `layers` launches a step, the last of them without a layer behind it
+            taken = [last for m, last in chained if m == batch]
+            assert taken == ([False] * (layers - 1) + [True]) * (len(taken) // layers) and bool(taken) == bool(rows)
+            off = size = 0.0
+            for prompt, out in zip(prompts, outs):
+                ids = prompt + out.token_ids[:-1]
+                want = plain.forward(weights, sizes, ids, torch.float64, rows=list(range(len(prompt) - 1, len(ids)))).float()
+                got = torch.stack([row for _, row in kept[out.request_id]])
+                assert (got - want).abs().max().item() < want.abs().max().item() / 16
+                off, size = off + (got - want).square().sum().item(), size + want.square().sum().item()
+            errors.setdefault(batch, []).append((off / size) ** 0.5)
+        chained.clear()
+        del llm
+    for batch, (one_launch, kernel_by_kernel) in errors.items():
+        print(f"width {width}, {layers} layers, {batch} rows: {one_launch:.5f} in one launch, {kernel_by_kernel:.5f} kernel by kernel")
+        assert one_launch < 1.1 * kernel_by_kernel
