@@ -1987,6 +1987,8 @@ constexpr int KEYS_PIECES = D / 8;                      // 16-byte pieces of a r
 constexpr int KEYS_LOADS = D / 32;                      // loads (of 1 KB) of 16 keys of K, and of V^T
 constexpr int KEYS_O_STRIDE = D + 4;                    // floats: rows of an odd number of 16-byte pieces
 
+typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+
 // LDS: the waves' tiles and, in their place, their sums; behind that their references and the columns' factors
 template <int W>
 constexpr int prefill_keys_tiles() {
@@ -2166,13 +2168,17 @@ __global__ __launch_bounds__(DISTIE_WAVE * W) __attribute__((amdgpu_waves_per_eu
     }
     const float from = m_run == -INFINITY ? 0.f : -m_run;
     bf16x8 p_reg[BLOCKS];                               // step t: keys 16 t + 8 h .. + 7 of the tile
+#pragma unroll
+    for (int e = 0; e < 16; ++e) p_reg[e / 8][e % 8] = static_cast<bf16_t>(fast_exp2(fmaf(s[e], scale_log2, from)));
+    // What the weights are divided by is the sum of them as they go into the product: what rounding does to one that outdoes the
+    // others cancels. Summed before they were rounded, the outputs of peaked scores (three units of spread) were further from 64 bits
+    // than those of attn_prefill, whose references are found among more keys (1,024 tokens: W = 2 0.00205, W = 4 0.00196, attn_prefill
+    // 0.00191; now 0.00186 and 0.00182). 1 to 3 % of the kernel: 2,048 tokens 26.5 -> 26.9 us, 301 7.63 -> 7.69.
     float sum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float p = fast_exp2(fmaf(s[e], scale_log2, from));
-      sum += p;
-      p_reg[e / 8][e % 8] = static_cast<bf16_t>(p);
-    }
+    for (int e = 0; e < 16; e += 2)
+      sum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{p_reg[e / 8][e % 8], p_reg[e / 8][e % 8 + 1]}, bf16x2{bf16_t(1.f), bf16_t(1.f)}, sum,
+                                            false);
     l_run += sum;
     if (more)
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");     // V^T is there; the next K is under way
