@@ -1973,8 +1973,8 @@ extern "C" int distie_attention_prefill_bf16(const void* qkv, int64_t q_stride, 
 //    K rows lie in LDS with their 16-byte pieces turned by the row's number (piece j of row r at j ^ r), which the loads
 //    do and which keeps the reads of 32 rows free of bank conflicts; a row of V^T of 16 keys is two pieces, read in order. The
 //    rows of a product are taken in an order in which a lane's scores are eight keys in a row, and those it reads of V^T.
-//    12 heads of 128 and 2 kv heads, us, attn_prefill with its merge / this: 40 tokens 6.4 / 6.0, 301 13.8 / 7.8, 512 18.1 / 9.0, 1,024
-//    27.9 / 14.2, 2,048 39.3 / 27.3. What bounds it: of the 6, 2 are the launch and the rest a chain of trips (requests, positions
+//    12 heads of 128 and 2 kv heads, us, attn_prefill with its merge / this: 40 tokens 6.3 / 5.6, 301 13.5 / 7.7, 512 17.5 / 8.8, 1,024
+//    27.2 / 14.0, 2,048 38.0 / 27.1. What bounds it: of the 5.6, 2 are the launch and the rest a chain of trips (requests, positions
 //    and pages, keys, the sums); a tile costs a wave about 1 us alone on its SIMD and 1.3 beside another, a quarter of it products: reads
 //    of LDS, the softmax and the next loads' addresses, one behind the other. Two waves a SIMD need the small tile: 64 keys at one wave
 //    a SIMD 51 us for 2,048 tokens, 64 keys and 64 columns 42 (then 41 at 32 keys). The columns' maximum went through LDS at first, the

@@ -21,7 +21,7 @@
 // `hidden`, `out`) hold UNWRITTEN everywhere when the launch begins, nobody writes that pattern (a NaN; `written`), words are stored and
 // loaded past the caches that workgroups do not share (stores and loads at device scope), and a reader repeats its loads until no word is
 // missing. So no order between two words, no acknowledgement, counter or fence is needed. With counters (store, acknowledgement,
-// count, poll, load) each boundary cost five trips instead of two: 37.8 us a layer.
+// count, poll, load) each boundary cost five trips instead of two, and the layer at 1 row 14 us more than now.
 //
 // Nothing here waits for a workgroup that has not started. A workgroup claims its slot of every phase when it starts; one that finds its x
 // incomplete for `patience` looks takes, of the earliest phase that has any, a slot that nobody has claimed, works on it as on its own,

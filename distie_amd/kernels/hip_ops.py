@@ -400,8 +400,8 @@ class HipOps(Ops):
     PREFILL_WORKGROUPS = 512         # as many workgroups a short portion's attention should have, if its keys allow
     # Heads of 64 and 128 in bfloat16 up to so many times the keys from which the tiled kernel's walk is cut (4,608 keys with up to 256
     # workgroups of 32 tokens, 3,584 with more): the kernel whose waves share the columns and split the keys. Tiled with its merge /
-    # that one, us, 12 heads of 128: prompts of 40 tokens 6.4 / 5.7, 301 13.8 / 7.8, 1,024 27.9 / 14.2, 2,048 39.3 / 27.3, 3,500 78 /
-    # 64, 300 behind 4,000 36.0 / 27.8, 600 41 / 32; beyond, 28 heads, 600 behind 4,000 76 / 81, 1,500 147 / 156 (64 heads, 600: 129 /
+    # that one, us, 12 heads of 128: prompts of 40 tokens 6.3 / 5.6, 301 13.5 / 7.7, 1,024 27.2 / 14.0, 2,048 38.0 / 27.1, 3,500 77 /
+    # 62, 300 behind 4,000 34.5 / 27.1, 600 39 / 30; beyond, 28 heads, 600 behind 4,000 76 / 81, 1,500 147 / 156 (64 heads, 600: 129 /
     # 149; heads of 64, 28 of them, 4,500 tokens 126 / 139); 12 heads, 128 behind 16,000 55 / 83
     PREFILL_WAVES_REACH = ((256, 4.5), (None, 3.5))
     # few tokens far behind are too few workgroups for either; the tiled kernel's parts are more: 64 behind 4,000 (16 heads) 23.2 /
