@@ -2269,7 +2269,11 @@ __global__ __launch_bounds__(DISTIE_WAVE * W) __attribute__((amdgpu_waves_per_eu
   }
 }
 
-extern "C" int distie_attention_prefill_keys_fits() { return 1; }
+// Whether it takes such pages: their bytes are counted in 32 bits, and a lane's place in a head's part of one.
+extern "C" int distie_attention_prefill_keys_fits(int kv_heads, int block_size) {
+  return kv_heads >= 1 && block_size >= 16 && block_size % 16 == 0 && block_size <= 65536 &&
+         2 * static_cast<int64_t>(kv_heads) * block_size * D <= 0xffffffffll;
+}
 
 // As distie_attention_prefill_bf16, with nothing between its parts. waves (of a workgroup): 2, 4 or 8.
 extern "C" int distie_attention_prefill_keys(const void* qkv, int64_t q_stride, const void* k_cache, const void* v_cache,
@@ -2278,8 +2282,7 @@ extern "C" int distie_attention_prefill_keys(const void* qkv, int64_t q_stride, 
                                              int heads, int kv_heads, int block_size, float scale, int window, int min_q_len,
                                              const float* sinks, int waves, hipStream_t stream) {
   if (tokens <= 0) return 0;
-  if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || block_size < 16 || block_size % 16 != 0 || block_size > 65536 ||
-      table_width < 1 || num_requests < 1 || min_q_len < 1 || (waves != 2 && waves != 4 && waves != 8) || !(scale > 0.f))
+  if (heads < 1 || !distie_attention_prefill_keys_fits(kv_heads, block_size) || heads % kv_heads != 0 || table_width < 1 || num_requests < 1 || min_q_len < 1 || (waves != 2 && waves != 4 && waves != 8) || !(scale > 0.f))
     return DISTIE_BAD_ARGUMENT;
   const int64_t tiles = (static_cast<int64_t>(tokens) + KEYS_BM - 1) / KEYS_BM + num_requests;     // an upper bound; spare blocks leave at once
   if (tiles > 65535) return DISTIE_BAD_ARGUMENT;
@@ -2295,7 +2298,7 @@ extern "C" int distie_attention_prefill_keys(const void* qkv, int64_t q_stride, 
                                  : run(attn_prefill_keys_kernel<2>, prefill_keys_lds<2>());
 }
 #else
-extern "C" int distie_attention_prefill_keys_fits() { return 0; }
+extern "C" int distie_attention_prefill_keys_fits(int, int) { return 0; }
 extern "C" int distie_attention_prefill_keys(const void*, int64_t, const void*, const void*, const int32_t*, const int32_t*,
                                              const int32_t*, int, const int32_t*, void*, int, int, int, int, int, float, int, int,
                                              const float*, int, hipStream_t) {
@@ -2615,7 +2618,7 @@ extern "C" int distie_attention_prefill_bf16(const void*, int64_t, const void*, 
   return DISTIE_BAD_ARGUMENT;
 }
 
-extern "C" int distie_attention_prefill_keys_fits() { return 0; }
+extern "C" int distie_attention_prefill_keys_fits(int, int) { return 0; }
 
 extern "C" int distie_attention_prefill_keys(const void*, int64_t, const void*, const void*, const int32_t*, const int32_t*,
                                              const int32_t*, int, const int32_t*, void*, int, int, int, int, int, float, int, int,

@@ -1838,7 +1838,7 @@ class HipOps(Ops):
             (meta.singles_bound is not None and not meta.all_decode)
         if plan["prefill"]:
             keys = self._portions_keys(meta) if plan["decode"] else meta.max_kv
-            plan["waves"] = self._prefill_waves(lib, meta, T, singles if plan["decode"] else 0, keys, num_heads, window)
+            plan["waves"] = self._prefill_waves(lib, meta, T, singles if plan["decode"] else 0, keys, num_heads, num_kv_heads, window)
             if not plan["waves"]:
                 plan.update(self._prefill_parts(meta, T, keys, num_heads, head_dim, window))
         return plan
@@ -1855,10 +1855,10 @@ class HipOps(Ops):
         tokens = np.diff(np.asarray(meta.host_cu_q))
         return int((np.asarray(meta.host_past) + tokens)[tokens > 1].max(initial=1))
 
-    def _prefill_waves(self, lib, meta: BatchMeta, T, singles, keys, num_heads, window) -> int:
+    def _prefill_waves(self, lib, meta: BatchMeta, T, singles, keys, num_heads, num_kv_heads, window) -> int:
         """How many waves of a workgroup share a tile of 32 tokens of the portions of prompts and split its keys; 0: the tiled
         kernel, whose waves share the keys."""
-        if not self.PREFILL_PARTS or not lib.distie_attention_prefill_keys_fits() or meta.block_size > 65536 or \
+        if not self.PREFILL_PARTS or not lib.distie_attention_prefill_keys_fits(num_kv_heads, meta.block_size) or \
                 -(-T // 32) + meta.num_requests > 65535:
             return 0
         visible = min(keys, int(window) + 32) if window else keys

@@ -350,7 +350,7 @@ def test_small_gated_weights_in_large_tiles(rules, rows, weight, takes):
     assert (rules._large(rows, *weight, "gated", ()) is not None) == takes
 
 
-def prompts_plan(heads, portions, single_keys, window=0, known=True, cls=HipOps):
+def prompts_plan(heads, portions, single_keys, window=0, known=True, cls=HipOps, kv_heads=None, block_size=16):
     """How a step's portions (tokens, keys behind them) go beside requests that decode behind `single_keys` keys: 28 heads on 4 kv
     heads, 12 on 2."""
     ops = cls.__new__(cls)
@@ -359,10 +359,10 @@ def prompts_plan(heads, portions, single_keys, window=0, known=True, cls=HipOps)
     past = [behind for _, behind in portions] + [keys - 1 for keys in single_keys]
     cu_q = np.concatenate([[0], np.cumsum(tokens)]).astype(np.int32)
     meta = BatchMeta(num_tokens=sum(tokens), num_requests=len(tokens), positions=None, token_request=None, cu_q=None, kv_len=None,
-                     state_slots=None, max_q=max(tokens), max_kv=max(n + p for n, p in zip(tokens, past)), block_size=16,
+                     state_slots=None, max_q=max(tokens), max_kv=max(n + p for n, p in zip(tokens, past)), block_size=block_size,
                      host_cu_q=cu_q if known else None, host_past=np.array(past) if known else None,
                      singles_bound=None if known else len(tokens))
-    plan = ops._attention_plan(attention(128), meta, sum(tokens), heads, heads // 6 if heads == 12 else 4, 128, window)
+    plan = ops._attention_plan(attention(128), meta, sum(tokens), heads, kv_heads or (heads // 6 if heads == 12 else 4), 128, window)
     return plan["waves"], plan.get("parts")
 
 
@@ -394,3 +394,13 @@ def test_a_steps_plan_of_attention_is_kept_by_every_rule_that_it_is_made_by():
             for known in (True, False):
                 prompts_plan(heads, portions, [700], known=known, cls=Watched)
     assert len(read) > 6 and read <= set(HipOps.ATTENTION_PLAN_RULES)
+
+
+@pytest.mark.parametrize("kv_heads,block_size,takes", [
+    (2, 16, True), (1, 65536, True), (255, 65536, True), (256, 65536, False), (4096, 4096, False), (4095, 4096, True), (1 << 20, 16, False),
+    (2, 65552, False), (2, 24, False)])
+def test_pages_whose_bytes_the_portions_kernel_cannot_count(kv_heads, block_size, takes):
+    """It counts a page's bytes in 32 bits: larger pages stay with the tiled kernel."""
+    assert bool(attention(128).distie_attention_prefill_keys_fits(kv_heads, block_size)) == takes
+    if kv_heads <= 256:                                # (more heads are too many workgroups for so few keys)
+        assert (prompts_plan(kv_heads, [(40, 0)], [], kv_heads=kv_heads, block_size=block_size)[0] > 0) == takes
