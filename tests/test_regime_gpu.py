@@ -338,7 +338,7 @@ def test_decode_batches_beyond_the_packed_kernels_rows(tmp_path, monkeypatch, mo
 @pytest.mark.parametrize("width,layers,ff,std", [(1024, 34, 544, 0.03), (2048, 3, 1056, 0.03)])
 def test_captured_steps_whose_layers_end_in_one_launch(tmp_path, monkeypatch, width, layers, ff, std):
     """Steps of 1 to 8 rows, replayed, at the widths of `layer_chain` that no benchmark has: more layers than one fill of the words
-    between workgroups is for, hidden values that fill no whole group of tiles. Judged by the plain model, beside the same engine
+    between workgroups is for, hidden values that fill no whole group of tiles. Held against the plain model, beside the same engine
     kernel by kernel: both round at the same places, so their errors are samples of one distribution, of some thousand logits each
     row and 24 rows a request; the chain's may be a tenth larger."""
     from distie_amd.kernels.hip_ops import HipOps
