@@ -1,8 +1,9 @@
 """Building and finding the native libraries.
 
-Five kinds of shared library, all built from the sources beside this file:
+Six kinds of shared library, all built from the sources beside this file:
 
 * `core`  - the id pool of the cache manager (C++, host only, g++);
+* `calls` - the extension module through which the others are called (C++ with torch's headers, host only, g++);
 * `ops`   - the HIP kernels that do not depend on the head size (hipcc, gfx950);
 * `library` - the calls of the vendor's matrix-product library for large products (hipcc, linked with hipBLASLt);
 * `attn_d<D>` - the attention kernels for head size D (hipcc, `-DDISTIE_HEAD_DIM=D`; the matrix-core
@@ -24,6 +25,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -43,7 +45,6 @@ OPS_SOURCES = ["elementwise.hip", "gemm.hip", "packed_tiles.hip", "large_tiles.h
 ATTN_SOURCES = ["attention.hip"]
 MIXED_ATTN_SOURCES = ["mixed_attention_mc.hip"]
 LIBRARY_SOURCES = ["library_products.hip"]
-LINK_LIBS = {"library": ["-lhipblaslt"]}
 
 
 class BuildError(RuntimeError):
@@ -77,6 +78,8 @@ def _spec(name: str):
     """-> (sources, compiler, flags)"""
     if name == "core":
         return ["block_pool.cpp"], os.environ.get("CXX", "g++"), list(CXX_FLAGS)
+    if name == "calls":
+        return ["calls.cpp"], os.environ.get("CXX", "g++"), list(CXX_FLAGS) + _torch_flags()
     if name == "ops":
         return list(OPS_SOURCES), _hipcc(), list(HIP_FLAGS)
     if name == "library":
@@ -92,6 +95,26 @@ def _spec(name: str):
             raise BuildError(f"the kernels of attention with mixed heads are built for multiples of 32 up to 256, not {dim}")
         return list(MIXED_ATTN_SOURCES), _hipcc(), list(HIP_FLAGS) + [f"-DDISTIE_HEAD_DIM={dim}"]
     raise BuildError(f"no native library named {name}")
+
+
+def _torch_flags() -> List[str]:
+    """Where the headers of Python and torch are, and for which builds of theirs the library is good."""
+    import torch
+
+    include = Path(torch.__file__).resolve().parent / "include"
+    return [f"-I{sysconfig.get_paths()['include']}", f"-isystem{include}", f"-isystem{include / 'torch' / 'csrc' / 'api' / 'include'}",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DDISTIE_BUILT_FOR="torch {torch.__version__}, Python {sysconfig.get_python_version()}"']
+
+
+def _link_libs(name: str, compiler: str) -> List[str]:
+    if name == "library":
+        return [f"-L{Path(compiler).resolve().parent.parent / 'lib'}", "-lhipblaslt"]
+    if name == "calls":
+        import torch
+
+        folder = Path(torch.__file__).resolve().parent / "lib"
+        return [f"-L{folder}", f"-Wl,-rpath,{folder}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    return []
 
 
 def _hipcc() -> str:
@@ -186,10 +209,7 @@ def build(name: str, force: bool = False) -> Path:
         objects = [str(scratch / (Path(s).stem + ".o")) for s in sources]
         link_flags = [f for f in flags if not f.startswith("-D")]
         staging = scratch / target.name
-        libs = LINK_LIBS.get(name, [])
-        if libs:
-            libs = [f"-L{Path(compiler).resolve().parent.parent / 'lib'}"] + libs
-        _run([compiler] + link_flags + ["-shared"] + objects + libs + ["-o", str(staging)], f"{name} (link)")
+        _run([compiler] + link_flags + ["-shared"] + objects + _link_libs(name, compiler) + ["-o", str(staging)], f"{name} (link)")
         os.replace(staging, target)
     finally:
         shutil.rmtree(scratch, ignore_errors=True)
@@ -214,7 +234,7 @@ DEFAULT_MIXED_HEAD_DIMS = (32, 64, 96, 128, 160)
 
 
 def build_all(head_dims=DEFAULT_HEAD_DIMS, force: bool = True) -> List[Path]:
-    out = [build("core", force), build("ops", force), build("library", force)]
+    out = [build("core", force), build("calls", force), build("ops", force), build("library", force)]
     for d in head_dims:
         out.append(build(f"attn_d{d}", force))
     for d in DEFAULT_MIXED_HEAD_DIMS:

@@ -1,7 +1,7 @@
 """`HipOps`: the kernel surface on hand-written HIP kernels for gfx950.
 
-The kernels live in shared libraries built from `distie_amd/csrc` and are called through
-ctypes with raw device pointers on torch's current HIP stream, so they take part in
+The kernels live in shared libraries built from `distie_amd/csrc` and are called (`calls.py`)
+with raw device pointers on torch's current HIP stream, so they take part in
 stream order and in graph capture like any other launch. torch is the allocator and the
 stream/graph owner; the only library routine on this path is the matrix product for
 large bfloat16 operands (the reference leaves its products to a library too).
@@ -13,6 +13,7 @@ the kernels refuse, raises: there is no fallback.
 from __future__ import annotations
 
 import ctypes
+import functools
 import logging
 from typing import Dict, Optional
 
@@ -20,6 +21,7 @@ import numpy as np
 import torch
 
 from ..csrc import build
+from . import calls
 from .interface import BatchMeta, Ops, RouteRule
 
 _log = logging.getLogger(__name__)
@@ -478,6 +480,9 @@ class HipOps(Ops):
             raise KernelError(f"the kernels are built for gfx950 (MI355X); this device is {name}")
         self._device_index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         self._compute_units = torch.cuda.get_device_properties(self.device).multi_processor_count
+        # (a device without a number is no tensor's device: `_own` refuses them one by one)
+        self._owned = functools.partial(calls.native().owned, -1 if self.device.index is None else self.device.index)
+        self._empty = functools.partial(calls.native().empty, self._device_index)       # (shape, dtype) -> tensor
         self._lib = None
         self._tuning = False
         self.library_timed_rows = self.library_timed_portion = 0
@@ -506,7 +511,7 @@ class HipOps(Ops):
         dtype = torch.from_numpy(np.empty(0, dtype=values.dtype)).dtype
         nbytes = values.nbytes
         if nbytes == 0:
-            return torch.empty(values.shape, dtype=dtype, device=self.device)
+            return self._empty(values.shape, dtype)
         slot = self._uploads[self._next_upload]
         self._next_upload = (self._next_upload + 1) % len(self._uploads)
         if slot[2] is not None:
@@ -516,7 +521,7 @@ class HipOps(Ops):
             slot[1] = slot[0].numpy()
             slot[2] = torch.cuda.Event()
         slot[1][:nbytes] = values.reshape(-1).view(np.uint8)
-        dev = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        dev = self._empty(nbytes, torch.uint8)
         dev.copy_(slot[0][:nbytes], non_blocking=True)
         slot[2].record()
         return dev.view(dtype).view(values.shape)
@@ -611,6 +616,7 @@ class HipOps(Ops):
         o.distie_argmax.argtypes = [_P, _P, _I, _I, _P, _P, _P]
         o.distie_argmax_parts.argtypes = [_I, _I]
         o.distie_sample.argtypes = [_P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P]
+        calls.quicken(o)
 
     def tune_library_products(self, on: bool) -> None:
         """While on, every new shape of a large product has the library's candidate kernels timed, and the
@@ -657,6 +663,7 @@ class HipOps(Ops):
             lib.distie_attention_decode_run_len.argtypes = [_P, _I, _I, _I, _P, _P]
             if lib.distie_attention_head_dim() != head_dim:
                 raise KernelError("attention library was built for another head size")
+            calls.quicken(lib)
             self._attn[head_dim] = lib
         return lib
 
@@ -669,10 +676,20 @@ class HipOps(Ops):
                                                         _F, _P, _I, _P, _P, _I, _I, _I, _I, _P, _P, _P]
             if lib.distie_mixed_head_dim() != head_dim:
                 raise KernelError("the library of attention with mixed heads was built for another head size")
+            calls.quicken(lib)
             self._mixed[head_dim] = lib
         return lib
 
+    # (the constructor puts the native ones in their place)
+    def _empty(self, shape, dtype):
+        return torch.empty(shape, dtype=dtype, device=self.device)
+
+    def _owned(self, *tensors) -> bool:
+        return False
+
     def _own(self, *tensors) -> None:
+        if self._owned(*tensors):
+            return
         for t in tensors:
             if t is None:
                 continue
@@ -694,7 +711,7 @@ class HipOps(Ops):
         if table.dtype != torch.int32 or index.dtype != torch.int32 or value.dtype != torch.int32 or \
                 index.shape != value.shape:
             raise KernelError("scatter_int32 takes int32 tensors, one value for each index")
-        _check(self._ops.distie_scatter_i32(table.data_ptr(), index.data_ptr(), value.data_ptr(), index.numel(),
+        _check(self._ops.distie_scatter_i32(table, index, value, index.numel(),
                                             table.numel(), self._stream()), "scatter_i32")
         _mark_written(table)
 
@@ -714,15 +731,15 @@ class HipOps(Ops):
             if held and not 0 <= row < rows:
                 raise KernelError(f"there is no row {row} to clear")
             if table is not None:
-                _check(self._ops.distie_clear_rows(table.data_ptr(), len(pieces), row, self._stream()), "clear_rows")
+                _check(self._ops.distie_clear_rows(table, len(pieces), row, self._stream()), "clear_rows")
             for t in others:
                 t[row].zero_()
         return clear
 
     def embed(self, ids, table, scale=1.0):
         self._own(ids, table)
-        out = torch.empty((ids.shape[0], table.shape[1]), dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_embed(ids.data_ptr(), table.data_ptr(), _code(table), out.data_ptr(),
+        out = self._empty((ids.shape[0], table.shape[1]), torch.float32)
+        _check(self._ops.distie_embed(ids, table, _code(table), out,
                                       ids.shape[0], table.shape[1], table.shape[0], float(scale), self._stream()), "embed")
         return out
 
@@ -744,9 +761,9 @@ class HipOps(Ops):
         return self._rmsnorm_now(x, weight, eps, out_dtype)
 
     def _rmsnorm_now(self, x, weight, eps, out_dtype):
-        out = torch.empty(x.shape, dtype=out_dtype, device=self.device)
-        _check(self._ops.distie_rmsnorm(x.data_ptr(), None, _F32, 1, weight.data_ptr(), _code(weight),
-                                        out.data_ptr(), _CODES[out_dtype], x.shape[0], x.shape[1], eps,
+        out = self._empty(x.shape, out_dtype)
+        _check(self._ops.distie_rmsnorm(x, None, _F32, 1, weight, _code(weight),
+                                        out, _CODES[out_dtype], x.shape[0], x.shape[1], eps,
                                         self._stream()), "rmsnorm")
         return out
 
@@ -765,9 +782,9 @@ class HipOps(Ops):
         self._own(residual, delta, weight)
         if residual.dtype != torch.float32 or residual.shape != delta.shape[-2:]:
             raise KernelError("add_rmsnorm: residual must be float32 and shaped like delta")
-        out = torch.empty(residual.shape, dtype=out_dtype, device=self.device)
-        _check(self._ops.distie_rmsnorm(residual.data_ptr(), delta.data_ptr(), _code(delta), slices,
-                                        weight.data_ptr(), _code(weight), out.data_ptr(), _CODES[out_dtype],
+        out = self._empty(residual.shape, out_dtype)
+        _check(self._ops.distie_rmsnorm(residual, delta, _code(delta), slices,
+                                        weight, _code(weight), out, _CODES[out_dtype],
                                         residual.shape[0], residual.shape[1], eps, self._stream()), "add_rmsnorm")
         _mark_written(residual)
         return out
@@ -780,7 +797,7 @@ class HipOps(Ops):
         if packed.numel() != self._packed_elements(N, K, False):
             raise KernelError("linear: the packed copy does not belong to this weight")
         _check(self._ops.distie_decode_product_residual(
-            x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, residual.data_ptr(),
+            x, packed, bias, residual,
             M, N, K, self._stream()), "decode_product_residual")
         _mark_written(residual)
 
@@ -839,14 +856,13 @@ class HipOps(Ops):
         if following is not None:
             next_norm, next_eps, packed, bias, table, slots, k_cache, v_cache, heads, kv_heads, dim, block_size, write = following
             next_norm = self._f32(next_norm)
-            qkv = torch.empty((M, (heads + 2 * kv_heads) * dim), dtype=torch.bfloat16, device=self.device)
-            rest = (table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), heads, kv_heads, dim, block_size, write)
-        ptr = lambda t: t.data_ptr() if t is not None else None
+            qkv = self._empty((M, (heads + 2 * kv_heads) * dim), torch.bfloat16)
+            rest = (table, slots, k_cache, v_cache, heads, kv_heads, dim, block_size, write)
         _check(self._ops.distie_layer_chain(
-            tail.mixed.data_ptr(), out_weight._distie_packed.data_ptr(), tail.residual.data_ptr(), mid.data_ptr(),
-            self._f32(norm_weight).data_ptr(), eps, gate_up_weight._distie_gated.data_ptr(), hidden.data_ptr(),
-            down_weight._distie_packed.data_ptr(), out.data_ptr(), ptr(next_norm), next_eps, ptr(packed), ptr(bias), ptr(qkv), *rest,
-            M, C, KO, inter, claims.data_ptr(), self._gave_up.data_ptr(), self._compute_units, self.CHAIN_WORKGROUPS or self._compute_units,
+            tail.mixed, out_weight._distie_packed, tail.residual, mid,
+            self._f32(norm_weight), eps, gate_up_weight._distie_gated, hidden,
+            down_weight._distie_packed, out, next_norm, next_eps, packed, bias, qkv, *rest,
+            M, C, KO, inter, claims, self._gave_up, self._compute_units, self.CHAIN_WORKGROUPS or self._compute_units,
             self.CHAIN_PATIENCE, self.CHAIN_LIMIT, self._stream()), "layer_chain")
         return out.view(torch.float32).view(M, C), qkv
 
@@ -862,8 +878,8 @@ class HipOps(Ops):
             return self._norm_chain(x.terms, x.weights, x.eps, x.scale, None, None, None, None)
         if not isinstance(x, PartialSums):
             return x
-        out = torch.empty(tuple(x.shape), dtype=x.dtype, device=self.device)
-        _check(self._ops.distie_sum_slices(x.data.data_ptr(), x.slices, out.numel(), out.data_ptr(),
+        out = self._empty(tuple(x.shape), x.dtype)
+        _check(self._ops.distie_sum_slices(x.data, x.slices, out.numel(), out,
                                            _CODES[x.dtype], self._stream()), "sum_slices")
         return out
 
@@ -926,8 +942,8 @@ class HipOps(Ops):
             self._packed_left_out += 1
             return
         row_map = row_map.to(device=self.device, dtype=torch.int32)
-        packed = torch.empty(self._packed_elements(N, K, gated), dtype=torch.bfloat16, device=self.device)
-        _check(self._ops.distie_pack_rows(weight.data_ptr(), packed.data_ptr(), row_map.data_ptr(),
+        packed = self._empty(self._packed_elements(N, K, gated), torch.bfloat16)
+        _check(self._ops.distie_pack_rows(weight, packed, row_map,
                                           row_map.numel() // 16, K, self._stream()), "pack_rows")
         torch.cuda.current_stream(self.device).synchronize()      # row_map is freed on return
         # the copy lives and dies with the weight
@@ -943,7 +959,6 @@ class HipOps(Ops):
         heads = kv_heads = dim = block_size = write = 0
         if rotary is not None:
             table, slots, k_cache, v_cache, heads, kv_heads, dim, block_size, write = rotary
-        ptr = lambda t: t.data_ptr() if t is not None else None
         norm_weight = x.weight
         if norm_weight.dtype != torch.float32:
             # the kernel takes the norm's weights in float32 (a bfloat16 value is one exactly); kept on the tensor
@@ -951,8 +966,8 @@ class HipOps(Ops):
             if norm_weight is None:
                 norm_weight = x.weight._distie_f32 = x.weight.float()
         _check(self._ops.distie_decode_norm_product(
-            x.residual.data_ptr(), norm_weight.data_ptr(), x.eps, packed.data_ptr(), ptr(bias),
-            out.data_ptr(), mode, M, N, K, ptr(table), ptr(slots), ptr(k_cache), ptr(v_cache), heads, kv_heads, dim,
+            x.residual, norm_weight, x.eps, packed, bias,
+            out, mode, M, N, K, table, slots, k_cache, v_cache, heads, kv_heads, dim,
             block_size, write, self._stream()), "decode_norm_product")
         return out
 
@@ -983,7 +998,7 @@ class HipOps(Ops):
             N, K = gate_up_weight.shape
             if packed.numel() != self._packed_elements(N, K, True):
                 raise KernelError("linear_silu_mul: the packed copy does not belong to this weight")
-            out = torch.empty((x.shape[0], N // 2), dtype=torch.bfloat16, device=self.device)
+            out = self._empty((x.shape[0], N // 2), torch.bfloat16)
             return self._norm_product(x, packed, None, out, gated, N)
         x = self.dense(x)
         M, K = x.shape
@@ -991,8 +1006,8 @@ class HipOps(Ops):
         if x.dtype == torch.float32 and gate_up_weight.dtype == torch.float32 and gate_up_weight.shape[1] == K and N % 2 == 0 and \
                 N * K >= self.ROWS_F32_MIN_ELEMENTS and self._ops.distie_rows_f32_slices(M, N, K, 1):
             self._own(x, gate_up_weight)
-            out = torch.empty((M, N // 2), dtype=torch.float32, device=self.device)
-            _check(self._ops.distie_rows_f32(x.data_ptr(), gate_up_weight.data_ptr(), None, out.data_ptr(), M, N, K, gated, 1,
+            out = self._empty((M, N // 2), torch.float32)
+            _check(self._ops.distie_rows_f32(x, gate_up_weight, None, out, M, N, K, gated, 1,
                                              *clamp, self._stream()), "rows_f32")
             return out
         plan, large = None, False
@@ -1008,13 +1023,13 @@ class HipOps(Ops):
             raise KernelError("linear_silu_mul: the packed copy does not belong to this weight")
         if plan is not None:
             return self._run_tiles(plan, x, packed, None, x.dtype, M, N, K, gated, clamp=clamp, large=large)
-        out = torch.empty((M, N // 2), dtype=x.dtype, device=self.device)
+        out = self._empty((M, N // 2), x.dtype)
         if M <= self.ONE_WAVE_MAX_ROWS:
-            _check(self._ops.distie_gemm_packed_bf16(x.data_ptr(), packed.data_ptr(), None, out.data_ptr(), _code(out),
+            _check(self._ops.distie_gemm_packed_bf16(x, packed, None, out, _code(out),
                                                      M, N, K, gated, *clamp, self._stream()), "gemm_packed_bf16")
         else:
             _check(self._ops.distie_gemm_packed_wide_bf16(
-                x.data_ptr(), packed.data_ptr(), None, out.data_ptr(), _code(out), M, N, K, gated,
+                x, packed, None, out, _code(out), M, N, K, gated,
                 self._pass_blocks(M, N * K), *clamp, self._stream()), "gemm_packed_wide_bf16")
         return out
 
@@ -1039,7 +1054,7 @@ class HipOps(Ops):
             if M != meta.num_tokens or slots.shape[0] != M:
                 raise KernelError("linear_rope_kv_write: rows do not match the batch")
             table = self._rope_table(meta, inv_freq)
-            out = torch.empty((M, N), dtype=torch.bfloat16, device=self.device)
+            out = self._empty((M, N), torch.bfloat16)
             return self._norm_product(x, packed, bias, out, 2, N, rotary=(
                 table, slots, k_cache, v_cache, num_heads, num_kv_heads, head_dim, meta.block_size, 1 if write else 0))
         x = self.dense(x)
@@ -1056,10 +1071,10 @@ class HipOps(Ops):
             if M != meta.num_tokens or slots.shape[0] != M:
                 raise KernelError("linear_rope_kv_write: rows do not match the batch")
             table = self._rope_table(meta, inv_freq)
-            out = torch.empty((M, N), dtype=torch.float32, device=self.device)
+            out = self._empty((M, N), torch.float32)
             _check(self._ops.distie_rows_f32_rotary(
-                x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
-                table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads, num_kv_heads,
+                x, weight, bias, out,
+                table, slots, k_cache, v_cache, M, K, num_heads, num_kv_heads,
                 head_dim, meta.block_size, 1 if write else 0, self._stream()), "rows_f32_rotary")
             return out
         plan, large = None, False
@@ -1091,9 +1106,9 @@ class HipOps(Ops):
             # slices) and the rotation with the cache write behind it adds the slices
             slices = self._ops.distie_gemm_packed_wide_slices(N, K)
             shape, dtype = ((M, N), torch.bfloat16) if slices == 1 else ((slices, M, N), torch.float32)
-            product = torch.empty(shape, dtype=dtype, device=self.device)
+            product = self._empty(shape, dtype)
             _check(self._ops.distie_gemm_packed_wide_qkv_bf16(
-                x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, product.data_ptr(),
+                x, packed, bias, product,
                 _code(product), M, K, num_heads, num_kv_heads, head_dim, self._pass_blocks(M, N * K), self._stream()),
                 "gemm_packed_wide_qkv_bf16")
             if slices > 1:
@@ -1101,18 +1116,18 @@ class HipOps(Ops):
             return self.rope_kv_write(product, meta, group, k_cache, v_cache, inv_freq, num_heads, num_kv_heads,
                                       head_dim, write)
         table = self._rope_table(meta, inv_freq)
-        out = torch.empty((M, N), dtype=torch.bfloat16, device=self.device)
+        out = self._empty((M, N), torch.bfloat16)
         if plan is not None:
             kernel, name = (self._ops.distie_large_tiles_rotary_bf16, "large_tiles_rotary_bf16") if large else \
                 (self._ops.distie_packed_tiles_rotary_bf16, "packed_tiles_rotary_bf16")
             _check(kernel(
-                x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
-                table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads,
+                x, packed, bias, out,
+                table, slots, k_cache, v_cache, M, K, num_heads,
                 num_kv_heads, head_dim, meta.block_size, 1 if write else 0, plan[0], self._stream()), name)
             return out
         _check(self._ops.distie_gemm_packed_rotary_bf16(
-            x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
-            table.data_ptr(), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), M, K, num_heads,
+            x, packed, bias, out,
+            table, slots, k_cache, v_cache, M, K, num_heads,
             num_kv_heads, head_dim, meta.block_size, 1 if write else 0, self._stream()), "gemm_packed_rotary_bf16")
         return out
 
@@ -1285,12 +1300,12 @@ class HipOps(Ops):
         """The tiled product; float32 slices if the plan cuts K."""
         shape, slices = plan
         columns = N // 2 if gated else N
-        out = torch.empty((M, columns), dtype=out_dtype, device=self.device) if slices == 1 else \
-            torch.empty((slices, M, columns), dtype=torch.float32, device=self.device)
+        out = self._empty((M, columns), out_dtype) if slices == 1 else \
+            self._empty((slices, M, columns), torch.float32)
         kernel, name = (self._ops.distie_large_tiles_bf16, "large_tiles_bf16") if large else \
             (self._ops.distie_packed_tiles_bf16, "packed_tiles_bf16")
         _check(kernel(
-            x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), _code(out),
+            x, packed, bias, out, _code(out),
             M, N, K, gated, shape, slices, *clamp, self._stream()), name)
         return out if slices == 1 else PartialSums(out, out_dtype)
 
@@ -1309,6 +1324,7 @@ class HipOps(Ops):
             lib.distie_lib_more_counts.restype = None
             with torch.cuda.device(self.device):
                 _check(lib.distie_lib_init(self._device_index), "lib_init")
+            calls.quicken(lib)
             self._lib = lib
         return self._lib
 
@@ -1338,7 +1354,7 @@ class HipOps(Ops):
             x = x.contiguous()
         if weight.stride(1) != 1 or weight.stride(0) != K:
             weight = weight.contiguous()
-        out = torch.empty((M, N), dtype=out_dtype, device=self.device)
+        out = self._empty((M, N), out_dtype)
         lib = self._library()
         code, size, w_size = _CODES[out_dtype], out.element_size(), weight.element_size()
         # The library's large bfloat16 kernels work on tiles of 256 x 256, one a compute unit at a time: a product
@@ -1389,8 +1405,8 @@ class HipOps(Ops):
         key = ("rope", inv_freq.data_ptr(), pairs)
         table = meta.scratch.get(key)
         if table is None:
-            table = torch.empty((meta.num_tokens, pairs, 2), dtype=torch.float32, device=self.device)
-            _check(self._ops.distie_rope_table(meta.positions.data_ptr(), inv_freq.data_ptr(), table.data_ptr(),
+            table = self._empty((meta.num_tokens, pairs, 2), torch.float32)
+            _check(self._ops.distie_rope_table(meta.positions, inv_freq, table,
                                                meta.num_tokens, pairs, self._stream()), "rope_table")
             meta.scratch[key] = table
         return table
@@ -1403,7 +1419,7 @@ class HipOps(Ops):
             N, K = weight.shape
             if packed.numel() != self._packed_elements(N, K, False):
                 raise KernelError("linear: the packed copy does not belong to this weight")
-            out = torch.empty((x.shape[0], N), dtype=torch.float32, device=self.device)
+            out = self._empty((x.shape[0], N), torch.float32)
             return self._norm_product(x, packed, None, out, 0, N)
         x = self.dense(x)
         self._own(x, weight, bias)
@@ -1432,11 +1448,11 @@ class HipOps(Ops):
                 raise KernelError("linear: the packed copy does not belong to this weight")
             slices = self._ops.distie_gemm_packed_wide_slices(N, K)
             if slices == 1:
-                out = torch.empty((M, N), dtype=out_dtype, device=self.device)
+                out = self._empty((M, N), out_dtype)
             else:
-                out = torch.empty((slices, M, N), dtype=torch.float32, device=self.device)
+                out = self._empty((slices, M, N), torch.float32)
             _check(self._ops.distie_gemm_packed_wide_bf16(
-                x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                x, packed, bias, out,
                 _code(out), M, N, K, 0, self._pass_blocks(M, N * K), 0.0, 1.0, 0.0, self._stream()),
                 "gemm_packed_wide_bf16")
             if slices == 1:
@@ -1448,16 +1464,16 @@ class HipOps(Ops):
                     raise KernelError("linear: the packed copy does not belong to this weight")
             slices = self._ops.distie_gemm_skinny_slices(M, N, K)       # the same cut for both kernels
             if slices == 1:
-                out = torch.empty((M, N), dtype=out_dtype, device=self.device)
+                out = self._empty((M, N), out_dtype)
             else:
-                out = torch.empty((slices, M, N), dtype=torch.float32, device=self.device)
+                out = self._empty((slices, M, N), torch.float32)
             if packed is not None:
                 _check(self._ops.distie_gemm_packed_bf16(
-                    x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                    x, packed, bias, out,
                     _code(out), M, N, K, 0, 0.0, 1.0, 0.0, self._stream()), "gemm_packed_bf16")
             else:
                 _check(self._ops.distie_gemm_skinny_bf16(
-                    x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                    x, weight, bias, out,
                     _code(out), M, N, K, self._stream()), "gemm_skinny_bf16")
             if slices == 1:
                 return out
@@ -1482,21 +1498,21 @@ class HipOps(Ops):
             # TB/s as it is): the weights streamed through the matrix cores' float32 products
             slices = self._ops.distie_rows_f32_slices(M, N, K, 0) if self._rows_f32_take(M, N, K) else 0
             if slices:
-                out = torch.empty((M, N) if slices == 1 else (slices, M, N), dtype=torch.float32, device=self.device)
+                out = self._empty((M, N) if slices == 1 else (slices, M, N), torch.float32)
                 _check(self._ops.distie_rows_f32(
-                    x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), M, N, K,
+                    x, weight, bias, out, M, N, K,
                     0, slices, 0.0, 1.0, 0.0, self._stream()), "rows_f32")
                 return out if slices == 1 else PartialSums(out, out_dtype)
-        out = torch.empty((M, N), dtype=out_dtype, device=self.device)
+        out = self._empty((M, N), out_dtype)
         if M <= self.ROWS_MAX_ROWS and K % 8 == 0:
             # few rows in float32 (or against a weight kept in float32): the weights are streamed, FMAs only
             _check(self._ops.distie_gemv_rows(
-                x.data_ptr(), _code(x), weight.data_ptr(), _code(weight), bias.data_ptr() if bias is not None else None,
-                out.data_ptr(), _CODES[out_dtype], M, N, K, self._stream()), "gemv_rows")
+                x, _code(x), weight, _code(weight), bias,
+                out, _CODES[out_dtype], M, N, K, self._stream()), "gemv_rows")
             return out
         _check(self._ops.distie_gemm_generic(
-            x.data_ptr(), _code(x), weight.data_ptr(), _code(weight), bias.data_ptr() if bias is not None else None,
-            out.data_ptr(), _CODES[out_dtype], M, N, K, self._stream()), "gemm_generic")
+            x, _code(x), weight, _code(weight), bias,
+            out, _CODES[out_dtype], M, N, K, self._stream()), "gemm_generic")
         return out
 
     def _rows_f32_take(self, M, N, K) -> bool:
@@ -1527,9 +1543,9 @@ class HipOps(Ops):
             raise KernelError("linear: bias must be float32 [N]")
         if packed.numel() != self._packed_elements(N, K, False):
             raise KernelError("linear: the packed copy does not belong to this weight")
-        out = torch.empty((M, N), dtype=x.dtype, device=self.device)
+        out = self._empty((M, N), x.dtype)
         _check(self._ops.distie_gemm_packed_bf16(
-            x.data_ptr(), packed.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), _code(out), M, N, K,
+            x, packed, bias, out, _code(out), M, N, K,
             2, 0.0, 1.0, 0.0, self._stream()), "gemm_packed_bf16")
         return out
 
@@ -1538,7 +1554,7 @@ class HipOps(Ops):
             return self._linear(x, weight, bias, torch.float32, partial_ok=True)
         out = self._linear(x, weight, bias, torch.float32)
         if scale != 1.0:
-            _check(self._ops.distie_scale_f32(out.data_ptr(), out.numel(), float(scale), self._stream()), "scale_f32")
+            _check(self._ops.distie_scale_f32(out, out.numel(), float(scale), self._stream()), "scale_f32")
         return out
 
     def rope_kv_write(self, qkv, meta: BatchMeta, group, k_cache, v_cache, inv_freq, num_heads, num_kv_heads,
@@ -1548,7 +1564,7 @@ class HipOps(Ops):
         slices, source = 1, qkv
         if isinstance(qkv, PartialSums):
             slices, source = qkv.slices, qkv.data
-            out = torch.empty(tuple(qkv.shape), dtype=qkv.dtype, device=self.device)
+            out = self._empty(tuple(qkv.shape), qkv.dtype)
         else:
             out = qkv
         self._own(source, k_cache, v_cache, inv_freq)
@@ -1562,10 +1578,10 @@ class HipOps(Ops):
         slots = meta.groups[group].slots
         table = self._rope_table(meta, inv_freq) if pairs else None
         _check(self._ops.distie_rope_kv_write(
-            source.data_ptr(), _code(source), slices, out.data_ptr(), _code(out),
-            table.data_ptr() if table is not None else None, meta.positions.data_ptr(),
-            slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
-            inv_freq.data_ptr() if inv_freq is not None else None, pairs, T, num_heads, num_kv_heads, head_dim,
+            source, _code(source), slices, out, _code(out),
+            table, meta.positions,
+            slots, k_cache, v_cache, _code(k_cache),
+            inv_freq, pairs, T, num_heads, num_kv_heads, head_dim,
             meta.block_size, 1 if write else 0, self._stream()), "rope_kv_write")
         _mark_written(out)
         return out
@@ -1586,8 +1602,8 @@ class HipOps(Ops):
         if T != meta.num_tokens or (rows is None and table.shape[0] != meta.num_requests) or \
                 (rows is not None and rows.shape[0] != meta.num_requests):
             raise KernelError("paged_attention: tensors do not match the batch")
-        rows_ptr = rows.data_ptr() if rows is not None else None
-        out = torch.empty((T, num_heads * head_dim), dtype=qkv.dtype, device=self.device)
+        rows_ptr = rows
+        out = self._empty((T, num_heads * head_dim), qkv.dtype)
         plain = extras is None or not extras.bends_scores
         slopes, cap = (None, 0.0) if plain else (extras.head_slopes, float(extras.score_cap or 0.0))
         sinks = extras.sinks if extras is not None else None
@@ -1596,7 +1612,7 @@ class HipOps(Ops):
                 self._own(vector)
                 if vector.dtype != torch.float32 or tuple(vector.shape) != (num_heads,):
                     raise KernelError(f"paged_attention: {name} must be float32 [num_heads]")
-        sinks_ptr = sinks.data_ptr() if sinks is not None else None
+        sinks_ptr = sinks
         chunk = extras.chunk if extras is not None else 0
         if chunk and (window or extras.mixes_heads):
             raise KernelError("paged_attention: chunks do not go with a window or with mixed heads")
@@ -1618,28 +1634,28 @@ class HipOps(Ops):
                 plan = meta.scratch[key] = self._attention_plan(lib, meta, T, num_heads, num_kv_heads, head_dim, abs(reach))
             if plan["decode"]:
                 _check(lib.distie_attention_decode_bf16(
-                    qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.kv_len.data_ptr(),
-                    meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(),
-                    plan["decode_o"].data_ptr(), plan["decode_ml"].data_ptr(), meta.num_requests, num_heads,
+                    qkv, qkv.shape[1], k_cache, v_cache, meta.kv_len,
+                    meta.cu_q, table, table.shape[1], rows_ptr, out,
+                    plan["decode_o"], plan["decode_ml"], meta.num_requests, num_heads,
                     num_kv_heads, meta.block_size, float(scale), reach, plan["split_len"],
                     plan["max_splits"], 1 if meta.all_decode else 0,
-                    plan["run_len"].data_ptr() if plan["run_len"] is not None else None, sinks_ptr, plan["together"],
+                    plan["run_len"], sinks_ptr, plan["together"],
                     self._stream()), "attention_decode_bf16")
             if plan["prefill"] and plan["waves"]:
                 _check(lib.distie_attention_prefill_keys(
-                    qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
-                    meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
+                    qkv, qkv.shape[1], k_cache, v_cache, meta.positions,
+                    meta.cu_q, table, table.shape[1], rows_ptr, out, T, meta.num_requests,
                     num_heads, num_kv_heads, meta.block_size, float(scale), reach, 2 if plan["decode"] else 1, sinks_ptr,
                     plan["waves"], self._stream()), "attention_prefill_keys")
             elif plan["prefill"]:
                 parts = plan["parts"]
                 _check(lib.distie_attention_prefill_bf16(
-                    qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
-                    meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
+                    qkv, qkv.shape[1], k_cache, v_cache, meta.positions,
+                    meta.cu_q, table, table.shape[1], rows_ptr, out, T, meta.num_requests,
                     num_heads, num_kv_heads, meta.block_size, float(scale), reach,
-                    2 if plan["decode"] else 1, meta.token_request.data_ptr(),
-                    plan["prefill_o"].data_ptr() if parts > 1 else None,
-                    plan["prefill_ml"].data_ptr() if parts > 1 else None, parts, sinks_ptr, self._stream()),
+                    2 if plan["decode"] else 1, meta.token_request,
+                    plan["prefill_o"] if parts > 1 else None,
+                    plan["prefill_ml"] if parts > 1 else None, parts, sinks_ptr, self._stream()),
                     "attention_prefill_bf16")
             return out
         f32 = qkv.dtype == torch.float32 and k_cache.dtype == torch.float32
@@ -1653,11 +1669,11 @@ class HipOps(Ops):
                 plan = meta.scratch[key] = self._prefill_parts(meta, T, meta.max_kv, num_heads, head_dim, abs(reach))
             parts = plan["parts"]
             _check(lib.distie_attention_prefill_f32(
-                qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
-                meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
+                qkv, qkv.shape[1], k_cache, v_cache, meta.positions,
+                meta.cu_q, table, table.shape[1], rows_ptr, out, T, meta.num_requests,
                 num_heads, num_kv_heads, meta.block_size, float(scale), reach, 1,
-                meta.token_request.data_ptr(), plan["prefill_o"].data_ptr() if parts > 1 else None,
-                plan["prefill_ml"].data_ptr() if parts > 1 else None, parts, sinks_ptr, self._stream()),
+                meta.token_request, plan["prefill_o"] if parts > 1 else None,
+                plan["prefill_ml"] if parts > 1 else None, parts, sinks_ptr, self._stream()),
                 "attention_prefill_f32")
             return out
         columns, runs, per, waves = 0, 1, 0, 0
@@ -1673,18 +1689,18 @@ class HipOps(Ops):
         if columns:
             # wide heads, or many tokens: a tile of tokens and a kv head's query heads are the columns of matrix products
             _check(lib.distie_attention_columns_f32(
-                qkv.data_ptr(), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
-                meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), T, meta.num_requests,
+                qkv, qkv.shape[1], k_cache, v_cache, meta.positions,
+                meta.cu_q, table, table.shape[1], rows_ptr, out, T, meta.num_requests,
                 num_heads, num_kv_heads, meta.block_size, float(scale), reach, sinks_ptr,
-                part_o.data_ptr() if runs > 1 else None, part_ml.data_ptr() if runs > 1 else None, runs, self._stream()),
+                part_o if runs > 1 else None, part_ml if runs > 1 else None, runs, self._stream()),
                 "attention_columns_f32")
             return out
         _check(lib.distie_attention_generic(
-            qkv.data_ptr(), _code(qkv), qkv.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
-            meta.positions.data_ptr(), meta.token_request.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr,
-            out.data_ptr(), T, num_heads, num_kv_heads, meta.block_size, float(scale), reach,
-            slopes.data_ptr() if slopes is not None else None, cap, sinks_ptr, part_o.data_ptr() if runs > 1 else None,
-            part_ml.data_ptr() if runs > 1 else None, runs, per, waves, self._stream()), "attention_generic")
+            qkv, _code(qkv), qkv.shape[1], k_cache, v_cache, _code(k_cache),
+            meta.positions, meta.token_request, table, table.shape[1], rows_ptr,
+            out, T, num_heads, num_kv_heads, meta.block_size, float(scale), reach,
+            slopes, cap, sinks_ptr, part_o if runs > 1 else None,
+            part_ml if runs > 1 else None, runs, per, waves, self._stream()), "attention_generic")
         return out
 
     def _mixed_attention(self, q, meta: BatchMeta, table, rows_ptr, k_cache, v_cache, out, num_heads, num_kv_heads, head_dim,
@@ -1702,7 +1718,6 @@ class HipOps(Ops):
             raise KernelError("paged_attention: head_mix must be [num_heads, num_heads]")
         if q.shape[1] != num_heads * head_dim:
             raise KernelError("paged_attention: mixed heads take q alone")
-        ptr = lambda t: t.data_ptr() if t is not None else None
         keep = int(extras.keep_first) if window else 0
         if q.dtype == torch.bfloat16 and k_cache.dtype == torch.bfloat16 and meta.block_size % 16 == 0 and \
                 head_dim % 32 == 0 and head_dim <= self.LARGEST_MATRIX_CORE_HEAD:
@@ -1717,21 +1732,21 @@ class HipOps(Ops):
                 if queries == 16 and q.shape[0] < self.MIXED_WIDE_TOKENS:
                     queries = 8
                 _check(lib.distie_mixed_attention_bf16(
-                    q.data_ptr(), q.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), meta.positions.data_ptr(),
-                    meta.cu_q.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr, out.data_ptr(), q.shape[0],
+                    q, q.shape[1], k_cache, v_cache, meta.positions,
+                    meta.cu_q, table, table.shape[1], rows_ptr, out, q.shape[0],
                     meta.num_requests, num_heads, num_kv_heads, meta.block_size, float(scale), int(window or 0), keep,
-                    float(extras.score_cap or 0.0), ptr(bias), bias.shape[1] if bias is not None else 0, ptr(mix),
-                    ptr(extras.sinks), 1 if plan["prefill"] else 0, queries, (2 if meta.all_decode else 1) if plan["decode"] else 0, plan["splits"],
-                    ptr(plan["partial_o"]), ptr(plan["partial_ml"]), self._stream()), "mixed_attention_bf16")
+                    float(extras.score_cap or 0.0), bias, bias.shape[1] if bias is not None else 0, mix,
+                    extras.sinks, 1 if plan["prefill"] else 0, queries, (2 if meta.all_decode else 1) if plan["decode"] else 0, plan["splits"],
+                    plan["partial_o"], plan["partial_ml"], self._stream()), "mixed_attention_bf16")
                 return
         if not self._ops.distie_mixed_attention_fits(num_heads, head_dim):
             raise KernelError(f"paged_attention: {num_heads} mixed heads of {head_dim} do not fit the LDS of a compute unit")
         _check(self._ops.distie_mixed_attention_generic(
-            q.data_ptr(), _code(q), q.shape[1], k_cache.data_ptr(), v_cache.data_ptr(), _code(k_cache),
-            meta.positions.data_ptr(), meta.token_request.data_ptr(), table.data_ptr(), table.shape[1], rows_ptr,
-            out.data_ptr(), q.shape[0], num_heads, num_kv_heads, head_dim, meta.block_size, float(scale), int(window or 0),
-            keep, float(extras.score_cap or 0.0), ptr(bias), bias.shape[1] if bias is not None else 0, ptr(mix),
-            ptr(extras.sinks), self._stream()), "mixed_attention_generic")
+            q, _code(q), q.shape[1], k_cache, v_cache, _code(k_cache),
+            meta.positions, meta.token_request, table, table.shape[1], rows_ptr,
+            out, q.shape[0], num_heads, num_kv_heads, head_dim, meta.block_size, float(scale), int(window or 0),
+            keep, float(extras.score_cap or 0.0), bias, bias.shape[1] if bias is not None else 0, mix,
+            extras.sinks, self._stream()), "mixed_attention_generic")
 
     def _mixed_plan(self, lib, meta: BatchMeta, num_heads, head_dim, window, keep) -> dict:
         """Which of the mixed heads' kernels a step needs, and the buffers for partial results of single tokens (one
@@ -1750,8 +1765,8 @@ class HipOps(Ops):
                 splits = min(splits, -(-keep // run) + (int(window) + run - 2) // run + 1)
             plan["splits"] = max(1, splits)
             shape = (meta.num_requests, plan["splits"], num_heads)
-            plan["partial_o"] = torch.empty((*shape, head_dim), dtype=torch.float32, device=self.device)
-            plan["partial_ml"] = torch.empty((*shape, 2), dtype=torch.float32, device=self.device)
+            plan["partial_o"] = self._empty((*shape, head_dim), torch.float32)
+            plan["partial_ml"] = self._empty((*shape, 2), torch.float32)
         return plan
 
     COLUMNS_KEYS = 32                # a window's keys begin anywhere in a chunk of so many
@@ -1791,8 +1806,8 @@ class HipOps(Ops):
         held = meta.scratch.get(key)
         if held is None:
             held = meta.scratch[key] = (
-                torch.empty((runs, T, num_heads, head_dim), dtype=torch.float32, device=self.device),
-                torch.empty((runs, T, num_heads, 2), dtype=torch.float32, device=self.device))
+                self._empty((runs, T, num_heads, head_dim), torch.float32),
+                self._empty((runs, T, num_heads, 2), torch.float32))
         return held
 
     def _attention_plan(self, lib, meta: BatchMeta, T, num_heads, num_kv_heads, head_dim, window) -> dict:
@@ -1821,19 +1836,17 @@ class HipOps(Ops):
             if meta.all_decode and not window and max_splits * pairs <= self.DECODE_SHARED_BELOW * self.DECODE_WAVES:
                 splits = max_splits
                 max_splits = max(1, min(self.DECODE_MAX_RUNS, 2 * splits, -(-visible // 64)))
-                plan["run_len"] = torch.empty(1, dtype=torch.int32, device=self.device)
-                _check(lib.distie_attention_decode_run_len(meta.kv_len.data_ptr(), meta.num_requests,
+                plan["run_len"] = self._empty(1, torch.int32)
+                _check(lib.distie_attention_decode_run_len(meta.kv_len, meta.num_requests,
                                                            max(1, self.DECODE_WAVES // num_kv_heads), max_splits,
-                                                           plan["run_len"].data_ptr(), self._stream()),
+                                                           plan["run_len"], self._stream()),
                        "attention_decode_run_len")
             plan["max_splits"] = max_splits
             # many runs: a workgroup puts consecutive ones together before it writes their result
             plan["together"] = together = lib.distie_attention_decode_together(max_splits, group, pairs)
             places = -(-max_splits // together)
-            plan["decode_o"] = torch.empty((meta.num_requests, num_heads, places, head_dim), dtype=torch.float32,
-                                           device=self.device)
-            plan["decode_ml"] = torch.empty((meta.num_requests, num_heads, places, 2), dtype=torch.float32,
-                                            device=self.device)
+            plan["decode_o"] = self._empty((meta.num_requests, num_heads, places, head_dim), torch.float32)
+            plan["decode_ml"] = self._empty((meta.num_requests, num_heads, places, 2), torch.float32)
         plan["prefill"] = singles < meta.num_requests or not plan["decode"] or \
             (meta.singles_bound is not None and not meta.all_decode)
         if plan["prefill"]:
@@ -1892,8 +1905,8 @@ class HipOps(Ops):
         parts = max(parts, min(wanted, visible // 128, 16))
         plan = {"parts": parts}
         if parts > 1:
-            plan["prefill_o"] = torch.empty((parts, T, num_heads, head_dim), dtype=torch.float32, device=self.device)
-            plan["prefill_ml"] = torch.empty((parts, T, num_heads, 2), dtype=torch.float32, device=self.device)
+            plan["prefill_o"] = self._empty((parts, T, num_heads, head_dim), torch.float32)
+            plan["prefill_ml"] = self._empty((parts, T, num_heads, 2), torch.float32)
         return plan
 
     # ---- residual streams, convolutions over time, decayed states, gates (csrc/sequence.hip)
@@ -1921,7 +1934,7 @@ class HipOps(Ops):
             count = (read if read is not None else write).shape[0]
             if init.dtype != torch.float32 or init.dim() != 2:
                 raise KernelError("hyper_step: init must be float32 [T, C]")
-            streams = torch.empty((init.shape[0], count, init.shape[1]), dtype=torch.float32, device=self.device)
+            streams = self._empty((init.shape[0], count, init.shape[1]), torch.float32)
         self._own(streams, mix, write, read, norm_weight)
         if streams.dtype != torch.float32 or streams.dim() != 3:
             raise KernelError("hyper_step: streams must be float32 [T, S, C]")
@@ -1959,12 +1972,11 @@ class HipOps(Ops):
         if read is not None:
             if norm != "none" and (norm_weight is None or tuple(norm_weight.shape) != (C,)):
                 raise KernelError("hyper_step: the norm needs a weight [C]")
-            h = torch.empty((T, C), dtype=out_dtype or torch.float32, device=self.device)
-        ptr = lambda t: t.data_ptr() if t is not None else None
+            h = self._empty((T, C), out_dtype or torch.float32)
         _check(self._ops.distie_hyper_step(
-            streams.data_ptr(), S, ptr(init), y, y_code, slices, g_ptr, g_code, g_ld, g_slices, ptr(mix), ptr(write), ptr(read),
-            ptr(norm_weight), _code(norm_weight) if norm_weight is not None else _F32, self.NORM_KINDS[norm], float(eps),
-            ptr(h), _code(h) if h is not None else _F32, T, C, self._stream()), "hyper_step")
+            streams, S, init, y, y_code, slices, g_ptr, g_code, g_ld, g_slices, mix, write, read,
+            norm_weight, _code(norm_weight) if norm_weight is not None else _F32, self.NORM_KINDS[norm], float(eps),
+            h, _code(h) if h is not None else _F32, T, C, self._stream()), "hyper_step")
         _mark_written(streams)
         return streams, h
 
@@ -1981,18 +1993,18 @@ class HipOps(Ops):
         if bias is not None and (bias.dtype != torch.float32 or tuple(bias.shape) != (N,)):
             raise KernelError("causal_conv: bias must be float32 [channels]")
         self._check_conv_state(state, taps, N)
-        out = torch.empty((T, N), dtype=x.dtype, device=self.device)
+        out = self._empty((T, N), x.dtype)
         _check(self._ops.distie_causal_conv(
-            x_ptr, _code(x), ldx, weight.data_ptr(), _code(weight), taps, state.data_ptr() if taps > 1 else None,
-            out.data_ptr(), _code(out), N, (1 if residual else 0) | (0 if act is None else (self.ACTIVATIONS[act] + 1) << 1),
-            bias.data_ptr() if bias is not None else None,
-            meta.cu_q.data_ptr(), meta.token_request.data_ptr(), meta.state_slots.data_ptr(), T, N, self._stream()),
+            x_ptr, _code(x), ldx, weight, _code(weight), taps, state if taps > 1 else None,
+            out, _code(out), N, (1 if residual else 0) | (0 if act is None else (self.ACTIVATIONS[act] + 1) << 1),
+            bias,
+            meta.cu_q, meta.token_request, meta.state_slots, T, N, self._stream()),
             "causal_conv")
         if taps > 1 and not meta.all_decode:
             # requests that bring one row moved their state on in the kernel above; the others here, once all
             # rows of the step have read the old one
-            _check(self._ops.distie_conv_state(x_ptr, _code(x), ldx, taps, state.data_ptr(), meta.cu_q.data_ptr(),
-                                               meta.state_slots.data_ptr(), meta.num_requests, N, 1, self._stream()),
+            _check(self._ops.distie_conv_state(x_ptr, _code(x), ldx, taps, state, meta.cu_q,
+                                               meta.state_slots, meta.num_requests, N, 1, self._stream()),
                    "conv_state")
         if taps > 1:
             _mark_written(state)
@@ -2041,22 +2053,21 @@ class HipOps(Ops):
                 raise KernelError("conv_rope_kv_write: keys and values are cached in one dtype")
         pairs = 0 if inv_freq is None else inv_freq.shape[0]
         table = self._rope_table(meta, inv_freq) if pairs else None
-        q = torch.empty((T, num_heads * padded_dim), dtype=q_dtype, device=self.device)
-        ptr = lambda t: t.data_ptr() if t is not None else None
+        q = self._empty((T, num_heads * padded_dim), q_dtype)
         _check(self._ops.distie_conv_rope_kv_write(
-            product.data_ptr(), _code(product), W, ptr(conv_weight), _code(conv_weight) if conv_weight is not None else _F32,
-            taps, ptr(state) if taps > 1 else None, ptr(table), pairs, float(magnitude), q.data_ptr(),
-            ptr(k_cache) if write else None, ptr(v_cache) if write else None, _code(k_cache) if write else _code(product),
-            meta.groups[group].slots.data_ptr() if write else None, meta.cu_q.data_ptr(), meta.token_request.data_ptr(),
-            meta.state_slots.data_ptr(), T, num_heads, num_kv_heads, dim, value_dim, padded_dim, meta.block_size,
-            2 if keys_are_values else (1 if has_kv else 0), 1 if write else 0, meta.positions.data_ptr(), float(q_temp[0]) if q_temp else 0.0,
-            int(q_temp[1]) if q_temp else 0, ptr(q_norm), ptr(k_norm) if has_kv else None, float(norm_eps),
+            product, _code(product), W, conv_weight, _code(conv_weight) if conv_weight is not None else _F32,
+            taps, state if taps > 1 else None, table, pairs, float(magnitude), q,
+            k_cache if write else None, v_cache if write else None, _code(k_cache) if write else _code(product),
+            meta.groups[group].slots if write else None, meta.cu_q, meta.token_request,
+            meta.state_slots, T, num_heads, num_kv_heads, dim, value_dim, padded_dim, meta.block_size,
+            2 if keys_are_values else (1 if has_kv else 0), 1 if write else 0, meta.positions, float(q_temp[0]) if q_temp else 0.0,
+            int(q_temp[1]) if q_temp else 0, q_norm, k_norm if has_kv else None, float(norm_eps),
             slices, _CODES[q_dtype], 1 if neighbours else 0, self._stream()), "conv_rope_kv_write")
         if taps > 1:
             if not meta.all_decode:
                 # (requests that bring one row had their state moved on by the kernel above)
-                _check(self._ops.distie_conv_state(product.data_ptr(), _code(product), W, taps, state.data_ptr(),
-                                                   meta.cu_q.data_ptr(), meta.state_slots.data_ptr(), meta.num_requests,
+                _check(self._ops.distie_conv_state(product, _code(product), W, taps, state,
+                                                   meta.cu_q, meta.state_slots, meta.num_requests,
                                                    channels, 1, self._stream()), "conv_state")
             _mark_written(state)
         return q
@@ -2071,15 +2082,15 @@ class HipOps(Ops):
             if gates is None:
                 raise KernelError("sigmoid_gate: a gate for each head needs the gates")
             g_ptr, g_ld = self._rows_view(gates, num_heads)
-            out = torch.empty((T, num_heads * width), dtype=x.dtype, device=self.device)
-            _check(self._ops.distie_head_gate(x.data_ptr(), _code(x), head_stride, width, g_ptr, _code(gates), g_ld,
-                                              out.data_ptr(), _code(out), T, num_heads * width, self._stream()), "head_gate")
+            out = self._empty((T, num_heads * width), x.dtype)
+            _check(self._ops.distie_head_gate(x, _code(x), head_stride, width, g_ptr, _code(gates), g_ld,
+                                              out, _code(out), T, num_heads * width, self._stream()), "head_gate")
             return out
         g_ptr, g_ld = self._rows_view(gates, num_heads * width) if gates is not None else (None, 0)
-        out = torch.empty((T, num_heads * width), dtype=x.dtype, device=self.device)
-        _check(self._ops.distie_sigmoid_gate(x.data_ptr(), _code(x), head_stride, width, g_ptr,
+        out = self._empty((T, num_heads * width), x.dtype)
+        _check(self._ops.distie_sigmoid_gate(x, _code(x), head_stride, width, g_ptr,
                                              _code(gates) if gates is not None else _code(x), g_ld,
-                                             out.data_ptr(), _code(out), T, num_heads * width, self._stream()),
+                                             out, _code(out), T, num_heads * width, self._stream()),
                "sigmoid_gate")
         return out
 
@@ -2103,8 +2114,7 @@ class HipOps(Ops):
         key = ("scan_chunks", rows, num_heads, dim, value_dim)
         scratch = meta.scratch.get(key)
         if scratch is None:
-            scratch = meta.scratch[key] = torch.empty((count, num_heads, dim, value_dim), dtype=torch.float32,
-                                                      device=self.device)
+            scratch = meta.scratch[key] = self._empty((count, num_heads, dim, value_dim), torch.float32)
         return count, packed, scratch
 
     def decay_scan(self, product, state, decay, meta, num_heads, dim, value_dim, act="silu", k_scale=1.0, inv_freq=None,
@@ -2127,7 +2137,7 @@ class HipOps(Ops):
             raise KernelError("decay_scan: the rotation turns more dimensions than a head has")
         table = self._rope_table(meta, inv_freq) if pairs else None
         turn = (1 if act else 0, table.data_ptr() if pairs else None, pairs, 1 if neighbours else 0, float(k_scale))
-        out = torch.empty((T, num_heads * value_dim), dtype=torch.float32, device=self.device)
+        out = self._empty((T, num_heads * value_dim), torch.float32)
         if not self.captured and meta.host_cu_q is not None and meta.max_q >= self.SCAN_CHUNKED_MIN_ROWS and \
                 dim <= self._ops.distie_decay_scan_chunked_max_dim():
             # portions of prompts: chunks of rows side by side instead of one row after the other. Which rows form
@@ -2135,13 +2145,13 @@ class HipOps(Ops):
             count, packed, scratch = self._scan_chunks(meta, self._ops.distie_decay_scan_chunk_rows(), num_heads, dim,
                                                        value_dim)
             _check(self._ops.distie_decay_scan_chunked(
-                product.data_ptr(), _code(product), W, state.data_ptr(), decay.data_ptr(), out.data_ptr(),
-                scratch.data_ptr(), packed.data_ptr(), packed.data_ptr() + 16 * count, meta.state_slots.data_ptr(),
+                product, _code(product), W, state, decay, out,
+                scratch, packed, packed.data_ptr() + 16 * count, meta.state_slots,
                 count, meta.num_requests, num_heads, dim, value_dim, *turn, self._stream()), "decay_scan_chunked")
             _mark_written(state)
             return out
-        _check(self._ops.distie_decay_scan(product.data_ptr(), _code(product), W, state.data_ptr(), decay.data_ptr(),
-                                           out.data_ptr(), meta.cu_q.data_ptr(), meta.state_slots.data_ptr(),
+        _check(self._ops.distie_decay_scan(product, _code(product), W, state, decay,
+                                           out, meta.cu_q, meta.state_slots,
                                            meta.num_requests, num_heads, dim, value_dim, *turn, self._stream()),
                "decay_scan")
         _mark_written(state)
@@ -2161,9 +2171,9 @@ class HipOps(Ops):
             T, N = x.shape
             size = group or N
             g_ptr, g_ld = self._rows_view(gates, N)
-            out = torch.empty((T, N), dtype=out_dtype, device=self.device)
-            _check(self._ops.distie_gate_rmsnorm(x.data_ptr(), weight.data_ptr(), _code(weight), float(eps), g_ptr,
-                                                 _code(gates), g_ld, out.data_ptr(), _code(out), T, size, N // size,
+            out = self._empty((T, N), out_dtype)
+            _check(self._ops.distie_gate_rmsnorm(x, weight, _code(weight), float(eps), g_ptr,
+                                                 _code(gates), g_ld, out, _code(out), T, size, N // size,
                                                  1 if gate == "silu" else 0, self._stream()), "gate_rmsnorm")
             return out
         if x.dtype != torch.float32 or x.dim() != 2 or (group is not None and (group < 1 or x.shape[1] % group)) or \
@@ -2174,10 +2184,10 @@ class HipOps(Ops):
         if gates is not None:
             g_ptr, g_ld = self._rows_view(gates, N)
             g_code = _code(gates)
-        out = torch.empty((T, N), dtype=out_dtype, device=self.device)
+        out = self._empty((T, N), out_dtype)
         size = group or N
-        _check(self._ops.distie_rmsnorm_gate(x.data_ptr(), weight.data_ptr(), _code(weight), float(eps), g_ptr, g_code,
-                                             g_ld, out.data_ptr(), _code(out), T, size, N // size,
+        _check(self._ops.distie_rmsnorm_gate(x, weight, _code(weight), float(eps), g_ptr, g_code,
+                                             g_ld, out, _code(out), T, size, N // size,
                                              1 if gate == "silu" else 0, 1 if weight.shape[0] != size else 0,
                                              self._stream()), "rmsnorm_gate")
         return out
@@ -2210,18 +2220,17 @@ class HipOps(Ops):
                 raise KernelError("norm chain: the residual is float32 [T, C]")
         out = y = None
         if residual is None:
-            y = torch.empty((T, C), dtype=torch.float32, device=self.device)
+            y = self._empty((T, C), torch.float32)
         elif out_dtype is not None:
             # with a norm in front of the next sub-layer (`pre`), or the new residual as it is, in `out_dtype`
-            out = torch.empty((T, C), dtype=out_dtype, device=self.device)
+            out = self._empty((T, C), out_dtype)
         (t0, s0), (t1, s1) = held[0], (held[1] if len(held) > 1 else (None, 1))
-        ptr = lambda t: t.data_ptr() if t is not None else None
         _check(self._ops.distie_norm_chain(
-            t0.data_ptr(), _code(t0), s0, ptr(weights[0]) if weights else None, ptr(t1), _code(t1) if t1 is not None else _F32,
-            s1, ptr(weights[1]) if weights and len(weights) > 1 else None, float(term_eps), float(scale),
-            ptr(post[0]) if post else None, float(post[1]) if post else 0.0, ptr(residual),
-            ptr(pre[0]) if pre else None, float(pre[1]) if pre else 0.0, ptr(out), _code(out) if out is not None else _F32,
-            ptr(y), T, C, self._stream()), "norm_chain")
+            t0, _code(t0), s0, weights[0] if weights else None, t1, _code(t1) if t1 is not None else _F32,
+            s1, weights[1] if weights and len(weights) > 1 else None, float(term_eps), float(scale),
+            post[0] if post else None, float(post[1]) if post else 0.0, residual,
+            pre[0] if pre else None, float(pre[1]) if pre else 0.0, out, _code(out) if out is not None else _F32,
+            y, T, C, self._stream()), "norm_chain")
         if residual is not None:
             _mark_written(residual)
         return out if residual is not None else y
@@ -2257,8 +2266,8 @@ class HipOps(Ops):
             raise KernelError("read_residual reads the float32 residual stream")
         if out_dtype == torch.float32:
             return residual
-        out = torch.empty(residual.shape, dtype=out_dtype, device=self.device)
-        _check(self._ops.distie_sum_slices(residual.data_ptr(), 1, out.numel(), out.data_ptr(), _CODES[out_dtype],
+        out = self._empty(residual.shape, out_dtype)
+        _check(self._ops.distie_sum_slices(residual, 1, out.numel(), out, _CODES[out_dtype],
                                            self._stream()), "sum_slices")
         return out
 
@@ -2301,24 +2310,24 @@ class HipOps(Ops):
         if decay_logits is not None and (decay_logits.dtype != torch.float32 or
                                          tuple(decay_logits.shape) != (T, num_heads * dim)):
             raise KernelError("gated_decay_scan: the decay's logits are float32 [T, heads * dim]")
-        out = torch.empty((T, num_heads * value_dim), dtype=torch.float32, device=self.device)
+        out = self._empty((T, num_heads * value_dim), torch.float32)
         if chunked:
             # portions of prompts: chunks of rows side by side instead of one row after the other
             count, packed, scratch = self._scan_chunks(meta, self._ops.distie_gated_decay_scan_chunk_rows(), num_heads,
                                                        dim, value_dim)
-            totals = torch.empty((count, num_heads, dim), dtype=torch.float32, device=self.device)
+            totals = self._empty((count, num_heads, dim), torch.float32)
             _check(self._ops.distie_gated_decay_scan_chunked(
-                product.data_ptr(), _code(product), W, decay_logits.data_ptr(), state.data_ptr(), out.data_ptr(),
-                scratch.data_ptr(), totals.data_ptr(), packed.data_ptr(), packed.data_ptr() + 16 * count,
-                meta.state_slots.data_ptr(), count, meta.num_requests, num_heads, dim, value_dim, float(q_scale),
+                product, _code(product), W, decay_logits, state, out,
+                scratch, totals, packed, packed.data_ptr() + 16 * count,
+                meta.state_slots, count, meta.num_requests, num_heads, dim, value_dim, float(q_scale),
                 float(tau), self._stream()), "gated_decay_scan_chunked")
             _mark_written(state)
             return out
         _check(self._ops.distie_gated_decay_scan(
-            product.data_ptr(), _code(product), W, decay_logits.data_ptr() if decay_logits is not None else None,
-            low_ptr, low_ld, up.data_ptr() if low_ptr is not None else None,
-            up_bias.data_ptr() if low_ptr is not None else None, rank if low_ptr is not None else 0, state.data_ptr(),
-            out.data_ptr(), meta.cu_q.data_ptr(), meta.state_slots.data_ptr(), meta.num_requests, num_heads, dim,
+            product, _code(product), W, decay_logits,
+            low_ptr, low_ld, up if low_ptr is not None else None,
+            up_bias if low_ptr is not None else None, rank if low_ptr is not None else 0, state,
+            out, meta.cu_q, meta.state_slots, meta.num_requests, num_heads, dim,
             value_dim, float(q_scale), float(tau), self._stream()), "gated_decay_scan")
         _mark_written(state)
         return out
@@ -2332,10 +2341,10 @@ class HipOps(Ops):
             raise KernelError("token_shift: x are the step's rows, mu float32 [mixes, C]")
         if state.dtype != torch.float32 or tuple(state.shape[1:]) != (C,):
             raise KernelError("token_shift: the state is float32 [slots, C]")
-        out = torch.empty((mu.shape[0], T, C), dtype=x.dtype, device=self.device)
-        _check(self._ops.distie_token_shift(x.data_ptr(), _code(x), mu.data_ptr(), mu.shape[0], state.data_ptr(),
-                                            out.data_ptr(), meta.cu_q.data_ptr(), None if meta.all_decode else meta.token_request.data_ptr(),
-                                            meta.state_slots.data_ptr(), T, C, self._stream()), "token_shift")
+        out = self._empty((mu.shape[0], T, C), x.dtype)
+        _check(self._ops.distie_token_shift(x, _code(x), mu, mu.shape[0], state,
+                                            out, meta.cu_q, None if meta.all_decode else meta.token_request,
+                                            meta.state_slots, T, C, self._stream()), "token_shift")
         _mark_written(state)
         return out
 
@@ -2356,14 +2365,14 @@ class HipOps(Ops):
         if free - 2 * sum(blocks) * -(-K // 32) * 512 < self.PACKED_KEEPS_FREE * total:
             self._packed_left_out += 1
             return
-        packed = torch.empty(sum(blocks) * -(-K // 32) * 512, dtype=torch.bfloat16, device=self.device)
+        packed = self._empty(sum(blocks) * -(-K // 32) * 512, torch.bfloat16)
         at, maps = 0, []
         for w, count in zip(weights, blocks):
             self._own(w)
             row_map = self._row_map(w.shape[0], False, None).to(device=self.device, dtype=torch.int32)
             maps.append(row_map)
             size = count * -(-K // 32) * 512
-            _check(self._ops.distie_pack_rows(w.data_ptr(), packed[at:at + size].data_ptr(), row_map.data_ptr(), count, K,
+            _check(self._ops.distie_pack_rows(w, packed[at:at + size], row_map, count, K,
                                               self._stream()), "pack_rows")
             at += size
         torch.cuda.current_stream(self.device).synchronize()      # the row maps are freed on return
@@ -2390,21 +2399,21 @@ class HipOps(Ops):
             raise KernelError("linear_each: an input [rows, K] for every weight [N, K], the weights it was prepared for")
         starts = [0] + [16 * int(e) for e in ends[:-1]]
         if plan is not None:
-            out = torch.empty((M, 16 * int(ends[rounded - 1])), dtype=torch.bfloat16, device=self.device)
-            _check(self._ops.distie_large_tiles_each_bf16(xs.data_ptr(), packed.data_ptr(), out.data_ptr(), M, K, rounded,
+            out = self._empty((M, 16 * int(ends[rounded - 1])), torch.bfloat16)
+            _check(self._ops.distie_large_tiles_each_bf16(xs, packed, out, M, K, rounded,
                                                           ends.ctypes.data, plan, self._stream()), "large_tiles_each_bf16")
             return [out[:, at:at + w.shape[0]] for at, w in zip(starts, weights[:rounded])] + \
                 [self.linear_f32out(xs[k], weights[k]) for k in range(rounded, count)]
-        out = torch.empty((M, 16 * int(ends[-1])), dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_gemm_packed_each_bf16(xs.data_ptr(), packed.data_ptr(), out.data_ptr(), M, K, count,
+        out = self._empty((M, 16 * int(ends[-1])), torch.float32)
+        _check(self._ops.distie_gemm_packed_each_bf16(xs, packed, out, M, K, count,
                                                       ends.ctypes.data, self._stream()), "gemm_packed_each_bf16")
         return [out[:, at:at + w.shape[0]] for at, w in zip(starts, weights)]
 
     def wkv_decay_logits(self, low, up, up_bias):
         low = low if low.dtype == torch.float32 else low.float()
         ptr, ld = self._rows_view(low, up.shape[1])
-        bent = torch.empty(low.shape, dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_tanh_f32(ptr, ld, bent.data_ptr(), low.shape[0], low.shape[1], self._stream()), "tanh_f32")
+        bent = self._empty(low.shape, torch.float32)
+        _check(self._ops.distie_tanh_f32(ptr, ld, bent, low.shape[0], low.shape[1], self._stream()), "tanh_f32")
         return self.linear_f32out(bent, up, up_bias)
 
     def wkv_mix(self, r, k, v, gates, low, up, up_bias, bonus, state, meta, num_heads, dim, norm_weight, eps, out_dtype):
@@ -2425,24 +2434,24 @@ class HipOps(Ops):
             raise KernelError(f"wkv_mix: heads of up to {self._ops.distie_wkv_scan_max_dim()} and decays through up to "
                               f"{self._ops.distie_wkv_scan_max_rank()} dimensions")
         low_ptr, low_ld = self._rows_view(low, rank)
-        out = torch.empty((T, N), dtype=out_dtype, device=self.device)
+        out = self._empty((T, N), out_dtype)
         if not self.captured and meta.host_cu_q is not None and meta.max_q >= self.SCAN_CHUNKED_MIN_ROWS and \
                 dim <= self._ops.distie_wkv_chunked_max_dim():
             # portions of prompts: chunks of rows side by side instead of one row after the other
             z = self.wkv_decay_logits(low, up, up_bias)
             count, packed, scratch = self._scan_chunks(meta, self._ops.distie_wkv_chunk_rows(), num_heads, dim, dim)
-            totals = torch.empty((count, num_heads, dim), dtype=torch.float32, device=self.device)
+            totals = self._empty((count, num_heads, dim), torch.float32)
             _check(self._ops.distie_wkv_scan_chunked(
-                views[0][0], views[1][0], views[2][0], views[3][0], _code(r), ld, z.data_ptr(), bonus.data_ptr(),
-                state.data_ptr(), norm_weight.data_ptr(), float(eps), out.data_ptr(), _code(out), scratch.data_ptr(),
-                totals.data_ptr(), packed.data_ptr(), packed.data_ptr() + 16 * count, meta.state_slots.data_ptr(), count,
+                views[0][0], views[1][0], views[2][0], views[3][0], _code(r), ld, z, bonus,
+                state, norm_weight, float(eps), out, _code(out), scratch,
+                totals, packed, packed.data_ptr() + 16 * count, meta.state_slots, count,
                 meta.num_requests, num_heads, dim, self._stream()), "wkv_scan_chunked")
             _mark_written(state)
             return out
         _check(self._ops.distie_wkv_scan(
-            views[0][0], views[1][0], views[2][0], views[3][0], _code(r), ld, low_ptr, _code(low), low_ld, rank, up.data_ptr(),
-            up_bias.data_ptr(), bonus.data_ptr(), state.data_ptr(), norm_weight.data_ptr(), float(eps), out.data_ptr(),
-            _code(out), None if meta.all_decode else meta.cu_q.data_ptr(), meta.state_slots.data_ptr(), meta.num_requests,
+            views[0][0], views[1][0], views[2][0], views[3][0], _code(r), ld, low_ptr, _code(low), low_ld, rank, up,
+            up_bias, bonus, state, norm_weight, float(eps), out,
+            _code(out), None if meta.all_decode else meta.cu_q, meta.state_slots, meta.num_requests,
             num_heads, dim, self._stream()), "wkv_scan")
         _mark_written(state)
         return out
@@ -2478,12 +2487,11 @@ class HipOps(Ops):
                                   "a request")
         out = None
         if out_dtype is not None:
-            out = torch.empty((T, C) if mu is None else (mu.shape[0], T, C), dtype=out_dtype, device=self.device)
-        ptr = lambda t: t.data_ptr() if t is not None else None
+            out = self._empty((T, C) if mu is None else (mu.shape[0], T, C), out_dtype)
         _check(self._ops.distie_group_chain(
-            delta.data_ptr(), _code(delta), slices, weight.data_ptr(), float(eps), int(groups), ptr(residual), ptr(into),
-            ptr(first), ptr(rest), int(index), ptr(weights), ptr(out), _code(out) if out is not None else _F32, T, C, ptr(mu),
-            mu.shape[0] if mu is not None else 0, ptr(state), ptr(slots), self._stream()), "group_chain")
+            delta, _code(delta), slices, weight, float(eps), int(groups), residual, into,
+            first, rest, int(index), weights, out, _code(out) if out is not None else _F32, T, C, mu,
+            mu.shape[0] if mu is not None else 0, state, slots, self._stream()), "group_chain")
         if state is not None:
             _mark_written(state)
         if into is not None:
@@ -2518,11 +2526,11 @@ class HipOps(Ops):
         for t in (recur_bias, input_bias, lam):
             if t.dtype != torch.float32 or t.numel() != R:
                 raise KernelError("lru_gates: biases and lam are float32 with R elements")
-        a = torch.empty((T, R), dtype=torch.float32, device=self.device)
-        x = torch.empty((T, R), dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_lru_gates(u_ptr, _code(u), ldu, recur_weight.data_ptr(), recur_bias.data_ptr(),
-                                          input_weight.data_ptr(), input_bias.data_ptr(), _code(recur_weight),
-                                          lam.data_ptr(), float(rate), a.data_ptr(), x.data_ptr(), T, R, blocks,
+        a = self._empty((T, R), torch.float32)
+        x = self._empty((T, R), torch.float32)
+        _check(self._ops.distie_lru_gates(u_ptr, _code(u), ldu, recur_weight, recur_bias,
+                                          input_weight, input_bias, _code(recur_weight),
+                                          lam, float(rate), a, x, T, R, blocks,
                                           self._stream()), "lru_gates")
         return a, x
 
@@ -2542,20 +2550,20 @@ class HipOps(Ops):
         if mul is not None:
             m_ptr, m_ld = self._rows_view(mul, R)
             m_code = _code(mul)
-        out = torch.empty((T, R), dtype=out_dtype, device=self.device)
+        out = self._empty((T, R), out_dtype)
         if not self.captured and meta.host_cu_q is not None and meta.max_q >= self.LRU_CHUNKED_MIN_ROWS:
             # portions of prompts: chunks of rows side by side, each scanned twice (alone, then from what stands before it)
             count, packed, sums = self._scan_chunks(meta, self._ops.distie_lru_scan_chunk_rows(), 1, 1, R)
-            factors = torch.empty((count, R), dtype=torch.float32, device=self.device)
-            init = torch.empty((meta.num_requests, R), dtype=torch.float32, device=self.device)
+            factors = self._empty((count, R), torch.float32)
+            init = self._empty((meta.num_requests, R), torch.float32)
             _check(self._ops.distie_lru_scan_chunked(
-                a.data_ptr(), x.data_ptr(), state.data_ptr(), factors.data_ptr(), sums.data_ptr(), init.data_ptr(), m_ptr,
-                m_code, m_ld, kind, out.data_ptr(), _code(out), packed.data_ptr(), packed.data_ptr() + 16 * count,
-                meta.state_slots.data_ptr(), count, meta.num_requests, R, self._stream()), "lru_scan_chunked")
+                a, x, state, factors, sums, init, m_ptr,
+                m_code, m_ld, kind, out, _code(out), packed, packed.data_ptr() + 16 * count,
+                meta.state_slots, count, meta.num_requests, R, self._stream()), "lru_scan_chunked")
             _mark_written(state)
             return out
-        _check(self._ops.distie_lru_scan(a.data_ptr(), x.data_ptr(), state.data_ptr(), m_ptr, m_code, m_ld, kind,
-                                         out.data_ptr(), _code(out), meta.cu_q.data_ptr(), meta.state_slots.data_ptr(),
+        _check(self._ops.distie_lru_scan(a, x, state, m_ptr, m_code, m_ld, kind,
+                                         out, _code(out), meta.cu_q, meta.state_slots,
                                          meta.num_requests, R, self._stream()), "lru_scan")
         _mark_written(state)
         return out
@@ -2586,11 +2594,11 @@ class HipOps(Ops):
         if tuple(weight.shape) != (rows, C) or (bias is not None and (bias.dtype != torch.float32 or tuple(bias.shape) != (rows,))):
             raise KernelError("route_topk: weight [experts (+ 1 with a shared one), C], bias float32 with a number a row")
         numbers = self._route_rule(rule, scoring, E)
-        experts = torch.empty((T, top), dtype=torch.int32, device=self.device)
-        gates = torch.empty((T, top + shared), dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_route_topk(x.data_ptr(), _code(x), weight.data_ptr(), _code(weight),
-                                           bias.data_ptr() if bias is not None else None, experts.data_ptr(),
-                                           gates.data_ptr(), T, C, E, int(top), self.SCORINGS[scoring], *numbers,
+        experts = self._empty((T, top), torch.int32)
+        gates = self._empty((T, top + shared), torch.float32)
+        _check(self._ops.distie_route_topk(x, _code(x), weight, _code(weight),
+                                           bias, experts,
+                                           gates, T, C, E, int(top), self.SCORINGS[scoring], *numbers,
                                            self._stream()), "route_topk")
         return experts, gates
 
@@ -2617,10 +2625,10 @@ class HipOps(Ops):
                               "[T, 2 * (experts * width + shared_width)]")
         if limit is not None and not limit > 0:
             raise KernelError("route_glu: the limit must be positive")
-        out = torch.empty((T, total), dtype=dtype, device=self.device)
-        _check(self._ops.distie_route_glu(source.data_ptr(), _code(source), ld, slices, experts.data_ptr(),
-                                          gates.data_ptr(), T, top, num_experts, width, float(limit or 0.0), float(slope),
-                                          float(up_shift), 1 if on_input else 0, int(shared_width), out.data_ptr(),
+        out = self._empty((T, total), dtype)
+        _check(self._ops.distie_route_glu(source, _code(source), ld, slices, experts,
+                                          gates, T, top, num_experts, width, float(limit or 0.0), float(slope),
+                                          float(up_shift), 1 if on_input else 0, int(shared_width), out,
                                           _code(out), self._stream()), "route_glu")
         return out
 
@@ -2650,19 +2658,19 @@ class HipOps(Ops):
             raise KernelError("route_experts_glu: x [T, C], router [E, C], bias float32 [E], gate_up [T, 2 * E * width]")
         if limit is not None and not limit > 0:
             raise KernelError("route_experts_glu: the limit must be positive")
-        out = torch.empty((T, total), dtype=dtype, device=self.device)
+        out = self._empty((T, total), dtype)
         _check(self._ops.distie_route_topk_glu(
-            x.data_ptr(), router_weight.data_ptr(), router_bias.data_ptr() if router_bias is not None else None, C,
-            self.SCORINGS[scoring], source.data_ptr(), _code(source), gate_up.shape[1], slices, T, int(top),
+            x, router_weight, router_bias, C,
+            self.SCORINGS[scoring], source, _code(source), gate_up.shape[1], slices, T, int(top),
             num_experts, width, float(limit or 0.0), float(slope), float(up_shift), 1 if on_input else 0, *numbers,
-            int(shared_width), out.data_ptr(), _code(out), self._stream()), "route_topk_glu")
+            int(shared_width), out, _code(out), self._stream()), "route_topk_glu")
         return out
 
     def softcap(self, x, cap):
         self._own(x)
         if x.dtype != torch.float32:
             raise KernelError("softcap works on float32 values")
-        _check(self._ops.distie_softcap_f32(x.data_ptr(), x.numel(), float(cap), self._stream()), "softcap_f32")
+        _check(self._ops.distie_softcap_f32(x, x.numel(), float(cap), self._stream()), "softcap_f32")
         _mark_written(x)
         return x
 
@@ -2673,8 +2681,8 @@ class HipOps(Ops):
         if experts.dtype != torch.int32 or gates.dtype != torch.float32 or gates.shape != experts.shape or \
                 hidden.shape[0] != T or hidden.shape[1] < num_experts * width:
             raise KernelError("route_scale: experts int32 and gates float32 [T, top], hidden [T, >= experts * width]")
-        _check(self._ops.distie_route_scale(hidden.data_ptr(), _code(hidden), hidden.shape[1], experts.data_ptr(),
-                                            gates.data_ptr(), T, top, num_experts, width, self._stream()), "route_scale")
+        _check(self._ops.distie_route_scale(hidden, _code(hidden), hidden.shape[1], experts,
+                                            gates, T, top, num_experts, width, self._stream()), "route_scale")
         _mark_written(hidden)
         return hidden
 
@@ -2687,8 +2695,8 @@ class HipOps(Ops):
         if isinstance(x, PartialSums):
             slices, source = x.slices, x.data
         self._own(source)
-        out = torch.empty(tuple(x.shape), dtype=dtype, device=self.device)
-        _check(self._ops.distie_activation(source.data_ptr(), _code(source), slices, out.data_ptr(), _code(out), out.numel(),
+        out = self._empty(tuple(x.shape), dtype)
+        _check(self._ops.distie_activation(source, _code(source), slices, out, _code(out), out.numel(),
                                            self.ACTIVATIONS[kind], self._stream()), "activation")
         return out
 
@@ -2712,7 +2720,7 @@ class HipOps(Ops):
         for vector in (a_log, dt_bias):
             if vector.dtype != torch.float32 or tuple(vector.shape) != (H,):
                 raise KernelError("delta_scan: a_log and dt_bias are float32 [heads]")
-        out = torch.empty((T, H * E), dtype=torch.float32, device=self.device)
+        out = self._empty((T, H * E), torch.float32)
         if not self.captured and meta.host_cu_q is not None and meta.max_q >= self.SCAN_CHUNKED_MIN_ROWS:
             # portions of prompts: chunks of rows, the triangular systems of all chunks side by side
             rows = self._ops.distie_delta_scan_chunk_rows()
@@ -2721,19 +2729,19 @@ class HipOps(Ops):
             key = ("delta_scratch", count, H, DP, EP)
             held = meta.scratch.get(key)
             if held is None:
-                held = meta.scratch[key] = [torch.empty((count, H, *shape), dtype=torch.float32, device=self.device)
+                held = meta.scratch[key] = [self._empty((count, H, *shape), torch.float32)
                                             for shape in ((rows, DP), (rows, EP), (rows, EP), (DP, rows), (rows, rows), (rows,),
                                                           ())]
             _check(self._ops.distie_delta_scan_chunked(
-                q_ptr, _code(qkv), ld, b_ptr, ldb, d_ptr, ldd, a_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(),
-                out.data_ptr(), *(t.data_ptr() for t in held), states.data_ptr(), packed.data_ptr(),
-                packed.data_ptr() + 16 * count, meta.state_slots.data_ptr(), count, meta.num_requests, H, G, D, E,
+                q_ptr, _code(qkv), ld, b_ptr, ldb, d_ptr, ldd, a_log, dt_bias, state,
+                out, *(t for t in held), states, packed,
+                packed.data_ptr() + 16 * count, meta.state_slots, count, meta.num_requests, H, G, D, E,
                 float(q_scale), float(unit_eps), self._stream()), "delta_scan_chunked")
             _mark_written(state)
             return out
         _check(self._ops.distie_delta_scan(
-            q_ptr, _code(qkv), ld, b_ptr, ldb, d_ptr, ldd, a_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(),
-            out.data_ptr(), meta.cu_q.data_ptr(), meta.state_slots.data_ptr(), meta.num_requests, H, G, D, E, float(q_scale),
+            q_ptr, _code(qkv), ld, b_ptr, ldb, d_ptr, ldd, a_log, dt_bias, state,
+            out, meta.cu_q, meta.state_slots, meta.num_requests, H, G, D, E, float(q_scale),
             float(unit_eps), self._stream()), "delta_scan")
         _mark_written(state)
         return out
@@ -2759,7 +2767,7 @@ class HipOps(Ops):
         for vector in (dt_bias, a_log, skip):
             if vector.dtype != torch.float32 or tuple(vector.shape) != (H,):
                 raise KernelError("ssm_scan: dt_bias, a_log and skip are float32 [heads]")
-        out = torch.empty((T, H * P), dtype=torch.float32, device=self.device)
+        out = self._empty((T, H * P), torch.float32)
         wide = N > self._ops.distie_ssm_scan_max_state()      # more rows a head than the row-by-row kernel keeps
         if not self.captured and meta.host_cu_q is not None and (meta.max_q >= self.SSM_CHUNKED_MIN_ROWS or wide):
             count, packed, scratch = self._scan_chunks(meta, self._ops.distie_ssm_scan_chunk_rows(), H, N, P)
@@ -2767,22 +2775,22 @@ class HipOps(Ops):
             held = meta.scratch.get(key)
             if held is None:
                 rows = self._ops.distie_ssm_scan_chunk_rows()
-                held = meta.scratch[key] = (torch.empty((count, H), dtype=torch.float32, device=self.device),
-                                            torch.empty((count, G, rows, rows), dtype=torch.float32, device=self.device))
+                held = meta.scratch[key] = (self._empty((count, H), torch.float32),
+                                            self._empty((count, G, rows, rows), torch.float32))
             totals, pairs = held
             _check(self._ops.distie_ssm_scan_chunked(
-                x_ptr, _code(xbc), ld, d_ptr, ldd, dt_bias.data_ptr(), a_log.data_ptr(), skip.data_ptr(),
-                state.data_ptr(), out.data_ptr(), scratch.data_ptr(), totals.data_ptr(), pairs.data_ptr(), packed.data_ptr(),
-                packed.data_ptr() + 16 * count, meta.state_slots.data_ptr(), count, meta.num_requests, H, P, N, G,
+                x_ptr, _code(xbc), ld, d_ptr, ldd, dt_bias, a_log, skip,
+                state, out, scratch, totals, pairs, packed,
+                packed.data_ptr() + 16 * count, meta.state_slots, count, meta.num_requests, H, P, N, G,
                 self._stream()), "ssm_scan_chunked")
             _mark_written(state)
             return out
         if wide:
             raise KernelError(f"ssm_scan: a state of {N} rows a head is beyond the row-by-row kernel, which is all a "
                               f"captured step can use")
-        _check(self._ops.distie_ssm_scan(x_ptr, _code(xbc), ld, d_ptr, ldd, dt_bias.data_ptr(), a_log.data_ptr(),
-                                         skip.data_ptr(), state.data_ptr(), out.data_ptr(), meta.cu_q.data_ptr(),
-                                         meta.state_slots.data_ptr(), meta.num_requests, H, P, N, G, self._stream()),
+        _check(self._ops.distie_ssm_scan(x_ptr, _code(xbc), ld, d_ptr, ldd, dt_bias, a_log,
+                                         skip, state, out, meta.cu_q,
+                                         meta.state_slots, meta.num_requests, H, P, N, G, self._stream()),
                "ssm_scan")
         _mark_written(state)
         return out
@@ -2813,12 +2821,11 @@ class HipOps(Ops):
         if pairs and 2 * pairs != rot_dim:
             raise KernelError("latent_norm_rope_write: the rotation turns all of the rotated part")
         table = self._rope_table(meta, inv_freq) if pairs else None
-        latent = torch.empty((T, q_rank), dtype=out_dtype, device=self.device) if q_rank else None
-        ptr = lambda t: t.data_ptr() if t is not None else None
+        latent = self._empty((T, q_rank), out_dtype) if q_rank else None
         _check(self._ops.distie_latent_norm_rope_write(
-            down.data_ptr(), slices, W, q_rank, ptr(q_weight), kv_rank, kv_weight.data_ptr(), float(eps), rot_dim, ptr(table),
-            float(magnitude), 1 if neighbours else 0, ptr(latent), _CODES[out_dtype], k_cache.data_ptr(),
-            v_cache.data_ptr(), _code(k_cache), meta.groups[group].slots.data_ptr(), T, meta.block_size, padded,
+            down, slices, W, q_rank, q_weight, kv_rank, kv_weight, float(eps), rot_dim, table,
+            float(magnitude), 1 if neighbours else 0, latent, _CODES[out_dtype], k_cache,
+            v_cache, _code(k_cache), meta.groups[group].slots, T, meta.block_size, padded,
             1 if write else 0, self._stream()), "latent_norm_rope_write")
         return latent
 
@@ -2839,10 +2846,10 @@ class HipOps(Ops):
         self._own(source, key_up, inv_freq)
         T = meta.num_tokens
         table = self._rope_table(meta, inv_freq)
-        out = torch.empty((T, num_heads * padded_dim), dtype=torch.bfloat16, device=self.device)
+        out = self._empty((T, num_heads * padded_dim), torch.bfloat16)
         _check(self._ops.distie_latent_queries(
-            source.data_ptr(), _code(source), slices, dim + rot_dim, key_up.data_ptr(), _code(key_up), out.data_ptr(),
-            padded_dim, T, num_heads, kv_rank, dim, rot_dim // 2, table.data_ptr(), float(magnitude),
+            source, _code(source), slices, dim + rot_dim, key_up, _code(key_up), out,
+            padded_dim, T, num_heads, kv_rank, dim, rot_dim // 2, table, float(magnitude),
             1 if neighbours else 0, self._stream()), "latent_queries")
         return out
 
@@ -2860,8 +2867,8 @@ class HipOps(Ops):
             out = make((T, H * out_stride), dtype=x.dtype, device=self.device)
         elif out.dtype != x.dtype or tuple(out.shape) != (T, H * out_stride):
             raise KernelError("heads_linear: out is [T, heads * out_stride] of x's dtype")
-        _check(self._ops.distie_heads_linear(x.data_ptr(), _code(x), in_stride, weight.data_ptr(), _code(weight),
-                                             out.data_ptr(), out_stride, T, H, N, K, self._stream()), "heads_linear")
+        _check(self._ops.distie_heads_linear(x, _code(x), in_stride, weight, _code(weight),
+                                             out, out_stride, T, H, N, K, self._stream()), "heads_linear")
         return out
 
     def rope_heads(self, x, in_stride, in_offset, out, out_stride, out_offset, num_heads, inv_freq, magnitude,
@@ -2873,8 +2880,8 @@ class HipOps(Ops):
                 or T != meta.num_tokens:
             raise KernelError("rope_heads: x [T, heads * in_stride] and out [T, heads * out_stride] of one dtype")
         table = self._rope_table(meta, inv_freq)
-        _check(self._ops.distie_rope_heads(x.data_ptr(), _code(x), in_stride, in_offset, out.data_ptr(), out_stride,
-                                           out_offset, T, num_heads, inv_freq.shape[0], table.data_ptr(),
+        _check(self._ops.distie_rope_heads(x, _code(x), in_stride, in_offset, out, out_stride,
+                                           out_offset, T, num_heads, inv_freq.shape[0], table,
                                            float(magnitude), 1 if neighbours else 0, self._stream()), "rope_heads")
         return out
 
@@ -2898,8 +2905,8 @@ class HipOps(Ops):
             slices, source = gate_up.slices, gate_up.data
         self._own(source)
         rows, two = gate_up.shape
-        out = torch.empty((rows, two // 2), dtype=dtype, device=self.device)
-        _check(self._ops.distie_glu_mul(source.data_ptr(), _code(source), slices, out.data_ptr(), _code(out), rows,
+        out = self._empty((rows, two // 2), dtype)
+        _check(self._ops.distie_glu_mul(source, _code(source), slices, out, _code(out), rows,
                                         two // 2, kind, *clamp, self._stream()), "glu_mul")
         return out
 
@@ -2911,16 +2918,16 @@ class HipOps(Ops):
             slices, source = gate_up.slices, gate_up.data
         self._own(source)
         rows, two = gate_up.shape
-        out = torch.empty((rows, two // 2), dtype=dtype, device=self.device)
-        _check(self._ops.distie_silu_mul(source.data_ptr(), _code(source), slices, out.data_ptr(), _code(out),
+        out = self._empty((rows, two // 2), dtype)
+        _check(self._ops.distie_silu_mul(source, _code(source), slices, out, _code(out),
                                          rows, two // 2, self._stream()), "silu_mul")
         return out
 
     def gather_rows(self, x, rows):
         x = self.dense(x)
         self._own(x, rows)
-        out = torch.empty((rows.shape[0], x.shape[1]), dtype=x.dtype, device=self.device)
-        _check(self._ops.distie_gather_rows(x.data_ptr(), rows.data_ptr(), out.data_ptr(), rows.shape[0],
+        out = self._empty((rows.shape[0], x.shape[1]), x.dtype)
+        _check(self._ops.distie_gather_rows(x, rows, out, rows.shape[0],
                                             x.shape[1] * x.element_size(), x.shape[0], self._stream()), "gather_rows")
         return out
 
@@ -2929,15 +2936,15 @@ class HipOps(Ops):
         if logits.dtype != torch.float32:
             raise KernelError("argmax reads float32 logits")
         rows, vocab = logits.shape
-        out = torch.empty(rows, dtype=torch.int32, device=self.device)
+        out = self._empty(rows, torch.int32)
         parts = self._ops.distie_argmax_parts(rows, vocab)
         values = indexes = None
         if parts > 1:
-            values = torch.empty(rows * parts, dtype=torch.float32, device=self.device)
-            indexes = torch.empty(rows * parts, dtype=torch.int32, device=self.device)
-        _check(self._ops.distie_argmax(logits.data_ptr(), out.data_ptr(), rows, vocab,
-                                       values.data_ptr() if parts > 1 else None,
-                                       indexes.data_ptr() if parts > 1 else None, self._stream()), "argmax")
+            values = self._empty(rows * parts, torch.float32)
+            indexes = self._empty(rows * parts, torch.int32)
+        _check(self._ops.distie_argmax(logits, out, rows, vocab,
+                                       values if parts > 1 else None,
+                                       indexes if parts > 1 else None, self._stream()), "argmax")
         return out
 
     def sample(self, logits, temperature, seeds, counters):
@@ -2946,16 +2953,16 @@ class HipOps(Ops):
                 seeds.dtype != torch.int64 or counters.dtype != torch.int64:
             raise KernelError("sample: logits/temperature float32, seeds/counters int64")
         rows, vocab = logits.shape
-        out = torch.empty(rows, dtype=torch.int32, device=self.device)
+        out = self._empty(rows, torch.int32)
         parts = self._ops.distie_argmax_parts(rows, vocab)
         values = indexes = sums = None
         if parts > 1:
-            values = torch.empty(rows * parts, dtype=torch.float32, device=self.device)
-            indexes = torch.empty(rows * parts, dtype=torch.int32, device=self.device)
-            sums = torch.empty(rows * parts, dtype=torch.float32, device=self.device)
-        _check(self._ops.distie_sample(logits.data_ptr(), temperature.data_ptr(), seeds.data_ptr(),
-                                       counters.data_ptr(), out.data_ptr(), rows, vocab,
-                                       values.data_ptr() if parts > 1 else None,
-                                       indexes.data_ptr() if parts > 1 else None,
-                                       sums.data_ptr() if parts > 1 else None, self._stream()), "sample")
+            values = self._empty(rows * parts, torch.float32)
+            indexes = self._empty(rows * parts, torch.int32)
+            sums = self._empty(rows * parts, torch.float32)
+        _check(self._ops.distie_sample(logits, temperature, seeds,
+                                       counters, out, rows, vocab,
+                                       values if parts > 1 else None,
+                                       indexes if parts > 1 else None,
+                                       sums if parts > 1 else None, self._stream()), "sample")
         return out
