@@ -1060,8 +1060,14 @@ extern "C" int distie_attention_decode_run_len(const int32_t* kv_len, int num_re
   return launch_status();
 }
 
+// What bounds a short run is its trips to memory, so all loads of a chunk go out together (48 at a head size of 128; only then are the
+// values behind the run's end cleared, and no load stands under a condition). With each block of 16 keys under a condition of its own
+// and its values cleared as they came, the compiler waited for every block before it asked for the next, and for every one of the last
+// 16 values of a head of 256: us a layer in a step, before / now:
+// 16 heads of 256 on one, 16 requests of 1,500 keys 23.2 / 10.0; 12 heads of 128 on 2, one request of 500 keys 6.5 / 4.8, 8 of 2,048
+// 7.9 / 6.7, 64 of 2,048 28.2 / 28.2 (that is 4.8 TB/s).
 // Two waves a SIMD where the registers allow it without spilling (one block of query heads, head sizes up to 128:
-// 234 registers; left to itself the compiler took a few more and one wave a SIMD). The chip then holds 2,048 waves
+// 206 registers). The chip then holds 2,048 waves
 // instead of 1,024, and a batch whose runs are a few more than 1,024, or whose requests differ in length, no
 // longer waits for the last waves to get a place: 7B shape's heads at 2,100 keys, 96 requests 91 -> 83 us a layer,
 // 160 requests 165 -> 130; contexts of 1,050 to 3,150 keys, 96 requests 121 -> 96, 160 requests 222 -> 157.
@@ -1136,40 +1142,33 @@ __global__ __launch_bounds__(DISTIE_WAVE * W, (MB == 1 && D <= 128 ? 2 : 1)) voi
     for (int b = 0; b < DC_BLOCKS; ++b) pages[b] = table[min((chunk_begin + 16 * b) / block_size, table_width - 1)];
   }
   for (int chunk = chunk_begin; chunk <= key_end; chunk += DC_KEYS) {
-    // ---- every load of the chunk first
-    bool live[DC_BLOCKS];
+    // ---- every load of the chunk first, none of them under a condition: a block outside the run, which may have no page, reads
+    // the nearest one inside again
+    const int low = max(key_begin - chunk, 0) / 16, high = min((key_end - chunk) / 16, DC_BLOCKS - 1);
     bf16x8 k_reg[DC_BLOCKS][DK32 > 0 ? DK32 : 1];
     shortx4 k_tail[DC_BLOCKS];
     uint2 v_reg[DC_BLOCKS][DB16];
+    const bf16_t* v_from[DC_BLOCKS];
 #pragma unroll
     for (int b = 0; b < DC_BLOCKS; ++b) {
-      const int key0 = chunk + 16 * b;
-      live[b] = key0 <= key_end && key0 + 15 >= key_begin;      // a block outside the run may have no page
+      const int inside = min(max(b, low), high);
+      int page = pages[0];
 #pragma unroll
-      for (int dk = 0; dk < DK32; ++dk) k_reg[b][dk] = bf16x8{};
-      k_tail[b] = shortx4{};
-#pragma unroll
-      for (int db = 0; db < DB16; ++db) v_reg[b][db] = uint2{0u, 0u};
-      if (!live[b]) continue;
-      const int page = pages[b];
+      for (int i = 1; i < DC_BLOCKS; ++i) page = inside == i ? pages[i] : page;
       const int64_t page_base = (static_cast<int64_t>(page) * kv_heads + kh) * block_size * D;
-      const int offset = key0 % block_size;
-      const bf16_t* k_row = k_cache + page_base + static_cast<int64_t>(offset + r) * D;
+      const int offset = (chunk + 16 * inside) % block_size;
+      const bf16_t* k_row = k_cache + page_base + static_cast<int64_t>(offset) * D;
 #pragma unroll
-      for (int dk = 0; dk < DK32; ++dk) k_reg[b][dk] = *reinterpret_cast<const bf16x8*>(k_row + 32 * dk + 8 * g);
-      if (DK_TAIL) k_tail[b] = *reinterpret_cast<const shortx4*>(k_row + (D - 16) + 4 * g);
-      // Slots after the run's last key were never written by this request: what a former owner of the page
-      // left there must not even be multiplied by a weight of zero (0 * NaN), so those values are cleared.
-      const int written = key_end - (key0 + 4 * g) + 1;          // of this lane's four keys
-      const uint32_t keep_lo = written >= 2 ? 0xffffffffu : (written == 1 ? 0x0000ffffu : 0u);
-      const uint32_t keep_hi = written >= 4 ? 0xffffffffu : (written == 3 ? 0x0000ffffu : 0u);
-      const bf16_t* v_col = v_cache + page_base + offset + 4 * g;
-#pragma unroll
-      for (int db = 0; db < DB16; ++db) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(v_col + static_cast<int64_t>(16 * db + r) * block_size);
-        v_reg[b][db] = uint2{raw.x & keep_lo, raw.y & keep_hi};
-      }
+      for (int dk = 0; dk < DK32; ++dk) k_reg[b][dk] = *reinterpret_cast<const bf16x8*>(k_row + (r * D + 32 * dk + 8 * g));
+      if (DK_TAIL) k_tail[b] = *reinterpret_cast<const shortx4*>(k_row + (r * D + (D - 16) + 4 * g));
+      v_from[b] = v_cache + page_base + offset;
     }
+#pragma unroll
+    for (int b = 0; b < DC_BLOCKS; ++b)
+#pragma unroll
+      for (int db = 0; db < DB16; ++db)
+        v_reg[b][db] = *reinterpret_cast<const uint2*>(v_from[b] + static_cast<int64_t>(16 * db) * block_size + (r * block_size + 4 * g));
+    __builtin_amdgcn_sched_barrier(0);
     // the next chunk's pages, while this chunk's keys and values are on their way
     if (chunk + DC_KEYS <= key_end) {
 #pragma unroll
@@ -1240,6 +1239,19 @@ __global__ __launch_bounds__(DISTIE_WAVE * W, (MB == 1 && D <= 128 ? 2 : 1)) voi
       for (int db = 0; db < DB16; ++db)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o_acc[mb][db][i] *= a4[i];
+    }
+    // Slots after the run's last key were never written by this request: what a former owner of the page left there must not
+    // even be multiplied by a weight of zero (0 * NaN), so those values are cleared, and those of blocks outside the run. (Here and
+    // not where they are loaded: there each block's values would be waited for before the next block's are asked for.)
+    if (chunk < key_begin || chunk + DC_KEYS - 1 > key_end) {
+#pragma unroll
+      for (int b = 0; b < DC_BLOCKS; ++b) {
+        const int written = b < low ? 0 : key_end - (chunk + 16 * b + 4 * g) + 1;          // of this lane's four keys
+        const uint32_t keep_lo = written >= 2 ? 0xffffffffu : (written == 1 ? 0x0000ffffu : 0u);
+        const uint32_t keep_hi = written >= 4 ? 0xffffffffu : (written == 3 ? 0x0000ffffu : 0u);
+#pragma unroll
+        for (int db = 0; db < DB16; ++db) v_reg[b][db].x &= keep_lo, v_reg[b][db].y &= keep_hi;
+      }
     }
     // ---- O += P . V, 32 keys (two blocks) a step; the vector is put together as whole 32-bit words
 #pragma unroll
