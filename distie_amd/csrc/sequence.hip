@@ -655,75 +655,126 @@ __global__ void causal_conv_bf16x8_kernel(const bf16_t* __restrict__ x, int64_t 
 
 __device__ __forceinline__ void load_f32x8(const float* __restrict__ p, float v[8]);
 
-// The same for filters of TAPS = 2, 3 or 4 taps: the filters, the last TAPS - 1 inputs and the sums stay in registers
-// (every index is known when the kernel is compiled), and a thread walks R rows of the step one after the other, so a
-// row of x is read once and serves the TAPS rows that see it. Where a row is its request's first of the step, the
-// inputs before it come from the request's state.
+// The same for filters of TAPS = 2, 3 or 4 taps: a thread takes eight channels of R rows of the step, whose filters, rows and TAPS - 1
+// rows before them are asked for together (a row of x is read once and serves the TAPS rows that see it). Where a row of the block is
+// among its request's first TAPS - 1 of the step, inputs before it come from the request's state, also asked for together, for all
+// rows of the block. What bounds it are three trips to memory (the row's request, its first row, the state) and the activation's
+// exponentials. 899 rows of 2,048 channels in four taps, portions beside single tokens, 7.6 us; with four rows a thread 9.0; with a
+// wait for every row and state row, a look at the activation's kind for every value and blocks of 2,048 channels 13.7.
+template <int N>
+__device__ __forceinline__ void activate_all(float (&v)[N], int kind) {
+  if (kind < 0) return;
+  if (kind == 1) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = activate(v[e], 1);
+  } else if (kind == 2) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = activate(v[e], 2);
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const float p = fmaxf(v[e], 0.f);
+      v[e] = kind == 0 ? p * p : p;
+    }
+  }
+}
+
 template <int TAPS, int R>
-__global__ void causal_conv_bf16_taps_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ weight,
+__global__ void __launch_bounds__(64) causal_conv_bf16_taps_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ weight,
                                              float* __restrict__ state, bf16_t* __restrict__ out, int64_t ldo, int mode,
                                              const float* __restrict__ bias, const int32_t* __restrict__ cu_q,
                                              const int32_t* __restrict__ token_request,
                                              const int32_t* __restrict__ state_slots, int N, int T) {
-  const int c0 = 8 * (blockIdx.y * blockDim.x + threadIdx.x);
-  if (c0 >= N) return;
+  constexpr int BEFORE = TAPS - 1;
+  const int mine = 8 * (blockIdx.y * blockDim.x + threadIdx.x), c0 = min(mine, N - 8);      // (the others ask for the last channels)
+  const bool inside = mine < N;
   const int t0 = blockIdx.x * R;
+  // lane j of a wave asks for row t0 + j's request (row after row through the scalar cache these were twelve trips)
+  const int request = token_request[min(t0 + min(static_cast<int>(threadIdx.x), R - 1), T - 1)];
+  uint4 raw[R + BEFORE], filters[TAPS];
+#pragma unroll
+  for (int r = 0; r < R + BEFORE; ++r) raw[r] = load16(x + static_cast<int64_t>(min(max(t0 + r - BEFORE, 0), T - 1)) * ldx + c0);
+#pragma unroll
+  for (int q = 0; q < TAPS; ++q) filters[q] = load16(weight + static_cast<int64_t>(c0) * TAPS + 8 * q);
+  float add[8] = {};
+  if (bias != nullptr) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) add[e] = bias[c0 + e];
+  }
+  // of the block's rows: place in the request, the request's state, whether it brings this row only
+  int place[R];
+  float* own[R];
+  bool single[R], early = false;
+  {
+    const int first = cu_q[request], next = cu_q[request + 1], row = state_slots[request];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int begin = __builtin_amdgcn_readlane(first, r);
+      place[r] = min(t0 + r, T - 1) - begin;
+      single[r] = __builtin_amdgcn_readlane(next, r) - begin == 1;
+      own[r] = state + static_cast<int64_t>(__builtin_amdgcn_readlane(row, r)) * BEFORE * N + c0;
+      early = early || place[r] < BEFORE;
+    }
+  }
+  float4 held[R][BEFORE][2];
+  if (early) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int k = 0; k < BEFORE; ++k)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) held[r][k][h] = reinterpret_cast<const float4*>(own[r] + static_cast<int64_t>(k) * N)[h];
+  }
   float w[TAPS][8];                     // w[j][e]: tap j of channel c0 + e
   {
     float flat[8 * TAPS];
 #pragma unroll
-    for (int q = 0; q < TAPS; ++q) unpack_bf16x8(load16(weight + static_cast<int64_t>(c0) * TAPS + 8 * q), flat + 8 * q);
+    for (int q = 0; q < TAPS; ++q) unpack_bf16x8(filters[q], flat + 8 * q);
 #pragma unroll
     for (int e = 0; e < 8; ++e)
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) w[j][e] = flat[e * TAPS + j];
   }
-  float add[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) add[e] = bias != nullptr ? bias[c0 + e] : 0.f;
-  float win[TAPS - 1][8];               // the inputs of the TAPS - 1 rows before this one, oldest first
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int t = t0 + r;
-    if (t >= T) break;
-    const int b = token_request[t];
-    const int first = cu_q[b];
-    const int i = t - first;
-    float* own = state + static_cast<int64_t>(state_slots[b]) * (TAPS - 1) * N;
-    if (r == 0 || i == 0) {
+    float win[BEFORE][8], self[8], sum[8];
 #pragma unroll
-      for (int k = 0; k < TAPS - 1; ++k) {
-        const int back = TAPS - 1 - k;
-        if (back <= i) unpack_bf16x8(load16(x + static_cast<int64_t>(t - back) * ldx + c0), win[k]);
-        else load_f32x8(own + static_cast<int64_t>(TAPS - 1 - (back - i)) * N + c0, win[k]);
+    for (int k = 0; k < BEFORE; ++k) unpack_bf16x8(raw[r + k], win[k]);
+    unpack_bf16x8(raw[r + BEFORE], self);
+    if (early) {
+#pragma unroll
+      for (int k = 0; k < BEFORE; ++k) {
+        // input BEFORE - k rows back: of the state, once that is more than `place` rows
+#pragma unroll
+        for (int j = 0; j < BEFORE; ++j) {
+          if (j == k + place[r] && BEFORE - k > place[r]) {
+            win[k][0] = held[r][j][0].x, win[k][1] = held[r][j][0].y, win[k][2] = held[r][j][0].z, win[k][3] = held[r][j][0].w;
+            win[k][4] = held[r][j][1].x, win[k][5] = held[r][j][1].y, win[k][6] = held[r][j][1].z, win[k][7] = held[r][j][1].w;
+          }
+        }
       }
     }
-    float self[8], acc[8];
-    unpack_bf16x8(load16(x + static_cast<int64_t>(t) * ldx + c0), self);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      float sum = 0.f;
+      sum[e] = 0.f;
 #pragma unroll
-      for (int k = 0; k < TAPS - 1; ++k) sum += w[k][e] * win[k][e];
-      sum += w[TAPS - 1][e] * self[e];
-      if (mode & 1) sum += self[e];
-      sum += add[e];
-      acc[e] = (mode >> 1) ? activate(sum, (mode >> 1) - 1) : sum;
+      for (int k = 0; k < BEFORE; ++k) sum[e] += w[k][e] * win[k][e];
+      sum[e] += w[BEFORE][e] * self[e];
+      if (mode & 1) sum[e] += self[e];
+      sum[e] += add[e];
     }
-    *reinterpret_cast<uint4*>(out + static_cast<int64_t>(t) * ldo + c0) = pack_bf16x8(acc);
+    activate_all(sum, (mode >> 1) - 1);
+    if (t0 + r < T && inside) {
+      *reinterpret_cast<uint4*>(out + static_cast<int64_t>(t0 + r) * ldo + c0) = pack_bf16x8(sum);
+      if (early && single[r]) {
+        // a request that brings one row: the window, moved on by that row, is its new state
 #pragma unroll
-    for (int k = 0; k + 1 < TAPS - 1; ++k)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) win[k][e] = win[k + 1][e];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) win[TAPS - 2][e] = self[e];
-    if (i == 0 && cu_q[b + 1] - first == 1) {
-      // a request that brings one row: the window, moved on by that row, is its new state
-#pragma unroll
-      for (int k = 0; k < TAPS - 1; ++k) {
-        float4* to = reinterpret_cast<float4*>(own + static_cast<int64_t>(k) * N + c0);
-        to[0] = float4{win[k][0], win[k][1], win[k][2], win[k][3]};
-        to[1] = float4{win[k][4], win[k][5], win[k][6], win[k][7]};
+        for (int k = 0; k < BEFORE; ++k) {
+          const float* from = k + 1 < BEFORE ? win[k + 1 < BEFORE ? k + 1 : 0] : self;
+          float4* to = reinterpret_cast<float4*>(own[r] + static_cast<int64_t>(k) * N);
+          to[0] = float4{from[0], from[1], from[2], from[3]};
+          to[1] = float4{from[4], from[5], from[6], from[7]};
+        }
       }
     }
   }
@@ -1039,7 +1090,10 @@ head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int64_t 
 // all the rows that see it; where a row is its request's first of the step, the inputs before it come from the request's
 // state. The head's sum of squares is a sum over its lanes; a pair of the rotation lies in the lane itself
 // (`neighbours`) or in the lane pairs / 8 away. The blocks from `qk_blocks` on write v: 16 rows each, one channel a thread.
-constexpr int CONV_ROWS = 4;
+// What bounds it are its trips to memory in a row: which request, where that begins, the state of rows that need it. Everything else a
+// run needs is asked for in front of them, and what is asked for a request is asked for by all rows at once: 899 rows of 8 and 2 heads
+// of 128, portions beside single tokens, 25.4 -> 12.5 us (runs of four rows 20.3, of which the v blocks, row after row, were most).
+constexpr int CONV_ROWS = 2;
 
 template <int TAPS>
 __global__ void __launch_bounds__(256)
@@ -1058,13 +1112,13 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
     const int t0 = (static_cast<int>(blockIdx.x) - qk_blocks) / G * VGROUP;
     const int g = (static_cast<int>(blockIdx.x) - qk_blocks) % G;
     const int n = min(VGROUP, T - t0);
-    const int64_t slot0 = write ? slots[t0] : 0;
-    bool together = write && n == VGROUP && block_size % 8 == 0 && slot0 % block_size % 8 == 0 &&
-                    slot0 % block_size + VGROUP <= block_size;
-    if (write) {
-#pragma unroll
-      for (int k = 1; k < VGROUP; ++k) together = together && slots[min(t0 + k, T - 1)] == slot0 + k;
-    }
+    // lane j of every wave: row t0 + j's request, its first row, the next request's, its state, its place in the cache
+    const int lane = threadIdx.x % 64, row = t0 + min(lane, n - 1);
+    const int request_of = token_request[row], slot_of = write ? slots[row] : 0;
+    const int first_of = cu_q[request_of], next_of = cu_q[request_of + 1], state_of = state_slots[request_of];
+    const int slot0 = __builtin_amdgcn_readlane(slot_of, 0);
+    const bool together = write && n == VGROUP && block_size % 8 == 0 && slot0 % block_size % 8 == 0 &&
+                          slot0 % block_size + VGROUP <= block_size && __all(lane >= VGROUP || slot_of == slot0 + lane);
     uint16_t* cache = reinterpret_cast<uint16_t*>(v_cache);
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
       const int c = (H + G) * D + g * E + e;
@@ -1075,20 +1129,29 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       for (int k = 0; k < VGROUP; ++k) x[k] = to_float(product[static_cast<int64_t>(t0 + min(k, n - 1)) * ld + c]);
 #pragma unroll
       for (int m = 0; m < TAPS - 1; ++m) before[m] = to_float(product[static_cast<int64_t>(max(t0 - 1 - m, 0)) * ld + c]);
+      // some row of the sixteen is among its request's first ones: all rows' states, together
+      float held[VGROUP][TAPS - 1];
+      if (__any(lane < VGROUP && row - first_of < TAPS - 1)) {
+#pragma unroll
+        for (int k = 0; k < VGROUP; ++k)
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j)
+            held[k][j] = state[(static_cast<int64_t>(__builtin_amdgcn_readlane(state_of, k)) * (TAPS - 1) + j) * N + c];
+      }
       uint32_t bits[VGROUP];
 #pragma unroll
       for (int k = 0; k < VGROUP; ++k) {
-        const int b = token_request[t0 + min(k, n - 1)];
-        const int first = cu_q[b];
+        const int first = __builtin_amdgcn_readlane(first_of, k);
         const int i = t0 + min(k, n - 1) - first;
-        float* own = state + static_cast<int64_t>(state_slots[b]) * (TAPS - 1) * N + c;
-        const bool single = k < n && cu_q[b + 1] - first == 1;
+        float* own = state + static_cast<int64_t>(__builtin_amdgcn_readlane(state_of, k)) * (TAPS - 1) * N + c;
+        const bool single = k < n && __builtin_amdgcn_readlane(next_of, k) - first == 1;
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < TAPS; ++j) {
           const int back = TAPS - 1 - j;
           float v = back <= k ? x[k - back < 0 ? 0 : k - back] : before[back - k - 1 < 0 ? 0 : back - k - 1];
-          if (back > i) v = own[static_cast<int64_t>(TAPS - 1 - (back - i)) * N];
+#pragma unroll
+          for (int m = j; m < TAPS - 1; ++m) v = back > i && m == j + i ? held[k][m] : v;
           sum += w[j] * v;
           if (single && j > 0) own[static_cast<int64_t>(j - 1) * N] = v;       // its inputs move on by this row
         }
@@ -1096,7 +1159,7 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       }
       if (!write) continue;
       if (together) {
-        uint16_t* dst = cache + ((slot0 / block_size * G + g) * DP + e) * block_size + slot0 % block_size;
+        uint16_t* dst = cache + ((static_cast<int64_t>(slot0 / block_size) * G + g) * DP + e) * block_size + slot0 % block_size;
         *reinterpret_cast<uint4*>(dst) = uint4{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16),
                                                bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16)};
         *reinterpret_cast<uint4*>(dst + 8) = uint4{bits[8] | (bits[9] << 16), bits[10] | (bits[11] << 16),
@@ -1105,7 +1168,7 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
 #pragma unroll
         for (int k = 0; k < VGROUP; ++k) {
           if (k >= n) break;
-          const int64_t slot = slots[t0 + k];
+          const int64_t slot = __builtin_amdgcn_readlane(slot_of, k);
           cache[((slot / block_size * G + g) * DP + e) * block_size + slot % block_size] = static_cast<uint16_t>(bits[k]);
         }
       }
@@ -1135,27 +1198,68 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
   }
   const float* norm_weight = head < H ? q_norm : k_norm;
   if (norm_weight != nullptr) load_f32x8(norm_weight + min(d0, D - 8), norm);
-  // all rows of the product that the run may need, under way together
+  // everything that the run may need, under way together: the product's rows, their requests, then where these begin, their angles
   uint4 raw[CONV_ROWS + TAPS - 1];
 #pragma unroll
   for (int r = 0; r < CONV_ROWS + TAPS - 1; ++r)
     raw[r] = load16(product + static_cast<int64_t>(min(max(t0 + r - (TAPS - 1), 0), T - 1)) * ld + c0);
+  int request[CONV_ROWS], first[CONV_ROWS], next[CONV_ROWS], state_row[CONV_ROWS], slot_of[CONV_ROWS] = {};
+#pragma unroll
+  for (int r = 0; r < CONV_ROWS; ++r) {
+    request[r] = token_request[min(t0 + r, T - 1)];
+    if (write) slot_of[r] = slots[min(t0 + r, T - 1)];
+  }
+  constexpr int ANGLES = 4;
+  float4 turn[CONV_ROWS][ANGLES];
+  if (neighbours) {
+#pragma unroll
+    for (int r = 0; r < CONV_ROWS; ++r)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        turn[r][e] = pairs > 0 ? reinterpret_cast<const float4*>(table + static_cast<int64_t>(min(t0 + r, T - 1)) * pairs +
+                                                                 min(d0 / 2, pairs - 4))[e] : float4{};
+  } else {
+    const int shift = pairs / 8, at = min(lane < shift ? lane : lane - shift, shift - 1);
+#pragma unroll
+    for (int r = 0; r < CONV_ROWS; ++r)
+#pragma unroll
+      for (int e = 0; e < ANGLES; ++e)
+        turn[r][e] = pairs > 0 ? reinterpret_cast<const float4*>(table + static_cast<int64_t>(min(t0 + r, T - 1)) * pairs + 8 * at)[e]
+                               : float4{};
+  }
+#pragma unroll
+  for (int r = 0; r < CONV_ROWS; ++r) {
+    first[r] = cu_q[request[r]];
+    next[r] = cu_q[request[r] + 1];
+    state_row[r] = state_slots[request[r]];
+  }
 #pragma unroll
   for (int r = 0; r < CONV_ROWS; ++r) {
     const int t = t0 + r;
     const int at = min(t, T - 1);
-    const int b = token_request[at];
-    const int first = cu_q[b];
-    const int i = at - first;
-    float* own = state + static_cast<int64_t>(state_slots[b]) * (TAPS - 1) * N + c0;
-    const bool single = inside && t < T && cu_q[b + 1] - first == 1;
+    const int i = at - first[r];
+    float* own = state + static_cast<int64_t>(state_row[r]) * (TAPS - 1) * N + c0;
+    const bool single = inside && t < T && next[r] - first[r] == 1;
+    float before[TAPS - 1][8];
+    if (__any(i < TAPS - 1)) {
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) load_f32x8(own + static_cast<int64_t>(j) * N, before[j]);
+    }
     float x[8] = {};
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) {
       const int back = TAPS - 1 - j;
       float v[8];
       unpack_bf16x8(raw[r + j], v);
-      if (back > i) load_f32x8(own + static_cast<int64_t>(TAPS - 1 - (back - i)) * N, v);
+      if (back > i) {                                      // row j + i of the state
+#pragma unroll
+        for (int m = j; m < TAPS - 1; ++m) {
+          if (m == j + i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = before[m][e];
+          }
+        }
+      }
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] += w[j][e] * v[e];
       if (single && j > 0) {                               // a request that brings one row: its inputs move on by that row
@@ -1182,10 +1286,9 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
 #pragma unroll
       for (int e = 0; e < 8; ++e) out[e] = x[e];
       if (d0 < 2 * pairs) {                                // (pairs a multiple of 4: all of the lane's pairs turn, or none)
-        const float4* angles = reinterpret_cast<const float4*>(table + static_cast<int64_t>(at) * pairs + d0 / 2);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          const float4 cs = angles[e];
+          const float4 cs = turn[r][e];
           const float* v = x + 4 * e;
           out[4 * e] = v[0] * (cs.x * magnitude) - v[1] * (cs.y * magnitude);
           out[4 * e + 1] = v[1] * (cs.x * magnitude) + v[0] * (cs.y * magnitude);
@@ -1201,10 +1304,9 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       for (int e = 0; e < 8; ++e) other[e] = __shfl(x[e], partner, 64), out[e] = x[e];
       if (lane < 2 * shift) {
         const bool lower = lane < shift;
-        const float4* angles = reinterpret_cast<const float4*>(table + static_cast<int64_t>(at) * pairs + 8 * (lower ? lane : lane - shift));
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float4 cs = angles[e];
+          const float4 cs = turn[r][e];
           const float s0 = lower ? -cs.y : cs.y, s1 = lower ? -cs.w : cs.w;
           out[2 * e] = x[2 * e] * (cs.x * magnitude) + other[2 * e] * (s0 * magnitude);
           out[2 * e + 1] = x[2 * e + 1] * (cs.z * magnitude) + other[2 * e + 1] * (s1 * magnitude);
@@ -1219,7 +1321,7 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       for (int e = 0; e < 8; ++e) out[e] *= qt;
       *reinterpret_cast<uint4*>(q_out + (static_cast<int64_t>(t) * H + head) * DP + d0) = pack_bf16x8(out);
     } else if (write && d0 < D) {
-      const int64_t slot = slots[t];
+      const int64_t slot = slot_of[r];
       bf16_t* dst = k_cache + ((slot / block_size * G + (head - H)) * block_size + slot % block_size) * DP;
       *reinterpret_cast<uint4*>(dst + d0) = pack_bf16x8(out);
     }
@@ -1582,12 +1684,12 @@ extern "C" int distie_causal_conv(const void* x, int x_dtype, int64_t ldx, const
       const bf16_t* xb = static_cast<const bf16_t*>(x);
       const bf16_t* wb = static_cast<const bf16_t*>(weight);
       bf16_t* ob = static_cast<bf16_t*>(out);
-      // few rows: a thread a row, narrow blocks, so that the chip has something to do; many: four rows a thread
-      const int rows = T >= 256 ? 4 : 1;
-      const int threads = T >= 256 ? threads8 : 64;
+      // few rows: a thread a row, so that the chip has something to do; many: two rows a thread
+      const int rows = T >= 256 ? 2 : 1;
+      const int threads = 64;
       const dim3 grid((T + rows - 1) / rows, (items + threads - 1) / threads);
 #define DISTIE_CONV_TAPS(TAPS)                                                                                          \
-  if (rows == 4) causal_conv_bf16_taps_kernel<TAPS, 4><<<grid, threads, 0, stream>>>(                                   \
+  if (rows == 2) causal_conv_bf16_taps_kernel<TAPS, 2><<<grid, threads, 0, stream>>>(                                   \
       xb, ldx, wb, state, ob, ldo, residual, bias, cu_q, token_request, state_slots, N, T);                             \
   else causal_conv_bf16_taps_kernel<TAPS, 1><<<grid, threads, 0, stream>>>(                                             \
       xb, ldx, wb, state, ob, ldo, residual, bias, cu_q, token_request, state_slots, N, T)
