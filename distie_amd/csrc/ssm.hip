@@ -32,7 +32,7 @@ __global__ void __launch_bounds__(64 * PARTS)
 ssm_scan_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restrict__ dt, int64_t ldd,
                 const float* __restrict__ dt_bias, const float* __restrict__ a_log, const float* __restrict__ skip,
                 float* __restrict__ state, float* __restrict__ out, const int32_t* __restrict__ cu_q,
-                const int32_t* __restrict__ state_slots, int H, int P, int N, int G) {
+                const int32_t* __restrict__ state_slots, int H, int P, int N, int G, int most) {
   __shared__ float b_s[PARTS * ROWS], c_s[PARTS * ROWS];
   __shared__ float partial[PARTS][64];
   const int b = blockIdx.x, head = blockIdx.y;
@@ -40,7 +40,7 @@ ssm_scan_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restrict__ dt,
   const int p = blockIdx.z * 64 + lane;
   const int group = head / (H / G);
   const int first = cu_q[b], last = cu_q[b + 1];
-  if (first >= last) return;
+  if (first >= last || last - first > most) return;       // (the others are the chunks')
   const float rate = -expf(a_log[head]);
   const float bias = dt_bias[head], through = skip[head];
   float* own = state + (static_cast<int64_t>(state_slots[b]) * H + head) * N * P;
@@ -96,8 +96,12 @@ ssm_scan_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restrict__ dt,
 //   states:   S_next   = total * S + U, chunk after chunk; S (the state in front) takes U's place in the scratch
 //   pairs:    (C_i . B_j) for the chunk's rows, once for every group of heads that shares B and C
 //   outputs:  y_i[p]   = exp(l_i) sum_n C_i[n] S[n][p] + sum_{j<=i} exp(l_i - l_j) d_j (C_i . B_j) x_j[p] + skip x_i[p]
-// Every exponent is <= 0 and no quotient of decays is formed. Float32 throughout, FMAs on tiles held in LDS; a chunk's
-// table entry is {request, first row, rows, unused}.
+// Every exponent is <= 0 and no quotient of decays is formed. Float32 throughout, matrix products on tiles held in LDS. What bounds
+// sums and outputs are trips to memory and then the float32 products, so whatever does not depend on a result is asked for at the start
+// (`loads_first`: left alone the compiler put each of the sixteen loads of a thread in front of its use), and the next tiles while the
+// ones at hand are multiplied; states: bytes. Two prompts of 450 tokens beside 12 single ones, 32 heads of 128 x 64, us a layer, before /
+// now: sums 22.7 + pairs 9.8 / 16.1 together, states 21.1 / 12.1, outputs 39.2 / 21.0, the single tokens (row by row now) - / 10.8. A chunk's
+// table entry is {request, first row, rows, whether they are all that the request brings and one}.
 constexpr int SSM_L = 64;
 constexpr int SSM_PAD = SSM_L + 1;
 
@@ -110,17 +114,24 @@ __device__ __forceinline__ int tile_row(int v, int lane) { return 8 * (v / 4) + 
 // A 64 x 64 tile of a chunk into LDS: rows j, columns n of `from` (row stride ld), zeros where n >= columns or j >= rows. The
 // sixteen elements a thread brings are asked for together: addresses are clamped into what is there, the rest is dropped.
 template <typename X>
-__device__ __forceinline__ void stage_tile(float (*tile)[SSM_PAD], const X* __restrict__ from, int64_t ld, int rows, int columns) {
+__device__ __forceinline__ void load_tile(X raw[16], const X* __restrict__ from, int64_t ld, int rows, int columns) {
   const int n = threadIdx.x % 64, part = threadIdx.x / 64;
-  X raw[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) raw[r] = from[static_cast<int64_t>(min(part + 4 * r, rows - 1)) * ld + min(n, columns - 1)];
+}
+
+template <typename X>
+__device__ __forceinline__ void put_tile(float (*tile)[SSM_PAD], const X raw[16], int rows, int columns) {
+  const int n = threadIdx.x % 64, part = threadIdx.x / 64;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int j = part + 4 * r;
     tile[j][n] = j < rows && n < columns ? to_float(raw[r]) : 0.f;
   }
 }
+
+// The loads in front of it are asked for before anything behind it (left to itself the compiler puts each in front of its use).
+__device__ __forceinline__ void loads_first() { __builtin_amdgcn_sched_barrier(0); }
 
 // d_j and l_j of a chunk's rows for one head, into LDS (the running sums by the first wave, one row a lane)
 template <typename X>
@@ -141,35 +152,87 @@ __device__ __forceinline__ void chunk_decays(const X* __restrict__ dt, int64_t l
   __syncthreads();
 }
 
-// blockIdx = (chunk, head, 64 columns p): U and the chunk's total decay
+// blockIdx = (chunk, group): (C_i . B_j) for the chunk's rows i and j, the same for every head of the group
+// -> pairs [chunks, G, L, L]. A wave: 32 rows i by 32 columns j.
+template <typename X>
+__device__ __forceinline__ void chunk_pairs(const X* __restrict__ xbc, int64_t ld, float* __restrict__ pairs, int chunk, int group,
+                                            int first, int rows, int H, int P, int N, int G, float (*c_s)[SSM_PAD],
+                                            float (*b_s)[SSM_PAD]) {
+  const int64_t b_at = static_cast<int64_t>(H) * P + static_cast<int64_t>(group) * N;
+  const int64_t c_at = b_at + static_cast<int64_t>(G) * N;
+  const X* from = xbc + static_cast<int64_t>(first) * ld;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int ib = 32 * (wave / 2), jb = 32 * (wave % 2);
+  X b[16], c[16];
+  load_tile(b, from + b_at, ld, rows, N);
+  load_tile(c, from + c_at, ld, rows, N);
+  loads_first();
+  ssm_floatx16 acc = {};
+  for (int n0 = 0; n0 < N; n0 += SSM_L) {
+    __syncthreads();
+    put_tile(b_s, b, rows, N - n0);
+    put_tile(c_s, c, rows, N - n0);
+    if (n0 + SSM_L < N) {
+      load_tile(b, from + b_at + n0 + SSM_L, ld, rows, N - n0 - SSM_L);
+      load_tile(c, from + c_at + n0 + SSM_L, ld, rows, N - n0 - SSM_L);
+      loads_first();
+    }
+    __syncthreads();
+    for (int n = 0; n < SSM_L; n += 2)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(c_s[ib + lane % 32][n + lane / 32], b_s[jb + lane % 32][n + lane / 32],
+                                                 acc, 0, 0, 0);
+  }
+  float* to = pairs + (static_cast<int64_t>(chunk) * G + group) * SSM_L * SSM_L;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) to[(ib + tile_row(v, lane)) * SSM_L + jb + lane % 32] = acc[v];
+}
+
+// blockIdx = (chunk, head, 64 columns p): U and the chunk's total decay; (chunk, H + group, 0): the group's pairs. apart: chunks of
+// requests that bring one row are not worked on (`ssm_scan_kernel` takes those)
 template <typename X>
 __global__ void __launch_bounds__(256)
 ssm_chunk_sums_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restrict__ dt, int64_t ldd,
                       const float* __restrict__ dt_bias, const float* __restrict__ a_log, float* __restrict__ scratch,
-                      float* __restrict__ totals, const int4* __restrict__ chunks, int H, int P, int N, int G) {
+                      float* __restrict__ totals, float* __restrict__ pairs, const int4* __restrict__ chunks, int H, int P, int N,
+                      int G, int apart) {
   __shared__ float d_s[SSM_L], l_s[SSM_L];
   __shared__ float x_s[SSM_L][SSM_PAD];     // [row][p], times the row's factor
   __shared__ float b_s[SSM_L][SSM_PAD];     // [row][n of this pass]
   const int chunk = blockIdx.x, head = blockIdx.y, p0 = blockIdx.z * 64;
   const int4 entry = chunks[chunk];
   const int first = entry.y, rows = entry.z;
+  if (apart && entry.w) return;
+  if (head >= H) {
+    if (blockIdx.z == 0) chunk_pairs(xbc, ld, pairs, chunk, head - H, first, rows, H, P, N, G, x_s, b_s);
+    return;
+  }
   const int group = head / (H / G);
+  const int64_t b_at = static_cast<int64_t>(H) * P + static_cast<int64_t>(group) * N;
+  const X* from = xbc + static_cast<int64_t>(first) * ld;
+  X x[16], b[16];
+  load_tile(x, from + head * P + p0, ld, rows, P - p0);
+  load_tile(b, from + b_at, ld, rows, N);
+  loads_first();
   chunk_decays(dt, ldd, first, rows, head, dt_bias[head], -expf(a_log[head]), d_s, l_s);
   const float l_end = l_s[rows - 1];
   if (threadIdx.x == 0 && blockIdx.z == 0) totals[static_cast<int64_t>(chunk) * H + head] = expf(l_end);
-  if (threadIdx.x < SSM_L) d_s[threadIdx.x] *= expf(l_end - l_s[threadIdx.x]);
-  stage_tile(x_s, xbc + static_cast<int64_t>(first) * ld + head * P + p0, ld, rows, P - p0);
-  __syncthreads();
+  put_tile(x_s, x, rows, P - p0);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) x_s[threadIdx.x / 64 + 4 * r][threadIdx.x % 64] *= d_s[threadIdx.x / 64 + 4 * r];
-  const int64_t b_at = static_cast<int64_t>(H) * P + static_cast<int64_t>(group) * N;
+  for (int r = 0; r < 16; ++r) {
+    const int j = threadIdx.x / 64 + 4 * r;
+    x_s[j][threadIdx.x % 64] *= d_s[j] * expf(l_end - l_s[j]);         // (this thread's own places)
+  }
   float* u = scratch + (static_cast<int64_t>(chunk) * H + head) * N * P;
   // a wave: 32 rows n by 32 columns p of the pass's 64 x 64, on float32 matrix products over the rows j
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const int nb = 32 * (wave / 2), pb = 32 * (wave % 2);
   for (int n0 = 0; n0 < N; n0 += SSM_L) {
-    __syncthreads();
-    stage_tile(b_s, xbc + static_cast<int64_t>(first) * ld + b_at + n0, ld, rows, N - n0);
+    if (n0 > 0) __syncthreads();
+    put_tile(b_s, b, rows, N - n0);
+    if (n0 + SSM_L < N) {
+      load_tile(b, from + b_at + n0 + SSM_L, ld, rows, N - n0 - SSM_L);
+      loads_first();
+    }
     __syncthreads();
     ssm_floatx16 acc = {};
     for (int j = 0; j < SSM_L; j += 2)
@@ -185,54 +248,37 @@ ssm_chunk_sums_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restrict
 
 // a thread an element of a (request, head)'s state: walks the request's chunks in order; the scratch gets the state
 // in front of each chunk, the state tensor the one behind the last
+// (up to STATES_AHEAD of the request's chunks asked for together)
+constexpr int STATES_AHEAD = 8;
 __global__ void ssm_chunk_states_kernel(float* __restrict__ scratch, const float* __restrict__ totals,
                                         float* __restrict__ state, const int32_t* __restrict__ first_chunk,
-                                        const int32_t* __restrict__ state_slots, int H, int64_t size) {
+                                        const int4* __restrict__ chunks, const int32_t* __restrict__ state_slots, int H,
+                                        int64_t size, int apart) {
   const int b = blockIdx.x, head = blockIdx.y;
   const int begin = first_chunk[b], end = first_chunk[b + 1];
-  if (begin >= end) return;
+  if (begin >= end || (apart && chunks[begin].w)) return;
   float* own = state + (static_cast<int64_t>(state_slots[b]) * H + head) * size;
   for (int64_t i = static_cast<int64_t>(blockIdx.z) * blockDim.x + threadIdx.x; i < size;
        i += static_cast<int64_t>(gridDim.z) * blockDim.x) {
     float s = own[i];
-    for (int c = begin; c < end; ++c) {
-      float* u = scratch + (static_cast<int64_t>(c) * H + head) * size + i;
-      const float next = totals[static_cast<int64_t>(c) * H + head] * s + *u;
-      *u = s;
-      s = next;
+    for (int c0 = begin; c0 < end; c0 += STATES_AHEAD) {
+      float u[STATES_AHEAD], total[STATES_AHEAD];
+#pragma unroll
+      for (int k = 0; k < STATES_AHEAD; ++k) {
+        const int64_t place = static_cast<int64_t>(min(c0 + k, end - 1)) * H + head;
+        u[k] = scratch[place * size + i];
+        total[k] = totals[place];
+      }
+      loads_first();
+#pragma unroll
+      for (int k = 0; k < STATES_AHEAD; ++k) {
+        if (c0 + k >= end) break;
+        scratch[(static_cast<int64_t>(c0 + k) * H + head) * size + i] = s;
+        s = total[k] * s + u[k];
+      }
     }
     own[i] = s;
   }
-}
-
-// blockIdx = (chunk, group): (C_i . B_j) for the chunk's rows i and j, the same for every head of the group
-// -> pairs [chunks, G, L, L]. A wave: 32 rows i by 32 columns j.
-template <typename X>
-__global__ void __launch_bounds__(256)
-ssm_chunk_pairs_kernel(const X* __restrict__ xbc, int64_t ld, float* __restrict__ pairs, const int4* __restrict__ chunks,
-                       int H, int P, int N, int G) {
-  __shared__ float c_s[SSM_L][SSM_PAD];       // [i][n of this pass]
-  __shared__ float b_s[SSM_L][SSM_PAD];       // [j][n of this pass]
-  const int chunk = blockIdx.x, group = blockIdx.y;
-  const int4 entry = chunks[chunk];
-  const int first = entry.y, rows = entry.z;
-  const int64_t b_at = static_cast<int64_t>(H) * P + static_cast<int64_t>(group) * N;
-  const int64_t c_at = b_at + static_cast<int64_t>(G) * N;
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int ib = 32 * (wave / 2), jb = 32 * (wave % 2);
-  ssm_floatx16 acc = {};
-  for (int n0 = 0; n0 < N; n0 += SSM_L) {
-    __syncthreads();
-    stage_tile(b_s, xbc + static_cast<int64_t>(first) * ld + b_at + n0, ld, rows, N - n0);
-    stage_tile(c_s, xbc + static_cast<int64_t>(first) * ld + c_at + n0, ld, rows, N - n0);
-    __syncthreads();
-    for (int n = 0; n < SSM_L; n += 2)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(c_s[ib + lane % 32][n + lane / 32], b_s[jb + lane % 32][n + lane / 32],
-                                                 acc, 0, 0, 0);
-  }
-  float* to = pairs + (static_cast<int64_t>(chunk) * G + group) * SSM_L * SSM_L;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) to[(ib + tile_row(v, lane)) * SSM_L + jb + lane % 32] = acc[v];
 }
 
 // blockIdx = (chunk, head, 64 columns p): the chunk's outputs from the state in front of it and its own rows
@@ -242,7 +288,7 @@ ssm_chunk_outputs_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restr
                          const float* __restrict__ dt_bias, const float* __restrict__ a_log,
                          const float* __restrict__ skip, const float* __restrict__ scratch,
                          const float* __restrict__ pairs, float* __restrict__ out, const int4* __restrict__ chunks, int H,
-                         int P, int N, int G) {
+                         int P, int N, int G, int apart) {
   __shared__ float d_s[SSM_L], l_s[SSM_L];
   __shared__ float a_s[SSM_L][SSM_PAD];     // [i][j]: the pair's weight
   __shared__ float t_s[SSM_L][SSM_PAD];     // a tile of C [i][n], then of x [j][p]
@@ -250,34 +296,48 @@ ssm_chunk_outputs_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restr
   const int chunk = blockIdx.x, head = blockIdx.y, p0 = blockIdx.z * 64;
   const int4 entry = chunks[chunk];
   const int first = entry.y, rows = entry.z;
+  if (apart && entry.w) return;
   const int group = head / (H / G);
-  chunk_decays(dt, ldd, first, rows, head, dt_bias[head], -expf(a_log[head]), d_s, l_s);
   const int64_t c_at = static_cast<int64_t>(H) * P + static_cast<int64_t>(G + group) * N;
   const float* s_in = scratch + (static_cast<int64_t>(chunk) * H + head) * N * P;
   const int col = threadIdx.x % 64, part = threadIdx.x / 64;     // a thread: column col, rows part, part + 4, ...
-  // the pairs' weights (zero above the diagonal): (C_i . B_j) exp(l_i - l_j) d_j
   const float* pair = pairs + (static_cast<int64_t>(chunk) * G + group) * SSM_L * SSM_L;
+  const X* from = xbc + static_cast<int64_t>(first) * ld;
+  float weight[16], st[16];
+  X c[16], x[16];
 #pragma unroll
-  for (int r = 0; r < SSM_L / 4; ++r) {
+  for (int r = 0; r < 16; ++r) weight[r] = pair[(part + 4 * r) * SSM_L + col];
+  load_tile(c, from + c_at, ld, rows, N);
+  load_tile(st, s_in + p0, P, N, P - p0);
+  load_tile(x, from + head * P + p0, ld, rows, P - p0);
+  loads_first();
+  chunk_decays(dt, ldd, first, rows, head, dt_bias[head], -expf(a_log[head]), d_s, l_s);
+  // the pairs' weights (zero above the diagonal): (C_i . B_j) exp(l_i - l_j) d_j
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
     const int i = part + 4 * r, j = col;
-    const float weight = pair[i * SSM_L + j];                      // (read whether it counts or not: sixteen loads together)
-    a_s[i][j] = (j <= i && i < rows) ? weight * expf(l_s[i] - l_s[j]) * d_s[j] : 0.f;
+    a_s[i][j] = (j <= i && i < rows) ? weight[r] * expf(l_s[i] - l_s[j]) * d_s[j] : 0.f;
   }
   // a wave: 32 rows i by 32 columns p of the outputs
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const int ib = 32 * (wave / 2), pb = 32 * (wave % 2);
   ssm_floatx16 y = {};                 // the state's share: sum_n C_i[n] S[n][p]
   for (int n0 = 0; n0 < N; n0 += SSM_L) {
-    __syncthreads();
-    stage_tile(t_s, xbc + static_cast<int64_t>(first) * ld + c_at + n0, ld, rows, N - n0);
-    stage_tile(u_s, s_in + static_cast<int64_t>(n0) * P + p0, P, N - n0, P - p0);
+    if (n0 > 0) __syncthreads();
+    put_tile(t_s, c, rows, N - n0);
+    put_tile(u_s, st, N - n0, P - p0);
+    if (n0 + SSM_L < N) {
+      load_tile(c, from + c_at + n0 + SSM_L, ld, rows, N - n0 - SSM_L);
+      load_tile(st, s_in + static_cast<int64_t>(n0 + SSM_L) * P + p0, P, N - n0 - SSM_L, P - p0);
+      loads_first();
+    }
     __syncthreads();
     for (int n = 0; n < SSM_L; n += 2)
       y = __builtin_amdgcn_mfma_f32_32x32x2f32(t_s[ib + lane % 32][n + lane / 32], u_s[n + lane / 32][pb + lane % 32], y,
                                                0, 0, 0);
   }
   __syncthreads();
-  stage_tile(t_s, xbc + static_cast<int64_t>(first) * ld + head * P + p0, ld, rows, P - p0);
+  put_tile(t_s, x, rows, P - p0);
   __syncthreads();
   // the chunk's own rows: sum_{j <= i} a[i][j] x_j[p]; rows j beyond the wave's last i have weight zero
   ssm_floatx16 own = {};
@@ -378,18 +438,17 @@ __global__ void glu_mul_bf16x8_kernel(const uint4* __restrict__ gate_up, uint4* 
 
 extern "C" int distie_ssm_scan_max_state() { return 256; }
 
-extern "C" int distie_ssm_scan(const void* xbc, int dtype, int64_t ld, const void* dt, int64_t ldd, const float* dt_bias,
-                               const float* a_log, const float* skip, float* state, float* out, const int32_t* cu_q,
-                               const int32_t* state_slots, int B, int H, int P, int N, int G, hipStream_t stream) {
-  if (B <= 0) return 0;
-  if (H < 1 || P < 1 || N < 1 || G < 1 || H % G || N > 256 || H > 65535 || ldd < H ||
-      ld < static_cast<int64_t>(H) * P + 2 * static_cast<int64_t>(G) * N)
-    return DISTIE_BAD_ARGUMENT;
+namespace {
+
+// The requests that bring at most `most` rows, row after row.
+int launch_ssm_scan(const void* xbc, int dtype, int64_t ld, const void* dt, int64_t ldd, const float* dt_bias, const float* a_log,
+                    const float* skip, float* state, float* out, const int32_t* cu_q, const int32_t* state_slots, int B, int H, int P,
+                    int N, int G, int most, hipStream_t stream) {
   const dim3 grid(B, H, (P + 63) / 64);
 #define DISTIE_SSM(PARTS, ROWS)                                                                                     \
   DISTIE_DISPATCH(dtype, X, ssm_scan_kernel<X, PARTS, ROWS><<<grid, 64 * PARTS, 0, stream>>>(                       \
       static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd, dt_bias, a_log, skip, state, out, cu_q,       \
-      state_slots, H, P, N, G))
+      state_slots, H, P, N, G, most))
   if (N <= 32) {
     DISTIE_SSM(4, 8);
   } else if (N <= 64) {
@@ -403,31 +462,51 @@ extern "C" int distie_ssm_scan(const void* xbc, int dtype, int64_t ld, const voi
   return launch_status();
 }
 
+}  // namespace
+
+extern "C" int distie_ssm_scan(const void* xbc, int dtype, int64_t ld, const void* dt, int64_t ldd, const float* dt_bias,
+                               const float* a_log, const float* skip, float* state, float* out, const int32_t* cu_q,
+                               const int32_t* state_slots, int B, int H, int P, int N, int G, hipStream_t stream) {
+  if (B <= 0) return 0;
+  if (H < 1 || P < 1 || N < 1 || G < 1 || H % G || N > 256 || H > 65535 || ldd < H ||
+      ld < static_cast<int64_t>(H) * P + 2 * static_cast<int64_t>(G) * N)
+    return DISTIE_BAD_ARGUMENT;
+  return launch_ssm_scan(xbc, dtype, ld, dt, ldd, dt_bias, a_log, skip, state, out, cu_q, state_slots, B, H, P, N, G, 0x7fffffff,
+                         stream);
+}
+
 extern "C" int distie_ssm_scan_chunk_rows() { return SSM_L; }
 
-// scratch float32 [chunks, H, N, P], totals float32 [chunks, H], pairs float32 [chunks, G, L, L]
+// scratch float32 [chunks, H, N, P], totals float32 [chunks, H], pairs float32 [chunks, G, L, L]. singles: how many requests bring one
+// row, whose chunks' fourth word is 1. For those the row-by-row kernel moves a third of the bytes (their state once in and once out;
+// a chunk's sums and the state in front of it go to memory and back as well).
 extern "C" int distie_ssm_scan_chunked(const void* xbc, int dtype, int64_t ld, const void* dt, int64_t ldd,
                                        const float* dt_bias, const float* a_log, const float* skip, float* state,
                                        float* out, float* scratch, float* totals, float* pairs, const void* chunks,
-                                       const int32_t* first_chunk, const int32_t* state_slots, int count, int B, int H,
-                                       int P, int N, int G, hipStream_t stream) {
+                                       const int32_t* first_chunk, const int32_t* cu_q, const int32_t* state_slots, int count, int B,
+                                       int singles, int H, int P, int N, int G, hipStream_t stream) {
   if (B <= 0 || count <= 0) return 0;
-  if (H < 1 || P < 1 || N < 1 || G < 1 || H % G || H > 65535 || ldd < H || pairs == nullptr ||
+  if (H < 1 || P < 1 || N < 1 || G < 1 || H % G || H + G > 65535 || ldd < H || pairs == nullptr ||
       ld < static_cast<int64_t>(H) * P + 2 * static_cast<int64_t>(G) * N)
     return DISTIE_BAD_ARGUMENT;
-  const dim3 grid(count, H, (P + 63) / 64);
   const int64_t size = static_cast<int64_t>(N) * P;
-  const int parts = static_cast<int>((size + 255) / 256 < 64 ? (size + 255) / 256 : 64);
+  const int parts = static_cast<int>((size + 255) / 256 < 64 ? (size + 255) / 256 : 64), columns = (P + 63) / 64;
+  const int apart = singles > 0 && N <= 256 ? 1 : 0;
+  const int4* table = static_cast<const int4*>(chunks);
+  if (apart) {
+    const int status = launch_ssm_scan(xbc, dtype, ld, dt, ldd, dt_bias, a_log, skip, state, out, cu_q, state_slots, B, H, P, N, G, 1,
+                                       stream);
+    if (status != 0) return status;
+  }
   DISTIE_DISPATCH(dtype, X, {
-    ssm_chunk_sums_kernel<X><<<grid, 256, 0, stream>>>(static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd,
-                                                      dt_bias, a_log, scratch, totals, static_cast<const int4*>(chunks),
-                                                      H, P, N, G);
-    ssm_chunk_pairs_kernel<X><<<dim3(count, G), 256, 0, stream>>>(static_cast<const X*>(xbc), ld, pairs,
-                                                                    static_cast<const int4*>(chunks), H, P, N, G);
-    ssm_chunk_states_kernel<<<dim3(B, H, parts), 256, 0, stream>>>(scratch, totals, state, first_chunk, state_slots, H, size);
-    ssm_chunk_outputs_kernel<X><<<grid, 256, 0, stream>>>(static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd,
-                                                         dt_bias, a_log, skip, scratch, pairs, out,
-                                                         static_cast<const int4*>(chunks), H, P, N, G);
+    ssm_chunk_sums_kernel<X><<<dim3(count, H + G, columns), 256, 0, stream>>>(
+        static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd, dt_bias, a_log, scratch, totals, pairs, table, H, P, N, G,
+        apart);
+    ssm_chunk_states_kernel<<<dim3(B, H, parts), 256, 0, stream>>>(scratch, totals, state, first_chunk, table, state_slots, H, size,
+                                                                   apart);
+    ssm_chunk_outputs_kernel<X><<<dim3(count, H, columns), 256, 0, stream>>>(
+        static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd, dt_bias, a_log, skip, scratch, pairs, out, table, H, P, N, G,
+        apart);
   });
   return launch_status();
 }

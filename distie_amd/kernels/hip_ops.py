@@ -600,7 +600,7 @@ class HipOps(Ops):
         o.distie_heads_linear.argtypes = [_P, _I, _I, _P, _I, _P, _I, _I, _I, _I, _I, _P]
         o.distie_head_gate.argtypes = [_P, _I, _I, _I, _P, _I, _L, _P, _I, _I, _I, _P]
         o.distie_ssm_scan.argtypes = [_P, _I, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]
-        o.distie_ssm_scan_chunked.argtypes = [_P, _I, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I,
+        o.distie_ssm_scan_chunked.argtypes = [_P, _I, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                                               _I, _I, _P]
         o.distie_gate_rmsnorm.argtypes = [_P, _P, _I, _F, _P, _I, _L, _P, _I, _I, _I, _I, _I, _P]
         o.distie_glu_mul.argtypes = [_P, _I, _I, _P, _I, _I, _I, _I, _F, _F, _F, _P]
@@ -2096,16 +2096,18 @@ class HipOps(Ops):
 
     def _scan_chunks(self, meta, rows, num_heads, dim, value_dim):
         """Which rows of the step form a chunk of a state's scan, worked out from the step's row counts (known on the
-        host outside captured steps): (number of chunks, the table {request, first row, rows, 0} with the first chunk
-        of every request behind it, scratch for a state a chunk)."""
+        host outside captured steps): (number of chunks, the table {request, first row, rows, 1 for a request that brings one row and
+        0 for the others} with the first chunk of every request behind it, scratch for a state a chunk)."""
         table_key = ("scan_chunk_table", rows)
         held = meta.scratch.get(table_key)
         if held is None:
             cu = np.asarray(meta.host_cu_q, dtype=np.int64)
             table, first = [], [0]
+            meta.scratch["scan_singles"] = int((cu[1:] - cu[:-1] == 1).sum())
             for b in range(meta.num_requests):
+                one = 1 if cu[b + 1] - cu[b] == 1 else 0
                 for at in range(int(cu[b]), int(cu[b + 1]), rows):
-                    table.append((b, at, min(rows, int(cu[b + 1]) - at), 0))
+                    table.append((b, at, min(rows, int(cu[b + 1]) - at), one))
                 first.append(len(table))
             packed = self.upload(np.concatenate([np.asarray(table, dtype=np.int32).reshape(-1),
                                                  np.asarray(first, dtype=np.int32)]))
@@ -2781,8 +2783,8 @@ class HipOps(Ops):
             _check(self._ops.distie_ssm_scan_chunked(
                 x_ptr, _code(xbc), ld, d_ptr, ldd, dt_bias, a_log, skip,
                 state, out, scratch, totals, pairs, packed,
-                packed.data_ptr() + 16 * count, meta.state_slots, count, meta.num_requests, H, P, N, G,
-                self._stream()), "ssm_scan_chunked")
+                packed.data_ptr() + 16 * count, meta.cu_q, meta.state_slots, count, meta.num_requests,
+                meta.scratch["scan_singles"], H, P, N, G, self._stream()), "ssm_scan_chunked")
             _mark_written(state)
             return out
         if wide:
