@@ -183,28 +183,58 @@ __device__ __forceinline__ float groups_sum(float v) {        // over the four l
 
 // a lane's channels of one row of a head (`row` points at the head's first column); zeros for a row that is not there
 template <int DP, typename X>
-__device__ __forceinline__ void load_channels(const X* __restrict__ row, int D, int g, bool there, bool whole, float out[DP / 4]) {
+__device__ __forceinline__ void load_channels(const X* __restrict__ row, int D, int g, bool there, float out[DP / 4]) {
   constexpr int DL = DP / 4;
 #pragma unroll
   for (int s = 0; s < DL; ++s) out[s] = 0.f;
   if (!there) return;
-  if (whole) {
 #pragma unroll
-    for (int s = 0; s < DL; s += 4) load_values<4>(row + DL * g + s, out + s);
-  } else {
-#pragma unroll
-    for (int s = 0; s < DL; ++s)
-      if (DL * g + s < D) out[s] = to_float(row[DL * g + s]);
-  }
+  for (int s = 0; s < DL; ++s)
+    if (DL * g + s < D) out[s] = to_float(row[DL * g + s]);
 }
 
-// log2 of the decays of a lane's channels, summed over the rows of the run up to the lane's own
-template <int DP>
-__device__ __forceinline__ void run_decays(const float* __restrict__ z, int D, int g, bool there, bool whole, float c[DP / 4]) {
-  constexpr int DL = DP / 4;
-  load_channels<DP>(z, D, g, there, whole, c);
+// Four neighbouring values as they lie in memory: asked for here, turned into float32 where they are needed.
+template <typename X> struct Four;
+template <> struct Four<float> {
+  float4 raw;
+  __device__ __forceinline__ void load(const float* p) { raw = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ void values(bool there, float v[4]) const {
+    v[0] = there ? raw.x : 0.f, v[1] = there ? raw.y : 0.f, v[2] = there ? raw.z : 0.f, v[3] = there ? raw.w : 0.f;
+  }
+};
+template <> struct Four<bf16_t> {
+  uint2 raw;
+  __device__ __forceinline__ void load(const bf16_t* p) { raw = *reinterpret_cast<const uint2*>(p); }
+  __device__ __forceinline__ void values(bool there, float v[4]) const {
+    const uint32_t a = there ? raw.x : 0u, b = there ? raw.y : 0u;
+    v[0] = __uint_as_float(a << 16), v[1] = __uint_as_float(a & 0xffff0000u);
+    v[2] = __uint_as_float(b << 16), v[3] = __uint_as_float(b & 0xffff0000u);
+  }
+};
+
+// The loads in front of it are asked for before anything behind it: what a lane needs at the start is one trip to memory then. (Left to
+// itself, and with a choice at every load between whole heads and others, the compiler waited for r, k, ln w, each piece of V and the
+// state one after the other: 2 prompts of 901, 32 heads of 64, outputs 42.2 -> 38.2 us, sums 16.3 -> 15.6; four workgroups a compute
+// unit hid the rest.)
+__device__ __forceinline__ void loads_first() { __builtin_amdgcn_sched_barrier(0); }
+
+// a lane's channels of a row of a whole head, which is there in memory whether it counts or not
+template <int DP, typename X>
+__device__ __forceinline__ void ask_channels(const X* __restrict__ row, int g, Four<X> (&raw)[DP / 16]) {
 #pragma unroll
-  for (int s = 0; s < DL; ++s) {
+  for (int s = 0; s < DP / 16; ++s) raw[s].load(row + DP / 4 * g + 4 * s);
+}
+template <int DP, typename X>
+__device__ __forceinline__ void take_channels(const Four<X> (&raw)[DP / 16], bool there, float out[DP / 4]) {
+#pragma unroll
+  for (int s = 0; s < DP / 16; ++s) raw[s].values(there, out + 4 * s);
+}
+
+// log2 of the decays of a lane's channels (c: ln of minus their ln), summed over the rows of the run up to the lane's own
+template <int DP>
+__device__ __forceinline__ void sum_decays(bool there, float c[DP / 4]) {
+#pragma unroll
+  for (int s = 0; s < DP / 4; ++s) {
     // (a factor of 2^-160 is zero in float32: smaller ones need no larger exponents, and infinities have no differences)
     c[s] = there ? fmaxf(-LOG2E * expf(c[s]), -160.f) : 0.f;
     c[s] += row_shift<1>(c[s]);
@@ -216,29 +246,45 @@ __device__ __forceinline__ void run_decays(const float* __restrict__ z, int D, i
 
 // V of a chunk into LDS as float32, rows DP + 4 apart, zeros for what is not there
 template <int DP, typename X>
-__device__ __forceinline__ void stage_rows(const X* __restrict__ v, int64_t ld, int len, int D, bool whole, float* __restrict__ to) {
+__device__ __forceinline__ void stage_rows(const X* __restrict__ v, int64_t ld, int len, int D, float* __restrict__ to) {
   constexpr int RUNS = DP / 4;
   for (int idx = threadIdx.x; idx < WK_ROWS * RUNS; idx += blockDim.x) {
     const int j = idx / RUNS, e = idx % RUNS * 4;
     float x[4] = {};
     if (j < len) {
-      if (whole) {
-        load_values<4>(v + j * ld + e, x);
-      } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (e + k < D) x[k] = to_float(v[j * ld + e + k]);
-      }
+      for (int k = 0; k < 4; ++k)
+        if (e + k < D) x[k] = to_float(v[j * ld + e + k]);
     }
     store_values<4>(to + j * (DP + 4) + e, x);
   }
 }
 
+// The same of whole heads, in two halves: a thread's pieces, and their places in LDS.
 template <int DP, typename X>
+__device__ __forceinline__ void ask_rows(const X* __restrict__ v, int64_t ld, int len, Four<X> (&raw)[DP / 16]) {
+#pragma unroll
+  for (int p = 0; p < DP / 16; ++p) {
+    const int idx = threadIdx.x + 256 * p;
+    raw[p].load(v + min(idx / (DP / 4), len - 1) * ld + idx % (DP / 4) * 4);
+  }
+}
+template <int DP, typename X>
+__device__ __forceinline__ void put_rows(const Four<X> (&raw)[DP / 16], int len, float* __restrict__ to) {
+#pragma unroll
+  for (int p = 0; p < DP / 16; ++p) {
+    const int idx = threadIdx.x + 256 * p, j = idx / (DP / 4);
+    float x[4];
+    raw[p].values(j < len, x);
+    store_values<4>(to + j * (DP + 4) + idx % (DP / 4) * 4, x);
+  }
+}
+
+// WHOLE: D is DP, and everything begins where four values may be loaded at once
+template <int DP, bool WHOLE, typename X>
 __global__ void __launch_bounds__(256)
 wkv_chunk_sums_kernel(const X* __restrict__ k_in, const X* __restrict__ v_in, int64_t ld, const float* __restrict__ z,
-                      float* __restrict__ scratch, float* __restrict__ totals, const int4* __restrict__ chunks, int H, int D,
-                      int whole) {
+                      float* __restrict__ scratch, float* __restrict__ totals, const int4* __restrict__ chunks, int H, int D) {
   constexpr int DL = DP / 4, STRIDE = DP + 4;
   __shared__ __attribute__((aligned(16))) float Ks[WK_ROWS * STRIDE];
   __shared__ __attribute__((aligned(16))) float Vs[WK_ROWS * STRIDE];
@@ -250,9 +296,23 @@ wkv_chunk_sums_kernel(const X* __restrict__ k_in, const X* __restrict__ v_in, in
   const int lane = threadIdx.x % 64, run = threadIdx.x / 64, i = lane % 16, g = lane / 16;
   const int row = 16 * run + i;
   float k[DL], c[DL];
-  load_channels<DP>(k_in + (row0 + row) * ld + head * D, D, g, row < len, whole, k);
-  run_decays<DP>(z + ((row0 + row) * H + head) * D, D, g, row < len, whole, c);
-  stage_rows<DP>(v_in + row0 * ld + head * D, ld, len, D, whole, Vs);
+  if constexpr (WHOLE) {
+    const int64_t at = row0 + min(row, len - 1);
+    Four<X> k4[DP / 16], v4[DP / 16];
+    Four<float> z4[DP / 16];
+    ask_channels<DP>(z + (at * H + head) * D, g, z4);
+    ask_channels<DP>(k_in + at * ld + head * D, g, k4);
+    ask_rows<DP>(v_in + row0 * ld + head * D, ld, len, v4);
+    loads_first();
+    take_channels<DP>(z4, row < len, c);
+    take_channels<DP>(k4, row < len, k);
+    put_rows<DP>(v4, len, Vs);
+  } else {
+    load_channels<DP>(k_in + (row0 + row) * ld + head * D, D, g, row < len, k);
+    load_channels<DP>(z + ((row0 + row) * H + head) * D, D, g, row < len, c);
+    stage_rows<DP>(v_in + row0 * ld + head * D, ld, len, D, Vs);
+  }
+  sum_decays<DP>(row < len, c);
 #pragma unroll
   for (int s = 0; s < DL; ++s) {
     const float total = row_lane<15>(c[s]);
@@ -355,12 +415,12 @@ constexpr int wk_shared() {
   return LATE ? (k > s ? k : s) : k + s;
 }
 
-template <int DP, bool LATE, typename X, typename O>
+template <int DP, bool LATE, bool WHOLE, typename X, typename O>
 __global__ void __launch_bounds__(256, LATE ? 4 : 2)
 wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in, const X* __restrict__ v_in,
                          const X* __restrict__ gates, int64_t ld, const float* __restrict__ z, const float* __restrict__ bonus,
                          const float* __restrict__ scratch, const float* __restrict__ norm_weight, float eps,
-                         O* __restrict__ out, const int4* __restrict__ chunks, int H, int D, int whole) {
+                         O* __restrict__ out, const int4* __restrict__ chunks, int H, int D) {
   constexpr int DL = DP / 4, STRIDE = DP + 4;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float* Vs = lds;                                  // [64][DP + 4]
@@ -374,10 +434,6 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
   const int lane = threadIdx.x % 64, run = threadIdx.x / 64, i = lane % 16, g = lane / 16;
   const int row = 16 * run + i;
   float r[DL], k[DL], c[DL], x[DL];
-  load_channels<DP>(r_in + (row0 + row) * ld + head * D, D, g, row < len, whole, r);
-  load_channels<DP>(k_in + (row0 + row) * ld + head * D, D, g, row < len, whole, k);
-  run_decays<DP>(z + ((row0 + row) * H + head) * D, D, g, row < len, whole, c);
-  stage_rows<DP>(v_in + row0 * ld + head * D, ld, len, D, whole, Vs);
   const float* src = scratch + (static_cast<int64_t>(blockIdx.x) * H + head) * D * D;
   constexpr int PIECES = (DP * DP / 4 + 255) / 256; // of S, a thread's
   float held[LATE ? PIECES : 1][4];
@@ -385,21 +441,51 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
     const int d = idx / (DP / 4), e = idx % (DP / 4) * 4;
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = 0.f;
-    if (whole) {
-      if (DP * DP / 4 % 256 == 0 || d < DP) load_values<4>(src + static_cast<int64_t>(d) * D + e, v);
+    if constexpr (WHOLE) {
+      load_values<4>(src + static_cast<int64_t>(min(d, DP - 1)) * D + e, v);
     } else if (d < D) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if (e + q < D) v[q] = src[static_cast<int64_t>(d) * D + e + q];
     }
   };
+  float u[DL];                                      // the bonus
+  if constexpr (WHOLE) {
+    const int64_t at = row0 + min(row, len - 1);
+    Four<X> r4[DP / 16], k4[DP / 16], v4[DP / 16];
+    Four<float> z4[DP / 16], u4[DP / 16];
+    ask_channels<DP>(z + (at * H + head) * D, g, z4);
+    ask_channels<DP>(k_in + at * ld + head * D, g, k4);
+    ask_channels<DP>(r_in + at * ld + head * D, g, r4);
+    ask_rows<DP>(v_in + row0 * ld + head * D, ld, len, v4);
+    ask_channels<DP>(bonus + head * D, g, u4);
+    if constexpr (LATE) {
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) load_state(threadIdx.x + 256 * p, held[p]);
+    }
+    loads_first();
+    take_channels<DP>(z4, row < len, c);
+    take_channels<DP>(k4, row < len, k);
+    take_channels<DP>(r4, row < len, r);
+    take_channels<DP>(u4, true, u);
+    put_rows<DP>(v4, len, Vs);
+  } else {
+    load_channels<DP>(r_in + (row0 + row) * ld + head * D, D, g, row < len, r);
+    load_channels<DP>(k_in + (row0 + row) * ld + head * D, D, g, row < len, k);
+    load_channels<DP>(z + ((row0 + row) * H + head) * D, D, g, row < len, c);
+    load_channels<DP>(bonus + head * D, D, g, true, u);
+    stage_rows<DP>(v_in + row0 * ld + head * D, ld, len, D, Vs);
+  }
+  sum_decays<DP>(row < len, c);
   auto stage_state = [&](int idx, const float v[4]) __attribute__((always_inline)) {
     const int d = idx / (DP / 4), e = idx % (DP / 4) * 4;
     if (DP * DP / 4 % 256 == 0 || d < DP) store_values<4>(Ss + d * DP + (e + 16 * (d / DL)) % DP, v);
   };
   if constexpr (LATE) {
+    if constexpr (!WHOLE) {
 #pragma unroll
-    for (int p = 0; p < PIECES; ++p) load_state(threadIdx.x + 256 * p, held[p]);
+      for (int p = 0; p < PIECES; ++p) load_state(threadIdx.x + 256 * p, held[p]);
+    }
   } else {
     for (int idx = threadIdx.x; idx < DP * DP / 4; idx += 256) {
       float v[4];
@@ -422,7 +508,7 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
 #pragma unroll
   for (int s = 0; s < DL; ++s) {
     x[s] = row_shift<1>(c[s]);
-    own += DL * g + s < D ? r[s] * bonus[head * D + DL * g + s] * k[s] : 0.f;
+    own += r[s] * u[s] * k[s];                      // (zeros beyond D)
   }
   own = groups_sum(own);
   float a[4] = {};
@@ -469,7 +555,17 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
 #pragma unroll
     for (int e = 0; e < DP / 16; ++e)
       acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(r[s], Ss[(DL * g + s) * DP + (16 * e + i + 16 * g) % DP], acc[e], 0, 0, 0);
-  // lane (i, g) now holds rows 4 g .. 4 g + 3 of the run, column i of every 16
+  // lane (i, g) now holds rows 4 g .. 4 g + 3 of the run, column i of every 16; their gates and weights, together
+  X gate_of[4][DP / 16];
+  float weight[DP / 16];
+#pragma unroll
+  for (int e = 0; e < DP / 16; ++e) weight[e] = norm_weight[head * D + min(16 * e + i, D - 1)];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int e = 0; e < DP / 16; ++e)
+      gate_of[q][e] = gates[(row0 + min(16 * run + 4 * g + q, len - 1)) * ld + head * D + min(16 * e + i, D - 1)];
+  loads_first();
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     float sq = 0.f;
@@ -479,15 +575,13 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
     for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
     const float scale = 1.f / sqrtf(sq / D + eps);
     const int at = 16 * run + 4 * g + q;
-    if (at >= len) continue;
     const int64_t t = row0 + at;
 #pragma unroll
     for (int e = 0; e < DP / 16; ++e) {
       const int col = 16 * e + i;
-      if (col >= D) continue;
-      const float gate = to_float(gates[t * ld + head * D + col]);
-      out[(t * H + head) * D + col] =
-          from_float<O>(acc[e][q] * scale * norm_weight[head * D + col] * (gate / (1.f + expf(-gate))));
+      const float gate = to_float(gate_of[q][e]);
+      const float value = acc[e][q] * scale * weight[e] * (gate / (1.f + expf(-gate)));
+      if (at < len && col < D) out[(t * H + head) * D + col] = from_float<O>(value);
     }
   }
 }
@@ -568,41 +662,48 @@ extern "C" int distie_wkv_scan_chunked(const void* r, const void* k, const void*
   const int4* table = reinterpret_cast<const int4*>(chunks);
   const dim3 grid(num_chunks, H);
   const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const int vectors = ld % 4 == 0 && aligned(r) && aligned(k) && aligned(v) && aligned(z) && aligned(scratch) ? 1 : 0;
+  const int vectors = ld % 4 == 0 && aligned(r) && aligned(k) && aligned(v) && aligned(z) && aligned(scratch) && aligned(bonus) ? 1 : 0;
   int status = 0;
-#define DISTIE_WKV_CHUNKS(DP)                                                                                            \
+#define DISTIE_WKV_CHUNKS(DP, WHOLE)                                                                                     \
   DISTIE_DISPATCH(dtype, X, DISTIE_DISPATCH(out_dtype, O, {                                                              \
     const bool late = DP <= 64 && static_cast<int64_t>(num_chunks) * H > WK_EARLY_WORKGROUPS;                            \
-    const auto outputs = late ? wkv_chunk_outputs_kernel<DP, DP <= 64, X, O> : wkv_chunk_outputs_kernel<DP, false, X, O>;\
+    const auto outputs = late ? wkv_chunk_outputs_kernel<DP, DP <= 64, WHOLE, X, O>                                      \
+                              : wkv_chunk_outputs_kernel<DP, false, WHOLE, X, O>;                                        \
     const int shared = late ? wk_shared<DP, true>() : wk_shared<DP, false>();                                            \
     const int bytes = (WK_ROWS * (DP + 4) + shared + 4 * DP) * static_cast<int>(sizeof(float));                          \
-    const int whole = vectors && D == DP ? 1 : 0;                                                                        \
     if (bytes > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(outputs),                                 \
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)       \
       return DISTIE_BAD_ARGUMENT;                                                                                        \
-    wkv_chunk_sums_kernel<DP, X><<<grid, 256, 0, stream>>>(static_cast<const X*>(k), static_cast<const X*>(v), ld, z,    \
-                                                           scratch, totals, table, H, D, whole);                         \
+    wkv_chunk_sums_kernel<DP, WHOLE, X><<<grid, 256, 0, stream>>>(static_cast<const X*>(k), static_cast<const X*>(v), ld, z,   \
+                                                                  scratch, totals, table, H, D);                         \
     if ((status = launch_status()) != 0) return status;                                                                  \
     wkv_chunk_states_kernel<<<dim3(B, H, (D * D + 255) / 256), 256, 0, stream>>>(scratch, totals, state, request_chunks, \
                                                                                 state_slots, H, D);                      \
     if ((status = launch_status()) != 0) return status;                                                                  \
     outputs<<<grid, 256, bytes, stream>>>(                                                                               \
         static_cast<const X*>(r), static_cast<const X*>(k), static_cast<const X*>(v), static_cast<const X*>(gates), ld,  \
-        z, bonus, scratch, norm_weight, eps, static_cast<O*>(out), table, H, D, whole);                                  \
+        z, bonus, scratch, norm_weight, eps, static_cast<O*>(out), table, H, D);                                         \
   }))
-  if (D <= 16) {
-    DISTIE_WKV_CHUNKS(16);
-  } else if (D <= 32) {
-    DISTIE_WKV_CHUNKS(32);
-  } else if (D <= 48) {
-    DISTIE_WKV_CHUNKS(48);
-  } else if (D <= 64) {
-    DISTIE_WKV_CHUNKS(64);
-  } else if (D <= 96) {
-    DISTIE_WKV_CHUNKS(96);
-  } else {
-    DISTIE_WKV_CHUNKS(128);
+#define DISTIE_WKV_WHOLE(DP)             \
+  if (vectors && D == DP) {              \
+    DISTIE_WKV_CHUNKS(DP, true);         \
+  } else {                               \
+    DISTIE_WKV_CHUNKS(DP, false);        \
   }
+  if (D <= 16) {
+    DISTIE_WKV_WHOLE(16);
+  } else if (D <= 32) {
+    DISTIE_WKV_WHOLE(32);
+  } else if (D <= 48) {
+    DISTIE_WKV_WHOLE(48);
+  } else if (D <= 64) {
+    DISTIE_WKV_WHOLE(64);
+  } else if (D <= 96) {
+    DISTIE_WKV_WHOLE(96);
+  } else {
+    DISTIE_WKV_WHOLE(128);
+  }
+#undef DISTIE_WKV_WHOLE
 #undef DISTIE_WKV_CHUNKS
   return launch_status();
 }
