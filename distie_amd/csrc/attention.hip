@@ -628,8 +628,8 @@ __global__ __launch_bounds__(DISTIE_WAVE * CF_WAVES, 1) void attn_columns_f32_ke
         best = fmaxf(best, s[b][i]);
       }
     }
-    best = fmaxf(best, __shfl_xor(best, 16, DISTIE_WAVE));
-    best = fmaxf(best, __shfl_xor(best, 32, DISTIE_WAVE));
+    best = lanes_max<16>(best);
+    best = lanes_max<32>(best);
     const float m_new = fmaxf(m_run, best);
     const float alpha = m_new == -INFINITY ? 0.f : expf(m_run - m_new);      // 0 on the first chunk with a key (m = -inf)
     float sum = 0.f;
@@ -669,8 +669,8 @@ __global__ __launch_bounds__(DISTIE_WAVE * CF_WAVES, 1) void attn_columns_f32_ke
       }
     }
   }
-  l_run += __shfl_xor(l_run, 16, DISTIE_WAVE);
-  l_run += __shfl_xor(l_run, 32, DISTIE_WAVE);
+  l_run = lanes_sum<16>(l_run);
+  l_run = lanes_sum<32>(l_run);
   // columns first_col .. end_col are this turn's
   const int first_col = turn > 0 ? (turn - 1) * group : 0, end_col = turn > 0 ? turn * group : 16;
   if (g == 0 && r >= first_col && r < end_col) {
@@ -1213,8 +1213,8 @@ __global__ __launch_bounds__(DISTIE_WAVE * W, (MB == 1 && D <= 128 ? 2 : 1)) voi
           s[mb][b][i] = v;
           best = fmaxf(best, v);
         }
-      best = fmaxf(best, __shfl_xor(best, 16, DISTIE_WAVE));
-      best = fmaxf(best, __shfl_xor(best, 32, DISTIE_WAVE));
+      best = lanes_max<16>(best);
+      best = lanes_max<32>(best);
       const float m_new = fmaxf(m_run[mb], best);      // finite: every chunk of the run holds a key
       alpha[mb] = fast_exp2(m_run[mb] - m_new);        // 0 while m_run is -inf
       float sum = 0.f;
@@ -1269,8 +1269,8 @@ __global__ __launch_bounds__(DISTIE_WAVE * W, (MB == 1 && D <= 128 ? 2 : 1)) voi
   // ---- sums over the lanes of a column, then the partial result of this run
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    l_run[mb] += __shfl_xor(l_run[mb], 16, DISTIE_WAVE);
-    l_run[mb] += __shfl_xor(l_run[mb], 32, DISTIE_WAVE);
+    l_run[mb] = lanes_sum<16>(l_run[mb]);
+    l_run[mb] = lanes_sum<32>(l_run[mb]);
   }
   const int places = (max_splits + W - 1) / W;                  // for partial results, per request and head
   const int64_t head0 = static_cast<int64_t>(request) * heads + kh * group;
@@ -1764,7 +1764,7 @@ __global__ __launch_bounds__(PF_THREADS, (D <= 128) ? 2 : 1) void attn_prefill_k
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) top = fmaxf(top, s[kb][e]);
-    top = fmaxf(top, __shfl_xor(top, 32, DISTIE_WAVE));
+    top = lanes_max<32>(top);
     const float best = top * scale_log2;                  // the scale is positive: the largest stays the largest
     if (__any(best > m_run + PF_GROW)) {                  // also the first score of a column (m = -inf)
       const float m_new = fmaxf(m_run, best);
@@ -1833,7 +1833,7 @@ __global__ __launch_bounds__(PF_THREADS, (D <= 128) ? 2 : 1) void attn_prefill_k
     compute(k0);
   }
   // ---- write: the lane holds, of its column, output rows 32 db + 8 i + 4 h + (0..3)
-  l_run += __shfl_xor(l_run, 32, DISTIE_WAVE);
+  l_run = lanes_sum<32>(l_run);
   if (wave_col0 + c >= columns) return;
   const int64_t row = static_cast<int64_t>(token0 + wave_col0 + c) * heads + head;
   if (gridDim.z == 1) {
@@ -2010,13 +2010,6 @@ constexpr int prefill_keys_tiles() {
 template <int W>
 constexpr int prefill_keys_lds() { return prefill_keys_tiles<W>() + (W + 1) * KEYS_BM * 8; }
 
-// The larger of a column's two values, in lanes c and c + 32.
-__device__ __forceinline__ float column_max(float v) {
-  const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
-  const uint32_t low = both[0], high = both[1];
-  return fmaxf(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
-}
-
 template <int W>
 __global__ __launch_bounds__(DISTIE_WAVE * W) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_keys_kernel(
     const bf16_t* __restrict__ qkv, int64_t q_stride, const bf16_t* __restrict__ k_cache,
@@ -2167,7 +2160,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * W) __attribute__((amdgpu_waves_per_eu
     float top = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) top = fmaxf(top, s[e]);
-    const float best = column_max(top) * scale_log2;
+    const float best = lanes_max<32>(top) * scale_log2;
     if (__any(best > m_run + PF_GROW)) {
       const float m_new = fmaxf(m_run, best);
       const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
@@ -2234,7 +2227,7 @@ __global__ __launch_bounds__(DISTIE_WAVE * W) __attribute__((amdgpu_waves_per_eu
   float* const sums = reinterpret_cast<float*>(keys_lds);
   float2* const refs = reinterpret_cast<float2*>(keys_lds + prefill_keys_tiles<W>());     // [wave][column]
   float* const inverse = reinterpret_cast<float*>(refs + W * KEYS_BM);                    // [column]
-  l_run += __shfl_xor(l_run, 32, DISTIE_WAVE);
+  l_run = lanes_sum<32>(l_run);
   if (h == 0) refs[wave * KEYS_BM + c] = float2{m_run, l_run};
   __syncthreads();
   {
@@ -2492,7 +2485,7 @@ __global__ __launch_bounds__(PF_THREADS, 1) void attn_prefill_f32_kernel(
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) top = fmaxf(top, s[kb][e]);
-    top = fmaxf(top, __shfl_xor(top, 32, DISTIE_WAVE));
+    top = lanes_max<32>(top);
     const float best = top * scale_log2;
     if (__any(best > m_run + PF_GROW)) {
       const float m_new = fmaxf(m_run, best);
@@ -2557,7 +2550,7 @@ __global__ __launch_bounds__(PF_THREADS, 1) void attn_prefill_f32_kernel(
     compute(k0);
   }
   // ---- write: the lane holds, of its column, output rows 32 db + 8 i + 4 h + (0..3)
-  l_run += __shfl_xor(l_run, 32, DISTIE_WAVE);
+  l_run = lanes_sum<32>(l_run);
   if (wave_col0 + c >= columns) return;
   const int64_t row = static_cast<int64_t>(token0 + wave_col0 + c) * heads + head;
   const bool whole = gridDim.z == 1;

@@ -213,10 +213,10 @@ delta_chunk_prepare_kernel(const X* __restrict__ qkv, int64_t ld, const X* __res
       }
     }
   }
-  q_sq += __shfl_xor(q_sq, 1, 64);
-  k_sq += __shfl_xor(k_sq, 1, 64);
-  q_sq += __shfl_xor(q_sq, 2, 64);
-  k_sq += __shfl_xor(k_sq, 2, 64);
+  q_sq = lanes_sum<1>(q_sq);
+  k_sq = lanes_sum<1>(k_sq);
+  q_sq = lanes_sum<2>(q_sq);
+  k_sq = lanes_sum<2>(k_sq);
   if (sum_part == 0) {
     q_unit[sum_row] = q_scale / sqrtf(q_sq + unit_eps);
     k_unit[sum_row] = 1.f / sqrtf(k_sq + unit_eps);

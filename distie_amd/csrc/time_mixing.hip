@@ -177,8 +177,7 @@ template <int N>
 __device__ __forceinline__ float row_lane(float x) { return row_move<0x150 + N>(x); }        // lane N of the row, to all
 
 __device__ __forceinline__ float groups_sum(float v) {        // over the four lanes that own a row
-  v += __shfl_xor(v, 16, 64);
-  return v + __shfl_xor(v, 32, 64);
+  return lanes_sum<32>(lanes_sum<16>(v));
 }
 
 // a lane's channels of one row of a head (`row` points at the head's first column); zeros for a row that is not there
@@ -571,8 +570,7 @@ wkv_chunk_outputs_kernel(const X* __restrict__ r_in, const X* __restrict__ k_in,
     float sq = 0.f;
 #pragma unroll
     for (int e = 0; e < DP / 16; ++e) sq += acc[e][q] * acc[e][q];
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+    sq = lanes_sum<1>(lanes_sum<2>(lanes_sum<4>(lanes_sum<8>(sq))));
     const float scale = 1.f / sqrtf(sq / D + eps);
     const int at = 16 * run + 4 * g + q;
     const int64_t t = row0 + at;
