@@ -230,21 +230,26 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_generic_kernel(
 }
 
 // The same walk in float32 for requests that decode, with loads that cover whole rows: one workgroup per
-// (token, kv head, part of up to G query heads of it). For the scores eight lanes share a key: each reads an
-// eighth of the key's row of K (a run of D / 8 floats, so a wave's load covers eight whole rows; with a lane
-// to a key every 16-byte load of a wave touched 64 lines) against its slices of the heads' queries, which it
-// keeps in registers; the sums of the eight lanes are added by three exchanges. With G > 1 every row of K
-// and every value of V^T is read once for G heads.
+// (token, kv head, part of up to G query heads of it). For the scores eight lanes share a key: each reads 16 of every 128 bytes
+// of the key's row of K (a load covers whole lines of eight rows) against its columns of the heads' queries, which it keeps in registers;
+// the sums of the eight lanes are added by three exchanges. For the output four lanes share a dimension: each reads four of every
+// sixteen keys (a load covers 64 bytes of sixteen neighbouring rows of V^T, one run of 1,024 bytes in pages of sixteen tokens), and
+// their sums meet when all keys are through. With G > 1 every row of K and every value of V^T is read once for G heads.
 //
-// What bounds it is the chain of trips to memory that a wave makes for 64 keys (page, K, V), so the keys of a token can go to
-// gridDim.z workgroups in runs of whole chunks (each token's own keys cut alike), which leave their sums for
-// attn_grouped_merge_kernel. `grouped_plan` chooses heads, waves and runs.
+// What bounds it is the chain of trips to memory that a wave makes for 64 keys (page, K, V) and the lines that its loads touch, so
+// the keys of a token can go to gridDim.z workgroups in runs of whole chunks (each token's own keys cut alike), which leave their
+// sums for attn_grouped_merge_kernel. `grouped_plan` chooses heads, waves and runs. With a lane on 64 neighbouring bytes of K and on a dimension of V^T
+// every load touched 64 lines. us with the merge, K and V from memory, so / now: 12 heads of 128 on 2, 8 requests of 1,000
+// keys 13.2 / 10.9, 1 of 500 12.7 / 8.7, 32 of 200 9.6 / 7.3, 32 of 1,000 22.4 / 19.7; 12 of 64, 8 of 1,000 19.7 / 15.4; 8 of 256 on
+// 4, 1 of 400 19.0 / 12.7; against 64 bits 2.3e-7 / 2.0e-7.
 constexpr bool GQ_FITS = D % 32 == 0;
-constexpr int GQ_SLICE = GQ_FITS ? D / 8 : 4;
+constexpr int GQ_SLICE = GQ_FITS ? D / 8 : 4;             // a lane's columns of K
+constexpr int GQ_DIMS = GQ_FITS ? D / 16 : 1;              // a lane's dimensions of V: lane / 4, 16 more, ...
 static bool grouped_fits(int64_t tokens, int heads) { return GQ_FITS && tokens * heads < 2048; }
 
+// (the second bound keeps as many waves a SIMD as there were with fewer sums a lane)
 template <int G, int WAVES>
-__global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
+__global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 ? 2 : 1)) void attn_grouped_f32_kernel(
     const float* __restrict__ qkv, int64_t q_stride, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_request,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ table_rows,
@@ -265,34 +270,41 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
   const int q_pos = positions[t];
   const int request_of_token = token_request[t];
   const int32_t* table = block_table + static_cast<int64_t>(table_rows != nullptr ? table_rows[request_of_token] : request_of_token) * table_width;
-  const int sub = lane % 8;                                // which eighth of a row
+  const int sub = lane % 8;                                // which 16 bytes of a line
   const int key_in_pass = lane / 8;
   float q_r[G][GQ_SLICE];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    const float* q = qkv + t * q_stride + static_cast<int64_t>(h0 + min(g, n - 1)) * D + sub * GQ_SLICE;
+    const float* q = qkv + t * q_stride + static_cast<int64_t>(h0 + min(g, n - 1)) * D + 4 * sub;
 #pragma unroll
     for (int d = 0; d < GQ_SLICE; d += 4) {
-      const float4 v = *reinterpret_cast<const float4*>(q + d);
+      const float4 v = *reinterpret_cast<const float4*>(q + 8 * d);
       q_r[g][d] = v.x; q_r[g][d + 1] = v.y; q_r[g][d + 2] = v.z; q_r[g][d + 3] = v.w;
     }
   }
   const int first = first_visible(q_pos, window);
   const int last = q_pos;   // inclusive
   float m[G], l[G];
-  float acc[G][DIMS_PER_LANE];
+  float acc[G][GQ_DIMS];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     m[g] = -INFINITY;
     l[g] = 0.f;
 #pragma unroll
-    for (int i = 0; i < DIMS_PER_LANE; ++i) acc[g][i] = 0.f;
+    for (int i = 0; i < GQ_DIMS; ++i) acc[g][i] = 0.f;
   }
 
   const int chunk0 = first / DISTIE_WAVE, chunks = last / DISTIE_WAVE - chunk0 + 1;
   const int per_run = runs == 1 ? chunks : (chunks + runs - 1) / runs;
   const int run0 = static_cast<int>(blockIdx.z) * per_run;
   const int run_end = min(chunks, run0 + per_run);          // (a run may hold no chunk)
+  // What is under way together is what the registers hold without a workgroup less on a compute unit. Heads of up to 128 (and
+  // beyond 64, where four waves a SIMD hide more than loads ahead do): all of a chunk's keys and, in their place as they are used up, its
+  // values; with three or four query heads half of the keys and of the values at a time.
+  constexpr bool AHEAD = D > 64 && D <= 128;
+  constexpr int ROUND = G == 1 || (AHEAD && G == 2) ? 8 : 4, V_EARLY = !AHEAD ? 0 : G <= 2 ? 2 : 1;
+  constexpr int V_LOADS = G <= (AHEAD ? 2 : 1) ? 16 : 8;       // about, in whole quarters of the chunk
+  constexpr int V_QUARTERS = V_LOADS >= 4 * GQ_DIMS ? 4 : V_LOADS >= 2 * GQ_DIMS ? 2 : 1, V_BATCHES = 4 / V_QUARTERS;
   for (int c = (chunk0 + run0 + wave) * DISTIE_WAVE; c < (chunk0 + run_end) * DISTIE_WAVE; c += DISTIE_WAVE * WAVES) {
     // Every load of a phase is issued before its results are used (a chunk costs a few trips to memory, not one
     // for every pass and page): lane j looks up the page of key c + j, the addresses go from lane to lane.
@@ -304,48 +316,71 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
       base = (static_cast<int64_t>(page) * kv_heads + kh) * block_size * D;
       row = base + static_cast<int64_t>(key % block_size) * D;
     }
-    // ---- scores: eight keys a pass, four passes of loads in flight; afterwards lane j holds the scores of key c + j
+    base_s[wave][lane] = base;
+    __builtin_amdgcn_wave_barrier();
+    // V^T's loads, sixteen keys a quarter (a lane's four lie in one page: pages hold a multiple of four tokens). No condition
+    // stands around a load.
+    const int lo = max(first - c, 0);                                   // keys lo .. hi of the chunk count
+    const int hi = min(DISTIE_WAVE - 1, last - c);
+    const int piece = lane % 4, dim0 = lane / 4;
+    float4 vv[4][GQ_DIMS];
+    const auto ask_values = [&](int batch) {
+#pragma unroll
+      for (int u = 0; u < V_QUARTERS; ++u) {
+        const int quarter = batch * V_QUARTERS + u, j = 16 * quarter + 4 * piece;
+        const int64_t page_base = base_s[wave][min(max(j, lo), hi)];      // of a key that counts
+        const float* v = v_cache + page_base + static_cast<int64_t>(dim0) * block_size + (c + j) % block_size;
+#pragma unroll
+        for (int i = 0; i < GQ_DIMS; ++i) vv[quarter][i] = *reinterpret_cast<const float4*>(v + 16 * i * block_size);
+      }
+    };
+    // ---- scores: eight keys a pass, ROUND passes of loads under way together; afterwards lane j holds the scores of key c + j.
+    // The first values are asked for behind the last keys, the next ones as each half of those is used up.
     float s[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) s[g] = 0.f;
-    constexpr int ROUND = G == 1 ? 8 : 4;                 // passes whose loads are in flight together: what the registers allow
+    float4 kk[8][GQ_SLICE / 4];
+    const auto ask_keys = [&](int pass) {
+      const int64_t from = __shfl(row, 8 * pass + key_in_pass, DISTIE_WAVE);
+      const float* k = k_cache + from + 4 * sub;
+#pragma unroll
+      for (int d = 0; d < GQ_SLICE / 4; ++d) kk[pass][d] = *reinterpret_cast<const float4*>(k + 32 * d);
+    };
+    const auto use_keys = [&](int pass) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        float v = 0.f;
+#pragma unroll
+        for (int d = 0; d < GQ_SLICE / 4; ++d) {
+          v = fmaf(q_r[g][4 * d], kk[pass][d].x, v);
+          v = fmaf(q_r[g][4 * d + 1], kk[pass][d].y, v);
+          v = fmaf(q_r[g][4 * d + 2], kk[pass][d].z, v);
+          v = fmaf(q_r[g][4 * d + 3], kk[pass][d].w, v);
+        }
+        v = lanes_sum<4>(lanes_sum<2>(lanes_sum<1>(v)));
+        if (sub == pass) s[g] = v;                          // lane 8 k + p holds the score of key 8 p + k
+      }
+    };
 #pragma unroll
     for (int round = 0; round < 8 / ROUND; ++round) {
-      float4 kk[ROUND][GQ_SLICE / 4];
 #pragma unroll
-      for (int ps = 0; ps < ROUND; ++ps) {
-        const int64_t from = __shfl(row, 8 * (ROUND * round + ps) + key_in_pass, DISTIE_WAVE);
-        const float* k = k_cache + from + sub * GQ_SLICE;
-#pragma unroll
-        for (int d = 0; d < GQ_SLICE / 4; ++d) kk[ps][d] = *reinterpret_cast<const float4*>(k + 4 * d);
-      }
+      for (int ps = 0; ps < ROUND; ++ps) ask_keys(ROUND * round + ps);
       __builtin_amdgcn_sched_barrier(0);                    // all of these loads are under way before the first is used
 #pragma unroll
       for (int ps = 0; ps < ROUND; ++ps) {
-        const int pass = ROUND * round + ps;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          float v = 0.f;
-#pragma unroll
-          for (int d = 0; d < GQ_SLICE / 4; ++d) {
-            v = fmaf(q_r[g][4 * d], kk[ps][d].x, v);
-            v = fmaf(q_r[g][4 * d + 1], kk[ps][d].y, v);
-            v = fmaf(q_r[g][4 * d + 2], kk[ps][d].z, v);
-            v = fmaf(q_r[g][4 * d + 3], kk[ps][d].w, v);
-          }
-          v += __shfl_xor(v, 1, DISTIE_WAVE);
-          v += __shfl_xor(v, 2, DISTIE_WAVE);
-          v += __shfl_xor(v, 4, DISTIE_WAVE);
-          // the lane that owns this key for the softmax is lane 8 pass + (the key's place in the pass)
-          const float mine = __shfl(v, (lane % 8) * 8, DISTIE_WAVE);
-          if (lane / 8 == pass) s[g] = mine;
+        use_keys(ROUND * round + ps);
+        const int half = (ps + 1) / (ROUND / 2) - 1;
+        if (round == 8 / ROUND - 1 && (ps + 1) % (ROUND / 2) == 0 && half < V_EARLY) {
+          __builtin_amdgcn_sched_barrier(0);
+          ask_values(half);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
     float alpha[G];
-    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int g = 0; g < G; ++g) {
+      s[g] = __shfl(s[g], sub * 8 + lane / 8, DISTIE_WAVE);
       const float sg = valid && g < n ? s[g] * scale : -INFINITY;
       const float m_new = fmaxf(m[g], wave_max(sg));
       alpha[g] = m_new == -INFINITY ? 0.f : expf(m[g] - m_new);     // 0 on the first chunk with a key (m = -inf)
@@ -354,50 +389,37 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
       m[g] = m_new;
       p_s[wave][g][lane] = p;
     }
-    base_s[wave][lane] = base;
     __builtin_amdgcn_wave_barrier();
-    // ---- output: the lane owns dimensions lane, lane + 64, ...; the chunk's values of a dimension are 16 pieces
-    // of four keys (a piece lies in one page: pages hold a multiple of four tokens)
-    const int lo = max(first - c, 0);                                   // keys lo .. hi of the chunk count
-    const int hi = min(DISTIE_WAVE - 1, last - c);
+    // ---- output
 #pragma unroll
-    for (int i = 0; i < DIMS_PER_LANE; ++i) {
-      const int d = lane + i * DISTIE_WAVE;
-      if (d >= D) continue;
-      float a[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) a[g] = acc[g][i] * alpha[g];
-      constexpr int GQ_PIECES = G == 1 ? 16 : 8;            // 16-byte pieces of V^T whose loads are in flight together
-#pragma unroll
-      for (int part = 0; part < 16 / GQ_PIECES; ++part) {
-        float4 vv[GQ_PIECES];
-#pragma unroll
-        for (int u = 0; u < GQ_PIECES; ++u) {
-          const int q = part * GQ_PIECES + u;
-          const int64_t page_base = base_s[wave][min(max(4 * q, lo), hi)];      // of a key that counts
-          vv[u] = *reinterpret_cast<const float4*>(v_cache + page_base + static_cast<int64_t>(d) * block_size +
-                                                   (c + 4 * q) % block_size);
-        }
+    for (int batch = 0; batch < V_BATCHES; ++batch) {
+      if (batch >= V_EARLY) {
+        __builtin_amdgcn_sched_barrier(0);
+        ask_values(batch);
         __builtin_amdgcn_sched_barrier(0);                  // all of these loads are under way before the first is used
+      }
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
+      for (int g = 0; g < G; ++g) {
+        if (batch == 0) {
 #pragma unroll
-          for (int u = 0; u < GQ_PIECES; ++u) {
-            const int q = part * GQ_PIECES + u;
-            const float4 pp = *reinterpret_cast<const float4*>(&p_s[wave][g][4 * q]);
-            const float v[4] = {vv[u].x, vv[u].y, vv[u].z, vv[u].w};
-            const float w[4] = {pp.x, pp.y, pp.z, pp.w};
+          for (int i = 0; i < GQ_DIMS; ++i) acc[g][i] *= alpha[g];
+        }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int j = 4 * q + e;
-              // never a value of a key that does not count (a weight of zero times what lies there could be NaN)
-              a[g] = fmaf(w[e], (j >= lo && j <= hi) ? v[e] : 0.f, a[g]);
-            }
+        for (int u = 0; u < V_QUARTERS; ++u) {
+          const int quarter = batch * V_QUARTERS + u, j = 16 * quarter + 4 * piece;
+          const float4 p = *reinterpret_cast<const float4*>(&p_s[wave][g][j]);
+          // never a value of a key that does not count (a weight of zero times what lies there could be NaN)
+          const bool in[4] = {j >= lo && j <= hi, j + 1 >= lo && j + 1 <= hi, j + 2 >= lo && j + 2 <= hi, j + 3 >= lo && j + 3 <= hi};
+#pragma unroll
+          for (int i = 0; i < GQ_DIMS; ++i) {
+            const float4 v = vv[quarter][i];
+            acc[g][i] = fmaf(p.x, in[0] ? v.x : 0.f, acc[g][i]);
+            acc[g][i] = fmaf(p.y, in[1] ? v.y : 0.f, acc[g][i]);
+            acc[g][i] = fmaf(p.z, in[2] ? v.z : 0.f, acc[g][i]);
+            acc[g][i] = fmaf(p.w, in[3] ? v.w : 0.f, acc[g][i]);
           }
         }
       }
-#pragma unroll
-      for (int g = 0; g < G; ++g) acc[g][i] = a[g];
     }
   }
   // ---- the waves' parts, put together by wave 0 in wave order
@@ -411,9 +433,9 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_grouped_f32_kernel(
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int i = 0; i < DIMS_PER_LANE; ++i) {
-      const int d = lane + i * DISTIE_WAVE;
-      if (d < D) acc_s[wave][g][d] = acc[g][i];
+    for (int i = 0; i < GQ_DIMS; ++i) {
+      const float sum = lanes_sum<2>(lanes_sum<1>(acc[g][i]));
+      if (lane % 4 == 0) acc_s[wave][g][lane / 4 + 16 * i] = sum;
     }
   __syncthreads();
   // wave w writes heads w, w + WAVES, ... of the part
