@@ -98,10 +98,11 @@ __device__ __forceinline__ float sum_strided(const T* p, int slices, int64_t str
     const float b = to_float(p[min(s + 1, last) * stride]);
     const float c = to_float(p[min(s + 2, last) * stride]);
     const float d = to_float(p[min(s + 3, last) * stride]);
+    __builtin_amdgcn_sched_barrier(0);          // (selects below: where a sum stands under a condition, its load is put there too)
     sum += a;
-    if (s + 1 <= last) sum += b;
-    if (s + 2 <= last) sum += c;
-    if (s + 3 <= last) sum += d;
+    sum = s + 1 <= last ? sum + b : sum;
+    sum = s + 2 <= last ? sum + c : sum;
+    sum = s + 3 <= last ? sum + d : sum;
   }
   return sum;
 }

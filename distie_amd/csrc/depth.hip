@@ -13,12 +13,14 @@ namespace {
 // SHIFT, for steps of one row a request: out is [mixes, T, C] instead, out[m] = h + (before - h) * mu[m] with h = x in out's
 // precision and `before` the request's row of `state` (float32 [slots, C], row state_slots[row]), which h replaces.
 // delta may be partial sums (slices that lie `stride` elements apart, added in order). A thread keeps Q runs of V columns
-// in registers; everything it reads is asked for before the first barrier. The sums of squares of the runs wait in LDS, a
+// in registers; everything it reads is asked for before the first barrier, residual, first layer and weight in front of the
+// partial sums. What bounds prompts is the layers' bytes (eight waves a SIMD, which 64 registers allow): 1,789 rows of 2,048, 16 layers, us a
+// layer on average 38.0 -> 36.2, without a residual 11.6 -> 10.7. The sums of squares of the runs wait in LDS, a
 // wave adds up those of a group in an order that only the sizes decide.
 constexpr int SHIFT_MIXES = 8;
 
 template <int V, int Q, bool SHIFT, typename A, typename O>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, (V == 4 && Q == 1 && !SHIFT ? 8 : 4))
 group_chain_kernel(const A* __restrict__ delta, int slices, int64_t stride, const float* __restrict__ weight, float eps,
                    int groups, const float* residual_in, float* residual_out, const float* __restrict__ first, float* rest,
                    int index, const float* __restrict__ weights, O* __restrict__ out, int C, int64_t layer_stride,
@@ -29,7 +31,7 @@ group_chain_kernel(const A* __restrict__ delta, int slices, int64_t stride, cons
   float* squares = lds;                       // [runs]
   float* scale = lds + runs;                  // [groups]
   const int64_t base = static_cast<int64_t>(blockIdx.x) * C;
-  float y[Q][V], x[Q][V], sum[Q][V];
+  float y[Q][V], x[Q][V], sum[Q][V], own_weight[Q][V];
   float before[SHIFT ? Q : 1][V], own_mu[SHIFT && Q == 1 ? SHIFT_MIXES : 1][V];
   float* own = nullptr;
   if constexpr (SHIFT) {
@@ -54,8 +56,10 @@ group_chain_kernel(const A* __restrict__ delta, int slices, int64_t stride, cons
     for (int k = 0; k < V; ++k) y[q][k] = 0.f, x[q][k] = 0.f, sum[q][k] = 0.f;
     if (run >= runs) continue;
     const int64_t at = base + static_cast<int64_t>(run) * V;
-    sum_values<V>(delta + at, slices, stride, y[q]);
+    load_values<V>(weight + static_cast<int64_t>(run) * V, own_weight[q]);
     if (residual_in != nullptr) load_values<V>(residual_in + at, x[q]);
+    if (weights != nullptr) load_values<V>(first + at, sum[q]);
+    sum_values<V>(delta + at, slices, stride, y[q]);
   }
   if (weights != nullptr) {
     const float w0 = weights[0];
@@ -64,21 +68,18 @@ group_chain_kernel(const A* __restrict__ delta, int slices, int64_t stride, cons
       const int run = threadIdx.x + q * blockDim.x;
       if (run >= runs) continue;
       const int64_t at = base + static_cast<int64_t>(run) * V;
-      float v[V];
-      load_values<V>(first + at, v);
 #pragma unroll
-      for (int k = 0; k < V; ++k) sum[q][k] = w0 * v[k];
+      for (int k = 0; k < V; ++k) sum[q][k] *= w0;
       for (int j = 0; j < index; j += 8) {
         float a[8][V];
 #pragma unroll
         for (int u = 0; u < 8; ++u) load_values<V>(rest + min(j + u, index - 1) * layer_stride + at, a[u]);
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (j + u < index) {
-            const float w = weights[j + u + 1];
+        for (int u = 0; u < 8; ++u) {
+          const float w = weights[min(j + u + 1, index)];          // (index + 2 weights)
 #pragma unroll
-            for (int k = 0; k < V; ++k) sum[q][k] += w * a[u][k];
-          }
+          for (int k = 0; k < V; ++k) sum[q][k] = j + u < index ? sum[q][k] + w * a[u][k] : sum[q][k];
+        }
       }
     }
   }
@@ -107,10 +108,8 @@ group_chain_kernel(const A* __restrict__ delta, int slices, int64_t stride, cons
     if (run >= runs) continue;
     const int64_t at = base + static_cast<int64_t>(run) * V;
     const float r = scale[run / per_group];
-    float w[V];
-    load_values<V>(weight + static_cast<int64_t>(run) * V, w);
 #pragma unroll
-    for (int k = 0; k < V; ++k) x[q][k] += y[q][k] * r * w[k];
+    for (int k = 0; k < V; ++k) x[q][k] += y[q][k] * r * own_weight[q][k];
     if (weights != nullptr) {
       store_values<V>(rest + index * layer_stride + at, x[q]);
 #pragma unroll

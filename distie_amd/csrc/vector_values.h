@@ -48,19 +48,46 @@ __device__ __forceinline__ void store_values(T* __restrict__ p, const float v[V]
   }
 }
 
-// the sum of `slices` vectors that lie `stride` elements apart, added in order; eight slices' loads under way together
+// N of them, of which the first `slices` count; the loads stand together, under no condition and in front of the first sum (where a value
+// was added under a condition, the compiler had put its load there too: a trip to memory of its own)
+template <int N, int V, typename T>
+__device__ __forceinline__ void load_slices(const T* __restrict__ p, int slices, int64_t stride, float a[N][V]) {
+#pragma unroll
+  for (int u = 0; u < N; ++u) load_values<V>(p + min(u, slices - 1) * stride, a[u]);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// the sum of `slices` vectors that lie `stride` elements apart, added in order. Up to eight slices, which is what products are cut into, cost
+// one trip to memory together with what the caller has asked for before (a loop waits for that in front of its first round). Steps, us,
+// with three trips / one: 64 requests of 2,048 keys 2,360 / 2,339, 8 requests 1,352 / 1,344, a prompt of 301 2,372 / 2,343.
 template <int V, typename T>
 __device__ __forceinline__ void sum_values(const T* __restrict__ p, int slices, int64_t stride, float out[V]) {
-  load_values<V>(p, out);
-  for (int s = 1; s < slices; s += 8) {
+  if (slices == 1) {
+    load_values<V>(p, out);
+  } else if (slices <= 4) {
+    float a[4][V];
+    load_slices<4, V>(p, slices, stride, a);
+#pragma unroll
+    for (int k = 0; k < V; ++k) out[k] = a[0][k];
+#pragma unroll
+    for (int u = 1; u < 4; ++u)
+#pragma unroll
+      for (int k = 0; k < V; ++k) out[k] = u < slices ? out[k] + a[u][k] : out[k];
+  } else {
     float a[8][V];
+    load_slices<8, V>(p, slices, stride, a);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) load_values<V>(p + min(s + u, slices - 1) * stride, a[u]);
+    for (int k = 0; k < V; ++k) out[k] = a[0][k];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (s + u < slices) {
+    for (int u = 1; u < 8; ++u)
 #pragma unroll
-        for (int k = 0; k < V; ++k) out[k] += a[u][k];
-      }
+      for (int k = 0; k < V; ++k) out[k] = u < slices ? out[k] + a[u][k] : out[k];
+    for (int s = 8; s < slices; s += 8) {
+      load_slices<8, V>(p + s * stride, slices - s, stride, a);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int k = 0; k < V; ++k) out[k] = s + u < slices ? out[k] + a[u][k] : out[k];
+    }
   }
 }
