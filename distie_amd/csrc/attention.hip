@@ -1348,8 +1348,10 @@ __global__ __launch_bounds__(DISTIE_WAVE * W, (MB == 1 && D <= 128 ? 2 : 1)) voi
 }
 
 // Combines the partial results of the runs of keys of one (request, head): grid (heads, requests), four waves.
-// All threads first find the maximum and the weight of every run; then each wave adds a quarter of the runs
-// (in order) for the output dims its lanes own, and the four sums are added in order through LDS.
+// The maximum and the weight of every run are found first; then each wave adds a quarter of the runs (in order) for the output
+// dims its lanes own, and the four sums are added in order through LDS. What bounds it is its chain: with weights through LDS
+// (three barriers, a branch and a read of LDS a run) steps took, us, so / now: one request of 500 keys 1,076 / 1,049, 8 of 2,048 1,344 / 1,315,
+// 64 of 2,048 2,339 / 2,318, 4 of 16,000 1,571 / 1,523.
 // FAST (at most RD_FAST_RUNS runs fit the buffers): every partial result the block may need is asked for at
 // once, before the request's length says which runs exist (their places are inside the buffers either way,
 // and what a run that does not exist left there is dropped by a select, never multiplied): one trip to
@@ -1359,6 +1361,7 @@ constexpr int RD_THREADS = RD_WAVES * DISTIE_WAVE;
 constexpr int RD_MAX_RUNS = 1024;
 constexpr int RD_FAST_PER_WAVE = 16;
 constexpr int RD_FAST_RUNS = RD_FAST_PER_WAVE * RD_WAVES;
+static_assert(RD_FAST_RUNS == DISTIE_WAVE, "a lane a run");
 
 template <bool FAST>
 __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
@@ -1366,7 +1369,7 @@ __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
     const int32_t* __restrict__ cu_q, bf16_t* __restrict__ out, int heads, int window, int all_splits, int together,
     int dense_rows, const int32_t* __restrict__ shared_run_len, const float* __restrict__ sinks) {
   const int max_splits = (all_splits + together - 1) / together;      // places: the runs of a workgroup share one
-  __shared__ float weight_s[FAST ? RD_FAST_RUNS : RD_MAX_RUNS];
+  __shared__ float weight_s[FAST ? 1 : RD_MAX_RUNS];
   __shared__ float sum_s[RD_WAVES][D];
   __shared__ float scratch[32];
   const int tid = threadIdx.x;
@@ -1376,25 +1379,25 @@ __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
   const int head = blockIdx.x;
   const int64_t base0 = (static_cast<int64_t>(request) * heads + head) * max_splits;
 
+  const int length = kv_len[request];
+  const int run_len = shared_run_len != nullptr ? *shared_run_len : 0;
   float early[FAST ? RD_FAST_PER_WAVE : 1][DIMS_PER_LANE];
   float2 early_ml = {0.f, 0.f};
   if constexpr (FAST) {
+    early_ml = *reinterpret_cast<const float2*>(part_ml + 2 * (base0 + min(lane, max_splits - 1)));
 #pragma unroll
     for (int u = 0; u < RD_FAST_PER_WAVE; ++u) {
       const int j = min(wave + RD_WAVES * u, max_splits - 1);
 #pragma unroll
-      for (int i = 0; i < DIMS_PER_LANE; ++i) {
-        const int d = lane + i * DISTIE_WAVE;
-        early[u][i] = d < D ? part_o[(base0 + j) * D + d] : 0.f;
-      }
+      for (int i = 0; i < DIMS_PER_LANE; ++i) early[u][i] = part_o[(base0 + j) * D + min(lane + i * DISTIE_WAVE, D - 1)];
     }
-    early_ml = *reinterpret_cast<const float2*>(part_ml + 2 * (base0 + min(tid, max_splits - 1)));
+    asm volatile("" ::"s"(length), "s"(run_len));           // (asked for here, not behind the branch below)
   }
 
   const int token = dense_rows ? request : cu_q[request];
   if (!dense_rows && cu_q[request + 1] - token != 1) return;
-  const int q_pos = kv_len[request] - 1;
-  const int all_runs = key_runs(q_pos, window, all_splits, shared_run_len != nullptr ? *shared_run_len : 0).count;
+  const int q_pos = length - 1;
+  const int all_runs = key_runs(q_pos, window, all_splits, run_len).count;
   const int runs = (all_runs + together - 1) / together;     // the first `runs` places hold results
   const int64_t base = base0;
   bf16_t* o = out + (static_cast<int64_t>(token) * heads + head) * D;
@@ -1402,28 +1405,25 @@ __global__ __launch_bounds__(RD_THREADS) void attn_reduce_kernel(
   const float sink = sinks != nullptr ? sinks[head] * 1.4426950408889634f : -INFINITY;
 
   if constexpr (FAST) {
-    const bool mine = tid < runs;
-    float m = mine ? early_ml.x : -INFINITY;
-    m = wave_max(m);
-    if (lane == 0) scratch[wave] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(fmaxf(scratch[0], scratch[1]), fmaxf(scratch[2], scratch[3])), sink);
+    // Every wave has all runs' maxima and sums in its lanes (RD_FAST_RUNS is a wave), and takes its own runs' weights from there: no
+    // barrier and no trip to LDS but the one that puts the waves together.
+    const bool mine = lane < runs;
+    const float m = fmaxf(wave_max(mine ? early_ml.x : -INFINITY), sink);
     const float w = mine ? fast_exp2(early_ml.x - m) : 0.f;
-    if (tid < RD_FAST_RUNS) weight_s[tid] = w;
-    const float l = block_sum(mine ? w * early_ml.y : 0.f, scratch + 16) +     // has the barrier that publishes the weights
-                    (sink == -INFINITY ? 0.f : fast_exp2(sink - m));
+    const float l = wave_sum(mine ? w * early_ml.y : 0.f) + (sink == -INFINITY ? 0.f : fast_exp2(sink - m));
+    const int own = __builtin_amdgcn_readfirstlane(wave);
+    float a[DIMS_PER_LANE] = {};
+#pragma unroll
+    for (int u = 0; u < RD_FAST_PER_WAVE; ++u) {
+      const int j = own + RD_WAVES * u;
+      const float weight = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), j));
+#pragma unroll
+      for (int i = 0; i < DIMS_PER_LANE; ++i) a[i] = j < runs ? fmaf(weight, early[u][i], a[i]) : a[i];
+    }
 #pragma unroll
     for (int i = 0; i < DIMS_PER_LANE; ++i) {
       const int d = lane + i * DISTIE_WAVE;
-      if (d >= D) continue;
-      float a = 0.f;
-#pragma unroll
-      for (int u = 0; u < RD_FAST_PER_WAVE; ++u) {
-        const int j = wave + RD_WAVES * u;
-        const bool exists = j < runs;
-        a = exists ? fmaf(weight_s[j], early[u][i], a) : a;
-      }
-      sum_s[wave][d] = a;
+      if (d < D) sum_s[wave][d] = a[i];
     }
     __syncthreads();
     if (wave != 0) return;

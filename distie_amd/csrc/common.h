@@ -74,15 +74,20 @@ __device__ __forceinline__ float wave_max(float v) {
 // Sum over a block of up to 1024 threads; `scratch` holds one float per wave (16).
 // The order of the additions depends only on the block size, never on the data's place in a batch.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
+  const int waves = (blockDim.x + DISTIE_WAVE - 1) / DISTIE_WAVE;
   v = wave_sum(v);
   const int wave = threadIdx.x / DISTIE_WAVE;
   const int lane = threadIdx.x % DISTIE_WAVE;
-  const int waves = (blockDim.x + DISTIE_WAVE - 1) / DISTIE_WAVE;
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  float total = 0.f;
-  for (int w = 0; w < waves; ++w) total += scratch[w];
+  // all sixteen places are read together, and those that no wave wrote are dropped (a loop over the waves waited for each)
+  float part[16];
+#pragma unroll
+  for (int w = 0; w < 16; ++w) part[w] = scratch[w];
+  float total = part[0];
+#pragma unroll
+  for (int w = 1; w < 16; ++w) total = w < waves ? total + part[w] : total;
   return total;
 }
 
