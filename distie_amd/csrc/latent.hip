@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "vector_values.h"
 
 namespace {
 
@@ -26,8 +27,15 @@ __device__ __forceinline__ float sigmoidf(float x) { return 1.f / (1.f + __expf(
 // was zero when the cache was made and is never written.
 // `down` may be `slices` partial sums of the product, `slice_stride` elements apart (added in order while the row is
 // read into LDS, where both norms and the rotation find it).
+//
+// What bounds a step of few tokens are trips to memory one after the other, so all that the kernel reads is asked for at the start, the row
+// in rounds of LN_AHEAD values a thread: 16 tokens, 768 + 192 + 64
+// columns in four slices, us, one trip a value and weight / now: 7.6 / 5.3; 1,787 tokens 11.5 / 9.9.
+constexpr int LN_AHEAD = 4;
+
 template <typename O, typename C>
-__global__ void latent_norm_rope_write_kernel(const float* __restrict__ down, int slices, int64_t slice_stride, int64_t ld,
+__global__ void __launch_bounds__(256)
+latent_norm_rope_write_kernel(const float* __restrict__ down, int slices, int64_t slice_stride, int64_t ld,
                                               int q_rank, const float* __restrict__ q_weight, int kv_rank,
                                               const float* __restrict__ kv_weight, float eps, int rot_dim,
                                               const float2* __restrict__ table, float magnitude, int neighbours,
@@ -37,14 +45,51 @@ __global__ void latent_norm_rope_write_kernel(const float* __restrict__ down, in
   __shared__ float scratch[16];
   const int64_t t = blockIdx.x;
   const int width = q_rank + kv_rank + rot_dim;
-  for (int c = threadIdx.x; c < width; c += blockDim.x) row[c] = sum_strided(down + t * ld + c, slices, slice_stride);
+  const int pairs = rot_dim / 2, tid = threadIdx.x, threads = blockDim.x;
+  float q_w[LN_AHEAD] = {}, kv_w[LN_AHEAD] = {};
+  float2 angle = {1.f, 0.f};
+  int slot = 0;
+  if (q_rank > 0) {
+#pragma unroll
+    for (int u = 0; u < LN_AHEAD; ++u) q_w[u] = q_weight[min(tid + u * threads, q_rank - 1)];
+  }
+  if (write) {
+    slot = slots[t];
+#pragma unroll
+    for (int u = 0; u < LN_AHEAD; ++u) kv_w[u] = kv_weight[min(tid + u * threads, kv_rank - 1)];
+    if (table != nullptr && pairs > 0) angle = table[t * pairs + min(tid, pairs - 1)];
+  }
+  for (int c0 = 0; c0 < width; c0 += LN_AHEAD * threads) {
+    const float* from = down + t * ld;
+    float part[4][LN_AHEAD];
+#pragma unroll
+    for (int u = 0; u < LN_AHEAD; ++u)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) part[s][u] = from[min(s, slices - 1) * slice_stride + min(c0 + tid + u * threads, width - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < LN_AHEAD; ++u) {
+      const int c = c0 + tid + u * threads;
+      float sum = part[0][u];
+#pragma unroll
+      for (int s = 1; s < 4; ++s) sum = s < slices ? sum + part[s][u] : sum;
+      if (c >= width) continue;
+      for (int s = 4; s < slices; ++s) sum += from[s * slice_stride + c];
+      row[c] = sum;
+    }
+  }
   __syncthreads();
   if (q_rank > 0) {
     float sq = 0.f;
     for (int c = threadIdx.x; c < q_rank; c += blockDim.x) sq += row[c] * row[c];
     sq = block_sum(sq, scratch);
     const float scale = 1.f / sqrtf(sq / q_rank + eps);
-    for (int c = threadIdx.x; c < q_rank; c += blockDim.x)
+#pragma unroll
+    for (int u = 0; u < LN_AHEAD; ++u) {
+      const int c = tid + u * threads;
+      if (c < q_rank) latent[t * q_rank + c] = from_float<O>(row[c] * scale * q_w[u]);
+    }
+    for (int c = tid + LN_AHEAD * threads; c < q_rank; c += threads)
       latent[t * q_rank + c] = from_float<O>(row[c] * scale * q_weight[c]);
   }
   if (!write) return;
@@ -53,23 +98,27 @@ __global__ void latent_norm_rope_write_kernel(const float* __restrict__ down, in
   for (int c = threadIdx.x; c < kv_rank; c += blockDim.x) sq += kv[c] * kv[c];
   sq = block_sum(sq, scratch);
   const float scale = 1.f / sqrtf(sq / kv_rank + eps);
-  const int slot = slots[t];
   const int64_t page = slot / P;
   const int off = slot % P;
   C* key = k_cache + (page * P + off) * DP;
   C* value = v_cache + page * DP * P + off;
-  for (int c = threadIdx.x; c < kv_rank; c += blockDim.x) {
-    const C v = from_float<C>(kv[c] * scale * kv_weight[c]);
+  const auto put = [&](int c, float w) {
+    const C v = from_float<C>(kv[c] * scale * w);
     key[c] = v;
     value[static_cast<int64_t>(c) * P] = v;
+  };
+#pragma unroll
+  for (int u = 0; u < LN_AHEAD; ++u) {
+    const int c = tid + u * threads;
+    if (c < kv_rank) put(c, kv_w[u]);
   }
+  for (int c = tid + LN_AHEAD * threads; c < kv_rank; c += threads) put(c, kv_weight[c]);
   const float* r = kv + kv_rank;
-  const int pairs = rot_dim / 2;
   for (int j = threadIdx.x; j < pairs; j += blockDim.x) {
     const int a = neighbours ? 2 * j : j, b = neighbours ? 2 * j + 1 : j + pairs;
     float cs = 1.f, sn = 0.f;
     if (table != nullptr) {
-      const float2 w = table[t * pairs + j];
+      const float2 w = j == tid ? angle : table[t * pairs + j];
       cs = w.x * magnitude, sn = w.y * magnitude;
     }
     const float u = r[a], v = r[b];
@@ -272,64 +321,68 @@ __device__ __forceinline__ float load_x(const void* x, int64_t at, int slices, i
   else return to_float(static_cast<const bf16_t*>(x)[at]);
 }
 
-template <int WT, int WN, int NB, bool SLICED>
+// The workgroup's rows of x, KC columns of them at a time, lie in LDS, summed and rounded once: read by each wave from memory, a load of
+// theirs touched 64 lines, and with four slices a workgroup made 256 of them for a tile, slice after slice. The weights of those columns are
+// asked for in front of that; KC is what the registers hold of them where waves are few (192), and where they are many what leaves room for
+// three or more of them a SIMD (64; 192 there: 20.3 us). A head's tail has a workgroup of its own behind the columns'. us a launch, so /
+// now, 16 heads: 16 rows in four slices, 128 columns times 192 rows with a tail 8.9 / 5.5; 16 rows, 192 times 128 6.4 / 5.8; 1,787 rows
+// 19.0 / 16.4.
+template <int WT, int WN, int NB, int KC, bool SLICED>
 __global__ void __launch_bounds__(64 * WT * WN)
 heads_linear_mfma_kernel(const void* __restrict__ x, int slices, int64_t slice_stride, int lx, const bf16_t* __restrict__ w,
                          bf16_t* __restrict__ out, int lo, int T, int H, int N, int K, QueryTail tail) {
+  constexpr int THREADS = 64 * WT * WN;
+  __shared__ __attribute__((aligned(16))) bf16_t x_s[WT * 32][KC + 8];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int h = blockIdx.z;
-  const int t0 = (blockIdx.y * WT + wave / WN) * 32;
-  const int n0 = (blockIdx.x * WN + wave % WN) * 32 * NB;
-  if (t0 < T && n0 < N) {
+  const int first = blockIdx.y * WT * 32;
+  const int rows = min(WT * 32, T - first);
+  if (tail.pairs == 0 || blockIdx.x != gridDim.x - 1) {
+    const int t0 = first + wave / WN * 32;
+    const int n0 = (blockIdx.x * WN + wave % WN) * 32 * NB;
     const int r = lane % 32, kk = 8 * (lane / 32);
-    const bool t_in = t0 + r < T;
-    const int64_t x_at = (static_cast<int64_t>(t_in ? t0 + r : t0) * H + h) * lx + kk;
+    // weight rows beyond N repeat the last, rows of x beyond T are whatever lies in LDS: what becomes of them is not stored
     const bf16_t* wr[NB];
-    bool n_in[NB];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      n_in[b] = n0 + 32 * b + r < N;
-      wr[b] = w + (static_cast<int64_t>(h) * N + (n_in[b] ? n0 + 32 * b + r : n0)) * K + kk;
-    }
+    for (int b = 0; b < NB; ++b) wr[b] = w + (static_cast<int64_t>(h) * N + min(n0 + 32 * b + r, N - 1)) * K;
     hl_floatx16 acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
-    for (int k0 = 0; k0 < K; k0 += 32) {
-      // two k-steps' loads under way together
-      hl_bf16x8 a[2], bw[2][NB];
+    for (int k0 = 0; k0 < K; k0 += KC) {
+      const int columns = min(KC, K - k0);
+      hl_bf16x8 bw[KC / 16][NB];
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int k = k0 + 16 * s;
-        const bool k_in = k + kk < K;
-        a[s] = hl_bf16x8{};
-        if (t_in && k_in) {
-          if constexpr (SLICED) {
-            const float* xf = static_cast<const float*>(x) + x_at + k;
-            float4 lo4 = *reinterpret_cast<const float4*>(xf), hi4 = *reinterpret_cast<const float4*>(xf + 4);
-            for (int q = 1; q < slices; ++q) {
-              const float4 l2 = *reinterpret_cast<const float4*>(xf + q * slice_stride);
-              const float4 h2 = *reinterpret_cast<const float4*>(xf + q * slice_stride + 4);
-              lo4.x += l2.x, lo4.y += l2.y, lo4.z += l2.z, lo4.w += l2.w;
-              hi4.x += h2.x, hi4.y += h2.y, hi4.z += h2.z, hi4.w += h2.w;
-            }
-            a[s][0] = static_cast<bf16_t>(lo4.x), a[s][1] = static_cast<bf16_t>(lo4.y);
-            a[s][2] = static_cast<bf16_t>(lo4.z), a[s][3] = static_cast<bf16_t>(lo4.w);
-            a[s][4] = static_cast<bf16_t>(hi4.x), a[s][5] = static_cast<bf16_t>(hi4.y);
-            a[s][6] = static_cast<bf16_t>(hi4.z), a[s][7] = static_cast<bf16_t>(hi4.w);
-          } else {
-            a[s] = *reinterpret_cast<const hl_bf16x8*>(static_cast<const bf16_t*>(x) + x_at + k);
-          }
+      for (int s = 0; s < KC / 16; ++s)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) bw[s][b] = *reinterpret_cast<const hl_bf16x8*>(wr[b] + min(k0 + 16 * s + kk, K - 8));
+      if (k0 > 0) __syncthreads();
+      const int pieces = columns / 8;                        // (K is a multiple of 8)
+      for (int i = threadIdx.x; i < rows * pieces; i += THREADS) {
+        const int row = i / pieces, c = 8 * (i % pieces);
+        const int64_t at = (static_cast<int64_t>(first + row) * H + h) * lx + k0 + c;
+        if constexpr (SLICED) {
+          float sum[8];
+          sum_values<8>(static_cast<const float*>(x) + at, slices, slice_stride, sum);
+          store_values<8>(&x_s[row][c], sum);
+        } else {
+          *reinterpret_cast<uint4*>(&x_s[row][c]) = *reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(x) + at);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < KC / 16; ++s) {
+        if (16 * s >= columns) break;
+        hl_bf16x8 a = *reinterpret_cast<const hl_bf16x8*>(&x_s[wave / WN * 32 + r][16 * s + kk]);
+        if (16 * s + kk >= columns) {
+          a = hl_bf16x8{};
+#pragma unroll
+          for (int b = 0; b < NB; ++b) bw[s][b] = hl_bf16x8{};
         }
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-          bw[s][b] = (n_in[b] && k_in) ? *reinterpret_cast<const hl_bf16x8*>(wr[b] + k) : hl_bf16x8{};
+        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bw[s][b], acc[b], 0, 0, 0);
       }
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], bw[s][b], acc[b], 0, 0, 0);
     }
     // acc[b][4 i + j]: row t0 + 8 i + 4 (lane / 32) + j of x, weight row n0 + 32 b + lane % 32
 #pragma unroll
@@ -344,11 +397,9 @@ heads_linear_mfma_kernel(const void* __restrict__ x, int slices, int64_t slice_s
           if (t < T) out[(static_cast<int64_t>(t) * H + h) * lo + n] = static_cast<bf16_t>(acc[b][4 * i + j]);
         }
     }
+    return;
   }
-  if (tail.pairs == 0 || blockIdx.x != 0) return;
   // the workgroup's rows of x, this head: the turned part behind the product's columns, zeros behind that
-  const int first = blockIdx.y * WT * 32;
-  const int rows = min(WT * 32, T - first);
   for (int i = threadIdx.x; i < rows * tail.pairs; i += blockDim.x) {
     const int t = first + i / tail.pairs, j = i % tail.pairs;
     const int a = tail.neighbours ? 2 * j : j, b = tail.neighbours ? 2 * j + 1 : j + tail.pairs;
@@ -459,14 +510,14 @@ static int heads_linear_mfma(const void* x, int slices, int lx, const void* w, v
   bf16_t* ob = static_cast<bf16_t*>(out);
   const int64_t stride = static_cast<int64_t>(T) * H * lx;
   if (T <= 32) {
-    const dim3 grid((N + 127) / 128, 1, H);
-    if (slices > 1) heads_linear_mfma_kernel<1, 4, 1, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
-    else heads_linear_mfma_kernel<1, 4, 1, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
+    const dim3 grid((N + 127) / 128 + (tail.pairs > 0 ? 1 : 0), 1, H);
+    if (slices > 1) heads_linear_mfma_kernel<1, 4, 1, 192, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
+    else heads_linear_mfma_kernel<1, 4, 1, 192, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
   } else {
-    const dim3 grid((N + 127) / 128, (T + 63) / 64, H);
+    const dim3 grid((N + 127) / 128 + (tail.pairs > 0 ? 1 : 0), (T + 63) / 64, H);
     if (grid.y > 65535) return DISTIE_BAD_ARGUMENT;
-    if (slices > 1) heads_linear_mfma_kernel<2, 2, 2, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
-    else heads_linear_mfma_kernel<2, 2, 2, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
+    if (slices > 1) heads_linear_mfma_kernel<2, 2, 2, 64, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
+    else heads_linear_mfma_kernel<2, 2, 2, 64, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
   }
   return launch_status();
 }
