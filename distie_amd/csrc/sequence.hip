@@ -1120,8 +1120,13 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
     const bool together = write && n == VGROUP && block_size % 8 == 0 && slot0 % block_size % 8 == 0 &&
                           slot0 % block_size + VGROUP <= block_size && __all(lane >= VGROUP || slot_of == slot0 + lane);
     uint16_t* cache = reinterpret_cast<uint16_t*>(v_cache);
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      const int c = (H + G) * D + g * E + e;
+    // whether some row of the sixteen is among its request's first ones
+    const bool early = __any(lane < VGROUP && row - first_of < TAPS - 1);
+    // A wave takes 64 channels at a time with all of its lanes, those beyond E the last channel again: the rows' requests lie in
+    // lanes 0 .. 15 of every wave, and a vote or a lane that is read counts only while it takes part. Only stores stand under `inside`.
+    for (int e0 = 64 * __builtin_amdgcn_readfirstlane(threadIdx.x / 64); e0 < E; e0 += blockDim.x) {
+      const bool inside = e0 + lane < E;
+      const int e = min(e0 + lane, E - 1), c = (H + G) * D + g * E + e;
       float w[TAPS], x[VGROUP], before[TAPS - 1];          // before[m]: row t0 - 1 - m
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) w[j] = to_float(weight[static_cast<int64_t>(c) * TAPS + j]);
@@ -1129,9 +1134,9 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       for (int k = 0; k < VGROUP; ++k) x[k] = to_float(product[static_cast<int64_t>(t0 + min(k, n - 1)) * ld + c]);
 #pragma unroll
       for (int m = 0; m < TAPS - 1; ++m) before[m] = to_float(product[static_cast<int64_t>(max(t0 - 1 - m, 0)) * ld + c]);
-      // some row of the sixteen is among its request's first ones: all rows' states, together
+      // all rows' states, together
       float held[VGROUP][TAPS - 1];
-      if (__any(lane < VGROUP && row - first_of < TAPS - 1)) {
+      if (early) {
 #pragma unroll
         for (int k = 0; k < VGROUP; ++k)
 #pragma unroll
@@ -1141,10 +1146,10 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       uint32_t bits[VGROUP];
 #pragma unroll
       for (int k = 0; k < VGROUP; ++k) {
-        const int first = __builtin_amdgcn_readlane(first_of, k);
+        const int first = __builtin_amdgcn_readlane(first_of, k), next = __builtin_amdgcn_readlane(next_of, k);
         const int i = t0 + min(k, n - 1) - first;
         float* own = state + static_cast<int64_t>(__builtin_amdgcn_readlane(state_of, k)) * (TAPS - 1) * N + c;
-        const bool single = k < n && __builtin_amdgcn_readlane(next_of, k) - first == 1;
+        const bool single = inside && k < n && next - first == 1;
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < TAPS; ++j) {
@@ -1160,16 +1165,18 @@ conv_head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int
       if (!write) continue;
       if (together) {
         uint16_t* dst = cache + ((static_cast<int64_t>(slot0 / block_size) * G + g) * DP + e) * block_size + slot0 % block_size;
-        *reinterpret_cast<uint4*>(dst) = uint4{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16),
-                                               bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16)};
-        *reinterpret_cast<uint4*>(dst + 8) = uint4{bits[8] | (bits[9] << 16), bits[10] | (bits[11] << 16),
-                                                   bits[12] | (bits[13] << 16), bits[14] | (bits[15] << 16)};
+        if (inside) {
+          *reinterpret_cast<uint4*>(dst) = uint4{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16),
+                                                 bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16)};
+          *reinterpret_cast<uint4*>(dst + 8) = uint4{bits[8] | (bits[9] << 16), bits[10] | (bits[11] << 16),
+                                                     bits[12] | (bits[13] << 16), bits[14] | (bits[15] << 16)};
+        }
       } else {
 #pragma unroll
         for (int k = 0; k < VGROUP; ++k) {
           if (k >= n) break;
           const int64_t slot = __builtin_amdgcn_readlane(slot_of, k);
-          cache[((slot / block_size * G + g) * DP + e) * block_size + slot % block_size] = static_cast<uint16_t>(bits[k]);
+          if (inside) cache[((slot / block_size * G + g) * DP + e) * block_size + slot % block_size] = static_cast<uint16_t>(bits[k]);
         }
       }
     }
