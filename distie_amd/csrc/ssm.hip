@@ -187,18 +187,18 @@ __device__ __forceinline__ void chunk_pairs(const X* __restrict__ xbc, int64_t l
   for (int v = 0; v < 16; ++v) to[(ib + tile_row(v, lane)) * SSM_L + jb + lane % 32] = acc[v];
 }
 
-// blockIdx = (chunk, head, 64 columns p): U and the chunk's total decay; (chunk, H + group, 0): the group's pairs. apart: chunks of
-// requests that bring one row are not worked on (`ssm_scan_kernel` takes those)
+// blockIdx = (chunk, head - first_head, 64 columns p): U and the chunk's total decay; head H + group, column 0: the group's pairs. apart:
+// chunks of requests that bring one row are not worked on (`ssm_scan_kernel` takes those)
 template <typename X>
 __global__ void __launch_bounds__(256)
 ssm_chunk_sums_kernel(const X* __restrict__ xbc, int64_t ld, const X* __restrict__ dt, int64_t ldd,
                       const float* __restrict__ dt_bias, const float* __restrict__ a_log, float* __restrict__ scratch,
                       float* __restrict__ totals, float* __restrict__ pairs, const int4* __restrict__ chunks, int H, int P, int N,
-                      int G, int apart) {
+                      int G, int apart, int first_head) {
   __shared__ float d_s[SSM_L], l_s[SSM_L];
   __shared__ float x_s[SSM_L][SSM_PAD];     // [row][p], times the row's factor
   __shared__ float b_s[SSM_L][SSM_PAD];     // [row][n of this pass]
-  const int chunk = blockIdx.x, head = blockIdx.y, p0 = blockIdx.z * 64;
+  const int chunk = blockIdx.x, head = first_head + blockIdx.y, p0 = blockIdx.z * 64;
   const int4 entry = chunks[chunk];
   const int first = entry.y, rows = entry.z;
   if (apart && entry.w) return;
@@ -486,7 +486,7 @@ extern "C" int distie_ssm_scan_chunked(const void* xbc, int dtype, int64_t ld, c
                                        const int32_t* first_chunk, const int32_t* cu_q, const int32_t* state_slots, int count, int B,
                                        int singles, int H, int P, int N, int G, hipStream_t stream) {
   if (B <= 0 || count <= 0) return 0;
-  if (H < 1 || P < 1 || N < 1 || G < 1 || H % G || H + G > 65535 || ldd < H || pairs == nullptr ||
+  if (H < 1 || P < 1 || N < 1 || G < 1 || H % G || H > 65535 || ldd < H || pairs == nullptr ||
       ld < static_cast<int64_t>(H) * P + 2 * static_cast<int64_t>(G) * N)
     return DISTIE_BAD_ARGUMENT;
   const int64_t size = static_cast<int64_t>(N) * P;
@@ -499,9 +499,11 @@ extern "C" int distie_ssm_scan_chunked(const void* xbc, int dtype, int64_t ld, c
     if (status != 0) return status;
   }
   DISTIE_DISPATCH(dtype, X, {
-    ssm_chunk_sums_kernel<X><<<dim3(count, H + G, columns), 256, 0, stream>>>(
-        static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd, dt_bias, a_log, scratch, totals, pairs, table, H, P, N, G,
-        apart);
+    // (heads and groups together may be more than a grid holds in y)
+    for (int at = 0; at < H + G; at += 65535)
+      ssm_chunk_sums_kernel<X><<<dim3(count, H + G - at < 65535 ? H + G - at : 65535, columns), 256, 0, stream>>>(
+          static_cast<const X*>(xbc), ld, static_cast<const X*>(dt), ldd, dt_bias, a_log, scratch, totals, pairs, table, H, P, N, G,
+          apart, at);
     ssm_chunk_states_kernel<<<dim3(B, H, parts), 256, 0, stream>>>(scratch, totals, state, first_chunk, table, state_slots, H, size,
                                                                    apart);
     ssm_chunk_outputs_kernel<X><<<dim3(count, H, columns), 256, 0, stream>>>(

@@ -88,3 +88,45 @@ def test_convolved_values_of_requests_that_begin_anywhere_in_a_group(ops, value_
                 off = (HALF * u.abs() + (taps + 16) * SINGLE * size[:, first:first + heads * D].view(T, heads, D)) * scale.abs()
                 assert ((got[..., :D].to(F) - u * scale).norm(dim=-1) <= off.norm(dim=-1)).all(), (begin, rest, heads)
                 assert not got[..., D:].any()
+
+
+def scanned(x, dt, dt_bias, a_log, skip, state, meta, H, P, N, G):
+    """-> (outputs, the sizes of what they are added up from, the state behind the step and its sizes, the largest exponent of a decay over a
+    chunk of 64 rows), in 64 bits"""
+    x, state, sizes, bend = x.to(F), state.to(F), state.to(F).abs(), 0.0
+    d = torch.nn.functional.softplus(dt.to(F) + dt_bias.to(F), threshold=80.0)
+    a = torch.exp(-torch.exp(a_log.to(F)) * d)
+    out, size = torch.empty(len(x), H, P, dtype=F, device="cuda"), torch.empty(len(x), H, P, dtype=F, device="cuda")
+    for b in range(meta.num_requests):
+        at = (5 * b + 2) % 31
+        s, most, first, end = state[at], sizes[at], *meta.host_cu_q[b:b + 2]
+        bend = max([bend] + [-a[t:min(t + 64, end)].log().sum(0).min().item() for t in range(first, end, 64)])
+        for t in range(first, end):
+            v = x[t, :H * P].view(H, 1, P)
+            B, C = (x[t, H * P + i * G * N:H * P + (i + 1) * G * N].view(G, N).repeat_interleave(H // G, 0)[:, :, None] for i in (0, 1))
+            s = a[t][:, None, None] * s + d[t][:, None, None] * B * v
+            most = a[t][:, None, None] * most + d[t][:, None, None] * (B * v).abs()
+            out[t] = (s * C).sum(1) + skip.to(F)[:, None] * v[:, 0]
+            size[t] = (most * C.abs()).sum(1) + (skip.to(F)[:, None] * v[:, 0]).abs()
+        state[at], sizes[at] = s, most
+    return out.view(len(x), H * P), size.view(len(x), H * P), state, sizes, bend
+
+
+def scan_case(ops, cuts, H, P, N, G, dtype):
+    """A result is off by a few roundings of each of its terms' products and of their sum over at most 64 rows and N state rows in eights, and
+    by those of the two sums of exponents of which a decay's is the difference."""
+    meta, _ = step(cuts)
+    T = meta.num_tokens
+    x, dt = rnd(T, H * P + 2 * G * N, seed=1).to(dtype), rnd(T, H, seed=2).to(dtype)
+    bias, a_log, skip = rnd(H, seed=3), rnd(H, seed=4, scale=0.5) - 2, rnd(H, seed=5)
+    state = rnd(31, H, N, P, seed=6, scale=2.0)
+    want, size, behind, sizes, bend = scanned(x, dt, bias, a_log, skip, state, meta, H, P, N, G)
+    got = ops.ssm_scan(x, dt, bias, a_log, skip, state, meta, H, P, N, G)
+    assert got.dtype == torch.float32
+    for got, want, size in ((got, want, size), (state, behind, sizes)):
+        assert ((got.to(F) - want).abs() <= (2 * bend + 64 + N / 8) * SINGLE * size).all()
+
+
+def test_as_many_heads_as_a_grid_holds(ops):
+    """Heads and groups together are more than a grid has rows."""
+    scan_case(ops, (33, 1), 65535, 1, 1, 1, torch.float32)
