@@ -93,6 +93,28 @@ __device__ __forceinline__ void load4(const bf16_t* p, float v[4]) {
   v[2] = __uint_as_float(raw.y << 16); v[3] = __uint_as_float(raw.y & 0xffff0000u);
 }
 
+// The sums over lanes of attn_generic_kernel. In the vector ALU only where that does not take registers away from waves: with it the
+// compiler has more loads under way, and heads of 96, 128 and 288 in bfloat16 went from 103 .. 118 registers to 132 .. 149, from four waves a
+// SIMD to three: 100 requests of 500 keys, 32 heads of 128 on one with a bias by distance, us, through the LDS unit / in the vector ALU
+// 118 / 202, of 288 261 / 450, 300 tokens of 12 heads of 96 on 2 53.2 / 60.5. Heads of 64 in bfloat16 take fewer with it (135 / 116; 0.86 of
+// the time on average), in float32 107 / 91 and up to 1.10 of the time; of 16 and 40 0.97 in both.
+template <typename C>
+constexpr bool GENERIC_SUMS_IN_VALU = D <= (sizeof(C) == 2 ? 64 : 48);
+template <typename C>
+__device__ __forceinline__ float generic_sum(float v) {
+  if constexpr (GENERIC_SUMS_IN_VALU<C>) return wave_sum(v);
+#pragma unroll
+  for (int o = DISTIE_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, DISTIE_WAVE);
+  return v;
+}
+template <typename C>
+__device__ __forceinline__ float generic_max(float v) {
+  if constexpr (GENERIC_SUMS_IN_VALU<C>) return wave_max(v);
+#pragma unroll
+  for (int o = DISTIE_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, DISTIE_WAVE));
+  return v;
+}
+
 // One workgroup of WAVES waves per (token, head). The keys are taken in chunks of 64 that begin at multiples of
 // 64; the chunks are dealt to the waves in turn (a token that decodes over thousands of keys then has eight
 // waves at work instead of one), every wave keeps its own running maximum, sum and output, and wave 0 puts them
@@ -146,10 +168,10 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES) void attn_generic_kernel(
       if (score_cap > 0.f) s = score_cap * tanhf(s / score_cap);
       s += slope * static_cast<float>(key - q_pos);
     }
-    const float m_new = fmaxf(m, wave_max(s));
+    const float m_new = fmaxf(m, generic_max<C>(s));
     const float alpha = m_new == -INFINITY ? 0.f : expf(m - m_new);     // 0 on the first chunk with a key (m = -inf)
     const float p = valid ? expf(s - m_new) : 0.f;
-    l = l * alpha + wave_sum(p);
+    l = l * alpha + generic_sum<C>(p);
     m = m_new;
     // what the lanes of this wave hand each other goes through the wave's own rows of LDS; the wave runs its
     // LDS traffic in order, so no barrier across waves is needed, only that the compiler keeps the order
