@@ -269,9 +269,10 @@ constexpr int GQ_SLICE = GQ_FITS ? D / 8 : 4;             // a lane's columns of
 constexpr int GQ_DIMS = GQ_FITS ? D / 16 : 1;              // a lane's dimensions of V: lane / 4, 16 more, ...
 static bool grouped_fits(int64_t tokens, int heads) { return GQ_FITS && tokens * heads < 2048; }
 
-// (the second bound keeps as many waves a SIMD as there were with fewer sums a lane)
+// (The second bound keeps as many waves a SIMD as there were with fewer sums a lane; for that one register goes to scratch memory with three
+// or four query heads of 64 and two or four of 256. With two heads beyond 256 it would be 127 to 489, for one wave a SIMD more.)
 template <int G, int WAVES>
-__global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 ? 2 : 1)) void attn_grouped_f32_kernel(
+__global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 && D <= 256 ? 2 : 1)) void attn_grouped_f32_kernel(
     const float* __restrict__ qkv, int64_t q_stride, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_request,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ table_rows,
@@ -324,7 +325,13 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 ? 2 : 1)
   // beyond 64, where four waves a SIMD hide more than loads ahead do): all of a chunk's keys and, in their place as they are used up, its
   // values; with three or four query heads half of the keys and of the values at a time.
   constexpr bool AHEAD = D > 64 && D <= 128;
-  constexpr int ROUND = G == 1 || (AHEAD && G == 2) ? 8 : 4, V_EARLY = !AHEAD ? 0 : G <= 2 ? 2 : 1;
+  // Heads beyond 288 don't fit so: their keys go in rounds of at most 72 loads (with two query heads 36, with more 18) and a quarter's
+  // values in parts; what does not fit goes through scratch memory. us without / with that: 8 heads of 512 on 4, 8 requests of 1,000 keys
+  // 69 / 28, 12 on 4, 32 of 200 98 / 23; 8 of 1,024 on one, 8 of 1,000 340 / 49; 12 of 320 on 4, 8 of 1,000 36.4 / 23.9.
+  constexpr int K_ROOM = (G == 1 ? 72 : G <= 2 || D <= 288 ? 36 : 18) / (GQ_SLICE / 4);
+  constexpr int ROUND = (G == 1 || (AHEAD && G == 2)) && K_ROOM >= 8 ? 8 : K_ROOM >= 4 ? 4 : K_ROOM >= 2 ? 2 : 1;
+  constexpr int V_EARLY = !AHEAD ? 0 : G <= 2 ? 2 : 1;
+  constexpr int V_PART = D <= 288 ? GQ_DIMS : G <= 2 ? 16 : 8, V_PARTS = (GQ_DIMS + V_PART - 1) / V_PART;      // dimensions
   constexpr int V_LOADS = G <= (AHEAD ? 2 : 1) ? 16 : 8;       // about, in whole quarters of the chunk
   constexpr int V_QUARTERS = V_LOADS >= 4 * GQ_DIMS ? 4 : V_LOADS >= 2 * GQ_DIMS ? 2 : 1, V_BATCHES = 4 / V_QUARTERS;
   for (int c = (chunk0 + run0 + wave) * DISTIE_WAVE; c < (chunk0 + run_end) * DISTIE_WAVE; c += DISTIE_WAVE * WAVES) {
@@ -346,14 +353,15 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 ? 2 : 1)
     const int hi = min(DISTIE_WAVE - 1, last - c);
     const int piece = lane % 4, dim0 = lane / 4;
     float4 vv[4][GQ_DIMS];
-    const auto ask_values = [&](int batch) {
+    const auto ask_values = [&](int batch, int part) {
 #pragma unroll
       for (int u = 0; u < V_QUARTERS; ++u) {
         const int quarter = batch * V_QUARTERS + u, j = 16 * quarter + 4 * piece;
         const int64_t page_base = base_s[wave][min(max(j, lo), hi)];      // of a key that counts
         const float* v = v_cache + page_base + static_cast<int64_t>(dim0) * block_size + (c + j) % block_size;
 #pragma unroll
-        for (int i = 0; i < GQ_DIMS; ++i) vv[quarter][i] = *reinterpret_cast<const float4*>(v + 16 * i * block_size);
+        for (int i = part * V_PART; i < min(GQ_DIMS, (part + 1) * V_PART); ++i)
+          vv[quarter][i] = *reinterpret_cast<const float4*>(v + 16 * i * block_size);
       }
     };
     // ---- scores: eight keys a pass, ROUND passes of loads under way together; afterwards lane j holds the scores of key c + j.
@@ -391,11 +399,13 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 ? 2 : 1)
 #pragma unroll
       for (int ps = 0; ps < ROUND; ++ps) {
         use_keys(ROUND * round + ps);
-        const int half = (ps + 1) / (ROUND / 2) - 1;
-        if (round == 8 / ROUND - 1 && (ps + 1) % (ROUND / 2) == 0 && half < V_EARLY) {
-          __builtin_amdgcn_sched_barrier(0);
-          ask_values(half);
-          __builtin_amdgcn_sched_barrier(0);
+        if constexpr (V_EARLY > 0) {
+          const int half = (ps + 1) / (ROUND / 2) - 1;
+          if (round == 8 / ROUND - 1 && (ps + 1) % (ROUND / 2) == 0 && half < V_EARLY) {
+            __builtin_amdgcn_sched_barrier(0);
+            ask_values(half, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
       }
     }
@@ -415,30 +425,34 @@ __global__ __launch_bounds__(DISTIE_WAVE * WAVES, (D <= 64 ? 4 : G == 2 ? 2 : 1)
     // ---- output
 #pragma unroll
     for (int batch = 0; batch < V_BATCHES; ++batch) {
-      if (batch >= V_EARLY) {
-        __builtin_amdgcn_sched_barrier(0);
-        ask_values(batch);
-        __builtin_amdgcn_sched_barrier(0);                  // all of these loads are under way before the first is used
-      }
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        if (batch == 0) {
-#pragma unroll
-          for (int i = 0; i < GQ_DIMS; ++i) acc[g][i] *= alpha[g];
+      for (int part = 0; part < V_PARTS; ++part) {
+        if (batch >= V_EARLY) {
+          __builtin_amdgcn_sched_barrier(0);
+          ask_values(batch, part);
+          __builtin_amdgcn_sched_barrier(0);                  // all of these loads are under way before the first is used
         }
+        const int first_dim = part * V_PART, end_dim = min(GQ_DIMS, first_dim + V_PART);
 #pragma unroll
-        for (int u = 0; u < V_QUARTERS; ++u) {
-          const int quarter = batch * V_QUARTERS + u, j = 16 * quarter + 4 * piece;
-          const float4 p = *reinterpret_cast<const float4*>(&p_s[wave][g][j]);
-          // never a value of a key that does not count (a weight of zero times what lies there could be NaN)
-          const bool in[4] = {j >= lo && j <= hi, j + 1 >= lo && j + 1 <= hi, j + 2 >= lo && j + 2 <= hi, j + 3 >= lo && j + 3 <= hi};
+        for (int g = 0; g < G; ++g) {
+          if (batch == 0) {
 #pragma unroll
-          for (int i = 0; i < GQ_DIMS; ++i) {
-            const float4 v = vv[quarter][i];
-            acc[g][i] = fmaf(p.x, in[0] ? v.x : 0.f, acc[g][i]);
-            acc[g][i] = fmaf(p.y, in[1] ? v.y : 0.f, acc[g][i]);
-            acc[g][i] = fmaf(p.z, in[2] ? v.z : 0.f, acc[g][i]);
-            acc[g][i] = fmaf(p.w, in[3] ? v.w : 0.f, acc[g][i]);
+            for (int i = first_dim; i < end_dim; ++i) acc[g][i] *= alpha[g];
+          }
+#pragma unroll
+          for (int u = 0; u < V_QUARTERS; ++u) {
+            const int quarter = batch * V_QUARTERS + u, j = 16 * quarter + 4 * piece;
+            const float4 p = *reinterpret_cast<const float4*>(&p_s[wave][g][j]);
+            // never a value of a key that does not count (a weight of zero times what lies there could be NaN)
+            const bool in[4] = {j >= lo && j <= hi, j + 1 >= lo && j + 1 <= hi, j + 2 >= lo && j + 2 <= hi, j + 3 >= lo && j + 3 <= hi};
+#pragma unroll
+            for (int i = first_dim; i < end_dim; ++i) {
+              const float4 v = vv[quarter][i];
+              acc[g][i] = fmaf(p.x, in[0] ? v.x : 0.f, acc[g][i]);
+              acc[g][i] = fmaf(p.y, in[1] ? v.y : 0.f, acc[g][i]);
+              acc[g][i] = fmaf(p.z, in[2] ? v.z : 0.f, acc[g][i]);
+              acc[g][i] = fmaf(p.w, in[3] ? v.w : 0.f, acc[g][i]);
+            }
           }
         }
       }

@@ -229,7 +229,7 @@ def ensure(name: str) -> Path:
     return build(name, force=False)
 
 
-DEFAULT_HEAD_DIMS = (16, 32, 40, 48, 64, 80, 96, 112, 128, 192, 256, 288)
+DEFAULT_HEAD_DIMS = (16, 32, 40, 48, 64, 80, 96, 112, 128, 192, 256, 288, 320)
 DEFAULT_MIXED_HEAD_DIMS = (32, 64, 96, 128, 160)
 
 

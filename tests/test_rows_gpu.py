@@ -172,3 +172,10 @@ def test_float32_decode_attention_at_the_ends_of_its_chunks(ops, heads, kv_heads
         per.value, waves.value, torch.cuda.current_stream().cuda_stream) == 0
     got = out.to(F).view(T, heads, dim)
     assert ((got - want).norm(dim=-1) <= 0.1 * (dim + 2) / 2 * 2.0 ** -24 * want.norm(dim=-1) + 2.0 ** -23 * want.norm(dim=-1)).all()
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(3, 3), (4, 2), (6, 2), (8, 2)])
+@pytest.mark.parametrize("keys", [1, 63, 65, 700])
+def test_float32_decode_attention_of_heads_beyond_the_registers(ops, heads, kv_heads, keys):
+    """One to four query heads of a size whose keys take several rounds and whose values several parts, the last of them shorter."""
+    test_float32_decode_attention_at_the_ends_of_its_chunks(ops, heads, kv_heads, 320, keys)
