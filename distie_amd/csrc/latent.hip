@@ -311,7 +311,21 @@ struct QueryTail {
   const float2* table;        // [T, pairs] cosine and sine
   float magnitude;
   int pairs, offset_in, neighbours;
+  int apart;                  // whether the layers of the grid behind the heads' work on it, a head a workgroup; else the head's first ones
 };
+
+// Which head and columns a workgroup works on; a head's tail: column -1. The grid is (column blocks, row blocks, heads, and with tails apart
+// the layers that hold a workgroup a head). Behind all products, because the chip's eight parts are dealt workgroups in turn: a tail behind
+// every product's one column block left the products to four of them (4,096 rows, 32 heads of 512 times 128 with 64 turned, us: the tail in the
+// product's own workgroup 112, behind it 192, behind all of them 110 and with x through LDS 90).
+struct HeadBlock {
+  int h, column;
+};
+__device__ __forceinline__ HeadBlock head_block(int H, const QueryTail& tail) {
+  const int z = blockIdx.z;
+  if (tail.pairs == 0 || z < H) return {z, static_cast<int>(blockIdx.x)};
+  return {static_cast<int>((z - H) * gridDim.x + blockIdx.x), -1};
+}
 
 // SLICED: x is float32 [slices, T, H * lx], partial sums of the product that made it, added in order and rounded to
 // bfloat16 once (what a kernel that adds them up in front of this one would hand over).
@@ -321,85 +335,10 @@ __device__ __forceinline__ float load_x(const void* x, int64_t at, int slices, i
   else return to_float(static_cast<const bf16_t*>(x)[at]);
 }
 
-// The workgroup's rows of x, KC columns of them at a time, lie in LDS, summed and rounded once: read by each wave from memory, a load of
-// theirs touched 64 lines, and with four slices a workgroup made 256 of them for a tile, slice after slice. The weights of those columns are
-// asked for in front of that; KC is what the registers hold of them where waves are few (192), and where they are many what leaves room for
-// three or more of them a SIMD (64; 192 there: 20.3 us). A head's tail has a workgroup of its own behind the columns'. us a launch, so /
-// now, 16 heads: 16 rows in four slices, 128 columns times 192 rows with a tail 8.9 / 5.5; 16 rows, 192 times 128 6.4 / 5.8; 1,787 rows
-// 19.0 / 16.4.
-template <int WT, int WN, int NB, int KC, bool SLICED>
-__global__ void __launch_bounds__(64 * WT * WN)
-heads_linear_mfma_kernel(const void* __restrict__ x, int slices, int64_t slice_stride, int lx, const bf16_t* __restrict__ w,
-                         bf16_t* __restrict__ out, int lo, int T, int H, int N, int K, QueryTail tail) {
-  constexpr int THREADS = 64 * WT * WN;
-  __shared__ __attribute__((aligned(16))) bf16_t x_s[WT * 32][KC + 8];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int h = blockIdx.z;
-  const int first = blockIdx.y * WT * 32;
-  const int rows = min(WT * 32, T - first);
-  if (tail.pairs == 0 || blockIdx.x != gridDim.x - 1) {
-    const int t0 = first + wave / WN * 32;
-    const int n0 = (blockIdx.x * WN + wave % WN) * 32 * NB;
-    const int r = lane % 32, kk = 8 * (lane / 32);
-    // weight rows beyond N repeat the last, rows of x beyond T are whatever lies in LDS: what becomes of them is not stored
-    const bf16_t* wr[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) wr[b] = w + (static_cast<int64_t>(h) * N + min(n0 + 32 * b + r, N - 1)) * K;
-    hl_floatx16 acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
-    for (int k0 = 0; k0 < K; k0 += KC) {
-      const int columns = min(KC, K - k0);
-      hl_bf16x8 bw[KC / 16][NB];
-#pragma unroll
-      for (int s = 0; s < KC / 16; ++s)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) bw[s][b] = *reinterpret_cast<const hl_bf16x8*>(wr[b] + min(k0 + 16 * s + kk, K - 8));
-      if (k0 > 0) __syncthreads();
-      const int pieces = columns / 8;                        // (K is a multiple of 8)
-      for (int i = threadIdx.x; i < rows * pieces; i += THREADS) {
-        const int row = i / pieces, c = 8 * (i % pieces);
-        const int64_t at = (static_cast<int64_t>(first + row) * H + h) * lx + k0 + c;
-        if constexpr (SLICED) {
-          float sum[8];
-          sum_values<8>(static_cast<const float*>(x) + at, slices, slice_stride, sum);
-          store_values<8>(&x_s[row][c], sum);
-        } else {
-          *reinterpret_cast<uint4*>(&x_s[row][c]) = *reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(x) + at);
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int s = 0; s < KC / 16; ++s) {
-        if (16 * s >= columns) break;
-        hl_bf16x8 a = *reinterpret_cast<const hl_bf16x8*>(&x_s[wave / WN * 32 + r][16 * s + kk]);
-        if (16 * s + kk >= columns) {
-          a = hl_bf16x8{};
-#pragma unroll
-          for (int b = 0; b < NB; ++b) bw[s][b] = hl_bf16x8{};
-        }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bw[s][b], acc[b], 0, 0, 0);
-      }
-    }
-    // acc[b][4 i + j]: row t0 + 8 i + 4 (lane / 32) + j of x, weight row n0 + 32 b + lane % 32
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int n = n0 + 32 * b + r;
-      if (n >= N) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int t = t0 + 8 * i + 4 * (lane / 32) + j;
-          if (t < T) out[(static_cast<int64_t>(t) * H + h) * lo + n] = static_cast<bf16_t>(acc[b][4 * i + j]);
-        }
-    }
-    return;
-  }
-  // the workgroup's rows of x, this head: the turned part behind the product's columns, zeros behind that
+// The tail of a head for `rows` rows of x from `first` on, by a workgroup: the turned part behind the product's columns, zeros behind that.
+template <bool SLICED>
+__device__ __forceinline__ void query_tail(const void* x, int slices, int64_t slice_stride, int lx, bf16_t* __restrict__ out, int lo,
+                                           int first, int rows, int h, int H, int N, const QueryTail& tail) {
   for (int i = threadIdx.x; i < rows * tail.pairs; i += blockDim.x) {
     const int t = first + i / tail.pairs, j = i % tail.pairs;
     const int a = tail.neighbours ? 2 * j : j, b = tail.neighbours ? 2 * j + 1 : j + tail.pairs;
@@ -417,6 +356,165 @@ heads_linear_mfma_kernel(const void* __restrict__ x, int slices, int64_t slice_s
     const int t = first + i / pad;
     out[(static_cast<int64_t>(t) * H + h) * lo + N + 2 * tail.pairs + i % pad] = static_cast<bf16_t>(0.f);
   }
+}
+
+// acc[b][4 i + j]: row t0 + 8 i + 4 (lane / 32) + j of x, weight row n0 + 32 b + lane % 32
+template <int NB>
+__device__ __forceinline__ void store_head(const hl_floatx16 (&acc)[NB], bf16_t* __restrict__ out, int lo, int t0, int n0, int h, int T, int H,
+                                           int N) {
+  const int lane = threadIdx.x % 64;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int n = n0 + 32 * b + lane % 32;
+    if (n >= N) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = t0 + 8 * i + 4 * (lane / 32) + j;
+        if (t < T) out[(static_cast<int64_t>(t) * H + h) * lo + n] = static_cast<bf16_t>(acc[b][4 * i + j]);
+      }
+  }
+}
+
+// The workgroup's rows of x, KC columns of them at a time, lie in LDS, summed and rounded once: read by each wave from memory, a load of
+// theirs touched 64 lines, and with four slices a workgroup made 256 of them for a tile, slice after slice. The weights of those columns are
+// asked for in front of that; KC is what the registers hold of them where waves are few (192), and where they are many what leaves room for
+// three or more of them a SIMD (64; 192 there: 20.3 us). `heads_linear_mfma` says which sizes take this kernel and which the one below.
+template <int WT, int WN, int NB, int KC, bool SLICED>
+__global__ void __launch_bounds__(64 * WT * WN)
+heads_linear_mfma_kernel(const void* __restrict__ x, int slices, int64_t slice_stride, int lx, const bf16_t* __restrict__ w,
+                         bf16_t* __restrict__ out, int lo, int T, int H, int N, int K, QueryTail tail) {
+  constexpr int THREADS = 64 * WT * WN;
+  __shared__ __attribute__((aligned(16))) bf16_t x_s[WT * 32][KC + 8];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const auto [h, column] = head_block(H, tail);
+  const int first = blockIdx.y * WT * 32;
+  const int rows = min(WT * 32, T - first);
+  if (h >= H) return;
+  if (column < 0) {
+    query_tail<SLICED>(x, slices, slice_stride, lx, out, lo, first, rows, h, H, N, tail);
+    return;
+  }
+  const int t0 = first + wave / WN * 32;
+  const int n0 = (column * WN + wave % WN) * 32 * NB;
+  const bool live = __builtin_amdgcn_readfirstlane(t0 < T && n0 < N);      // (the others only help with x)
+  const int r = lane % 32, kk = 8 * (lane / 32);
+  // weight rows beyond N repeat the last, rows of x beyond T are whatever lies in LDS: what becomes of them is not stored
+  const bf16_t* wr[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) wr[b] = w + (static_cast<int64_t>(h) * N + min(n0 + 32 * b + r, N - 1)) * K;
+  hl_floatx16 acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
+  for (int k0 = 0; k0 < K; k0 += KC) {
+    const int columns = min(KC, K - k0);
+    hl_bf16x8 bw[KC / 16][NB];
+    if (live) {
+#pragma unroll
+      for (int s = 0; s < KC / 16; ++s)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) bw[s][b] = *reinterpret_cast<const hl_bf16x8*>(wr[b] + min(k0 + 16 * s + kk, K - 8));
+    }
+    if (k0 > 0) __syncthreads();
+    const int pieces = columns / 8;                        // (K is a multiple of 8)
+    for (int i = threadIdx.x; i < rows * pieces; i += THREADS) {
+      const int row = i / pieces, c = 8 * (i % pieces);
+      const int64_t at = (static_cast<int64_t>(first + row) * H + h) * lx + k0 + c;
+      if constexpr (SLICED) {
+        float sum[8];
+        sum_values<8>(static_cast<const float*>(x) + at, slices, slice_stride, sum);
+        store_values<8>(&x_s[row][c], sum);
+      } else {
+        *reinterpret_cast<uint4*>(&x_s[row][c]) = *reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(x) + at);
+      }
+    }
+    __syncthreads();
+    if (!live) continue;
+#pragma unroll
+    for (int s = 0; s < KC / 16; ++s) {
+      if (16 * s >= columns) break;
+      hl_bf16x8 a = *reinterpret_cast<const hl_bf16x8*>(&x_s[wave / WN * 32 + r][16 * s + kk]);
+      if (16 * s + kk >= columns) {
+        a = hl_bf16x8{};
+#pragma unroll
+        for (int b = 0; b < NB; ++b) bw[s][b] = hl_bf16x8{};
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bw[s][b], acc[b], 0, 0, 0);
+    }
+  }
+  if (live) store_head<NB>(acc, out, lo, t0, n0, h, T, H, N);
+  if (tail.pairs > 0 && !tail.apart && column == 0) query_tail<SLICED>(x, slices, slice_stride, lx, out, lo, first, rows, h, H, N, tail);
+}
+
+// The same with each wave's operands straight from memory, two steps of sixteen columns under way together and no barrier.
+template <int WT, int WN, int NB, bool SLICED>
+__global__ void __launch_bounds__(64 * WT * WN)
+heads_linear_direct_kernel(const void* __restrict__ x, int slices, int64_t slice_stride, int lx, const bf16_t* __restrict__ w,
+                           bf16_t* __restrict__ out, int lo, int T, int H, int N, int K, QueryTail tail) {
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const auto [h, column] = head_block(H, tail);
+  const int first = blockIdx.y * WT * 32;
+  if (h >= H) return;
+  if (tail.pairs > 0 && (column < 0 || (!tail.apart && column == 0)))
+    query_tail<SLICED>(x, slices, slice_stride, lx, out, lo, first, min(WT * 32, T - first), h, H, N, tail);
+  if (column < 0) return;
+  const int t0 = first + wave / WN * 32;
+  const int n0 = (column * WN + wave % WN) * 32 * NB;
+  if (t0 >= T || n0 >= N) return;
+  const int r = lane % 32, kk = 8 * (lane / 32);
+  const bool t_in = t0 + r < T;
+  const int64_t x_at = (static_cast<int64_t>(t_in ? t0 + r : t0) * H + h) * lx + kk;
+  const bf16_t* wr[NB];
+  bool n_in[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    n_in[b] = n0 + 32 * b + r < N;
+    wr[b] = w + (static_cast<int64_t>(h) * N + (n_in[b] ? n0 + 32 * b + r : n0)) * K + kk;
+  }
+  hl_floatx16 acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    hl_bf16x8 a[2], bw[2][NB];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + 16 * s;
+      const bool k_in = k + kk < K;
+      a[s] = hl_bf16x8{};
+      if (t_in && k_in) {
+        if constexpr (SLICED) {
+          const float* xf = static_cast<const float*>(x) + x_at + k;
+          float4 lo4 = *reinterpret_cast<const float4*>(xf), hi4 = *reinterpret_cast<const float4*>(xf + 4);
+          for (int q = 1; q < slices; ++q) {
+            const float4 l2 = *reinterpret_cast<const float4*>(xf + q * slice_stride);
+            const float4 h2 = *reinterpret_cast<const float4*>(xf + q * slice_stride + 4);
+            lo4.x += l2.x, lo4.y += l2.y, lo4.z += l2.z, lo4.w += l2.w;
+            hi4.x += h2.x, hi4.y += h2.y, hi4.z += h2.z, hi4.w += h2.w;
+          }
+          a[s][0] = static_cast<bf16_t>(lo4.x), a[s][1] = static_cast<bf16_t>(lo4.y);
+          a[s][2] = static_cast<bf16_t>(lo4.z), a[s][3] = static_cast<bf16_t>(lo4.w);
+          a[s][4] = static_cast<bf16_t>(hi4.x), a[s][5] = static_cast<bf16_t>(hi4.y);
+          a[s][6] = static_cast<bf16_t>(hi4.z), a[s][7] = static_cast<bf16_t>(hi4.w);
+        } else {
+          a[s] = *reinterpret_cast<const hl_bf16x8*>(static_cast<const bf16_t*>(x) + x_at + k);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        bw[s][b] = (n_in[b] && k_in) ? *reinterpret_cast<const hl_bf16x8*>(wr[b] + k) : hl_bf16x8{};
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], bw[s][b], acc[b], 0, 0, 0);
+  }
+  store_head<NB>(acc, out, lo, t0, n0, h, T, H, N);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -509,15 +607,26 @@ static int heads_linear_mfma(const void* x, int slices, int lx, const void* w, v
   const bf16_t* wb = static_cast<const bf16_t*>(w);
   bf16_t* ob = static_cast<bf16_t*>(out);
   const int64_t stride = static_cast<int64_t>(T) * H * lx;
+  const int columns = (N + 127) / 128, row_blocks = T <= 32 ? 1 : (T + 63) / 64;
+  if (row_blocks > 65535) return DISTIE_BAD_ARGUMENT;
+  const int tails = tail.pairs > 0 ? (H + columns - 1) / columns : 0;
+  tail.apart = H + tails <= 65535;
+  const dim3 grid(columns, row_blocks, H + (tail.apart ? tails : 0));
+  // x through LDS pays where it is added up from slices, or where workgroups are many enough to hide a trip behind each other, two a compute
+  // unit and their rows full; and where both column waves have work. us, straight / through LDS: 16 rows, 32 heads of 512 times 128 8.6 /
+  // 10.3; 300 rows of it 15.6 / 22.4, 1,000 29.7 / 29.2, 4,096 102 / 81; 1,787 rows, 8 heads of 128 times 64 5.5 / 6.7. In two slices,
+  // before / through LDS: 16 rows, 16 heads of 192 times 128 with a tail 9.0 / 6.2, 1,787 rows 31 / 25.7; straight / through LDS, 1,787 rows,
+  // 8 heads of 128 times 64 8.4 / 8.8, 4,096 rows, 16 of 40 times 48 11.2 / 15.0.
+  const int64_t full_blocks = static_cast<int64_t>(columns) * T * H / 64;
   if (T <= 32) {
-    const dim3 grid((N + 127) / 128 + (tail.pairs > 0 ? 1 : 0), 1, H);
     if (slices > 1) heads_linear_mfma_kernel<1, 4, 1, 192, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
-    else heads_linear_mfma_kernel<1, 4, 1, 192, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
+    else heads_linear_direct_kernel<1, 4, 1, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
+  } else if (slices > 1) {
+    if (N <= 64) heads_linear_direct_kernel<2, 2, 2, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
+    else heads_linear_mfma_kernel<2, 2, 2, 64, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
   } else {
-    const dim3 grid((N + 127) / 128 + (tail.pairs > 0 ? 1 : 0), (T + 63) / 64, H);
-    if (grid.y > 65535) return DISTIE_BAD_ARGUMENT;
-    if (slices > 1) heads_linear_mfma_kernel<2, 2, 2, 64, true><<<grid, 256, 0, stream>>>(x, slices, stride, lx, wb, ob, lo, T, H, N, K, tail);
-    else heads_linear_mfma_kernel<2, 2, 2, 64, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
+    if (N > 64 && full_blocks >= 512) heads_linear_mfma_kernel<2, 2, 2, 64, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
+    else heads_linear_direct_kernel<2, 2, 2, false><<<grid, 256, 0, stream>>>(x, 1, 0, lx, wb, ob, lo, T, H, N, K, tail);
   }
   return launch_status();
 }
@@ -534,7 +643,7 @@ extern "C" int distie_latent_queries(const void* x, int dtype, int slices, int l
       table == nullptr || !heads_linear_mfma_fits(x, dtype, w, w_dtype, lx, K, slices) || (slices == 1 && dtype != DISTIE_BF16))
     return DISTIE_BAD_ARGUMENT;
   return heads_linear_mfma(x, slices, lx, w, out, lo, T, H, N, K,
-                           QueryTail{static_cast<const float2*>(table), magnitude, pairs, K, neighbours}, stream);
+                           QueryTail{static_cast<const float2*>(table), magnitude, pairs, K, neighbours, 0}, stream);
 }
 
 extern "C" int distie_heads_linear(const void* x, int dtype, int lx, const void* w, int w_dtype, void* out, int lo, int T,
@@ -542,7 +651,7 @@ extern "C" int distie_heads_linear(const void* x, int dtype, int lx, const void*
   if (T <= 0) return 0;
   if (H < 1 || N < 1 || K < 1 || lx < K || lo < N || H > 65535) return DISTIE_BAD_ARGUMENT;
   if (heads_linear_mfma_fits(x, dtype, w, w_dtype, lx, K, 1))
-    return heads_linear_mfma(x, 1, lx, w, out, lo, T, H, N, K, QueryTail{nullptr, 1.f, 0, 0, 0}, stream);
+    return heads_linear_mfma(x, 1, lx, w, out, lo, T, H, N, K, QueryTail{nullptr, 1.f, 0, 0, 0, 0}, stream);
   if (T <= 2 * HLR_ROWS) {
     const int64_t items = static_cast<int64_t>(H) * N;
     const dim3 grid(static_cast<unsigned>((items + 3) / 4), (T + HLR_ROWS - 1) / HLR_ROWS);

@@ -179,3 +179,21 @@ def test_float32_decode_attention_at_the_ends_of_its_chunks(ops, heads, kv_heads
 def test_float32_decode_attention_of_heads_beyond_the_registers(ops, heads, kv_heads, keys):
     """One to four query heads of a size whose keys take several rounds and whose values several parts, the last of them shorter."""
     test_float32_decode_attention_at_the_ends_of_its_chunks(ops, heads, kv_heads, 320, keys)
+
+
+@pytest.mark.parametrize("T", [5461, 5462, 5500])
+@pytest.mark.parametrize("dim,kv_rank", [(72, 129), (200, 129), (192, 64)])
+def test_queries_of_a_latent_where_workgroups_are_many(ops, T, dim, kv_rank):
+    """Three heads: where the input begins to go through LDS, and where one wave's columns are all there are."""
+    test_queries_of_a_latent(ops, T, dim, 8, kv_rank, 1)
+
+
+def test_queries_of_as_many_heads_as_a_grid_holds(ops):
+    """Each head's tail has a workgroup of its own while a grid holds them, here not: the same bits as of a third of the heads."""
+    heads, dim, rot_dim, kv_rank, T = 65535, 8, 2, 8, 2
+    q, up = rnd(T, heads * (dim + rot_dim), seed=1).bfloat16(), rnd(heads, kv_rank, dim, seed=2).bfloat16()
+    freq = torch.ones(1, device="cuda")
+    meta = SimpleNamespace(num_tokens=T, positions=torch.arange(T, dtype=torch.int32, device="cuda"), scratch={})
+    call = lambda q, up: ops.latent_queries(q.contiguous(), up.contiguous(), len(up), dim, rot_dim, 11, freq, 1.0, False, meta).view(T, -1, 11)  # noqa: E731
+    parts = zip(q.view(T, 3, -1).unbind(1), up.view(3, -1, kv_rank, dim).unbind(0))
+    assert torch.equal(call(q, up), torch.cat([call(*p) for p in parts], 1))
