@@ -81,13 +81,23 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  // all sixteen places are read together, and those that no wave wrote are dropped (a loop over the waves waited for each)
+  // a few waves' places, or all sixteen, are read together, and those that no wave wrote are dropped (a loop over the waves waited for
+  // each; sixteen for every block: norms of groups of 128, 2,048 rows of 2,048, 13.9 -> 14.7 us)
   float part[16];
+  float total;
+  if (waves <= 4) {
 #pragma unroll
-  for (int w = 0; w < 16; ++w) part[w] = scratch[w];
-  float total = part[0];
+    for (int w = 0; w < 4; ++w) part[w] = scratch[w];
+    total = part[0];
 #pragma unroll
-  for (int w = 1; w < 16; ++w) total = w < waves ? total + part[w] : total;
+    for (int w = 1; w < 4; ++w) total = w < waves ? total + part[w] : total;
+  } else {
+#pragma unroll
+    for (int w = 0; w < 16; ++w) part[w] = scratch[w];
+    total = part[0];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) total = w < waves ? total + part[w] : total;
+  }
   return total;
 }
 
