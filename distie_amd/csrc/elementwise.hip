@@ -112,19 +112,37 @@ __global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(float* __restrict__ r
   const int64_t row = blockIdx.x;
   const int quads = width / 4;
   float4 v[NV], wq[NV];
+  float sum[NV][4] = {};
   float ss = 0.f;
+  // (all of a thread's groups are asked for before the first is stored: a store waits for its sum)
+#pragma unroll
+  for (int e = 0; e < NV; ++e) {
+    const int q = threadIdx.x + e * blockDim.x;
+    v[e] = *reinterpret_cast<const float4*>(residual + row * width + 4 * static_cast<int64_t>(q < quads ? q : 0));
+    wq[e] = load_weights4(weight + 4 * (q < quads ? q : 0));
+  }
+  if (delta != nullptr) {
+    const D* from[NV];
+#pragma unroll
+    for (int e = 0; e < NV; ++e) {
+      const int q = threadIdx.x + e * blockDim.x;
+      from[e] = delta + row * width + 4 * static_cast<int64_t>(q < quads ? q : 0);
+    }
+    if (slices == 1) {
+#pragma unroll
+      for (int e = 0; e < NV; ++e) load_values<4>(from[e], sum[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < NV; ++e) sum_values<4>(from[e], slices, slice_stride, sum[e]);
+    }
+  }
 #pragma unroll
   for (int e = 0; e < NV; ++e) {
     const int q = threadIdx.x + e * blockDim.x;
     const bool in = q < quads;
-    const int64_t at = row * width + 4 * static_cast<int64_t>(in ? q : 0);
-    const float4 x4 = *reinterpret_cast<const float4*>(residual + at);
-    wq[e] = load_weights4(weight + 4 * (in ? q : 0));
-    float sum[4] = {0.f, 0.f, 0.f, 0.f};
-    if (delta != nullptr) sum_values<4>(delta + at, slices, slice_stride, sum);
-    v[e] = float4{x4.x + sum[0], x4.y + sum[1], x4.z + sum[2], x4.w + sum[3]};
+    v[e] = float4{v[e].x + sum[e][0], v[e].y + sum[e][1], v[e].z + sum[e][2], v[e].w + sum[e][3]};
     if (!in) v[e] = float4{0.f, 0.f, 0.f, 0.f};
-    if (in && delta != nullptr) *reinterpret_cast<float4*>(residual + at) = v[e];
+    if (in && delta != nullptr) *reinterpret_cast<float4*>(residual + row * width + 4 * static_cast<int64_t>(q)) = v[e];
     ss += v[e].x * v[e].x + v[e].y * v[e].y + v[e].z * v[e].z + v[e].w * v[e].w;
   }
   const float scale = rsqrtf(block_sum(ss, scratch) / static_cast<float>(width) + eps);
