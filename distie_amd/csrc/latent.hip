@@ -59,13 +59,17 @@ latent_norm_rope_write_kernel(const float* __restrict__ down, int slices, int64_
     for (int u = 0; u < LN_AHEAD; ++u) kv_w[u] = kv_weight[min(tid + u * threads, kv_rank - 1)];
     if (table != nullptr && pairs > 0) angle = table[t * pairs + min(tid, pairs - 1)];
   }
+  const float* from = down + t * ld;
   for (int c0 = 0; c0 < width; c0 += LN_AHEAD * threads) {
-    const float* from = down + t * ld;
     float part[4][LN_AHEAD];
 #pragma unroll
-    for (int u = 0; u < LN_AHEAD; ++u)
+    for (int u = 0; u < LN_AHEAD; ++u) part[0][u] = from[min(c0 + tid + u * threads, width - 1)];
+    if (slices > 1) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) part[s][u] = from[min(s, slices - 1) * slice_stride + min(c0 + tid + u * threads, width - 1)];
+      for (int u = 0; u < LN_AHEAD; ++u)
+#pragma unroll
+        for (int s = 1; s < 4; ++s) part[s][u] = from[min(s, slices - 1) * slice_stride + min(c0 + tid + u * threads, width - 1)];
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < LN_AHEAD; ++u) {
