@@ -34,9 +34,9 @@ __device__ __forceinline__ float activate(float z, int kind) {   // the kinds of
 //   x  += y                                          (residual, float32, in place; null: y goes to y_out)
 //   out = rms(x) * pre_w                             (the norm in front of the next sub-layer)
 // rms(v) = v / sqrt(mean(v^2) + eps). A term may be partial sums (slices that lie `stride` apart, added in order).
-// The row waits in LDS between the passes; a thread meets the same columns in every pass. `held`: the terms and the
-// residual are read once, up front and together, and wait in LDS too (rows of up to NORM_HELD_MAX columns); else
-// they are read again where they are needed.
+// The row waits in LDS between the passes; a thread meets the same columns in every pass. `in_lds`: the terms and the
+// residual are read once, up front and together, and wait in LDS too (rows of up to NORM_HELD_MAX columns; where four columns can be
+// read at once those are norm_chain_row_kernel's); else they are read again where they are needed.
 constexpr int NORM_HELD_MAX = 8192;
 
 template <int V, typename A, typename B, typename O>
@@ -44,8 +44,9 @@ __global__ void norm_chain_kernel(const A* __restrict__ t0, int slices0, int64_t
                                   const B* __restrict__ t1, int slices1, int64_t stride1, const float* __restrict__ w1,
                                   float term_eps, float scale, const float* __restrict__ post_w, float post_eps,
                                   float* __restrict__ residual, const float* __restrict__ pre_w, float pre_eps,
-                                  O* __restrict__ out, float* __restrict__ y_out, int C, int held) {
+                                  O* __restrict__ out, float* __restrict__ y_out, int C, int in_lds) {
   extern __shared__ float row[];
+  const bool held = V == 1 && in_lds;
   __shared__ float scratch[16];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * C;
   float* held_a = row + C;
