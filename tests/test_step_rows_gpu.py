@@ -130,3 +130,76 @@ def scan_case(ops, cuts, H, P, N, G, dtype):
 def test_as_many_heads_as_a_grid_holds(ops):
     """Heads and groups together are more than a grid has rows."""
     scan_case(ops, (33, 1), 65535, 1, 1, 1, torch.float32)
+
+
+@pytest.mark.parametrize("T", [255, 256, 257, 300])
+@pytest.mark.parametrize("channels", [8, 424, 520])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_convolution_of_two_rows_a_thread(ops, T, channels, taps):
+    """From 256 rows on a thread has two, which may belong to one request or to two, one of them a single row; channels that leave lanes of the
+    last wave without any. With a bias and silu, whose slope is below 1.1, or with the row itself added."""
+    cuts = [1, 2, 3, 1, 1, 5, 1, 2, 61, 1, 1, 3, 2, 1, 4]
+    cuts += [T - sum(cuts) - 2, 1, 1]
+    filters, bias = rnd(channels, taps, seed=1, scale=0.5).bfloat16(), rnd(channels, seed=2)
+    x, first = rnd(T, channels, seed=3).bfloat16(), rnd(31, taps - 1, channels, seed=4, scale=2.0)
+    meta, _ = step(cuts)
+    sums, size, behind = convolved(x, filters, first, meta)
+    for residual, act in ((False, "silu"), (True, None)):
+        state = first.clone()
+        got = ops.causal_conv(x, filters, state, meta, residual, bias, act)
+        want = sums + bias.to(F) + (x.to(F) if residual else 0.0)
+        off = (taps + 3) * SINGLE * (size + bias.abs() + (x.abs() if residual else 0.0))
+        if act:
+            want, off = want * torch.sigmoid(want), 1.1 * off + 8 * SINGLE * want.abs()
+        assert ((got.to(F) - want).abs() <= HALF * want.abs() + off).all()
+        assert torch.equal(state.to(F), behind)
+
+
+@pytest.mark.parametrize("cuts", [(33, 1, 1, 40, 1), (1,) * 20 + (64,), (65, 1), (1, 200, 2, 1, 3), (32,), (1, 128)])
+@pytest.mark.parametrize("H,P,N,G", [(4, 64, 16, 2), (2, 40, 33, 1), (3, 130, 64, 3), (2, 64, 128, 1), (2, 24, 256, 2), (2, 16, 257, 1)])
+def test_single_rows_beside_portions_of_state_spaces(ops, cuts, H, P, N, G):
+    """Single rows go row by row, portions in chunks; a state of more rows than the row-by-row kernel keeps goes in chunks with both."""
+    scan_case(ops, cuts, H, P, N, G, torch.bfloat16 if N % 2 == 0 else torch.float32)
+
+
+@pytest.mark.parametrize("cuts", [(16,), (17, 1), (64, 1, 63), (65, 16, 1, 130)])
+@pytest.mark.parametrize("heads,dim", [(3, 16), (2, 24), (2, 64), (2, 72), (1, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_time_mixing_at_the_ends_of_its_chunks(ops, cuts, heads, dim, dtype, pad):
+    """Whole and partial chunks and runs of sixteen rows, heads that fill their channels and others, rows that four values can be read from and
+    others. A sum is off by a few roundings of its terms and by those of the decays' exponents, added up over at most 64 rows; the
+    norm carries the head's relative error on."""
+    meta, _ = step(cuts)
+    T, N, rank, eps = meta.num_tokens, heads * dim, 5, 1e-5
+    rows = rnd(T, 4 * N + pad, seed=1).to(dtype)
+    r, k, v, gates = (rows[:, i * N:(i + 1) * N] for i in range(4))
+    low, up, up_bias = rnd(T, rank, seed=2), rnd(N, rank, seed=3, scale=0.3), rnd(N, seed=4, scale=0.3)
+    bonus, weight = rnd(N, seed=5), 1 + rnd(N, seed=6, scale=0.2)
+    state = rnd(31, heads, dim, dim, seed=7)
+    z = torch.tanh(low.to(F)) @ up.to(F).t().contiguous() + up_bias.to(F)
+    rate = torch.exp(z).view(T, heads, dim)
+    r_, k_, v_ = (t.to(F).reshape(T, heads, dim) for t in (r, k, v))
+    u = bonus.to(F).view(heads, dim, 1)
+    out, size = torch.empty(T, heads, dim, dtype=F, device="cuda"), torch.empty(T, heads, dim, dtype=F, device="cuda")
+    behind, sizes, bend = state.to(F), state.to(F).abs(), 0.0
+    for b in range(meta.num_requests):
+        at, first, end = (5 * b + 2) % 31, *meta.host_cu_q[b:b + 2]
+        bend = max([bend] + [rate[t:min(t + 64, end)].sum(0).max().item() for t in range(first, end, 64)])
+        s, most = behind[at], sizes[at]
+        for t in range(first, end):
+            pair, decay = k_[t][:, :, None] * v_[t][:, None, :], torch.exp(-rate[t])[:, :, None]
+            out[t] = ((s + u * pair) * r_[t][:, :, None]).sum(1)
+            size[t] = ((most + (u * pair).abs()) * r_[t].abs()[:, :, None]).sum(1)
+            s, most = decay * s + pair, decay * most + pair.abs()
+        behind[at], sizes[at] = s, most
+    g = gates.to(F).view(T, heads, dim)
+    normed = out / torch.sqrt((out * out).mean(-1, keepdim=True) + eps)
+    factor = weight.to(F).view(heads, dim) * g * torch.sigmoid(g)
+    got = ops.wkv_mix(r, k, v, gates, low, up, up_bias, bonus, state, meta, heads, dim, weight, eps, dtype).to(F).view(T, heads, dim)
+    # (the decay's logit: rank + 2 roundings of its terms and those of tanh; a decay's relative error is its exponent's absolute one)
+    coefficient = (bend * (rank + 8) + 64 + dim / 4) * SINGLE
+    off = 2 * coefficient * size.norm(dim=-1) / out.norm(dim=-1) * (normed.norm(dim=-1) * factor.abs().amax(-1))
+    want = normed * factor
+    assert ((got - want).norm(dim=-1) <= off + ((HALF if dtype == torch.bfloat16 else 0.0) + 16 * SINGLE) * want.norm(dim=-1)).all()
+    assert ((state.to(F) - behind).abs() <= coefficient * sizes).all()
