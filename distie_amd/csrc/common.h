@@ -25,6 +25,9 @@ __device__ __forceinline__ float from_float<float>(float x) { return x; }
 template <>
 __device__ __forceinline__ bf16_t from_float<bf16_t>(float x) { return static_cast<bf16_t>(x); }  // round to nearest even
 
+// The loads in front of it are asked for before anything behind it (left to itself the compiler puts each in front of its use).
+__device__ __forceinline__ void loads_first() { __builtin_amdgcn_sched_barrier(0); }
+
 // The values of lanes i and i ^ O, in one order or the other: whoever adds them or takes the larger has the same in both lanes. Within
 // rows of 16 lanes by DPP (8: rotated by half a row; 4: each half of a row mirrored, then each quad; 2 and 1: a quad's lanes permuted),
 // beyond by the swaps of 16 and 32 lanes: a step of a sum is a move and an add in the vector ALU, where `__shfl_xor` sends the
@@ -113,7 +116,7 @@ __device__ __forceinline__ float sum_strided(const T* p, int slices, int64_t str
     const float b = to_float(p[min(s + 1, last) * stride]);
     const float c = to_float(p[min(s + 2, last) * stride]);
     const float d = to_float(p[min(s + 3, last) * stride]);
-    __builtin_amdgcn_sched_barrier(0);          // (selects below: where a sum stands under a condition, its load is put there too)
+    loads_first();                              // (selects below: where a sum stands under a condition, its load is put there too)
     sum += a;
     sum = s + 1 <= last ? sum + b : sum;
     sum = s + 2 <= last ? sum + c : sum;

@@ -70,7 +70,7 @@ latent_norm_rope_write_kernel(const float* __restrict__ down, int slices, int64_
 #pragma unroll
         for (int s = 1; s < 4; ++s) part[s][u] = from[min(s, slices - 1) * slice_stride + min(c0 + tid + u * threads, width - 1)];
     }
-    __builtin_amdgcn_sched_barrier(0);
+    loads_first();
 #pragma unroll
     for (int u = 0; u < LN_AHEAD; ++u) {
       const int c = c0 + tid + u * threads;

@@ -1092,7 +1092,8 @@ head_norm_rope_kv_write_bf16_kernel(const bf16_t* __restrict__ product, int64_t 
 // (`neighbours`) or in the lane pairs / 8 away. The blocks from `qk_blocks` on write v: 16 rows each, one channel a thread.
 // What bounds it are its trips to memory in a row: which request, where that begins, the state of rows that need it. Everything else a
 // run needs is asked for in front of them, and what is asked for a request is asked for by all rows at once: 899 rows of 8 and 2 heads
-// of 128, portions beside single tokens, 25.4 -> 12.5 us (runs of four rows 20.3, of which the v blocks, row after row, were most).
+// of 128, portions beside single tokens, 17.6 -> 13.8 us (25.4 by a trace, and runs of four rows 20.3, of which the v blocks, row after row,
+// were most).
 constexpr int CONV_ROWS = 2;
 
 template <int TAPS>

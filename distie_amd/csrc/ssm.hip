@@ -130,9 +130,6 @@ __device__ __forceinline__ void put_tile(float (*tile)[SSM_PAD], const X raw[16]
   }
 }
 
-// The loads in front of it are asked for before anything behind it (left to itself the compiler puts each in front of its use).
-__device__ __forceinline__ void loads_first() { __builtin_amdgcn_sched_barrier(0); }
-
 // d_j and l_j of a chunk's rows for one head, into LDS (the running sums by the first wave, one row a lane)
 template <typename X>
 __device__ __forceinline__ void chunk_decays(const X* __restrict__ dt, int64_t ldd, int first, int rows, int head,

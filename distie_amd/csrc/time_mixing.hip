@@ -211,12 +211,10 @@ template <> struct Four<bf16_t> {
   }
 };
 
-// The loads in front of it are asked for before anything behind it: what a lane needs at the start is one trip to memory then. (Left to
-// itself, and with a choice at every load between whole heads and others, the compiler waited for r, k, ln w, each piece of V and the
-// state one after the other: 2 prompts of 901, 32 heads of 64, outputs 42.2 -> 38.2 us, sums 16.3 -> 15.6; four workgroups a compute
-// unit hid the rest.)
-__device__ __forceinline__ void loads_first() { __builtin_amdgcn_sched_barrier(0); }
 
+// `loads_first` behind what a lane needs at the start makes that one trip to memory. (Left to itself, and with a choice at every load between
+// whole heads and others, the compiler waited for r, k, ln w, each piece of V and the state one after the other: 2 prompts of 901, 32 heads
+// of 64, outputs 42.2 -> 38.2 us, sums 16.3 -> 15.6; four workgroups a compute unit hid the rest.)
 // a lane's channels of a row of a whole head, which is there in memory whether it counts or not
 template <int DP, typename X>
 __device__ __forceinline__ void ask_channels(const X* __restrict__ row, int g, Four<X> (&raw)[DP / 16]) {

@@ -54,7 +54,7 @@ template <int N, int V, typename T>
 __device__ __forceinline__ void load_slices(const T* __restrict__ p, int slices, int64_t stride, float a[N][V]) {
 #pragma unroll
   for (int u = 0; u < N; ++u) load_values<V>(p + min(u, slices - 1) * stride, a[u]);
-  __builtin_amdgcn_sched_barrier(0);
+  loads_first();
 }
 
 // the sum of `slices` vectors that lie `stride` elements apart, added in order. Up to eight slices, which is what products are cut into, cost
