@@ -163,11 +163,8 @@ __global__ void norm_chain_kernel(const A* __restrict__ t0, int slices0, int64_t
 
 // The same for rows whose every thread has at most Q runs of four columns: the row, the residual and all weights are asked for together
 // and wait in registers. What bounds a step of few rows is trips to memory: norm_chain_kernel, with the row in LDS, asked for each weight
-// behind the sum in front of it (three or four trips in a row), and its LDS left few rows a compute unit. The same bits: every square
-// joins its sum in one rounding, as in that kernel's loops (left to the compiler, of the first two the first one did). us, so / now:
+// behind the sum in front of it (three or four trips in a row), and its LDS left few rows a compute unit. The sums' order is the same. us, so / now:
 // 16 rows of 2,048 5.6 / 4.5, 899 of 1,024 6.7 / 5.6 with slices in front, 8.0 / 6.9 without.
-__device__ __forceinline__ float square_added(float v, float sum) { return __builtin_fmaf(v, v, sum); }
-
 template <int Q, typename A, typename B, typename O>
 __global__ void __launch_bounds__(1024)
 norm_chain_row_kernel(const A* __restrict__ t0, int slices0, int64_t stride0, const float* __restrict__ w0,
@@ -216,14 +213,14 @@ norm_chain_row_kernel(const A* __restrict__ t0, int slices0, int64_t stride0, co
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) q0 = square_added(in[q] ? y[q][k] : 0.f, q0);
+      for (int k = 0; k < 4; ++k) q0 += in[q] ? y[q][k] * y[q][k] : 0.f;
     const float r0 = 1.f / sqrtf(block_sum(q0, scratch) / C + term_eps);
     float r1 = 1.f;
     if (t1 != nullptr) {
 #pragma unroll
       for (int q = 0; q < Q; ++q)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) q1 = square_added(in[q] ? b[q][k] : 0.f, q1);
+        for (int k = 0; k < 4; ++k) q1 += in[q] ? b[q][k] * b[q][k] : 0.f;
       r1 = 1.f / sqrtf(block_sum(q1, scratch) / C + term_eps);
     }
 #pragma unroll
@@ -240,7 +237,7 @@ norm_chain_row_kernel(const A* __restrict__ t0, int slices0, int64_t stride0, co
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) sq = square_added(in[q] ? y[q][k] : 0.f, sq);
+      for (int k = 0; k < 4; ++k) sq += in[q] ? y[q][k] * y[q][k] : 0.f;
     const float rp = 1.f / sqrtf(block_sum(sq, scratch) / C + post_eps);
 #pragma unroll
     for (int q = 0; q < Q; ++q)
@@ -257,7 +254,7 @@ norm_chain_row_kernel(const A* __restrict__ t0, int slices0, int64_t stride0, co
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) x[q][k] += y[q][k], sq = square_added(in[q] ? x[q][k] : 0.f, sq);
+    for (int k = 0; k < 4; ++k) x[q][k] += y[q][k], sq += in[q] ? x[q][k] * x[q][k] : 0.f;
     if (in[q]) store_values<4>(residual + base + col[q], x[q]);
   }
   if (out == nullptr) return;

@@ -197,20 +197,3 @@ def test_queries_of_as_many_heads_as_a_grid_holds(ops):
     call = lambda q, up: ops.latent_queries(q.contiguous(), up.contiguous(), len(up), dim, rot_dim, 11, freq, 1.0, False, meta).view(T, -1, 11)  # noqa: E731
     parts = zip(q.view(T, 3, -1).unbind(1), up.view(3, -1, kv_rank, dim).unbind(0))
     assert torch.equal(call(q, up), torch.cat([call(*p) for p in parts], 1))
-
-
-def test_squares_of_a_row_join_their_sum_in_one_rounding(ops):
-    """A norm of 256 columns, bit for bit: a lane's four squares each in a fused multiply-add, then the lanes' sums 32, 16, .. lanes apart."""
-    import numpy as np
-
-    T, C, eps = 2000, 256, np.float32(1e-5)
-    x, w = rnd(T, C, seed=1, scale=3.0), 1 + rnd(C, seed=2, scale=0.1)
-    got = ops._norm_chain([torch.zeros(T, C, device="cuda")], None, 0.0, 1.0, None, x.clone(), (w, float(eps)), torch.float32)
-    rows, w = x.cpu().numpy(), w.cpu().numpy()
-    total = np.zeros((T, 64), np.float32)
-    for k in range(4):                                       # (exact products of float32; the sums of two float64 are rounded once more)
-        total = (rows[:, k::4].astype(np.float64) ** 2 + total).astype(np.float32)
-    for o in (32, 16, 8, 4, 2, 1):
-        total = total + total[:, np.arange(64) ^ o]
-    scale = np.float32(1) / np.sqrt(total[:, :1] / np.float32(C) + eps)
-    assert np.array_equal(got.cpu().numpy(), rows * scale * w)
