@@ -163,8 +163,11 @@ __global__ void norm_chain_kernel(const A* __restrict__ t0, int slices0, int64_t
 
 // The same for rows whose every thread has at most Q runs of four columns: the row, the residual and all weights are asked for together
 // and wait in registers. What bounds a step of few rows is trips to memory: norm_chain_kernel, with the row in LDS, asked for each weight
-// behind the sum in front of it (three or four trips in a row), and its LDS left few rows a compute unit. The sums' order is the same. us, so / now:
-// 16 rows of 2,048 5.6 / 4.5, 899 of 1,024 6.7 / 5.6 with slices in front, 8.0 / 6.9 without.
+// behind the sum in front of it (three or four trips in a row), and its LDS left few rows a compute unit. The sums' order is the same, not their
+// bits: the squares of columns beyond the row are dropped behind the product, and so the compiler fuses other squares into the sum than in that
+// kernel's loops, a rounding of float32 in the statistics (Dufelix's decode step by 0.006 of its logits' norm, where bfloat16 roundings flip;
+// the error against 64 bits is the same, 0.011). us, so / now: 16 rows of 2,048 5.6 / 4.5, 899 of 1,024 6.7 / 5.6 with slices in front, 8.0 / 6.9
+// without.
 template <int Q, typename A, typename B, typename O>
 __global__ void __launch_bounds__(1024)
 norm_chain_row_kernel(const A* __restrict__ t0, int slices0, int64_t stride0, const float* __restrict__ w0,
