@@ -103,7 +103,11 @@ static __device__ __forceinline__ void store4(bf16_t* p, const float4& v) {
   *reinterpret_cast<uint2*>(p) = uint2{a | (b << 16), c | (d << 16)};
 }
 
-template <typename D, typename W, typename O, int NV>
+// A thread's groups of four go one after the other, each stored before the next is asked for. ONE: delta is null or one slice, as a kernel of its own:
+// with the loads of several slices beside them two groups took 64 registers instead of 36, and rows of more than 4,096 columns were slower from
+// the second workgroup of a compute unit on. us, 301 rows of 8,192 in one slice of float32 8.8 / 8.1, 2,048 rows 47.5 / 43.7, 900 of 7,168 22.1 / 20.2;
+// all groups' loads in front of the first store: 2,048 rows of 8,192 in two slices 61.4, one after the other 58.4.
+template <typename D, typename W, typename O, int NV, bool ONE>
 __global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(float* __restrict__ residual, const D* __restrict__ delta,
                                                            int slices, int64_t slice_stride,
                                                            const W* __restrict__ weight, O* __restrict__ out, int width,
@@ -112,37 +116,22 @@ __global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(float* __restrict__ r
   const int64_t row = blockIdx.x;
   const int quads = width / 4;
   float4 v[NV], wq[NV];
-  float sum[NV][4] = {};
   float ss = 0.f;
-  // (all of a thread's groups are asked for before the first is stored: a store waits for its sum)
-#pragma unroll
-  for (int e = 0; e < NV; ++e) {
-    const int q = threadIdx.x + e * blockDim.x;
-    v[e] = *reinterpret_cast<const float4*>(residual + row * width + 4 * static_cast<int64_t>(q < quads ? q : 0));
-    wq[e] = load_weights4(weight + 4 * (q < quads ? q : 0));
-  }
-  if (delta != nullptr) {
-    const D* from[NV];
-#pragma unroll
-    for (int e = 0; e < NV; ++e) {
-      const int q = threadIdx.x + e * blockDim.x;
-      from[e] = delta + row * width + 4 * static_cast<int64_t>(q < quads ? q : 0);
-    }
-    if (slices == 1) {
-#pragma unroll
-      for (int e = 0; e < NV; ++e) load_values<4>(from[e], sum[e]);
-    } else {
-#pragma unroll
-      for (int e = 0; e < NV; ++e) sum_values<4>(from[e], slices, slice_stride, sum[e]);
-    }
-  }
 #pragma unroll
   for (int e = 0; e < NV; ++e) {
     const int q = threadIdx.x + e * blockDim.x;
     const bool in = q < quads;
-    v[e] = float4{v[e].x + sum[e][0], v[e].y + sum[e][1], v[e].z + sum[e][2], v[e].w + sum[e][3]};
+    const int64_t at = row * width + 4 * static_cast<int64_t>(in ? q : 0);
+    const float4 x4 = *reinterpret_cast<const float4*>(residual + at);
+    wq[e] = load_weights4(weight + 4 * (in ? q : 0));
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    if (delta != nullptr) {
+      if constexpr (ONE) load_values<4>(delta + at, sum);
+      else sum_values<4>(delta + at, slices, slice_stride, sum);
+    }
+    v[e] = float4{x4.x + sum[0], x4.y + sum[1], x4.z + sum[2], x4.w + sum[3]};
     if (!in) v[e] = float4{0.f, 0.f, 0.f, 0.f};
-    if (in && delta != nullptr) *reinterpret_cast<float4*>(residual + row * width + 4 * static_cast<int64_t>(q)) = v[e];
+    if (in && delta != nullptr) *reinterpret_cast<float4*>(residual + at) = v[e];
     ss += v[e].x * v[e].x + v[e].y * v[e].y + v[e].z * v[e].z + v[e].w * v[e].w;
   }
   const float scale = rsqrtf(block_sum(ss, scratch) / static_cast<float>(width) + eps);
@@ -171,10 +160,13 @@ static int rmsnorm_launch_out(float* residual, const D* delta, int slices, const
       const int nv = (threads > 1024 || (quads > 64 && static_cast<int64_t>(rows) * (threads / 64) > 8192)) ? 2 : 1;
       if (nv == 2) threads = ((quads + 1) / 2 + 63) / 64 * 64;
       if (nv == 1) {
-        DISTIE_DISPATCH(out_dtype, O, (rmsnorm_vec_kernel<D, W, O, 1><<<rows, threads, 0, stream>>>(
+        DISTIE_DISPATCH(out_dtype, O, (rmsnorm_vec_kernel<D, W, O, 1, false><<<rows, threads, 0, stream>>>(
+                                          residual, delta, slices, slice_stride, weight, static_cast<O*>(out), width, eps)));
+      } else if (slices == 1) {
+        DISTIE_DISPATCH(out_dtype, O, (rmsnorm_vec_kernel<D, W, O, 2, true><<<rows, threads, 0, stream>>>(
                                           residual, delta, slices, slice_stride, weight, static_cast<O*>(out), width, eps)));
       } else {
-        DISTIE_DISPATCH(out_dtype, O, (rmsnorm_vec_kernel<D, W, O, 2><<<rows, threads, 0, stream>>>(
+        DISTIE_DISPATCH(out_dtype, O, (rmsnorm_vec_kernel<D, W, O, 2, false><<<rows, threads, 0, stream>>>(
                                           residual, delta, slices, slice_stride, weight, static_cast<O*>(out), width, eps)));
       }
       return launch_status();
